@@ -244,7 +244,8 @@ int mi_moe_gather_qmm_typed(const void *x, const uint32_t *w, const void *scales
  * transpose = 0 (the op's own default; test_quantized_matmul, ops/quantization.rs:318-342):
  * w [K, N*bits/32], scales, biases [K, N/group_size], y = x . dequantize(w), a plain kernel; so are
  * group sizes 32 / 128 and 2-bit codes.
- * workspace >= mi_moe_quantized_matmul_workspace_size (the plain kernels need none). */
+ * workspace >= mi_moe_quantized_matmul_workspace_size; products that the bf16, group-64 kernels do not
+ * serve also run with less or none, more slowly. */
 int mi_moe_quantized_matmul_workspace_size(int64_t M, int32_t K, int32_t bits, size_t *bytes);
 int mi_moe_quantized_matmul(const uint16_t *x, const uint32_t *w, const uint16_t *scales,
                             const uint16_t *biases, int64_t M, int32_t N, int32_t K,

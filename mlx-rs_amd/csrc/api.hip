@@ -867,16 +867,29 @@ static size_t qmm_dense_bytes(int64_t M, int32_t K, int32_t bits, size_t *mt_wor
   return b;
 }
 
+static size_t codes_bytes(int64_t M, int32_t K, int32_t group_size, int32_t bits, int32_t dtype) {
+  return 256 + align_up(codes_copy_bytes(dtype, bits, M, K)) + align_up(codes_sums_bytes(M, K, group_size));
+}
+
 int mi_moe_quantized_matmul_workspace_size(int64_t M, int32_t K, int32_t bits, size_t *bytes) try {
   if (!bytes) return fail("quantized_matmul_workspace_size: bytes is NULL");
   if (M < 0 || K <= 0 || M * (int64_t)K > (int64_t)1 << 40) return fail("quantized_matmul_workspace_size: bad sizes");
   size_t mt = 0;
-  *bytes = qmm_dense_bytes(M, K, bits, &mt);
+  const size_t tuned = qmm_dense_bytes(M, K, bits, &mt), codes = codes_bytes(M, K, 32, bits, MI_MOE_DTYPE_F16);
+  *bytes = tuned > codes ? tuned : codes;  // (the group size and the element type are not known here: the largest need)
   return 0;
 } MI_CATCH("quantized_matmul_workspace_size")
 
+// The tiled product on raw codes: transposed weights that the bf16, group-64 kernels do not take.  Its descriptors hold
+// a 32-bit size of one matrix.
+static bool codes_shape(int32_t dtype, int32_t transpose, int32_t group_size, int32_t bits, int32_t N, int32_t K) {
+  return transpose && bits != 2 && !tuned_shape(dtype, transpose, group_size, bits, N, K) && K % 128 == 0 &&
+         (int64_t)N * K * bits / 8 < (int64_t)1 << 31 && (int64_t)N * K < (int64_t)1 << 33;
+}
+
+// linear_bias: [N] added with a rounding of its own, or nullptr
 static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *scales, const void *biases,
-                                 int64_t M, int32_t N, int32_t K, int32_t transpose, int32_t group_size,
+                                 const void *linear_bias, int64_t M, int32_t N, int32_t K, int32_t transpose, int32_t group_size,
                                  int32_t bits, int32_t dtype, void *y, void *workspace, size_t workspace_bytes,
                                  void *stream) {
   if (check_qmm_shape("quantized_matmul", dtype, transpose, group_size, bits, N, K)) return 1;
@@ -884,9 +897,32 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
   if (M == 0) return 0;
   if (!x || !w || !scales || !biases || !y) return fail("quantized_matmul: x, w, scales, biases and y must be non-NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // From six rows on (eight with f32): the plain kernel's time grows with the rows, 3.4 us each after 7 us for one at
+  // N = K = 4096 and 4 bits (f16; 6 with 8 bits), against 19 us flat for the smallest tile (30 with f32).
+  if (codes_shape(dtype, transpose, group_size, bits, N, K) && M >= (dtype == MI_MOE_DTYPE_F32 ? 8 : 6) && M * K * 4 < (int64_t)1 << 31 && workspace &&
+      workspace_bytes >= codes_bytes(M, K, group_size, bits, dtype) && aligned16(x) && aligned16(w) && aligned16(y)) {
+    Carver cv(workspace);
+    const size_t copy_bytes = codes_copy_bytes(dtype, bits, M, K);
+    uint16_t *copy = copy_bytes ? reinterpret_cast<uint16_t *>(cv.take<char>(copy_bytes)) : nullptr;
+    uint16_t *sums = reinterpret_cast<uint16_t *>(cv.take<char>(codes_sums_bytes(M, K, group_size)));
+    MI_HIP(launch_prepare_rows(x, M, K, group_size, dtype, copy, sums, st));
+    CodesArgs a{};
+    a.x = copy ? copy : x;
+    a.x_rows = M;
+    a.sums = sums;
+    a.w0 = w; a.s0 = scales; a.b0 = biases;
+    a.bias = linear_bias;
+    a.y = y;
+    a.N = N;
+    a.K = K;
+    a.M = M;
+    MI_HIP(launch_qmm_codes_dense(a, group_size, bits, dtype, st));
+    return 0;
+  }
   if (!tuned_shape(dtype, transpose, group_size, bits, N, K)) {  // the plain kernels, no workspace
     MI_HIP(launch_qmm_plain(x, w, scales, biases, nullptr, nullptr, nullptr, nullptr, 0u, 1u, M, 1, N, K, group_size, bits,
                             transpose != 0, dtype, y, st));
+    if (linear_bias) MI_HIP(launch_add_row_bias(y, linear_bias, M, N, dtype, st));
     return 0;
   }
   if (!aligned16(x) || !aligned16(w) || !aligned16(scales) || !aligned16(biases) || !aligned16(y))
@@ -920,6 +956,7 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
   a.total_rows = M;
   a.max_rows_per_expert = M;
   MI_HIP(launch_grouped_qmm(a, false, st));
+  if (linear_bias) MI_HIP(launch_add_row_bias(y, linear_bias, M, N, dtype, st));
   return 0;
 }
 
@@ -927,7 +964,7 @@ int mi_moe_quantized_matmul(const uint16_t *x, const uint32_t *w, const uint16_t
                             const uint16_t *biases, int64_t M, int32_t N, int32_t K, int32_t transpose,
                             int32_t group_size, int32_t bits, uint16_t *y, void *workspace,
                             size_t workspace_bytes, void *stream) try {
-  return quantized_matmul_impl(x, w, scales, biases, M, N, K, transpose, group_size, bits, MI_MOE_DTYPE_BF16, y,
+  return quantized_matmul_impl(x, w, scales, biases, nullptr, M, N, K, transpose, group_size, bits, MI_MOE_DTYPE_BF16, y,
                                workspace, workspace_bytes, stream);
 } MI_CATCH("quantized_matmul")
 
@@ -935,7 +972,7 @@ int mi_moe_quantized_matmul_typed(const void *x, const uint32_t *w, const void *
                                   int64_t M, int32_t N, int32_t K, int32_t transpose, int32_t group_size,
                                   int32_t bits, int32_t dtype, void *y, void *workspace, size_t workspace_bytes,
                                   void *stream) try {
-  return quantized_matmul_impl(x, w, scales, biases, M, N, K, transpose, group_size, bits, dtype, y, workspace,
+  return quantized_matmul_impl(x, w, scales, biases, nullptr, M, N, K, transpose, group_size, bits, dtype, y, workspace,
                                workspace_bytes, stream);
 } MI_CATCH("quantized_matmul_typed")
 
@@ -943,10 +980,8 @@ int mi_moe_quantized_linear_typed(const void *x, const uint32_t *w, const void *
                                   const void *linear_bias, int64_t M, int32_t N, int32_t K, int32_t group_size,
                                   int32_t bits, int32_t dtype, void *y, void *workspace, size_t workspace_bytes,
                                   void *stream) try {
-  if (quantized_matmul_impl(x, w, scales, biases, M, N, K, 1, group_size, bits, dtype, y, workspace, workspace_bytes, stream))
-    return 1;
-  if (linear_bias && M > 0) MI_HIP(launch_add_row_bias(y, linear_bias, M, N, dtype, static_cast<hipStream_t>(stream)));
-  return 0;
+  return quantized_matmul_impl(x, w, scales, biases, linear_bias, M, N, K, 1, group_size, bits, dtype, y, workspace,
+                               workspace_bytes, stream);
 } MI_CATCH("quantized_linear_typed")
 
 int mi_moe_swiglu(const uint16_t *gate, const uint16_t *up, int64_t n, uint16_t *out, void *stream) try {

@@ -326,6 +326,27 @@ hipError_t launch_qmm_plain(const void *x, const uint32_t *w, const void *scales
                             const uint32_t *lhs, const uint32_t *rhs, const uint32_t *rhs_map,
                             const uint32_t *dst_map, uint32_t n_lhs, uint32_t n_rhs, int64_t rows, int M, int N,
                             int K, int group, int bits, bool transpose, int dt, void *y, hipStream_t st);
+// The tiled product on raw codes (qmm_codes.hip): any float type, groups of 32 / 64 / 128, 4- and 8-bit codes,
+// transposed weights.  x: what launch_prepare_rows made of the rows (`copy` where codes_copy_bytes is not zero, else
+// the rows themselves), sums: the group sums it wrote.
+struct CodesArgs {
+  const void *x;
+  int64_t x_rows;  // rows of x (and of sums)
+  const uint16_t *sums;
+  const uint32_t *src_rows, *dst_rows;  // as in GroupedArgs
+  const uint32_t *w0, *w1;
+  const void *s0, *b0, *s1, *b1;
+  const void *bias;  // [N] added after the rounding of the product, with a rounding of its own; or nullptr
+  void *y;
+  bool y_paired;
+  int N, K;
+  int64_t M;  // rows (dense launches)
+};
+size_t codes_copy_bytes(int dt, int bits, int64_t rows, int K);
+size_t codes_sums_bytes(int64_t rows, int K, int group);
+hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
+                               uint16_t *sums, hipStream_t st);
+hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
 hipError_t launch_quantize(const float *w, int64_t rows, int64_t cols, int group, int bits,
                            uint32_t *q, void *s, void *b, int dt, hipStream_t st);
 hipError_t launch_dequantize(const uint32_t *q, const void *s, const void *b,

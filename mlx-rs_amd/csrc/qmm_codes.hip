@@ -1,0 +1,716 @@
+// Tiled quantized product on raw codes, for everything the bfloat16 / group-64 kernels do not take: activations in
+// bfloat16, float16 or float32, groups of 32, 64 or 128, any number of output columns.
+//
+// Contract: mlx_quantized_matmul / mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:91-122,160-230).
+//
+// Arithmetic: sum_c x_c (s q_c + b) = s sum_c x_c q_c + b sum_c x_c per quantisation group.  The codes are exact in
+// bf16 and in f16, so the matrix cores multiply the activations with raw codes and nothing is rounded on the way in:
+//   bf16  x as it is; 4-bit codes as 128 + q (one and-or per pair), the 128 taken back through the bias term
+//   f16   x as it is, codes in f16 (v_mfma_f32_32x32x16_f16)
+//   f32   x as three bf16 pieces of 8 significant bits each (an exact split), three products per code operand
+// The fp32 sums of a group are scaled once, when the group ends.  The bias term sum_g b_g (sum_c x_c) is a product of
+// its own over the groups: the group sums of x (fp32, split into three bf16 pieces) against the biases (three pieces
+// as well), eight K slots a group (xh bh, xm bh, xl bh, xh bm, xm bm, xh bl: every product down to 2^-24), which the
+// matrix cores accumulate straight into the result: K / group * 8 / K = 12 % more MFMA work with groups of 64.
+//
+// A kernel of its own (prepare_rows) walks x once and writes the group sums in that form and, for 4-bit codes with bf16
+// and f16, the copy with paired 8-blocks that their unpacking wants.
+#include <type_traits>
+
+#include "common.hpp"
+
+namespace mi_moe {
+
+namespace {
+
+constexpr int kStep = 64;      // K values per step; two steps between barriers
+constexpr int kRow = 17;       // LDS row stride in 16-byte units: 128 values and 16 bytes that keep rows off each other's banks
+constexpr uint32_t kOutside = 0x80000000u;  // an offset past every descriptor here: such a load returns zeros
+constexpr int kSlots = 8;      // K slots of a group in the bias product
+#ifndef MI_CODES_WEAVE
+#define MI_CODES_WEAVE 7
+#endif
+constexpr int kWeave = MI_CODES_WEAVE;  // vector instructions between two matrix instructions
+constexpr size_t kLdsAtLeast = 4 * 32 * (32 * 4 + 16);  // the epilogue's staging
+
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
+
+template <int DT> struct ElemOf;
+template <> struct ElemOf<0> { typedef uint16_t type; };
+template <> struct ElemOf<1> { typedef _Float16 type; };
+template <> struct ElemOf<2> { typedef float type; };
+
+__device__ __forceinline__ float as_f32(uint16_t v) { return bf16_to_f32(v); }
+__device__ __forceinline__ float as_f32(_Float16 v) { return (float)v; }
+__device__ __forceinline__ float as_f32(float v) { return v; }
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void *base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+
+template <int DT>
+__device__ __forceinline__ f32x16_t mfma(u32x4_t a, u32x4_t b, f32x16_t c) {
+  if constexpr (DT == 1)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// v = h + m + l exactly, each a bf16 (8 significant bits; by truncation, so nothing overflows).  A value that is not
+// finite gives a NaN.
+struct Pieces { uint32_t h, m, l; };  // bf16 bits in the low halves
+__device__ __forceinline__ Pieces split3(float v) {
+  const uint32_t u = __float_as_uint(v);
+  const uint32_t hu = u & 0xffff0000u;
+  const float r = v - __uint_as_float(hu);
+  const uint32_t mu = __float_as_uint(r) & 0xffff0000u;
+  const float q = r - __uint_as_float(mu);
+  return Pieces{hu >> 16, mu >> 16, __float_as_uint(q) >> 16};
+}
+
+// a multiply function together with the instruction mix its step is scheduled in
+template <class Weave, class F>
+struct Woven : F {
+  __device__ __forceinline__ Woven(F f) : F(f) {}
+  static __device__ __forceinline__ void weave() { Weave::weave(); }
+};
+template <class Weave, class F>
+__device__ __forceinline__ Woven<Weave, F> with_weave(F f) { return Woven<Weave, F>(f); }
+
+template <class T>
+__device__ __forceinline__ T load_elem(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
+  else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0));
+}
+
+// a thread's share of a step's token rows
+template <int P, int NA>
+struct RowStage {
+  u32x4_t v[P][NA];
+};
+
+constexpr bool paired_order(int dt, int bits) { return bits == 4 && dt != 2; }  // 8-blocks as (0,4)(1,5)(2,6)(3,7)
+constexpr int n_parts(int dt) { return dt == 2 ? 3 : 1; }
+constexpr int padded_groups(int G) { return (G + 15) / 16 * 16; }  // the bias product runs an even number of steps of eight groups
+
+__device__ __forceinline__ uint32_t f16_minus_1024(uint32_t v) {  // two halves 1024 + q -> q: exact
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) - half2_t{(_Float16)1024, (_Float16)1024});
+}
+template <class T> __device__ __forceinline__ T rounded(float v) { return (T)v; }
+template <> __device__ __forceinline__ uint16_t rounded<uint16_t>(float v) { return (uint16_t)(cvt_pk_bf16(v, 0.f) & 0xffffu); }
+
+}  // namespace
+
+// One thread per eight values of x.
+template <int DT>
+__global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf<DT>::type *__restrict__ x, int64_t n_octets,
+                                                           int octets_per_row, int lanes_log2,
+                                                           uint16_t *__restrict__ copy, uint16_t *__restrict__ sums, int sums_row) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n_octets) return;  // whole groups leave together
+  float v[8];
+  if constexpr (DT == 2) {
+    const float4 lo = reinterpret_cast<const float4 *>(x)[2 * i], hi = reinterpret_cast<const float4 *>(x)[2 * i + 1];
+    v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+  } else {
+    const uint4 w = reinterpret_cast<const uint4 *>(x)[i];
+    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (DT == 0) {
+        v[2 * j] = bf16lo_to_f32(u[j]);
+        v[2 * j + 1] = bf16hi_to_f32(u[j]);
+      } else {
+        const half2_t hh = __builtin_bit_cast(half2_t, u[j]);
+        v[2 * j] = (float)hh.x;
+        v[2 * j + 1] = (float)hh.y;
+      }
+    }
+    if (copy) {
+      uint4 p;
+      p.x = (w.x & 0xffffu) | (w.z << 16);
+      p.y = (w.x >> 16) | (w.z & 0xffff0000u);
+      p.z = (w.y & 0xffffu) | (w.w << 16);
+      p.w = (w.y >> 16) | (w.w & 0xffff0000u);
+      *reinterpret_cast<uint4 *>(copy + 8 * i) = p;
+    }
+  }
+  float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
+  sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
+  if (lanes_log2 >= 3) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
+  if (lanes_log2 == 4) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
+  if ((i & ((1 << lanes_log2) - 1)) == 0) {
+    const int64_t row = i / octets_per_row;
+    const int g = (int)(i % octets_per_row) >> lanes_log2, G = octets_per_row >> lanes_log2;
+    const Pieces p = split3(sum);
+    uint4 *const to = reinterpret_cast<uint4 *>(sums + row * sums_row) + g;
+    *to = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, 0u);
+    if (g == G - 1)
+      for (int k = 1; g + k < sums_row / kSlots; ++k) to[k] = make_uint4(0, 0, 0, 0);
+  }
+}
+
+// A block computes 32 MS token rows x 32 WN NT weight rows with WN KW waves.  A wave owns 32 weight rows (NT = 2: and
+// the 32 matching ones of the up matrix, or 32 WN rows further on) for all the block's token rows, so it loads its own codes straight
+// into the lanes that multiply them and unpacks them in registers: nothing of the weights passes through LDS, and no
+// wave unpacks what another one does.  A lane (weight row l % 32, half l / 32) loads 16 bytes; which K values its
+// eight codes of a multiply stand for is free as long as the token operand agrees:
+//   4-bit, groups >= 64: 16 bytes are 32 codes, half h holds K values 32 h ..: multiply t takes word t of both halves;
+//   4-bit, groups of 32: two v_permlane32_swap deal the words so that a multiply stays inside one group;
+//   8-bit: 16 bytes are 16 codes, two loads a step, groups of 32 stay apart by themselves.
+// Token rows pass through LDS (128 K values between two barriers, double-buffered).
+// A step takes one 32 x 32 sub-tile after the other: its four multiplies follow each other in one accumulator, and the
+// scaled addition of the sub-tile before it (16 fma) and the unpacking of the next step's codes (9 to 11 instructions a
+// multiply) run between them, which is as much vector work as fits beside the matrix cores.
+// What bounds it (777 x 4096 x 4096, f16, 8-bit; 26 GFLOP): 62 us for the call = 420 TFLOP/s, 50 times the plain kernel's
+// 3160 us; the matrix cores alone would take 18.  Taken apart at one block a CU (cycles per 64 K values of 128 x 32 a
+// wave, 512 of them matrix work): multiplies and barriers 575, with the vector work 640, with the reads of LDS 840, with
+// the loads 1350.  The loads cost their line visits: a wave's codes sit in 32 rows.
+// KW > 1: the block's waves form KW groups that share K among them, each with LDS buffers of its own; their sums meet in
+// LDS at the end, added in group order.  For launches that give a CU one block or less.
+// DT: 0 bf16, 1 f16, 2 f32.  G32: groups of 32; otherwise a group is one or two steps (scale_shift).
+template <int DT, int BITS, bool G32, bool GLU, int MS, int NT, int WN, int KW>
+__global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2, 4))) void qmm_codes_kernel(
+    CodesArgs a, const uint32_t *__restrict__ tiles, int n_mtiles, int n_ntiles, int sub_log2, int scale_shift) {
+  static_assert(!GLU || NT == 2, "a gate tile and its up tile");
+  typedef typename ElemOf<DT>::type T;
+  constexpr int NP = n_parts(DT);
+  constexpr int BM = 32 * MS;
+  constexpr int NI = 32 * WN * (GLU ? 1 : NT);  // distinct output columns per block
+  constexpr int NA = BM * 8 / (64 * WN);     // 16-byte activation loads per thread, piece and step
+  constexpr int RS = 8 * WN;                 // rows one such load of a group covers
+  constexpr int NQ = BITS == 4 ? 1 : 2;      // 16-byte code loads per lane, tile and step
+  constexpr int NS = G32 ? 2 : 1;            // scaled additions per sub-tile and step
+  constexpr bool SPLIT = BITS == 8 || G32;   // which K values a multiply takes: see chunk below
+  constexpr float kOffset = BITS == 4 && DT == 0 ? 128.0f : 0.0f;  // the codes are multiplied as offset + q
+  constexpr int A_SZ = BM * kRow, BUF = NP * A_SZ;                 // 16-byte units
+  static_assert(BM % RS == 0, "whole loads");
+
+  // block -> (M tile, N tile).  Ids are dealt round-robin over the 8 XCDs.  Dense: an XCD takes every eighth N tile
+  // and all M tiles of it, so its L2 holds the weights of a few N tiles and x streams through.  Tile lists: whole M
+  // tiles per XCD (the blocks of one share its gathered rows).
+  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+  int e = 0, rows, nt;
+  int64_t row0;
+  if (tiles) {
+    const uint32_t mt_id = (uint32_t)(j / n_ntiles) * 8u + xcd;
+    nt = j % n_ntiles;
+    if (mt_id >= tiles[0] << sub_log2) return;
+    const uint4 rec = reinterpret_cast<const uint4 *>(tiles)[1 + (mt_id >> sub_log2)];
+    const int part = (int)(mt_id & ((1u << sub_log2) - 1u)) * BM;
+    e = (int)rec.x;
+    row0 = (int64_t)rec.y + part;
+    rows = (int)rec.z - part < BM ? (int)rec.z - part : BM;
+  } else {
+    nt = j / n_mtiles * 8 + xcd;
+    if (nt >= n_ntiles) return;
+    row0 = (int64_t)(j % n_mtiles) * BM;
+    rows = a.M - row0 < BM ? (int)(a.M - row0) : BM;
+  }
+  if (rows <= 0) return;
+
+  const int lane = threadIdx.x & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave_all % WN, kg = wave_all / WN;  // column tile, K group
+  const int tid = wave * 64 + lane;                    // within the K group
+  const int N = a.N, K = a.K;
+  const int n0 = nt * NI;
+  const int G = K / (G32 ? 32 : 64 << scale_shift), row_bytes = K * BITS / 8;
+
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  u32x4_t *const lds = reinterpret_cast<u32x4_t *>(lds_raw) + kg * (2 * BUF);
+
+  // ---- what a thread stages: chunk acp (8 K values) of token rows arg, arg + RS, ...  Offsets are 32 bits: the host
+  // takes this kernel for operands below 4 GiB only.
+  const int acp = tid & 7, arg = tid >> 3;
+  const int pg = padded_groups(G), ext = pg * kSlots;
+  const __amdgpu_buffer_rsrc_t xr = rsrc_of(a.x, (uint32_t)(a.x_rows * K * sizeof(T))), xsr = rsrc_of(a.sums, (uint32_t)(a.x_rows * ext * 2));
+  uint32_t x_voff[NA], xs_voff[NA];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+    int tr = arg + RS * i;
+    tr = tr < rows ? tr : rows - 1;  // rows past the end repeat the last one (never stored)
+    const uint32_t r = a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr);
+    x_voff[i] = (r * (uint32_t)K + acp * 8) * sizeof(T);
+    xs_voff[i] = (r * (uint32_t)ext + acp * 8) * 2;
+  }
+  // ---- the weight rows of this lane
+  const int ln = lane & 31, kb = lane >> 5;
+  const int64_t ebase = (int64_t)e * N;
+  __amdgpu_buffer_rsrc_t wr[NT], sr[NT], br[NT];
+  uint32_t w_voff[NT], s_voff[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const bool up = GLU && t == 1;
+    // paired output (see GroupedArgs::y_paired): the lane at position p of an 8-block takes the row whose result belongs there
+    const int lnp = a.y_paired ? ((ln & ~7) | (((ln & 7) >> 1) + ((ln & 1) ? 4 : 0))) : ln;
+    int row = n0 + 32 * wave + lnp + (GLU ? 0 : 32 * WN * t);
+    row = row < N ? row : N - 1;  // columns past the end repeat the last one (never stored)
+    wr[t] = rsrc_of((up ? a.w1 : a.w0) + ebase * (row_bytes / 4), (uint32_t)N * row_bytes);
+    sr[t] = rsrc_of(static_cast<const T *>(up ? a.s1 : a.s0) + ebase * G, ((uint32_t)N * G * sizeof(T) + 3u) & ~3u);  // (read in words)
+    br[t] = rsrc_of(static_cast<const T *>(up ? a.b1 : a.b0) + ebase * G, (uint32_t)N * G * sizeof(T));
+    w_voff[t] = (uint32_t)row * row_bytes + kb * 16;
+    s_voff[t] = (uint32_t)row * G * sizeof(T);
+  }
+
+  f32x16_t tot[MS][NT];
+  const f32x16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int m = 0; m < MS; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) tot[m][t] = zero;
+
+  struct Operand {  // a step's weight operand: eight values a lane and multiply
+    u32x4_t v[NT][4];
+  };
+  auto nk_share = [](int nk) __attribute__((always_inline)) { return (nk / 2 + KW - 1) / KW * 2; };  // steps of a K group
+  // One pipelined pass of nk steps (an even number), dealt to the K groups in even shares (what a share has past the
+  // last step is multiplied with zeros).  Two steps at a time: while they are multiplied out of one LDS buffer, the
+  // token rows of the next two are on their way into registers, the codes run two steps ahead and are unpacked one
+  // step ahead.
+  // window_steps, window: called ahead of every so many steps.
+  auto pass = [&](int nk, auto a_type, auto b_type, auto load_a, auto put_a, auto load_b, auto unpack, auto multiply, int window_steps, auto window) __attribute__((always_inline)) {
+    decltype(a_type) RA[2];
+    decltype(b_type) RB[2];
+    auto put = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int i = 0; i < NA; ++i) put_a(lds + buf * BUF + (arg + RS * i) * kRow + 8 * d + acp, RA[d], i);
+    };
+    const int share = nk_share(nk);  // the same number of barriers for every group
+    const int k0 = kg * share, k1 = k0 + share < nk ? k0 + share : nk;
+    auto clamped = [&](int ks) __attribute__((always_inline)) { return ks < nk ? ks : nk - 1; };
+    load_b(clamped(k0), RB[0]);
+    load_a(clamped(k0), k0 < k1, RA[0]);
+    load_a(clamped(k0 + 1), k0 < k1, RA[1]);
+    load_b(clamped(k0 + 1), RB[1]);
+    Operand op[2];
+    unpack(RB[0], op[0]);
+    put(0);
+    __syncthreads();
+    int buf = 0;
+    for (int kw = k0; kw < k0 + share; kw += window_steps) {
+      window(kw);
+      for (int kq = kw; kq < k0 + share && kq < kw + window_steps; kq += 2) {
+        const u32x4_t *const At = lds + buf * BUF;
+        buf ^= 1;
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          load_b(clamped(kq + d + 2), RB[d]);
+          if (d == 0) {
+            load_a(clamped(kq + 2), kq + 2 < k1, RA[0]);
+            load_a(clamped(kq + 3), kq + 2 < k1, RA[1]);
+          }
+          __builtin_amdgcn_sched_barrier(0);  // (the loads stay at the head of the step)
+          multiply(At + 8 * d, op[d], d, kq + d);
+          unpack(RB[d ^ 1], op[d ^ 1]);
+          decltype(multiply)::weave();
+          if (d == 1) {
+            put(buf);
+            __syncthreads();
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  };
+
+  // ---- the bias product: group sums of x against b - offset s, accumulated into the result
+  {
+    typedef RowStage<1, NA> StageA;
+    auto put_a = [&](u32x4_t *to, const StageA &R, int i) __attribute__((always_inline)) { *to = R.v[0][i]; };
+    struct StageB {
+      T s[NT][4], b[NT][4];
+    };
+    auto load_a = [&](int ks, bool real, StageA &R) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+        R.v[0][i] = __builtin_amdgcn_raw_buffer_load_b128(xsr, KW == 1 || real ? xs_voff[i] : kOutside, ks * (kStep * 2), 0);
+    };
+    auto load_b = [&](int ks, StageB &R) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          int g = ks * 8 + 2 * h + kb;
+          g = g < G ? g : G - 1;  // (padding groups: their sums are zero)
+          R.b[t][h] = load_elem<T>(br[t], s_voff[t] + g * (uint32_t)sizeof(T), 0);
+          R.s[t][h] = kOffset != 0.f ? load_elem<T>(sr[t], s_voff[t] + g * (uint32_t)sizeof(T), 0) : T{};
+        }
+    };
+    auto unpack = [&](const StageB &R, Operand &o) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const Pieces p = split3(__builtin_fmaf(-kOffset, as_f32(R.s[t][h]), as_f32(R.b[t][h])));
+          o.v[t][h] = u32x4_t{p.h | p.h << 16, p.h | p.m << 16, p.m | p.l << 16, 0u};
+        }
+    };
+    struct Multiply {
+      static __device__ __forceinline__ void weave() {}
+    };
+    auto body = [&](const u32x4_t *At, const Operand &o, int, int) __attribute__((always_inline)) {
+#pragma unroll
+      for (int m = 0; m < MS; ++m)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const u32x4_t av = At[(32 * m + ln) * kRow + 2 * h + kb];
+#pragma unroll
+          for (int t = 0; t < NT; ++t) tot[m][t] = mfma<0>(av, o.v[t][h], tot[m][t]);
+        }
+    };
+    pass(pg / 8, StageA{}, StageB{}, load_a, put_a, load_b, unpack, with_weave<Multiply>(body), 1 << 30, [](int) {});
+  }
+
+  // ---- the product of the codes
+  {
+    constexpr int XP = DT == 2 ? 2 : 1;  // 16-byte pieces of eight values
+    typedef RowStage<XP, NA> StageA;
+    auto put_a = [&](u32x4_t *to, const StageA &R, int i) __attribute__((always_inline)) {
+      if constexpr (DT == 2) {
+        u32x4_t h, m, l;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const Pieces a = split3(__uint_as_float(R.v[q >> 1][i][2 * (q & 1)])), b = split3(__uint_as_float(R.v[q >> 1][i][2 * (q & 1) + 1]));
+          h[q] = a.h | b.h << 16;
+          m[q] = a.m | b.m << 16;
+          l[q] = a.l | b.l << 16;
+        }
+        to[0] = h;
+        to[A_SZ] = m;
+        to[2 * A_SZ] = l;
+      } else {
+        *to = R.v[0][i];
+      }
+    };
+    struct StageB {
+      u32x4_t q[NT][NQ];
+    };
+    f32x16_t acc[2][NS];  // the sub-tile being multiplied, and the one before it
+    float acc_s[2][NS];
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      acc[1][i] = zero;  // (nothing is pending yet)
+      acc_s[1][i] = 0.f;
+    }
+    auto add_scaled = [&](int which, int m, int t) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < NS; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tot[m][t][r] = __builtin_fmaf(acc_s[which][i], acc[which][i][r], tot[m][t][r]);
+    };
+    auto load_a = [&](int ks, bool real, StageA &R) __attribute__((always_inline)) {
+#pragma unroll
+      for (int p = 0; p < XP; ++p)
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+          R.v[p][i] = __builtin_amdgcn_raw_buffer_load_b128(xr, KW == 1 || real ? x_voff[i] : kOutside, ks * (kStep * (uint32_t)sizeof(T)) + 16 * p, 0);
+    };
+    auto load_b = [&](int ks, StageB &R) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+#pragma unroll
+        for (int h = 0; h < NQ; ++h)
+          R.q[t][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[t], w_voff[t], ks * (kStep * BITS / 8) + 32 * h, 0);
+      }
+    };
+    auto unpack = [&](const StageB &cur, Operand &o) __attribute__((always_inline)) {
+      StageB R = cur;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        if constexpr (BITS == 4 && G32) {
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            const auto r = __builtin_amdgcn_permlane32_swap(R.q[t][0][w], R.q[t][0][w + 2], false, false);
+            R.q[t][0][w] = r[0];
+            R.q[t][0][w + 2] = r[1];
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          if constexpr (BITS == 4 && DT != 2) {
+            const uint32_t w = R.q[t][0][h];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              if constexpr (DT == 0) {
+                o.v[t][h][i] = __builtin_amdgcn_bitop3_b32(w >> (4 * i), 0x000f000fu, 0x43004300u, 0xEA);  // (a & b) | c
+              } else if (i % 2 == 0) {
+                o.v[t][h][i] = f16_minus_1024(__builtin_amdgcn_bitop3_b32(w >> (4 * i), 0x000f000fu, 0x64006400u, 0xEA));
+              } else {  // 1024 + 16 q -> q, exact as well: one shift serves two nibbles
+                const half2_t v = __builtin_bit_cast(half2_t, __builtin_amdgcn_bitop3_b32(w >> (4 * (i - 1)), 0x00f000f0u, 0x64006400u, 0xEA));
+                o.v[t][h][i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, half2_t{(_Float16)0.0625f, (_Float16)0.0625f}, half2_t{(_Float16)-64.0f, (_Float16)-64.0f}));
+              }
+            }
+          } else if constexpr (DT == 1) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)  // bytes 2 i, 2 i + 1 under the exponent of 1024
+              o.v[t][h][i] = f16_minus_1024(__builtin_amdgcn_perm(0x64646464u, R.q[t][h >> 1][2 * (h & 1) + (i >> 1)],
+                                                                  (i & 1) ? 0x07030702u : 0x07010700u));
+          } else {  // codes through v_cvt_f32_ubyte, upper halves packed
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              uint32_t c0, c1;  // codes 2 i, 2 i + 1
+              if constexpr (BITS == 4) {
+                const uint32_t w = R.q[t][0][h];
+                c0 = ((w & 0x0f0f0f0fu) >> (8 * i)) & 0xffu;
+                c1 = (((w >> 4) & 0x0f0f0f0fu) >> (8 * i)) & 0xffu;
+              } else {
+                const uint32_t w = R.q[t][h >> 1][2 * (h & 1) + (i >> 1)];
+                c0 = (w >> (16 * (i & 1))) & 0xffu;
+                c1 = (w >> (16 * (i & 1) + 8)) & 0xffu;
+              }
+              o.v[t][h][i] = __builtin_amdgcn_perm(__float_as_uint((float)c1), __float_as_uint((float)c0), 0x07060302u);
+            }
+          }
+        }
+      }
+    };
+    struct Multiply {  // the step's instruction mix: matrix, vector and LDS instructions in turn
+      static __device__ __forceinline__ void weave() {
+        __builtin_amdgcn_sched_group_barrier(0x100, 4 * NP, 0);
+#pragma unroll
+        for (int i = 0; i < MS * NT * NP * 4; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, kWeave, 0);
+          if (i % NT == 0 && i < (MS - 1) * NT * NP * 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+      }
+    };
+    // The scales of this wave's rows pass through LDS a window at a time: a lane fetches 16 bytes of its row (half kb of
+    // the window) one window ahead, and reads one value per group back.  One 2-byte load per group from a row each
+    // touches as many lines as the codes themselves (measured: a quarter of the kernel's time).
+    // The fetch is aligned down to 4 bytes (with an odd number of 2-byte scales per row, every second row starts between
+    // two words): the window then gives up its last scale.
+    const int win = sizeof(T) == 2 && (G & 1) ? 8 : 2 * 16 / (int)sizeof(T);  // scales of a window
+    constexpr int SROW = 32 + 16;                  // bytes per row of the window
+    unsigned char *const swin = reinterpret_cast<unsigned char *>(lds_raw) + 2 * KW * BUF * 16 + wave_all * (NT * 32 * SROW);
+    const int first_group = (nk_share(K / kStep) * kg) * (G32 ? 2 : 1) >> scale_shift;
+    u32x4_t swin_next[NT];
+    auto load_window = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        swin_next[t] = __builtin_amdgcn_raw_buffer_load_b128(sr[t], ((s_voff[t] + g * (uint32_t)sizeof(T)) & ~3u) + kb * 16, 0, 0);
+    };
+    load_window(first_group);
+    int gw = first_group;        // first group of the window in LDS
+    const unsigned char *s_at[NT];  // this lane's scale of that group
+    auto window = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) *reinterpret_cast<u32x4_t *>(swin + (t * 32 + ln) * SROW + kb * 16) = swin_next[t];
+      gw = (ks * (G32 ? 2 : 1)) >> scale_shift;
+      load_window(gw + win);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) s_at[t] = swin + (t * 32 + ln) * SROW + ((s_voff[t] + gw * (uint32_t)sizeof(T)) & 3u);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    auto body = [&](const u32x4_t *At, const Operand &o, int d, int ks) __attribute__((always_inline)) {
+      float step_s[NT][NS];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < NS; ++i)
+          step_s[t][i] = as_f32(*reinterpret_cast<const T *>(s_at[t] + ((G32 ? 2 * ks + i : ks >> scale_shift) - gw) * (int)sizeof(T)));
+#pragma unroll
+      for (int m = 0; m < MS; ++m) {
+        u32x4_t av[4][NP];
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+#pragma unroll
+          for (int p = 0; p < NP; ++p) {
+            const int c = SPLIT ? 4 * (h >> 1) + 2 * kb + (h & 1) : 4 * kb + h;  // the chunk of K values multiply h takes
+            av[h][p] = At[p * A_SZ + (32 * m + ln) * kRow + c];
+          }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const int which = (d * MS * NT + m * NT + t) & 1;
+#pragma unroll
+          for (int h = 0; h < 4; ++h) {
+            const int i = G32 ? h >> 1 : 0;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+              const bool first = p == 0 && (G32 ? (h & 1) == 0 : h == 0);
+              acc[which][i] = mfma<DT>(av[h][p], o.v[t][h], first ? zero : acc[which][i]);
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < NS; ++i) acc_s[which][i] = step_s[t][i];
+          const int before = m * NT + t > 0 ? m * NT + t - 1 : MS * NT - 1;
+          add_scaled(which ^ 1, before / NT, before % NT);
+        }
+      }
+    };
+    pass(K / kStep, StageA{}, StageB{}, load_a, put_a, load_b, unpack, with_weave<Multiply>(body),
+         (win >> (G32 ? 1 : 0)) << scale_shift, window);
+    add_scaled(1, MS - 1, NT - 1);  // an even number of steps ends in accumulator 1
+  }
+
+  if constexpr (KW > 1) {  // (the passes end in a barrier: LDS is free)
+    float *const parts = reinterpret_cast<float *>(lds_raw) + (wave * 64 + lane) * 4;  // 16-byte pieces, lane by lane
+    constexpr int kPiece = 64 * WN * 4;
+#pragma unroll
+    for (int g = 1; g < KW; ++g) {
+      if (kg == g) {
+#pragma unroll
+        for (int m = 0; m < MS; ++m)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              *reinterpret_cast<float4 *>(parts + ((m * NT + t) * 4 + r) * kPiece) =
+                  make_float4(tot[m][t][4 * r], tot[m][t][4 * r + 1], tot[m][t][4 * r + 2], tot[m][t][4 * r + 3]);
+      }
+      __syncthreads();
+      if (kg == 0) {
+#pragma unroll
+        for (int m = 0; m < MS; ++m)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float4 v = *reinterpret_cast<const float4 *>(parts + ((m * NT + t) * 4 + r) * kPiece);
+              tot[m][t][4 * r] += v.x;
+              tot[m][t][4 * r + 1] += v.y;
+              tot[m][t][4 * r + 2] += v.z;
+              tot[m][t][4 * r + 3] += v.w;
+            }
+      }
+      __syncthreads();
+    }
+    if (kg != 0) return;
+  }
+
+  // ---- epilogue: a wave turns its 32 x 32 sub-tiles round in a private piece of LDS and stores 16 bytes a lane
+  constexpr int ROWB = 32 * (int)sizeof(T) + 16;
+  constexpr int PV = 16 / (int)sizeof(T);             // values per 16-byte piece
+  constexpr int CPR = 32 / PV;                        // pieces per row
+  constexpr int RPI = 64 / CPR;                       // rows one store instruction covers
+  static_assert(WN * 32 * ROWB <= kLdsAtLeast, "staging does not fit");
+  unsigned char *const mine = lds_raw + wave * (32 * ROWB);
+  const int my_piece = lane % CPR, my_row = lane / CPR;
+  const bool vec = N % PV == 0;
+#pragma unroll
+  for (int m = 0; m < MS; ++m)
+#pragma unroll
+    for (int t = 0; t < (GLU ? 1 : NT); ++t) {
+      const int col0 = n0 + 32 * wave + 32 * WN * t;
+      const int bc = col0 + ln < N ? col0 + ln : N - 1;
+      const float lb = a.bias ? as_f32(static_cast<const T *>(a.bias)[bc]) : 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = 8 * (r >> 2) + 4 * kb + (r & 3);
+        float v;
+        if constexpr (GLU) {
+          const float g = tot[m][0][r], u = tot[m][1][r];
+          v = g / (1.0f + __expf(-g)) * u;
+        } else {
+          v = tot[m][t][r];
+        }
+        T o = rounded<T>(v);
+        if (a.bias) o = rounded<T>(as_f32(o) + lb);
+        reinterpret_cast<T *>(mine + row * ROWB)[ln] = o;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const int my_col = col0 + PV * my_piece;
+#pragma unroll
+      for (int i = 0; i < 32 / RPI; ++i) {
+        const int row = RPI * i + my_row;
+        const int tr = 32 * m + row;
+        if (tr < rows && my_col < N) {
+          const int64_t dst = a.dst_rows ? (int64_t)a.dst_rows[row0 + tr] : row0 + tr;
+          T *const to = static_cast<T *>(a.y) + dst * N + my_col;
+          const T *const from = reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece;
+          if (vec) {
+            *reinterpret_cast<u32x4_t *>(to) = *reinterpret_cast<const u32x4_t *>(from);
+          } else {
+            for (int c = 0; c < PV && my_col + c < N; ++c) to[c] = from[c];
+          }
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+}
+
+size_t codes_copy_bytes(int dt, int bits, int64_t rows, int K) {
+  return paired_order(dt, bits) ? (size_t)rows * K * 2 : 0;
+}
+size_t codes_sums_bytes(int64_t rows, int K, int group) { return (size_t)rows * padded_groups(K / group) * kSlots * 2; }
+
+hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
+                               uint16_t *sums, hipStream_t st) {
+  const int64_t n = rows * (K / 8);
+  if (n == 0) return hipSuccess;
+  const unsigned grid = (unsigned)((n + 255) / 256);
+  const int ll = group == 32 ? 2 : (group == 64 ? 3 : 4), row = padded_groups(K / group) * kSlots;
+  if (dt == 0) prepare_rows_kernel<0><<<grid, 256, 0, st>>>(static_cast<const uint16_t *>(x), n, K / 8, ll, copy, sums, row);
+  else if (dt == 1) prepare_rows_kernel<1><<<grid, 256, 0, st>>>(static_cast<const _Float16 *>(x), n, K / 8, ll, copy, sums, row);
+  else prepare_rows_kernel<2><<<grid, 256, 0, st>>>(static_cast<const float *>(x), n, K / 8, ll, copy, sums, row);
+  return hipGetLastError();
+}
+
+template <int DT, int BITS, bool G32, bool GLU, int MS, int NT, int WN, int KW>
+static hipError_t start_codes(const CodesArgs &a, int scale_shift, const uint32_t *tiles, int cap, int sub_log2, hipStream_t st) {
+  constexpr int NI = 32 * WN * (GLU ? 1 : NT), BM = 32 * MS;
+  constexpr size_t bufs = (size_t)2 * KW * n_parts(DT) * BM * kRow * 16 + WN * KW * NT * 32 * 48, sums = KW > 1 ? (size_t)BM * 32 * WN * NT * 4 : 0;
+  constexpr size_t most = bufs > sums ? bufs : sums, lds = most > kLdsAtLeast ? most : kLdsAtLeast;
+  static_assert(lds <= 160 * 1024, "more LDS than a CU has");
+  const int n_ntiles = (a.N + NI - 1) / NI;
+  const int mtiles = tiles ? cap << sub_log2 : (int)((a.M + BM - 1) / BM);
+  const int64_t grid = tiles ? (int64_t)((mtiles + 7) / 8) * 8 * n_ntiles : (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
+  if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
+  const auto kernel = &qmm_codes_kernel<DT, BITS, G32, GLU, MS, NT, WN, KW>;
+  if (lds > 64 * 1024)
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        e != hipSuccess)
+      return e;
+  kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, tiles, mtiles, n_ntiles, sub_log2, scale_shift);
+  return hipGetLastError();
+}
+
+// Which tile, from the number of tiles a launch of each has (256 CUs).  Measured with f16, 4-bit, groups of 64, us of the
+// whole call at (M, N, K) = (96, 4096, 4096) / (160, 4096, 4096) / (400, 4096, 4096) / (640, 2304, 2304) / (1000, 1024, 4096)
+// / (1000, 4096, 4096):
+//   32 x 64, K shared by four groups:   22.0 / 31.5 / 58.6 / 39.7 / 38.7 / 121   while there are at most two such tiles a CU
+//   64 x 128, K shared by two groups:   35.6 / 36.5 / 41.1 / 29.7 / 39.9 / 75.8  while a CU gets one at most
+//   64 x 128:                           41.5 / 42.4 / 46.7 / 31.0 / 45.6 / 66.7  (several blocks a CU overlap as K groups do)
+// (128 x 128 tiles: 65.1 / 67.0 / 70.2 / 45.9 / 69.3 / 76.0.)  f32 multiplies three times as much and holds three times
+// the rows in LDS: 32 x 64 with two groups up to 320 tiles, then 32 x 256 (1000, 4096, 4096: 147 against 164 for 64 x 128).
+template <int DT, int BITS, bool G32>
+static hipError_t start_dense(const CodesArgs &a, int scale_shift, hipStream_t st) {
+  auto tiles = [&](int rows, int cols) { return (a.M + rows - 1) / rows * ((a.N + cols - 1) / cols); };
+  if constexpr (DT == 2) {
+    if (tiles(32, 64) <= 320) return start_codes<DT, BITS, G32, false, 1, 1, 2, 2>(a, scale_shift, nullptr, 0, 0, st);
+    return start_codes<DT, BITS, G32, false, 1, 2, 4, 1>(a, scale_shift, nullptr, 0, 0, st);
+  } else {
+    if (tiles(32, 64) <= 512) return start_codes<DT, BITS, G32, false, 1, 1, 2, 4>(a, scale_shift, nullptr, 0, 0, st);
+    if (tiles(64, 128) <= 256) return start_codes<DT, BITS, G32, false, 2, 1, 4, 2>(a, scale_shift, nullptr, 0, 0, st);
+    return start_codes<DT, BITS, G32, false, 2, 1, 4, 1>(a, scale_shift, nullptr, 0, 0, st);
+  }
+}
+
+hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st) {
+  if (a.M == 0) return hipSuccess;
+  auto with_group = [&](auto d, auto b) {
+    constexpr int DT = decltype(d)::value, BITS = decltype(b)::value;
+    if (group == 32) return start_dense<DT, BITS, true>(a, 0, st);
+    return start_dense<DT, BITS, false>(a, group == 128, st);
+  };
+  auto with_bits = [&](auto d) {
+    return bits == 4 ? with_group(d, std::integral_constant<int, 4>{}) : with_group(d, std::integral_constant<int, 8>{});
+  };
+  if (dt == 0) return with_bits(std::integral_constant<int, 0>{});
+  if (dt == 1) return with_bits(std::integral_constant<int, 1>{});
+  return with_bits(std::integral_constant<int, 2>{});
+}
+
+}  // namespace mi_moe
