@@ -127,10 +127,25 @@ struct ForwardWs {
   void *disp_scratch;
   uint16_t *hh, *y, *xperm, *xnorm;
   uint16_t *gu;  // plain products only: the gate and the up product, [P, I] each
+  bool raw;             // group sizes 32 / 128: the products on raw codes (qmm_rows, qmm_codes)
+  uint32_t *raw_tiles;  // their tile lists, the paired copy of x (4-bit) and the group sums of x and h, or nullptr: all
+  int raw_cap;          // segments go through the kernel of a few rows, in as many passes as they need
+  uint16_t *raw_copy, *raw_xsums, *raw_hsums;
+  size_t bytes_raw;     // up to the end of those
   void *router_scratch;  // byte planes of x and of the router matrix (logits on the int8 matrix cores), or nullptr
   size_t bytes_min;      // without the byte planes: a workspace of this size makes the forward take the fp64 logits (same bits)
   size_t bytes;
 };
+
+// Group sizes 32 and 128: tile lists are built (for segments of more rows than one pass of the kernel of a few rows)
+// from an average of four rows per expert on; see forward_impl for what that costs and gives.  The tiled kernel takes operands below 2 GiB, in multiples of 128 values.
+bool raw_tiled_batch(const mi_moe_config &c, int64_t T) {
+  const int64_t P = T * c.top_k, most = (int64_t)1 << 31;
+  return P >= (int64_t)4 * c.n_experts && c.hidden % 128 == 0 && c.intermediate % 128 == 0 && T * c.hidden * 2 < most &&
+         P * c.intermediate * 2 < most && (int64_t)codes_sums_bytes(P, c.intermediate, c.group_size) < most &&
+         (int64_t)codes_sums_bytes(T, c.hidden, c.group_size) < most &&
+         (int64_t)c.hidden * c.intermediate * c.bits / 8 < most;
+}
 
 ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws) {
   const int64_t P = T * c.top_k;
@@ -160,8 +175,27 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws) {
   f.y = cv.take<uint16_t>((size_t)P * c.hidden);
   f.xperm = cv.take<uint16_t>(f.tiled && c.bits == 4 ? (size_t)T * c.hidden : 0);
   f.xnorm = cv.take<uint16_t>((size_t)T * c.hidden);  // rms_norm(x) of the residual variant
-  f.gu = cv.take<uint16_t>(plain_config(c) ? 2 * (size_t)P * c.intermediate : 0);
+  RowsArgs up{}, down{};  // (the extents only)
+  static const uint32_t records[1] = {};
+  up.work = down.work = records;
+  up.max_active = down.max_active = (int)(P < c.n_experts ? P : c.n_experts);
+  up.max_rows = down.max_rows = T;
+  up.N = down.K = c.intermediate;
+  up.K = down.N = c.hidden;
+  f.raw = plain_config(c) && qmm_rows_applies(up, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true) &&
+          qmm_rows_applies(down, c.group_size, c.bits, MI_MOE_DTYPE_BF16, false);
+  f.gu = cv.take<uint16_t>(plain_config(c) && !f.raw ? 2 * (size_t)P * c.intermediate : 0);
   f.bytes_min = cv.off;
+  f.raw_tiles = nullptr;
+  f.raw_cap = 0;
+  if (f.raw && raw_tiled_batch(c, T)) {
+    f.raw_cap = (int)(P / kBigTileM + (P / (kRowsMost + 1) < c.n_experts ? P / (kRowsMost + 1) : c.n_experts));
+    f.raw_tiles = cv.take<uint32_t>(tile_list_words(f.raw_cap, c.n_experts));
+    f.raw_copy = cv.take<uint16_t>(codes_copy_bytes(MI_MOE_DTYPE_BF16, c.bits, T, c.hidden) / 2);
+    f.raw_xsums = cv.take<uint16_t>(codes_sums_bytes(T, c.hidden, c.group_size) / 2);
+    f.raw_hsums = cv.take<uint16_t>(codes_sums_bytes(P, c.intermediate, c.group_size) / 2);
+  }
+  f.bytes_raw = cv.off;
   const bool i8_router = router_logits_i8_applies(T, c.hidden, c.n_experts);  // (the last region: optional, see bytes_min)
   f.router_scratch = cv.take<char>(i8_router ? router_logits_i8_bytes(T, c.hidden, c.n_experts) : 0);
   if (!i8_router) f.router_scratch = nullptr;
@@ -364,6 +398,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   ForwardWs f = carve_forward(c, T, workspace);
   if (workspace_bytes < f.bytes_min)
     return fail("forward: workspace too small (%zu bytes, need %zu)", workspace_bytes, f.bytes);
+  if (workspace_bytes < f.bytes_raw) f.raw_tiles = nullptr;
   if (workspace_bytes < f.bytes) f.router_scratch = nullptr;  // room for everything but the byte planes: fp64 logits, same bits
   int stage = 0;
 #define MI_STAGE_DONE()                                  \
@@ -372,6 +407,8 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   } while (0)
   if (ev) MI_HIP(hipEventRecord(ev[0], st));
   const bool fused_router = router_fused_applies(T, c.n_experts, c.top_k);
+  uint32_t *const tile_lists = f.tiled ? f.mtiles : f.raw_tiles;
+  const int tile_cap = f.tiled ? f.max_mtiles : f.raw_cap, tile_from = f.tiled ? f.tmr : kRowsMost + 1;
   if (norm_weight) {  // the block's input is rms_norm(x); x itself is added back in the combine
     if (!fused_router) MI_HIP(launch_rms_norm(x_in, norm_weight, eps, T, c.hidden, f.xnorm, st));
     x = f.xnorm;      // decode: written by the router kernel below
@@ -389,8 +426,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     MI_HIP(launch_router_fused(x_in, h->w.router_w, h->w.router_bias, norm_weight, eps, f.xnorm, T, c.hidden,
                                c.n_experts, c.top_k,
                                c.score_mode, f.logits, f.topk_idx, f.topk_w, h->counters, f.counts, f.offsets,
-                               f.perm, f.inv_perm, f.src_of, f.work, f.tiled ? f.mtiles : nullptr, f.max_mtiles,
-                               f.tmr, st));
+                               f.perm, f.inv_perm, f.src_of, f.work, tile_lists, tile_cap, tile_from, st));
     MI_STAGE_DONE();
     MI_STAGE_DONE();
     MI_STAGE_DONE();
@@ -419,16 +455,97 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
       MI_STAGE_DONE();
     }
     MI_HIP(launch_dispatch(f.topk_idx, P, c.n_experts, c.top_k, f.counts, f.offsets, f.perm, f.inv_perm,
-                           f.src_of, f.work, f.tiled ? f.mtiles : nullptr, f.max_mtiles, f.tmr,
-                           f.disp_scratch, st));
+                           f.src_of, f.work, tile_lists, tile_cap, tile_from, f.disp_scratch, st));
     MI_STAGE_DONE();
   }
   GroupedArgs a{}, d{};
   grouped_args(c, h->w, f, x, T, a, d);
   const int max_active = a.max_active;
   if (f.tiled && paired && !streamed_first && !pair_in_router) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));
-  if (plain_config(c)) {
-    // group sizes 32 / 128 or 2-bit codes: the plain products, one output row per sorted pair.  Row r of
+  if (f.raw) {
+    // group sizes 32 / 128: short segments on the kernel of a few rows, longer ones (where lists are built) in tiles
+    RowsArgs ra{}, rd{};
+    ra.work = f.work;
+    ra.max_active = max_active;
+    ra.max_rows = f.raw_tiles ? kRowsMost : T;
+    rd = ra;
+    ra.x = x;
+    ra.src_rows = f.src_of;
+    ra.src_in_work = true;
+    ra.w0 = h->w.gate.w; ra.s0 = h->w.gate.scales; ra.b0 = h->w.gate.biases;
+    ra.w1 = h->w.up.w; ra.s1 = h->w.up.scales; ra.b1 = h->w.up.biases;
+    ra.y = f.hh;
+    ra.N = c.intermediate; ra.K = c.hidden;
+    rd.x = f.hh;
+    rd.dst_rows = f.perm;
+    rd.w0 = h->w.down.w; rd.s0 = h->w.down.scales; rd.b0 = h->w.down.biases;
+    rd.y = f.y;
+    rd.N = c.hidden; rd.K = c.intermediate;
+    CodesArgs ca{}, cd{};
+    const bool copied = codes_copy_bytes(MI_MOE_DTYPE_BF16, c.bits, T, c.hidden) > 0;
+    ca.x = copied ? f.raw_copy : x;
+    ca.x_rows = T;
+    ca.sums = f.raw_xsums;
+    ca.src_rows = f.src_of;
+    ca.w0 = ra.w0; ca.s0 = ra.s0; ca.b0 = ra.b0;
+    ca.w1 = ra.w1; ca.s1 = ra.s1; ca.b1 = ra.b1;
+    ca.y = f.hh;
+    ca.y_paired = copied;
+    ca.N = ra.N; ca.K = ra.K;
+    cd.x = f.hh;
+    cd.x_rows = P;
+    cd.sums = f.raw_hsums;
+    cd.dst_rows = f.perm;
+    cd.w0 = rd.w0; cd.s0 = rd.s0; cd.b0 = rd.b0;
+    cd.y = f.y;
+    cd.N = rd.N; cd.K = rd.K;
+    auto tiles_up = [&](hipStream_t s) -> hipError_t {
+      if (hipError_t e = launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, s);
+          e != hipSuccess)
+        return e;
+      return launch_qmm_codes_tiles(ca, f.raw_tiles, f.raw_cap, c.n_experts, c.group_size, c.bits, true, s);
+    };
+    auto tiles_down = [&](hipStream_t s) -> hipError_t {
+      // (the sums of all rows of h: those of the short segments, which another stream may still be writing, are not read)
+      if (hipError_t e = launch_prepare_rows(f.hh, P, c.intermediate, c.group_size, MI_MOE_DTYPE_BF16, nullptr, f.raw_hsums, s);
+          e != hipSuccess)
+        return e;
+      return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.n_experts, c.group_size, c.bits, false, s);
+    };
+    if (f.raw_tiles && !ev) {
+      // The two chains share no rows.  The tiles run on a side stream beside the short segments: which of the two is the
+      // longer depends on the routing, and with even routing one of them is all but empty.  Measured, 128-expert shape,
+      // groups of 32, us of a forward at 64 / 96 / 128 / 200 / 512 tokens:
+      //   all segments through the kernel of a few rows  even 125 / 137 / 146 / 181 / 328   Zipf-1.1 183 / 256 / 324 / 458 / 1017
+      //   one chain after the other                           145 / 153 / 178 / 224 / 252            171 / 221 / 236 / 246 / 310
+      //   side by side                                        148 / 158 / 174 / 198 / 263            152 / 177 / 198 / 224 / 274
+      // (the plain kernels, which these shapes ran on before: 5630 at 512 tokens)
+      DeviceStreams &ds = *h->streams;
+      std::lock_guard<std::mutex> streams_guard(ds.lock);
+      hipStream_t s = ds.side[0];
+      MI_HIP(hipEventRecord(ds.fork, st));
+      MI_HIP(hipStreamWaitEvent(s, ds.fork, 0));
+      const bool tiles_lead = P >= (int64_t)20 * c.n_experts;  // the longer chain, as far as the host can tell, stays here
+      const hipStream_t ts = tiles_lead ? st : s, rs = tiles_lead ? s : st;
+      hipError_t e = tiles_up(ts);
+      if (e == hipSuccess) e = tiles_down(ts);
+      if (e == hipSuccess) e = launch_qmm_rows(ra, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true, rs);
+      if (e == hipSuccess) e = launch_qmm_rows(rd, c.group_size, c.bits, MI_MOE_DTYPE_BF16, false, rs);
+      // whatever happened: the caller's stream waits for what the side stream was given
+      hipError_t je = hipEventRecord(ds.join[0], s);
+      if (je == hipSuccess) je = hipStreamWaitEvent(st, ds.join[0], 0);
+      MI_HIP(e);
+      MI_HIP(je);
+    } else {
+      if (f.raw_tiles) MI_HIP(tiles_up(st));
+      MI_HIP(launch_qmm_rows(ra, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true, st));
+      MI_STAGE_DONE();
+      if (f.raw_tiles) MI_HIP(tiles_down(st));
+      MI_HIP(launch_qmm_rows(rd, c.group_size, c.bits, MI_MOE_DTYPE_BF16, false, st));
+      MI_STAGE_DONE();
+    }
+  } else if (plain_config(c)) {
+    // 2-bit codes, or rows the kernels on raw codes do not take: the plain products, one output row per sorted pair.  Row r of
     // the sorted order belongs to pair perm[r], token src_of[r], expert topk_idx[perm[r]].
     const size_t PI = (size_t)P * c.intermediate;
     MI_HIP(launch_qmm_plain(x, h->w.gate.w, h->w.gate.scales, h->w.gate.biases, f.src_of, f.topk_idx, f.perm, nullptr,
@@ -897,9 +1014,28 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
   if (M == 0) return 0;
   if (!x || !w || !scales || !biases || !y) return fail("quantized_matmul: x, w, scales, biases and y must be non-NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // From six rows on (eight with f32): the plain kernel's time grows with the rows, 3.4 us each after 7 us for one at
-  // N = K = 4096 and 4 bits (f16; 6 with 8 bits), against 19 us flat for the smallest tile (30 with f32).
-  if (codes_shape(dtype, transpose, group_size, bits, N, K) && M >= (dtype == MI_MOE_DTYPE_F32 ? 8 : 6) && M * K * 4 < (int64_t)1 << 31 && workspace &&
+  // A few rows: nothing to prepare.  Measured at 4096 x 4096, us of the kernels: 16 rows of 4-bit codes 18.3 (f16), 20.7
+  // (bf16, groups of 32), 30.1 (f32) against 19.8, 26.8, 35.7 for the tiles; of 8-bit codes 26.7, 27.4, 29.5 against
+  // 23.5, 24.8, 34.3.  One row of 4-bit codes or f32 is still the plain kernel's: 6.7 (f16 4-bit), 7.1 and 9.8 (f32)
+  // against 7.5, 9.1 and 10.8.
+  const bool one_plain = M == 1 && (bits == 4 || dtype == MI_MOE_DTYPE_F32);
+  if (codes_shape(dtype, transpose, group_size, bits, N, K) && !one_plain &&
+      M <= (bits == 4 || dtype == MI_MOE_DTYPE_F32 ? kRowsMost : 12) && aligned16(x) && aligned16(w) &&
+      aligned16(scales) && aligned16(biases)) {
+    RowsArgs a{};
+    a.x = x;
+    a.w0 = w; a.s0 = scales; a.b0 = biases;
+    a.bias = linear_bias;
+    a.y = y;
+    a.N = N;
+    a.K = K;
+    a.M = M;
+    if (qmm_rows_applies(a, group_size, bits, dtype, false)) {
+      MI_HIP(launch_qmm_rows(a, group_size, bits, dtype, false, st));
+      return 0;
+    }
+  }
+  if (codes_shape(dtype, transpose, group_size, bits, N, K) && !one_plain && M * K * 4 < (int64_t)1 << 31 && workspace &&
       workspace_bytes >= codes_bytes(M, K, group_size, bits, dtype) && aligned16(x) && aligned16(w) && aligned16(y)) {
     Carver cv(workspace);
     const size_t copy_bytes = codes_copy_bytes(dtype, bits, M, K);

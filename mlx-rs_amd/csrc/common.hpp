@@ -342,11 +342,31 @@ struct CodesArgs {
   int N, K;
   int64_t M;  // rows (dense launches)
 };
+// The product of a few rows on raw codes (qmm_rows.hip): the same types, groups and code widths, nothing prepared.
+// Rows: M dense ones (work == nullptr), or the records' segments.
+struct RowsArgs {
+  const void *x;
+  const uint32_t *src_rows, *dst_rows, *work;  // as in GroupedArgs
+  bool src_in_work;
+  int max_active;
+  int64_t max_rows;  // of a record, at most
+  const uint32_t *w0, *w1;
+  const void *s0, *b0, *s1, *b1;
+  const void *bias;  // as in CodesArgs
+  void *y;
+  int N, K;
+  int64_t M;
+};
+constexpr int kRowsMost = 16;  // rows of one pass of that kernel
+bool qmm_rows_applies(const RowsArgs &a, int group, int bits, int dt, bool glu);
+hipError_t launch_qmm_rows(const RowsArgs &a, int group, int bits, int dt, bool glu, hipStream_t st);
 size_t codes_copy_bytes(int dt, int bits, int64_t rows, int K);
 size_t codes_sums_bytes(int64_t rows, int K, int group);
 hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
                                uint16_t *sums, hipStream_t st);
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
+hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *lists, int cap256, int n_experts, int group, int bits,
+                                  bool glu, hipStream_t st);
 hipError_t launch_quantize(const float *w, int64_t rows, int64_t cols, int group, int bits,
                            uint32_t *q, void *s, void *b, int dt, hipStream_t st);
 hipError_t launch_dequantize(const uint32_t *q, const void *s, const void *b,

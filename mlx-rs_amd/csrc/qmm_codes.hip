@@ -70,14 +70,14 @@ __device__ __forceinline__ Pieces split3(float v) {
   return Pieces{hu >> 16, mu >> 16, __float_as_uint(q) >> 16};
 }
 
-// a multiply function together with the instruction mix its step is scheduled in
-template <class Weave, class F>
-struct Woven : F {
-  __device__ __forceinline__ Woven(F f) : F(f) {}
-  static __device__ __forceinline__ void weave() { Weave::weave(); }
+// a multiply function together with how it deals K values to its four multiplies (see qmm_codes_kernel)
+template <bool SPLIT, class F>
+struct Split : F {
+  static constexpr bool split = SPLIT;
+  __device__ __forceinline__ Split(F f) : F(f) {}
 };
-template <class Weave, class F>
-__device__ __forceinline__ Woven<Weave, F> with_weave(F f) { return Woven<Weave, F>(f); }
+template <bool SPLIT, class F>
+__device__ __forceinline__ Split<SPLIT, F> with_split(F f) { return Split<SPLIT, F>(f); }
 
 template <class T>
 __device__ __forceinline__ T load_elem(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf
 // DT: 0 bf16, 1 f16, 2 f32.  G32: groups of 32; otherwise a group is one or two steps (scale_shift).
 template <int DT, int BITS, bool G32, bool GLU, int MS, int NT, int WN, int KW>
 __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2, 4))) void qmm_codes_kernel(
-    CodesArgs a, const uint32_t *__restrict__ tiles, int n_mtiles, int n_ntiles, int sub_log2, int scale_shift) {
+    CodesArgs a, const uint32_t *__restrict__ lists, int n_mtiles, int n_experts, int n_ntiles, int scale_shift) {
   static_assert(!GLU || NT == 2, "a gate tile and its up tile");
   typedef typename ElemOf<DT>::type T;
   constexpr int NP = n_parts(DT);
@@ -195,12 +195,23 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
   int e = 0, rows, nt;
   int64_t row0;
-  if (tiles) {
-    const uint32_t mt_id = (uint32_t)(j / n_ntiles) * 8u + xcd;
+  if (lists) {
+    // the three lists behind each other, every tile cut into pieces of BM rows: ids in the order of the lists' capacities
+    uint32_t id = (uint32_t)(j / n_ntiles) * 8u + xcd;
     nt = j % n_ntiles;
-    if (mt_id >= tiles[0] << sub_log2) return;
-    const uint4 rec = reinterpret_cast<const uint4 *>(tiles)[1 + (mt_id >> sub_log2)];
-    const int part = (int)(mt_id & ((1u << sub_log2) - 1u)) * BM;
+    int cls = 0, pieces = kBigTileM / BM;
+    uint32_t capacity = (uint32_t)n_mtiles * pieces;
+    while (cls < 2 && id >= capacity) {
+      id -= capacity;
+      ++cls;
+      pieces /= 2;
+      capacity = (uint32_t)n_experts * pieces;
+    }
+    const uint32_t *const list = tile_list(lists, cls, n_mtiles, n_experts);
+    const uint32_t in_list = id / (uint32_t)pieces;
+    if (in_list >= list[0]) return;
+    const uint4 rec = reinterpret_cast<const uint4 *>(list)[1 + in_list];
+    const int part = (int)(id % (uint32_t)pieces) * BM;
     e = (int)rec.x;
     row0 = (int64_t)rec.y + part;
     rows = (int)rec.z - part < BM ? (int)rec.z - part : BM;
@@ -272,7 +283,10 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   // token rows of the next two are on their way into registers, the codes run two steps ahead and are unpacked one
   // step ahead.
   // window_steps, window: called ahead of every so many steps.
-  auto pass = [&](int nk, auto a_type, auto b_type, auto load_a, auto put_a, auto load_b, auto unpack, auto multiply, int window_steps, auto window) __attribute__((always_inline)) {
+  // Inside a step the sub-tiles follow each other, each with the reads of the next one's token rows ahead of its
+  // multiplies and its share of the unpacking between them; nothing moves across a sub-tile.
+  auto pass = [&](int nk, auto parts, auto a_type, auto b_type, auto load_a, auto put_a, auto load_b, auto unpack, auto begin, auto multiply, int window_steps, auto window) __attribute__((always_inline)) {
+    constexpr int P = decltype(parts)::value;
     decltype(a_type) RA[2];
     decltype(b_type) RB[2];
     auto put = [&](int buf) __attribute__((always_inline)) {
@@ -289,15 +303,27 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     load_a(clamped(k0 + 1), k0 < k1, RA[1]);
     load_b(clamped(k0 + 1), RB[1]);
     Operand op[2];
-    unpack(RB[0], op[0]);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int h = 0; h < 4; ++h) unpack(RB[0], op[0], t, h);
     put(0);
     __syncthreads();
+    u32x4_t F[2][4][P];  // the token operand of a sub-tile row, and of the next
+    auto fetch = [&](const u32x4_t *At, int m, bool split, u32x4_t (&to)[4][P]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          to[h][p] = At[p * A_SZ + (32 * m + ln) * kRow + (split ? 4 * (h >> 1) + 2 * kb + (h & 1) : 4 * kb + h)];  // the chunk multiply h takes
+    };
     int buf = 0;
     for (int kw = k0; kw < k0 + share; kw += window_steps) {
       window(kw);
       for (int kq = kw; kq < k0 + share && kq < kw + window_steps; kq += 2) {
         const u32x4_t *const At = lds + buf * BUF;
         buf ^= 1;
+        fetch(At, 0, decltype(multiply)::split, F[0]);
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
           load_b(clamped(kq + d + 2), RB[d]);
@@ -305,10 +331,26 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
             load_a(clamped(kq + 2), kq + 2 < k1, RA[0]);
             load_a(clamped(kq + 3), kq + 2 < k1, RA[1]);
           }
+          begin(kq + d, d);
           __builtin_amdgcn_sched_barrier(0);  // (the loads stay at the head of the step)
-          multiply(At + 8 * d, op[d], d, kq + d);
-          unpack(RB[d ^ 1], op[d ^ 1]);
-          decltype(multiply)::weave();
+#pragma unroll
+          for (int m = 0; m < MS; ++m)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+              if (t == 0 && m + 1 < MS) fetch(At + 8 * d, m + 1, decltype(multiply)::split, F[(d * MS + m + 1) & 1]);
+              if (t == 0 && m + 1 == MS && d == 0) fetch(At + 8, 0, decltype(multiply)::split, F[MS & 1]);
+              multiply(F[(d * MS + m) & 1], op[d], d, m, t);
+              constexpr int UNITS = 4 * NT, TILES = MS * NT;
+#pragma unroll
+              for (int u = UNITS * (m * NT + t) / TILES; u < UNITS * (m * NT + t + 1) / TILES; ++u) unpack(RB[d ^ 1], op[d ^ 1], u / 4, u % 4);
+              if (t == 0 && (m + 1 < MS || d == 0)) __builtin_amdgcn_sched_group_barrier(0x100, 4 * P, 0);
+#pragma unroll
+              for (int i = 0; i < 4 * P; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, kWeave, 0);
+              }
+              __builtin_amdgcn_sched_barrier(0);
+            }
           if (d == 1) {
             put(buf);
             __syncthreads();
@@ -336,35 +378,22 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int h = 0; h < 4; ++h) {
-          int g = ks * 8 + 2 * h + kb;
+          int g = ks * 8 + 4 * kb + h;
           g = g < G ? g : G - 1;  // (padding groups: their sums are zero)
           R.b[t][h] = load_elem<T>(br[t], s_voff[t] + g * (uint32_t)sizeof(T), 0);
           R.s[t][h] = kOffset != 0.f ? load_elem<T>(sr[t], s_voff[t] + g * (uint32_t)sizeof(T), 0) : T{};
         }
     };
-    auto unpack = [&](const StageB &R, Operand &o) __attribute__((always_inline)) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const Pieces p = split3(__builtin_fmaf(-kOffset, as_f32(R.s[t][h]), as_f32(R.b[t][h])));
-          o.v[t][h] = u32x4_t{p.h | p.h << 16, p.h | p.m << 16, p.m | p.l << 16, 0u};
-        }
+    auto unpack = [&](const StageB &R, Operand &o, int t, int h) __attribute__((always_inline)) {
+      const Pieces p = split3(__builtin_fmaf(-kOffset, as_f32(R.s[t][h]), as_f32(R.b[t][h])));
+      o.v[t][h] = u32x4_t{p.h | p.h << 16, p.h | p.m << 16, p.m | p.l << 16, 0u};
     };
-    struct Multiply {
-      static __device__ __forceinline__ void weave() {}
+    auto body = [&](const u32x4_t (&av)[4][1], const Operand &o, int, int m, int t) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < 4; ++h) tot[m][t] = mfma<0>(av[h][0], o.v[t][h], tot[m][t]);
     };
-    auto body = [&](const u32x4_t *At, const Operand &o, int, int) __attribute__((always_inline)) {
-#pragma unroll
-      for (int m = 0; m < MS; ++m)
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const u32x4_t av = At[(32 * m + ln) * kRow + 2 * h + kb];
-#pragma unroll
-          for (int t = 0; t < NT; ++t) tot[m][t] = mfma<0>(av, o.v[t][h], tot[m][t]);
-        }
-    };
-    pass(pg / 8, StageA{}, StageB{}, load_a, put_a, load_b, unpack, with_weave<Multiply>(body), 1 << 30, [](int) {});
+    pass(pg / 8, std::integral_constant<int, 1>{}, StageA{}, StageB{}, load_a, put_a, load_b, unpack, [](int, int) {},
+         with_split<false>(body), 1 << 30, [](int) {});
   }
 
   // ---- the product of the codes
@@ -391,18 +420,13 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     struct StageB {
       u32x4_t q[NT][NQ];
     };
-    f32x16_t acc[2][NS];  // the sub-tile being multiplied, and the one before it
-    float acc_s[2][NS];
+    f32x16_t acc[2];  // the group of a sub-tile being multiplied, and the one before it
+    float acc_s[2];
+    acc[1] = zero;  // (nothing is pending yet)
+    acc_s[1] = 0.f;
+    auto add_scaled = [&](int which, int tile) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      acc[1][i] = zero;  // (nothing is pending yet)
-      acc_s[1][i] = 0.f;
-    }
-    auto add_scaled = [&](int which, int m, int t) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < NS; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) tot[m][t][r] = __builtin_fmaf(acc_s[which][i], acc[which][i][r], tot[m][t][r]);
+      for (int r = 0; r < 16; ++r) tot[tile / NT][tile % NT][r] = __builtin_fmaf(acc_s[which], acc[which][r], tot[tile / NT][tile % NT][r]);
     };
     auto load_a = [&](int ks, bool real, StageA &R) __attribute__((always_inline)) {
 #pragma unroll
@@ -419,11 +443,9 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
           R.q[t][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[t], w_voff[t], ks * (kStep * BITS / 8) + 32 * h, 0);
       }
     };
-    auto unpack = [&](const StageB &cur, Operand &o) __attribute__((always_inline)) {
-      StageB R = cur;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        if constexpr (BITS == 4 && G32) {
+    auto unpack = [&](StageB &R, Operand &o, int t, int h) __attribute__((always_inline)) {
+      if constexpr (BITS == 4 && G32) {
+        if (h == 0) {
 #pragma unroll
           for (int w = 0; w < 2; ++w) {
             const auto r = __builtin_amdgcn_permlane32_swap(R.q[t][0][w], R.q[t][0][w + 2], false, false);
@@ -431,8 +453,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
             R.q[t][0][w + 2] = r[1];
           }
         }
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
+      }
           if constexpr (BITS == 4 && DT != 2) {
             const uint32_t w = R.q[t][0][h];
 #pragma unroll
@@ -467,19 +488,6 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
               o.v[t][h][i] = __builtin_amdgcn_perm(__float_as_uint((float)c1), __float_as_uint((float)c0), 0x07060302u);
             }
           }
-        }
-      }
-    };
-    struct Multiply {  // the step's instruction mix: matrix, vector and LDS instructions in turn
-      static __device__ __forceinline__ void weave() {
-        __builtin_amdgcn_sched_group_barrier(0x100, 4 * NP, 0);
-#pragma unroll
-        for (int i = 0; i < MS * NT * NP * 4; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, kWeave, 0);
-          if (i % NT == 0 && i < (MS - 1) * NT * NP * 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-      }
     };
     // The scales of this wave's rows pass through LDS a window at a time: a lane fetches 16 bytes of its row (half kb of
     // the window) one window ahead, and reads one value per group back.  One 2-byte load per group from a row each
@@ -510,45 +518,31 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    auto body = [&](const u32x4_t *At, const Operand &o, int d, int ks) __attribute__((always_inline)) {
-      float step_s[NT][NS];
+    float step_s[2][NT][NS];
+    auto begin = [&](int ks, int d) __attribute__((always_inline)) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < NS; ++i)
-          step_s[t][i] = as_f32(*reinterpret_cast<const T *>(s_at[t] + ((G32 ? 2 * ks + i : ks >> scale_shift) - gw) * (int)sizeof(T)));
+          step_s[d][t][i] = as_f32(*reinterpret_cast<const T *>(s_at[t] + ((G32 ? 2 * ks + i : ks >> scale_shift) - gw) * (int)sizeof(T)));
+    };
+    auto body = [&](const u32x4_t (&av)[4][NP], const Operand &o, int d, int m, int t) __attribute__((always_inline)) {
+      const int tile = m * NT + t;
 #pragma unroll
-      for (int m = 0; m < MS; ++m) {
-        u32x4_t av[4][NP];
+      for (int i = 0; i < NS; ++i) {
+        const int which = ((d * MS * NT + tile) * NS + i) & 1;
 #pragma unroll
-        for (int h = 0; h < 4; ++h)
+        for (int h = 4 / NS * i; h < 4 / NS * (i + 1); ++h)
 #pragma unroll
-          for (int p = 0; p < NP; ++p) {
-            const int c = SPLIT ? 4 * (h >> 1) + 2 * kb + (h & 1) : 4 * kb + h;  // the chunk of K values multiply h takes
-            av[h][p] = At[p * A_SZ + (32 * m + ln) * kRow + c];
-          }
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const int which = (d * MS * NT + m * NT + t) & 1;
-#pragma unroll
-          for (int h = 0; h < 4; ++h) {
-            const int i = G32 ? h >> 1 : 0;
-#pragma unroll
-            for (int p = 0; p < NP; ++p) {
-              const bool first = p == 0 && (G32 ? (h & 1) == 0 : h == 0);
-              acc[which][i] = mfma<DT>(av[h][p], o.v[t][h], first ? zero : acc[which][i]);
-            }
-          }
-#pragma unroll
-          for (int i = 0; i < NS; ++i) acc_s[which][i] = step_s[t][i];
-          const int before = m * NT + t > 0 ? m * NT + t - 1 : MS * NT - 1;
-          add_scaled(which ^ 1, before / NT, before % NT);
-        }
+          for (int p = 0; p < NP; ++p)
+            acc[which] = mfma<DT>(av[h][p], o.v[t][h], p == 0 && h == 4 / NS * i ? zero : acc[which]);
+        acc_s[which] = step_s[d][t][i];
+        add_scaled(which ^ 1, i > 0 ? tile : tile > 0 ? tile - 1 : MS * NT - 1);
       }
     };
-    pass(K / kStep, StageA{}, StageB{}, load_a, put_a, load_b, unpack, with_weave<Multiply>(body),
+    pass(K / kStep, std::integral_constant<int, NP>{}, StageA{}, StageB{}, load_a, put_a, load_b, unpack, begin, with_split<SPLIT>(body),
          (win >> (G32 ? 1 : 0)) << scale_shift, window);
-    add_scaled(1, MS - 1, NT - 1);  // an even number of steps ends in accumulator 1
+    add_scaled(1, MS * NT - 1);  // an even number of steps ends in accumulator 1
   }
 
   if constexpr (KW > 1) {  // (the passes end in a barrier: LDS is free)
@@ -659,21 +653,22 @@ hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, in
 }
 
 template <int DT, int BITS, bool G32, bool GLU, int MS, int NT, int WN, int KW>
-static hipError_t start_codes(const CodesArgs &a, int scale_shift, const uint32_t *tiles, int cap, int sub_log2, hipStream_t st) {
+static hipError_t start_codes(const CodesArgs &a, int scale_shift, const uint32_t *lists, int cap256, int n_experts, hipStream_t st) {
   constexpr int NI = 32 * WN * (GLU ? 1 : NT), BM = 32 * MS;
   constexpr size_t bufs = (size_t)2 * KW * n_parts(DT) * BM * kRow * 16 + WN * KW * NT * 32 * 48, sums = KW > 1 ? (size_t)BM * 32 * WN * NT * 4 : 0;
   constexpr size_t most = bufs > sums ? bufs : sums, lds = most > kLdsAtLeast ? most : kLdsAtLeast;
   static_assert(lds <= 160 * 1024, "more LDS than a CU has");
   const int n_ntiles = (a.N + NI - 1) / NI;
-  const int mtiles = tiles ? cap << sub_log2 : (int)((a.M + BM - 1) / BM);
-  const int64_t grid = tiles ? (int64_t)((mtiles + 7) / 8) * 8 * n_ntiles : (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
+  const int mtiles = lists ? cap256 : (int)((a.M + BM - 1) / BM);
+  const int64_t pieces = (int64_t)cap256 * (256 / BM) + (int64_t)n_experts * (128 / BM + 64 / BM);
+  const int64_t grid = lists ? (pieces + 7) / 8 * 8 * n_ntiles : (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
   if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
   const auto kernel = &qmm_codes_kernel<DT, BITS, G32, GLU, MS, NT, WN, KW>;
   if (lds > 64 * 1024)
     if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         e != hipSuccess)
       return e;
-  kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, tiles, mtiles, n_ntiles, sub_log2, scale_shift);
+  kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, lists, mtiles, n_experts, n_ntiles, scale_shift);
   return hipGetLastError();
 }
 
@@ -696,6 +691,22 @@ static hipError_t start_dense(const CodesArgs &a, int scale_shift, hipStream_t s
     if (tiles(64, 128) <= 256) return start_codes<DT, BITS, G32, false, 2, 1, 4, 2>(a, scale_shift, nullptr, 0, 0, st);
     return start_codes<DT, BITS, G32, false, 2, 1, 4, 1>(a, scale_shift, nullptr, 0, 0, st);
   }
+}
+
+// The M-tile lists of a grouped product (see tile_list) in one launch, in blocks of 64 rows x 128 columns.  Measured on
+// the 128-expert shape with groups of 32, us of a forward at 200 / 512 tokens, even and Zipf-1.1 routing: three launches,
+// a list each, 225, 314 / 260, 373; one launch 224, 246 / 252, 310; one launch with gate/up blocks of 32 rows 217, 242 /
+// 332, 335; with gate/up blocks of 32 x 64 and K shared by two groups 288, 347 / 628, 524.
+hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *lists, int cap256, int n_experts, int group, int bits,
+                                  bool glu, hipStream_t st) {
+  auto run = [&](auto b, auto g32) {
+    constexpr int BITS = decltype(b)::value;
+    constexpr bool G32 = decltype(g32)::value;
+    if (glu) return start_codes<0, BITS, G32, true, 2, 2, 4, 1>(a, group == 128, lists, cap256, n_experts, st);
+    return start_codes<0, BITS, G32, false, 2, 1, 4, 1>(a, group == 128, lists, cap256, n_experts, st);
+  };
+  auto with_group = [&](auto b) { return group == 32 ? run(b, std::true_type{}) : run(b, std::false_type{}); };
+  return bits == 4 ? with_group(std::integral_constant<int, 4>{}) : with_group(std::integral_constant<int, 8>{});
 }
 
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st) {

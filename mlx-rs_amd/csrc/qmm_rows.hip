@@ -1,0 +1,473 @@
+// Quantized products of a few rows (a decode batch's linear layer, short expert segments) for everything the bfloat16 /
+// group-64 streaming kernel does not take: activations in bfloat16, float16 or float32, groups of 32, 64 or 128.
+//
+// Contract: mlx_quantized_matmul / mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:91-122,160-230);
+// with GLU also nn::silu and multiply (nn/activation.rs:142-144,876-880).
+//
+// Arithmetic as in the tiled product on raw codes (qmm_codes.hip): sum_c x_c (s q_c + b) = s sum_c x_c q_c + b sum_c x_c
+// per group, codes unrounded on the matrix cores, fp32 sums.  Here the bias term is fp32 vector work: a tile is 16
+// tokens by 16 weight rows (v_mfma_f32_16x16x32), so it is four fma a lane and group.
+#include <type_traits>
+
+#include "common.hpp"
+
+namespace mi_moe {
+
+namespace {
+
+constexpr int kTokens = 16;  // token slots of a tile
+constexpr int kRing = 4;     // 16-byte code loads in flight per lane and matrix (8: no change at any size)
+
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
+
+template <int DT> struct ElemOf;
+template <> struct ElemOf<0> { typedef uint16_t type; };
+template <> struct ElemOf<1> { typedef _Float16 type; };
+template <> struct ElemOf<2> { typedef float type; };
+
+__device__ __forceinline__ float as_f32(uint16_t v) { return bf16_to_f32(v); }
+__device__ __forceinline__ float as_f32(_Float16 v) { return (float)v; }
+__device__ __forceinline__ float as_f32(float v) { return v; }
+template <class T> __device__ __forceinline__ T rounded(float v) { return (T)v; }
+template <> __device__ __forceinline__ uint16_t rounded<uint16_t>(float v) { return (uint16_t)(cvt_pk_bf16(v, 0.f) & 0xffffu); }
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void *base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+template <int DT>
+__device__ __forceinline__ f32x4_t mfma(u32x4_t a, u32x4_t b, f32x4_t c) {
+  if constexpr (DT == 1)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ uint32_t f16_minus_1024(uint32_t v) {  // two halves 1024 + q -> q: exact
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) - half2_t{(_Float16)1024, (_Float16)1024});
+}
+
+constexpr int n_parts(int dt) { return dt == 2 ? 3 : 1; }  // f32 rows: three bf16 pieces (exact), as in qmm_codes.hip
+
+// LDS of a launch: token rows of sk values (tt of them, NP pieces each), 64 zero bytes, the sums of x over each group and
+// token slot, the (scale, bias) pairs of the block's weight rows, and the partial sums of a shared K.
+struct RowsLds {
+  int x_stride, zeros, sums, pairs, pair_row, parts, bytes;
+  __host__ __device__ RowsLds(int dt, int group, int nm, int kw, int K, int sk, int tt) {
+    const int np = n_parts(dt), elem = dt == 2 ? 4 : 2, nw = 4 / kw;
+    x_stride = 2 * np * sk + 16;
+    zeros = tt * x_stride;
+    sums = zeros + 64;
+    pairs = sums + sk / group * kTokens * 4;
+    pair_row = (K / group) * 2 * elem + 4;  // (an odd number of words: 16 rows read one group each without a conflict)
+    parts = pairs + ((nw * nm * 16 * pair_row + 15) & ~15);
+    bytes = parts + (kw > 1 ? kw * nw * nm * 64 * 16 : 0);
+  }
+};
+
+}  // namespace
+
+// One block: 16 * 4 / KW weight rows (GLU: of both matrices) of one expert times up to 16 token rows a pass; KW waves
+// share the K of a row tile, chunk by chunk.  A lane (weight row l % 16, quarter l / 16) loads 16 bytes: 32 4-bit codes or
+// 16 8-bit codes.  A multiply takes 32 K values, eight a lane, and must stay inside one group:
+//   4-bit: the four quarters of a row hold 32 consecutive codes each; four lane swaps transpose words against quarters,
+//   so that multiply s takes codes 32 s .. 32 s + 31;
+//   8-bit: multiply t takes the t-th half of every quarter (groups >= 64), or after two swaps 32 consecutive codes.
+// What bounds it: the bytes of the weights and, for one row of a small matrix, the latency of its few dependent steps.
+// Measured, 4096 x 4096, us of the kernel at 1 / 4 / 8 / 16 rows (the plain kernel, a wave per output element: f16 4-bit
+// 6.7 / 17.5 / 30.2 / 55.6, f32 8-bit 9.8 / 23.1 / 41.2 / 77.3): f16 4-bit 7.5 / 9.8 / 13.0 / 18.3, bf16 groups of 32
+// 8.5 / 10.9 / 14.4 / 20.7, f32 8-bit 10.8 / 14.9 / 20.5 / 29.5.  Every block stages all rows: that is what grows.
+template <int DT, int BITS, int GROUP, bool GLU, int KW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void qmm_rows_kernel(RowsArgs a, int tt, int sk) {
+  typedef typename ElemOf<DT>::type T;
+  constexpr int NP = n_parts(DT);
+  constexpr int NM = GLU ? 2 : 1;
+  constexpr int NW = 4 / KW;
+  constexpr int CH = BITS == 4 ? 128 : 64;     // codes per chunk and row
+  constexpr int MUL = CH / 32;                 // multiplies per chunk
+  constexpr float kOffset = BITS == 4 && DT == 0 ? 128.0f : 0.0f;
+  constexpr bool PAIRED = BITS == 4 && DT != 2;  // token rows as 8-blocks (0,4)(1,5)(2,6)(3,7), the order of the unpacking
+
+  int e = 0, cnt = (int)a.M;
+  int64_t r0 = 0;
+  bool inline_src = false;
+  if (a.work) {
+    const uint4 rec = reinterpret_cast<const uint4 *>(a.work)[(size_t)blockIdx.y * 4];
+    e = (int)rec.x;
+    r0 = rec.y;
+    cnt = (int)rec.z;
+    inline_src = a.src_in_work && rec.w != 0u;
+    if (cnt == 0) return;
+  }
+  const int lane = lane_id(), tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wk = wave % KW, wn = wave / KW;
+  const int c = lane & 15, kb = lane >> 4;
+  const int N = a.N, K = a.K;
+  const int n0 = (blockIdx.x * NW + wn) * 16;
+  const int G = K / GROUP, row_bytes = K * BITS / 8, nchunks = K / CH;
+  const int64_t ebase = (int64_t)e * N;
+
+  extern __shared__ __align__(16) unsigned char lds[];
+  const RowsLds L(DT, GROUP, NM, KW, K, sk, tt);
+  float *const sums = reinterpret_cast<float *>(lds + L.sums);
+
+  __amdgpu_buffer_rsrc_t wr[NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) wr[m] = rsrc_of((m ? a.w1 : a.w0) + ebase * (row_bytes / 4), (uint32_t)N * row_bytes);
+  const uint32_t w_voff = (uint32_t)(n0 + c) * row_bytes + kb * 16;  // rows >= N read zeros
+
+  struct Codes {
+    u32x4_t q[NM];
+  };
+  Codes ring[kRing];
+  auto issue = [&](int j, Codes &R) __attribute__((always_inline)) {  // the wave's j-th chunk; unconditional (clamped)
+    int ch = wk + KW * j;
+    ch = ch < nchunks ? ch : nchunks - 1;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) R.q[m] = __builtin_amdgcn_raw_buffer_load_b128(wr[m], w_voff, ch * 64, 0);
+  };
+#pragma unroll
+  for (int d = 0; d < kRing; ++d) issue(d, ring[d]);
+
+  // (scale, bias) pairs of the block's rows, one LDS read per group and row later on.  The 16 rows of a tile are 16 G
+  // consecutive values of each tensor, 16-byte aligned.
+  {
+    constexpr int PV = 16 / (int)sizeof(T);
+    const int per_tile = 16 * G / PV, total = NW * NM * per_tile;
+    for (int p = tid; p < total; p += 256) {
+      const int tile = p / per_tile, q = p - tile * per_tile;  // tile = wn * NM + m
+      const int m = tile % NM, row0 = (blockIdx.x * NW + tile / NM) * 16;
+      const __amdgpu_buffer_rsrc_t sr = rsrc_of(static_cast<const T *>(m ? a.s1 : a.s0) + ebase * G, ((uint32_t)N * G * sizeof(T) + 3u) & ~3u);
+      const __amdgpu_buffer_rsrc_t br = rsrc_of(static_cast<const T *>(m ? a.b1 : a.b0) + ebase * G, ((uint32_t)N * G * sizeof(T) + 3u) & ~3u);
+      const uint32_t off = ((uint32_t)row0 * G + q * PV) * sizeof(T);
+      const u32x4_t sv = __builtin_amdgcn_raw_buffer_load_b128(sr, off, 0, 0), bv = __builtin_amdgcn_raw_buffer_load_b128(br, off, 0, 0);
+      int row = q * PV / G, g = q * PV - row * G;
+      unsigned char *to = lds + L.pairs + (tile * 16 + row) * L.pair_row + g * 2 * (int)sizeof(T);
+#pragma unroll
+      for (int i = 0; i < PV; ++i) {
+        if constexpr (sizeof(T) == 4) {
+          reinterpret_cast<uint32_t *>(to)[0] = sv[i];
+          reinterpret_cast<uint32_t *>(to)[1] = bv[i];
+        } else {
+          *reinterpret_cast<uint32_t *>(to) = (i & 1) ? __builtin_amdgcn_perm(bv[i >> 1], sv[i >> 1], 0x07060302u)
+                                                      : __builtin_amdgcn_perm(bv[i >> 1], sv[i >> 1], 0x05040100u);
+        }
+        to += 2 * sizeof(T);
+        if (++g == G) {
+          g = 0;
+          to += 4;
+        }
+      }
+    }
+  }
+  for (int i = tid; i < 4; i += 256) *reinterpret_cast<uint4 *>(lds + L.zeros + 16 * i) = make_uint4(0, 0, 0, 0);
+  const unsigned char *const my_pairs = lds + L.pairs + (wn * NM * 16 + c) * L.pair_row;
+
+  for (int t0 = 0; t0 < cnt; t0 += tt) {
+    const int nt = cnt - t0 < tt ? cnt - t0 : tt;
+    const bool on = c < nt;
+    const unsigned char *const xl = on ? lds + c * L.x_stride : lds + L.zeros;
+    const int x_step = on ? 1 : 0;
+    f32x4_t tot[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) tot[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (t0 > 0)
+#pragma unroll
+      for (int d = 0; d < kRing; ++d) issue(d, ring[d]);
+
+    for (int s0 = 0; s0 < K; s0 += sk) {
+      const int sl = K - s0 < sk ? K - s0 : sk;
+      if (t0 > 0 || s0 > 0) __syncthreads();  // every wave is done with the previous slab
+      // ---- token rows of the slab, eight values a thread, with the sums of their groups
+      const int per_row = sl / 8;
+      int row = tid / per_row, piece = tid - row * per_row;
+      while (row < nt) {
+        const int64_t r = r0 + t0 + row;
+        int64_t src = r;
+        if (inline_src && t0 + row < 12) src = a.work[(size_t)blockIdx.y * 16 + 4 + t0 + row];
+        else if (a.src_rows) src = a.src_rows[r];
+        const T *const xr = static_cast<const T *>(a.x) + src * K + s0 + piece * 8;
+        unsigned char *const to = lds + row * L.x_stride + piece * 16;
+        float v[8];
+        if constexpr (DT == 2) {
+          const float4 lo = reinterpret_cast<const float4 *>(xr)[0], hi = reinterpret_cast<const float4 *>(xr)[1];
+          v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+          uint32_t h[4], m[4], l[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            uint32_t p[2][3];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {  // truncated pieces: exact, nothing overflows
+              const float f = v[2 * j + i];
+              p[i][0] = __float_as_uint(f) & 0xffff0000u;
+              const float f1 = f - __uint_as_float(p[i][0]);
+              p[i][1] = __float_as_uint(f1) & 0xffff0000u;
+              p[i][2] = __float_as_uint(f1 - __uint_as_float(p[i][1]));
+            }
+            h[j] = p[0][0] >> 16 | p[1][0];
+            m[j] = p[0][1] >> 16 | p[1][1];
+            l[j] = p[0][2] >> 16 | (p[1][2] & 0xffff0000u);
+          }
+          *reinterpret_cast<uint4 *>(to) = make_uint4(h[0], h[1], h[2], h[3]);
+          *reinterpret_cast<uint4 *>(to + 2 * sk) = make_uint4(m[0], m[1], m[2], m[3]);
+          *reinterpret_cast<uint4 *>(to + 4 * sk) = make_uint4(l[0], l[1], l[2], l[3]);
+        } else {
+          const uint4 w = *reinterpret_cast<const uint4 *>(xr);
+          const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if constexpr (DT == 0) {
+              v[2 * j] = bf16lo_to_f32(u[j]);
+              v[2 * j + 1] = bf16hi_to_f32(u[j]);
+            } else {
+              const half2_t hh = __builtin_bit_cast(half2_t, u[j]);
+              v[2 * j] = (float)hh.x;
+              v[2 * j + 1] = (float)hh.y;
+            }
+          }
+          uint4 p = w;
+          if constexpr (PAIRED) {
+            p.x = (w.x & 0xffffu) | (w.z << 16);
+            p.y = (w.x >> 16) | (w.z & 0xffff0000u);
+            p.z = (w.y & 0xffffu) | (w.w << 16);
+            p.w = (w.y >> 16) | (w.w & 0xffff0000u);
+          }
+          *reinterpret_cast<uint4 *>(to) = p;
+        }
+        float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+        sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
+        sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
+        if constexpr (GROUP >= 64) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
+        if constexpr (GROUP == 128) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
+        if (piece % (GROUP / 8) == 0) sums[piece / (GROUP / 8) * kTokens + row] = sum;
+        piece += 256;
+        while (piece >= per_row) {
+          piece -= per_row;
+          ++row;
+        }
+      }
+      __syncthreads();
+
+      // ---- the wave's chunks of the slab.  A slab is a whole number of kRing chunks a wave (or the last one): a chunk
+      // keeps its slot of the ring.
+      const int j1 = ((s0 + sl) / CH - wk + KW - 1) / KW;
+      for (int jb = s0 / (CH * KW); jb < j1; jb += kRing) {
+#pragma unroll
+        for (int d = 0; d < kRing; ++d) {
+          const int j = jb + d;
+          if (j < j1) {
+            const int ch = wk + KW * j, ch_slab = ch - s0 / CH;
+            f32x4_t acc[NM];
+            u32x4_t q[NM];
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+              q[m] = ring[d].q[m];
+              if constexpr (BITS == 4) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                  const auto r = __builtin_amdgcn_permlane32_swap(q[m][i], q[m][i + 2], false, false);
+                  q[m][i] = r[0];
+                  q[m][i + 2] = r[1];
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i += 2) {
+                  const auto r = __builtin_amdgcn_permlane16_swap(q[m][i], q[m][i + 1], false, false);
+                  q[m][i] = r[0];
+                  q[m][i + 1] = r[1];
+                }
+              } else if constexpr (GROUP == 32) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                  const auto r = __builtin_amdgcn_permlane32_swap(q[m][i], q[m][i + 2], false, false);
+                  q[m][i] = r[0];
+                  q[m][i + 2] = r[1];
+                }
+              }
+            }
+            issue(j + kRing, ring[d]);
+#pragma unroll
+            for (int s = 0; s < MUL; ++s) {
+              // the eight K values of this lane in multiply s
+              const int k = BITS == 4 ? 32 * s + 8 * kb : (GROUP == 32 ? 32 * s + 16 * (kb & 1) + 8 * (kb >> 1) : 16 * kb + 8 * s);
+              const bool first = GROUP == 32 || (GROUP == 64 ? (BITS == 4 ? s % 2 == 0 : s == 0) : s == 0);
+              const bool last = GROUP == 32 || (GROUP == 64 ? (BITS == 4 ? s % 2 == 1 : s == 1) : s == MUL - 1);
+              u32x4_t av[NP];
+#pragma unroll
+              for (int p = 0; p < NP; ++p)
+                av[p] = *reinterpret_cast<const u32x4_t *>(xl + x_step * ((ch_slab * CH + k) * 2 + p * 2 * sk));
+#pragma unroll
+              for (int m = 0; m < NM; ++m) {
+                u32x4_t bv;
+                if constexpr (PAIRED) {
+                  const uint32_t w = q[m][s];
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) {
+                    const uint32_t o = __builtin_amdgcn_bitop3_b32(w >> (4 * i), 0x000f000fu, DT == 0 ? 0x43004300u : 0x64006400u, 0xEA);  // (a & b) | c
+                    bv[i] = DT == 0 ? o : f16_minus_1024(o);
+                  }
+                } else if constexpr (DT == 1) {
+#pragma unroll
+                  for (int i = 0; i < 4; ++i)
+                    bv[i] = f16_minus_1024(__builtin_amdgcn_perm(0x64646464u, q[m][2 * s + (i >> 1)], (i & 1) ? 0x07030702u : 0x07010700u));
+                } else {
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) {
+                    uint32_t c0, c1;
+                    if constexpr (BITS == 4) {
+                      c0 = ((q[m][s] & 0x0f0f0f0fu) >> (8 * i)) & 0xffu;
+                      c1 = (((q[m][s] >> 4) & 0x0f0f0f0fu) >> (8 * i)) & 0xffu;
+                    } else {
+                      const uint32_t w = q[m][2 * s + (i >> 1)];
+                      c0 = (w >> (16 * (i & 1))) & 0xffu;
+                      c1 = (w >> (16 * (i & 1) + 8)) & 0xffu;
+                    }
+                    bv[i] = __builtin_amdgcn_perm(__float_as_uint((float)c1), __float_as_uint((float)c0), 0x07060302u);
+                  }
+                }
+#pragma unroll
+                for (int p = 0; p < NP; ++p) acc[m] = mfma<DT>(av[p], bv, first && p == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[m]);
+              }
+              if (last || (GROUP == 128 && BITS == 8 && s == MUL - 1)) {  // (8-bit groups of 128: half a group, same scale)
+                const int gs = GROUP == 128 && BITS == 8 ? ch : (ch * CH + 32 * s) / GROUP;
+                const int g = GROUP == 128 && BITS == 8 ? ch >> 1 : gs;
+                const int g_slab = g - s0 / GROUP;
+                const float4 xs = *reinterpret_cast<const float4 *>(sums + g_slab * kTokens + 4 * kb);
+                const bool with_bias = !(GROUP == 128 && BITS == 8) || (ch & 1) == 0;  // (once per group)
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                  float sc, bi;
+                  if constexpr (sizeof(T) == 4) {
+                    const float *const p = reinterpret_cast<const float *>(my_pairs + m * 16 * L.pair_row + g * 8);
+                    sc = p[0];
+                    bi = p[1];
+                  } else {
+                    const uint32_t p = *reinterpret_cast<const uint32_t *>(my_pairs + m * 16 * L.pair_row + g * 4);
+                    sc = as_f32(__builtin_bit_cast(T, (uint16_t)(p & 0xffffu)));
+                    bi = as_f32(__builtin_bit_cast(T, (uint16_t)(p >> 16)));
+                  }
+                  if constexpr (kOffset != 0.f) bi = __builtin_fmaf(-kOffset, sc, bi);
+                  if (!with_bias) bi = 0.f;
+                  tot[m][0] = __builtin_fmaf(sc, acc[m][0], __builtin_fmaf(bi, xs.x, tot[m][0]));
+                  tot[m][1] = __builtin_fmaf(sc, acc[m][1], __builtin_fmaf(bi, xs.y, tot[m][1]));
+                  tot[m][2] = __builtin_fmaf(sc, acc[m][2], __builtin_fmaf(bi, xs.z, tot[m][2]));
+                  tot[m][3] = __builtin_fmaf(sc, acc[m][3], __builtin_fmaf(bi, xs.w, tot[m][3]));
+                }
+              }
+            }
+          }
+        }
+      }
+    }
+
+    // ---- the K groups' sums, added in order, and the results: lane (c, kb) holds tokens 4 kb .. 4 kb + 3 of column c
+    if constexpr (KW > 1) {
+      float4 *const red = reinterpret_cast<float4 *>(lds + L.parts);
+#pragma unroll
+      for (int m = 0; m < NM; ++m) red[((wk * NW + wn) * NM + m) * 64 + lane] = make_float4(tot[m][0], tot[m][1], tot[m][2], tot[m][3]);
+      __syncthreads();
+      if (wk == 0)
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+          for (int w = 1; w < KW; ++w) {
+            const float4 v = red[((w * NW + wn) * NM + m) * 64 + lane];
+            tot[m][0] += v.x;
+            tot[m][1] += v.y;
+            tot[m][2] += v.z;
+            tot[m][3] += v.w;
+          }
+    }
+    if (wk == 0 && n0 + c < N) {
+      const float lb = a.bias ? as_f32(static_cast<const T *>(a.bias)[n0 + c]) : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int slot = 4 * kb + r;
+        if (slot < nt) {
+          const int64_t rr = r0 + t0 + slot;
+          const int64_t dst = a.dst_rows ? (int64_t)a.dst_rows[rr] : rr;
+          float v = tot[0][r];
+          if constexpr (GLU) v = v / (1.0f + __expf(-v)) * tot[1][r];
+          T o = rounded<T>(v);
+          if (a.bias) o = rounded<T>(as_f32(o) + lb);
+          static_cast<T *>(a.y)[dst * N + n0 + c] = o;
+        }
+      }
+    }
+  }
+}
+
+template <int DT, int BITS, int GROUP, bool GLU, int KW>
+static hipError_t start_rows(const RowsArgs &a, int sk, int tt, hipStream_t st) {
+  const RowsLds L(DT, GROUP, GLU ? 2 : 1, KW, a.K, sk, tt);
+  const auto kernel = &qmm_rows_kernel<DT, BITS, GROUP, GLU, KW>;
+  if (L.bytes > 160 * 1024) return hipErrorInvalidConfiguration;
+  if (L.bytes > 64 * 1024)
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, L.bytes);
+        e != hipSuccess)
+      return e;
+  const dim3 grid((unsigned)((a.N + 16 * (4 / KW) - 1) / (16 * (4 / KW))), (unsigned)(a.work ? a.max_active : 1));
+  kernel<<<grid, 256, (size_t)L.bytes, st>>>(a, tt, sk);
+  return hipGetLastError();
+}
+
+// How the launch is cut: K values of the token rows in LDS at a time (the whole row, or slabs that are a whole number of
+// ring turns for every wave), token rows a pass, waves that share a row tile's K.
+struct RowsCut {
+  int kw, sk, tt;
+};
+static RowsCut cut_rows(const RowsArgs &a, int group, int bits, int dt, bool glu) {
+  const int ch = bits == 4 ? 128 : 64, nm = glu ? 2 : 1;
+  const int64_t longest = a.work ? a.max_rows : a.M;
+  const int tt = (int)(longest < kTokens ? longest : kTokens);
+  const int64_t tiles = (int64_t)((a.N + 15) / 16) * (a.work ? a.max_active : 1);
+  int kw = tiles < 1024 ? 4 : (tiles < 2048 ? 2 : 1);
+  for (;; kw /= 2) {
+    const int unit = ch * kw * kRing;  // a slab: a multiple of this
+    auto bytes = [&](int sk) { return RowsLds(dt, group, nm, kw, a.K, sk, tt).bytes; };
+    int sk = a.K;
+    if (bytes(sk) > 64 * 1024) {  // (two blocks a CU at least)
+      sk = a.K / unit * unit;
+      while (sk > unit && bytes(sk) > 64 * 1024) sk -= unit;
+      if (sk < unit) sk = a.K;
+    }
+    if (bytes(sk) <= 150 * 1024) return RowsCut{kw, sk, tt};
+    if (kw == 1) return RowsCut{0, 0, 0};  // does not fit
+  }
+}
+
+bool qmm_rows_applies(const RowsArgs &a, int group, int bits, int dt, bool glu) {
+  return bits != 2 && a.K % (bits == 4 ? 128 : 64) == 0 && a.K % group == 0 && (int64_t)a.N * a.K < (int64_t)1 << 31 &&
+         cut_rows(a, group, bits, dt, glu).kw > 0;
+}
+
+hipError_t launch_qmm_rows(const RowsArgs &a, int group, int bits, int dt, bool glu, hipStream_t st) {
+  const RowsCut cut = cut_rows(a, group, bits, dt, glu);
+  if (cut.kw == 0) return hipErrorInvalidConfiguration;
+  auto with_kw = [&](auto d, auto b, auto g, auto gl) {
+    constexpr int DT = decltype(d)::value, BITS = decltype(b)::value, GROUP = decltype(g)::value;
+    constexpr bool GLU = decltype(gl)::value;
+    if (cut.kw == 4) return start_rows<DT, BITS, GROUP, GLU, 4>(a, cut.sk, cut.tt, st);
+    if (cut.kw == 2) return start_rows<DT, BITS, GROUP, GLU, 2>(a, cut.sk, cut.tt, st);
+    return start_rows<DT, BITS, GROUP, GLU, 1>(a, cut.sk, cut.tt, st);
+  };
+  auto with_glu = [&](auto d, auto b, auto g) {
+    if constexpr (decltype(d)::value == 0)
+      if (glu) return with_kw(d, b, g, std::true_type{});
+    return with_kw(d, b, g, std::false_type{});
+  };
+  auto with_group = [&](auto d, auto b) {
+    if (group == 32) return with_glu(d, b, std::integral_constant<int, 32>{});
+    if (group == 64) return with_glu(d, b, std::integral_constant<int, 64>{});
+    return with_glu(d, b, std::integral_constant<int, 128>{});
+  };
+  auto with_bits = [&](auto d) {
+    return bits == 4 ? with_group(d, std::integral_constant<int, 4>{}) : with_group(d, std::integral_constant<int, 8>{});
+  };
+  if (glu && dt != 0) return hipErrorInvalidValue;
+  if (dt == 0) return with_bits(std::integral_constant<int, 0>{});
+  if (dt == 1) return with_bits(std::integral_constant<int, 1>{});
+  return with_bits(std::integral_constant<int, 2>{});
+}
+
+}  // namespace mi_moe

@@ -58,3 +58,45 @@ def test_large_float32_values_survive_the_split():
     q, s, b = m.ops.quantize(w, 64, 4, torch.float32)
     y = m.ops.quantized_linear(x, q, s, b, group_size=64, bits=4)
     assert torch.allclose(y[0], (x[0].double().sum()).float().expand(16), rtol=1e-6) and (y[1] == 0).all()
+
+
+def block_truth(blk, x, routing):
+    """The block in float64 on the dequantised weights, with the routing the block itself reports."""
+    c = blk.config
+    out = torch.zeros(x.shape, dtype=torch.float64, device=x.device)
+    for e in range(c.n_experts):
+        hit = (routing["topk_idx"] == e).nonzero()
+        if hit.numel() == 0:
+            continue
+        mats = (blk.gate_proj, blk.up_proj, blk.down_proj)
+        prod = lambda v, p: product(v, p.weight[e], p.scales[e], p.biases[e], c.group_size, c.bits)  # noqa: E731
+        g, u = prod(x[hit[:, 0]], mats[0]), prod(x[hit[:, 0]], mats[1])
+        y = prod(g * torch.sigmoid(g) * u, mats[2])
+        out.index_add_(0, hit[:, 0], y * routing["topk_w"][hit[:, 0], hit[:, 1]].double()[:, None])
+    return out
+
+
+@pytest.mark.parametrize("hidden,inter,experts,k", [(256, 384, 8, 2), (1152, 128, 5, 3), (256, 192, 4, 2)])
+@pytest.mark.parametrize("bits,group", [(4, 32), (4, 128), (8, 32), (8, 128)])
+@pytest.mark.parametrize("tokens,zipf", [(1, None), (17, None), (40, 1.5), (200, None), (700, 1.5)])
+def test_blocks_with_groups_of_32_and_128(tokens, zipf, bits, group, hidden, inter, experts, k):
+    """One row, one pass and several passes of the kernel of a few rows, tile lists with and without short segments, tiles
+    of every list; the last shape is one the plain products keep with 4-bit codes.  Three roundings to bfloat16 (h, y and
+    the result), each at most 2^-8 of its values and typically 0.42 of that, so 0.73 * 2^-8 together: 2^-8.  The plain
+products round gate and up as well (0.94 * 2^-8, over as few as 256 values): 1.5 * 2^-8."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    if inter % group:
+        pytest.skip("the intermediate size is a multiple of the group")
+    cfg = m.MoeConfig(hidden, experts, k, inter, bits, group, 0)
+    blk = synth.make_block(cfg, seed=tokens, device="cuda", zipf_s=zipf, gen_device="cuda")
+    x = synth.make_tokens(cfg, tokens, seed=bits, device="cuda")
+    out, routing = blk.forward(x, debug=True)
+    ref = block_truth(blk, x, routing)
+    err = float((out.double() - ref).norm() / ref.norm())
+    bound = 1.5 * 2.0 ** -8 if bits == 4 and inter % 128 else 2.0 ** -8
+    assert err <= bound, err
+    # the same from the built-in scratch (no room for tile lists) where it fits
+    if blk.workspace_bytes(tokens) < 8 << 20:
+        again = blk.forward_static(x)
+        assert float((again.double() - ref).norm() / ref.norm()) <= bound
