@@ -1055,6 +1055,20 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
     MI_HIP(launch_qmm_codes_dense(a, group_size, bits, dtype, st));
     return 0;
   }
+  if (!transpose && aligned16(x) && aligned16(w) && aligned16(y)) {
+    ColsArgs a{};
+    a.x = x;
+    a.w = w;
+    a.s = scales; a.b = biases;
+    a.y = y;
+    a.N = N;
+    a.K = K;
+    a.M = M;
+    if (qmm_cols_applies(a, bits, dtype)) {
+      MI_HIP(launch_qmm_cols(a, group_size, bits, dtype, st));
+      return 0;
+    }
+  }
   if (!tuned_shape(dtype, transpose, group_size, bits, N, K)) {  // the plain kernels, no workspace
     MI_HIP(launch_qmm_plain(x, w, scales, biases, nullptr, nullptr, nullptr, nullptr, 0u, 1u, M, 1, N, K, group_size, bits,
                             transpose != 0, dtype, y, st));

@@ -360,6 +360,17 @@ struct RowsArgs {
 constexpr int kRowsMost = 16;  // rows of one pass of that kernel
 bool qmm_rows_applies(const RowsArgs &a, int group, int bits, int dt, bool glu);
 hipError_t launch_qmm_rows(const RowsArgs &a, int group, int bits, int dt, bool glu, hipStream_t st);
+// The tiled product over weights packed along N (qmm_cols.hip): x [M, K], w [K, N].
+struct ColsArgs {
+  const void *x;
+  const uint32_t *w;
+  const void *s, *b;
+  void *y;
+  int N, K;
+  int64_t M;
+};
+bool qmm_cols_applies(const ColsArgs &a, int bits, int dt);
+hipError_t launch_qmm_cols(const ColsArgs &a, int group, int bits, int dt, hipStream_t st);
 size_t codes_copy_bytes(int dt, int bits, int64_t rows, int K);
 size_t codes_sums_bytes(int64_t rows, int K, int group);
 hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,

@@ -1,0 +1,396 @@
+// Tiled quantized product over weights that are packed along the output columns: y [M, N] = x [M, K] w [K, N], each row
+// of w quantised along N.  This is the gradient of a quantized linear layer with respect to its input.
+//
+// Contract: mlx_quantized_matmul with transpose = false (mlx-rs/src/ops/quantization.rs:91-122).
+//
+// Arithmetic: a group has a scale of its own for every k, so nothing can be taken out of the sum; the weights are
+// dequantised, w = fma(s, q, b) in fp32, and enter the matrix cores in pieces (each the rounded rest of the ones before
+// it), as do f32 rows of x:
+//   bf16  x as it is, w in two pieces (16 bits and more): 2 products
+//   f16   x as it is, 2^10 w in two f16 pieces (22 bits down to |w| = 2^-13, and never off by more than 2^-35; the factor
+//         keeps the second piece clear of the smallest numbers and leaves |w| < 64 without an overflow): 2 products
+//   f32   x in three pieces (exact), w in three (exact): the 6 products down to 2^-18 of the first
+// A result that is not finite is computed again the plain way, one fma per k: pieces of an infinity are no numbers, and
+// where nothing but a piece has overflowed that gives the number.
+#include <type_traits>
+
+#include "common.hpp"
+
+namespace mi_moe {
+
+namespace {
+
+constexpr int kStep = 32;                   // K values per step
+constexpr uint32_t kOutside = 0x80000000u;  // an offset past every descriptor here: such a load returns zeros
+
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
+
+template <int DT> struct ElemOf;
+template <> struct ElemOf<0> { typedef uint16_t type; };
+template <> struct ElemOf<1> { typedef _Float16 type; };
+template <> struct ElemOf<2> { typedef float type; };
+
+__device__ __forceinline__ float as_f32(uint16_t v) { return bf16_to_f32(v); }
+__device__ __forceinline__ float as_f32(_Float16 v) { return (float)v; }
+__device__ __forceinline__ float as_f32(float v) { return v; }
+template <class T> __device__ __forceinline__ T rounded(float v) { return (T)v; }
+template <> __device__ __forceinline__ uint16_t rounded<uint16_t>(float v) { return f32_to_bf16(v); }
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void *base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+template <int DT>
+__device__ __forceinline__ f32x16_t mfma(u32x4_t a, u32x4_t b, f32x16_t c) {
+  if constexpr (DT == 1)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+constexpr int pieces_of_x(int dt) { return dt == 2 ? 3 : 1; }
+constexpr int pieces_of_w(int dt) { return dt == 2 ? 3 : 2; }
+constexpr float factor_of_w(int dt) { return dt == 1 ? 1024.0f : 1.0f; }
+
+// the pieces of two values, P registers: the first piece of both, the next one of what it left, ...
+template <int DT, int P>
+__device__ __forceinline__ void split_pair(float v0, float v1, uint32_t (&to)[P]) {
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    if constexpr (DT == 1) {
+      const half2_t h = __builtin_convertvector(f32x2_t{v0, v1}, half2_t);
+      to[p] = __builtin_bit_cast(uint32_t, h);
+      v0 -= (float)h.x;
+      v1 -= (float)h.y;
+    } else {
+      to[p] = cvt_pk_bf16(v0, v1);
+      v0 -= bf16lo_to_f32(to[p]);
+      v1 -= bf16hi_to_f32(to[p]);
+    }
+  }
+}
+
+// LDS of a wave: x [pieces][32 MS rows][32 K values], w [pieces][32 NT columns][32 K values], (s, b) of 32 K values of
+// two groups.  A row is four 16-byte chunks; chunk c of row r sits at c ^ (r / 4 % 4), so that the 16 lanes of one LDS
+// cycle, which read one chunk of 16 rows or write four chunks of four, meet 16 different places.
+constexpr int kRowPieces = 4;
+__device__ __forceinline__ int at(int row, int chunk) { return row * kRowPieces + (chunk ^ ((row >> 2) & 3)); }
+constexpr int kScaleRow = 32 * 8 + 16;  // bytes of one group's (s, b) pairs
+constexpr int wave_lds(int dt, int ms, int nt) {
+  return (pieces_of_x(dt) * ms + pieces_of_w(dt) * nt) * 32 * kRowPieces * 16 + 2 * kScaleRow;
+}
+
+}  // namespace
+
+// A block computes 32 MS rows x 32 NT columns; its KW waves share K among them, each on LDS of its own, and meet only to
+// add their sums: no wave waits for another in the loop, so the unpacking of one runs beside the multiplies of the other
+// on its SIMD.  A lane unpacks eight K values of 2 NT consecutive columns (a byte to a word of eight rows): the eight
+// values of a column are then one 16-byte chunk of a weight operand, and no exchange between lanes is needed although
+// memory holds the codes the other way round.  The columns are dealt to the sub-tiles so that a lane ends up with NT
+// consecutive ones: column n = 2 NT u + j goes to place 16 (j % NT * 2 + j / NT) + u, that is
+// sub-tile j % NT, lane 16 (j / NT) + u.
+// What bounds it (128 x 64 tiles, bf16): a step of a wave is 1024 cycles of matrix work (two products) beside about 800 of
+// unpacking and 32 KB through LDS, each near the CU's rate.  1000 x 2048 x 4096, 4-bit, groups of 64: 46 us for the call,
+// 360 TFLOP/s of the product (a thread per packed word of an output row, one k after the other: 1360 us); 8 rows 19 us
+// (1450); f32 141 us (1350).
+// Error against 64 bits at that size: bf16 1.6609e-3 and f16 2.0758e-4 as before (the result's rounding), f32 4.9e-7 (one
+// fma after the other: 1.07e-6).
+template <int DT, int BITS, int MS, int NT, int KW>
+__global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mtiles, int n_ntiles, int group_log2) {
+  typedef typename ElemOf<DT>::type T;
+  typedef typename std::conditional<BITS * NT == 4, uint8_t, typename std::conditional<BITS * NT == 16, uint32_t, uint16_t>::type>::type Codes;
+  constexpr int PX = pieces_of_x(DT), PW = pieces_of_w(DT);
+  constexpr float kFactor = factor_of_w(DT);
+  constexpr int CN = 2 * NT;          // columns a lane unpacks
+  constexpr int NX = 2 * MS;          // 16-row pieces of the token rows
+  constexpr int XP = DT == 2 ? 2 : 1; // 16-byte pieces of eight values of x
+  constexpr int X_SZ = 32 * MS * kRowPieces, W_SZ = 32 * NT * kRowPieces;
+  static_assert(sizeof(Codes) * 8 == BITS * CN, "a lane's columns of one row are one load");
+
+  // block -> tile.  Ids are dealt round-robin over the 8 XCDs: an XCD takes every eighth column tile and all row tiles
+  // of it, so its L2 holds those weights.
+  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+  const int nt = j / n_mtiles * 8 + xcd;
+  if (nt >= n_ntiles) return;
+  const int64_t row0 = (int64_t)(j % n_mtiles) * (32 * MS);
+  const int rows = a.M - row0 < 32 * MS ? (int)(a.M - row0) : 32 * MS;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int N = a.N, K = a.K, n0 = nt * (32 * NT);
+  const int row_bytes = N / 8 * BITS, G = N >> group_log2;
+
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  u32x4_t *const Xs = reinterpret_cast<u32x4_t *>(lds_raw + wave * wave_lds(DT, MS, NT));
+  u32x4_t *const Ws = Xs + PX * X_SZ;
+  unsigned char *const Ss = reinterpret_cast<unsigned char *>(Ws + PW * W_SZ);
+
+  // ---- this lane's share of a step: rows xrow + 16 i and chunk oct of x; columns CN u .. and rows 8 oct .. of the codes;
+  // row lane % 32 of the scales and biases, of the tile's first (lane / 32 = 0) or second 32 columns
+  const int xrow = lane >> 2, xoct = lane & 3;
+  const int u = lane & 15, oct = lane >> 4;
+  int wcol = n0 + CN * u;
+  wcol = wcol < N ? wcol : N - CN;  // columns past the end repeat the last ones (never stored)
+  const int skl = lane & 31;
+  int sgroup = (n0 + 32 * (lane >> 5)) >> group_log2;
+  sgroup = sgroup < G ? sgroup : G - 1;
+  const T *const sp = static_cast<const T *>(a.s), *const bp = static_cast<const T *>(a.b);
+
+  struct Stage {
+    u32x4_t x[NX][XP];
+    uint32_t q[8];
+    T s, b;
+  };
+  auto load = [&](int ks, Stage &R) __attribute__((always_inline)) {
+    const int k = ks * kStep;
+    // rows past the end are past the descriptor, K values past the end are sent there: both read zeros
+    const __amdgpu_buffer_rsrc_t xr = rsrc_of(static_cast<const T *>(a.x) + row0 * K + k, ((uint32_t)rows * K - k) * (uint32_t)sizeof(T));
+#pragma unroll
+    for (int i = 0; i < NX; ++i)
+#pragma unroll
+      for (int p = 0; p < XP; ++p) {
+        const uint32_t off = ((xrow + 16 * i) * (uint32_t)K + 8 * xoct) * (uint32_t)sizeof(T) + 16 * p;
+        R.x[i][p] = __builtin_amdgcn_raw_buffer_load_b128(xr, k + 8 * xoct < K ? off : kOutside, 0, 0);
+      }
+    const int left = K - k < kStep ? K - k : kStep;  // rows past the end read zeros, with a scale and a bias of zero
+    const __amdgpu_buffer_rsrc_t wr = rsrc_of(reinterpret_cast<const unsigned char *>(a.w) + (int64_t)k * row_bytes, (uint32_t)left * row_bytes);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const uint32_t off = (uint32_t)(8 * oct + r) * row_bytes + wcol * BITS / 8;
+      if constexpr (sizeof(Codes) == 1) R.q[r] = __builtin_amdgcn_raw_buffer_load_b8(wr, off, 0, 0);
+      else if constexpr (sizeof(Codes) == 2) R.q[r] = __builtin_amdgcn_raw_buffer_load_b16(wr, off, 0, 0);
+      else R.q[r] = __builtin_amdgcn_raw_buffer_load_b32(wr, off, 0, 0);
+    }
+    const bool on = skl < left;
+    const int64_t sat = (int64_t)(k + (on ? skl : 0)) * G + sgroup;
+    const T s = sp[sat], b = bp[sat];
+    R.s = on ? s : T{};
+    R.b = on ? b : T{};
+  };
+  auto wave_fence = [&]() __attribute__((always_inline)) {  // LDS serves a wave in order: this pins the program's order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  auto put = [&](const Stage &R) __attribute__((always_inline)) {
+    *reinterpret_cast<float2 *>(Ss + (lane >> 5) * kScaleRow + skl * 8) = make_float2(kFactor * as_f32(R.s), kFactor * as_f32(R.b));
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      u32x4_t *const to = Xs + at(xrow + 16 * i, xoct);
+      if constexpr (DT != 2) {
+        *to = R.x[i][0];
+      } else {
+        u32x4_t o[PX];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          uint32_t pc[PX];
+          split_pair<DT, PX>(__uint_as_float(R.x[i][c >> 1][2 * (c & 1)]), __uint_as_float(R.x[i][c >> 1][2 * (c & 1) + 1]), pc);
+#pragma unroll
+          for (int p = 0; p < PX; ++p) o[p][c] = pc[p];
+        }
+#pragma unroll
+        for (int p = 0; p < PX; ++p) to[p * X_SZ] = o[p];
+      }
+    }
+    wave_fence();
+    const float4 *const pairs = reinterpret_cast<const float4 *>(Ss + (CN * u / 32) * kScaleRow + oct * 64);
+    u32x4_t o[CN][PW];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {  // two rows
+      const float4 sb = pairs[r];
+      const uint32_t q0 = R.q[2 * r], q1 = R.q[2 * r + 1];
+#pragma unroll
+      for (int c = 0; c < CN; ++c) {
+        const float v0 = __builtin_fmaf(sb.x, (float)((q0 >> (BITS * c)) & ((1u << BITS) - 1u)), sb.y);
+        const float v1 = __builtin_fmaf(sb.z, (float)((q1 >> (BITS * c)) & ((1u << BITS) - 1u)), sb.w);
+        uint32_t pc[PW];
+        split_pair<DT, PW>(v0, v1, pc);
+#pragma unroll
+        for (int p = 0; p < PW; ++p) o[c][p][r] = pc[p];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < CN; ++c)
+#pragma unroll
+      for (int p = 0; p < PW; ++p) Ws[p * W_SZ + at(16 * (c % NT * 2 + c / NT) + u, oct)] = o[c][p];
+    wave_fence();
+  };
+
+  f32x16_t tot[MS][NT];
+#pragma unroll
+  for (int m = 0; m < MS; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) tot[m][t][r] = 0.f;
+  const int ln = lane & 31, kb = lane >> 5;
+  auto multiply = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      u32x4_t wv[NT][PW];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int p = 0; p < PW; ++p) wv[t][p] = Ws[p * W_SZ + at(32 * t + ln, 2 * h + kb)];
+#pragma unroll
+      for (int m = 0; m < MS; ++m) {
+        u32x4_t xv[PX];
+#pragma unroll
+        for (int p = 0; p < PX; ++p) xv[p] = Xs[p * X_SZ + at(32 * m + ln, 2 * h + kb)];
+#pragma unroll
+        for (int px = PX - 1; px >= 0; --px)
+#pragma unroll
+          for (int pw = PW - 1; pw >= 0; --pw)
+            if (px + pw < PW)
+#pragma unroll
+              for (int t = 0; t < NT; ++t) tot[m][t] = mfma<DT>(xv[px], wv[t][pw], tot[m][t]);
+      }
+    }
+    wave_fence();
+  };
+
+  const int steps = (K + kStep - 1) / kStep, share = (steps + KW - 1) / KW;
+  const int k0 = wave * share, k1 = k0 + share < steps ? k0 + share : steps;
+  if (k0 < k1) {
+    Stage R;
+    load(k0, R);
+    for (int ks = k0; ks < k1; ++ks) {
+      put(R);
+      load(ks + 1 < k1 ? ks + 1 : ks, R);
+      multiply();
+    }
+  }
+
+  // ---- the waves' sums: the second half of the waves hands its sums to the first, whose sums every wave then adds for a
+  // share of the rows, in a fixed order
+  constexpr int HALF = KW / 2, PIECES = MS * NT * 4;
+  float4 *const parts = reinterpret_cast<float4 *>(lds_raw);
+  auto give = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int m = 0; m < MS; ++m)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          parts[((wave % HALF) * PIECES + (m * 4 + r) * NT + t) * 64 + lane] =
+              make_float4(tot[m][t][4 * r], tot[m][t][4 * r + 1], tot[m][t][4 * r + 2], tot[m][t][4 * r + 3]);
+  };
+  __syncthreads();
+  if (wave >= HALF) give();
+  __syncthreads();
+  if (wave < HALF) {
+#pragma unroll
+    for (int m = 0; m < MS; ++m)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float4 v = parts[(wave * PIECES + (m * 4 + r) * NT + t) * 64 + lane];
+          tot[m][t][4 * r] += v.x;
+          tot[m][t][4 * r + 1] += v.y;
+          tot[m][t][4 * r + 2] += v.z;
+          tot[m][t][4 * r + 3] += v.w;
+        }
+    give();  // (its own slot, which only this wave has read)
+  }
+  __syncthreads();
+
+  const int col = n0 + CN * (ln & 15) + NT * (ln >> 4);
+  for (int piece = wave; piece < MS * 4; piece += KW) {  // rows 32 (piece / 4) + 8 (piece % 4) + 4 kb + 0 .. 3
+    float v[NT][4];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      float4 sum = parts[(piece * NT + t) * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < HALF; ++w) {
+        const float4 more = parts[(w * PIECES + piece * NT + t) * 64 + lane];
+        sum.x += more.x;
+        sum.y += more.y;
+        sum.z += more.z;
+        sum.w += more.w;
+      }
+      v[t][0] = sum.x;
+      v[t][1] = sum.y;
+      v[t][2] = sum.z;
+      v[t][3] = sum.w;
+    }
+    if (col >= N) continue;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 32 * (piece >> 2) + 8 * (piece & 3) + 4 * kb + r;
+      if (row >= rows) continue;
+      T o[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        float f = v[t][r] * (1.0f / kFactor);
+        if ((__float_as_uint(f) & 0x7f800000u) == 0x7f800000u) {
+          const T *const xk = static_cast<const T *>(a.x) + (row0 + row) * K;
+          const int n = col + t;
+          f = 0.f;
+          for (int k = 0; k < K; ++k) {
+            const uint32_t word = a.w[(int64_t)k * (row_bytes / 4) + n * BITS / 32];
+            const float qv = (float)((word >> (n * BITS % 32)) & ((1u << BITS) - 1u));
+            const int64_t g = (int64_t)k * G + (n >> group_log2);
+            f = __builtin_fmaf(as_f32(xk[k]), __builtin_fmaf(as_f32(sp[g]), qv, as_f32(bp[g])), f);
+          }
+        }
+        o[t] = rounded<T>(f);
+      }
+      T *const to = static_cast<T *>(a.y) + (row0 + row) * N + col;
+      __builtin_memcpy(__builtin_assume_aligned(to, NT * sizeof(T)), o, sizeof o);
+    }
+  }
+}
+
+template <int DT, int BITS, int MS, int NT, int KW>
+static hipError_t start_cols(const ColsArgs &a, int group_log2, hipStream_t st) {
+  constexpr int loop = KW * wave_lds(DT, MS, NT), sums = KW / 2 * MS * NT * 32 * 32 * 4, lds = loop > sums ? loop : sums;
+  static_assert(lds <= 160 * 1024, "more LDS than a CU has");
+  const int n_ntiles = (a.N + 32 * NT - 1) / (32 * NT);
+  const int64_t mtiles = (a.M + 32 * MS - 1) / (32 * MS), grid = (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
+  if (grid > INT32_MAX) return hipErrorInvalidValue;
+  const auto kernel = &qmm_cols_kernel<DT, BITS, MS, NT, KW>;
+  if (lds > 64 * 1024)
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        e != hipSuccess)
+      return e;
+  kernel<<<(unsigned)grid, 64 * KW, lds, st>>>(a, (int)mtiles, n_ntiles, group_log2);
+  return hipGetLastError();
+}
+
+// Whole 16-byte pieces of x, offsets that fit their 32 bits, no 2-bit codes; every other shape stays with the plain kernel.
+bool qmm_cols_applies(const ColsArgs &a, int bits, int dt) {
+  const int64_t elem = dt == 2 ? 4 : 2, most = (int64_t)1 << 31;
+  return bits != 2 && a.K % 8 == 0 && 128 * (int64_t)a.K * elem < most && 32 * (int64_t)a.N * bits / 8 < most && a.N % 32 == 0;
+}
+
+// Which tile: the smallest one of which the launch has at most one a CU; a CU's time is that of its unpacking and
+// multiplies, so a second tile on some CUs costs a whole further round.  Measured, 4-bit, groups of 64, bf16, N = 2048,
+// K = 4096, us of the call with 32 x 32 / 64 x 32 / 64 x 64 / 128 x 64 tiles at 64 / 130 / 300 / 1000 rows:
+// 21.0, 26.2, 28.4, 37.0 / 32.2, 21.6, 29.4, 38.0 / 47.9, 40.8, 31.3, 39.8 / 136, 86.7, 65.9, 46.3 (f16 the same to 5 %).
+// f32 holds three times the rows in LDS and multiplies three times as much: at 64 / 130 / 300 / 1000 rows 27.8, 38.5,
+// 80.2, 118 / 54.2, 40.7, 88.0, 121 / 85.2, 78.0, 91.0, 121 / 249, 174, 196, 141, so 64 x 32 for two rounds, and 128 x 64
+// beyond (K shared by four waves there: what LDS holds).
+template <int DT, int BITS>
+static hipError_t pick_cols(const ColsArgs &a, int group_log2, hipStream_t st) {
+  auto tiles = [&](int ms, int nt) { return (a.M + 32 * ms - 1) / (32 * ms) * ((a.N + 32 * nt - 1) / (32 * nt)); };
+  constexpr int kCus = 256;
+  if (tiles(1, 1) <= kCus) return start_cols<DT, BITS, 1, 1, 8>(a, group_log2, st);
+  if (tiles(2, 1) <= (DT == 2 ? 2 : 1) * kCus) return start_cols<DT, BITS, 2, 1, 8>(a, group_log2, st);
+  if constexpr (DT != 2)
+    if (tiles(2, 2) <= kCus) return start_cols<DT, BITS, 2, 2, 8>(a, group_log2, st);
+  return start_cols<DT, BITS, 4, 2, DT == 2 ? 4 : 8>(a, group_log2, st);
+}
+
+hipError_t launch_qmm_cols(const ColsArgs &a, int group, int bits, int dt, hipStream_t st) {
+  if (a.M == 0) return hipSuccess;
+  const int gl = group == 32 ? 5 : (group == 64 ? 6 : 7);
+  auto with_bits = [&](auto d) {
+    constexpr int DT = decltype(d)::value;
+    return bits == 4 ? pick_cols<DT, 4>(a, gl, st) : pick_cols<DT, 8>(a, gl, st);
+  };
+  if (dt == 0) return with_bits(std::integral_constant<int, 0>{});
+  if (dt == 1) return with_bits(std::integral_constant<int, 1>{});
+  return with_bits(std::integral_constant<int, 2>{});
+}
+
+}  // namespace mi_moe
