@@ -176,6 +176,36 @@ __host__ __device__ inline P *tile_list(P *base, int cls, int cap256, int n_expe
   return base + 4 + 4 * (size_t)cap256 + 4 + 4 * (size_t)n_experts;
 }
 
+// ---------------------------------------------------------------- element types, one element the plain way
+__device__ __forceinline__ float as_f32(uint16_t v) { return bf16_to_f32(v); }  // bfloat16, raw bits
+__device__ __forceinline__ float as_f32(_Float16 v) { return (float)v; }
+__device__ __forceinline__ float as_f32(float v) { return v; }
+
+__device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
+
+// One element of a product of weights packed along K, an fma per k on the dequantised weight.  The products on raw codes
+// take it where their own sum is not finite: an infinity against codes and biases apart cancels to no number where
+// the dequantised weight keeps its sign, and sums of unscaled codes overflow earlier.  paired: x has every 8-block as
+// (0,4)(1,5)(2,6)(3,7).
+template <int BITS, class T>
+__device__ __forceinline__ float plain_element(const T *x, bool paired, const uint32_t *w, const T *s, const T *b, int K, int group) {
+  constexpr int PER = 32 / BITS;  // a word of codes at a time; the x of a word is 8 to 32 aligned bytes
+  float sum = 0.f;
+#pragma unroll 1
+  for (int k = 0; k < K && sum == sum; k += PER) {  // (no number stays none)
+    T v[PER];
+    __builtin_memcpy(v, __builtin_assume_aligned(x + k, PER * sizeof(T) < 16 ? 8 : 16), sizeof v);
+    const uint32_t word = w[k / PER];
+    const float sc = as_f32(s[k / group]), bi = as_f32(b[k / group]);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const float xv = as_f32(paired ? v[(i & ~7) | (i & 3) << 1 | (i >> 2 & 1)] : v[i]);
+      sum = __builtin_fmaf(xv, __builtin_fmaf(sc, (float)((word >> (i * BITS)) & ((1u << BITS) - 1u)), bi), sum);
+    }
+  }
+  return sum;
+}
+
 // ---------------------------------------------------------------- device-coherent accesses
 // A load that observes what other workgroups have written before an agent-scope release
 // (bypasses the per-CU cache).  Used for data produced earlier in the same launch.

@@ -42,10 +42,6 @@ template <> struct ElemOf<0> { typedef uint16_t type; };
 template <> struct ElemOf<1> { typedef _Float16 type; };
 template <> struct ElemOf<2> { typedef float type; };
 
-__device__ __forceinline__ float as_f32(uint16_t v) { return bf16_to_f32(v); }
-__device__ __forceinline__ float as_f32(_Float16 v) { return (float)v; }
-__device__ __forceinline__ float as_f32(float v) { return v; }
-
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void *base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
 }
@@ -253,6 +249,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   const int64_t ebase = (int64_t)e * N;
   __amdgpu_buffer_rsrc_t wr[NT], sr[NT], br[NT];
   uint32_t w_voff[NT], s_voff[NT];
+  int w_row[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const bool up = GLU && t == 1;
@@ -263,6 +260,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     wr[t] = rsrc_of((up ? a.w1 : a.w0) + ebase * (row_bytes / 4), (uint32_t)N * row_bytes);
     sr[t] = rsrc_of(static_cast<const T *>(up ? a.s1 : a.s0) + ebase * G, ((uint32_t)N * G * sizeof(T) + 3u) & ~3u);  // (read in words)
     br[t] = rsrc_of(static_cast<const T *>(up ? a.b1 : a.b0) + ebase * G, (uint32_t)N * G * sizeof(T));
+    w_row[t] = row;
     w_voff[t] = (uint32_t)row * row_bytes + kb * 16;
     s_voff[t] = (uint32_t)row * G * sizeof(T);
   }
@@ -596,19 +594,35 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
       const int col0 = n0 + 32 * wave + 32 * WN * t;
       const int bc = col0 + ln < N ? col0 + ln : N - 1;
       const float lb = a.bias ? as_f32(static_cast<const T *>(a.bias)[bc]) : 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = 8 * (r >> 2) + 4 * kb + (r & 3);
-        float v;
-        if constexpr (GLU) {
-          const float g = tot[m][0][r], u = tot[m][1][r];
-          v = g / (1.0f + __expf(-g)) * u;
-        } else {
-          v = tot[m][t][r];
-        }
+      auto put = [&](int r, float v, float up) __attribute__((always_inline)) {
+        if constexpr (GLU) v = v / (1.0f + __expf(-v)) * up;
         T o = rounded<T>(v);
         if (a.bias) o = rounded<T>(as_f32(o) + lb);
-        reinterpret_cast<T *>(mine + row * ROWB)[ln] = o;
+        reinterpret_cast<T *>(mine + (8 * (r >> 2) + 4 * kb + (r & 3)) * ROWB)[ln] = o;
+      };
+      uint32_t again = 0;  // (bits: which of the sixteen sums are not finite)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float v = tot[m][t][r], up = tot[m][GLU ? 1 : t][r];
+        put(r, v, up);
+        again |= (not_finite(v) || (GLU && not_finite(up)) ? 1u : 0u) << r;
+      }
+      while (again) {
+        const int r = __builtin_ctz(again);
+        again &= again - 1;
+        const int tr = 32 * m + 8 * (r >> 2) + 4 * kb + (r & 3);
+        if (tr >= rows) continue;
+        const T *const xs = static_cast<const T *>(a.x) + (int64_t)(a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr)) * K;
+        float v[2];
+#pragma unroll
+        for (int i = 0; i < (GLU ? 2 : 1); ++i) {
+          const int tt = GLU ? i : t;
+          const int64_t wrow = ebase + w_row[tt];
+          v[i] = plain_element<BITS, T>(xs, paired_order(DT, BITS), (GLU && i ? a.w1 : a.w0) + wrow * (row_bytes / 4),
+                                        static_cast<const T *>(GLU && i ? a.s1 : a.s0) + wrow * G,
+                                        static_cast<const T *>(GLU && i ? a.b1 : a.b0) + wrow * G, K, K / G);
+        }
+        put(r, v[0], v[GLU ? 1 : 0]);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();

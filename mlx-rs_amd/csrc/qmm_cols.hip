@@ -32,9 +32,6 @@ template <> struct ElemOf<0> { typedef uint16_t type; };
 template <> struct ElemOf<1> { typedef _Float16 type; };
 template <> struct ElemOf<2> { typedef float type; };
 
-__device__ __forceinline__ float as_f32(uint16_t v) { return bf16_to_f32(v); }
-__device__ __forceinline__ float as_f32(_Float16 v) { return (float)v; }
-__device__ __forceinline__ float as_f32(float v) { return v; }
 template <class T> __device__ __forceinline__ T rounded(float v) { return (T)v; }
 template <> __device__ __forceinline__ uint16_t rounded<uint16_t>(float v) { return f32_to_bf16(v); }
 
@@ -322,11 +319,11 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         float f = v[t][r] * (1.0f / kFactor);
-        if ((__float_as_uint(f) & 0x7f800000u) == 0x7f800000u) {
+        if (not_finite(f)) {
           const T *const xk = static_cast<const T *>(a.x) + (row0 + row) * K;
           const int n = col + t;
           f = 0.f;
-          for (int k = 0; k < K; ++k) {
+          for (int k = 0; k < K && f == f; ++k) {  // (no number stays none)
             const uint32_t word = a.w[(int64_t)k * (row_bytes / 4) + n * BITS / 32];
             const float qv = (float)((word >> (n * BITS % 32)) & ((1u << BITS) - 1u));
             const int64_t g = (int64_t)k * G + (n >> group_log2);

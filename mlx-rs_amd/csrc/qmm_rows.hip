@@ -27,9 +27,6 @@ template <> struct ElemOf<0> { typedef uint16_t type; };
 template <> struct ElemOf<1> { typedef _Float16 type; };
 template <> struct ElemOf<2> { typedef float type; };
 
-__device__ __forceinline__ float as_f32(uint16_t v) { return bf16_to_f32(v); }
-__device__ __forceinline__ float as_f32(_Float16 v) { return (float)v; }
-__device__ __forceinline__ float as_f32(float v) { return v; }
 template <class T> __device__ __forceinline__ T rounded(float v) { return (T)v; }
 template <> __device__ __forceinline__ uint16_t rounded<uint16_t>(float v) { return (uint16_t)(cvt_pk_bf16(v, 0.f) & 0xffffu); }
 
@@ -380,18 +377,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
     }
     if (wk == 0 && n0 + c < N) {
       const float lb = a.bias ? as_f32(static_cast<const T *>(a.bias)[n0 + c]) : 0.f;
+      uint32_t again = 0;  // (bits: which of the four sums are not finite)
+      auto put = [&](int r, float v, float up) __attribute__((always_inline)) {
+        const int64_t rr = r0 + t0 + 4 * kb + r;
+        const int64_t dst = a.dst_rows ? (int64_t)a.dst_rows[rr] : rr;
+        if constexpr (GLU) v = v / (1.0f + __expf(-v)) * up;
+        T o = rounded<T>(v);
+        if (a.bias) o = rounded<T>(as_f32(o) + lb);
+        static_cast<T *>(a.y)[dst * N + n0 + c] = o;
+      };
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int slot = 4 * kb + r;
-        if (slot < nt) {
-          const int64_t rr = r0 + t0 + slot;
-          const int64_t dst = a.dst_rows ? (int64_t)a.dst_rows[rr] : rr;
-          float v = tot[0][r];
-          if constexpr (GLU) v = v / (1.0f + __expf(-v)) * tot[1][r];
-          T o = rounded<T>(v);
-          if (a.bias) o = rounded<T>(as_f32(o) + lb);
-          static_cast<T *>(a.y)[dst * N + n0 + c] = o;
+        if (4 * kb + r < nt) {
+          put(r, tot[0][r], tot[NM - 1][r]);
+          if (not_finite(tot[0][r]) || not_finite(tot[NM - 1][r])) again |= 1u << r;
         }
+      }
+      while (again) {
+        const int r = __builtin_ctz(again);
+        again &= again - 1;
+        const int64_t rr = r0 + t0 + 4 * kb + r;
+        const T *const xr = static_cast<const T *>(a.x) + (a.src_rows ? (int64_t)a.src_rows[rr] : rr) * K;
+        float v[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+          const int64_t wrow = ebase + n0 + c;
+          v[m] = plain_element<BITS, T>(xr, false, (m ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const T *>(m ? a.s1 : a.s0) + wrow * G,
+                                        static_cast<const T *>(m ? a.b1 : a.b0) + wrow * G, K, GROUP);
+        }
+        put(r, v[0], v[NM - 1]);
       }
     }
   }

@@ -100,3 +100,38 @@ products round gate and up as well (0.94 * 2^-8, over as few as 256 values): 1.5
     if blk.workspace_bytes(tokens) < 8 << 20:
         again = blk.forward_static(x)
         assert float((again.double() - ref).norm() / ref.norm()) <= bound
+
+
+@pytest.mark.parametrize("dtype,group", [("float16", 64), ("bfloat16", 32), ("float32", 128)])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows", [7, 70, 1100])
+def test_values_that_are_not_finite(rows, bits, dtype, group):
+    """Infinities and NaNs in the rows, the scales and the biases: every element is one where the product of the
+    dequantised matrix is, with its sign, in the kernel of a few rows and in the tiles of both code orders."""
+    import mlx_rs_amd as m
+    dt = getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(rows + bits)
+    q, s, b = m.ops.quantize(torch.randn((200, 384), generator=gen, device="cuda") * 0.02, group, bits, dt)
+    x = torch.randn((rows, 384), generator=gen, device="cuda").to(dt)
+    x[0, 3], x[rows - 1, 383], x[rows // 2, 130] = float("inf"), float("-inf"), float("nan")
+    b[17, 1], s[199, 2] = float("inf"), float("inf")
+    ref = product(x, q, s, b, group, bits)
+    y = m.ops.quantized_linear(x, q, s, b, group_size=group, bits=bits)
+    odd = ~ref.isfinite()
+    assert odd.any() and torch.equal(y.isfinite(), ~odd)
+    assert torch.equal(y[odd].double().nan_to_num(), ref[odd].nan_to_num())
+
+
+@pytest.mark.parametrize("tokens,zipf", [(9, None), (300, 1.5)])
+def test_a_block_whose_gate_is_not_finite(tokens, zipf):
+    """Gate products that are infinite or no number (a scale that is) go through the activation as they are."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(256, 4, 2, 128, 4, 32, 0)
+    blk = synth.make_block(cfg, seed=tokens, device="cuda", zipf_s=zipf, gen_device="cuda")
+    x = synth.make_tokens(cfg, tokens, seed=1, device="cuda")
+    blk.gate_proj.biases[1, 5, 2] = float("inf")
+    blk.up_proj.biases[2, 7, 0] = float("-inf")
+    out, routing = blk.forward(x, debug=True)
+    ref = block_truth(blk, x, routing)
+    assert not ref.isfinite().all() and torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
