@@ -242,8 +242,7 @@ int mi_moe_gather_qmm_typed(const void *x, const uint32_t *w, const void *scales
  * y (M x N) = x (M x K) . dequantize(w)^T on the same kernels as gather_qmm (one matrix, every row).
  * x: bf16 [M, K]; w: [N, K*bits/32]; scales, biases: bf16 [N, K/group_size]; y: bf16 [M, N].
  * transpose = 0 (the op's own default; test_quantized_matmul, ops/quantization.rs:318-342):
- * w [K, N*bits/32], scales, biases [K, N/group_size], y = x . dequantize(w), a plain kernel; so are
- * group sizes 32 / 128 and 2-bit codes.
+ * w [K, N*bits/32], scales, biases [K, N/group_size], y = x . dequantize(w).
  * workspace >= mi_moe_quantized_matmul_workspace_size; products that the bf16, group-64 kernels do not
  * serve also run with less or none, more slowly. */
 int mi_moe_quantized_matmul_workspace_size(int64_t M, int32_t K, int32_t bits, size_t *bytes);

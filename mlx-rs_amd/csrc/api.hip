@@ -997,11 +997,39 @@ int mi_moe_quantized_matmul_workspace_size(int64_t M, int32_t K, int32_t bits, s
   return 0;
 } MI_CATCH("quantized_matmul_workspace_size")
 
-// The tiled product on raw codes: transposed weights that the bf16, group-64 kernels do not take.  Its descriptors hold
-// a 32-bit size of one matrix.
-static bool codes_shape(int32_t dtype, int32_t transpose, int32_t group_size, int32_t bits, int32_t N, int32_t K) {
-  return transpose && bits != 2 && !tuned_shape(dtype, transpose, group_size, bits, N, K) && K % 128 == 0 &&
-         (int64_t)N * K * bits / 8 < (int64_t)1 << 31 && (int64_t)N * K < (int64_t)1 << 33;
+// What the products on raw codes take: transposed weights, any element type and group.  Their descriptors hold a 32-bit
+// size of one matrix.
+static bool codes_shape(int32_t transpose, int32_t bits, int32_t N, int32_t K) {
+  return transpose && bits != 2 && K % 128 == 0 && (int64_t)N * K * bits / 8 < (int64_t)1 << 31 && (int64_t)N * K < (int64_t)1 << 33;
+}
+
+// Which transposed dense products take the kernel of a few rows (nothing to prepare, one launch).  Measured, us of the kernels
+// (few rows / the one it stands against):
+//   4096 x 4096, 16 rows of 4-bit codes 18.3 (f16), 20.7 (bf16, groups of 32), 30.1 (f32) / tiles on raw codes 19.8, 26.8, 35.7;
+//   of 8-bit codes 26.7, 27.4, 29.5 / 23.5, 24.8, 34.3.  One row of 4-bit codes or f32 is still the plain kernel's: 7.5, 9.1
+//   and 10.8 / 6.7 (f16 4-bit), 7.1 and 9.8 (f32), unless the tuned bf16 shapes apply (no plain kernel there).
+//   More rows of short 4-bit ones: 4096 x 2048 at 20 / 32 rows 14.0, 18.0 / tiles 17.9, 18.1; 4096 x 4096 23.9, 31.6 / 21.7, 21.9;
+//   1024 x 1024 8.9, 11.0 / 15.5, 15.6.
+//   bf16, groups of 64 / streaming kernel and its record's launch: 4-bit 4096 x 2048 at 1 / 8 / 16 rows 5.4, 7.9, 10.5 /
+//   7.9, 9.5, 13.5, 4096 x 4096 7.0, 12.3, 17.6 / 10.4, 12.6, 20.2; 8-bit 2048 x 4096 at 1 / 2 / 4 / 8 / 16 rows 8.6, 9.3, 10.9,
+//   14.1, 20.8 / 10.1, 10.2, 10.7, 13.6, 17.7, 4096 x 1024 4.7, 4.8, 5.4, 6.1, 7.5 / 7.4, 7.7, 8.1, 8.9, 10.6.
+static bool dense_takes_rows(bool tuned, int32_t dtype, int32_t bits, int64_t M, int32_t K) {
+  const bool narrow = bits == 4 || dtype == MI_MOE_DTYPE_F32;
+  if (tuned && bits == 8) return M <= kRowsMost && M * K <= (int64_t)1 << 14;
+  if (M == 1 && !tuned && narrow) return false;
+  if (M <= (narrow ? kRowsMost : 12)) return true;
+  return bits == 4 && dtype != MI_MOE_DTYPE_F32 && M <= 2 * kRowsMost && M * K <= (int64_t)1 << 16;
+}
+
+// bf16, groups of 64: whether the 256 x 256 tiles with dequantised weights are faster than the 64 x 128 (or smaller) tiles
+// on raw codes.  The larger tiles pay once their launch fills the chip.  Their time is close to 55 + 0.37 per tile (up to
+// 256 tiles, K = 4096), that of the others to 15 + 0.113 per 64 x 128 tile; both go with K, so the line is the same for
+// every K.  Measured, 256 x 256 / raw codes, us of the call, 4-bit: 4096 x 4096 at 64 / 128 / 512 / 1024 / 1280 / 2048 / 8192 rows
+// 59.2, 61.5, 66.8, 79.1, 80.3, 104, 279 / 22.6, 24.2, 41.4, 66.4, 90.9, 124, 466; 14336 x 4096 at 256 / 512 / 2048 rows 80.4, 103,
+// 248 / 65.2, 113, 406; 8-bit 2048 x 4096 at 64 / 1024 / 2048 / 4096 rows 56.9, 61.9, 72.6, 98.9 / 22.7, 39.8, 64.9, 129.
+static bool dense_takes_large_tiles(int64_t M, int32_t N) {
+  const int64_t large = (M + 255) / 256 * ((N + 255) / 256), small = (M + 63) / 64 * ((N + 127) / 128);
+  return 10 * small > 33 * large + 3540;
 }
 
 // linear_bias: [N] added with a rounding of its own, or nullptr
@@ -1014,14 +1042,16 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
   if (M == 0) return 0;
   if (!x || !w || !scales || !biases || !y) return fail("quantized_matmul: x, w, scales, biases and y must be non-NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // A few rows: nothing to prepare.  Measured at 4096 x 4096, us of the kernels: 16 rows of 4-bit codes 18.3 (f16), 20.7
-  // (bf16, groups of 32), 30.1 (f32) against 19.8, 26.8, 35.7 for the tiles; of 8-bit codes 26.7, 27.4, 29.5 against
-  // 23.5, 24.8, 34.3.  One row of 4-bit codes or f32 is still the plain kernel's: 6.7 (f16 4-bit), 7.1 and 9.8 (f32)
-  // against 7.5, 9.1 and 10.8.
-  const bool one_plain = M == 1 && (bits == 4 || dtype == MI_MOE_DTYPE_F32);
-  if (codes_shape(dtype, transpose, group_size, bits, N, K) && !one_plain &&
-      M <= (bits == 4 || dtype == MI_MOE_DTYPE_F32 ? kRowsMost : 12) && aligned16(x) && aligned16(w) &&
-      aligned16(scales) && aligned16(biases)) {
+  const bool tuned = tuned_shape(dtype, transpose, group_size, bits, N, K), codes = codes_shape(transpose, bits, N, K);
+  size_t mt_words = 0;
+  if (tuned) {
+    if (!aligned16(x) || !aligned16(w) || !aligned16(scales) || !aligned16(biases) || !aligned16(y))
+      return fail("quantized_matmul: pointers must be 16-byte aligned");
+    const size_t need = qmm_dense_bytes(M, K, bits, &mt_words);
+    if (!workspace || workspace_bytes < need) return fail("quantized_matmul: workspace too small (need %zu bytes)", need);
+  }
+  const bool one_plain = M == 1 && !tuned && (bits == 4 || dtype == MI_MOE_DTYPE_F32);
+  if (codes && dense_takes_rows(tuned, dtype, bits, M, K) && aligned16(x) && aligned16(w) && aligned16(scales) && aligned16(biases)) {
     RowsArgs a{};
     a.x = x;
     a.w0 = w; a.s0 = scales; a.b0 = biases;
@@ -1035,8 +1065,9 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
       return 0;
     }
   }
-  if (codes_shape(dtype, transpose, group_size, bits, N, K) && !one_plain && M * K * 4 < (int64_t)1 << 31 && workspace &&
-      workspace_bytes >= codes_bytes(M, K, group_size, bits, dtype) && aligned16(x) && aligned16(w) && aligned16(y)) {
+  const bool streamed = tuned && bits == 8 && M < tiled_avg_rows(bits);  // (see dense_takes_rows)
+  const bool large_tiles = tuned && codes && !streamed && dense_takes_large_tiles(M, N);
+  if (codes && !one_plain && !streamed && !large_tiles && M * K * 4 < (int64_t)1 << 31 && workspace && workspace_bytes >= codes_bytes(M, K, group_size, bits, dtype) && aligned16(x) && aligned16(w) && aligned16(y)) {
     Carver cv(workspace);
     const size_t copy_bytes = codes_copy_bytes(dtype, bits, M, K);
     uint16_t *copy = copy_bytes ? reinterpret_cast<uint16_t *>(cv.take<char>(copy_bytes)) : nullptr;
@@ -1069,26 +1100,23 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
       return 0;
     }
   }
-  if (!tuned_shape(dtype, transpose, group_size, bits, N, K)) {  // the plain kernels, no workspace
+  if (!tuned) {  // the plain kernels, no workspace
     MI_HIP(launch_qmm_plain(x, w, scales, biases, nullptr, nullptr, nullptr, nullptr, 0u, 1u, M, 1, N, K, group_size, bits,
                             transpose != 0, dtype, y, st));
     if (linear_bias) MI_HIP(launch_add_row_bias(y, linear_bias, M, N, dtype, st));
     return 0;
   }
-  if (!aligned16(x) || !aligned16(w) || !aligned16(scales) || !aligned16(biases) || !aligned16(y))
-    return fail("quantized_matmul: pointers must be 16-byte aligned");
-  size_t mt_words = 0;
-  const size_t need = qmm_dense_bytes(M, K, bits, &mt_words);
-  if (!workspace || workspace_bytes < need) return fail("quantized_matmul: workspace too small (need %zu bytes)", need);
   Carver cv(workspace);
   uint32_t *work = cv.take<uint32_t>(16);
   uint32_t *mtiles = cv.take<uint32_t>(mt_words);
-  // one segment of M rows: the tiled kernel from the batch threshold on (fewer rows: streaming passes)
+  // one segment of M rows: the tiled kernel from the batch threshold on (fewer rows: streaming passes).  Where the 256-row
+  // tiles fill the chip the rows behind the last whole tile are one more of them, in the same launch (in a class of their
+  // own, one launch after the other: 1800 x 4096 x 4096 140 us; 2048 rows 104)
   const bool big = M >= tiled_avg_rows(bits) && (K / 64) % 2 == 0;
   const uint16_t *xb = static_cast<const uint16_t *>(x);
   uint16_t *xperm = (bits == 4 && big) ? cv.take<uint16_t>((size_t)M * K) : nullptr;
   const int cap256 = (int)((M + kBigTileM - 1) / kBigTileM);
-  MI_HIP(launch_dense_records(M, big ? tiled_avg_rows(bits) : 0, work, mtiles, cap256, st));
+  MI_HIP(launch_dense_records(M, big ? tiled_avg_rows(bits) : 0, large_tiles, work, mtiles, cap256, st));
   if (xperm) MI_HIP(launch_pair_rows(xb, M, K, xperm, st));
   GroupedArgs a{};
   a.x = xb;
@@ -1105,7 +1133,8 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
   a.bits = bits;
   a.total_rows = M;
   a.max_rows_per_expert = M;
-  MI_HIP(launch_grouped_qmm(a, false, st));
+  if (large_tiles) MI_HIP(launch_large_qmm_class(a, false, 0, st));
+  else MI_HIP(launch_grouped_qmm(a, false, st));
   if (linear_bias) MI_HIP(launch_add_row_bias(y, linear_bias, M, N, dtype, st));
   return 0;
 }

@@ -133,13 +133,17 @@ hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, ui
 }
 
 // One dense segment (a plain quantized matmul: every row goes to matrix 0): the work record or, from
-// big_thr rows on, its M tiles.
-__global__ void dense_records_kernel(uint32_t M, uint32_t big_thr, uint32_t *__restrict__ work,
+// big_thr rows on, its M tiles (one_list: 256-row tiles only, the last one short).
+__global__ void dense_records_kernel(uint32_t M, uint32_t big_thr, bool one_list, uint32_t *__restrict__ work,
                                      uint32_t *__restrict__ mtiles, int cap256) {
   const uint32_t tid = threadIdx.x;
   const bool big = big_thr != 0u && M >= big_thr;
   if (tid < kWorkWords) work[tid] = (tid == 2 && !big) ? M : 0u;  // {expert 0, row 0, M rows, no inline rows}
-  const TileSplit ts = split_segment(big ? M : 0u);
+  TileSplit ts = split_segment(big ? M : 0u);
+  if (big && one_list) {
+    ts.n256 = (M + kBigTileM - 1) / kBigTileM;
+    ts.r = 0u;
+  }
   uint32_t *const l128 = tile_list(mtiles, 1, cap256, 1), *const l64 = tile_list(mtiles, 2, cap256, 1);
   if (tid == 0) {
     mtiles[0] = ts.n256;
@@ -162,9 +166,9 @@ __global__ void dense_records_kernel(uint32_t M, uint32_t big_thr, uint32_t *__r
   }
 }
 
-hipError_t launch_dense_records(int64_t M, int big_thr, uint32_t *work, uint32_t *mtiles, int cap256,
+hipError_t launch_dense_records(int64_t M, int big_thr, bool one_list, uint32_t *work, uint32_t *mtiles, int cap256,
                                 hipStream_t st) {
-  dense_records_kernel<<<1, 256, 0, st>>>((uint32_t)M, (uint32_t)big_thr, work, mtiles, cap256);
+  dense_records_kernel<<<1, 256, 0, st>>>((uint32_t)M, (uint32_t)big_thr, one_list, work, mtiles, cap256);
   return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
-// Tiled quantized product on raw codes, for everything the bfloat16 / group-64 kernels do not take: activations in
-// bfloat16, float16 or float32, groups of 32, 64 or 128, any number of output columns.
+// Tiled quantized product on raw codes: activations in bfloat16, float16 or float32, groups of 32, 64 or 128, any number of
+// output columns.
 //
 // Contract: mlx_quantized_matmul / mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:91-122,160-230).
 //
@@ -689,9 +689,11 @@ static hipError_t start_codes(const CodesArgs &a, int scale_shift, const uint32_
 // Which tile, from the number of tiles a launch of each has (256 CUs).  Measured with f16, 4-bit, groups of 64, us of the
 // whole call at (M, N, K) = (96, 4096, 4096) / (160, 4096, 4096) / (400, 4096, 4096) / (640, 2304, 2304) / (1000, 1024, 4096)
 // / (1000, 4096, 4096):
-//   32 x 64, K shared by four groups:   22.0 / 31.5 / 58.6 / 39.7 / 38.7 / 121   while there are at most two such tiles a CU
+//   32 x 64, K shared by four groups:   22.0 / 31.5 / 58.6 / 39.7 / 38.7 / 121   while a CU gets one at most
 //   64 x 128, K shared by two groups:   35.6 / 36.5 / 41.1 / 29.7 / 39.9 / 75.8  while a CU gets one at most
 //   64 x 128:                           41.5 / 42.4 / 46.7 / 31.0 / 45.6 / 66.7  (several blocks a CU overlap as K groups do)
+// Between one and two 32 x 64 tiles a CU the two are as fast with f16 and K = 4096; bf16, 4-bit, 32 x 64 / 64 x 128:
+// (200, 4096, 2048) 32.0 / 24.8, (200, 4096, 4096) 39.9 / 37.4, (1000, 1024, 1024) 29.7 / 21.8, (400, 2048, 768) 19.7 / 14.7.
 // (128 x 128 tiles: 65.1 / 67.0 / 70.2 / 45.9 / 69.3 / 76.0.)  f32 multiplies three times as much and holds three times
 // the rows in LDS: 32 x 64 with two groups up to 320 tiles, then 32 x 256 (1000, 4096, 4096: 147 against 164 for 64 x 128).
 template <int DT, int BITS, bool G32>
@@ -701,7 +703,7 @@ static hipError_t start_dense(const CodesArgs &a, int scale_shift, hipStream_t s
     if (tiles(32, 64) <= 320) return start_codes<DT, BITS, G32, false, 1, 1, 2, 2>(a, scale_shift, nullptr, 0, 0, st);
     return start_codes<DT, BITS, G32, false, 1, 2, 4, 1>(a, scale_shift, nullptr, 0, 0, st);
   } else {
-    if (tiles(32, 64) <= 512) return start_codes<DT, BITS, G32, false, 1, 1, 2, 4>(a, scale_shift, nullptr, 0, 0, st);
+    if (tiles(32, 64) <= 256) return start_codes<DT, BITS, G32, false, 1, 1, 2, 4>(a, scale_shift, nullptr, 0, 0, st);
     if (tiles(64, 128) <= 256) return start_codes<DT, BITS, G32, false, 2, 1, 4, 2>(a, scale_shift, nullptr, 0, 0, st);
     return start_codes<DT, BITS, G32, false, 2, 1, 4, 1>(a, scale_shift, nullptr, 0, 0, st);
   }

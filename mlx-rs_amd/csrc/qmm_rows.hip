@@ -1,5 +1,5 @@
-// Quantized products of a few rows (a decode batch's linear layer, short expert segments) for everything the bfloat16 /
-// group-64 streaming kernel does not take: activations in bfloat16, float16 or float32, groups of 32, 64 or 128.
+// Quantized products of a few rows (a decode batch's linear layer; short expert segments with groups of 32 or 128):
+// activations in bfloat16, float16 or float32, groups of 32, 64 or 128.
 //
 // Contract: mlx_quantized_matmul / mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:91-122,160-230);
 // with GLU also nn::silu and multiply (nn/activation.rs:142-144,876-880).
