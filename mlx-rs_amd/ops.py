@@ -7,6 +7,7 @@ take float16 and float32); packed weights and indices ``torch.int32`` holding th
 patterns (torch has no arithmetic on uint32).
 """
 import ctypes as C
+import functools
 
 import torch
 
@@ -15,11 +16,12 @@ from .capi import check, load_library
 
 
 def _ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()  # (the prototypes convert it)
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream's handle, without the Stream object around it (a decode step calls a linear layer every 10 us)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _need(t, dtype, name):
@@ -176,6 +178,13 @@ def _check_qmat(who, w, scales, biases, K, transpose, group_size, bits):
     return N
 
 
+@functools.lru_cache(maxsize=1024)
+def _matmul_workspace_bytes(M, K, bits):
+    need = C.c_size_t()
+    check(load_library().mi_moe_quantized_matmul_workspace_size(M, K, bits, C.byref(need)))
+    return need.value
+
+
 def quantized_matmul(x, w, scales, biases, transpose=False, group_size=64, bits=4):
     """ops::quantized_matmul (mlx-rs/src/ops/quantization.rs:91-122), same argument order and defaults
     (``transpose`` defaults to False as there; QuantizedLinear passes True, mlx-rs/src/nn/quantized.rs:363-386).
@@ -207,20 +216,19 @@ def quantized_linear(x, w, scales, biases, linear_bias=None, transpose=True, gro
         _need(linear_bias, x.dtype, "linear_bias")
         if linear_bias.numel() != N:
             raise capi.MoeError(f"{_who}: linear_bias must have {N} elements, got {linear_bias.numel()}")
-    x2 = x.reshape(-1, K)
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
     M = x2.shape[0]
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    need = C.c_size_t()
-    check(lib.mi_moe_quantized_matmul_workspace_size(M, K, bits, C.byref(need)))
-    ws = _workspace(need.value, x.device)
+    ws_bytes = _matmul_workspace_bytes(M, K, bits) + 256
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
     if linear_bias is None:
         check(lib.mi_moe_quantized_matmul_typed(_ptr(x2), _ptr(w), _ptr(scales), _ptr(biases), M, N, K,
                                                 1 if transpose else 0, group_size, bits, dt, _ptr(y), _ptr(ws),
-                                                ws.numel(), _stream()))
+                                                ws_bytes, _stream()))
     else:
         check(lib.mi_moe_quantized_linear_typed(_ptr(x2), _ptr(w), _ptr(scales), _ptr(biases), _ptr(linear_bias), M, N, K,
-                                                group_size, bits, dt, _ptr(y), _ptr(ws), ws.numel(), _stream()))
-    return y.reshape(*x.shape[:-1], N)
+                                                group_size, bits, dt, _ptr(y), _ptr(ws), ws_bytes, _stream()))
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], N)
 
 
 def rms_norm(x, weight, eps=1e-5):
