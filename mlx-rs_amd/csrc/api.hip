@@ -68,8 +68,8 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 size_t align_up(size_t v, size_t a = 256) { return (v + a - 1) / a * a; }
 
-// the block runs on the tuned kernels with 4- or 8-bit codes in groups of 64; other group sizes and
-// 2-bit codes take the plain products
+// the block runs on the tuned kernels with 4- or 8-bit codes in groups of 64; other group sizes take the
+// products on raw codes where those serve the shape (ForwardWs::raw), the rest and 2-bit codes the plain products
 bool plain_config(const mi_moe_config &c) { return c.group_size != 64 || c.bits == 2; }
 
 int check_config(const mi_moe_config *c) {
@@ -997,28 +997,26 @@ int mi_moe_quantized_matmul_workspace_size(int64_t M, int32_t K, int32_t bits, s
   return 0;
 } MI_CATCH("quantized_matmul_workspace_size")
 
-// What the products on raw codes take: transposed weights, any element type and group.  Their descriptors hold a 32-bit
+// What the products on raw codes take: transposed weights, bf16 or f16 (see qmm_codes.hip for f32), any group.  Their descriptors hold a 32-bit
 // size of one matrix.
-static bool codes_shape(int32_t transpose, int32_t bits, int32_t N, int32_t K) {
-  return transpose && bits != 2 && K % 128 == 0 && (int64_t)N * K * bits / 8 < (int64_t)1 << 31 && (int64_t)N * K < (int64_t)1 << 33;
+static bool codes_shape(int32_t dtype, int32_t transpose, int32_t bits, int32_t N, int32_t K) {
+  return transpose && dtype != MI_MOE_DTYPE_F32 && bits != 2 && K % 128 == 0 && (int64_t)N * K * bits / 8 < (int64_t)1 << 31 && (int64_t)N * K < (int64_t)1 << 33;
 }
 
 // Which transposed dense products take the kernel of a few rows (nothing to prepare, one launch).  Measured, us of the kernels
 // (few rows / the one it stands against):
-//   4096 x 4096, 16 rows of 4-bit codes 18.3 (f16), 20.7 (bf16, groups of 32), 30.1 (f32) / tiles on raw codes 19.8, 26.8, 35.7;
-//   of 8-bit codes 26.7, 27.4, 29.5 / 23.5, 24.8, 34.3.  One row of 4-bit codes or f32 is still the plain kernel's: 7.5, 9.1
-//   and 10.8 / 6.7 (f16 4-bit), 7.1 and 9.8 (f32), unless the tuned bf16 shapes apply (no plain kernel there).
+//   4096 x 4096, 16 rows of 4-bit codes 18.3 (f16), 20.7 (bf16, groups of 32) / tiles on raw codes 19.8, 26.8;
+//   of 8-bit codes 26.7, 27.4 / 23.5, 24.8.  One row of 4-bit codes is still the plain kernel's: 7.5 / 6.7 (f16), unless the tuned bf16 shapes apply (no plain kernel there).
 //   More rows of short 4-bit ones: 4096 x 2048 at 20 / 32 rows 14.0, 18.0 / tiles 17.9, 18.1; 4096 x 4096 23.9, 31.6 / 21.7, 21.9;
 //   1024 x 1024 8.9, 11.0 / 15.5, 15.6.
 //   bf16, groups of 64 / streaming kernel and its record's launch: 4-bit 4096 x 2048 at 1 / 8 / 16 rows 5.4, 7.9, 10.5 /
 //   7.9, 9.5, 13.5, 4096 x 4096 7.0, 12.3, 17.6 / 10.4, 12.6, 20.2; 8-bit 2048 x 4096 at 1 / 2 / 4 / 8 / 16 rows 8.6, 9.3, 10.9,
 //   14.1, 20.8 / 10.1, 10.2, 10.7, 13.6, 17.7, 4096 x 1024 4.7, 4.8, 5.4, 6.1, 7.5 / 7.4, 7.7, 8.1, 8.9, 10.6.
-static bool dense_takes_rows(bool tuned, int32_t dtype, int32_t bits, int64_t M, int32_t K) {
-  const bool narrow = bits == 4 || dtype == MI_MOE_DTYPE_F32;
+static bool dense_takes_rows(bool tuned, int32_t bits, int64_t M, int32_t K) {
   if (tuned && bits == 8) return M <= kRowsMost && M * K <= (int64_t)1 << 14;
-  if (M == 1 && !tuned && narrow) return false;
-  if (M <= (narrow ? kRowsMost : 12)) return true;
-  return bits == 4 && dtype != MI_MOE_DTYPE_F32 && M <= 2 * kRowsMost && M * K <= (int64_t)1 << 16;
+  if (M == 1 && !tuned && bits == 4) return false;
+  if (M <= (bits == 4 ? kRowsMost : 12)) return true;
+  return bits == 4 && M <= 2 * kRowsMost && M * K <= (int64_t)1 << 16;
 }
 
 // bf16, groups of 64: whether the 256 x 256 tiles with dequantised weights are faster than the 64 x 128 (or smaller) tiles
@@ -1042,7 +1040,7 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
   if (M == 0) return 0;
   if (!x || !w || !scales || !biases || !y) return fail("quantized_matmul: x, w, scales, biases and y must be non-NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const bool tuned = tuned_shape(dtype, transpose, group_size, bits, N, K), codes = codes_shape(transpose, bits, N, K);
+  const bool tuned = tuned_shape(dtype, transpose, group_size, bits, N, K), codes = codes_shape(dtype, transpose, bits, N, K);
   size_t mt_words = 0;
   if (tuned) {
     if (!aligned16(x) || !aligned16(w) || !aligned16(scales) || !aligned16(biases) || !aligned16(y))
@@ -1050,8 +1048,8 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
     const size_t need = qmm_dense_bytes(M, K, bits, &mt_words);
     if (!workspace || workspace_bytes < need) return fail("quantized_matmul: workspace too small (need %zu bytes)", need);
   }
-  const bool one_plain = M == 1 && !tuned && (bits == 4 || dtype == MI_MOE_DTYPE_F32);
-  if (codes && dense_takes_rows(tuned, dtype, bits, M, K) && aligned16(x) && aligned16(w) && aligned16(scales) && aligned16(biases)) {
+  const bool one_plain = M == 1 && !tuned && bits == 4;
+  if (codes && dense_takes_rows(tuned, bits, M, K) && aligned16(x) && aligned16(w) && aligned16(scales) && aligned16(biases)) {
     RowsArgs a{};
     a.x = x;
     a.w0 = w; a.s0 = scales; a.b0 = biases;

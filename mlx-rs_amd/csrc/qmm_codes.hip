@@ -1,4 +1,4 @@
-// Tiled quantized product on raw codes: activations in bfloat16, float16 or float32, groups of 32, 64 or 128, any number of
+// Tiled quantized product on raw codes: activations in bfloat16 or float16, groups of 32, 64 or 128, any number of
 // output columns.
 //
 // Contract: mlx_quantized_matmul / mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:91-122,160-230).
@@ -7,7 +7,8 @@
 // bf16 and in f16, so the matrix cores multiply the activations with raw codes and nothing is rounded on the way in:
 //   bf16  x as it is; 4-bit codes as 128 + q (one and-or per pair), the 128 taken back through the bias term
 //   f16   x as it is, codes in f16 (v_mfma_f32_32x32x16_f16)
-//   f32   x as three bf16 pieces of 8 significant bits each (an exact split), three products per code operand
+// float32 does not come here: the code and bias terms of a group cancel to about an eighth, which costs two of its bits
+// (error against 64 bits 3.3e-7 to 5.7e-7, a wave per output element 1.0e-7 to 1.3e-7, over 1 to 1000 rows).
 // The fp32 sums of a group are scaled once, when the group ends.  The bias term sum_g b_g (sum_c x_c) is a product of
 // its own over the groups: the group sums of x (fp32, split into three bf16 pieces) against the biases (three pieces
 // as well), eight K slots a group (xh bh, xm bh, xl bh, xh bm, xm bm, xh bl: every product down to 2^-24), which the
@@ -40,7 +41,6 @@ typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
 template <int DT> struct ElemOf;
 template <> struct ElemOf<0> { typedef uint16_t type; };
 template <> struct ElemOf<1> { typedef _Float16 type; };
-template <> struct ElemOf<2> { typedef float type; };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void *base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
@@ -87,8 +87,7 @@ struct RowStage {
   u32x4_t v[P][NA];
 };
 
-constexpr bool paired_order(int dt, int bits) { return bits == 4 && dt != 2; }  // 8-blocks as (0,4)(1,5)(2,6)(3,7)
-constexpr int n_parts(int dt) { return dt == 2 ? 3 : 1; }
+constexpr bool paired_order(int bits) { return bits == 4; }  // 8-blocks as (0,4)(1,5)(2,6)(3,7)
 constexpr int padded_groups(int G) { return (G + 15) / 16 * 16; }  // the bias product runs an even number of steps of eight groups
 
 __device__ __forceinline__ uint32_t f16_minus_1024(uint32_t v) {  // two halves 1024 + q -> q: exact
@@ -107,10 +106,7 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n_octets) return;  // whole groups leave together
   float v[8];
-  if constexpr (DT == 2) {
-    const float4 lo = reinterpret_cast<const float4 *>(x)[2 * i], hi = reinterpret_cast<const float4 *>(x)[2 * i + 1];
-    v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
-  } else {
+  {
     const uint4 w = reinterpret_cast<const uint4 *>(x)[i];
     const uint32_t u[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
@@ -161,19 +157,18 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf
 // A step takes one 32 x 32 sub-tile after the other: its four multiplies follow each other in one accumulator, and the
 // scaled addition of the sub-tile before it (16 fma) and the unpacking of the next step's codes (9 to 11 instructions a
 // multiply) run between them, which is as much vector work as fits beside the matrix cores.
-// What bounds it (777 x 4096 x 4096, f16, 8-bit; 26 GFLOP): 62 us for the call = 420 TFLOP/s, 50 times the plain kernel's
+// What bounds it (777 x 4096 x 4096, f16, 8-bit; 26 GFLOP): 58 us for the call = 450 TFLOP/s, 50 times the plain kernel's
 // 3160 us; the matrix cores alone would take 18.  Taken apart at one block a CU (cycles per 64 K values of 128 x 32 a
 // wave, 512 of them matrix work): multiplies and barriers 575, with the vector work 640, with the reads of LDS 840, with
 // the loads 1350.  The loads cost their line visits: a wave's codes sit in 32 rows.
 // KW > 1: the block's waves form KW groups that share K among them, each with LDS buffers of its own; their sums meet in
 // LDS at the end, added in group order.  For launches that give a CU one block or less.
-// DT: 0 bf16, 1 f16, 2 f32.  G32: groups of 32; otherwise a group is one or two steps (scale_shift).
+// DT: 0 bf16, 1 f16.  G32: groups of 32; otherwise a group is one or two steps (scale_shift).
 template <int DT, int BITS, bool G32, bool GLU, int MS, int NT, int WN, int KW>
 __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2, 4))) void qmm_codes_kernel(
     CodesArgs a, const uint32_t *__restrict__ lists, int n_mtiles, int n_experts, int n_ntiles, int scale_shift) {
   static_assert(!GLU || NT == 2, "a gate tile and its up tile");
   typedef typename ElemOf<DT>::type T;
-  constexpr int NP = n_parts(DT);
   constexpr int BM = 32 * MS;
   constexpr int NI = 32 * WN * (GLU ? 1 : NT);  // distinct output columns per block
   constexpr int NA = BM * 8 / (64 * WN);     // 16-byte activation loads per thread, piece and step
@@ -182,7 +177,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   constexpr int NS = G32 ? 2 : 1;            // scaled additions per sub-tile and step
   constexpr bool SPLIT = BITS == 8 || G32;   // which K values a multiply takes: see chunk below
   constexpr float kOffset = BITS == 4 && DT == 0 ? 128.0f : 0.0f;  // the codes are multiplied as offset + q
-  constexpr int A_SZ = BM * kRow, BUF = NP * A_SZ;                 // 16-byte units
+  constexpr int A_SZ = BM * kRow, BUF = A_SZ;                      // 16-byte units
   static_assert(BM % RS == 0, "whole loads");
 
   // block -> (M tile, N tile).  Ids are dealt round-robin over the 8 XCDs.  Dense: an XCD takes every eighth N tile
@@ -396,24 +391,9 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
 
   // ---- the product of the codes
   {
-    constexpr int XP = DT == 2 ? 2 : 1;  // 16-byte pieces of eight values
-    typedef RowStage<XP, NA> StageA;
+    typedef RowStage<1, NA> StageA;
     auto put_a = [&](u32x4_t *to, const StageA &R, int i) __attribute__((always_inline)) {
-      if constexpr (DT == 2) {
-        u32x4_t h, m, l;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const Pieces a = split3(__uint_as_float(R.v[q >> 1][i][2 * (q & 1)])), b = split3(__uint_as_float(R.v[q >> 1][i][2 * (q & 1) + 1]));
-          h[q] = a.h | b.h << 16;
-          m[q] = a.m | b.m << 16;
-          l[q] = a.l | b.l << 16;
-        }
-        to[0] = h;
-        to[A_SZ] = m;
-        to[2 * A_SZ] = l;
-      } else {
-        *to = R.v[0][i];
-      }
+      *to = R.v[0][i];
     };
     struct StageB {
       u32x4_t q[NT][NQ];
@@ -428,7 +408,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     };
     auto load_a = [&](int ks, bool real, StageA &R) __attribute__((always_inline)) {
 #pragma unroll
-      for (int p = 0; p < XP; ++p)
+      for (int p = 0; p < 1; ++p)
 #pragma unroll
         for (int i = 0; i < NA; ++i)
           R.v[p][i] = __builtin_amdgcn_raw_buffer_load_b128(xr, KW == 1 || real ? x_voff[i] : kOutside, ks * (kStep * (uint32_t)sizeof(T)) + 16 * p, 0);
@@ -452,7 +432,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
           }
         }
       }
-          if constexpr (BITS == 4 && DT != 2) {
+          if constexpr (BITS == 4) {
             const uint32_t w = R.q[t][0][h];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -474,15 +454,9 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               uint32_t c0, c1;  // codes 2 i, 2 i + 1
-              if constexpr (BITS == 4) {
-                const uint32_t w = R.q[t][0][h];
-                c0 = ((w & 0x0f0f0f0fu) >> (8 * i)) & 0xffu;
-                c1 = (((w >> 4) & 0x0f0f0f0fu) >> (8 * i)) & 0xffu;
-              } else {
-                const uint32_t w = R.q[t][h >> 1][2 * (h & 1) + (i >> 1)];
-                c0 = (w >> (16 * (i & 1))) & 0xffu;
-                c1 = (w >> (16 * (i & 1) + 8)) & 0xffu;
-              }
+              const uint32_t w = R.q[t][h >> 1][2 * (h & 1) + (i >> 1)];
+              c0 = (w >> (16 * (i & 1))) & 0xffu;
+              c1 = (w >> (16 * (i & 1) + 8)) & 0xffu;
               o.v[t][h][i] = __builtin_amdgcn_perm(__float_as_uint((float)c1), __float_as_uint((float)c0), 0x07060302u);
             }
           }
@@ -524,21 +498,19 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
         for (int i = 0; i < NS; ++i)
           step_s[d][t][i] = as_f32(*reinterpret_cast<const T *>(s_at[t] + ((G32 ? 2 * ks + i : ks >> scale_shift) - gw) * (int)sizeof(T)));
     };
-    auto body = [&](const u32x4_t (&av)[4][NP], const Operand &o, int d, int m, int t) __attribute__((always_inline)) {
+    auto body = [&](const u32x4_t (&av)[4][1], const Operand &o, int d, int m, int t) __attribute__((always_inline)) {
       const int tile = m * NT + t;
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
         const int which = ((d * MS * NT + tile) * NS + i) & 1;
 #pragma unroll
         for (int h = 4 / NS * i; h < 4 / NS * (i + 1); ++h)
-#pragma unroll
-          for (int p = 0; p < NP; ++p)
-            acc[which] = mfma<DT>(av[h][p], o.v[t][h], p == 0 && h == 4 / NS * i ? zero : acc[which]);
+          acc[which] = mfma<DT>(av[h][0], o.v[t][h], h == 4 / NS * i ? zero : acc[which]);
         acc_s[which] = step_s[d][t][i];
         add_scaled(which ^ 1, i > 0 ? tile : tile > 0 ? tile - 1 : MS * NT - 1);
       }
     };
-    pass(K / kStep, std::integral_constant<int, NP>{}, StageA{}, StageB{}, load_a, put_a, load_b, unpack, begin, with_split<SPLIT>(body),
+    pass(K / kStep, std::integral_constant<int, 1>{}, StageA{}, StageB{}, load_a, put_a, load_b, unpack, begin, with_split<SPLIT>(body),
          (win >> (G32 ? 1 : 0)) << scale_shift, window);
     add_scaled(1, MS * NT - 1);  // an even number of steps ends in accumulator 1
   }
@@ -618,7 +590,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
         for (int i = 0; i < (GLU ? 2 : 1); ++i) {
           const int tt = GLU ? i : t;
           const int64_t wrow = ebase + w_row[tt];
-          v[i] = plain_element<BITS, T>(xs, paired_order(DT, BITS), (GLU && i ? a.w1 : a.w0) + wrow * (row_bytes / 4),
+          v[i] = plain_element<BITS, T>(xs, paired_order(BITS), (GLU && i ? a.w1 : a.w0) + wrow * (row_bytes / 4),
                                         static_cast<const T *>(GLU && i ? a.s1 : a.s0) + wrow * G,
                                         static_cast<const T *>(GLU && i ? a.b1 : a.b0) + wrow * G, K, K / G);
         }
@@ -650,7 +622,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
 }
 
 size_t codes_copy_bytes(int dt, int bits, int64_t rows, int K) {
-  return paired_order(dt, bits) ? (size_t)rows * K * 2 : 0;
+  return paired_order(bits) ? (size_t)rows * K * 2 : 0;
 }
 size_t codes_sums_bytes(int64_t rows, int K, int group) { return (size_t)rows * padded_groups(K / group) * kSlots * 2; }
 
@@ -662,14 +634,14 @@ hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, in
   const int ll = group == 32 ? 2 : (group == 64 ? 3 : 4), row = padded_groups(K / group) * kSlots;
   if (dt == 0) prepare_rows_kernel<0><<<grid, 256, 0, st>>>(static_cast<const uint16_t *>(x), n, K / 8, ll, copy, sums, row);
   else if (dt == 1) prepare_rows_kernel<1><<<grid, 256, 0, st>>>(static_cast<const _Float16 *>(x), n, K / 8, ll, copy, sums, row);
-  else prepare_rows_kernel<2><<<grid, 256, 0, st>>>(static_cast<const float *>(x), n, K / 8, ll, copy, sums, row);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
 template <int DT, int BITS, bool G32, bool GLU, int MS, int NT, int WN, int KW>
 static hipError_t start_codes(const CodesArgs &a, int scale_shift, const uint32_t *lists, int cap256, int n_experts, hipStream_t st) {
   constexpr int NI = 32 * WN * (GLU ? 1 : NT), BM = 32 * MS;
-  constexpr size_t bufs = (size_t)2 * KW * n_parts(DT) * BM * kRow * 16 + WN * KW * NT * 32 * 48, sums = KW > 1 ? (size_t)BM * 32 * WN * NT * 4 : 0;
+  constexpr size_t bufs = (size_t)2 * KW * BM * kRow * 16 + WN * KW * NT * 32 * 48, sums = KW > 1 ? (size_t)BM * 32 * WN * NT * 4 : 0;
   constexpr size_t most = bufs > sums ? bufs : sums, lds = most > kLdsAtLeast ? most : kLdsAtLeast;
   static_assert(lds <= 160 * 1024, "more LDS than a CU has");
   const int n_ntiles = (a.N + NI - 1) / NI;
@@ -694,19 +666,13 @@ static hipError_t start_codes(const CodesArgs &a, int scale_shift, const uint32_
 //   64 x 128:                           41.5 / 42.4 / 46.7 / 31.0 / 45.6 / 66.7  (several blocks a CU overlap as K groups do)
 // Between one and two 32 x 64 tiles a CU the two are as fast with f16 and K = 4096; bf16, 4-bit, 32 x 64 / 64 x 128:
 // (200, 4096, 2048) 32.0 / 24.8, (200, 4096, 4096) 39.9 / 37.4, (1000, 1024, 1024) 29.7 / 21.8, (400, 2048, 768) 19.7 / 14.7.
-// (128 x 128 tiles: 65.1 / 67.0 / 70.2 / 45.9 / 69.3 / 76.0.)  f32 multiplies three times as much and holds three times
-// the rows in LDS: 32 x 64 with two groups up to 320 tiles, then 32 x 256 (1000, 4096, 4096: 147 against 164 for 64 x 128).
+// (128 x 128 tiles: 65.1 / 67.0 / 70.2 / 45.9 / 69.3 / 76.0.)
 template <int DT, int BITS, bool G32>
 static hipError_t start_dense(const CodesArgs &a, int scale_shift, hipStream_t st) {
   auto tiles = [&](int rows, int cols) { return (a.M + rows - 1) / rows * ((a.N + cols - 1) / cols); };
-  if constexpr (DT == 2) {
-    if (tiles(32, 64) <= 320) return start_codes<DT, BITS, G32, false, 1, 1, 2, 2>(a, scale_shift, nullptr, 0, 0, st);
-    return start_codes<DT, BITS, G32, false, 1, 2, 4, 1>(a, scale_shift, nullptr, 0, 0, st);
-  } else {
-    if (tiles(32, 64) <= 256) return start_codes<DT, BITS, G32, false, 1, 1, 2, 4>(a, scale_shift, nullptr, 0, 0, st);
-    if (tiles(64, 128) <= 256) return start_codes<DT, BITS, G32, false, 2, 1, 4, 2>(a, scale_shift, nullptr, 0, 0, st);
-    return start_codes<DT, BITS, G32, false, 2, 1, 4, 1>(a, scale_shift, nullptr, 0, 0, st);
-  }
+  if (tiles(32, 64) <= 256) return start_codes<DT, BITS, G32, false, 1, 1, 2, 4>(a, scale_shift, nullptr, 0, 0, st);
+  if (tiles(64, 128) <= 256) return start_codes<DT, BITS, G32, false, 2, 1, 4, 2>(a, scale_shift, nullptr, 0, 0, st);
+  return start_codes<DT, BITS, G32, false, 2, 1, 4, 1>(a, scale_shift, nullptr, 0, 0, st);
 }
 
 // The M-tile lists of a grouped product (see tile_list) in one launch, in blocks of 64 rows x 128 columns.  Measured on
@@ -737,7 +703,7 @@ hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int d
   };
   if (dt == 0) return with_bits(std::integral_constant<int, 0>{});
   if (dt == 1) return with_bits(std::integral_constant<int, 1>{});
-  return with_bits(std::integral_constant<int, 2>{});
+  return hipErrorInvalidValue;
 }
 
 }  // namespace mi_moe

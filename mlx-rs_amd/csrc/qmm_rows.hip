@@ -1,5 +1,5 @@
 // Quantized products of a few rows (a decode batch's linear layer; short expert segments with groups of 32 or 128):
-// activations in bfloat16, float16 or float32, groups of 32, 64 or 128.
+// activations in bfloat16 or float16, groups of 32, 64 or 128.
 //
 // Contract: mlx_quantized_matmul / mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:91-122,160-230);
 // with GLU also nn::silu and multiply (nn/activation.rs:142-144,876-880).
@@ -25,7 +25,6 @@ typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
 template <int DT> struct ElemOf;
 template <> struct ElemOf<0> { typedef uint16_t type; };
 template <> struct ElemOf<1> { typedef _Float16 type; };
-template <> struct ElemOf<2> { typedef float type; };
 
 template <class T> __device__ __forceinline__ T rounded(float v) { return (T)v; }
 template <> __device__ __forceinline__ uint16_t rounded<uint16_t>(float v) { return (uint16_t)(cvt_pk_bf16(v, 0.f) & 0xffffu); }
@@ -44,19 +43,17 @@ __device__ __forceinline__ uint32_t f16_minus_1024(uint32_t v) {  // two halves 
   return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) - half2_t{(_Float16)1024, (_Float16)1024});
 }
 
-constexpr int n_parts(int dt) { return dt == 2 ? 3 : 1; }  // f32 rows: three bf16 pieces (exact), as in qmm_codes.hip
-
-// LDS of a launch: token rows of sk values (tt of them, NP pieces each), 64 zero bytes, the sums of x over each group and
+// LDS of a launch: token rows of sk values (tt of them), 64 zero bytes, the sums of x over each group and
 // token slot, the (scale, bias) pairs of the block's weight rows, and the partial sums of a shared K.
 struct RowsLds {
   int x_stride, zeros, sums, pairs, pair_row, parts, bytes;
   __host__ __device__ RowsLds(int dt, int group, int nm, int kw, int K, int sk, int tt) {
-    const int np = n_parts(dt), elem = dt == 2 ? 4 : 2, nw = 4 / kw;
-    x_stride = 2 * np * sk + 16;
+    const int nw = 4 / kw;
+    x_stride = 2 * sk + 16;
     zeros = tt * x_stride;
     sums = zeros + 64;
     pairs = sums + sk / group * kTokens * 4;
-    pair_row = (K / group) * 2 * elem + 4;  // (an odd number of words: 16 rows read one group each without a conflict)
+    pair_row = (K / group) * 4 + 4;  // (an odd number of words: 16 rows read one group each without a conflict)
     parts = pairs + ((nw * nm * 16 * pair_row + 15) & ~15);
     bytes = parts + (kw > 1 ? kw * nw * nm * 64 * 16 : 0);
   }
@@ -72,18 +69,17 @@ struct RowsLds {
 //   8-bit: multiply t takes the t-th half of every quarter (groups >= 64), or after two swaps 32 consecutive codes.
 // What bounds it: the bytes of the weights and, for one row of a small matrix, the latency of its few dependent steps.
 // Measured, 4096 x 4096, us of the kernel at 1 / 4 / 8 / 16 rows (the plain kernel, a wave per output element: f16 4-bit
-// 6.7 / 17.5 / 30.2 / 55.6, f32 8-bit 9.8 / 23.1 / 41.2 / 77.3): f16 4-bit 7.5 / 9.8 / 13.0 / 18.3, bf16 groups of 32
-// 8.5 / 10.9 / 14.4 / 20.7, f32 8-bit 10.8 / 14.9 / 20.5 / 29.5.  Every block stages all rows: that is what grows.
+// 6.7 / 17.5 / 30.2 / 55.6): f16 4-bit 7.5 / 9.8 / 13.0 / 18.3, bf16 groups of 32 8.5 / 10.9 / 14.4 / 20.7.  Every block
+// stages all rows: that is what grows.
 template <int DT, int BITS, int GROUP, bool GLU, int KW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void qmm_rows_kernel(RowsArgs a, int tt, int sk) {
   typedef typename ElemOf<DT>::type T;
-  constexpr int NP = n_parts(DT);
   constexpr int NM = GLU ? 2 : 1;
   constexpr int NW = 4 / KW;
   constexpr int CH = BITS == 4 ? 128 : 64;     // codes per chunk and row
   constexpr int MUL = CH / 32;                 // multiplies per chunk
   constexpr float kOffset = BITS == 4 && DT == 0 ? 128.0f : 0.0f;
-  constexpr bool PAIRED = BITS == 4 && DT != 2;  // token rows as 8-blocks (0,4)(1,5)(2,6)(3,7), the order of the unpacking
+  constexpr bool PAIRED = BITS == 4;  // token rows as 8-blocks (0,4)(1,5)(2,6)(3,7), the order of the unpacking
 
   int e = 0, cnt = (int)a.M;
   int64_t r0 = 0;
@@ -187,29 +183,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
         const T *const xr = static_cast<const T *>(a.x) + src * K + s0 + piece * 8;
         unsigned char *const to = lds + row * L.x_stride + piece * 16;
         float v[8];
-        if constexpr (DT == 2) {
-          const float4 lo = reinterpret_cast<const float4 *>(xr)[0], hi = reinterpret_cast<const float4 *>(xr)[1];
-          v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
-          uint32_t h[4], m[4], l[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            uint32_t p[2][3];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {  // truncated pieces: exact, nothing overflows
-              const float f = v[2 * j + i];
-              p[i][0] = __float_as_uint(f) & 0xffff0000u;
-              const float f1 = f - __uint_as_float(p[i][0]);
-              p[i][1] = __float_as_uint(f1) & 0xffff0000u;
-              p[i][2] = __float_as_uint(f1 - __uint_as_float(p[i][1]));
-            }
-            h[j] = p[0][0] >> 16 | p[1][0];
-            m[j] = p[0][1] >> 16 | p[1][1];
-            l[j] = p[0][2] >> 16 | (p[1][2] & 0xffff0000u);
-          }
-          *reinterpret_cast<uint4 *>(to) = make_uint4(h[0], h[1], h[2], h[3]);
-          *reinterpret_cast<uint4 *>(to + 2 * sk) = make_uint4(m[0], m[1], m[2], m[3]);
-          *reinterpret_cast<uint4 *>(to + 4 * sk) = make_uint4(l[0], l[1], l[2], l[3]);
-        } else {
+        {
           const uint4 w = *reinterpret_cast<const uint4 *>(xr);
           const uint32_t u[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
@@ -289,10 +263,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
               const int k = BITS == 4 ? 32 * s + 8 * kb : (GROUP == 32 ? 32 * s + 16 * (kb & 1) + 8 * (kb >> 1) : 16 * kb + 8 * s);
               const bool first = GROUP == 32 || (GROUP == 64 ? (BITS == 4 ? s % 2 == 0 : s == 0) : s == 0);
               const bool last = GROUP == 32 || (GROUP == 64 ? (BITS == 4 ? s % 2 == 1 : s == 1) : s == MUL - 1);
-              u32x4_t av[NP];
-#pragma unroll
-              for (int p = 0; p < NP; ++p)
-                av[p] = *reinterpret_cast<const u32x4_t *>(xl + x_step * ((ch_slab * CH + k) * 2 + p * 2 * sk));
+              const u32x4_t av = *reinterpret_cast<const u32x4_t *>(xl + x_step * ((ch_slab * CH + k) * 2));
 #pragma unroll
               for (int m = 0; m < NM; ++m) {
                 u32x4_t bv;
@@ -311,19 +282,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
 #pragma unroll
                   for (int i = 0; i < 4; ++i) {
                     uint32_t c0, c1;
-                    if constexpr (BITS == 4) {
-                      c0 = ((q[m][s] & 0x0f0f0f0fu) >> (8 * i)) & 0xffu;
-                      c1 = (((q[m][s] >> 4) & 0x0f0f0f0fu) >> (8 * i)) & 0xffu;
-                    } else {
-                      const uint32_t w = q[m][2 * s + (i >> 1)];
-                      c0 = (w >> (16 * (i & 1))) & 0xffu;
-                      c1 = (w >> (16 * (i & 1) + 8)) & 0xffu;
-                    }
+                    const uint32_t w = q[m][2 * s + (i >> 1)];
+                    c0 = (w >> (16 * (i & 1))) & 0xffu;
+                    c1 = (w >> (16 * (i & 1) + 8)) & 0xffu;
                     bv[i] = __builtin_amdgcn_perm(__float_as_uint((float)c1), __float_as_uint((float)c0), 0x07060302u);
                   }
                 }
-#pragma unroll
-                for (int p = 0; p < NP; ++p) acc[m] = mfma<DT>(av[p], bv, first && p == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[m]);
+                acc[m] = mfma<DT>(av, bv, first ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[m]);
               }
               if (last || (GROUP == 128 && BITS == 8 && s == MUL - 1)) {  // (8-bit groups of 128: half a group, same scale)
                 const int gs = GROUP == 128 && BITS == 8 ? ch : (ch * CH + 32 * s) / GROUP;
@@ -333,16 +298,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
                 const bool with_bias = !(GROUP == 128 && BITS == 8) || (ch & 1) == 0;  // (once per group)
 #pragma unroll
                 for (int m = 0; m < NM; ++m) {
-                  float sc, bi;
-                  if constexpr (sizeof(T) == 4) {
-                    const float *const p = reinterpret_cast<const float *>(my_pairs + m * 16 * L.pair_row + g * 8);
-                    sc = p[0];
-                    bi = p[1];
-                  } else {
-                    const uint32_t p = *reinterpret_cast<const uint32_t *>(my_pairs + m * 16 * L.pair_row + g * 4);
-                    sc = as_f32(__builtin_bit_cast(T, (uint16_t)(p & 0xffffu)));
-                    bi = as_f32(__builtin_bit_cast(T, (uint16_t)(p >> 16)));
-                  }
+                  const uint32_t p = *reinterpret_cast<const uint32_t *>(my_pairs + m * 16 * L.pair_row + g * 4);
+                  const float sc = as_f32(__builtin_bit_cast(T, (uint16_t)(p & 0xffffu)));
+                  float bi = as_f32(__builtin_bit_cast(T, (uint16_t)(p >> 16)));
                   if constexpr (kOffset != 0.f) bi = __builtin_fmaf(-kOffset, sc, bi);
                   if (!with_bias) bi = 0.f;
                   tot[m][0] = __builtin_fmaf(sc, acc[m][0], __builtin_fmaf(bi, xs.x, tot[m][0]));
@@ -451,7 +409,7 @@ static RowsCut cut_rows(const RowsArgs &a, int group, int bits, int dt, bool glu
 }
 
 bool qmm_rows_applies(const RowsArgs &a, int group, int bits, int dt, bool glu) {
-  return bits != 2 && a.K % (bits == 4 ? 128 : 64) == 0 && a.K % group == 0 && (int64_t)a.N * a.K < (int64_t)1 << 31 &&
+  return bits != 2 && dt != 2 && a.K % (bits == 4 ? 128 : 64) == 0 && a.K % group == 0 && (int64_t)a.N * a.K < (int64_t)1 << 31 &&
          cut_rows(a, group, bits, dt, glu).kw > 0;
 }
 
@@ -481,7 +439,7 @@ hipError_t launch_qmm_rows(const RowsArgs &a, int group, int bits, int dt, bool 
   if (glu && dt != 0) return hipErrorInvalidValue;
   if (dt == 0) return with_bits(std::integral_constant<int, 0>{});
   if (dt == 1) return with_bits(std::integral_constant<int, 1>{});
-  return with_bits(std::integral_constant<int, 2>{});
+  return hipErrorInvalidValue;
 }
 
 }  // namespace mi_moe
