@@ -248,6 +248,74 @@ __global__ __launch_bounds__(256) void qmm_plain_t_kernel(const T *__restrict__ 
   if (lane == 0) Elem<T>::store(y + dr * N + n, acc);
 }
 
+// The same product of dense float32 rows, 4- and 8-bit codes, R rows by C columns a wave: a word of codes is read and
+// dequantised once for R rows, a value of x once for C columns.  Every sum runs over the same lanes in the same order as
+// in qmm_plain_t_kernel, so the bits are the same.  (The matrix cores on raw codes lose two bits: see qmm_codes.hip.)
+// Sums meet by halving: at lane distance d each lane hands the half of its sums that its partner keeps; an addition
+// commutes, so the tree of a sum does not depend on the lane that holds it.
+// What bounds it: the vector unit, an fma per value and sum (430 us of it at 1000 x 4096 x 4096) beside the loads of x.
+// us of the call, a wave per output element / here: 1000 x 4096 x 4096 4-bit 2759 / 1007, 8-bit 3591 / 1387; 100 x 4096 x
+// 4096 305 / 103; 30 x 4096 x 2304 70.6 / 18.9; 300 x 1024 x 1024 80.9 / 20.5; 16 and 8 x 4096 x 4096 8-bit 80.7 and 41.5 /
+// 41.2 and 21.3.
+template <int BITS, int R, int C>
+__global__ __launch_bounds__(256) void qmm_plain_f32_kernel(const float *__restrict__ x, const uint32_t *__restrict__ w,
+                                                            const float *__restrict__ scales, const float *__restrict__ biases,
+                                                            int64_t rows, int N, int K, int group, float *__restrict__ y) {
+  constexpr int CPW = 32 / BITS, V = R * C;
+  const int64_t r0 = (int64_t)blockIdx.x * R;
+  const int n0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * C;
+  if (n0 >= N) return;
+  const int lane = lane_id(), wpr = K / CPW, gpr = K / group;
+  const float *xr[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) xr[i] = x + (r0 + i < rows ? r0 + i : rows - 1) * K;  // (rows and columns outside: the last one again, not stored)
+  float acc[V] = {};
+  for (int wi = lane; wi < wpr; wi += kWave) {
+    const int k0 = wi * CPW, g = k0 / group;
+    float4 xv[R][CPW / 4];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int p = 0; p < CPW / 4; ++p) xv[i][p] = reinterpret_cast<const float4 *>(xr[i] + k0)[p];
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const int64_t n = n0 + j < N ? n0 + j : N - 1;
+      const uint32_t word = w[n * wpr + wi];
+      const float sc = scales[n * gpr + g], bi = biases[n * gpr + g];
+#pragma unroll
+      for (int c = 0; c < CPW; ++c) {
+        const float wv = __builtin_fmaf(sc, (float)((word >> (c * BITS)) & ((1u << BITS) - 1u)), bi);
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+          const float4 q = xv[i][c / 4];
+          acc[i * C + j] = __builtin_fmaf(c % 4 == 0 ? q.x : c % 4 == 1 ? q.y : c % 4 == 2 ? q.z : q.w, wv, acc[i * C + j]);
+        }
+      }
+    }
+  }
+  int held = V, first = 0;  // this lane holds sums first .. first + held - 1
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    if (held > 1) {
+      held /= 2;
+      const bool upper = lane & d;
+      if (upper) first += held;
+#pragma unroll
+      for (int i = 0; i < V / 2; ++i) {
+        if (i < held) {
+          const float lo = acc[i], hi = acc[i + held], away = upper ? lo : hi;
+          acc[i] = (upper ? hi : lo) + __shfl_xor(away, d, kWave);
+        }
+      }
+    } else {
+      acc[0] += __shfl_xor(acc[0], d, kWave);
+    }
+  }
+  const int64_t row = r0 + first / C;
+  const int n = n0 + first % C;
+  if (lane < V && row < rows && n < N) y[row * N + n] = acc[0];
+}
+
 // transpose = false: w [E, K, N*bits/32], scales / biases [E, K, N/group] (K x N matrices quantised
 // along N).  One thread per packed word of an output row, fp32 accumulation in k order.
 template <class T, int BITS>
@@ -308,6 +376,25 @@ static hipError_t launch_plain_t(const void *x, const uint32_t *w, const void *s
   return hipGetLastError();
 }
 
+template <int BITS>
+static hipError_t launch_plain_f32(const float *x, const uint32_t *w, const float *s, const float *b, int64_t rows, int N, int K,
+                                   int group, float *y, hipStream_t st) {
+  auto run = [&](auto r, auto c) {
+    constexpr int R = decltype(r)::value, C = decltype(c)::value;
+    const dim3 grid((unsigned)((rows + R - 1) / R), (unsigned)((N + 4 * C - 1) / (4 * C)));
+    qmm_plain_f32_kernel<BITS, R, C><<<grid, 256, 0, st>>>(x, w, s, b, rows, N, K, group, y);
+    return hipGetLastError();
+  };
+  auto with_rows = [&](auto c) {
+    if (rows <= 2) return run(std::integral_constant<int, 2>{}, c);
+    if (rows <= 4) return run(std::integral_constant<int, 4>{}, c);
+    return run(std::integral_constant<int, 8>{}, c);
+  };
+  // four columns a wave read x a fourth as often; where that leaves a SIMD fewer than four waves, one column
+  if ((rows + 7) / 8 * N >= 4 * 4096) return with_rows(std::integral_constant<int, 4>{});
+  return with_rows(std::integral_constant<int, 1>{});
+}
+
 // dt: 0 bf16, 1 fp16, 2 fp32.  rows = n_idx * M output rows (at most 2^31 - 1: they are the grid's x extent).
 hipError_t launch_qmm_plain(const void *x, const uint32_t *w, const void *scales, const void *biases,
                             const uint32_t *lhs, const uint32_t *rhs, const uint32_t *rhs_map,
@@ -316,6 +403,11 @@ hipError_t launch_qmm_plain(const void *x, const uint32_t *w, const void *scales
   if (rows == 0) return hipSuccess;
   if (transpose && (N + 3) / 4 > 65535) return hipErrorInvalidValue;  // the grid's y extent
   const PlainMaps mp{lhs, rhs, rhs_map, dst_map, n_lhs, n_rhs};
+  if (dt == 2 && transpose && bits != 2 && rows > 1 && !lhs && !rhs && !dst_map && (reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
+    const float *xs = static_cast<const float *>(x), *ss = static_cast<const float *>(scales), *bs = static_cast<const float *>(biases);
+    if (bits == 4) return launch_plain_f32<4>(xs, w, ss, bs, rows, N, K, group, static_cast<float *>(y), st);
+    return launch_plain_f32<8>(xs, w, ss, bs, rows, N, K, group, static_cast<float *>(y), st);
+  }
   if (dt == 0) return launch_plain_t<uint16_t>(x, w, scales, biases, mp, rows, M, N, K, group, bits, y, transpose, st);
   if (dt == 1) return launch_plain_t<_Float16>(x, w, scales, biases, mp, rows, M, N, K, group, bits, y, transpose, st);
   return launch_plain_t<float>(x, w, scales, biases, mp, rows, M, N, K, group, bits, y, transpose, st);
