@@ -74,8 +74,8 @@ typedef struct {
   int32_t n_experts;    /* E, 1..512 */
   int32_t top_k;        /* k, 1..min(E,32) */
   int32_t intermediate; /* I, multiple of group_size */
-  int32_t bits;         /* 4 or 8 (tuned kernels); 2 runs on the plain products */
-  int32_t group_size;   /* 64 (tuned kernels); 32 and 128 run on the plain products */
+  int32_t bits;         /* 4 or 8 (matrix cores); 2 runs on the plain products */
+  int32_t group_size;   /* 64, or 32 / 128 (the products on raw codes) */
   int32_t score_mode;   /* mi_moe_score_mode */
 } mi_moe_config;
 
