@@ -464,12 +464,12 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     // The scales of this wave's rows pass through LDS a window at a time: a lane fetches 16 bytes of its row (half kb of
     // the window) one window ahead, and reads one value per group back.  One 2-byte load per group from a row each
     // touches as many lines as the codes themselves (measured: a quarter of the kernel's time).
-    // The fetch is aligned down to 4 bytes (with an odd number of 2-byte scales per row, every second row starts between
-    // two words): the window then gives up its last scale.
-    const int win = sizeof(T) == 2 && (G & 1) ? 8 : 2 * 16 / (int)sizeof(T);  // scales of a window
+    // The fetch is aligned down to 4 bytes.  Where a window can start between two words (an odd number of 2-byte scales
+    // per row, or per K group: groups of 128), the sixteenth scale would lie behind the fetch: windows of eight then.
+    const int first_group = (nk_share(K / kStep) * kg) * (G32 ? 2 : 1) >> scale_shift, share_groups = nk_share(K / kStep) * (G32 ? 2 : 1) >> scale_shift;
+    const int win = ((G | share_groups) & 1) ? 8 : 16;  // scales of a window
     constexpr int SROW = 32 + 16;                  // bytes per row of the window
     unsigned char *const swin = reinterpret_cast<unsigned char *>(lds_raw) + 2 * KW * BUF * 16 + wave_all * (NT * 32 * SROW);
-    const int first_group = (nk_share(K / kStep) * kg) * (G32 ? 2 : 1) >> scale_shift;
     u32x4_t swin_next[NT];
     auto load_window = [&](int g) __attribute__((always_inline)) {
 #pragma unroll

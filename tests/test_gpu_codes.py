@@ -49,6 +49,23 @@ def test_products_on_raw_codes(rows, n, k, bits, dtype, group):
         assert float((one.double() - ref[:1]).norm() / ref[:1].norm()) <= BOUND[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows,n,k", [(200, 4096, 4352), (200, 4096, 11008), (40, 2048, 8704)])
+def test_shares_of_k_of_an_odd_number_of_groups(rows, n, k, bits, dtype):
+    """Groups of 128 and K shared by two and by four groups of waves, each of 17, 43 and 17 groups: a share's scales start
+    between two words and are more than one fetch holds.  Each row within the bound, which one wrong group in 34 is not."""
+    import mlx_rs_amd as m
+    dt = getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(rows + n + k)
+    q, s, b = m.ops.quantize(torch.randn((n, k), generator=gen, device="cuda") * 0.02, 128, bits, dt)
+    x = torch.randn((rows, k), generator=gen, device="cuda").to(dt)
+    ref = product(x, q, s, b, 128, bits)
+    y = m.ops.quantized_linear(x, q, s, b, group_size=128, bits=bits)
+    err = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= BOUND[dtype], float(err.max())
+
+
 def test_large_float32_values_survive_the_split():
     """The three pieces are cut by truncation: the largest finite values do not overflow on the way."""
     import mlx_rs_amd as m
