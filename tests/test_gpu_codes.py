@@ -66,6 +66,33 @@ def test_shares_of_k_of_an_odd_number_of_groups(rows, n, k, bits, dtype):
     assert float(err.max()) <= BOUND[dtype], float(err.max())
 
 
+def off_by_one(t):
+    """The same values one element behind an aligned address."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    buf[1:] = t.reshape(-1)
+    return buf[1:].reshape(t.shape)
+
+
+@pytest.mark.parametrize("dtype,group", [("float16", 64), ("float16", 128), ("bfloat16", 32), ("bfloat16", 128)])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows", [7, 40, 300])
+def test_scales_between_two_words(rows, bits, dtype, group):
+    """Scales or biases that start two bytes behind a word: scales, which the kernels on raw codes read by words, send the product
+    to the plain kernel (as rows at such an address do); biases alone are fine in tiles."""
+    import mlx_rs_amd as m
+    dt = getattr(torch, dtype)
+    for n, k in ((48, 384), (37, 384)):
+        gen = torch.Generator(device="cuda").manual_seed(rows + n)
+        q, s, b = m.ops.quantize(torch.randn((n, k), generator=gen, device="cuda") * 0.02, group, bits, dt)
+        x = torch.randn((rows, k), generator=gen, device="cuda").to(dt)
+        run = lambda *a: m.ops.quantized_linear(*a, group_size=group, bits=bits)  # noqa: E731
+        plain = run(off_by_one(x), q, s, b)
+        assert torch.equal(run(x, q, off_by_one(s), b), plain)
+        ref = product(x, q, s, b, group, bits)
+        y = run(x, q, s, off_by_one(b))
+        assert float((y.double() - ref).norm() / ref.norm()) <= BOUND[dtype]
+
+
 def test_large_float32_values_survive_the_split():
     """The three pieces are cut by truncation: the largest finite values do not overflow on the way."""
     import mlx_rs_amd as m
