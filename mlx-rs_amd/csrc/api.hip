@@ -997,10 +997,12 @@ int mi_moe_quantized_matmul_workspace_size(int64_t M, int32_t K, int32_t bits, s
   return 0;
 } MI_CATCH("quantized_matmul_workspace_size")
 
-// What the products on raw codes take: transposed weights, bf16 or f16 (see qmm_codes.hip for f32), any group.  Their descriptors hold a 32-bit
-// size of one matrix.
-static bool codes_shape(int32_t dtype, int32_t transpose, int32_t bits, int32_t N, int32_t K) {
-  return transpose && dtype != MI_MOE_DTYPE_F32 && bits != 2 && K % 128 == 0 && (int64_t)N * K * bits / 8 < (int64_t)1 << 31 && (int64_t)N * K < (int64_t)1 << 33;
+// What the products on raw codes take: transposed weights, bf16 or f16 (see qmm_codes.hip for f32), any group.  Their descriptors
+// hold a 32-bit size of one matrix, and both kernels read scales a word or more at a time: an even number of them, so that no
+// word reaches behind the tensor (groups of 128 only: K / 128 and N both odd).
+static bool codes_shape(int32_t dtype, int32_t transpose, int32_t group_size, int32_t bits, int32_t N, int32_t K) {
+  return transpose && dtype != MI_MOE_DTYPE_F32 && bits != 2 && K % 128 == 0 && (int64_t)N * K * bits / 8 < (int64_t)1 << 31 && (int64_t)N * K < (int64_t)1 << 33 &&
+         (int64_t)N * (K / group_size) % 2 == 0;
 }
 
 // Which transposed dense products take the kernel of a few rows (nothing to prepare, one launch).  Measured, us of the kernels
@@ -1040,7 +1042,7 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
   if (M == 0) return 0;
   if (!x || !w || !scales || !biases || !y) return fail("quantized_matmul: x, w, scales, biases and y must be non-NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const bool tuned = tuned_shape(dtype, transpose, group_size, bits, N, K), codes = codes_shape(dtype, transpose, bits, N, K);
+  const bool tuned = tuned_shape(dtype, transpose, group_size, bits, N, K), codes = codes_shape(dtype, transpose, group_size, bits, N, K);
   size_t mt_words = 0;
   if (tuned) {
     if (!aligned16(x) || !aligned16(w) || !aligned16(scales) || !aligned16(biases) || !aligned16(y))

@@ -253,7 +253,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     int row = n0 + 32 * wave + lnp + (GLU ? 0 : 32 * WN * t);
     row = row < N ? row : N - 1;  // columns past the end repeat the last one (never stored)
     wr[t] = rsrc_of((up ? a.w1 : a.w0) + ebase * (row_bytes / 4), (uint32_t)N * row_bytes);
-    sr[t] = rsrc_of(static_cast<const T *>(up ? a.s1 : a.s0) + ebase * G, ((uint32_t)N * G * sizeof(T) + 3u) & ~3u);  // (read in words)
+    sr[t] = rsrc_of(static_cast<const T *>(up ? a.s1 : a.s0) + ebase * G, (uint32_t)N * G * sizeof(T));  // (read in words: the host takes an even number of them)
     br[t] = rsrc_of(static_cast<const T *>(up ? a.b1 : a.b0) + ebase * G, (uint32_t)N * G * sizeof(T));
     w_row[t] = row;
     w_voff[t] = (uint32_t)row * row_bytes + kb * 16;

@@ -131,8 +131,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
     for (int p = tid; p < total; p += 256) {
       const int tile = p / per_tile, q = p - tile * per_tile;  // tile = wn * NM + m
       const int m = tile % NM, row0 = (blockIdx.x * NW + tile / NM) * 16;
-      const __amdgpu_buffer_rsrc_t sr = rsrc_of(static_cast<const T *>(m ? a.s1 : a.s0) + ebase * G, ((uint32_t)N * G * sizeof(T) + 3u) & ~3u);
-      const __amdgpu_buffer_rsrc_t br = rsrc_of(static_cast<const T *>(m ? a.b1 : a.b0) + ebase * G, ((uint32_t)N * G * sizeof(T) + 3u) & ~3u);
+      const __amdgpu_buffer_rsrc_t sr = rsrc_of(static_cast<const T *>(m ? a.s1 : a.s0) + ebase * G, (uint32_t)N * G * sizeof(T));
+      const __amdgpu_buffer_rsrc_t br = rsrc_of(static_cast<const T *>(m ? a.b1 : a.b0) + ebase * G, (uint32_t)N * G * sizeof(T));
       const uint32_t off = ((uint32_t)row0 * G + q * PV) * sizeof(T);
       const u32x4_t sv = __builtin_amdgcn_raw_buffer_load_b128(sr, off, 0, 0), bv = __builtin_amdgcn_raw_buffer_load_b128(br, off, 0, 0);
       int row = q * PV / G, g = q * PV - row * G;

@@ -93,6 +93,21 @@ def test_scales_between_two_words(rows, bits, dtype, group):
         assert float((y.double() - ref).norm() / ref.norm()) <= BOUND[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows", [2, 40, 300])
+def test_an_odd_number_of_scales(rows, bits, dtype):
+    """37 x 3 scales: their last word reaches behind the tensor, so the plain kernel takes them (as it does rows that start between
+    two words)."""
+    import mlx_rs_amd as m
+    dt = getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    q, s, b = m.ops.quantize(torch.randn((37, 384), generator=gen, device="cuda") * 0.02, 128, bits, dt)
+    x = torch.randn((rows, 384), generator=gen, device="cuda").to(dt)
+    run = lambda v: m.ops.quantized_linear(v, q, s, b, group_size=128, bits=bits)  # noqa: E731
+    assert torch.equal(run(x), run(off_by_one(x)))
+
+
 def test_large_float32_values_survive_the_split():
     """The three pieces are cut by truncation: the largest finite values do not overflow on the way."""
     import mlx_rs_amd as m
