@@ -28,19 +28,31 @@ template <> struct Elem<float> {
   static __device__ __forceinline__ void store(float *p, float v) { *p = v; }
 };
 
-// Eight consecutive values of one element type: one 16-byte access (two for float).
+// Eight consecutive values of one element type: one 16-byte access (two for float).  No address needs more than the
+// alignment of its elements: global memory takes such accesses anywhere, and the compiler is told nothing else.
 template <class O>
 __device__ __forceinline__ void store8(O *p, const float (&v)[8]) {
   O o[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) Elem<O>::store(o + j, v[j]);
-  __builtin_memcpy(__builtin_assume_aligned(p, 16), o, sizeof o);
+  __builtin_memcpy(p, o, sizeof o);
 }
 // The codes of eight consecutive values: half a word, one word or two.
 template <int BITS> struct Codes8;
 template <> struct Codes8<2> { typedef uint16_t type; };
 template <> struct Codes8<4> { typedef uint32_t type; };
 template <> struct Codes8<8> { typedef uint64_t type; };
+// the codes of octet i: q is aligned for its words
+template <int BITS>
+__device__ __forceinline__ typename Codes8<BITS>::type load_codes(const uint32_t *q, int64_t i) {
+  typename Codes8<BITS>::type c;
+  __builtin_memcpy(&c, reinterpret_cast<const unsigned char *>(q) + i * BITS, BITS);
+  return c;
+}
+template <int BITS>
+__device__ __forceinline__ void store_codes(uint32_t *q, int64_t i, typename Codes8<BITS>::type c) {
+  __builtin_memcpy(reinterpret_cast<unsigned char *>(q) + i * BITS, &c, BITS);
+}
 
 // Groups are runs of the flat array (columns are a multiple of the group), so the matrix is one stream of
 // values.  A thread takes eight of them: two 16-byte loads, and the 4, 8 or 16 lanes of a group sit in one
@@ -49,15 +61,14 @@ template <> struct Codes8<8> { typedef uint64_t type; };
 // copy's rate (a thread per packed word, eight 4-byte loads 32 bytes apart: 474 us).
 template <class T, int BITS, int GROUP>
 __global__ __launch_bounds__(256) void quantize_kernel(const float *__restrict__ w, int64_t n_octets,
-                                                       typename Codes8<BITS>::type *__restrict__ q,
+                                                       uint32_t *__restrict__ q,
                                                        T *__restrict__ scales, T *__restrict__ biases) {
 #pragma clang fp contract(off)
   constexpr int LANES = GROUP / 8;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const bool on = i < n_octets;
-  const float4 *const src = reinterpret_cast<const float4 *>(w) + 2 * (on ? i : n_octets - 1);  // keep every lane in the exchanges
-  const float4 lo = src[0], hi = src[1];
-  const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  float v[8];
+  __builtin_memcpy(v, w + 8 * (on ? i : n_octets - 1), sizeof v);  // (keep every lane in the exchanges)
   float w_min = INFINITY, w_max = -INFINITY;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -92,7 +103,7 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float *__restrict__
     codes |= (typename Codes8<BITS>::type)((typename Codes8<BITS>::type)(uint32_t)c << (j * BITS));
   }
   if (on) {
-    q[i] = codes;
+    store_codes<BITS>(q, i, codes);
     if (i % LANES == 0) {  // the codes come from the fp32 scale and bias; these are cast afterwards
       Elem<T>::store(scales + i / LANES, scale);
       Elem<T>::store(biases + i / LANES, bias);
@@ -104,7 +115,7 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float *__restrict__
 // thread writes eight values with one or two 16-byte stores; bound by the bytes written.  Measured at
 // 98304 x 2048, 4-bit groups of 64 to bfloat16 (516 MB): 114 us = 4.5 TB/s (eight 2-byte stores a thread: 245 us).
 template <class T, class O, int BITS>
-__global__ __launch_bounds__(256) void dequantize_kernel(const typename Codes8<BITS>::type *__restrict__ q,
+__global__ __launch_bounds__(256) void dequantize_kernel(const uint32_t *__restrict__ q,
                                                          const T *__restrict__ scales,
                                                          const T *__restrict__ biases, int64_t n_octets,
                                                          int lanes_log2, O *__restrict__ out) {
@@ -112,7 +123,7 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const typename Codes8<B
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n_octets) return;
   const int64_t g = i >> lanes_log2;
-  const typename Codes8<BITS>::type codes = q[i];
+  const typename Codes8<BITS>::type codes = load_codes<BITS>(q, i);
   const float s = Elem<T>::load(scales + g), b = Elem<T>::load(biases + g);
   float v[8];
 #pragma unroll
@@ -124,11 +135,10 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const typename Codes8<B
 template <class T, int BITS>
 static void start_quantize(const float *w, int64_t n_octets, int group, uint32_t *q, void *s, void *b, hipStream_t st) {
   const unsigned grid = (unsigned)((n_octets + 255) / 256);
-  auto *const codes = reinterpret_cast<typename Codes8<BITS>::type *>(q);
   T *const sc = static_cast<T *>(s), *const bi = static_cast<T *>(b);
-  if (group == 32) quantize_kernel<T, BITS, 32><<<grid, 256, 0, st>>>(w, n_octets, codes, sc, bi);
-  else if (group == 64) quantize_kernel<T, BITS, 64><<<grid, 256, 0, st>>>(w, n_octets, codes, sc, bi);
-  else quantize_kernel<T, BITS, 128><<<grid, 256, 0, st>>>(w, n_octets, codes, sc, bi);
+  if (group == 32) quantize_kernel<T, BITS, 32><<<grid, 256, 0, st>>>(w, n_octets, q, sc, bi);
+  else if (group == 64) quantize_kernel<T, BITS, 64><<<grid, 256, 0, st>>>(w, n_octets, q, sc, bi);
+  else quantize_kernel<T, BITS, 128><<<grid, 256, 0, st>>>(w, n_octets, q, sc, bi);
 }
 
 template <class T, class O>
@@ -138,9 +148,9 @@ static void start_dequantize(const uint32_t *q, const void *s, const void *b, in
   const int lanes_log2 = group == 32 ? 2 : (group == 64 ? 3 : 4);
   const T *const sc = static_cast<const T *>(s), *const bi = static_cast<const T *>(b);
   O *const o = static_cast<O *>(out);
-  if (bits == 2) dequantize_kernel<T, O, 2><<<grid, 256, 0, st>>>(reinterpret_cast<const uint16_t *>(q), sc, bi, n_octets, lanes_log2, o);
+  if (bits == 2) dequantize_kernel<T, O, 2><<<grid, 256, 0, st>>>(q, sc, bi, n_octets, lanes_log2, o);
   else if (bits == 4) dequantize_kernel<T, O, 4><<<grid, 256, 0, st>>>(q, sc, bi, n_octets, lanes_log2, o);
-  else dequantize_kernel<T, O, 8><<<grid, 256, 0, st>>>(reinterpret_cast<const uint64_t *>(q), sc, bi, n_octets, lanes_log2, o);
+  else dequantize_kernel<T, O, 8><<<grid, 256, 0, st>>>(q, sc, bi, n_octets, lanes_log2, o);
 }
 
 // dt: 0 bf16, 1 fp16, 2 fp32 (mi_moe_dtype)

@@ -50,3 +50,32 @@ def test_codec_at_the_edges(rows, cols, bits, group, dtype):
     for out in {dt, torch.float32}:
         got = m.ops.dequantize(q, s, b, group, bits, out)
         assert torch.equal(got.cpu(), torch.from_numpy(v).to(out))
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_addresses_aligned_for_their_elements_only(bits, dtype):
+    """Operands and results one element behind a 16-byte address: the same values, nothing around them touched."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import capi
+    lib, dt = m.load_library(), getattr(torch, dtype)
+    code = {"bfloat16": capi.DTYPE_BF16, "float16": capi.DTYPE_F16, "float32": capi.DTYPE_F32}[dtype]
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def room(n, of):  # n elements with one before and one behind, all set
+        return torch.full((n + 2,), 7, dtype=of, device="cuda")
+
+    def inner(t, like):
+        assert t[0] == 7 and t[-1] == 7
+        return t[1:-1].reshape(like.shape)
+    w = torch.randn((5, 192), device="cuda") * 0.02
+    q, s, b = m.ops.quantize(w, 64, bits, dt)
+    w1, q1, s1, b1 = room(w.numel(), torch.float32), room(q.numel(), torch.int32), room(s.numel(), dt), room(b.numel(), dt)
+    w1[1:-1] = w.reshape(-1)
+    at = lambda t: t.data_ptr() + t.element_size()  # noqa: E731
+    assert lib.mi_moe_quantize_typed(at(w1), 5, 192, 64, bits, code, at(q1), at(s1), at(b1), stream) == 0
+    assert torch.equal(inner(q1, q), q) and torch.equal(inner(s1, s), s) and torch.equal(inner(b1, b), b)
+    for fn, of in ((lib.mi_moe_dequantize_native, dt), (lib.mi_moe_dequantize_typed, torch.float32)):
+        want, got = m.ops.dequantize(q, s, b, 64, bits, of), room(w.numel(), of)
+        assert fn(at(q1), at(s1), at(b1), 5, 192, 64, bits, code, at(got), stream) == 0
+        assert torch.equal(inner(got, want), want)
