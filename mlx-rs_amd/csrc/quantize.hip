@@ -132,25 +132,33 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint32_t *__restr
   store8(out + i * 8, v);
 }
 
+constexpr int64_t kOctetsMost = (int64_t)1 << 31;  // of one launch, which takes fewer than 2^32 threads: a whole number of groups
+
 template <class T, int BITS>
 static void start_quantize(const float *w, int64_t n_octets, int group, uint32_t *q, void *s, void *b, hipStream_t st) {
-  const unsigned grid = (unsigned)((n_octets + 255) / 256);
-  T *const sc = static_cast<T *>(s), *const bi = static_cast<T *>(b);
-  if (group == 32) quantize_kernel<T, BITS, 32><<<grid, 256, 0, st>>>(w, n_octets, q, sc, bi);
-  else if (group == 64) quantize_kernel<T, BITS, 64><<<grid, 256, 0, st>>>(w, n_octets, q, sc, bi);
-  else quantize_kernel<T, BITS, 128><<<grid, 256, 0, st>>>(w, n_octets, q, sc, bi);
+  T *sc = static_cast<T *>(s), *bi = static_cast<T *>(b);
+  for (int64_t n; n_octets > 0; n_octets -= n, w += 8 * n, q += n * BITS / 4, sc += 8 * n / group, bi += 8 * n / group) {
+    n = n_octets < kOctetsMost ? n_octets : kOctetsMost;
+    const unsigned grid = (unsigned)((n + 255) / 256);
+    if (group == 32) quantize_kernel<T, BITS, 32><<<grid, 256, 0, st>>>(w, n, q, sc, bi);
+    else if (group == 64) quantize_kernel<T, BITS, 64><<<grid, 256, 0, st>>>(w, n, q, sc, bi);
+    else quantize_kernel<T, BITS, 128><<<grid, 256, 0, st>>>(w, n, q, sc, bi);
+  }
 }
 
 template <class T, class O>
 static void start_dequantize(const uint32_t *q, const void *s, const void *b, int64_t n_octets, int group, int bits,
                              void *out, hipStream_t st) {
-  const unsigned grid = (unsigned)((n_octets + 255) / 256);
   const int lanes_log2 = group == 32 ? 2 : (group == 64 ? 3 : 4);
-  const T *const sc = static_cast<const T *>(s), *const bi = static_cast<const T *>(b);
-  O *const o = static_cast<O *>(out);
-  if (bits == 2) dequantize_kernel<T, O, 2><<<grid, 256, 0, st>>>(q, sc, bi, n_octets, lanes_log2, o);
-  else if (bits == 4) dequantize_kernel<T, O, 4><<<grid, 256, 0, st>>>(q, sc, bi, n_octets, lanes_log2, o);
-  else dequantize_kernel<T, O, 8><<<grid, 256, 0, st>>>(q, sc, bi, n_octets, lanes_log2, o);
+  const T *sc = static_cast<const T *>(s), *bi = static_cast<const T *>(b);
+  O *o = static_cast<O *>(out);
+  for (int64_t n; n_octets > 0; n_octets -= n, q += n * bits / 4, sc += 8 * n / group, bi += 8 * n / group, o += 8 * n) {
+    n = n_octets < kOctetsMost ? n_octets : kOctetsMost;
+    const unsigned grid = (unsigned)((n + 255) / 256);
+    if (bits == 2) dequantize_kernel<T, O, 2><<<grid, 256, 0, st>>>(q, sc, bi, n, lanes_log2, o);
+    else if (bits == 4) dequantize_kernel<T, O, 4><<<grid, 256, 0, st>>>(q, sc, bi, n, lanes_log2, o);
+    else dequantize_kernel<T, O, 8><<<grid, 256, 0, st>>>(q, sc, bi, n, lanes_log2, o);
+  }
 }
 
 // dt: 0 bf16, 1 fp16, 2 fp32 (mi_moe_dtype)

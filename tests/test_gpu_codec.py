@@ -79,3 +79,34 @@ def test_addresses_aligned_for_their_elements_only(bits, dtype):
         want, got = m.ops.dequantize(q, s, b, 64, bits, of), room(w.numel(), of)
         assert fn(at(q1), at(s1), at(b1), 5, 192, 64, bits, code, at(got), stream) == 0
         assert torch.equal(inner(got, want), want)
+
+
+def test_more_values_than_one_launch_has_threads_for():
+    """2^35 + 4096 values of 2-bit codes (8.6 GB, 69 GB dequantised): more than 2^32 threads of eight values; and quantised again."""
+    import mlx_rs_amd as m
+    rows = (1 << 23) + 1
+    if torch.cuda.mem_get_info()[0] < 250e9:
+        pytest.skip("the card has no 250 GB left")
+    q = torch.zeros((rows, 256), dtype=torch.int32, device="cuda")
+    s, b = torch.ones((rows, 32), device="cuda").bfloat16(), torch.zeros((rows, 32), device="cuda").bfloat16()
+    marks = [0, (1 << 22) - 1, 1 << 22, (1 << 23) - 1, 1 << 23]  # around the joints of the launches
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    for r in marks:
+        w = torch.randn((1, 4096), generator=gen, device="cuda")
+        for whole, row in zip((q, s, b), m.ops.quantize(w, 128, 2)):
+            whole[r] = row[0]
+    out = m.ops.dequantize(q, s, b, 128, 2)
+    for r in marks:
+        assert torch.equal(out[r:r + 1], m.ops.dequantize(q[r:r + 1], s[r:r + 1], b[r:r + 1], 128, 2))
+    assert out[5].eq(0).all() and out[-5].eq(0).all()
+    del q, s, b, out
+    torch.cuda.empty_cache()
+    w = torch.zeros((rows, 4096), device="cuda")
+    for r in marks:
+        w[r] = torch.randn(4096, generator=gen, device="cuda")
+    got = m.ops.quantize(w, 128, 2)
+    for r in marks:
+        for whole, row in zip(got, m.ops.quantize(w[r:r + 1], 128, 2)):
+            assert torch.equal(whole[r:r + 1], row)
+    del w, got
+    torch.cuda.empty_cache()
