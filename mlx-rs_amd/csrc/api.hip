@@ -137,11 +137,12 @@ struct ForwardWs {
   size_t bytes;
 };
 
-// Group sizes 32 and 128: tile lists are built (for segments of more rows than one pass of the kernel of a few rows)
-// from an average of four rows per expert on; see forward_impl for what that costs and gives.  The tiled kernel takes operands below 2 GiB, in multiples of 128 values.
+// Group sizes 32 and 128: tile lists are built (for segments of more rows than one pass of the kernel of a few rows, which
+// a segment of at most T rows has to be able to have) from an average of four rows per expert on; see forward_impl for what that
+// costs and gives.  The tiled kernel takes operands below 2 GiB, in multiples of 128 values.
 bool raw_tiled_batch(const mi_moe_config &c, int64_t T) {
   const int64_t P = T * c.top_k, most = (int64_t)1 << 31;
-  return P >= (int64_t)4 * c.n_experts && c.hidden % 128 == 0 && c.intermediate % 128 == 0 && T * c.hidden * 2 < most &&
+  return T > kRowsMost && P >= (int64_t)4 * c.n_experts && c.hidden % 128 == 0 && c.intermediate % 128 == 0 && T * c.hidden * 2 < most &&
          P * c.intermediate * 2 < most && (int64_t)codes_sums_bytes(P, c.intermediate, c.group_size) < most &&
          (int64_t)codes_sums_bytes(T, c.hidden, c.group_size) < most &&
          (int64_t)c.hidden * c.intermediate * c.bits / 8 < most;

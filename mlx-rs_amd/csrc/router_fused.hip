@@ -91,8 +91,8 @@ __global__ __launch_bounds__(kDispThreads) void router_fused_kernel(
   if (!last) return;
 
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  // at most 64 tokens, distinct experts per token: the mask form of the dispatch (the tiled lists
-  // belong to batches far above this kernel's, the host passes none)
+  // at most 64 tokens, distinct experts per token: the mask form of the dispatch, where the host wants no tile lists (few
+  // experts and more than 16 tokens in groups of 32 or 128 do)
   if (mtiles == nullptr && T <= kMaskTokens)
     dispatch_tokens_block(topk_idx, T, k, E, lds, counts, offsets, perm, inv_perm, src_of, work);
   else

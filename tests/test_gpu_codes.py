@@ -161,6 +161,20 @@ products round gate and up as well (0.94 * 2^-8, over as few as 256 values): 1.5
         assert float((again.double() - ref).norm() / ref.norm()) <= bound
 
 
+@pytest.mark.parametrize("tokens", [4, 6, 14])
+def test_a_small_batch_with_long_rows(tokens):
+    """No segment can be longer than one pass of the kernel of a few rows: no tile lists, and that kernel's LDS is that of the
+    batch's own rows (with 16 of them 8576 values in groups of 32 would not fit)."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(8576, 8, 8, 4096, 4, 32, 0)
+    blk = synth.make_block(cfg, seed=tokens, device="cuda", gen_device="cuda")
+    x = synth.make_tokens(cfg, tokens, seed=2, device="cuda")
+    out, routing = blk.forward(x, debug=True)
+    ref = block_truth(blk, x, routing)
+    assert float((out.double() - ref).norm() / ref.norm()) <= 2.0 ** -8
+
+
 @pytest.mark.parametrize("dtype,group", [("float16", 64), ("bfloat16", 32), ("float32", 128)])
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("rows", [7, 70, 1100])
