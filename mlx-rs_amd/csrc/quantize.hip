@@ -272,9 +272,7 @@ __global__ __launch_bounds__(256) void qmm_plain_t_kernel(const T *__restrict__ 
 // Sums meet by halving: at lane distance d each lane hands the half of its sums that its partner keeps; an addition
 // commutes, so the tree of a sum does not depend on the lane that holds it.
 // What bounds it: the vector unit, an fma per value and sum (430 us of it at 1000 x 4096 x 4096) beside the loads of x.
-// us of the call, a wave per output element / here: 1000 x 4096 x 4096 4-bit 2759 / 1007, 8-bit 3591 / 1387; 100 x 4096 x
-// 4096 305 / 103; 30 x 4096 x 2304 70.6 / 18.9; 300 x 1024 x 1024 80.9 / 20.5; 16 and 8 x 4096 x 4096 8-bit 80.7 and 41.5 /
-// 41.2 and 21.3.
+// (Figures: at the rule that picks R and C.)
 template <int BITS, int R, int C>
 __global__ __launch_bounds__(256) void qmm_plain_f32_kernel(const float *__restrict__ x, const uint32_t *__restrict__ w,
                                                             const float *__restrict__ scales, const float *__restrict__ biases,
@@ -394,6 +392,16 @@ static hipError_t launch_plain_t(const void *x, const uint32_t *w, const void *s
   return hipGetLastError();
 }
 
+// Which tile: the largest that leaves the launch two waves a SIMD (8 x 4 with 4-bit codes and 4 x 4; the 8-bit 4 x 4 tile
+// holds twice the values of x and wants four; 4 x 2 one), if half of its rows are there: fewer waves do not hide the loads.
+// Measured, us of the kernel with a wave per output element / 2 x 1 / 4 x 2 / 4 x 4 / 8 x 4 (rows, N, K):
+//   4-bit (8, 256, 1024) 2.9 / 2.8 / 3.4 / 4.6 / 6.7, (8, 1024, 4096) 9.1 / 7.4 / 6.1 / 10.9 / 17.4, (12, 2080, 3968) 23.9 / 20.0 / 12.0 /
+//   12.1 / 17.7, (17, 4096, 4096) 54.7 / 51.1 / 36.6 / 23.9 / 26.2, (32, 4096, 4096) 96.5 / 82.6 / 57.7 / 40.4 / 31.7,
+//   (1000, 4096, 4096) 2754 / 2379 / 1670 / 1063 / 1005;
+//   8-bit (8, 256, 1024) 3.2 / 3.1 / 3.7 / 5.6 / 10.4, (12, 2080, 3968) 33.0 / 22.1 / 14.7 / 26.1 / 30.9, (24, 4096, 4096) 106 / 68.8 /
+//   37.9 / 35.4 / 61.6, (1000, 4096, 4096) 3601 / 2488 / 1497 / 1079 / 1387.
+// (8 rows by one column from five rows on, whatever the waves: 3.9, 7.9, 23.7, 60.2 in the first four, slower than a wave per
+// output element in three of them.)
 template <int BITS>
 static hipError_t launch_plain_f32(const float *x, const uint32_t *w, const float *s, const float *b, int64_t rows, int N, int K,
                                    int group, float *y, hipStream_t st) {
@@ -403,14 +411,14 @@ static hipError_t launch_plain_f32(const float *x, const uint32_t *w, const floa
     qmm_plain_f32_kernel<BITS, R, C><<<grid, 256, 0, st>>>(x, w, s, b, rows, N, K, group, y);
     return hipGetLastError();
   };
-  auto with_rows = [&](auto c) {
-    if (rows <= 2) return run(std::integral_constant<int, 2>{}, c);
-    if (rows <= 4) return run(std::integral_constant<int, 4>{}, c);
-    return run(std::integral_constant<int, 8>{}, c);
-  };
-  // four columns a wave read x a fourth as often; where that leaves a SIMD fewer than four waves, one column
-  if ((rows + 7) / 8 * N >= 4 * 4096) return with_rows(std::integral_constant<int, 4>{});
-  return with_rows(std::integral_constant<int, 1>{});
+  const std::integral_constant<int, 2> two{};
+  const std::integral_constant<int, 4> four{};
+  const auto waves = [&](int r, int c) { return (rows + r - 1) / r * ((N + c - 1) / c); };
+  if constexpr (BITS == 4)
+    if (rows > 4 && waves(8, 4) >= 2048) return run(std::integral_constant<int, 8>{}, four);
+  if (rows > 2 && waves(4, 4) >= (BITS == 4 ? 2048 : 4096)) return run(four, four);
+  if (rows > 2 && waves(4, 2) >= 1024) return run(four, two);
+  return run(two, std::integral_constant<int, 1>{});
 }
 
 // dt: 0 bf16, 1 fp16, 2 fp32.  rows = n_idx * M output rows (at most 2^31 - 1: they are the grid's x extent).
