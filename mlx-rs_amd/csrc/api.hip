@@ -1068,9 +1068,9 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
   }
   const bool streamed = tuned && bits == 8 && M < tiled_avg_rows(bits);  // (see dense_takes_rows)
   const bool large_tiles = tuned && codes && !streamed && dense_takes_large_tiles(M, N);
-  // (x and w are read and y is written 16 bytes at a time, scales by words, biases one by one)
+  // (x and w are read and y is written 16 bytes at a time, scales and biases by words)
   if (codes && !one_plain && !streamed && !large_tiles && M * K * 4 < (int64_t)1 << 31 && workspace && workspace_bytes >= codes_bytes(M, K, group_size, bits, dtype) && aligned16(x) && aligned16(w) && aligned16(y) &&
-      (reinterpret_cast<uintptr_t>(scales) & 3u) == 0) {
+      ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 3u) == 0) {
     Carver cv(workspace);
     const size_t copy_bytes = codes_copy_bytes(dtype, bits, M, K);
     uint16_t *copy = copy_bytes ? reinterpret_cast<uint16_t *>(cv.take<char>(copy_bytes)) : nullptr;

@@ -183,6 +183,27 @@ __device__ __forceinline__ float as_f32(float v) { return v; }
 
 __device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
 
+// The products on raw codes multiply centred codes q - 8 and q - 128: s q + b = s (q - c) + (b + c s).  Without the centre the code
+// and bias terms of a group are several times their sum, and what they lose to each other's rounding is too.
+constexpr float centre_of(int bits) { return (float)(1 << (bits - 1)); }
+// Centred codes of one word as f32: two 4-bit codes a byte, times 16 (their byte's upper half), or 8-bit ones.  The signed byte
+// comes out of the conversion itself.
+__device__ __forceinline__ void centred_codes(uint32_t w, float (&v)[8]) {  // 4-bit: 16 (q_i - 8)
+  const uint32_t even = ((w << 4) ^ 0x88888888u) & 0xf0f0f0f0u, odd = (w ^ 0x88888888u) & 0xf0f0f0f0u;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[2 * i] = (float)(int8_t)(even >> (8 * i));
+    v[2 * i + 1] = (float)(int8_t)(odd >> (8 * i));
+  }
+}
+__device__ __forceinline__ void centred_codes(uint32_t w, float (&v)[4]) {  // 8-bit: q_i - 128
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = (float)(int8_t)((w ^ 0x80808080u) >> (8 * i));
+}
+__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {  // two bf16 of values that are bf16 already
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+
 // One element of a product of weights packed along K, an fma per k on the dequantised weight.  The products on raw codes
 // take it where their own sum is not finite: an infinity against codes and biases apart cancels to no number where
 // the dequantised weight keeps its sign, and sums of unscaled codes overflow earlier.  paired: x has every 8-block as

@@ -3,12 +3,16 @@
 //
 // Contract: mlx_quantized_matmul / mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:91-122,160-230).
 //
-// Arithmetic: sum_c x_c (s q_c + b) = s sum_c x_c q_c + b sum_c x_c per quantisation group.  The codes are exact in
-// bf16 and in f16, so the matrix cores multiply the activations with raw codes and nothing is rounded on the way in:
-//   bf16  x as it is; 4-bit codes as 128 + q (one and-or per pair), the 128 taken back through the bias term
+// Arithmetic: sum_c x_c (s q_c + b) = s sum_c x_c (q_c - c) + (b + c s) sum_c x_c per quantisation group, with the codes' centre c
+// (8 or 128).  Centred codes are exact in bf16 and in f16, so the matrix cores multiply the activations with them and nothing is
+// rounded on the way in:
+//   bf16  x as it is; codes through v_cvt_f32_i32 of signed bytes (4-bit codes times 16)
 //   f16   x as it is, codes in f16 (v_mfma_f32_32x32x16_f16)
-// float32 does not come here: the code and bias terms of a group cancel to about an eighth, which costs two of its bits
-// (error against 64 bits 3.3e-7 to 5.7e-7, a wave per output element 1.0e-7 to 1.3e-7, over 1 to 1000 rows).
+// The centre keeps the sums as exact as plain ones: share of results that are not the float64 product's nearest value, plain / codes
+// as they are (bf16, 4-bit: 128 + q) / centred, 17 to 1000 rows: bf16 4-bit 9e-5 / 4.7e-3 / 1.0e-4, 8-bit 1.5e-4 / 4.0e-4 / 1.1e-4, f16
+// 1.1e-3 / 2.7e-3 / 7.3e-4.  What it costs is the conversion of 4-bit codes in bf16, 15 instructions a multiply for 7: 51 us of
+// 1000 x 2080 x 3968 against 55, nothing below 300 rows.
+// float32 does not come here: without the centre its error was 3.3e-7 to 5.7e-7 (a wave per output element 1.0e-7 to 1.5e-7).
 // The fp32 sums of a group are scaled once, when the group ends.  The bias term sum_g b_g (sum_c x_c) is a product of
 // its own over the groups: the group sums of x (fp32, split into three bf16 pieces) against the biases (three pieces
 // as well), eight K slots a group (xh bh, xm bh, xl bh, xh bm, xm bm, xh bl: every product down to 2^-24), which the
@@ -35,6 +39,7 @@ constexpr int kWeave = MI_CODES_WEAVE;  // vector instructions between two matri
 constexpr size_t kLdsAtLeast = 4 * 32 * (32 * 4 + 16);  // the epilogue's staging
 
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
+typedef uint32_t u32x3_t __attribute__((ext_vector_type(3)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
 
@@ -75,12 +80,6 @@ struct Split : F {
 template <bool SPLIT, class F>
 __device__ __forceinline__ Split<SPLIT, F> with_split(F f) { return Split<SPLIT, F>(f); }
 
-template <class T>
-__device__ __forceinline__ T load_elem(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
-  else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0));
-}
-
 // a thread's share of a step's token rows
 template <int P, int NA>
 struct RowStage {
@@ -90,8 +89,10 @@ struct RowStage {
 constexpr bool paired_order(int bits) { return bits == 4; }  // 8-blocks as (0,4)(1,5)(2,6)(3,7)
 constexpr int padded_groups(int G) { return (G + 15) / 16 * 16; }  // the bias product runs an even number of steps of eight groups
 
-__device__ __forceinline__ uint32_t f16_minus_1024(uint32_t v) {  // two halves 1024 + q -> q: exact
-  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) - half2_t{(_Float16)1024, (_Float16)1024});
+template <int BITS>
+__device__ __forceinline__ uint32_t f16_centred(uint32_t v) {  // two halves 1024 + q -> q - centre: exact
+  constexpr _Float16 off = (_Float16)(1024.0f + centre_of(BITS));
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) - half2_t{off, off});
 }
 template <class T> __device__ __forceinline__ T rounded(float v) { return (T)v; }
 template <> __device__ __forceinline__ uint16_t rounded<uint16_t>(float v) { return (uint16_t)(cvt_pk_bf16(v, 0.f) & 0xffffu); }
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf
 //   8-bit: 16 bytes are 16 codes, two loads a step, groups of 32 stay apart by themselves.
 // Token rows pass through LDS (128 K values between two barriers, double-buffered).
 // A step takes one 32 x 32 sub-tile after the other: its four multiplies follow each other in one accumulator, and the
-// scaled addition of the sub-tile before it (16 fma) and the unpacking of the next step's codes (9 to 11 instructions a
+// scaled addition of the sub-tile before it (16 fma) and the unpacking of the next step's codes (10 to 15 instructions a
 // multiply) run between them, which is as much vector work as fits beside the matrix cores.
 // What bounds it (777 x 4096 x 4096, f16, 8-bit; 26 GFLOP): 58 us for the call = 450 TFLOP/s, 50 times the plain kernel's
 // 3160 us; the matrix cores alone would take 18.  Taken apart at one block a CU (cycles per 64 K values of 128 x 32 a
@@ -176,7 +177,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   constexpr int NQ = BITS == 4 ? 1 : 2;      // 16-byte code loads per lane, tile and step
   constexpr int NS = G32 ? 2 : 1;            // scaled additions per sub-tile and step
   constexpr bool SPLIT = BITS == 8 || G32;   // which K values a multiply takes: see chunk below
-  constexpr float kOffset = BITS == 4 && DT == 0 ? 128.0f : 0.0f;  // the codes are multiplied as offset + q
+  constexpr float kUnit = BITS == 4 && DT == 0 ? 0.0625f : 1.0f;  // the codes are multiplied as (q - centre) / kUnit
   constexpr int A_SZ = BM * kRow, BUF = A_SZ;                      // 16-byte units
   static_assert(BM % RS == 0, "whole loads");
 
@@ -354,12 +355,14 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     }
   };
 
-  // ---- the bias product: group sums of x against b - offset s, accumulated into the result
+  // ---- the bias product: group sums of x against b + centre s, accumulated into the result
   {
     typedef RowStage<1, NA> StageA;
     auto put_a = [&](u32x4_t *to, const StageA &R, int i) __attribute__((always_inline)) { *to = R.v[0][i]; };
+    // A lane's four groups of a step are three words, as a row may start between two.  Groups past the row's end are another
+    // row's or zeros: their sums are zero.
     struct StageB {
-      T s[NT][4], b[NT][4];
+      u32x3_t s[NT], b[NT];
     };
     auto load_a = [&](int ks, bool real, StageA &R) __attribute__((always_inline)) {
 #pragma unroll
@@ -368,17 +371,18 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     };
     auto load_b = [&](int ks, StageB &R) __attribute__((always_inline)) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          int g = ks * 8 + 4 * kb + h;
-          g = g < G ? g : G - 1;  // (padding groups: their sums are zero)
-          R.b[t][h] = load_elem<T>(br[t], s_voff[t] + g * (uint32_t)sizeof(T), 0);
-          R.s[t][h] = kOffset != 0.f ? load_elem<T>(sr[t], s_voff[t] + g * (uint32_t)sizeof(T), 0) : T{};
-        }
+      for (int t = 0; t < NT; ++t) {
+        const uint32_t off = (s_voff[t] + (ks * 8 + 4 * kb) * (uint32_t)sizeof(T)) & ~3u;
+        R.s[t] = __builtin_amdgcn_raw_buffer_load_b96(sr[t], off, 0, 0);
+        R.b[t] = __builtin_amdgcn_raw_buffer_load_b96(br[t], off, 0, 0);
+      }
     };
     auto unpack = [&](const StageB &R, Operand &o, int t, int h) __attribute__((always_inline)) {
-      const Pieces p = split3(__builtin_fmaf(-kOffset, as_f32(R.s[t][h]), as_f32(R.b[t][h])));
+      const auto group = [&](const u32x3_t &v) __attribute__((always_inline)) {  // (row starts are even numbers of bytes)
+        const uint32_t pair = __builtin_amdgcn_alignbyte(v[h / 2 + 1], v[h / 2], s_voff[t]);
+        return as_f32(__builtin_bit_cast(T, (uint16_t)(h % 2 ? pair >> 16 : pair)));
+      };
+      const Pieces p = split3(__builtin_fmaf(centre_of(BITS), group(R.s[t]), group(R.b[t])));
       o.v[t][h] = u32x4_t{p.h | p.h << 16, p.h | p.m << 16, p.m | p.l << 16, 0u};
     };
     auto body = [&](const u32x4_t (&av)[4][1], const Operand &o, int, int m, int t) __attribute__((always_inline)) {
@@ -432,34 +436,36 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
           }
         }
       }
-          if constexpr (BITS == 4) {
-            const uint32_t w = R.q[t][0][h];
+      if constexpr (BITS == 4 && DT == 0) {
+        float v[8];
+        centred_codes(R.q[t][0][h], v);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              if constexpr (DT == 0) {
-                o.v[t][h][i] = __builtin_amdgcn_bitop3_b32(w >> (4 * i), 0x000f000fu, 0x43004300u, 0xEA);  // (a & b) | c
-              } else if (i % 2 == 0) {
-                o.v[t][h][i] = f16_minus_1024(__builtin_amdgcn_bitop3_b32(w >> (4 * i), 0x000f000fu, 0x64006400u, 0xEA));
-              } else {  // 1024 + 16 q -> q, exact as well: one shift serves two nibbles
-                const half2_t v = __builtin_bit_cast(half2_t, __builtin_amdgcn_bitop3_b32(w >> (4 * (i - 1)), 0x00f000f0u, 0x64006400u, 0xEA));
-                o.v[t][h][i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, half2_t{(_Float16)0.0625f, (_Float16)0.0625f}, half2_t{(_Float16)-64.0f, (_Float16)-64.0f}));
-              }
-            }
-          } else if constexpr (DT == 1) {
+        for (int i = 0; i < 4; ++i) o.v[t][h][i] = upper_halves(v[i], v[i + 4]);
+      } else if constexpr (BITS == 4) {
+        const uint32_t w = R.q[t][0][h];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)  // bytes 2 i, 2 i + 1 under the exponent of 1024
-              o.v[t][h][i] = f16_minus_1024(__builtin_amdgcn_perm(0x64646464u, R.q[t][h >> 1][2 * (h & 1) + (i >> 1)],
-                                                                  (i & 1) ? 0x07030702u : 0x07010700u));
-          } else {  // codes through v_cvt_f32_ubyte, upper halves packed
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              uint32_t c0, c1;  // codes 2 i, 2 i + 1
-              const uint32_t w = R.q[t][h >> 1][2 * (h & 1) + (i >> 1)];
-              c0 = (w >> (16 * (i & 1))) & 0xffu;
-              c1 = (w >> (16 * (i & 1) + 8)) & 0xffu;
-              o.v[t][h][i] = __builtin_amdgcn_perm(__float_as_uint((float)c1), __float_as_uint((float)c0), 0x07060302u);
-            }
+        for (int i = 0; i < 4; ++i) {
+          if (i % 2 == 0) {
+            o.v[t][h][i] = f16_centred<4>(__builtin_amdgcn_bitop3_b32(w >> (4 * i), 0x000f000fu, 0x64006400u, 0xEA));  // (a & b) | c
+          } else {  // 1024 + 16 q -> q - 8, exact as well: one shift serves two nibbles
+            const half2_t v = __builtin_bit_cast(half2_t, __builtin_amdgcn_bitop3_b32(w >> (4 * (i - 1)), 0x00f000f0u, 0x64006400u, 0xEA));
+            o.v[t][h][i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, half2_t{(_Float16)0.0625f, (_Float16)0.0625f}, half2_t{(_Float16)-72.0f, (_Float16)-72.0f}));
           }
+        }
+      } else if constexpr (DT == 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)  // bytes 2 i, 2 i + 1 under the exponent of 1024
+          o.v[t][h][i] = f16_centred<8>(__builtin_amdgcn_perm(0x64646464u, R.q[t][h >> 1][2 * (h & 1) + (i >> 1)],
+                                                              (i & 1) ? 0x07030702u : 0x07010700u));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          float v[4];
+          centred_codes(R.q[t][h >> 1][2 * (h & 1) + (i >> 1)], v);
+          o.v[t][h][i] = upper_halves(v[0], v[1]);
+          o.v[t][h][i + 1] = upper_halves(v[2], v[3]);
+        }
+      }
     };
     // The scales of this wave's rows pass through LDS a window at a time: a lane fetches 16 bytes of its row (half kb of
     // the window) one window ahead, and reads one value per group back.  One 2-byte load per group from a row each
@@ -496,7 +502,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < NS; ++i)
-          step_s[d][t][i] = as_f32(*reinterpret_cast<const T *>(s_at[t] + ((G32 ? 2 * ks + i : ks >> scale_shift) - gw) * (int)sizeof(T)));
+          step_s[d][t][i] = kUnit * as_f32(*reinterpret_cast<const T *>(s_at[t] + ((G32 ? 2 * ks + i : ks >> scale_shift) - gw) * (int)sizeof(T)));
     };
     auto body = [&](const u32x4_t (&av)[4][1], const Operand &o, int d, int m, int t) __attribute__((always_inline)) {
       const int tile = m * NT + t;

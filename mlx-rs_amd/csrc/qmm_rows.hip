@@ -5,7 +5,9 @@
 // with GLU also nn::silu and multiply (nn/activation.rs:142-144,876-880).
 //
 // Arithmetic as in the tiled product on raw codes (qmm_codes.hip): sum_c x_c (s q_c + b) = s sum_c x_c q_c + b sum_c x_c
-// per group, codes unrounded on the matrix cores, fp32 sums.  Here the bias term is fp32 vector work: a tile is 16
+// per group with centred codes, unrounded on the matrix cores, fp32 sums; the same precision as plain sums have (results that
+// are not the float64 product's nearest value, plain / codes as they are or 128 + q / centred: bf16 4-bit 1.0e-4 / 1.7e-3 / 1.0e-4, f16
+// 1.1e-3 / 1.4e-3 / 8e-4).  Here the bias term is fp32 vector work: a tile is 16
 // tokens by 16 weight rows (v_mfma_f32_16x16x32), so it is four fma a lane and group.
 #include <type_traits>
 
@@ -39,8 +41,15 @@ __device__ __forceinline__ f32x4_t mfma(u32x4_t a, u32x4_t b, f32x4_t c) {
   else
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
-__device__ __forceinline__ uint32_t f16_minus_1024(uint32_t v) {  // two halves 1024 + q -> q: exact
-  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) - half2_t{(_Float16)1024, (_Float16)1024});
+// Two bytes 0 to 15 as bf16, the lower or the upper ones of v: below 16 an e4m3 number is its byte in units of 2^-9.
+template <int UPPER>
+__device__ __forceinline__ uint32_t small_codes(uint32_t v) {
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f, UPPER != 0));
+}
+template <int BITS>
+__device__ __forceinline__ uint32_t f16_centred(uint32_t v) {  // two halves 1024 + q -> q - centre: exact
+  constexpr _Float16 off = (_Float16)(1024.0f + centre_of(BITS));
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) - half2_t{off, off});
 }
 
 // LDS of a launch: token rows of sk values (tt of them), 64 zero bytes, the sums of x over each group and
@@ -78,8 +87,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
   constexpr int NW = 4 / KW;
   constexpr int CH = BITS == 4 ? 128 : 64;     // codes per chunk and row
   constexpr int MUL = CH / 32;                 // multiplies per chunk
-  constexpr float kOffset = BITS == 4 && DT == 0 ? 128.0f : 0.0f;
-  constexpr bool PAIRED = BITS == 4;  // token rows as 8-blocks (0,4)(1,5)(2,6)(3,7), the order of the unpacking
+  // 4-bit codes in bf16 come out of their conversion as they are; a group's sum starts from -8 times that of x instead, which is
+  // what the sums of x in LDS hold then.
+  constexpr bool kStart = BITS == 4 && DT == 0;
+  constexpr bool PAIRED = BITS == 4;  // token rows as 8-blocks (0,4)(1,5)(2,6)(3,7), bf16 (0,2)(1,3)(4,6)(5,7): the order of the unpacking
 
   int e = 0, cnt = (int)a.M;
   int64_t r0 = 0;
@@ -198,7 +209,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
             }
           }
           uint4 p = w;
-          if constexpr (PAIRED) {
+          if constexpr (kStart) {
+            p.x = (w.x & 0xffffu) | (w.y << 16);
+            p.y = (w.x >> 16) | (w.y & 0xffff0000u);
+            p.z = (w.z & 0xffffu) | (w.w << 16);
+            p.w = (w.z >> 16) | (w.w & 0xffff0000u);
+          } else if constexpr (PAIRED) {
             p.x = (w.x & 0xffffu) | (w.z << 16);
             p.y = (w.x >> 16) | (w.z & 0xffff0000u);
             p.z = (w.y & 0xffffu) | (w.w << 16);
@@ -211,7 +227,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
         sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
         if constexpr (GROUP >= 64) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
         if constexpr (GROUP == 128) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
-        if (piece % (GROUP / 8) == 0) sums[piece / (GROUP / 8) * kTokens + row] = sum;
+        if (piece % (GROUP / 8) == 0) sums[piece / (GROUP / 8) * kTokens + row] = kStart ? -centre_of(BITS) * sum : sum;
         piece += 256;
         while (piece >= per_row) {
           piece -= per_row;
@@ -230,6 +246,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
           if (j < j1) {
             const int ch = wk + KW * j, ch_slab = ch - s0 / CH;
             f32x4_t acc[NM];
+            constexpr int NG = GROUP < CH ? CH / GROUP : 1;  // groups of a chunk (8-bit groups of 128: half a one)
+            float4 xs[NG];
+#pragma unroll
+            for (int i = 0; i < NG; ++i) xs[i] = *reinterpret_cast<const float4 *>(sums + (ch * CH / GROUP + i - s0 / GROUP) * kTokens + 4 * kb);
             u32x4_t q[NM];
 #pragma unroll
             for (int m = 0; m < NM; ++m) {
@@ -263,50 +283,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
               const int k = BITS == 4 ? 32 * s + 8 * kb : (GROUP == 32 ? 32 * s + 16 * (kb & 1) + 8 * (kb >> 1) : 16 * kb + 8 * s);
               const bool first = GROUP == 32 || (GROUP == 64 ? (BITS == 4 ? s % 2 == 0 : s == 0) : s == 0);
               const bool last = GROUP == 32 || (GROUP == 64 ? (BITS == 4 ? s % 2 == 1 : s == 1) : s == MUL - 1);
+              const int g = ch * CH / GROUP + 32 * s / GROUP;
+              const float4 x_sum = xs[32 * s / GROUP % NG];
               const u32x4_t av = *reinterpret_cast<const u32x4_t *>(xl + x_step * ((ch_slab * CH + k) * 2));
 #pragma unroll
               for (int m = 0; m < NM; ++m) {
                 u32x4_t bv;
-                if constexpr (PAIRED) {
+                if constexpr (PAIRED && DT == 0) {
+                  const uint32_t w = q[m][s], even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
+                  bv = u32x4_t{small_codes<0>(even), small_codes<0>(odd), small_codes<1>(even), small_codes<1>(odd)};
+                } else if constexpr (PAIRED) {
                   const uint32_t w = q[m][s];
 #pragma unroll
-                  for (int i = 0; i < 4; ++i) {
-                    const uint32_t o = __builtin_amdgcn_bitop3_b32(w >> (4 * i), 0x000f000fu, DT == 0 ? 0x43004300u : 0x64006400u, 0xEA);  // (a & b) | c
-                    bv[i] = DT == 0 ? o : f16_minus_1024(o);
-                  }
+                  for (int i = 0; i < 4; ++i)
+                    bv[i] = f16_centred<4>(__builtin_amdgcn_bitop3_b32(w >> (4 * i), 0x000f000fu, 0x64006400u, 0xEA));  // (a & b) | c
                 } else if constexpr (DT == 1) {
 #pragma unroll
                   for (int i = 0; i < 4; ++i)
-                    bv[i] = f16_minus_1024(__builtin_amdgcn_perm(0x64646464u, q[m][2 * s + (i >> 1)], (i & 1) ? 0x07030702u : 0x07010700u));
+                    bv[i] = f16_centred<8>(__builtin_amdgcn_perm(0x64646464u, q[m][2 * s + (i >> 1)], (i & 1) ? 0x07030702u : 0x07010700u));
                 } else {
 #pragma unroll
-                  for (int i = 0; i < 4; ++i) {
-                    uint32_t c0, c1;
-                    const uint32_t w = q[m][2 * s + (i >> 1)];
-                    c0 = (w >> (16 * (i & 1))) & 0xffu;
-                    c1 = (w >> (16 * (i & 1) + 8)) & 0xffu;
-                    bv[i] = __builtin_amdgcn_perm(__float_as_uint((float)c1), __float_as_uint((float)c0), 0x07060302u);
+                  for (int i = 0; i < 4; i += 2) {
+                    float v[4];
+                    centred_codes(q[m][2 * s + (i >> 1)], v);
+                    bv[i] = upper_halves(v[0], v[1]);
+                    bv[i + 1] = upper_halves(v[2], v[3]);
                   }
                 }
-                acc[m] = mfma<DT>(av, bv, first ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[m]);
+                acc[m] = mfma<DT>(av, bv, !first ? acc[m] : kStart ? f32x4_t{x_sum.x, x_sum.y, x_sum.z, x_sum.w} : f32x4_t{0.f, 0.f, 0.f, 0.f});
               }
-              if (last || (GROUP == 128 && BITS == 8 && s == MUL - 1)) {  // (8-bit groups of 128: half a group, same scale)
-                const int gs = GROUP == 128 && BITS == 8 ? ch : (ch * CH + 32 * s) / GROUP;
-                const int g = GROUP == 128 && BITS == 8 ? ch >> 1 : gs;
-                const int g_slab = g - s0 / GROUP;
-                const float4 xs = *reinterpret_cast<const float4 *>(sums + g_slab * kTokens + 4 * kb);
+              if (last) {  // (8-bit groups of 128: half a group, same scale)
                 const bool with_bias = !(GROUP == 128 && BITS == 8) || (ch & 1) == 0;  // (once per group)
 #pragma unroll
                 for (int m = 0; m < NM; ++m) {
                   const uint32_t p = *reinterpret_cast<const uint32_t *>(my_pairs + m * 16 * L.pair_row + g * 4);
                   const float sc = as_f32(__builtin_bit_cast(T, (uint16_t)(p & 0xffffu)));
-                  float bi = as_f32(__builtin_bit_cast(T, (uint16_t)(p >> 16)));
-                  if constexpr (kOffset != 0.f) bi = __builtin_fmaf(-kOffset, sc, bi);
-                  if (!with_bias) bi = 0.f;
-                  tot[m][0] = __builtin_fmaf(sc, acc[m][0], __builtin_fmaf(bi, xs.x, tot[m][0]));
-                  tot[m][1] = __builtin_fmaf(sc, acc[m][1], __builtin_fmaf(bi, xs.y, tot[m][1]));
-                  tot[m][2] = __builtin_fmaf(sc, acc[m][2], __builtin_fmaf(bi, xs.z, tot[m][2]));
-                  tot[m][3] = __builtin_fmaf(sc, acc[m][3], __builtin_fmaf(bi, xs.w, tot[m][3]));
+                  const float b = as_f32(__builtin_bit_cast(T, (uint16_t)(p >> 16)));
+                  const float bi = !with_bias ? 0.f : kStart ? -__builtin_fmaf(1.0f / centre_of(BITS), b, sc) : __builtin_fmaf(centre_of(BITS), sc, b);
+                  tot[m][0] = __builtin_fmaf(sc, acc[m][0], __builtin_fmaf(bi, x_sum.x, tot[m][0]));
+                  tot[m][1] = __builtin_fmaf(sc, acc[m][1], __builtin_fmaf(bi, x_sum.y, tot[m][1]));
+                  tot[m][2] = __builtin_fmaf(sc, acc[m][2], __builtin_fmaf(bi, x_sum.z, tot[m][2]));
+                  tot[m][3] = __builtin_fmaf(sc, acc[m][3], __builtin_fmaf(bi, x_sum.w, tot[m][3]));
                 }
               }
             }

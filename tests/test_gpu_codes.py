@@ -77,8 +77,8 @@ def off_by_one(t):
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("rows", [7, 40, 300])
 def test_scales_between_two_words(rows, bits, dtype, group):
-    """Scales or biases that start two bytes behind a word: scales, which the kernels on raw codes read by words, send the product
-    to the plain kernel (as rows at such an address do); biases alone are fine in tiles."""
+    """Scales or biases that start two bytes behind a word, which the kernels on raw codes read by words: the product goes to the
+    plain kernel (as rows at such an address do)."""
     import mlx_rs_amd as m
     dt = getattr(torch, dtype)
     for n, k in ((48, 384), (37, 384)):
@@ -88,9 +88,7 @@ def test_scales_between_two_words(rows, bits, dtype, group):
         run = lambda *a: m.ops.quantized_linear(*a, group_size=group, bits=bits)  # noqa: E731
         plain = run(off_by_one(x), q, s, b)
         assert torch.equal(run(x, q, off_by_one(s), b), plain)
-        ref = product(x, q, s, b, group, bits)
-        y = run(x, q, s, off_by_one(b))
-        assert float((y.double() - ref).norm() / ref.norm()) <= BOUND[dtype]
+        assert torch.equal(run(x, q, s, off_by_one(b)), plain)
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
@@ -106,6 +104,27 @@ def test_an_odd_number_of_scales(rows, bits, dtype):
     x = torch.randn((rows, 384), generator=gen, device="cuda").to(dt)
     run = lambda v: m.ops.quantized_linear(v, q, s, b, group_size=128, bits=bits)  # noqa: E731
     assert torch.equal(run(x), run(off_by_one(x)))
+
+
+@pytest.mark.parametrize("dtype,group", [("bfloat16", 32), ("bfloat16", 64), ("bfloat16", 128), ("float16", 32), ("float16", 64), ("float16", 128)])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows,n", [(16, 16384), (300, 4096)])  # the kernel of a few rows, tiles
+def test_sums_lose_no_more_than_plain_ones(rows, n, bits, dtype, group):
+    """The share of results that are not the float64 product's nearest value measures what the sums lose before the last rounding:
+    an error d moves a result over a rounding boundary with probability |d| / spacing.  Plain float32 sums over 4096 values are
+    1.5e-7 of the results' root mean square off; 2^-22, 1.6 times that, is allowed, and its mean over a normal error is 0.8 of it.
+    (Codes that are not centred: 3e-7 in float16, 1e-5 with bfloat16's 128 + q.)"""
+    import mlx_rs_amd as m
+    dt = getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(rows + group + bits)
+    q, s, b = m.ops.quantize(torch.randn((n, 4096), generator=gen, device="cuda") * 0.02, group, bits, dt)
+    x = torch.randn((rows, 4096), generator=gen, device="cuda").to(dt)
+    ref = product(x, q, s, b, group, bits)
+    y = m.ops.quantized_linear(x, q, s, b, group_size=group, bits=bits)
+    spacing = torch.finfo(dt).eps * torch.exp2(torch.floor(torch.log2(ref.abs())))
+    allowed = float((0.8 * 2.0 ** -22 * ref.square().mean().sqrt() / spacing).clamp(max=1).mean())
+    share = float((y != ref.to(dt)).double().mean())
+    assert share <= allowed, (share, allowed)
 
 
 def test_large_float32_values_survive_the_split():
