@@ -6,10 +6,13 @@
 // Arithmetic: a group has a scale of its own for every k, so nothing can be taken out of the sum; the weights are
 // dequantised, w = fma(s, q, b) in fp32, and enter the matrix cores in pieces (each the rounded rest of the ones before
 // it), as do f32 rows of x:
-//   bf16  x as it is, w in two pieces (16 bits and more): 2 products
-//   f16   x as it is, 2^10 w in two f16 pieces (22 bits down to |w| = 2^-13, and never off by more than 2^-35; the factor
-//         keeps the second piece clear of the smallest numbers and leaves |w| < 64 without an overflow): 2 products
+//   bf16  x as it is, w in two pieces: 2 products
+//   f16   x as it is, 2^10 w in two f16 pieces (the factor keeps every piece clear of the smallest numbers: w is a multiple of 2^-24,
+//         and leaves |w| < 64 without an overflow): 2 products
 //   f32   x in three pieces (exact), w in three (exact): the 6 products down to 2^-18 of the first
+// Two pieces hold 17 bits (f16: 23), which is all of w unless its bias is 2^10 (f16: 2^13) times its scale or more; groups whose values
+// have both signs keep it below 2^4 (4-bit codes) and 2^8 (8-bit).  A wave that met such a scale goes over its K once more, for the
+// third pieces (another step inside the loop would spill): the weights are those of the plain product in every case.
 // A result that is not finite is computed again the plain way, one fma per k: pieces of an infinity are no numbers, and
 // where nothing but a piece has overflowed that gives the number.
 #include <type_traits>
@@ -88,11 +91,12 @@ constexpr int wave_lds(int dt, int ms, int nt) {
 // consecutive ones: column n = 2 NT u + j goes to place 16 (j % NT * 2 + j / NT) + u, that is
 // sub-tile j % NT, lane 16 (j / NT) + u.
 // What bounds it (128 x 64 tiles, bf16): a step of a wave is 1024 cycles of matrix work (two products) beside about 800 of
-// unpacking and 32 KB through LDS, each near the CU's rate.  1000 x 2048 x 4096, 4-bit, groups of 64: 46 us for the call,
+// unpacking and 32 KB through LDS, each near the CU's rate.  1000 x 2048 x 4096, 4-bit, groups of 64: 47 us for the call,
 // 360 TFLOP/s of the product (a thread per packed word of an output row, one k after the other: 1360 us); 8 rows 19 us
 // (1450); f32 141 us (1350).
-// Error against 64 bits at that size: bf16 1.6609e-3 and f16 2.0758e-4 as before (the result's rounding), f32 4.9e-7 (one
-// fma after the other: 1.07e-6).
+// Error: share of results that are not the float64 product's nearest value, here / a thread per packed word: 300 x 2048 x 2048 bf16 1.1e-4
+// to 2.2e-4 / 1.8e-4 to 5.4e-4, f16 1.2e-3 / 3.6e-3; groups at 1 + q / 2^13 and rows that sum to zero, bf16, 3e-3 to 1.1e-2 / 1.4e-3 to
+// 3.2e-3 (two pieces alone: 0.11 to 0.14); f32 against 64 bits 4.9e-7 / 1.07e-6.  What looking at the scales costs: 1 us of 47.
 template <int DT, int BITS, int MS, int NT, int KW>
 __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mtiles, int n_ntiles, int group_log2) {
   typedef typename ElemOf<DT>::type T;
@@ -168,7 +172,20 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  auto put = [&](const Stage &R) __attribute__((always_inline)) {
+  // By how many powers of two a bias is ahead of its scale, at most and at least, in the exponent's place.  Weights have two pieces'
+  // bits, from the leading one of the largest value (at most 2 max(|b|, 2^BITS |s|)) down to the last one of scale or bias, while
+  // that is at most kBits and at least BITS - kBits.
+  constexpr int kBits = DT == 1 ? 11 : 8;  // of s, b and a piece
+  int most = 0, least = 0;
+  auto see_scale = [&](const Stage &R) __attribute__((always_inline)) {
+    const uint32_t s = __float_as_uint(as_f32(R.s)), b = __float_as_uint(as_f32(R.b));
+    const int ahead = (int)(b & 0x7f800000u) - (int)(s & 0x7f800000u);
+    most = ahead > most ? ahead : most;
+    least = b << 1 != 0u && ahead < least ? ahead : least;
+  };
+  // rows, and pieces FIRST .. FIRST + COUNT - 1 of the weights
+  auto put = [&](const Stage &R, auto first, auto count) __attribute__((always_inline)) {
+    constexpr int FIRST = decltype(first)::value, COUNT = decltype(count)::value;
     *reinterpret_cast<float2 *>(Ss + (lane >> 5) * kScaleRow + skl * 8) = make_float2(kFactor * as_f32(R.s), kFactor * as_f32(R.b));
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
@@ -190,7 +207,7 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
     }
     wave_fence();
     const float4 *const pairs = reinterpret_cast<const float4 *>(Ss + (CN * u / 32) * kScaleRow + oct * 64);
-    u32x4_t o[CN][PW];
+    u32x4_t o[CN][COUNT];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {  // two rows
       const float4 sb = pairs[r];
@@ -199,16 +216,16 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
       for (int c = 0; c < CN; ++c) {
         const float v0 = __builtin_fmaf(sb.x, (float)((q0 >> (BITS * c)) & ((1u << BITS) - 1u)), sb.y);
         const float v1 = __builtin_fmaf(sb.z, (float)((q1 >> (BITS * c)) & ((1u << BITS) - 1u)), sb.w);
-        uint32_t pc[PW];
-        split_pair<DT, PW>(v0, v1, pc);
+        uint32_t pc[FIRST + COUNT];
+        split_pair<DT, FIRST + COUNT>(v0, v1, pc);
 #pragma unroll
-        for (int p = 0; p < PW; ++p) o[c][p][r] = pc[p];
+        for (int p = 0; p < COUNT; ++p) o[c][p][r] = pc[FIRST + p];
       }
     }
 #pragma unroll
     for (int c = 0; c < CN; ++c)
 #pragma unroll
-      for (int p = 0; p < PW; ++p) Ws[p * W_SZ + at(16 * (c % NT * 2 + c / NT) + u, oct)] = o[c][p];
+      for (int p = 0; p < COUNT; ++p) Ws[p * W_SZ + at(16 * (c % NT * 2 + c / NT) + u, oct)] = o[c][p];
     wave_fence();
   };
 
@@ -220,14 +237,15 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
 #pragma unroll
       for (int r = 0; r < 16; ++r) tot[m][t][r] = 0.f;
   const int ln = lane & 31, kb = lane >> 5;
-  auto multiply = [&]() __attribute__((always_inline)) {
+  auto multiply = [&](auto pieces) __attribute__((always_inline)) {
+    constexpr int COUNT = decltype(pieces)::value;  // of the weights
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      u32x4_t wv[NT][PW];
+      u32x4_t wv[NT][COUNT];
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int p = 0; p < PW; ++p) wv[t][p] = Ws[p * W_SZ + at(32 * t + ln, 2 * h + kb)];
+        for (int p = 0; p < COUNT; ++p) wv[t][p] = Ws[p * W_SZ + at(32 * t + ln, 2 * h + kb)];
 #pragma unroll
       for (int m = 0; m < MS; ++m) {
         u32x4_t xv[PX];
@@ -236,7 +254,7 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
 #pragma unroll
         for (int px = PX - 1; px >= 0; --px)
 #pragma unroll
-          for (int pw = PW - 1; pw >= 0; --pw)
+          for (int pw = COUNT - 1; pw >= 0; --pw)
             if (px + pw < PW)
 #pragma unroll
               for (int t = 0; t < NT; ++t) tot[m][t] = mfma<DT>(xv[px], wv[t][pw], tot[m][t]);
@@ -247,14 +265,20 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
 
   const int steps = (K + kStep - 1) / kStep, share = (steps + KW - 1) / KW;
   const int k0 = wave * share, k1 = k0 + share < steps ? k0 + share : steps;
-  if (k0 < k1) {
+  auto pass = [&](auto first, auto count) __attribute__((always_inline)) {
     Stage R;
     load(k0, R);
     for (int ks = k0; ks < k1; ++ks) {
-      put(R);
+      if constexpr (DT != 2) see_scale(R);
+      put(R, first, count);
       load(ks + 1 < k1 ? ks + 1 : ks, R);
-      multiply();
+      multiply(count);
     }
+  };
+  if (k0 < k1) {
+    pass(std::integral_constant<int, 0>{}, std::integral_constant<int, PW>{});
+    if constexpr (DT != 2)
+      if (__ballot((most >> 23) > kBits || (least >> 23) < BITS - kBits)) pass(std::integral_constant<int, PW>{}, std::integral_constant<int, 1>{});
   }
 
   // ---- the waves' sums: the second half of the waves hands its sums to the first, whose sums every wave then adds for a

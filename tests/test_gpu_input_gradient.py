@@ -70,3 +70,37 @@ def test_values_that_are_not_finite_or_leave_the_pieces(bits, dtype):
     assert torch.equal(y.isfinite(), plain.isfinite())
     ok = plain.isfinite()
     assert float((y[ok].double() - plain[ok].double()).norm()) <= 2.0 ** -7 * float(plain[ok].double().norm())
+
+
+def shares_not_nearest(x, q, s, b, group, bits, ref):
+    """Of the results, and of the plain kernel's: the share that is not the float64 product's nearest value.  It measures what the sums
+    lose before the last rounding, an error d moving a result over a rounding boundary with probability |d| / spacing."""
+    import mlx_rs_amd as m
+    run = lambda v: m.ops.quantized_matmul(v, q, s, b, transpose=False, group_size=group, bits=bits)  # noqa: E731
+    return tuple(float((v != ref.to(x.dtype)).double().mean()) for v in (run(x), run(off_by_one(x))))
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("bits,group", [(4, 32), (4, 64), (8, 64), (8, 128)])
+@pytest.mark.parametrize("rows,n,k", [(20, 1024, 4096), (300, 2048, 2048), (1100, 2176, 1024)])
+def test_sums_lose_no_more_than_plain_ones(rows, n, k, bits, group, dtype):
+    """Matrices as quantize makes them, whose weights two pieces hold."""
+    x, q, s, b = operands(rows, n, k, bits, group, getattr(torch, dtype))
+    share, plain = shares_not_nearest(x, q, s, b, group, bits, x.double() @ dequantized(q, s, b, group, bits))
+    assert share <= 1.25 * plain + 1e-4, (share, plain)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows,n,k", [(20, 256, 1096), (300, 2176, 264), (1100, 2176, 328)])
+def test_weights_of_more_bits_than_two_pieces(rows, n, k, bits):
+    """Groups far from zero, 1 + q / 2^13, in some steps of K only, and rows that sum to zero, so that the rest of a weight is all that
+    counts.  Two pieces of bfloat16 hold 17 bits of its 20 and more, which leaves a share of 0.11 to 0.14.  (Sums that
+    cancel as a whole: a matrix instruction cuts a unit of its largest term off each of its sums where an fma rounds once.)"""
+    x, q, s, b = operands(rows, n, k, bits, 64, torch.bfloat16)
+    q = torch.randint(-2 ** 31, 2 ** 31, q.shape, dtype=torch.int32, device="cuda")
+    x[:, 1::2] = -x[:, ::2]
+    far = (torch.arange(k, device="cuda") // 32 % 3 != 1).unsqueeze(1)
+    s, b = torch.where(far, torch.full_like(s, 1.37 * 2.0 ** -13), torch.zeros_like(s)), torch.where(far, torch.ones_like(b), b.abs())
+    pairs = dequantized(q, s, b, 64, bits)
+    share, plain = shares_not_nearest(x, q, s, b, 64, bits, x[:, ::2].double() @ (pairs[::2] - pairs[1::2]))
+    assert share <= 6 * plain + 2e-3, (share, plain)
