@@ -204,27 +204,46 @@ __device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {  // two b
   return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
 
-// One element of a product of weights packed along K, an fma per k on the dequantised weight.  The products on raw codes
-// take it where their own sum is not finite: an infinity against codes and biases apart cancels to no number where
+// ROWS rows of x against one row of weights packed along K, an fma per k on the dequantised weight, in the order of k.  The products
+// on raw codes take it where their own sum is not finite: an infinity against codes and biases apart cancels to no number where
 // the dequantised weight keeps its sign, and sums of unscaled codes overflow earlier.  paired: x has every 8-block as
-// (0,4)(1,5)(2,6)(3,7).
-template <int BITS, class T>
-__device__ __forceinline__ float plain_element(const T *x, bool paired, const uint32_t *w, const T *s, const T *b, int K, int group) {
-  constexpr int PER = 32 / BITS;  // a word of codes at a time; the x of a word is 8 to 32 aligned bytes
-  float sum = 0.f;
+// (0,4)(1,5)(2,6)(3,7).  open: the rows that are wanted.  K and the group are multiples of 32, x and w are aligned for 16 bytes.
+// It is one lane's chain over K and the latency of its loads, so 32 values of each row are fetched at a time.
+// us of a product 4096 x 4096 with finite rows / one infinity in one row / one in each: bf16 4-bit 1 row 12 / 79, 16 rows 17 / 89 / 284, 200 rows 36 /
+// 200 / 1460, 1000 rows 66 / 274 / 1840; f16 8-bit 777 rows 58 / 222 / 1830 (one row and word at a time 12 / 108, 17 / 118 / 480, 38 / 174 / 5530, 73 /
+// 268 / 11800, 61 / 290 / 24000; a wave per output element 3160 for the last).  Rows of NaNs cost next to nothing.
+template <int BITS, int ROWS, class T>
+__device__ __forceinline__ void plain_rows(const T *const (&x)[ROWS], bool paired, const uint32_t *w, const T *s, const T *b, int K, int group,
+                                           uint32_t open, float (&sum)[ROWS]) {
+  static_assert(sizeof(T) == 2, "eight values are 16 bytes");
+  constexpr int PER = 32 / BITS;  // codes of a word
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) sum[r] = 0.f;
 #pragma unroll 1
-  for (int k = 0; k < K && sum == sum; k += PER) {  // (no number stays none)
-    T v[PER];
-    __builtin_memcpy(v, __builtin_assume_aligned(x + k, PER * sizeof(T) < 16 ? 8 : 16), sizeof v);
-    const uint32_t word = w[k / PER];
+  for (int k = 0; k < K && open; k += 32) {
+    uint4 xv[ROWS][4];
+    uint32_t words[BITS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xv[r][i] = reinterpret_cast<const uint4 *>(x[r] + k)[i];
+    __builtin_memcpy(words, __builtin_assume_aligned(w + k / PER, 16), sizeof words);
     const float sc = as_f32(s[k / group]), bi = as_f32(b[k / group]);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const float xv = as_f32(paired ? v[(i & ~7) | (i & 3) << 1 | (i >> 2 & 1)] : v[i]);
-      sum = __builtin_fmaf(xv, __builtin_fmaf(sc, (float)((word >> (i * BITS)) & ((1u << BITS) - 1u)), bi), sum);
+    for (int i = 0; i < 32; ++i) {
+      const int at = i & 7, from = paired ? (at & 3) << 1 | at >> 2 : at;
+      const float wf = __builtin_fmaf(sc, (float)((words[i / PER] >> (i % PER * BITS)) & ((1u << BITS) - 1u)), bi);
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        T v[8];
+        __builtin_memcpy(v, &xv[r][i / 8], sizeof v);
+        sum[r] = __builtin_fmaf(as_f32(v[from]), wf, sum[r]);
+      }
     }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+      if (sum[r] != sum[r]) open &= ~(1u << r);  // (no number stays none)
   }
-  return sum;
 }
 
 // ---------------------------------------------------------------- device-coherent accesses

@@ -585,22 +585,31 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
         put(r, v, up);
         again |= (not_finite(v) || (GLU && not_finite(up)) ? 1u : 0u) << r;
       }
-      while (again) {
-        const int r = __builtin_ctz(again);
-        again &= again - 1;
-        const int tr = 32 * m + 8 * (r >> 2) + 4 * kb + (r & 3);
-        if (tr >= rows) continue;
-        const T *const xs = static_cast<const T *>(a.x) + (int64_t)(a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr)) * K;
-        float v[2];
+#pragma unroll 1
+      for (int quad = 0; quad < 4; ++quad) {  // rows 8 quad + 4 kb + 0 .. 3
+        uint32_t open = again >> (4 * quad) & 15u;
+        const T *xs[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          int tr = 32 * m + 8 * quad + 4 * kb + i;
+          if (tr >= rows) {  // (never stored)
+            open &= ~(1u << i);
+            tr = rows - 1;
+          }
+          xs[i] = static_cast<const T *>(a.x) + (int64_t)(a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr)) * K;
+        }
+        if (!open) continue;
+        float v[GLU ? 2 : 1][4];
 #pragma unroll
         for (int i = 0; i < (GLU ? 2 : 1); ++i) {
-          const int tt = GLU ? i : t;
-          const int64_t wrow = ebase + w_row[tt];
-          v[i] = plain_element<BITS, T>(xs, paired_order(BITS), (GLU && i ? a.w1 : a.w0) + wrow * (row_bytes / 4),
-                                        static_cast<const T *>(GLU && i ? a.s1 : a.s0) + wrow * G,
-                                        static_cast<const T *>(GLU && i ? a.b1 : a.b0) + wrow * G, K, K / G);
+          const int64_t wrow = ebase + w_row[GLU ? i : t];
+          plain_rows<BITS, 4, T>(xs, paired_order(BITS), (GLU && i ? a.w1 : a.w0) + wrow * (row_bytes / 4),
+                              static_cast<const T *>(GLU && i ? a.s1 : a.s0) + wrow * G,
+                              static_cast<const T *>(GLU && i ? a.b1 : a.b0) + wrow * G, K, K / G, open, v[i]);
         }
-        put(r, v[0], v[GLU ? 1 : 0]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (open >> i & 1u) put(4 * quad + i, v[0][i], v[GLU ? 1 : 0][i]);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();

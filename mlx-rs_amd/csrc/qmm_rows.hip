@@ -371,16 +371,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
       while (again) {
         const int r = __builtin_ctz(again);
         again &= again - 1;
-        const int64_t rr = r0 + t0 + 4 * kb + r;
-        const T *const xr = static_cast<const T *>(a.x) + (a.src_rows ? (int64_t)a.src_rows[rr] : rr) * K;
-        float v[NM];
+        const int64_t rr = r0 + t0 + 4 * kb + r, wrow = ebase + n0 + c;
+        const T *const xr[1] = {static_cast<const T *>(a.x) + (a.src_rows ? (int64_t)a.src_rows[rr] : rr) * K};
+        float v[NM][1];
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-          const int64_t wrow = ebase + n0 + c;
-          v[m] = plain_element<BITS, T>(xr, false, (m ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const T *>(m ? a.s1 : a.s0) + wrow * G,
-                                        static_cast<const T *>(m ? a.b1 : a.b0) + wrow * G, K, GROUP);
-        }
-        put(r, v[0], v[NM - 1]);
+        for (int m = 0; m < NM; ++m)
+          plain_rows<BITS, 1, T>(xr, false, (m ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const T *>(m ? a.s1 : a.s0) + wrow * G,
+                                 static_cast<const T *>(m ? a.b1 : a.b0) + wrow * G, K, GROUP, 1u, v[m]);
+        put(r, v[0][0], v[NM - 1][0]);
       }
     }
   }
