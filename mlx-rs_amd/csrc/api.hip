@@ -192,7 +192,7 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws) {
   if (f.raw && raw_tiled_batch(c, T)) {
     f.raw_cap = (int)(P / kBigTileM + (P / (kRowsMost + 1) < c.n_experts ? P / (kRowsMost + 1) : c.n_experts));
     f.raw_tiles = cv.take<uint32_t>(tile_list_words(f.raw_cap, c.n_experts));
-    f.raw_copy = cv.take<uint16_t>(codes_copy_bytes(MI_MOE_DTYPE_BF16, c.bits, T, c.hidden) / 2);
+    f.raw_copy = cv.take<uint16_t>(codes_copy_bytes(c.bits, T, c.hidden) / 2);
     f.raw_xsums = cv.take<uint16_t>(codes_sums_bytes(T, c.hidden, c.group_size) / 2);
     f.raw_hsums = cv.take<uint16_t>(codes_sums_bytes(P, c.intermediate, c.group_size) / 2);
   }
@@ -483,7 +483,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     rd.y = f.y;
     rd.N = c.hidden; rd.K = c.intermediate;
     CodesArgs ca{}, cd{};
-    const bool copied = codes_copy_bytes(MI_MOE_DTYPE_BF16, c.bits, T, c.hidden) > 0;
+    const bool copied = codes_copy_bytes(c.bits, T, c.hidden) > 0;
     ca.x = copied ? f.raw_copy : x;
     ca.x_rows = T;
     ca.sums = f.raw_xsums;
@@ -985,16 +985,16 @@ static size_t qmm_dense_bytes(int64_t M, int32_t K, int32_t bits, size_t *mt_wor
   return b;
 }
 
-static size_t codes_bytes(int64_t M, int32_t K, int32_t group_size, int32_t bits, int32_t dtype) {
-  return 256 + align_up(codes_copy_bytes(dtype, bits, M, K)) + align_up(codes_sums_bytes(M, K, group_size));
+static size_t codes_bytes(int64_t M, int32_t K, int32_t group_size, int32_t bits) {
+  return 256 + align_up(codes_copy_bytes(bits, M, K)) + align_up(codes_sums_bytes(M, K, group_size));
 }
 
 int mi_moe_quantized_matmul_workspace_size(int64_t M, int32_t K, int32_t bits, size_t *bytes) try {
   if (!bytes) return fail("quantized_matmul_workspace_size: bytes is NULL");
   if (M < 0 || K <= 0 || M * (int64_t)K > (int64_t)1 << 40) return fail("quantized_matmul_workspace_size: bad sizes");
   size_t mt = 0;
-  const size_t tuned = qmm_dense_bytes(M, K, bits, &mt), codes = codes_bytes(M, K, 32, bits, MI_MOE_DTYPE_F16);
-  *bytes = tuned > codes ? tuned : codes;  // (the group size and the element type are not known here: the largest need)
+  const size_t tuned = qmm_dense_bytes(M, K, bits, &mt), codes = codes_bytes(M, K, 32, bits);
+  *bytes = tuned > codes ? tuned : codes;  // (the group size is not known here: the largest need)
   return 0;
 } MI_CATCH("quantized_matmul_workspace_size")
 
@@ -1069,10 +1069,10 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
   const bool streamed = tuned && bits == 8 && M < tiled_avg_rows(bits);  // (see dense_takes_rows)
   const bool large_tiles = tuned && codes && !streamed && dense_takes_large_tiles(M, N);
   // (x and w are read and y is written 16 bytes at a time, scales and biases by words)
-  if (codes && !one_plain && !streamed && !large_tiles && M * K * 4 < (int64_t)1 << 31 && workspace && workspace_bytes >= codes_bytes(M, K, group_size, bits, dtype) && aligned16(x) && aligned16(w) && aligned16(y) &&
+  if (codes && !one_plain && !streamed && !large_tiles && M * K * 4 < (int64_t)1 << 31 && workspace && workspace_bytes >= codes_bytes(M, K, group_size, bits) && aligned16(x) && aligned16(w) && aligned16(y) &&
       ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 3u) == 0) {
     Carver cv(workspace);
-    const size_t copy_bytes = codes_copy_bytes(dtype, bits, M, K);
+    const size_t copy_bytes = codes_copy_bytes(bits, M, K);
     uint16_t *copy = copy_bytes ? reinterpret_cast<uint16_t *>(cv.take<char>(copy_bytes)) : nullptr;
     uint16_t *sums = reinterpret_cast<uint16_t *>(cv.take<char>(codes_sums_bytes(M, K, group_size)));
     MI_HIP(launch_prepare_rows(x, M, K, group_size, dtype, copy, sums, st));

@@ -176,75 +176,12 @@ __host__ __device__ inline P *tile_list(P *base, int cls, int cap256, int n_expe
   return base + 4 + 4 * (size_t)cap256 + 4 + 4 * (size_t)n_experts;
 }
 
-// ---------------------------------------------------------------- element types, one element the plain way
+// ---------------------------------------------------------------- element types
 __device__ __forceinline__ float as_f32(uint16_t v) { return bf16_to_f32(v); }  // bfloat16, raw bits
 __device__ __forceinline__ float as_f32(_Float16 v) { return (float)v; }
 __device__ __forceinline__ float as_f32(float v) { return v; }
 
 __device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
-
-// The products on raw codes multiply centred codes q - 8 and q - 128: s q + b = s (q - c) + (b + c s).  Without the centre the code
-// and bias terms of a group are several times their sum, and what they lose to each other's rounding is too.
-constexpr float centre_of(int bits) { return (float)(1 << (bits - 1)); }
-// Centred codes of one word as f32: two 4-bit codes a byte, times 16 (their byte's upper half), or 8-bit ones.  The signed byte
-// comes out of the conversion itself.
-__device__ __forceinline__ void centred_codes(uint32_t w, float (&v)[8]) {  // 4-bit: 16 (q_i - 8)
-  const uint32_t even = ((w << 4) ^ 0x88888888u) & 0xf0f0f0f0u, odd = (w ^ 0x88888888u) & 0xf0f0f0f0u;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    v[2 * i] = (float)(int8_t)(even >> (8 * i));
-    v[2 * i + 1] = (float)(int8_t)(odd >> (8 * i));
-  }
-}
-__device__ __forceinline__ void centred_codes(uint32_t w, float (&v)[4]) {  // 8-bit: q_i - 128
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = (float)(int8_t)((w ^ 0x80808080u) >> (8 * i));
-}
-__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {  // two bf16 of values that are bf16 already
-  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-
-// ROWS rows of x against one row of weights packed along K, an fma per k on the dequantised weight, in the order of k.  The products
-// on raw codes take it where their own sum is not finite: an infinity against codes and biases apart cancels to no number where
-// the dequantised weight keeps its sign, and sums of unscaled codes overflow earlier.  paired: x has every 8-block as
-// (0,4)(1,5)(2,6)(3,7).  open: the rows that are wanted.  K and the group are multiples of 32, x and w are aligned for 16 bytes.
-// It is one lane's chain over K and the latency of its loads, so 32 values of each row are fetched at a time.
-// us of a product 4096 x 4096 with finite rows / one infinity in one row / one in each: bf16 4-bit 1 row 12 / 79, 16 rows 17 / 89 / 284, 200 rows 36 /
-// 200 / 1460, 1000 rows 66 / 274 / 1840; f16 8-bit 777 rows 58 / 222 / 1830 (one row and word at a time 12 / 108, 17 / 118 / 480, 38 / 174 / 5530, 73 /
-// 268 / 11800, 61 / 290 / 24000; a wave per output element 3160 for the last).  Rows of NaNs cost next to nothing.
-template <int BITS, int ROWS, class T>
-__device__ __forceinline__ void plain_rows(const T *const (&x)[ROWS], bool paired, const uint32_t *w, const T *s, const T *b, int K, int group,
-                                           uint32_t open, float (&sum)[ROWS]) {
-  static_assert(sizeof(T) == 2, "eight values are 16 bytes");
-  constexpr int PER = 32 / BITS;  // codes of a word
-#pragma unroll
-  for (int r = 0; r < ROWS; ++r) sum[r] = 0.f;
-#pragma unroll 1
-  for (int k = 0; k < K && open; k += 32) {
-    uint4 xv[ROWS][4];
-    uint32_t words[BITS];
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) xv[r][i] = reinterpret_cast<const uint4 *>(x[r] + k)[i];
-    __builtin_memcpy(words, __builtin_assume_aligned(w + k / PER, 16), sizeof words);
-    const float sc = as_f32(s[k / group]), bi = as_f32(b[k / group]);
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-      const int at = i & 7, from = paired ? (at & 3) << 1 | at >> 2 : at;
-      const float wf = __builtin_fmaf(sc, (float)((words[i / PER] >> (i % PER * BITS)) & ((1u << BITS) - 1u)), bi);
-#pragma unroll
-      for (int r = 0; r < ROWS; ++r) {
-        T v[8];
-        __builtin_memcpy(v, &xv[r][i / 8], sizeof v);
-        sum[r] = __builtin_fmaf(as_f32(v[from]), wf, sum[r]);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r)
-      if (sum[r] != sum[r]) open &= ~(1u << r);  // (no number stays none)
-  }
-}
 
 // ---------------------------------------------------------------- device-coherent accesses
 // A load that observes what other workgroups have written before an agent-scope release
@@ -271,9 +208,9 @@ struct KernelTimer {
 extern thread_local KernelTimer *g_kernel_timer;
 
 // ---------------------------------------------------------------- which kernels the library holds, and which ran
-// Every instantiation of a grouped-product kernel that a launcher can reach owns one slot (a static of
-// the launcher's template, registered when the library is loaded), so the list is complete whether or
-// not a kernel has ever run.  launch_kernel counts the launch in the slot.  With a plan installed on the
+// Every instantiation of the streaming and the 256-column grouped product (qmm.hip, qmm_large.hip) that a launcher can reach
+// owns one slot (a static of the launcher's template, registered when the library is loaded), so the list is complete
+// whether or not a kernel has ever run.  The products on raw codes and the input gradient have none.  launch_kernel counts the launch in the slot.  With a plan installed on the
 // calling thread (mi_moe_debug_plan) nothing is launched: the slot's name, grid and LDS size are
 // written to the plan instead, which lets the launchers' host-side choices be checked without a GPU.
 struct KernelSlot {
@@ -396,7 +333,7 @@ hipError_t launch_qmm_plain(const void *x, const uint32_t *w, const void *scales
                             const uint32_t *lhs, const uint32_t *rhs, const uint32_t *rhs_map,
                             const uint32_t *dst_map, uint32_t n_lhs, uint32_t n_rhs, int64_t rows, int M, int N,
                             int K, int group, int bits, bool transpose, int dt, void *y, hipStream_t st);
-// The tiled product on raw codes (qmm_codes.hip): any float type, groups of 32 / 64 / 128, 4- and 8-bit codes,
+// The tiled product on raw codes (qmm_codes.hip): bfloat16 and float16, groups of 32 / 64 / 128, 4- and 8-bit codes,
 // transposed weights.  x: what launch_prepare_rows made of the rows (`copy` where codes_copy_bytes is not zero, else
 // the rows themselves), sums: the group sums it wrote.
 struct CodesArgs {
@@ -441,7 +378,7 @@ struct ColsArgs {
 };
 bool qmm_cols_applies(const ColsArgs &a, int bits, int dt);
 hipError_t launch_qmm_cols(const ColsArgs &a, int group, int bits, int dt, hipStream_t st);
-size_t codes_copy_bytes(int dt, int bits, int64_t rows, int K);
+size_t codes_copy_bytes(int bits, int64_t rows, int K);
 size_t codes_sums_bytes(int64_t rows, int K, int group);
 hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
                                uint16_t *sums, hipStream_t st);

@@ -22,7 +22,7 @@
 // and f16, the copy with paired 8-blocks that their unpacking wants.
 #include <type_traits>
 
-#include "common.hpp"
+#include "qmm_dev.hpp"
 
 namespace mi_moe {
 
@@ -32,32 +32,10 @@ constexpr int kStep = 64;      // K values per step; two steps between barriers
 constexpr int kRow = 17;       // LDS row stride in 16-byte units: 128 values and 16 bytes that keep rows off each other's banks
 constexpr uint32_t kOutside = 0x80000000u;  // an offset past every descriptor here: such a load returns zeros
 constexpr int kSlots = 8;      // K slots of a group in the bias product
-#ifndef MI_CODES_WEAVE
-#define MI_CODES_WEAVE 7
-#endif
-constexpr int kWeave = MI_CODES_WEAVE;  // vector instructions between two matrix instructions
-constexpr size_t kLdsAtLeast = 4 * 32 * (32 * 4 + 16);  // the epilogue's staging
+constexpr int kWeave = 7;  // vector instructions between two matrix instructions
+constexpr size_t kLdsAtLeast = 4 * 32 * (32 * 2 + 16);  // the epilogue's staging
 
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
 typedef uint32_t u32x3_t __attribute__((ext_vector_type(3)));
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
-
-template <int DT> struct ElemOf;
-template <> struct ElemOf<0> { typedef uint16_t type; };
-template <> struct ElemOf<1> { typedef _Float16 type; };
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void *base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
-}
-
-template <int DT>
-__device__ __forceinline__ f32x16_t mfma(u32x4_t a, u32x4_t b, f32x16_t c) {
-  if constexpr (DT == 1)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
 
 // v = h + m + l exactly, each a bf16 (8 significant bits; by truncation, so nothing overflows).  A value that is not
 // finite gives a NaN.
@@ -80,22 +58,8 @@ struct Split : F {
 template <bool SPLIT, class F>
 __device__ __forceinline__ Split<SPLIT, F> with_split(F f) { return Split<SPLIT, F>(f); }
 
-// a thread's share of a step's token rows
-template <int P, int NA>
-struct RowStage {
-  u32x4_t v[P][NA];
-};
-
 constexpr bool paired_order(int bits) { return bits == 4; }  // 8-blocks as (0,4)(1,5)(2,6)(3,7)
 constexpr int padded_groups(int G) { return (G + 15) / 16 * 16; }  // the bias product runs an even number of steps of eight groups
-
-template <int BITS>
-__device__ __forceinline__ uint32_t f16_centred(uint32_t v) {  // two halves 1024 + q -> q - centre: exact
-  constexpr _Float16 off = (_Float16)(1024.0f + centre_of(BITS));
-  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) - half2_t{off, off});
-}
-template <class T> __device__ __forceinline__ T rounded(float v) { return (T)v; }
-template <> __device__ __forceinline__ uint16_t rounded<uint16_t>(float v) { return (uint16_t)(cvt_pk_bf16(v, 0.f) & 0xffffu); }
 
 }  // namespace
 
@@ -268,6 +232,9 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
     for (int t = 0; t < NT; ++t) tot[m][t] = zero;
 
+  struct StageA {  // a thread's share of a step's token rows
+    u32x4_t v[NA];
+  };
   struct Operand {  // a step's weight operand: eight values a lane and multiply
     u32x4_t v[NT][4];
   };
@@ -279,15 +246,14 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   // window_steps, window: called ahead of every so many steps.
   // Inside a step the sub-tiles follow each other, each with the reads of the next one's token rows ahead of its
   // multiplies and its share of the unpacking between them; nothing moves across a sub-tile.
-  auto pass = [&](int nk, auto parts, auto a_type, auto b_type, auto load_a, auto put_a, auto load_b, auto unpack, auto begin, auto multiply, int window_steps, auto window) __attribute__((always_inline)) {
-    constexpr int P = decltype(parts)::value;
-    decltype(a_type) RA[2];
+  auto pass = [&](int nk, auto b_type, auto load_a, auto load_b, auto unpack, auto begin, auto multiply, int window_steps, auto window) __attribute__((always_inline)) {
+    StageA RA[2];
     decltype(b_type) RB[2];
     auto put = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
       for (int d = 0; d < 2; ++d)
 #pragma unroll
-        for (int i = 0; i < NA; ++i) put_a(lds + buf * BUF + (arg + RS * i) * kRow + 8 * d + acp, RA[d], i);
+        for (int i = 0; i < NA; ++i) lds[buf * BUF + (arg + RS * i) * kRow + 8 * d + acp] = RA[d].v[i];
     };
     const int share = nk_share(nk);  // the same number of barriers for every group
     const int k0 = kg * share, k1 = k0 + share < nk ? k0 + share : nk;
@@ -303,13 +269,11 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
       for (int h = 0; h < 4; ++h) unpack(RB[0], op[0], t, h);
     put(0);
     __syncthreads();
-    u32x4_t F[2][4][P];  // the token operand of a sub-tile row, and of the next
-    auto fetch = [&](const u32x4_t *At, int m, bool split, u32x4_t (&to)[4][P]) __attribute__((always_inline)) {
+    u32x4_t F[2][4];  // the token operand of a sub-tile row, and of the next
+    auto fetch = [&](const u32x4_t *At, int m, bool split, u32x4_t (&to)[4]) __attribute__((always_inline)) {
 #pragma unroll
       for (int h = 0; h < 4; ++h)
-#pragma unroll
-        for (int p = 0; p < P; ++p)
-          to[h][p] = At[p * A_SZ + (32 * m + ln) * kRow + (split ? 4 * (h >> 1) + 2 * kb + (h & 1) : 4 * kb + h)];  // the chunk multiply h takes
+        to[h] = At[(32 * m + ln) * kRow + (split ? 4 * (h >> 1) + 2 * kb + (h & 1) : 4 * kb + h)];  // the chunk multiply h takes
     };
     int buf = 0;
     for (int kw = k0; kw < k0 + share; kw += window_steps) {
@@ -337,9 +301,9 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
               constexpr int UNITS = 4 * NT, TILES = MS * NT;
 #pragma unroll
               for (int u = UNITS * (m * NT + t) / TILES; u < UNITS * (m * NT + t + 1) / TILES; ++u) unpack(RB[d ^ 1], op[d ^ 1], u / 4, u % 4);
-              if (t == 0 && (m + 1 < MS || d == 0)) __builtin_amdgcn_sched_group_barrier(0x100, 4 * P, 0);
+              if (t == 0 && (m + 1 < MS || d == 0)) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
-              for (int i = 0; i < 4 * P; ++i) {
+              for (int i = 0; i < 4; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x002, kWeave, 0);
               }
@@ -357,8 +321,6 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
 
   // ---- the bias product: group sums of x against b + centre s, accumulated into the result
   {
-    typedef RowStage<1, NA> StageA;
-    auto put_a = [&](u32x4_t *to, const StageA &R, int i) __attribute__((always_inline)) { *to = R.v[0][i]; };
     // A lane's four groups of a step are three words, as a row may start between two.  Groups past the row's end are another
     // row's or zeros: their sums are zero.
     struct StageB {
@@ -367,7 +329,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     auto load_a = [&](int ks, bool real, StageA &R) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < NA; ++i)
-        R.v[0][i] = __builtin_amdgcn_raw_buffer_load_b128(xsr, KW == 1 || real ? xs_voff[i] : kOutside, ks * (kStep * 2), 0);
+        R.v[i] = __builtin_amdgcn_raw_buffer_load_b128(xsr, KW == 1 || real ? xs_voff[i] : kOutside, ks * (kStep * 2), 0);
     };
     auto load_b = [&](int ks, StageB &R) __attribute__((always_inline)) {
 #pragma unroll
@@ -385,20 +347,16 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
       const Pieces p = split3(__builtin_fmaf(centre_of(BITS), group(R.s[t]), group(R.b[t])));
       o.v[t][h] = u32x4_t{p.h | p.h << 16, p.h | p.m << 16, p.m | p.l << 16, 0u};
     };
-    auto body = [&](const u32x4_t (&av)[4][1], const Operand &o, int, int m, int t) __attribute__((always_inline)) {
+    auto body = [&](const u32x4_t (&av)[4], const Operand &o, int, int m, int t) __attribute__((always_inline)) {
 #pragma unroll
-      for (int h = 0; h < 4; ++h) tot[m][t] = mfma<0>(av[h][0], o.v[t][h], tot[m][t]);
+      for (int h = 0; h < 4; ++h) tot[m][t] = mfma<0>(av[h], o.v[t][h], tot[m][t]);
     };
-    pass(pg / 8, std::integral_constant<int, 1>{}, StageA{}, StageB{}, load_a, put_a, load_b, unpack, [](int, int) {},
+    pass(pg / 8, StageB{}, load_a, load_b, unpack, [](int, int) {},
          with_split<false>(body), 1 << 30, [](int) {});
   }
 
   // ---- the product of the codes
   {
-    typedef RowStage<1, NA> StageA;
-    auto put_a = [&](u32x4_t *to, const StageA &R, int i) __attribute__((always_inline)) {
-      *to = R.v[0][i];
-    };
     struct StageB {
       u32x4_t q[NT][NQ];
     };
@@ -412,10 +370,8 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     };
     auto load_a = [&](int ks, bool real, StageA &R) __attribute__((always_inline)) {
 #pragma unroll
-      for (int p = 0; p < 1; ++p)
-#pragma unroll
-        for (int i = 0; i < NA; ++i)
-          R.v[p][i] = __builtin_amdgcn_raw_buffer_load_b128(xr, KW == 1 || real ? x_voff[i] : kOutside, ks * (kStep * (uint32_t)sizeof(T)) + 16 * p, 0);
+      for (int i = 0; i < NA; ++i)
+        R.v[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, KW == 1 || real ? x_voff[i] : kOutside, ks * (kStep * (uint32_t)sizeof(T)), 0);
     };
     auto load_b = [&](int ks, StageB &R) __attribute__((always_inline)) {
 #pragma unroll
@@ -504,19 +460,19 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
         for (int i = 0; i < NS; ++i)
           step_s[d][t][i] = kUnit * as_f32(*reinterpret_cast<const T *>(s_at[t] + ((G32 ? 2 * ks + i : ks >> scale_shift) - gw) * (int)sizeof(T)));
     };
-    auto body = [&](const u32x4_t (&av)[4][1], const Operand &o, int d, int m, int t) __attribute__((always_inline)) {
+    auto body = [&](const u32x4_t (&av)[4], const Operand &o, int d, int m, int t) __attribute__((always_inline)) {
       const int tile = m * NT + t;
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
         const int which = ((d * MS * NT + tile) * NS + i) & 1;
 #pragma unroll
         for (int h = 4 / NS * i; h < 4 / NS * (i + 1); ++h)
-          acc[which] = mfma<DT>(av[h][0], o.v[t][h], h == 4 / NS * i ? zero : acc[which]);
+          acc[which] = mfma<DT>(av[h], o.v[t][h], h == 4 / NS * i ? zero : acc[which]);
         acc_s[which] = step_s[d][t][i];
         add_scaled(which ^ 1, i > 0 ? tile : tile > 0 ? tile - 1 : MS * NT - 1);
       }
     };
-    pass(K / kStep, std::integral_constant<int, 1>{}, StageA{}, StageB{}, load_a, put_a, load_b, unpack, begin, with_split<SPLIT>(body),
+    pass(K / kStep, StageB{}, load_a, load_b, unpack, begin, with_split<SPLIT>(body),
          (win >> (G32 ? 1 : 0)) << scale_shift, window);
     add_scaled(1, MS * NT - 1);  // an even number of steps ends in accumulator 1
   }
@@ -636,7 +592,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     }
 }
 
-size_t codes_copy_bytes(int dt, int bits, int64_t rows, int K) {
+size_t codes_copy_bytes(int bits, int64_t rows, int K) {
   return paired_order(bits) ? (size_t)rows * K * 2 : 0;
 }
 size_t codes_sums_bytes(int64_t rows, int K, int group) { return (size_t)rows * padded_groups(K / group) * kSlots * 2; }

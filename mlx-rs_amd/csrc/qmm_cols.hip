@@ -19,7 +19,7 @@
 // one result at a time 50 / 1620 / 11700); 20 rows f16 20 / 256 / 270, weights beyond 64 270 (4120).
 #include <type_traits>
 
-#include "common.hpp"
+#include "qmm_dev.hpp"
 
 namespace mi_moe {
 
@@ -27,29 +27,6 @@ namespace {
 
 constexpr int kStep = 32;                   // K values per step
 constexpr uint32_t kOutside = 0x80000000u;  // an offset past every descriptor here: such a load returns zeros
-
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
-
-template <int DT> struct ElemOf;
-template <> struct ElemOf<0> { typedef uint16_t type; };
-template <> struct ElemOf<1> { typedef _Float16 type; };
-template <> struct ElemOf<2> { typedef float type; };
-
-template <class T> __device__ __forceinline__ T rounded(float v) { return (T)v; }
-template <> __device__ __forceinline__ uint16_t rounded<uint16_t>(float v) { return f32_to_bf16(v); }
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void *base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
-}
-template <int DT>
-__device__ __forceinline__ f32x16_t mfma(u32x4_t a, u32x4_t b, f32x16_t c) {
-  if constexpr (DT == 1)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
 
 constexpr int pieces_of_x(int dt) { return dt == 2 ? 3 : 1; }
 constexpr int pieces_of_w(int dt) { return dt == 2 ? 3 : 2; }

@@ -11,7 +11,7 @@
 // tokens by 16 weight rows (v_mfma_f32_16x16x32), so it is four fma a lane and group.
 #include <type_traits>
 
-#include "common.hpp"
+#include "qmm_dev.hpp"
 
 namespace mi_moe {
 
@@ -20,43 +20,16 @@ namespace {
 constexpr int kTokens = 16;  // token slots of a tile
 constexpr int kRing = 4;     // 16-byte code loads in flight per lane and matrix (8: no change at any size)
 
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
-
-template <int DT> struct ElemOf;
-template <> struct ElemOf<0> { typedef uint16_t type; };
-template <> struct ElemOf<1> { typedef _Float16 type; };
-
-template <class T> __device__ __forceinline__ T rounded(float v) { return (T)v; }
-template <> __device__ __forceinline__ uint16_t rounded<uint16_t>(float v) { return (uint16_t)(cvt_pk_bf16(v, 0.f) & 0xffffu); }
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void *base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
-}
-template <int DT>
-__device__ __forceinline__ f32x4_t mfma(u32x4_t a, u32x4_t b, f32x4_t c) {
-  if constexpr (DT == 1)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
 // Two bytes 0 to 15 as bf16, the lower or the upper ones of v: below 16 an e4m3 number is its byte in units of 2^-9.
 template <int UPPER>
 __device__ __forceinline__ uint32_t small_codes(uint32_t v) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f, UPPER != 0));
 }
-template <int BITS>
-__device__ __forceinline__ uint32_t f16_centred(uint32_t v) {  // two halves 1024 + q -> q - centre: exact
-  constexpr _Float16 off = (_Float16)(1024.0f + centre_of(BITS));
-  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v) - half2_t{off, off});
-}
-
 // LDS of a launch: token rows of sk values (tt of them), 64 zero bytes, the sums of x over each group and
 // token slot, the (scale, bias) pairs of the block's weight rows, and the partial sums of a shared K.
 struct RowsLds {
   int x_stride, zeros, sums, pairs, pair_row, parts, bytes;
-  __host__ __device__ RowsLds(int dt, int group, int nm, int kw, int K, int sk, int tt) {
+  __host__ __device__ RowsLds(int group, int nm, int kw, int K, int sk, int tt) {
     const int nw = 4 / kw;
     x_stride = 2 * sk + 16;
     zeros = tt * x_stride;
@@ -113,7 +86,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
   const int64_t ebase = (int64_t)e * N;
 
   extern __shared__ __align__(16) unsigned char lds[];
-  const RowsLds L(DT, GROUP, NM, KW, K, sk, tt);
+  const RowsLds L(GROUP, NM, KW, K, sk, tt);
   float *const sums = reinterpret_cast<float *>(lds + L.sums);
 
   __amdgpu_buffer_rsrc_t wr[NM];
@@ -150,13 +123,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
       unsigned char *to = lds + L.pairs + (tile * 16 + row) * L.pair_row + g * 2 * (int)sizeof(T);
 #pragma unroll
       for (int i = 0; i < PV; ++i) {
-        if constexpr (sizeof(T) == 4) {
-          reinterpret_cast<uint32_t *>(to)[0] = sv[i];
-          reinterpret_cast<uint32_t *>(to)[1] = bv[i];
-        } else {
-          *reinterpret_cast<uint32_t *>(to) = (i & 1) ? __builtin_amdgcn_perm(bv[i >> 1], sv[i >> 1], 0x07060302u)
-                                                      : __builtin_amdgcn_perm(bv[i >> 1], sv[i >> 1], 0x05040100u);
-        }
+        *reinterpret_cast<uint32_t *>(to) = (i & 1) ? __builtin_amdgcn_perm(bv[i >> 1], sv[i >> 1], 0x07060302u)
+                                                    : __builtin_amdgcn_perm(bv[i >> 1], sv[i >> 1], 0x05040100u);
         to += 2 * sizeof(T);
         if (++g == G) {
           g = 0;
@@ -386,7 +354,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
 
 template <int DT, int BITS, int GROUP, bool GLU, int KW>
 static hipError_t start_rows(const RowsArgs &a, int sk, int tt, hipStream_t st) {
-  const RowsLds L(DT, GROUP, GLU ? 2 : 1, KW, a.K, sk, tt);
+  const RowsLds L(GROUP, GLU ? 2 : 1, KW, a.K, sk, tt);
   const auto kernel = &qmm_rows_kernel<DT, BITS, GROUP, GLU, KW>;
   if (L.bytes > 160 * 1024) return hipErrorInvalidConfiguration;
   if (L.bytes > 64 * 1024)
@@ -400,10 +368,16 @@ static hipError_t start_rows(const RowsArgs &a, int sk, int tt, hipStream_t st) 
 
 // How the launch is cut: K values of the token rows in LDS at a time (the whole row, or slabs that are a whole number of
 // ring turns for every wave), token rows a pass, waves that share a row tile's K.
+// The waves: with KW = 4 a block has 16 weight rows, so 1024 tiles are four blocks a CU, which is what the launch takes at once; from
+// there on fewer and longer waves are better.  Measured, us of the kernel with 4 / 2 / 1 waves a tile at 2 and at 8 rows, K = 4096
+// (1024 tiles and more: 2048): bf16 4-bit groups of 64, 128 tiles 6.8 / 8.8 / 12.6 and 11.4 / 13.1 / 17.5, 512 tiles 9.6 / 10.8 / 14.0 and 14.0 / 15.8 /
+// 19.0, 1024 tiles 9.6 / 8.9 / 9.2 and 15.2 / 10.9 / 11.5, 2048 tiles 14.1 / 11.9 / 11.3 and 22.8 / 18.7 / 14.3, 4096 tiles 23.2 / 19.5 / 17.4 and
+// 41.7 / 29.4 / 25.4; f16 8-bit, 512 tiles 12.8 / 15.6 / 20.8 and 18.5 / 21.6 / 26.5, 1024 tiles 10.8 / 11.0 / 12.6 and 17.9 / 13.8 / 15.4, 2048 tiles 18.6 /
+// 15.3 / 16.1 and 27.4 / 24.9 / 18.9.
 struct RowsCut {
   int kw, sk, tt;
 };
-static RowsCut cut_rows(const RowsArgs &a, int group, int bits, int dt, bool glu) {
+static RowsCut cut_rows(const RowsArgs &a, int group, int bits, bool glu) {
   const int ch = bits == 4 ? 128 : 64, nm = glu ? 2 : 1;
   const int64_t longest = a.work ? a.max_rows : a.M;
   const int tt = (int)(longest < kTokens ? longest : kTokens);
@@ -411,7 +385,7 @@ static RowsCut cut_rows(const RowsArgs &a, int group, int bits, int dt, bool glu
   int kw = tiles < 1024 ? 4 : (tiles < 2048 ? 2 : 1);
   for (;; kw /= 2) {
     const int unit = ch * kw * kRing;  // a slab: a multiple of this
-    auto bytes = [&](int sk) { return RowsLds(dt, group, nm, kw, a.K, sk, tt).bytes; };
+    auto bytes = [&](int sk) { return RowsLds(group, nm, kw, a.K, sk, tt).bytes; };
     int sk = a.K;
     if (bytes(sk) > 64 * 1024) {  // (two blocks a CU at least)
       sk = a.K / unit * unit;
@@ -425,11 +399,11 @@ static RowsCut cut_rows(const RowsArgs &a, int group, int bits, int dt, bool glu
 
 bool qmm_rows_applies(const RowsArgs &a, int group, int bits, int dt, bool glu) {
   return bits != 2 && dt != 2 && a.K % (bits == 4 ? 128 : 64) == 0 && a.K % group == 0 && (int64_t)a.N * a.K < (int64_t)1 << 31 &&
-         cut_rows(a, group, bits, dt, glu).kw > 0;
+         cut_rows(a, group, bits, glu).kw > 0;
 }
 
 hipError_t launch_qmm_rows(const RowsArgs &a, int group, int bits, int dt, bool glu, hipStream_t st) {
-  const RowsCut cut = cut_rows(a, group, bits, dt, glu);
+  const RowsCut cut = cut_rows(a, group, bits, glu);
   if (cut.kw == 0) return hipErrorInvalidConfiguration;
   auto with_kw = [&](auto d, auto b, auto g, auto gl) {
     constexpr int DT = decltype(d)::value, BITS = decltype(b)::value, GROUP = decltype(g)::value;
@@ -439,7 +413,7 @@ hipError_t launch_qmm_rows(const RowsArgs &a, int group, int bits, int dt, bool 
     return start_rows<DT, BITS, GROUP, GLU, 1>(a, cut.sk, cut.tt, st);
   };
   auto with_glu = [&](auto d, auto b, auto g) {
-    if constexpr (decltype(d)::value == 0)
+    if constexpr (decltype(d)::value == 0 && decltype(g)::value != 64)  // (blocks with groups of 32 / 128)
       if (glu) return with_kw(d, b, g, std::true_type{});
     return with_kw(d, b, g, std::false_type{});
   };
@@ -451,7 +425,7 @@ hipError_t launch_qmm_rows(const RowsArgs &a, int group, int bits, int dt, bool 
   auto with_bits = [&](auto d) {
     return bits == 4 ? with_group(d, std::integral_constant<int, 4>{}) : with_group(d, std::integral_constant<int, 8>{});
   };
-  if (glu && dt != 0) return hipErrorInvalidValue;
+  if (glu && (dt != 0 || group == 64)) return hipErrorInvalidValue;
   if (dt == 0) return with_bits(std::integral_constant<int, 0>{});
   if (dt == 1) return with_bits(std::integral_constant<int, 1>{});
   return hipErrorInvalidValue;

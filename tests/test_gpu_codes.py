@@ -1,5 +1,5 @@
-"""The tiled product on raw codes (quantized_linear in float16 and float32, and in bfloat16 with groups of 32 and 128)
-at the edges of its tiles and of its sharing of K, against the float64 product of the dequantised matrix."""
+"""The products on raw codes (quantized_linear in float16 and bfloat16; blocks with groups of 32 and 128) at the edges of their tiles
+and of their sharing of K, and float32's plain sums, against the float64 product of the dequantised matrix."""
 import numpy as np
 import pytest
 
@@ -7,9 +7,10 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 # One rounding to the result's type, half a unit of 8 (bfloat16) or 11 (float16) significant bits, is at most 2^-8 or
-# 2^-11 of each value, and so of the whole in the 2-norm (typically 0.4 of that).  float32: the sums run in
-# float32 and the code and bias terms cancel to about an eighth, so 8 * 4 units of 2^-24.
-BOUND = {"bfloat16": 2.0 ** -8, "float16": 2.0 ** -11, "float32": 32 * 2.0 ** -24}
+# 2^-11 of each value, and so of the whole in the 2-norm (typically 0.4 of that).  float32: a wave's 64 sums of up to K / 64 terms and
+# their tree, each addition off by half a unit of 2^-24 at random: 1.0e-7 to 1.5e-7 up to K = 4096.  Sums that cancel against a
+# bias term (codes that are not centred) are 3.3e-7 and more off.
+BOUND = {"bfloat16": 2.0 ** -8, "float16": 2.0 ** -11, "float32": 2.0 ** -22}
 SHAPES = [  # rows, N, K: one row; odd rows and columns; K of 3, 9 and 17 times 128 (uneven shares); each tile of the rule
     (1, 16, 128), (33, 37, 384), (65, 200, 1152), (31, 4100, 2176), (130, 1000, 256),
     (700, 1088, 640), (300, 4000, 384), (1100, 4112, 256),
@@ -127,15 +128,18 @@ def test_sums_lose_no_more_than_plain_ones(rows, n, bits, dtype, group):
     assert share <= allowed, (share, allowed)
 
 
-def test_large_float32_values_survive_the_split():
-    """The three pieces are cut by truncation: the largest finite values do not overflow on the way."""
+@pytest.mark.parametrize("transpose", [True, False])
+def test_float32_values_near_the_largest(transpose):
+    """Plain sums of them, and the input gradient's, which splits them into pieces: the first piece of the largest number is an
+    infinity, and the result is computed again."""
     import mlx_rs_amd as m
-    x = torch.full((2, 128), np.finfo(np.float32).max / 1024, device="cuda")
-    x[1] = 0
-    w = torch.full((16, 128), 1.0, device="cuda")
-    q, s, b = m.ops.quantize(w, 64, 4, torch.float32)
-    y = m.ops.quantized_linear(x, q, s, b, group_size=64, bits=4)
-    assert torch.allclose(y[0], (x[0].double().sum()).float().expand(16), rtol=1e-6) and (y[1] == 0).all()
+    most = float(np.finfo(np.float32).max)
+    x = torch.zeros((3, 128), device="cuda")
+    x[0], x[2, 5] = most / 1024, most
+    q, s, b = m.ops.quantize(torch.ones((64, 128) if transpose else (128, 64), device="cuda"), 64, 4, torch.float32)
+    y = m.ops.quantized_matmul(x, q, s, b, transpose=transpose, group_size=64, bits=4)
+    want = torch.tensor([[most / 8], [0.0], [most]], device="cuda").expand(3, 64)
+    assert torch.allclose(y, want, rtol=1e-6)
 
 
 def block_truth(blk, x, routing):
@@ -178,6 +182,33 @@ products round gate and up as well (0.94 * 2^-8, over as few as 256 values): 1.5
     if blk.workspace_bytes(tokens) < 8 << 20:
         again = blk.forward_static(x)
         assert float((again.double() - ref).norm() / ref.norm()) <= bound
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("n", [208, 16384, 32784])
+def test_waves_that_share_k_in_the_kernel_of_a_few_rows(n, group, bits, dtype):
+    """Four, two and one (1024 and 2048 tiles of 16 weight rows), with columns past the last whole block; 17 chunks of 4-bit codes, so the shares
+    are uneven."""
+    import mlx_rs_amd as m
+    dt, k = getattr(torch, dtype), 2176
+    gen = torch.Generator(device="cuda").manual_seed(n + group + bits)
+    q, s, b = m.ops.quantize(torch.randn((n, k), generator=gen, device="cuda") * 0.02, group, bits, dt)
+    for rows in (2, 11):
+        x = torch.randn((rows, k), generator=gen, device="cuda").to(dt)
+        ref = product(x, q, s, b, group, bits)
+        y = m.ops.quantized_linear(x, q, s, b, group_size=group, bits=bits)
+        err = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+        assert float(err.max()) <= BOUND[dtype], (rows, err)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("group", [32, 128])
+@pytest.mark.parametrize("experts", [16, 32, 64])
+def test_waves_that_share_k_in_a_block(experts, group, bits):
+    """The same for the gate and up product: 512, 1024 and 2048 tiles of 16 weight rows."""
+    test_blocks_with_groups_of_32_and_128(15, None, bits, group, 256, 512, experts, 5)
 
 
 @pytest.mark.parametrize("tokens", [4, 6, 14])
