@@ -542,8 +542,8 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
         again |= (not_finite(v) || (GLU && not_finite(up)) ? 1u : 0u) << r;
       }
 #pragma unroll 1
-      for (int quad = 0; quad < 4; ++quad) {  // rows 8 quad + 4 kb + 0 .. 3
-        uint32_t open = again >> (4 * quad) & 15u;
+      for (int quad = 0; __builtin_expect(again != 0, 0); ++quad, again >>= 4) {  // rows 8 quad + 4 kb + 0 .. 3
+        uint32_t open = again & 15u;
         const T *xs[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {

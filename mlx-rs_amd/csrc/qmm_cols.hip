@@ -323,7 +323,7 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
         v[t][r] *= 1.0f / kFactor;
         again |= (r_first + r < rows && not_finite(v[t][r]) ? 1u : 0u) << (r * NT + t);
       }
-    if (again) {  // all of the lane's sums in one pass over K, eight values at a time: it costs the latency of their loads
+    if (__builtin_expect(again != 0, 0)) {  // all of the lane's sums in one pass over K, eight values at a time: it costs the latency of their loads
       float f[4][NT] = {};
       uint32_t open = again;
       for (int k = 0; k < K && open; k += 8) {  // (no number stays none)

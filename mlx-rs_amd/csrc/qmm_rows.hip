@@ -336,7 +336,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
           if (not_finite(tot[0][r]) || not_finite(tot[NM - 1][r])) again |= 1u << r;
         }
       }
-      while (again) {
+      while (__builtin_expect(again != 0, 0)) {
         const int r = __builtin_ctz(again);
         again &= again - 1;
         const int64_t rr = r0 + t0 + 4 * kb + r, wrow = ebase + n0 + c;

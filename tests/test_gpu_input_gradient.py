@@ -94,13 +94,15 @@ def test_sums_lose_no_more_than_plain_ones(rows, n, k, bits, group, dtype):
 @pytest.mark.parametrize("rows,n,k", [(20, 256, 1096), (300, 2176, 264), (1100, 2176, 328)])
 def test_weights_of_more_bits_than_two_pieces(rows, n, k, bits):
     """Groups far from zero, 1 + q / 2^13, in some steps of K only, and rows that sum to zero, so that the rest of a weight is all that
-    counts.  Two pieces of bfloat16 hold 17 bits of its 20 and more, which leaves a share of 0.11 to 0.14.  (Sums that
-    cancel as a whole: a matrix instruction cuts a unit of its largest term off each of its sums where an fma rounds once.)"""
+    counts.  Two pieces of bfloat16 hold 17 bits of its 20 and more, which leaves a share of 0.11 to 0.14.  Sums that cancel as a whole show
+    what a matrix instruction cuts off: about 2^-23 (half a unit of 2^-24 of its largest term, 4), 3 K / 16 times at random, 1.7e-6 for K =
+    1096 against a spacing of 1.1e-4 at the results' root mean square 0.02 (4-bit), a share of 0.012.  Twice that is allowed."""
     x, q, s, b = operands(rows, n, k, bits, 64, torch.bfloat16)
-    q = torch.randint(-2 ** 31, 2 ** 31, q.shape, dtype=torch.int32, device="cuda")
+    gen = torch.Generator(device="cuda").manual_seed(bits)
+    q = torch.randint(-2 ** 31, 2 ** 31, q.shape, generator=gen, dtype=torch.int32, device="cuda")
     x[:, 1::2] = -x[:, ::2]
     far = (torch.arange(k, device="cuda") // 32 % 3 != 1).unsqueeze(1)
     s, b = torch.where(far, torch.full_like(s, 1.37 * 2.0 ** -13), torch.zeros_like(s)), torch.where(far, torch.ones_like(b), b.abs())
     pairs = dequantized(q, s, b, 64, bits)
-    share, plain = shares_not_nearest(x, q, s, b, 64, bits, x[:, ::2].double() @ (pairs[::2] - pairs[1::2]))
-    assert share <= 6 * plain + 2e-3, (share, plain)
+    share, _ = shares_not_nearest(x, q, s, b, 64, bits, x[:, ::2].double() @ (pairs[::2] - pairs[1::2]))
+    assert share <= 0.024, share
