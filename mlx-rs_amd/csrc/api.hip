@@ -520,7 +520,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
       //   all segments through the kernel of a few rows  even 125 / 137 / 146 / 181 / 328   Zipf-1.1 183 / 256 / 324 / 458 / 1017
       //   one chain after the other                           145 / 153 / 178 / 224 / 252            171 / 221 / 236 / 246 / 310
       //   side by side                                        148 / 158 / 174 / 198 / 263            152 / 177 / 198 / 224 / 274
-      // (the plain kernels, which these shapes ran on before: 5630 at 512 tokens)
+      // (the plain kernels, which these shapes ran on before: 5630 at 512 tokens; with centred codes side by side, even, 512 tokens: 251)
       DeviceStreams &ds = *h->streams;
       std::lock_guard<std::mutex> streams_guard(ds.lock);
       hipStream_t s = ds.side[0];
@@ -1015,6 +1015,9 @@ static bool codes_shape(int32_t dtype, int32_t transpose, int32_t group_size, in
 //   bf16, groups of 64 / streaming kernel and its record's launch: 4-bit 4096 x 2048 at 1 / 8 / 16 rows 5.4, 7.9, 10.5 /
 //   7.9, 9.5, 13.5, 4096 x 4096 7.0, 12.3, 17.6 / 10.4, 12.6, 20.2; 8-bit 2048 x 4096 at 1 / 2 / 4 / 8 / 16 rows 8.6, 9.3, 10.9,
 //   14.1, 20.8 / 10.1, 10.2, 10.7, 13.6, 17.7, 4096 x 1024 4.7, 4.8, 5.4, 6.1, 7.5 / 7.4, 7.7, 8.1, 8.9, 10.6.
+// (Before the codes were centred.  The kernel of a few rows now: 4096 x 4096, 16 rows of 4-bit codes 17.1, 17.3; 4096 x 2048 f16 at 20 / 32 rows
+//   13.2, 17.3; 1024 x 1024 8.8, 11.0; bf16, groups of 64 4-bit 4096 x 2048 4.4, 7.1, 9.6, 4096 x 4096 5.8, 11.1, 16.3; 8-bit 4096 x 1024 4.1, 4.3,
+//   4.7, 5.4, 6.8; tiles on raw codes 4096 x 4096 f16 at 20 / 32 rows 16.7, 16.9.)
 static bool dense_takes_rows(bool tuned, int32_t bits, int64_t M, int32_t K) {
   if (tuned && bits == 8) return M <= kRowsMost && M * K <= (int64_t)1 << 14;
   if (M == 1 && !tuned && bits == 4) return false;
@@ -1028,6 +1031,8 @@ static bool dense_takes_rows(bool tuned, int32_t bits, int64_t M, int32_t K) {
 // every K.  Measured, 256 x 256 / raw codes, us of the call, 4-bit: 4096 x 4096 at 64 / 128 / 512 / 1024 / 1280 / 2048 / 8192 rows
 // 59.2, 61.5, 66.8, 79.1, 80.3, 104, 279 / 22.6, 24.2, 41.4, 66.4, 90.9, 124, 466; 14336 x 4096 at 256 / 512 / 2048 rows 80.4, 103,
 // 248 / 65.2, 113, 406; 8-bit 2048 x 4096 at 64 / 1024 / 2048 / 4096 rows 56.9, 61.9, 72.6, 98.9 / 22.7, 39.8, 64.9, 129.
+// (Before the codes were centred.  On raw codes, us of the kernels, now: 4096 x 4096 at 64 / 128 / 512 / 1024 rows 18.3, 20.0, 38.8, 64.7;
+// 14336 x 4096 at 256 rows 58.2; 8-bit 2048 x 4096 at 64 / 1024 / 2048 rows 20.3, 40.3, 66.4.)
 static bool dense_takes_large_tiles(int64_t M, int32_t N) {
   const int64_t large = (M + 255) / 256 * ((N + 255) / 256), small = (M + 63) / 64 * ((N + 127) / 128);
   return 10 * small > 33 * large + 3540;

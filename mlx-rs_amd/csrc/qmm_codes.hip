@@ -10,8 +10,8 @@
 //   f16   x as it is, codes in f16 (v_mfma_f32_32x32x16_f16)
 // The centre keeps the sums as exact as plain ones: share of results that are not the float64 product's nearest value, plain / codes
 // as they are (bf16, 4-bit: 128 + q) / centred, 17 to 1000 rows: bf16 4-bit 9e-5 / 4.7e-3 / 1.0e-4, 8-bit 1.5e-4 / 4.0e-4 / 1.1e-4, f16
-// 1.1e-3 / 2.7e-3 / 7.3e-4.  What it costs is the conversion of 4-bit codes in bf16, 15 instructions a multiply for 7: 51 us of
-// 1000 x 2080 x 3968 against 55, nothing below 300 rows.
+// 1.1e-3 / 2.7e-3 / 7.3e-4.  What it costs is the conversion of 4-bit codes in bf16, 15 instructions a multiply for 7: 50 us of
+// 1000 x 2080 x 3968 against 53, nothing below 300 rows.
 // float32 does not come here: without the centre its error was 3.3e-7 to 5.7e-7 (a wave per output element 1.0e-7 to 1.5e-7).
 // The fp32 sums of a group are scaled once, when the group ends.  The bias term sum_g b_g (sum_c x_c) is a product of
 // its own over the groups: the group sums of x (fp32, split into three bf16 pieces) against the biases (three pieces
@@ -122,8 +122,8 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf
 // A step takes one 32 x 32 sub-tile after the other: its four multiplies follow each other in one accumulator, and the
 // scaled addition of the sub-tile before it (16 fma) and the unpacking of the next step's codes (10 to 15 instructions a
 // multiply) run between them, which is as much vector work as fits beside the matrix cores.
-// What bounds it (777 x 4096 x 4096, f16, 8-bit; 26 GFLOP): 58 us for the call = 450 TFLOP/s, 50 times the plain kernel's
-// 3160 us; the matrix cores alone would take 18.  Taken apart at one block a CU (cycles per 64 K values of 128 x 32 a
+// What bounds it (777 x 4096 x 4096, f16, 8-bit; 26 GFLOP): 54 us for the call = 480 TFLOP/s (the plain kernel
+// 3160 us); the matrix cores alone would take 18.  Taken apart at one block a CU (cycles per 64 K values of 128 x 32 a
 // wave, 512 of them matrix work): multiplies and barriers 575, with the vector work 640, with the reads of LDS 840, with
 // the loads 1350.  The loads cost their line visits: a wave's codes sit in 32 rows.
 // KW > 1: the block's waves form KW groups that share K among them, each with LDS buffers of its own; their sums meet in
@@ -637,7 +637,8 @@ static hipError_t start_codes(const CodesArgs &a, int scale_shift, const uint32_
 //   64 x 128:                           41.5 / 42.4 / 46.7 / 31.0 / 45.6 / 66.7  (several blocks a CU overlap as K groups do)
 // Between one and two 32 x 64 tiles a CU the two are as fast with f16 and K = 4096; bf16, 4-bit, 32 x 64 / 64 x 128:
 // (200, 4096, 2048) 32.0 / 24.8, (200, 4096, 4096) 39.9 / 37.4, (1000, 1024, 1024) 29.7 / 21.8, (400, 2048, 768) 19.7 / 14.7.
-// (128 x 128 tiles: 65.1 / 67.0 / 70.2 / 45.9 / 69.3 / 76.0.)
+// (128 x 128 tiles: 65.1 / 67.0 / 70.2 / 45.9 / 69.3 / 76.0.)  These compare tiles as they were before the codes were centred; the rule's
+// choices by the kernels' time now: 17.9 / 29.7 / 34.7 / 25.3 / 34.0 / 62.0 and, bf16, 20.0, 33.1, 16.7, 14.1.
 template <int DT, int BITS, bool G32>
 static hipError_t start_dense(const CodesArgs &a, int scale_shift, hipStream_t st) {
   auto tiles = [&](int rows, int cols) { return (a.M + rows - 1) / rows * ((a.N + cols - 1) / cols); };
@@ -649,7 +650,8 @@ static hipError_t start_dense(const CodesArgs &a, int scale_shift, hipStream_t s
 // The M-tile lists of a grouped product (see tile_list) in one launch, in blocks of 64 rows x 128 columns.  Measured on
 // the 128-expert shape with groups of 32, us of a forward at 200 / 512 tokens, even and Zipf-1.1 routing: three launches,
 // a list each, 225, 314 / 260, 373; one launch 224, 246 / 252, 310; one launch with gate/up blocks of 32 rows 217, 242 /
-// 332, 335; with gate/up blocks of 32 x 64 and K shared by two groups 288, 347 / 628, 524.
+// 332, 335; with gate/up blocks of 32 x 64 and K shared by two groups 288, 347 / 628, 524.  (Before the codes were centred; the kept form
+// takes 251 at 512 tokens and even routing now, where it took 268.)
 hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *lists, int cap256, int n_experts, int group, int bits,
                                   bool glu, hipStream_t st) {
   auto run = [&](auto b, auto g32) {

@@ -50,8 +50,8 @@ struct RowsLds {
 //   so that multiply s takes codes 32 s .. 32 s + 31;
 //   8-bit: multiply t takes the t-th half of every quarter (groups >= 64), or after two swaps 32 consecutive codes.
 // What bounds it: the bytes of the weights and, for one row of a small matrix, the latency of its few dependent steps.
-// Measured, 4096 x 4096, us of the kernel at 1 / 4 / 8 / 16 rows (the plain kernel, a wave per output element: f16 4-bit
-// 6.7 / 17.5 / 30.2 / 55.6): f16 4-bit 7.5 / 9.8 / 13.0 / 18.3, bf16 groups of 32 8.5 / 10.9 / 14.4 / 20.7.  Every block
+// Measured, 4096 x 4096, us of the kernel at 2 / 4 / 8 / 16 rows (the plain kernel, a wave per output element: f16 4-bit
+// 17.5 / 30.2 / 55.6 from 4 rows on): f16 4-bit 7.2 / 8.5 / 11.7 / 17.2, bf16 groups of 32 7.4 / 8.7 / 11.8 / 17.0.  Every block
 // stages all rows: that is what grows.
 template <int DT, int BITS, int GROUP, bool GLU, int KW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void qmm_rows_kernel(RowsArgs a, int tt, int sk) {
