@@ -252,6 +252,29 @@ static hipError_t device_streams(int dev, DeviceStreams **out) {
   return hipSuccess;
 }
 
+// Whether work of `st` may be forked to `side`.  A stream that a capture has forked to stays in it until the capture ends, also
+// where it has been joined back: work of another stream would be recorded in that graph instead of run, and its stream with it.
+static bool may_fork(hipStream_t st, hipStream_t side) {
+  hipStreamCaptureStatus of_side = hipStreamCaptureStatusNone, of_st = hipStreamCaptureStatusNone;
+  unsigned long long id_side = 0, id_st = 0;
+  if (hipStreamGetCaptureInfo(side, &of_side, &id_side) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (of_side == hipStreamCaptureStatusNone) return true;
+  if (hipStreamGetCaptureInfo(st, &of_st, &id_st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return of_side == hipStreamCaptureStatusActive && of_st == hipStreamCaptureStatusActive && id_side == id_st;
+}
+// The same for all of a device's side streams, whose lock the caller holds.
+static bool may_fork(hipStream_t st, const DeviceStreams &ds) {
+  for (hipStream_t s : ds.side)
+    if (!may_fork(st, s)) return false;
+  return true;
+}
+
 struct mi_moe_s {
   mi_moe_config cfg;
   mi_moe_weights w;
@@ -463,6 +486,12 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   grouped_args(c, h->w, f, x, T, a, d);
   const int max_active = a.max_active;
   if (f.tiled && paired && !streamed_first && !pair_in_router) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));
+  // independent chains run beside each other where side streams are to be had, whose lock is held until they have been joined back
+  std::unique_lock<std::mutex> streams_guard;
+  const bool chains = !ev && (f.raw ? f.raw_tiles != nullptr : !plain_config(c) && large_qmm_applies(a));
+  if (chains) streams_guard = std::unique_lock<std::mutex>(h->streams->lock);
+  const bool fork = chains && may_fork(st, *h->streams);
+  if (!fork && streamed_first && paired && large_qmm_applies(a)) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));  // (a side stream's work)
   if (f.raw) {
     // group sizes 32 / 128: short segments on the kernel of a few rows, longer ones (where lists are built) in tiles
     RowsArgs ra{}, rd{};
@@ -513,7 +542,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
         return e;
       return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.n_experts, c.group_size, c.bits, false, s);
     };
-    if (f.raw_tiles && !ev) {
+    if (fork) {
       // The two chains share no rows.  The tiles run on a side stream beside the short segments: which of the two is the
       // longer depends on the routing, and with even routing one of them is all but empty.  Measured, 128-expert shape,
       // groups of 32, us of a forward at 64 / 96 / 128 / 200 / 512 tokens:
@@ -522,7 +551,6 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
       //   side by side                                        148 / 158 / 174 / 198 / 263            152 / 177 / 198 / 224 / 274
       // (the plain kernels, which these shapes ran on before: 5630 at 512 tokens; with centred codes side by side, even, 512 tokens: 251)
       DeviceStreams &ds = *h->streams;
-      std::lock_guard<std::mutex> streams_guard(ds.lock);
       hipStream_t s = ds.side[0];
       MI_HIP(hipEventRecord(ds.fork, st));
       MI_HIP(hipStreamWaitEvent(s, ds.fork, 0));
@@ -558,7 +586,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     MI_HIP(launch_qmm_plain(f.hh, h->w.down.w, h->w.down.scales, h->w.down.biases, nullptr, f.topk_idx, f.perm, f.perm,
                             0u, (uint32_t)c.n_experts, P, 1, c.hidden, c.intermediate, c.group_size, c.bits, true, MI_MOE_DTYPE_BF16, f.y, st));
     MI_STAGE_DONE();
-  } else if (large_qmm_applies(a) && !ev) {
+  } else if (fork) {
     // Four chains that share no rows: the three tile classes and the streamed segments, each
     // gate/up then down.  The short classes leave most of the chip idle when they run alone
     // (a few dozen workgroups of 64 K steps each); side by side they fill it.  The chain that is
@@ -572,7 +600,6 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     const bool exists[4] = {T > 128, T > 64, true, true};
     int n_side = 0;
     DeviceStreams &ds = *h->streams;
-    std::lock_guard<std::mutex> streams_guard(ds.lock);  // until the side streams have been joined back
     MI_HIP(hipEventRecord(ds.fork, st));
     // the launches, in a function of their own: whatever happens in it, the side streams it has
     // used are joined back below (a caller must never be left with work of ours running beside
@@ -673,6 +700,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     MI_HIP(launch_grouped_qmm(d, false, st));
     MI_STAGE_DONE();
   }
+  if (streams_guard.owns_lock()) streams_guard.unlock();
   MI_HIP(launch_combine(f.y, f.topk_w, nullptr, T, c.top_k, c.hidden, norm_weight ? x_in : nullptr, out, st));
   MI_STAGE_DONE();
 #undef MI_STAGE_DONE
