@@ -127,9 +127,11 @@ struct ForwardWs {
   void *disp_scratch;
   uint16_t *hh, *y, *xperm, *xnorm;
   uint16_t *gu;  // plain products only: the gate and the up product, [P, I] each
+  bool mid;             // groups of 64: all segments in short tiles (see mid_batch)
   bool raw;             // group sizes 32 / 128: the products on raw codes (qmm_rows, qmm_codes)
-  uint32_t *raw_tiles;  // their tile lists, the paired copy of x (4-bit) and the group sums of x and h, or nullptr: all
-  int raw_cap;          // segments go through the kernel of a few rows, in as many passes as they need
+  uint32_t *raw_tiles;  // the short tiles of qmm_codes, the paired copy of x (4-bit) and the group sums of x and h, or nullptr:
+  int raw_cap;          // (groups of 32 / 128) all segments go through the kernel of a few rows, in as many passes as they need
+  int raw_from;         // segments of this many rows and more are cut into short tiles
   uint16_t *raw_copy, *raw_xsums, *raw_hsums;
   size_t bytes_raw;     // up to the end of those
   void *router_scratch;  // byte planes of x and of the router matrix (logits on the int8 matrix cores), or nullptr
@@ -140,12 +142,28 @@ struct ForwardWs {
 // Group sizes 32 and 128: tile lists are built (for segments of more rows than one pass of the kernel of a few rows, which
 // a segment of at most T rows has to be able to have) from an average of four rows per expert on; see forward_impl for what that
 // costs and gives.  The tiled kernel takes operands below 2 GiB, in multiples of 128 values.
-bool raw_tiled_batch(const mi_moe_config &c, int64_t T) {
+bool codes_tiles_fit(const mi_moe_config &c, int64_t T) {
   const int64_t P = T * c.top_k, most = (int64_t)1 << 31;
-  return T > kRowsMost && P >= (int64_t)4 * c.n_experts && c.hidden % 128 == 0 && c.intermediate % 128 == 0 && T * c.hidden * 2 < most &&
+  return c.hidden % 128 == 0 && c.intermediate % 128 == 0 && T * c.hidden * 2 < most &&
          P * c.intermediate * 2 < most && (int64_t)codes_sums_bytes(P, c.intermediate, c.group_size) < most &&
          (int64_t)codes_sums_bytes(T, c.hidden, c.group_size) < most &&
          (int64_t)c.hidden * c.intermediate * c.bits / 8 < most;
+}
+bool raw_tiled_batch(const mi_moe_config &c, int64_t T) {
+  return T > kRowsMost && T * c.top_k >= (int64_t)4 * c.n_experts && codes_tiles_fit(c, T);
+}
+// Groups of 64, 4-bit codes: batches whose segments all go through short tiles on raw codes, in one launch a product on the caller's
+// stream (the others: streamed segments, and tiles of 256 weight rows on side streams).  From the batches on for which the tile lists
+// are built and the router has kernels of its own, up to 96 rows per expert on average.  Measured, us of a forward, other route / this one:
+//   128 experts, hidden 2048, even routing at 96 / 128 / 203 / 320 / 512 / 1024 / 2048 / 4096 tokens 145, 151, 176, 216, 218, 266, 360, 484 /
+//   128, 124, 128, 134, 168, 221, 350, 566; Zipf-1.1 136, 139, 160, 173, 193, 237, 344, 490 / 92, 95, 114, 134, 157, 219, 341, 560;
+//   hidden 4096, intermediate 1536, even at 128 / 256 / 512 / 1024 / 2048 tokens 536, 587, 665, 785, 1144 / 372, 375, 449, 649, 1101; Zipf-1.3
+//   315, 442, 510, 698, 1079 / 271, 354, 477, 693, 1123.
+// Longer segments in 256-row tiles beside this (a fork, six launches more): 203 for 169 at 512 tokens, 516 for 490 at 4096.
+// 8-bit codes (8 experts, 4096 x 14336, 256 / 512 tokens): 741, 737 / 835, 1107.  Few pairs or experts leave most of the chip idle.
+bool mid_batch(const mi_moe_config &c, int64_t T, bool tiled) {
+  const int64_t P = T * c.top_k;
+  return tiled && c.bits == 4 && T > kFusedRouterMaxTokens && P <= (int64_t)96 * c.n_experts && P >= 512 && c.n_experts >= 8 && codes_tiles_fit(c, T);
 }
 
 ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws) {
@@ -186,12 +204,26 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws) {
   f.raw = plain_config(c) && qmm_rows_applies(up, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true) &&
           qmm_rows_applies(down, c.group_size, c.bits, MI_MOE_DTYPE_BF16, false);
   f.gu = cv.take<uint16_t>(plain_config(c) && !f.raw ? 2 * (size_t)P * c.intermediate : 0);
-  f.bytes_min = cv.off;
   f.raw_tiles = nullptr;
   f.raw_cap = 0;
+  f.raw_from = kRowsMost + 1;
+  f.bytes_min = cv.off;
+  f.mid = mid_batch(c, T, f.tiled);
+  if (f.mid) {
+    // All of it lies in memory that is free at the time where it fits, so that batches which have to fit a scratch of a given size take
+    // this route as well: the list in place of the work records (nothing is streamed), the group sums of x where the down product writes
+    // its rows later, those of h in the normalised rows, which only the router and the copy of x read.
+    f.raw_from = 1;
+    f.raw_cap = short_list_cap(P, c.n_experts, 1);
+    const size_t list = short_list_words(f.raw_cap), xsums = codes_sums_bytes(T, c.hidden, c.group_size), hsums = codes_sums_bytes(P, c.intermediate, c.group_size);
+    f.raw_tiles = list <= (size_t)c.n_experts * 16 ? f.work : cv.take<uint32_t>(list);
+    f.raw_copy = f.xperm;
+    f.raw_xsums = xsums <= (size_t)P * c.hidden * 2 ? f.y : cv.take<uint16_t>(xsums / 2);
+    f.raw_hsums = hsums <= (size_t)T * c.hidden * 2 ? f.xnorm : cv.take<uint16_t>(hsums / 2);
+  }
   if (f.raw && raw_tiled_batch(c, T)) {
-    f.raw_cap = (int)(P / kBigTileM + (P / (kRowsMost + 1) < c.n_experts ? P / (kRowsMost + 1) : c.n_experts));
-    f.raw_tiles = cv.take<uint32_t>(tile_list_words(f.raw_cap, c.n_experts));
+    f.raw_cap = short_list_cap(P, c.n_experts, f.raw_from);
+    f.raw_tiles = cv.take<uint32_t>(short_list_words(f.raw_cap));
     f.raw_copy = cv.take<uint16_t>(codes_copy_bytes(c.bits, T, c.hidden) / 2);
     f.raw_xsums = cv.take<uint16_t>(codes_sums_bytes(T, c.hidden, c.group_size) / 2);
     f.raw_hsums = cv.take<uint16_t>(codes_sums_bytes(P, c.intermediate, c.group_size) / 2);
@@ -422,7 +454,10 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   ForwardWs f = carve_forward(c, T, workspace);
   if (workspace_bytes < f.bytes_min)
     return fail("forward: workspace too small (%zu bytes, need %zu)", workspace_bytes, f.bytes);
-  if (workspace_bytes < f.bytes_raw) f.raw_tiles = nullptr;
+  if (workspace_bytes < f.bytes_raw) {
+    f.raw_tiles = nullptr;
+    f.mid = false;
+  }
   if (workspace_bytes < f.bytes) f.router_scratch = nullptr;  // room for everything but the byte planes: fp64 logits, same bits
   int stage = 0;
 #define MI_STAGE_DONE()                                  \
@@ -431,8 +466,11 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   } while (0)
   if (ev) MI_HIP(hipEventRecord(ev[0], st));
   const bool fused_router = router_fused_applies(T, c.n_experts, c.top_k);
-  uint32_t *const tile_lists = f.tiled ? f.mtiles : f.raw_tiles;
-  const int tile_cap = f.tiled ? f.max_mtiles : f.raw_cap, tile_from = f.tiled ? f.tmr : kRowsMost + 1;
+  const bool mid = f.mid && !kt;  // (kt times the kernels of the other route)
+  uint32_t *const tile_lists = f.tiled && !mid ? f.mtiles : nullptr;
+  const int tile_cap = f.max_mtiles, tile_from = f.tmr;
+  const ShortTiles shorts = {mid || f.raw ? f.raw_tiles : nullptr, (uint32_t)f.raw_from};
+  uint32_t *const records = mid ? nullptr : f.work;
   if (norm_weight) {  // the block's input is rms_norm(x); x itself is added back in the combine
     if (!fused_router) MI_HIP(launch_rms_norm(x_in, norm_weight, eps, T, c.hidden, f.xnorm, st));
     x = f.xnorm;      // decode: written by the router kernel below
@@ -442,15 +480,15 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   // per forward (prefill-sized T only): by the router's logits kernel, which holds every piece of x in
   // registers anyway, or by a kernel of its own (light batches pair the rows beside their streamed segments)
   const bool paired = c.bits == 4;
-  const bool streamed_first = f.tiled && !f.heavy && !ev;  // light batches start their streamed segments first
-  const bool pair_in_router = f.tiled && paired && !streamed_first && !fused_router && !plain_config(c) &&
+  const bool streamed_first = f.tiled && !f.heavy && !ev && !mid;  // light batches start their streamed segments first
+  const bool pair_in_router = f.tiled && paired && !mid && !streamed_first && !fused_router && !plain_config(c) &&
                               router_logits_pairs_rows(T, c.hidden);
   if (fused_router) {
     // decode: one launch for the three stages (the stage times then all land in the first)
     MI_HIP(launch_router_fused(x_in, h->w.router_w, h->w.router_bias, norm_weight, eps, f.xnorm, T, c.hidden,
                                c.n_experts, c.top_k,
                                c.score_mode, f.logits, f.topk_idx, f.topk_w, h->counters, f.counts, f.offsets,
-                               f.perm, f.inv_perm, f.src_of, f.work, tile_lists, tile_cap, tile_from, st));
+                               f.perm, f.inv_perm, f.src_of, records, tile_lists, tile_cap, tile_from, shorts, st));
     MI_STAGE_DONE();
     MI_STAGE_DONE();
     MI_STAGE_DONE();
@@ -479,20 +517,58 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
       MI_STAGE_DONE();
     }
     MI_HIP(launch_dispatch(f.topk_idx, P, c.n_experts, c.top_k, f.counts, f.offsets, f.perm, f.inv_perm,
-                           f.src_of, f.work, tile_lists, tile_cap, tile_from, f.disp_scratch, st));
+                           f.src_of, records, tile_lists, tile_cap, tile_from, shorts, f.disp_scratch, st));
     MI_STAGE_DONE();
   }
   GroupedArgs a{}, d{};
   grouped_args(c, h->w, f, x, T, a, d);
   const int max_active = a.max_active;
-  if (f.tiled && paired && !streamed_first && !pair_in_router) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));
+  if (f.tiled && paired && !streamed_first && !pair_in_router && !mid) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));
   // independent chains run beside each other where side streams are to be had, whose lock is held until they have been joined back
   std::unique_lock<std::mutex> streams_guard;
-  const bool chains = !ev && (f.raw ? f.raw_tiles != nullptr : !plain_config(c) && large_qmm_applies(a));
+  const bool chains = !ev && !mid && (f.raw ? f.raw_tiles != nullptr : !plain_config(c) && large_qmm_applies(a));
   if (chains) streams_guard = std::unique_lock<std::mutex>(h->streams->lock);
   const bool fork = chains && may_fork(st, *h->streams);
   if (!fork && streamed_first && paired && large_qmm_applies(a)) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));  // (a side stream's work)
-  if (f.raw) {
+  // the short tiles on raw codes
+  CodesArgs ca{}, cd{};
+  const bool copied = codes_copy_bytes(c.bits, T, c.hidden) > 0;
+  ca.x = copied ? f.raw_copy : x;
+  ca.x_rows = T;
+  ca.sums = f.raw_xsums;
+  ca.src_rows = f.src_of;
+  ca.w0 = h->w.gate.w; ca.s0 = h->w.gate.scales; ca.b0 = h->w.gate.biases;
+  ca.w1 = h->w.up.w; ca.s1 = h->w.up.scales; ca.b1 = h->w.up.biases;
+  ca.y = f.hh;
+  ca.y_paired = copied;
+  ca.N = c.intermediate; ca.K = c.hidden;
+  cd.x = f.hh;
+  cd.x_rows = P;
+  cd.sums = f.raw_hsums;
+  cd.dst_rows = f.perm;
+  cd.w0 = h->w.down.w; cd.s0 = h->w.down.scales; cd.b0 = h->w.down.biases;
+  cd.y = f.y;
+  cd.N = c.hidden; cd.K = c.intermediate;
+  auto prepare_x = [&](hipStream_t s) -> hipError_t {
+    return launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, s);
+  };
+  auto tiles_up = [&](hipStream_t s) -> hipError_t {
+    return launch_qmm_codes_tiles(ca, f.raw_tiles, f.raw_cap, c.group_size, c.bits, true, s);
+  };
+  auto tiles_down = [&](hipStream_t s) -> hipError_t {
+    // (the sums of all rows of h: those of other segments, which another stream may still be writing, are not read)
+    if (hipError_t e = launch_prepare_rows(f.hh, P, c.intermediate, c.group_size, MI_MOE_DTYPE_BF16, nullptr, f.raw_hsums, s);
+        e != hipSuccess)
+      return e;
+    return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.group_size, c.bits, false, s);
+  };
+  if (mid) {
+    MI_HIP(prepare_x(st));
+    MI_HIP(tiles_up(st));
+    MI_STAGE_DONE();
+    MI_HIP(tiles_down(st));
+    MI_STAGE_DONE();
+  } else if (f.raw) {
     // group sizes 32 / 128: short segments on the kernel of a few rows, longer ones (where lists are built) in tiles
     RowsArgs ra{}, rd{};
     ra.work = f.work;
@@ -511,37 +587,6 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     rd.w0 = h->w.down.w; rd.s0 = h->w.down.scales; rd.b0 = h->w.down.biases;
     rd.y = f.y;
     rd.N = c.hidden; rd.K = c.intermediate;
-    CodesArgs ca{}, cd{};
-    const bool copied = codes_copy_bytes(c.bits, T, c.hidden) > 0;
-    ca.x = copied ? f.raw_copy : x;
-    ca.x_rows = T;
-    ca.sums = f.raw_xsums;
-    ca.src_rows = f.src_of;
-    ca.w0 = ra.w0; ca.s0 = ra.s0; ca.b0 = ra.b0;
-    ca.w1 = ra.w1; ca.s1 = ra.s1; ca.b1 = ra.b1;
-    ca.y = f.hh;
-    ca.y_paired = copied;
-    ca.N = ra.N; ca.K = ra.K;
-    cd.x = f.hh;
-    cd.x_rows = P;
-    cd.sums = f.raw_hsums;
-    cd.dst_rows = f.perm;
-    cd.w0 = rd.w0; cd.s0 = rd.s0; cd.b0 = rd.b0;
-    cd.y = f.y;
-    cd.N = rd.N; cd.K = rd.K;
-    auto tiles_up = [&](hipStream_t s) -> hipError_t {
-      if (hipError_t e = launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, s);
-          e != hipSuccess)
-        return e;
-      return launch_qmm_codes_tiles(ca, f.raw_tiles, f.raw_cap, c.n_experts, c.group_size, c.bits, true, s);
-    };
-    auto tiles_down = [&](hipStream_t s) -> hipError_t {
-      // (the sums of all rows of h: those of the short segments, which another stream may still be writing, are not read)
-      if (hipError_t e = launch_prepare_rows(f.hh, P, c.intermediate, c.group_size, MI_MOE_DTYPE_BF16, nullptr, f.raw_hsums, s);
-          e != hipSuccess)
-        return e;
-      return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.n_experts, c.group_size, c.bits, false, s);
-    };
     if (fork) {
       // The two chains share no rows.  The tiles run on a side stream beside the short segments: which of the two is the
       // longer depends on the routing, and with even routing one of them is all but empty.  Measured, 128-expert shape,
@@ -556,7 +601,8 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
       MI_HIP(hipStreamWaitEvent(s, ds.fork, 0));
       const bool tiles_lead = P >= (int64_t)20 * c.n_experts;  // the longer chain, as far as the host can tell, stays here
       const hipStream_t ts = tiles_lead ? st : s, rs = tiles_lead ? s : st;
-      hipError_t e = tiles_up(ts);
+      hipError_t e = prepare_x(ts);
+      if (e == hipSuccess) e = tiles_up(ts);
       if (e == hipSuccess) e = tiles_down(ts);
       if (e == hipSuccess) e = launch_qmm_rows(ra, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true, rs);
       if (e == hipSuccess) e = launch_qmm_rows(rd, c.group_size, c.bits, MI_MOE_DTYPE_BF16, false, rs);
@@ -566,7 +612,10 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
       MI_HIP(e);
       MI_HIP(je);
     } else {
-      if (f.raw_tiles) MI_HIP(tiles_up(st));
+      if (f.raw_tiles) {
+        MI_HIP(prepare_x(st));
+        MI_HIP(tiles_up(st));
+      }
       MI_HIP(launch_qmm_rows(ra, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true, st));
       MI_STAGE_DONE();
       if (f.raw_tiles) MI_HIP(tiles_down(st));
@@ -891,7 +940,7 @@ int mi_moe_dispatch(const uint32_t *expert_of_pair, int64_t P, int32_t n_experts
   void *scratch = cv.take<char>(dispatch_workspace_bytes(n_experts, P));
   hipStream_t st = static_cast<hipStream_t>(stream);
   MI_HIP(launch_dispatch(expert_of_pair, P, n_experts, 1, counts, offsets, perm, inv_perm, nullptr, nullptr,
-                         nullptr, 0, 0, scratch, st));
+                         nullptr, 0, 0, ShortTiles{}, scratch, st));
   return 0;
 } MI_CATCH("dispatch")
 
@@ -966,7 +1015,7 @@ static int gather_qmm_impl(const void *x, const uint32_t *w, const void *scales,
   uint32_t *src_rows = cv.take<uint32_t>((size_t)rows);
   uint32_t *dst_rows = cv.take<uint32_t>((size_t)rows);
   MI_HIP(launch_dispatch(rhs_indices, n_idx, n_experts, 1, counts, offsets, perm, nullptr, nullptr, work,
-                         nullptr, 0, 0, scratch, st));
+                         nullptr, 0, 0, ShortTiles{}, scratch, st));
   MI_HIP(launch_row_maps(perm, lhs_indices, n_lhs, offsets, n_idx, M, n_experts, src_rows, dst_rows, work, st));
   GroupedArgs a{};
   a.x = static_cast<const uint16_t *>(x);

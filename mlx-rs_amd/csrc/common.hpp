@@ -176,6 +176,18 @@ __host__ __device__ inline P *tile_list(P *base, int cls, int cap256, int n_expe
   return base + 4 + 4 * (size_t)cap256 + 4 + 4 * (size_t)n_experts;
 }
 
+// A list of the same form for the tiles of the products on raw codes: segments of `from` rows and more that the three lists do
+// not take, in pieces of kShortTileM rows; experts in ascending order.
+constexpr int kShortTileM = 64;
+struct ShortTiles {
+  uint32_t *list = nullptr;
+  uint32_t from = 1;
+};
+__host__ __device__ inline size_t short_list_words(int cap) { return 4 + 4 * (size_t)cap; }
+inline int short_list_cap(int64_t pairs, int n_experts, int from) {  // full pieces, and a segment's last one
+  return (int)(pairs / kShortTileM + (pairs / from < n_experts ? pairs / from : n_experts));
+}
+
 // ---------------------------------------------------------------- element types
 __device__ __forceinline__ float as_f32(uint16_t v) { return bf16_to_f32(v); }  // bfloat16, raw bits
 __device__ __forceinline__ float as_f32(_Float16 v) { return (float)v; }
@@ -292,7 +304,7 @@ size_t dispatch_workspace_bytes(int E, int64_t P);
 hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, uint32_t *counts,
                            uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
                            uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, int big_thr,
-                           void *scratch, hipStream_t st);
+                           ShortTiles shorts, void *scratch, hipStream_t st);
 // decode-sized batches: logits + selection + dispatch in one launch.  counters: 1 +
 // kFusedRouterMaxTokens zero-initialised words that the kernel leaves zeroed again.  norm_w != nullptr:
 // the rows are RMS-normalised first (weight norm_w, eps) and kept in xnorm.
@@ -303,7 +315,7 @@ hipError_t launch_router_fused(const uint16_t *x, const uint16_t *wg, const floa
                                uint16_t *topk_w, uint32_t *counters, uint32_t *counts,
                                uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
                                uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256,
-                               int big_thr, hipStream_t st);
+                               int big_thr, ShortTiles shorts, hipStream_t st);
 hipError_t launch_grouped_qmm(const GroupedArgs &a, bool glu, hipStream_t st);
 hipError_t launch_large_qmm(const GroupedArgs &a, bool glu, hipStream_t st);
 // the same work in its independent parts: one tile class (0, 1, 2 = 256-, 128-, 64-row tiles) of
@@ -383,8 +395,7 @@ size_t codes_sums_bytes(int64_t rows, int K, int group);
 hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
                                uint16_t *sums, hipStream_t st);
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
-hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *lists, int cap256, int n_experts, int group, int bits,
-                                  bool glu, hipStream_t st);
+hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st);
 hipError_t launch_quantize(const float *w, int64_t rows, int64_t cols, int group, int bits,
                            uint32_t *q, void *s, void *b, int dt, hipStream_t st);
 hipError_t launch_dequantize(const uint32_t *q, const void *s, const void *b,

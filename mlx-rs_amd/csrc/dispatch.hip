@@ -16,9 +16,9 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_single_kernel(
     const uint32_t *flat, int64_t P, int E, int nbits, int k_div,
     uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets, uint32_t *__restrict__ perm,
     uint32_t *__restrict__ inv_perm, uint32_t *__restrict__ src_of,
-    uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr) {
+    uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr, ShortTiles shorts) {
   extern __shared__ uint32_t lds[];
-  dispatch_block(flat, P, E, nbits, k_div, lds, counts, offsets, perm, inv_perm, src_of, work, mtiles, cap256, big_thr);
+  dispatch_block(flat, P, E, nbits, k_div, lds, counts, offsets, perm, inv_perm, src_of, work, mtiles, cap256, big_thr, shorts);
 }
 
 // ---- three kernels for prefill-sized P: block b owns pairs [b*span, (b+1)*span)
@@ -48,7 +48,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_hist_kernel(
 __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     const uint32_t *flat, int64_t P, int E, int nbits, int k_div, int64_t span,
     const uint32_t *__restrict__ blockhist, int nb, uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets,
-    uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr,
+    uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr, ShortTiles shorts,
     uint32_t *__restrict__ perm, uint32_t *__restrict__ inv_perm, uint32_t *__restrict__ src_of) {
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t n_active, total;
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
   }
   __syncthreads();
   if (mine == nb) {
-    finish_counts(cnt, tmp, cur, E, counts, offsets, work, mtiles, cap256, big_thr, &n_active);
+    finish_counts(cnt, tmp, cur, E, counts, offsets, work, mtiles, cap256, big_thr, shorts, &n_active);
     return;
   }
   block_exclusive_scan(cnt, tmp, E, &total);
@@ -109,14 +109,14 @@ size_t dispatch_workspace_bytes(int E, int64_t P) {
 hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, uint32_t *counts,
                            uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
                            uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, int big_thr,
-                           void *scratch, hipStream_t st) {
+                           ShortTiles shorts, void *scratch, hipStream_t st) {
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
   if (k_div < 1) k_div = 1;
   if (P <= kSingleMaxP) {
     size_t lds = (size_t)(3 + kDispWaves) * E * sizeof(uint32_t);
     dispatch_single_kernel<<<1, kDispThreads, lds, st>>>(flat, P, E, nbits, k_div, counts, offsets,
-                                                        perm, inv_perm, src_of, work, mtiles, cap256, (uint32_t)big_thr);
+                                                        perm, inv_perm, src_of, work, mtiles, cap256, (uint32_t)big_thr, shorts);
     return hipGetLastError();
   }
   uint32_t *blockhist = reinterpret_cast<uint32_t *>(scratch);
@@ -127,7 +127,7 @@ hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, ui
   const size_t e3 = (size_t)3 * (E > kDispWaves ? E : kDispWaves);
   const size_t tail = (size_t)kDispWaves * E > 2u * kDispThreads ? (size_t)kDispWaves * E : 2u * kDispThreads;
   dispatch_scatter_kernel<<<nb + 1, kDispThreads, (e3 + tail) * 4, st>>>(flat, P, E, nbits, k_div, kSpan, blockhist, nb, counts,
-                                                                        offsets, work, mtiles, cap256, (uint32_t)big_thr, perm,
+                                                                        offsets, work, mtiles, cap256, (uint32_t)big_thr, shorts, perm,
                                                                         inv_perm, src_of);
   return hipGetLastError();
 }

@@ -112,11 +112,11 @@ __device__ __forceinline__ TileSplit split_segment(uint32_t c) {
   return t;
 }
 
-// counts -> offsets, work records and M tiles; runs in one block.  LDS cnt[E] in, cur[E] out.
+// counts -> offsets, work records, M tiles and short tiles; runs in one block.  LDS cnt[E] in, cur[E] out.
 __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint32_t *cur, int E,
                               uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets,
                               uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256,
-                              uint32_t big_thr, uint32_t *n_active_lds) {
+                              uint32_t big_thr, ShortTiles shorts, uint32_t *n_active_lds) {
   __shared__ uint32_t total;
   const int tid = threadIdx.x;
   if (tid < E && counts) counts[tid] = cnt[tid];
@@ -132,13 +132,14 @@ __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint
   if (tid < kWave) {
     uint32_t *const l256 = mtiles, *const l128 = mtiles ? tile_list(mtiles, 1, cap256, E) : nullptr,
                    *const l64 = mtiles ? tile_list(mtiles, 2, cap256, E) : nullptr;
-    uint32_t base = 0, t256 = 0, t128 = 0, t64 = 0;
+    uint32_t base = 0, t256 = 0, t128 = 0, t64 = 0, t_short = 0;
     for (int e0 = 0; e0 < E; e0 += kWave) {
       const int e = e0 + tid;
       uint32_t c = 0;
       if (e < E) c = (e + 1 < E ? cnt[e + 1] : total) - cnt[e];
       const bool big = mtiles && big_thr != 0u && c >= big_thr;
-      const bool small = c != 0u && !big;
+      const bool brief = shorts.list && !big && c >= shorts.from;
+      const bool small = c != 0u && !big && !brief;
       const uint64_t bm = __ballot(small);
       if (small && work) {
         uint32_t *rec = work + (size_t)(base + __popcll(bm & lanemask_lt())) * kWorkWords;
@@ -165,6 +166,20 @@ __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint
         rec[3] = 0u;
       }
       t256 += __shfl(incl, kWave - 1, kWave);
+      if (shorts.list) {  // pieces of kShortTileM rows
+        const uint32_t n = brief ? (c + kShortTileM - 1) / kShortTileM : 0u;
+        uint32_t before = n;
+        for (int d = 1; d < kWave; d <<= 1) {
+          const uint32_t v = __shfl_up(before, d, kWave);
+          if (tid >= d) before += v;
+        }
+        for (uint32_t i = 0; i < n; ++i) {
+          const uint32_t left = c - i * kShortTileM;
+          reinterpret_cast<uint4 *>(shorts.list)[1 + t_short + before - n + i] =
+              make_uint4((uint32_t)e, cnt[e] + i * kShortTileM, left < (uint32_t)kShortTileM ? left : (uint32_t)kShortTileM, 0u);
+        }
+        t_short += __shfl(before, kWave - 1, kWave);
+      }
       const bool r128 = big && ts.r != 0u && ts.rcls == 1, r64 = big && ts.r != 0u && ts.rcls == 2;
       const uint64_t b128 = __ballot(r128), b64 = __ballot(r64);
       if (r128 || r64) {
@@ -190,6 +205,7 @@ __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint
         l128[0] = t128;
         l64[0] = t64;
       }
+      if (shorts.list) shorts.list[0] = t_short;
     }
   }
   __syncthreads();
@@ -203,7 +219,7 @@ __device__ __forceinline__ void dispatch_block(const uint32_t *flat, int64_t P, 
                                uint32_t *__restrict__ offsets, uint32_t *__restrict__ perm,
                                uint32_t *__restrict__ inv_perm, uint32_t *__restrict__ src_of,
                                uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256,
-                               uint32_t big_thr) {
+                               uint32_t big_thr, ShortTiles shorts) {
   __shared__ uint32_t n_active;
   uint32_t *cnt = lds, *tmp = lds + E, *cur = lds + 2 * E, *wcnt = lds + 3 * E;
   const int tid = threadIdx.x;
@@ -214,7 +230,7 @@ __device__ __forceinline__ void dispatch_block(const uint32_t *flat, int64_t P, 
     atomicAdd(&cnt[e < (uint32_t)E ? e : (uint32_t)E - 1u], 1u);
   }
   __syncthreads();
-  finish_counts(cnt, tmp, cur, E, counts, offsets, work, mtiles, cap256, big_thr, &n_active);
+  finish_counts(cnt, tmp, cur, E, counts, offsets, work, mtiles, cap256, big_thr, shorts, &n_active);
   scatter_range(flat, 0, P, E, nbits, k_div, cur, wcnt, perm, inv_perm, src_of);
   // source rows of the first rows of every segment, so that a consumer needs one load
   if (work) {

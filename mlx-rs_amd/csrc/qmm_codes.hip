@@ -1,28 +1,8 @@
-// Tiled quantized product on raw codes: activations in bfloat16 or float16, groups of 32, 64 or 128, any number of
-// output columns.
-//
-// Contract: mlx_quantized_matmul / mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:91-122,160-230).
-//
-// Arithmetic: sum_c x_c (s q_c + b) = s sum_c x_c (q_c - c) + (b + c s) sum_c x_c per quantisation group, with the codes' centre c
-// (8 or 128).  Centred codes are exact in bf16 and in f16, so the matrix cores multiply the activations with them and nothing is
-// rounded on the way in:
-//   bf16  x as it is; codes through v_cvt_f32_i32 of signed bytes (4-bit codes times 16)
-//   f16   x as it is, codes in f16 (v_mfma_f32_32x32x16_f16)
-// The centre keeps the sums as exact as plain ones: share of results that are not the float64 product's nearest value, plain / codes
-// as they are (bf16, 4-bit: 128 + q) / centred, 17 to 1000 rows: bf16 4-bit 9e-5 / 4.7e-3 / 1.0e-4, 8-bit 1.5e-4 / 4.0e-4 / 1.1e-4, f16
-// 1.1e-3 / 2.7e-3 / 7.3e-4.  What it costs is the conversion of 4-bit codes in bf16, 15 instructions a multiply for 7: 50 us of
-// 1000 x 2080 x 3968 against 53, nothing below 300 rows.
-// float32 does not come here: without the centre its error was 3.3e-7 to 5.7e-7 (a wave per output element 1.0e-7 to 1.5e-7).
-// The fp32 sums of a group are scaled once, when the group ends.  The bias term sum_g b_g (sum_c x_c) is a product of
-// its own over the groups: the group sums of x (fp32, split into three bf16 pieces) against the biases (three pieces
-// as well), eight K slots a group (xh bh, xm bh, xl bh, xh bm, xm bm, xh bl: every product down to 2^-24), which the
-// matrix cores accumulate straight into the result: K / group * 8 / K = 12 % more MFMA work with groups of 64.
-//
-// A kernel of its own (prepare_rows) walks x once and writes the group sums in that form and, for 4-bit codes with bf16
-// and f16, the copy with paired 8-blocks that their unpacking wants.
+// The middle of the range of dense products on raw codes (which: start_dense in qmm_tiles.hip, whose contract, arithmetic and prepared
+// rows these are, with c = 8 or 128): tiles of 64 x 128 whose waves load their codes straight into the registers that unpack them.
 #include <type_traits>
 
-#include "qmm_dev.hpp"
+#include "qmm_codes_dev.hpp"
 
 namespace mi_moe {
 
@@ -31,23 +11,10 @@ namespace {
 constexpr int kStep = 64;      // K values per step; two steps between barriers
 constexpr int kRow = 17;       // LDS row stride in 16-byte units: 128 values and 16 bytes that keep rows off each other's banks
 constexpr uint32_t kOutside = 0x80000000u;  // an offset past every descriptor here: such a load returns zeros
-constexpr int kSlots = 8;      // K slots of a group in the bias product
 constexpr int kWeave = 7;  // vector instructions between two matrix instructions
 constexpr size_t kLdsAtLeast = 4 * 32 * (32 * 2 + 16);  // the epilogue's staging
 
 typedef uint32_t u32x3_t __attribute__((ext_vector_type(3)));
-
-// v = h + m + l exactly, each a bf16 (8 significant bits; by truncation, so nothing overflows).  A value that is not
-// finite gives a NaN.
-struct Pieces { uint32_t h, m, l; };  // bf16 bits in the low halves
-__device__ __forceinline__ Pieces split3(float v) {
-  const uint32_t u = __float_as_uint(v);
-  const uint32_t hu = u & 0xffff0000u;
-  const float r = v - __uint_as_float(hu);
-  const uint32_t mu = __float_as_uint(r) & 0xffff0000u;
-  const float q = r - __uint_as_float(mu);
-  return Pieces{hu >> 16, mu >> 16, __float_as_uint(q) >> 16};
-}
 
 // a multiply function together with how it deals K values to its four multiplies (see qmm_codes_kernel)
 template <bool SPLIT, class F>
@@ -58,60 +25,10 @@ struct Split : F {
 template <bool SPLIT, class F>
 __device__ __forceinline__ Split<SPLIT, F> with_split(F f) { return Split<SPLIT, F>(f); }
 
-constexpr bool paired_order(int bits) { return bits == 4; }  // 8-blocks as (0,4)(1,5)(2,6)(3,7)
-constexpr int padded_groups(int G) { return (G + 15) / 16 * 16; }  // the bias product runs an even number of steps of eight groups
-
 }  // namespace
 
-// One thread per eight values of x.
-template <int DT>
-__global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf<DT>::type *__restrict__ x, int64_t n_octets,
-                                                           int octets_per_row, int lanes_log2,
-                                                           uint16_t *__restrict__ copy, uint16_t *__restrict__ sums, int sums_row) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n_octets) return;  // whole groups leave together
-  float v[8];
-  {
-    const uint4 w = reinterpret_cast<const uint4 *>(x)[i];
-    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if constexpr (DT == 0) {
-        v[2 * j] = bf16lo_to_f32(u[j]);
-        v[2 * j + 1] = bf16hi_to_f32(u[j]);
-      } else {
-        const half2_t hh = __builtin_bit_cast(half2_t, u[j]);
-        v[2 * j] = (float)hh.x;
-        v[2 * j + 1] = (float)hh.y;
-      }
-    }
-    if (copy) {
-      uint4 p;
-      p.x = (w.x & 0xffffu) | (w.z << 16);
-      p.y = (w.x >> 16) | (w.z & 0xffff0000u);
-      p.z = (w.y & 0xffffu) | (w.w << 16);
-      p.w = (w.y >> 16) | (w.w & 0xffff0000u);
-      *reinterpret_cast<uint4 *>(copy + 8 * i) = p;
-    }
-  }
-  float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-  sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
-  sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
-  if (lanes_log2 >= 3) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
-  if (lanes_log2 == 4) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
-  if ((i & ((1 << lanes_log2) - 1)) == 0) {
-    const int64_t row = i / octets_per_row;
-    const int g = (int)(i % octets_per_row) >> lanes_log2, G = octets_per_row >> lanes_log2;
-    const Pieces p = split3(sum);
-    uint4 *const to = reinterpret_cast<uint4 *>(sums + row * sums_row) + g;
-    *to = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, 0u);
-    if (g == G - 1)
-      for (int k = 1; g + k < sums_row / kSlots; ++k) to[k] = make_uint4(0, 0, 0, 0);
-  }
-}
-
-// A block computes 32 MS token rows x 32 WN NT weight rows with WN KW waves.  A wave owns 32 weight rows (NT = 2: and
-// the 32 matching ones of the up matrix, or 32 WN rows further on) for all the block's token rows, so it loads its own codes straight
+// A block computes 32 MS token rows x 32 WN weight rows with WN KW waves.  A wave owns 32 weight rows
+// for all the block's token rows, so it loads its own codes straight
 // into the lanes that multiply them and unpacks them in registers: nothing of the weights passes through LDS, and no
 // wave unpacks what another one does.  A lane (weight row l % 32, half l / 32) loads 16 bytes; which K values its
 // eight codes of a multiply stand for is free as long as the token operand agrees:
@@ -129,13 +46,13 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf
 // KW > 1: the block's waves form KW groups that share K among them, each with LDS buffers of its own; their sums meet in
 // LDS at the end, added in group order.  For launches that give a CU one block or less.
 // DT: 0 bf16, 1 f16.  G32: groups of 32; otherwise a group is one or two steps (scale_shift).
-template <int DT, int BITS, bool G32, bool GLU, int MS, int NT, int WN, int KW>
+template <int DT, int BITS, bool G32, int MS, int WN, int KW>
 __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2, 4))) void qmm_codes_kernel(
-    CodesArgs a, const uint32_t *__restrict__ lists, int n_mtiles, int n_experts, int n_ntiles, int scale_shift) {
-  static_assert(!GLU || NT == 2, "a gate tile and its up tile");
+    CodesArgs a, int n_mtiles, int n_ntiles, int scale_shift) {
+  constexpr int NT = 1;
   typedef typename ElemOf<DT>::type T;
   constexpr int BM = 32 * MS;
-  constexpr int NI = 32 * WN * (GLU ? 1 : NT);  // distinct output columns per block
+  constexpr int NI = 32 * WN;                // output columns per block
   constexpr int NA = BM * 8 / (64 * WN);     // 16-byte activation loads per thread, piece and step
   constexpr int RS = 8 * WN;                 // rows one such load of a group covers
   constexpr int NQ = BITS == 4 ? 1 : 2;      // 16-byte code loads per lane, tile and step
@@ -145,39 +62,13 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   constexpr int A_SZ = BM * kRow, BUF = A_SZ;                      // 16-byte units
   static_assert(BM % RS == 0, "whole loads");
 
-  // block -> (M tile, N tile).  Ids are dealt round-robin over the 8 XCDs.  Dense: an XCD takes every eighth N tile
-  // and all M tiles of it, so its L2 holds the weights of a few N tiles and x streams through.  Tile lists: whole M
-  // tiles per XCD (the blocks of one share its gathered rows).
+  // block -> (M tile, N tile).  Ids are dealt round-robin over the 8 XCDs: an XCD takes every eighth N tile and all M tiles of it, so its
+  // L2 holds the weights of a few N tiles and x streams through.
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-  int e = 0, rows, nt;
-  int64_t row0;
-  if (lists) {
-    // the three lists behind each other, every tile cut into pieces of BM rows: ids in the order of the lists' capacities
-    uint32_t id = (uint32_t)(j / n_ntiles) * 8u + xcd;
-    nt = j % n_ntiles;
-    int cls = 0, pieces = kBigTileM / BM;
-    uint32_t capacity = (uint32_t)n_mtiles * pieces;
-    while (cls < 2 && id >= capacity) {
-      id -= capacity;
-      ++cls;
-      pieces /= 2;
-      capacity = (uint32_t)n_experts * pieces;
-    }
-    const uint32_t *const list = tile_list(lists, cls, n_mtiles, n_experts);
-    const uint32_t in_list = id / (uint32_t)pieces;
-    if (in_list >= list[0]) return;
-    const uint4 rec = reinterpret_cast<const uint4 *>(list)[1 + in_list];
-    const int part = (int)(id % (uint32_t)pieces) * BM;
-    e = (int)rec.x;
-    row0 = (int64_t)rec.y + part;
-    rows = (int)rec.z - part < BM ? (int)rec.z - part : BM;
-  } else {
-    nt = j / n_mtiles * 8 + xcd;
-    if (nt >= n_ntiles) return;
-    row0 = (int64_t)(j % n_mtiles) * BM;
-    rows = a.M - row0 < BM ? (int)(a.M - row0) : BM;
-  }
-  if (rows <= 0) return;
+  const int nt = j / n_mtiles * 8 + xcd;
+  if (nt >= n_ntiles) return;
+  const int64_t row0 = (int64_t)(j % n_mtiles) * BM;
+  const int rows = a.M - row0 < BM ? (int)(a.M - row0) : BM;
 
   const int lane = threadIdx.x & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -200,26 +91,22 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   for (int i = 0; i < NA; ++i) {
     int tr = arg + RS * i;
     tr = tr < rows ? tr : rows - 1;  // rows past the end repeat the last one (never stored)
-    const uint32_t r = a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr);
+    const uint32_t r = (uint32_t)(row0 + tr);
     x_voff[i] = (r * (uint32_t)K + acp * 8) * sizeof(T);
     xs_voff[i] = (r * (uint32_t)ext + acp * 8) * 2;
   }
   // ---- the weight rows of this lane
   const int ln = lane & 31, kb = lane >> 5;
-  const int64_t ebase = (int64_t)e * N;
   __amdgpu_buffer_rsrc_t wr[NT], sr[NT], br[NT];
   uint32_t w_voff[NT], s_voff[NT];
   int w_row[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const bool up = GLU && t == 1;
-    // paired output (see GroupedArgs::y_paired): the lane at position p of an 8-block takes the row whose result belongs there
-    const int lnp = a.y_paired ? ((ln & ~7) | (((ln & 7) >> 1) + ((ln & 1) ? 4 : 0))) : ln;
-    int row = n0 + 32 * wave + lnp + (GLU ? 0 : 32 * WN * t);
+    int row = n0 + 32 * wave + ln;
     row = row < N ? row : N - 1;  // columns past the end repeat the last one (never stored)
-    wr[t] = rsrc_of((up ? a.w1 : a.w0) + ebase * (row_bytes / 4), (uint32_t)N * row_bytes);
-    sr[t] = rsrc_of(static_cast<const T *>(up ? a.s1 : a.s0) + ebase * G, (uint32_t)N * G * sizeof(T));  // (read in words: the host takes an even number of them)
-    br[t] = rsrc_of(static_cast<const T *>(up ? a.b1 : a.b0) + ebase * G, (uint32_t)N * G * sizeof(T));
+    wr[t] = rsrc_of(a.w0, (uint32_t)N * row_bytes);
+    sr[t] = rsrc_of(a.s0, (uint32_t)N * G * sizeof(T));  // (read in words: the host takes an even number of them)
+    br[t] = rsrc_of(a.b0, (uint32_t)N * G * sizeof(T));
     w_row[t] = row;
     w_voff[t] = (uint32_t)row * row_bytes + kb * 16;
     s_voff[t] = (uint32_t)row * G * sizeof(T);
@@ -524,12 +411,11 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
   for (int m = 0; m < MS; ++m)
 #pragma unroll
-    for (int t = 0; t < (GLU ? 1 : NT); ++t) {
-      const int col0 = n0 + 32 * wave + 32 * WN * t;
+    for (int t = 0; t < NT; ++t) {
+      const int col0 = n0 + 32 * wave;
       const int bc = col0 + ln < N ? col0 + ln : N - 1;
       const float lb = a.bias ? as_f32(static_cast<const T *>(a.bias)[bc]) : 0.f;
-      auto put = [&](int r, float v, float up) __attribute__((always_inline)) {
-        if constexpr (GLU) v = v / (1.0f + __expf(-v)) * up;
+      auto put = [&](int r, float v) __attribute__((always_inline)) {
         T o = rounded<T>(v);
         if (a.bias) o = rounded<T>(as_f32(o) + lb);
         reinterpret_cast<T *>(mine + (8 * (r >> 2) + 4 * kb + (r & 3)) * ROWB)[ln] = o;
@@ -537,9 +423,8 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
       uint32_t again = 0;  // (bits: which of the sixteen sums are not finite)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float v = tot[m][t][r], up = tot[m][GLU ? 1 : t][r];
-        put(r, v, up);
-        again |= (not_finite(v) || (GLU && not_finite(up)) ? 1u : 0u) << r;
+        put(r, tot[m][t][r]);
+        again |= (not_finite(tot[m][t][r]) ? 1u : 0u) << r;
       }
 #pragma unroll 1
       for (int quad = 0; __builtin_expect(again != 0, 0); ++quad, again >>= 4) {  // rows 8 quad + 4 kb + 0 .. 3
@@ -552,20 +437,15 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
             open &= ~(1u << i);
             tr = rows - 1;
           }
-          xs[i] = static_cast<const T *>(a.x) + (int64_t)(a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr)) * K;
+          xs[i] = static_cast<const T *>(a.x) + (row0 + tr) * K;
         }
         if (!open) continue;
-        float v[GLU ? 2 : 1][4];
-#pragma unroll
-        for (int i = 0; i < (GLU ? 2 : 1); ++i) {
-          const int64_t wrow = ebase + w_row[GLU ? i : t];
-          plain_rows<BITS, 4, T>(xs, paired_order(BITS), (GLU && i ? a.w1 : a.w0) + wrow * (row_bytes / 4),
-                              static_cast<const T *>(GLU && i ? a.s1 : a.s0) + wrow * G,
-                              static_cast<const T *>(GLU && i ? a.b1 : a.b0) + wrow * G, K, K / G, open, v[i]);
-        }
+        float v[4];
+        plain_rows<BITS, 4, T>(xs, paired_order(BITS), a.w0 + (int64_t)w_row[t] * (row_bytes / 4), static_cast<const T *>(a.s0) + (int64_t)w_row[t] * G,
+                               static_cast<const T *>(a.b0) + (int64_t)w_row[t] * G, K, K / G, open, v);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (open >> i & 1u) put(4 * quad + i, v[0][i], v[GLU ? 1 : 0][i]);
+          if (open >> i & 1u) put(4 * quad + i, v[i]);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -576,8 +456,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
         const int row = RPI * i + my_row;
         const int tr = 32 * m + row;
         if (tr < rows && my_col < N) {
-          const int64_t dst = a.dst_rows ? (int64_t)a.dst_rows[row0 + tr] : row0 + tr;
-          T *const to = static_cast<T *>(a.y) + dst * N + my_col;
+          T *const to = static_cast<T *>(a.y) + (row0 + tr) * N + my_col;
           const T *const from = reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece;
           if (vec) {
             *reinterpret_cast<u32x4_t *>(to) = *reinterpret_cast<const u32x4_t *>(from);
@@ -592,84 +471,28 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     }
 }
 
-size_t codes_copy_bytes(int bits, int64_t rows, int K) {
-  return paired_order(bits) ? (size_t)rows * K * 2 : 0;
-}
-size_t codes_sums_bytes(int64_t rows, int K, int group) { return (size_t)rows * padded_groups(K / group) * kSlots * 2; }
-
-hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
-                               uint16_t *sums, hipStream_t st) {
-  const int64_t n = rows * (K / 8);
-  if (n == 0) return hipSuccess;
-  const unsigned grid = (unsigned)((n + 255) / 256);
-  const int ll = group == 32 ? 2 : (group == 64 ? 3 : 4), row = padded_groups(K / group) * kSlots;
-  if (dt == 0) prepare_rows_kernel<0><<<grid, 256, 0, st>>>(static_cast<const uint16_t *>(x), n, K / 8, ll, copy, sums, row);
-  else if (dt == 1) prepare_rows_kernel<1><<<grid, 256, 0, st>>>(static_cast<const _Float16 *>(x), n, K / 8, ll, copy, sums, row);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-
-template <int DT, int BITS, bool G32, bool GLU, int MS, int NT, int WN, int KW>
-static hipError_t start_codes(const CodesArgs &a, int scale_shift, const uint32_t *lists, int cap256, int n_experts, hipStream_t st) {
-  constexpr int NI = 32 * WN * (GLU ? 1 : NT), BM = 32 * MS;
-  constexpr size_t bufs = (size_t)2 * KW * BM * kRow * 16 + WN * KW * NT * 32 * 48, sums = KW > 1 ? (size_t)BM * 32 * WN * NT * 4 : 0;
+template <int DT, int BITS, bool G32>
+static hipError_t start_codes(const CodesArgs &a, int scale_shift, hipStream_t st) {
+  constexpr int MS = 2, WN = 4, KW = 2, NI = 32 * WN, BM = 32 * MS;
+  constexpr size_t bufs = (size_t)2 * KW * BM * kRow * 16 + WN * KW * 32 * 48, sums = (size_t)BM * 32 * WN * 4;
   constexpr size_t most = bufs > sums ? bufs : sums, lds = most > kLdsAtLeast ? most : kLdsAtLeast;
   static_assert(lds <= 160 * 1024, "more LDS than a CU has");
-  const int n_ntiles = (a.N + NI - 1) / NI;
-  const int mtiles = lists ? cap256 : (int)((a.M + BM - 1) / BM);
-  const int64_t pieces = (int64_t)cap256 * (256 / BM) + (int64_t)n_experts * (128 / BM + 64 / BM);
-  const int64_t grid = lists ? (pieces + 7) / 8 * 8 * n_ntiles : (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
+  const int n_ntiles = (a.N + NI - 1) / NI, mtiles = (int)((a.M + BM - 1) / BM);
+  const int64_t grid = (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
   if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
-  const auto kernel = &qmm_codes_kernel<DT, BITS, G32, GLU, MS, NT, WN, KW>;
+  const auto kernel = &qmm_codes_kernel<DT, BITS, G32, MS, WN, KW>;
   if (lds > 64 * 1024)
     if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         e != hipSuccess)
       return e;
-  kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, lists, mtiles, n_experts, n_ntiles, scale_shift);
+  kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, mtiles, n_ntiles, scale_shift);
   return hipGetLastError();
 }
 
-// Which tile, from the number of tiles a launch of each has (256 CUs).  Measured with f16, 4-bit, groups of 64, us of the
-// whole call at (M, N, K) = (96, 4096, 4096) / (160, 4096, 4096) / (400, 4096, 4096) / (640, 2304, 2304) / (1000, 1024, 4096)
-// / (1000, 4096, 4096):
-//   32 x 64, K shared by four groups:   22.0 / 31.5 / 58.6 / 39.7 / 38.7 / 121   while a CU gets one at most
-//   64 x 128, K shared by two groups:   35.6 / 36.5 / 41.1 / 29.7 / 39.9 / 75.8  while a CU gets one at most
-//   64 x 128:                           41.5 / 42.4 / 46.7 / 31.0 / 45.6 / 66.7  (several blocks a CU overlap as K groups do)
-// Between one and two 32 x 64 tiles a CU the two are as fast with f16 and K = 4096; bf16, 4-bit, 32 x 64 / 64 x 128:
-// (200, 4096, 2048) 32.0 / 24.8, (200, 4096, 4096) 39.9 / 37.4, (1000, 1024, 1024) 29.7 / 21.8, (400, 2048, 768) 19.7 / 14.7.
-// (128 x 128 tiles: 65.1 / 67.0 / 70.2 / 45.9 / 69.3 / 76.0.)  These compare tiles as they were before the codes were centred; the rule's
-// choices by the kernels' time now: 17.9 / 29.7 / 34.7 / 25.3 / 34.0 / 62.0 and, bf16, 20.0, 33.1, 16.7, 14.1.
-template <int DT, int BITS, bool G32>
-static hipError_t start_dense(const CodesArgs &a, int scale_shift, hipStream_t st) {
-  auto tiles = [&](int rows, int cols) { return (a.M + rows - 1) / rows * ((a.N + cols - 1) / cols); };
-  if (tiles(32, 64) <= 256) return start_codes<DT, BITS, G32, false, 1, 1, 2, 4>(a, scale_shift, nullptr, 0, 0, st);
-  if (tiles(64, 128) <= 256) return start_codes<DT, BITS, G32, false, 2, 1, 4, 2>(a, scale_shift, nullptr, 0, 0, st);
-  return start_codes<DT, BITS, G32, false, 2, 1, 4, 1>(a, scale_shift, nullptr, 0, 0, st);
-}
-
-// The M-tile lists of a grouped product (see tile_list) in one launch, in blocks of 64 rows x 128 columns.  Measured on
-// the 128-expert shape with groups of 32, us of a forward at 200 / 512 tokens, even and Zipf-1.1 routing: three launches,
-// a list each, 225, 314 / 260, 373; one launch 224, 246 / 252, 310; one launch with gate/up blocks of 32 rows 217, 242 /
-// 332, 335; with gate/up blocks of 32 x 64 and K shared by two groups 288, 347 / 628, 524.  (Before the codes were centred; the kept form
-// takes 251 at 512 tokens and even routing now, where it took 268.)
-hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *lists, int cap256, int n_experts, int group, int bits,
-                                  bool glu, hipStream_t st) {
-  auto run = [&](auto b, auto g32) {
-    constexpr int BITS = decltype(b)::value;
-    constexpr bool G32 = decltype(g32)::value;
-    if (glu) return start_codes<0, BITS, G32, true, 2, 2, 4, 1>(a, group == 128, lists, cap256, n_experts, st);
-    return start_codes<0, BITS, G32, false, 2, 1, 4, 1>(a, group == 128, lists, cap256, n_experts, st);
-  };
-  auto with_group = [&](auto b) { return group == 32 ? run(b, std::true_type{}) : run(b, std::false_type{}); };
-  return bits == 4 ? with_group(std::integral_constant<int, 4>{}) : with_group(std::integral_constant<int, 8>{});
-}
-
-hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st) {
-  if (a.M == 0) return hipSuccess;
+hipError_t launch_qmm_codes_middle(const CodesArgs &a, int group, int bits, int dt, hipStream_t st) {
   auto with_group = [&](auto d, auto b) {
     constexpr int DT = decltype(d)::value, BITS = decltype(b)::value;
-    if (group == 32) return start_dense<DT, BITS, true>(a, 0, st);
-    return start_dense<DT, BITS, false>(a, group == 128, st);
+    return group == 32 ? start_codes<DT, BITS, true>(a, 0, st) : start_codes<DT, BITS, false>(a, group == 128, st);
   };
   auto with_bits = [&](auto d) {
     return bits == 4 ? with_group(d, std::integral_constant<int, 4>{}) : with_group(d, std::integral_constant<int, 8>{});

@@ -1,0 +1,27 @@
+// What the two tiled products on raw codes (qmm_tiles.hip, qmm_codes.hip) share: the layout of the prepared rows.
+#pragma once
+#include "qmm_dev.hpp"
+
+namespace mi_moe {
+
+constexpr int kSlots = 8;  // K slots of a group in the bias product
+
+// v = h + m + l exactly, each a bf16 (8 significant bits; by truncation, so nothing overflows).  A value that is not
+// finite gives a NaN.
+struct Pieces { uint32_t h, m, l; };  // bf16 bits in the low halves
+__device__ __forceinline__ Pieces split3(float v) {
+  const uint32_t u = __float_as_uint(v);
+  const uint32_t hu = u & 0xffff0000u;
+  const float r = v - __uint_as_float(hu);
+  const uint32_t mu = __float_as_uint(r) & 0xffff0000u;
+  const float q = r - __uint_as_float(mu);
+  return Pieces{hu >> 16, mu >> 16, __float_as_uint(q) >> 16};
+}
+
+constexpr bool paired_order(int bits) { return bits == 4; }  // 8-blocks as (0,4)(1,5)(2,6)(3,7)
+constexpr int padded_groups(int G) { return (G + 15) / 16 * 16; }  // whole windows of the bias product; the groups past the row's end are zeros
+
+// The middle of the range of dense products, which qmm_codes.hip still takes (see start_dense in qmm_tiles.hip).
+hipError_t launch_qmm_codes_middle(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
+
+}  // namespace mi_moe

@@ -1,0 +1,747 @@
+// Tiled quantized product on raw codes: activations in bfloat16 or float16, groups of 32, 64 or 128, any number of
+// output columns; dense, or the tiles of a list (the segments of a mixture-of-experts block).
+//
+// Contract: mlx_quantized_matmul / mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:91-122,160-230).
+//
+// Arithmetic: sum_c x_c (s q_c + b) = s sum_c x_c (q_c - c) + (b + c s) sum_c x_c per quantisation group, with a centre c of
+// the codes.  q - c is exact in bf16 and in f16, so the matrix cores multiply the activations with it and nothing is
+// rounded on the way in:
+//   bf16  x as it is; codes through v_cvt_f32_i32 of signed bytes (4-bit codes times 16), c = 8 or 128
+//   f16   x as it is, codes in f16 (v_mfma_f32_32x32x16_f16), the same c
+//   blocks with 4-bit codes in groups of 64: c = 0, codes through v_cvt_scalef32_pk_bf16_fp8 (a byte of 0 .. 15 is that many 2^-9 as an
+//         8-bit float, exactly), 8 instructions a multiply for 15
+// Share of results that are not the float64 product's nearest value (bf16, 4-bit, 64 to 777 rows): plain float32 sums 0.9e-4 .. 1.5e-4, c = 8
+// 1.1e-4 .. 1.7e-4, c = 0 3.3e-4, 128 + q (what the streaming kernel multiplies with) 4.7e-3, weights rounded to bf16 (the 256-column
+// tiles) no comparison.  Groups of 32 and 128 and the dense products keep c = 8.
+// float32 does not come here: without the centre its error was 3.3e-7 to 5.7e-7 (a wave per output element 1.0e-7 to 1.5e-7).
+// The fp32 sums of a group are scaled once, when the group ends.  The bias term sum_g b_g (sum_c x_c) is a product of
+// its own over the groups: the group sums of x (fp32, split into three bf16 pieces) against the biases (three pieces
+// as well), eight K slots a group (xh bh, xm bh, xl bh, xh bm, xm bm, xh bl: every product down to 2^-24): K / group * 8 / K = 12 % more
+// matrix work with groups of 64.  It runs a window of 8 or 16 groups ahead of the window's codes, so that the sums never drift far.
+//
+// A kernel of its own (prepare_rows) walks x once and writes the group sums in that form and, for 4-bit codes with bf16
+// and f16, the copy with paired 8-blocks that their unpacking wants.
+#include <type_traits>
+
+#include "qmm_codes_dev.hpp"
+
+namespace mi_moe {
+
+// One thread per eight values of x.
+template <int DT>
+__global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf<DT>::type *__restrict__ x, int64_t n_octets,
+                                                           int octets_per_row, int lanes_log2,
+                                                           uint16_t *__restrict__ copy, uint16_t *__restrict__ sums, int sums_row) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n_octets) return;  // whole groups leave together
+  float v[8];
+  {
+    const uint4 w = reinterpret_cast<const uint4 *>(x)[i];
+    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (DT == 0) {
+        v[2 * j] = bf16lo_to_f32(u[j]);
+        v[2 * j + 1] = bf16hi_to_f32(u[j]);
+      } else {
+        const half2_t hh = __builtin_bit_cast(half2_t, u[j]);
+        v[2 * j] = (float)hh.x;
+        v[2 * j + 1] = (float)hh.y;
+      }
+    }
+    if (copy) {
+      uint4 p;
+      p.x = (w.x & 0xffffu) | (w.z << 16);
+      p.y = (w.x >> 16) | (w.z & 0xffff0000u);
+      p.z = (w.y & 0xffffu) | (w.w << 16);
+      p.w = (w.y >> 16) | (w.w & 0xffff0000u);
+      *reinterpret_cast<uint4 *>(copy + 8 * i) = p;
+    }
+  }
+  float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
+  sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
+  if (lanes_log2 >= 3) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
+  if (lanes_log2 == 4) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
+  if ((i & ((1 << lanes_log2) - 1)) == 0) {
+    const int64_t row = i / octets_per_row;
+    const int g = (int)(i % octets_per_row) >> lanes_log2, G = octets_per_row >> lanes_log2;
+    const Pieces p = split3(sum);
+    uint4 *const to = reinterpret_cast<uint4 *>(sums + row * sums_row) + g;
+    *to = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, 0u);
+    if (g == G - 1)
+      for (int k = 1; g + k < sums_row / kSlots; ++k) to[k] = make_uint4(0, 0, 0, 0);
+  }
+}
+
+// ---- copies from memory straight into LDS
+// Written out because the compiler waits for every copy in flight ahead of any read of LDS; it knows nothing of these, and the
+// kernel counts them itself.  (The compiler's own counts of loads in flight stay safe: with loads it does not know of in
+// between it waits for more than it has to.)  A lane's 16 bytes go to LDS at `to` + 16 lane; what lies past the descriptor's end is zeros.
+// Measured out of L2, bytes a cycle and CU: pieces of 64 consecutive bytes 31, of 128 and more 60; 32 bytes a row, as matrix operands
+// loaded straight into registers are, 18.
+typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ i32x4_t words_of(const void *base, uint32_t bytes) {
+  const uint64_t p = reinterpret_cast<uint64_t>(base);
+  return i32x4_t{(int32_t)(uint32_t)p, (int32_t)(uint32_t)(p >> 32), (int32_t)bytes, 0x00020000};
+}
+__device__ __forceinline__ void copy_to_lds(i32x4_t rsrc, uint32_t voff, uint32_t soff, uint32_t to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(to), "v"(voff), "s"(rsrc), "s"(soff));
+}
+template <int N>
+__device__ __forceinline__ void wait_copies() {  // all but the last N have arrived; LDS reads are done
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void block_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
+// What a launch of the kernel below is made of, for its two sides.
+template <int BITS, int MS, int NT, int WN, int S>
+struct Ring {
+  static constexpr int KS = BITS == 4 ? 128 : 64;  // K values of a stage: 64 bytes of codes per weight row
+  static constexpr int XROW = KS * 2;              // bytes of a token row
+  static constexpr int X = 32 * MS * XROW;         // token rows of a stage
+  static constexpr int W = NT * 2048;              // one wave's codes
+  static constexpr int STAGE = X + WN * W;
+  static constexpr int XI = (X + 1024 * WN - 1) / (1024 * WN);  // copies a wave makes of a stage's token rows
+  static constexpr int COPIES = XI + 2 * NT;                    // and in all
+  static constexpr int WINDOW = NT * 1024;                      // 32 bytes of scales per weight row of a wave
+  static constexpr int BYTES = S * STAGE + WN * WINDOW;
+};
+
+// LDS of a block: where two blocks share a CU, each takes its half.
+constexpr int kHalfLds = 80 * 1024;
+constexpr int lds_of(int kw, int bytes) { return kw == 1 && bytes > kHalfLds / 2 && bytes <= kHalfLds ? kHalfLds : kw * bytes; }
+
+template <int DT, int BITS, bool G32, bool MID, int MS, int NT, int WN, int S>
+struct Tile {
+  typedef typename ElemOf<DT>::type T;
+  typedef Ring<BITS, MS, NT, WN, S> R;
+  static constexpr bool SPLIT = BITS == 8 || G32;  // which K values a multiply takes: see unpack
+  static constexpr bool kPlainCodes = MID && BITS == 4 && DT == 0;
+  static constexpr float kCentre = kPlainCodes ? 0.0f : centre_of(BITS);                       // the codes are multiplied as
+  static constexpr float kUnit = BITS == 4 && DT == 0 && !kPlainCodes ? 0.0625f : 1.0f;  // (q - kCentre) / kUnit
+  static constexpr int JS = R::KS / 64;  // steps of a stage
+  static constexpr int NQ = BITS == 4 ? 1 : 2;
+  static constexpr int NS = G32 ? 2 : 1;
+  static constexpr int GB = R::KS / 8;   // groups of a stage of the bias product
+
+  // 4-bit codes in groups of 32: the words dealt so that a multiply stays inside one group
+  static __device__ __forceinline__ void deal(u32x4_t (&q)[NQ]) {
+    if constexpr (BITS == 4 && G32) {
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        const auto r = __builtin_amdgcn_permlane32_swap(q[0][w], q[0][w + 2], false, false);
+        q[0][w] = r[0];
+        q[0][w + 2] = r[1];
+      }
+    }
+  }
+  // the eight codes of multiply h
+  static __device__ __forceinline__ void unpack(const u32x4_t (&q)[NQ], int h, u32x4_t &o) {
+      if constexpr (kPlainCodes) {
+        // a byte of 0 to 15 is that many 2^-9 as an 8-bit float (four exponent bits, three of mantissa): the conversion takes two at a time
+        const uint32_t w = __builtin_amdgcn_perm(q[0][h], q[0][h], 0x03010200u), even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
+        o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false));
+        o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false));
+        o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true));
+        o[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, true));
+      } else if constexpr (BITS == 4 && DT == 0) {
+        float v[8];
+        centred_codes(q[0][h], v);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = upper_halves(v[i], v[i + 4]);
+      } else if constexpr (BITS == 4) {
+        const uint32_t w = q[0][h];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (i % 2 == 0) {
+            o[i] = f16_centred<4>(__builtin_amdgcn_bitop3_b32(w >> (4 * i), 0x000f000fu, 0x64006400u, 0xEA));  // (a & b) | c
+          } else {  // 1024 + 16 q -> q - 8, exact as well: one shift serves two nibbles
+            const half2_t v = __builtin_bit_cast(half2_t, __builtin_amdgcn_bitop3_b32(w >> (4 * (i - 1)), 0x00f000f0u, 0x64006400u, 0xEA));
+            o[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, half2_t{(_Float16)0.0625f, (_Float16)0.0625f}, half2_t{(_Float16)-72.0f, (_Float16)-72.0f}));
+          }
+        }
+      } else if constexpr (DT == 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)  // bytes 2 i, 2 i + 1 under the exponent of 1024
+          o[i] = f16_centred<8>(__builtin_amdgcn_perm(0x64646464u, q[h >> 1][2 * (h & 1) + (i >> 1)], (i & 1) ? 0x07030702u : 0x07010700u));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          float v[4];
+          centred_codes(q[h >> 1][2 * (h & 1) + (i >> 1)], v);
+          o[i] = upper_halves(v[0], v[1]);
+          o[i + 1] = upper_halves(v[2], v[3]);
+        }
+      }
+  }
+};
+
+
+// One tile: 32 MS token rows from sorted row `row0` (`rows` of them real) x 32 WN NT weight rows from n0 of matrix e (GLU: of two matrices).
+// A wave owns 32 NT weight rows for all the tile's token rows.  K runs in stages of 64 bytes of codes a weight row; token rows and codes are
+// copied straight into a ring of S stages in LDS, the rows for all waves (one barrier a stage), the codes for the wave that
+// unpacks them.  A lane (weight row l % 32, half l / 32) reads 16 bytes of codes at a time; which K values its eight codes of a multiply
+// stand for is free as long as the token operand agrees:
+//   4-bit, groups >= 64: 16 bytes are 32 codes, half h holds K values 32 h ..: multiply t takes word t of both halves;
+//   4-bit, groups of 32: two v_permlane32_swap deal the words so that a multiply stays inside one group;
+//   8-bit: 16 bytes are 16 codes, two reads a step of 64, groups of 32 stay apart by themselves.
+// KW > 1: the block's waves form KW groups that share K among them, each with a ring of its own; their sums meet in
+// LDS at the end, added in group order.
+// What bounds it: the vector instructions (unpacking 8 to 15 a multiply and 32 weight rows, the scaled addition of a group 16 a
+// sub-tile) issue beside the matrix instructions at 4 cycles each, about 1250 cycles a stage of 64 x 64 x 128 in c = 0 where its multiplies are
+// 1024; two waves a SIMD reach 0.55 of that, as reads, copies and the barrier of a stage add their latencies.  4096 x 4096, 777 rows, bf16 4-bit:
+// 58.7 us for the call = 444 TFLOP/s (tiles of 64 x 128 with the codes loaded into registers 63.4).
+// Blocks (128 experts, hidden 2048, 4-bit, groups of 64), us of a forward at 128 / 320 / 1024 tokens, even routing: 127 / 132 / 221; with streamed
+// segments, 256-column tiles and a copy of x on four streams, which they took before, 151 / 216 / 266.
+template <int DT, int BITS, bool G32, bool GLU, bool MID, int MS, int NT, int WN, int KW, int S>
+__device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t row0, int rows, int n0, int scale_shift, unsigned char *lds_raw) {
+  typedef Tile<DT, BITS, G32, MID, MS, NT, WN, S> P;
+  typedef typename P::R R;
+  typedef typename P::T T;
+  constexpr int GB = P::GB;
+  constexpr int NM = GLU ? 2 : 1;  // matrices
+  const int lane = threadIdx.x & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave_all % WN, kg = wave_all / WN;  // column tile, K group
+  const int N = a.N, K = a.K;
+  const int ln = lane & 31, kb = lane >> 5;
+  const int glog = G32 ? 5 : 6 + scale_shift, G = K >> glog;
+  const int row_bytes = K * BITS / 8;
+  unsigned char *const ring = lds_raw + kg * R::BYTES;
+  const uint32_t ring_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds_raw + (uint32_t)kg * R::BYTES;
+
+  // ---- operands.  Offsets are 32 bits: the host takes this kernel for operands below 4 GiB only.
+  const int64_t ebase = (int64_t)e * N;
+  const int ext = padded_groups(G) * kSlots;
+  const i32x4_t xr = words_of(a.x, (uint32_t)(a.x_rows * K * sizeof(T))), xsr = words_of(a.sums, (uint32_t)(a.x_rows * ext * 2));
+  const T *s_of[NM], *b_of[NM];
+  i32x4_t wr[NM], sr[NM], br[NM];
+#pragma unroll
+  for (int t = 0; t < NM; ++t) {
+    s_of[t] = static_cast<const T *>(t ? a.s1 : a.s0) + ebase * G, b_of[t] = static_cast<const T *>(t ? a.b1 : a.b0) + ebase * G;
+    wr[t] = words_of((t ? a.w1 : a.w0) + ebase * (row_bytes / 4), (uint32_t)N * row_bytes);
+    sr[t] = words_of(s_of[t], (uint32_t)N * G * sizeof(T)), br[t] = words_of(b_of[t], (uint32_t)N * G * sizeof(T));  // (read in words: the host takes an even number of them)
+  }
+  // weight row of place `at` (0 .. 31) of the wave's tile t.  Columns past the end repeat the last one (never stored).  Paired output
+  // (see GroupedArgs::y_paired): the place p of an 8-block takes the row whose result belongs there.
+  const int col0 = n0 + 32 * (GLU ? 1 : NT) * wave;
+  auto weight_row = [&](int t, int at) __attribute__((always_inline)) {
+    const int p = a.y_paired ? ((at & ~7) | (((at & 7) >> 1) + ((at & 1) ? 4 : 0))) : at, row = col0 + (GLU ? 0 : 32 * t) + p;
+    return row < N ? row : N - 1;
+  };
+  // ---- what a lane copies, and where it lies in LDS.  LDS gives 256 bytes a cycle, sixteen lanes' pieces, if they lie in different
+  // banks: place p of a row holds piece p ^ (a number of the row), so that sixteen rows' pieces of one number do.  (Turned by
+  // eight rows only: 7.3 cycles a read of a wave for 4.)
+  constexpr int XP = R::XROW / 16;  // pieces of a token row
+  constexpr int XALL = R::X / 1024;  // copies of a stage's token rows (fewer than waves: the first XALL of them make one each)
+  auto turned = [](int row) __attribute__((always_inline)) { return XP == 16 ? row & 15 : (row >> 1) & 7; };
+  uint32_t x_row[R::XI], x_piece[R::XI];
+#pragma unroll
+  for (int i = 0; i < R::XI; ++i) {
+    const int r = (wave * R::XI + i) % XALL * (64 / XP) + lane / XP;
+    const int tr = r < rows ? r : rows - 1;  // rows past the end repeat the last one (never stored)
+    x_row[i] = a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr);
+    x_piece[i] = ((lane % XP) ^ turned(r)) << 4;
+  }
+  uint32_t w_off[2 * NT], first_scale[NT], window_row[NT];
+#pragma unroll
+  for (int i = 0; i < 2 * NT; ++i) {
+    const int at = 16 * (i & 1) + (lane >> 2);
+    w_off[i] = (uint32_t)weight_row(i / 2, at) * row_bytes + (((lane & 3) ^ ((at >> 2) & 3)) << 4);
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) first_scale[t] = (uint32_t)weight_row(t, ln) * G, window_row[t] = (uint32_t)weight_row(t, lane >> 1) * G;
+
+  // ---- the stages.  K is dealt to the K groups in even shares; a share runs in windows of GB quantisation groups, each a stage of the
+  // bias product (which brings the window's scales) and then its stages of codes.
+  const int per_window = 1 << (glog - 3);  // stages of codes: GB groups
+  const int share = (K / 128 + 2 * KW - 1) / (2 * KW) * 256;  // K values
+  const int k_first = kg * share, k_end = k_first + share < K ? k_first + share : K;
+  const int stages_all = (share < K ? share : K) / R::KS, total = stages_all + (stages_all + per_window - 1) / per_window;  // of every K group
+  struct Next {  // a stage to be copied
+    int k, pos;  // first K value, place in the window (0: the bias product)
+  } next_w = {k_first, 0}, next_x = {k_first, 0};
+  auto advance = [&](Next &n) __attribute__((always_inline)) {
+    if (n.pos) n.k += R::KS;
+    n.pos = n.pos == per_window ? 0 : n.pos + 1;
+  };
+  // A stage's token rows are copied S - 1 stages ahead, its weights S: a wave's place in the ring is its own, and free as soon as it has read
+  // the codes out of it.  (Stages past the end copy the last one again: the number of copies in flight is always the same.)
+  auto copy_w = [&](int slot, int i) __attribute__((always_inline)) {  // copy i of 2 NT: the codes or a window's scales and biases
+    const int k = next_w.k < K ? next_w.k : K - R::KS;
+    const bool bias = next_w.pos == 0;
+    i32x4_t from;
+    const int of = GLU ? i / 2 : 0, t = i % NT, of_bias = GLU ? t : 0;  // (codes: two copies a tile; bias product: the tiles' scales, then their biases)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) from[w] = bias ? (i < NT ? sr : br)[of_bias][w] : wr[of][w];
+    const uint32_t off = ((window_row[t] + (k >> glog)) * (uint32_t)sizeof(T) & ~3u) + ((lane & 1) << 4);
+    copy_to_lds(from, bias ? off : w_off[i], bias ? 0 : k * BITS / 8, ring_at + slot * R::STAGE + R::X + wave * R::W + i * 1024);
+  };
+  auto copy_x = [&](int slot, int c) __attribute__((always_inline)) {  // copy c of XI: the token rows or their group sums
+    const int k = next_x.k < K ? next_x.k : K - R::KS;
+    const bool bias = next_x.pos == 0;
+    i32x4_t from;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) from[w] = bias ? xsr[w] : xr[w];
+    copy_to_lds(from, x_row[c] * (uint32_t)(bias ? ext * 2 : K * (int)sizeof(T)) + x_piece[c], bias ? (k >> glog) * 16 : k * (int)sizeof(T),
+                ring_at + slot * R::STAGE + (wave * R::XI + c) % XALL * 1024);
+  };
+  auto copy_weights = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) copy_w(slot, i);
+  };
+  auto copy_rows = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < R::XI; ++c) copy_x(slot, c);
+  };
+
+  float tot[MS][NT][16];  // (not vectors: the multiplies never touch them, and each may lie in a register of its own)
+  const f32x16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int m = 0; m < MS; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) tot[m][t][v] = 0.f;
+
+  // the bias product of the window that begins at k: group sums of x against b + centre s, accumulated into the result
+  unsigned char *const scales = ring + S * R::STAGE + wave * R::WINDOW;  // [tile][weight row][16 scales]
+  auto bias_product = [&](const unsigned char *at, int real, auto scale_and_bias) __attribute__((always_inline)) {
+    f32x16_t sum[MS][NT];
+#pragma unroll
+    for (int m = 0; m < MS; ++m)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) sum[m][t] = zero;
+#pragma unroll 1
+    for (int i = 0; i < GB / 2; ++i) {
+      const int g = 2 * i + kb;
+      u32x4_t F[MS];
+#pragma unroll
+      for (int m = 0; m < MS; ++m) F[m] = *reinterpret_cast<const u32x4_t *>(at + (32 * m + ln) * R::XROW + ((g ^ turned(ln)) << 4));
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        float sv, bv;
+        scale_and_bias(t, g, sv, bv);
+        const Pieces p = split3(g < real ? __builtin_fmaf(P::kCentre, sv, bv) : 0.f);
+        const u32x4_t o = {p.h | p.h << 16, p.h | p.m << 16, p.m | p.l << 16, 0u};
+#pragma unroll
+        for (int m = 0; m < MS; ++m) sum[m][t] = mfma<0>(F[m], o, sum[m][t]);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < MS; ++m)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) tot[m][t][v] += sum[m][t][v];
+  };
+  auto bias_stage = [&](int k, const unsigned char *at) __attribute__((always_inline)) {
+    const int g0 = k >> glog, real = (k_end >> glog) - g0;  // (groups past the share's end are another share's)
+    if (G & 1) {  // rows that start between two words: read where they are
+      bias_product(at, real, [&](int t, int g, float &sv, float &bv) __attribute__((always_inline)) {
+        const uint32_t from = first_scale[t] + g0 + (g < real ? g : 0);
+        const T s1 = s_of[GLU ? t : 0][from];
+        sv = as_f32(s1);
+        bv = as_f32(b_of[GLU ? t : 0][from]);
+        *reinterpret_cast<T *>(scales + t * 1024 + ln * 32 + g * 2) = s1;
+      });
+    } else {
+      const unsigned char *const mine = at + R::X + wave * R::W;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) *reinterpret_cast<u32x4_t *>(scales + t * 1024 + lane * 16) = *reinterpret_cast<const u32x4_t *>(mine + t * 1024 + lane * 16);
+      bias_product(at, real, [&](int t, int g, float &sv, float &bv) __attribute__((always_inline)) {
+        sv = as_f32(*reinterpret_cast<const T *>(mine + t * 1024 + ln * 32 + g * 2));
+        bv = as_f32(*reinterpret_cast<const T *>(mine + (NT + t) * 1024 + ln * 32 + g * 2));
+      });
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+
+  uint32_t xa[4], wa[2];  // this lane's pieces of a step
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    const int piece = P::SPLIT ? 4 * (h >> 1) + 2 * kb + (h & 1) : 4 * kb + h;
+    xa[h] = ln * R::XROW + ((piece ^ turned(ln)) << 4);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) wa[i] = R::X + wave * R::W + ln * 64 + (((2 * i + kb) ^ ((ln >> 2) & 3)) << 4);
+  // A stage of codes that begins k values into its window.  Program order is kept as it stands: behind every multiply a few of the
+  // scaled additions of the sub-tile before it, the reads and the unpacking that the operands it was the last to use make room
+  // for, and now and then one of the next stage's copies.
+  constexpr int SUBS = P::JS * MS * P::NS;  // sub-tiles' groups of a stage
+  auto code_stage = [&](int k, const unsigned char *at, int slot, int to) __attribute__((always_inline)) {
+    f32x16_t acc[2][NT];  // the group sums being multiplied, and those before them, which are still to be scaled
+    float pending_s[NT];
+    const unsigned char *const sc = scales + ln * 32 + (k >> glog) * 2;
+    u32x4_t F[4], q[NT][P::NQ], op[NT][4];
+    float s[NT][P::NS];
+    auto fetch = [&](int j, int m, int h) __attribute__((always_inline)) {
+      F[h] = *reinterpret_cast<const u32x4_t *>(at + (xa[h] ^ (j * 128)) + m * (32 * R::XROW));  // (the turn reaches over both steps of a row)
+    };
+    auto fetch_codes = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < P::NQ; ++i) q[t][i] = *reinterpret_cast<const u32x4_t *>(at + wa[BITS == 4 ? j : i] + t * 2048);
+    };
+    auto fetch_scales = [&](int j, float (&to)[NT][P::NS]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < P::NS; ++i) to[t][i] = P::kUnit * as_f32(*reinterpret_cast<const T *>(sc + t * 1024 + (G32 ? 2 * j + i : j >> scale_shift) * 2));
+    };
+    fetch_codes(0);
+#pragma unroll
+    for (int h = 0; h < 4; ++h) fetch(0, 0, h);
+    fetch_scales(0, s);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      P::deal(q[t]);
+#pragma unroll
+      for (int h = 0; h < 4; ++h) P::unpack(q[t], h, op[t][h]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < P::JS; ++j) {
+      float s_next[NT][P::NS];
+      if (j + 1 < P::JS) {
+        fetch_codes(j + 1);
+        fetch_scales(j + 1, s_next);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int m = 0; m < MS; ++m) {
+        const bool more = m + 1 < MS || j + 1 < P::JS;
+        const int nj = m + 1 < MS ? j : j + 1, nm = m + 1 < MS ? m + 1 : 0;
+#pragma unroll
+        for (int i = 0; i < P::NS; ++i) {
+          const int sub = (j * MS + m) * P::NS + i, cur = sub & 1;
+          const int pm = i > 0 ? m : (m > 0 ? m - 1 : MS - 1);  // the pending sub-tile
+          constexpr int SLOTS = 4 / P::NS * NT, EACH = 16 * NT / SLOTS, PLACES = SUBS * SLOTS;
+          constexpr int W_FROM = P::JS == 1 ? PLACES / 2 : PLACES / P::JS * (P::JS - 1);  // (the last step's codes have been read)
+          if (m == MS - 1 && i == 0 && j + 1 < P::JS) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) P::deal(q[t]);
+          }
+#pragma unroll
+          for (int n = 0; n < SLOTS; ++n) {
+            const int h = 4 / P::NS * i + n / NT, t = n % NT, place = sub * SLOTS + n;
+            acc[cur][t] = mfma<DT>(F[h], op[t][h], n < NT ? zero : acc[cur][t]);
+#pragma unroll
+            for (int v = n * EACH; v < (n + 1) * EACH && sub > 0; ++v)
+              tot[pm][v / 16][v % 16] = __builtin_fmaf(pending_s[v / 16], acc[cur ^ 1][v / 16][v % 16], tot[pm][v / 16][v % 16]);
+            if (t == NT - 1 && more) fetch(nj, nm, h);
+            if (m == MS - 1 && j + 1 < P::JS) P::unpack(q[t], h, op[t][h]);
+#pragma unroll
+            for (int c = R::XI * place / W_FROM; c < R::XI * (place + 1) / W_FROM && place < W_FROM; ++c) copy_x(to, c);
+#pragma unroll
+            for (int c = 2 * NT * (place - W_FROM) / (PLACES - W_FROM); c < 2 * NT * (place - W_FROM + 1) / (PLACES - W_FROM) && place >= W_FROM; ++c)
+              copy_w(slot, c);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+          for (int t = 0; t < NT; ++t) pending_s[t] = s[t][i];
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < P::NS; ++i) s[t][i] = j + 1 < P::JS ? s_next[t][i] : 0.f;
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) tot[MS - 1][t][v] = __builtin_fmaf(pending_s[t], acc[(SUBS - 1) & 1][t][v], tot[MS - 1][t][v]);
+  };
+
+  copy_weights(0);
+  advance(next_w);
+#pragma unroll
+  for (int p = 0; p < S - 1; ++p) {
+    copy_rows(p);
+    advance(next_x);
+    copy_weights(p + 1);
+    advance(next_w);
+  }
+  int slot = 0, to = S - 1, left = total;
+  auto begin = [&]() __attribute__((always_inline)) {  // this stage's copies have arrived, in every wave, and its predecessor's rows are read
+    wait_copies<2 * NT + (S - 2) * R::COPIES>();
+    block_barrier();
+  };
+  auto end = [&]() __attribute__((always_inline)) {
+    advance(next_x);
+    advance(next_w);
+    slot = slot + 1 == S ? 0 : slot + 1;
+    to = to + 1 == S ? 0 : to + 1;
+    --left;
+  };
+  for (int k = k_first; k < k_end;) {
+    const int k_window = k, k_last = k + per_window * R::KS < k_end ? k + per_window * R::KS : k_end;
+    begin();
+    copy_rows(to);
+    bias_stage(k, ring + slot * R::STAGE);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    copy_weights(slot);
+    end();
+#pragma unroll 1
+    for (; k < k_last; k += R::KS) {
+      begin();
+      code_stage(k - k_window, ring + slot * R::STAGE, slot, to);
+      end();
+    }
+  }
+  for (; KW > 1 && left > 0; --left) {  // (the last share may be a shorter one)
+    wait_copies<0>();
+    block_barrier();
+  }
+  wait_copies<0>();
+  block_barrier();
+
+  if constexpr (KW > 1) {  // the K groups' sums meet in LDS, added in group order
+    constexpr int kPiece = 64 * WN * 4;
+    float *const parts = reinterpret_cast<float *>(lds_raw) + (wave * 64 + lane) * 4;  // 16-byte pieces, lane by lane
+#pragma unroll
+    for (int g = 1; g < KW; ++g) {
+#pragma unroll
+      for (int m = 0; m < MS; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (kg == g)
+              *reinterpret_cast<float4 *>(parts + ((m * NT + t) * 4 + r) * kPiece) =
+                  make_float4(tot[m][t][4 * r], tot[m][t][4 * r + 1], tot[m][t][4 * r + 2], tot[m][t][4 * r + 3]);
+      __syncthreads();
+      if (kg == 0) {
+#pragma unroll
+        for (int m = 0; m < MS; ++m)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float4 v = *reinterpret_cast<const float4 *>(parts + ((m * NT + t) * 4 + r) * kPiece);
+              tot[m][t][4 * r] += v.x;
+              tot[m][t][4 * r + 1] += v.y;
+              tot[m][t][4 * r + 2] += v.z;
+              tot[m][t][4 * r + 3] += v.w;
+            }
+      }
+      __syncthreads();
+    }
+    if (kg != 0) return;
+  }
+
+  // ---- epilogue: a wave turns its 32 x 32 sub-tiles round in a private piece of LDS and stores 16 bytes a lane
+  constexpr int ROWB = 32 * (int)sizeof(T) + 16;
+  constexpr int PV = 16 / (int)sizeof(T);             // values per 16-byte piece
+  constexpr int CPR = 32 / PV;                        // pieces per row
+  constexpr int RPI = 64 / CPR;                       // rows one store instruction covers
+  unsigned char *const mine = lds_raw + wave * (32 * ROWB);
+  const int my_piece = lane % CPR, my_row = lane / CPR;
+  const bool vec = N % PV == 0;
+#pragma unroll
+  for (int u = 0; u < MS * (GLU ? 1 : NT); ++u) {
+    const int m = u / (GLU ? 1 : NT), t = u % (GLU ? 1 : NT), col = col0 + 32 * t;
+    const float lb = a.bias ? as_f32(static_cast<const T *>(a.bias)[col + ln < N ? col + ln : N - 1]) : 0.f;
+    auto put = [&](int r, float v, float up) __attribute__((always_inline)) {
+      if constexpr (GLU) v = v / (1.0f + __expf(-v)) * up;
+      T o = rounded<T>(v);
+      if (a.bias) o = rounded<T>(as_f32(o) + lb);
+      reinterpret_cast<T *>(mine + (8 * (r >> 2) + 4 * kb + (r & 3)) * ROWB)[ln] = o;
+    };
+    uint32_t again = 0;  // (bits: which of the sixteen sums are not finite)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float v = tot[m][t][r], up = GLU ? tot[m][NT - 1][r] : 0.f;
+      put(r, v, up);
+      again |= (not_finite(v) || (GLU && not_finite(up)) ? 1u : 0u) << r;
+    }
+#pragma unroll 1
+    for (int quad = 0; __builtin_expect(again != 0, 0); ++quad, again >>= 4) {  // rows 8 quad + 4 kb + 0 .. 3
+      uint32_t open = again & 15u;
+      const T *xs[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        int tr = 32 * m + 8 * quad + 4 * kb + i;
+        if (tr >= rows) {  // (never stored)
+          open &= ~(1u << i);
+          tr = rows - 1;
+        }
+        xs[i] = static_cast<const T *>(a.x) + (int64_t)(a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr)) * K;
+      }
+      if (!open) continue;
+      float v[GLU ? 2 : 1][4];
+#pragma unroll
+      for (int i = 0; i < (GLU ? 2 : 1); ++i) {
+        const int64_t wrow = ebase + weight_row(GLU ? i : t, ln);
+        plain_rows<BITS, 4, T>(xs, paired_order(BITS), (GLU && i ? a.w1 : a.w0) + wrow * (row_bytes / 4),
+                               static_cast<const T *>(GLU && i ? a.s1 : a.s0) + wrow * G,
+                               static_cast<const T *>(GLU && i ? a.b1 : a.b0) + wrow * G, K, K / G, open, v[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (open >> i & 1u) put(4 * quad + i, v[0][i], v[GLU ? 1 : 0][i]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int my_col = col + PV * my_piece;
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) {
+      const int row = RPI * i + my_row;
+      const int tr = 32 * m + row;
+      if (tr < rows && my_col < N) {
+        const int64_t dst = a.dst_rows ? (int64_t)a.dst_rows[row0 + tr] : row0 + tr;
+        T *const to = static_cast<T *>(a.y) + dst * N + my_col;
+        const T *const from = reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece;
+        if (vec) {
+          *reinterpret_cast<u32x4_t *>(to) = *reinterpret_cast<const u32x4_t *>(from);
+        } else {
+          for (int c = 0; c < PV && my_col + c < N; ++c) to[c] = from[c];
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+}
+
+// A block computes 32 MS token rows x 32 WN weight rows with WN KW waves (see codes_tile), tiles of up to 32 rows with half the
+// token operand.
+template <int DT, int BITS, bool G32, bool GLU, bool MID, int MS, int NT, int WN, int KW, int S>
+__global__ __launch_bounds__(64 * WN * KW, NT == 2 ? 2 : (WN * KW == 4 ? 3 : 4)) void qmm_tiles_kernel(
+    CodesArgs a, const uint32_t *__restrict__ list, int n_mtiles, int n_ntiles, int scale_shift) {
+  static_assert(!GLU || NT == 2, "a gate tile and its up tile");
+  constexpr int BM = 32 * MS;
+  constexpr int NI = 32 * WN * (GLU ? 1 : NT);  // distinct output columns per block
+  // block -> (M tile, N tile).  Ids are dealt round-robin over the 8 XCDs.  Dense: an XCD takes every eighth N tile
+  // and all M tiles of it, so its L2 holds the weights of a few N tiles and x streams through.  A tile list: whole M
+  // tiles per XCD (the blocks of one share its gathered rows).
+  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+  int e = 0, rows, nt;
+  int64_t row0;
+  if (list) {
+    const uint32_t id = (uint32_t)(j / n_ntiles) * 8u + xcd;
+    nt = j % n_ntiles;
+    if (id >= list[0]) return;
+    const uint4 rec = reinterpret_cast<const uint4 *>(list)[1 + id];
+    e = __builtin_amdgcn_readfirstlane((int)rec.x);
+    row0 = (int64_t)__builtin_amdgcn_readfirstlane((int)rec.y);
+    rows = __builtin_amdgcn_readfirstlane((int)rec.z);
+  } else {
+    nt = j / n_mtiles * 8 + xcd;
+    if (nt >= n_ntiles) return;
+    row0 = (int64_t)(j % n_mtiles) * BM;
+    rows = a.M - row0 < BM ? (int)(a.M - row0) : BM;
+  }
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  if constexpr (MS > 1) {
+    if (rows <= 32) {
+      typedef Ring<BITS, 1, NT, WN, 2> Short;
+      constexpr int S1 = (lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES) / KW - WN * Short::WINDOW) / Short::STAGE;  // as many stages as fit
+      multiply_tile<DT, BITS, G32, GLU, MID, 1, NT, WN, KW, S1>(a, e, row0, rows, nt * NI, scale_shift, lds_raw);
+      return;
+    }
+  }
+  multiply_tile<DT, BITS, G32, GLU, MID, MS, NT, WN, KW, S>(a, e, row0, rows, nt * NI, scale_shift, lds_raw);
+}
+
+size_t codes_copy_bytes(int bits, int64_t rows, int K) {
+  return paired_order(bits) ? (size_t)rows * K * 2 : 0;
+}
+size_t codes_sums_bytes(int64_t rows, int K, int group) { return (size_t)rows * padded_groups(K / group) * kSlots * 2; }
+
+hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
+                               uint16_t *sums, hipStream_t st) {
+  const int64_t n = rows * (K / 8);
+  if (n == 0) return hipSuccess;
+  const unsigned grid = (unsigned)((n + 255) / 256);
+  const int ll = group == 32 ? 2 : (group == 64 ? 3 : 4), row = padded_groups(K / group) * kSlots;
+  if (dt == 0) prepare_rows_kernel<0><<<grid, 256, 0, st>>>(static_cast<const uint16_t *>(x), n, K / 8, ll, copy, sums, row);
+  else if (dt == 1) prepare_rows_kernel<1><<<grid, 256, 0, st>>>(static_cast<const _Float16 *>(x), n, K / 8, ll, copy, sums, row);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+template <int DT, int BITS, bool G32, bool GLU, bool MID, int MS, int NT, int WN, int KW, int S>
+static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_t *list, int cap, hipStream_t st) {
+  constexpr int NI = 32 * WN * (GLU ? 1 : NT), BM = 32 * MS;
+  constexpr int bufs = lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES), sums = KW > 1 ? BM * 32 * WN * NT * 4 : WN * 32 * 80;
+  constexpr int lds = bufs > sums ? bufs : sums;
+  static_assert(lds <= 160 * 1024, "more LDS than a CU has");
+  const int n_ntiles = (a.N + NI - 1) / NI;
+  const int mtiles = list ? cap : (int)((a.M + BM - 1) / BM);
+  const int64_t grid = list ? ((int64_t)cap + 7) / 8 * 8 * n_ntiles : (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
+  if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
+  const auto kernel = &qmm_tiles_kernel<DT, BITS, G32, GLU, MID, MS, NT, WN, KW, S>;
+  if (lds > 64 * 1024)
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        e != hipSuccess)
+      return e;
+  kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, list, mtiles, n_ntiles, scale_shift);
+  return hipGetLastError();
+}
+
+// Which tile, from the number of tiles a launch of each has (256 CUs).  Measured, us of the whole call, bf16 4-bit / f16 8-bit, groups of 64
+// (M, N, K):                            (96, 4096, 4096) (200, 4096, 4096) (1000, 1024, 4096) (400, 4096, 4096) (640, 2304, 2304) (777, 4096, 4096) (2048, 4096, 4096)
+//   32 x 64, K shared by four groups       16.9 / 17.5      29.0 / 24.6       40.1 / 28.8        55.7 / 45.1       43.5 / 33.6       102 / 90          - / 211
+//   32 x 128, four groups                  21.5 / 22.3      25.8 / 27.2       31.2 / 31.9        49.7 / 52.8       35.8 / 37.0       94 / 106          - / 214
+//   32 x 128, two groups                   22.9 / 25.0      27.7 / 31.0       34.3 / 35.3        42.7 / 40.1       29.6 / 26.5       79 / 81           - / 178
+//   64 x 256, two groups, 2 tiles a wave   41 / 46          48.9 / 48.1       55.0 / 52.6        53.7 / 50.9       38.3 / 35.0       58.8 / 57.8       - / 124
+//   64 x 128, two groups                   32 / 31          - / 33.1          - / 37.1           - / 36.2          - / 25.4          - / 56.6          - / 123
+//   64 x 256, one group, 2 tiles a wave    51 / 59          - / 60.9          - / 62.0           - / 61.7          - / 39.9          - / 69.5          - / 114
+//   64 x 128, two groups, codes loaded into registers (qmm_codes.hip)
+//                                          - / -            32.4 / 32.9       37.9 / 36.0        37.1 / 34.9       26.9 / 25.4       63.4 / 60.4       - / 124
+// (32 x 64 was 18.6 / 19.2 in that kernel at 96 rows.)  bf16 takes the larger tiles (2048 rows) in qmm_large.hip.
+template <int DT, int BITS, bool G32>
+static hipError_t start_dense(const CodesArgs &a, int group, hipStream_t st) {
+  const int scale_shift = group == 128;
+  auto tiles = [&](int rows, int cols) { return (a.M + rows - 1) / rows * ((a.N + cols - 1) / cols); };
+  if (tiles(32, 64) <= (BITS == 4 ? 256 : 512)) return start_tiles<DT, BITS, G32, false, false, 1, 1, 2, 4, 2>(a, scale_shift, nullptr, 0, st);
+  if constexpr (BITS == 4)
+    if (tiles(32, 128) <= 256) return start_tiles<DT, BITS, G32, false, false, 1, 1, 4, 4, 2>(a, scale_shift, nullptr, 0, st);
+  if (tiles(64, 128) <= 256) return launch_qmm_codes_middle(a, group, BITS, DT, st);
+  if constexpr (BITS == 4) return start_tiles<DT, BITS, G32, false, false, 2, 2, 4, 2, 2>(a, scale_shift, nullptr, 0, st);
+  if (tiles(64, 256) <= 256) return start_tiles<DT, BITS, G32, false, false, 2, 1, 4, 2, 2>(a, scale_shift, nullptr, 0, st);
+  return start_tiles<DT, BITS, G32, false, false, 2, 2, 4, 1, 2>(a, scale_shift, nullptr, 0, st);
+}
+
+// The tiles of a list in one launch: 64 rows x 256 weight rows (128 gate and the matching 128 up ones), two blocks a CU.
+// Groups of 32, 512 tokens and even routing (128 experts, hidden 2048), us of gate/up / down: 107 / 57; tiles of 64 x 128 with the codes loaded into
+// registers, gate and up in one wave, 121 / 77.  One tile a wave in eight waves: 20 % slower; blocks of two waves, or of one CU each with more stages: slower.
+hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st) {
+  auto run = [&](auto b, auto g32, auto mid) {
+    constexpr int BITS = decltype(b)::value;
+    constexpr bool G32 = decltype(g32)::value, MID = decltype(mid)::value;
+    if (glu) return start_tiles<0, BITS, G32, true, MID, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
+    return start_tiles<0, BITS, G32, false, MID, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
+  };
+  const std::true_type yes{};
+  const std::false_type no{};
+  if (bits == 4) {
+    const std::integral_constant<int, 4> b{};
+    return group == 32 ? run(b, yes, no) : group == 64 ? run(b, no, yes) : run(b, no, no);
+  }
+  const std::integral_constant<int, 8> b{};
+  return group == 32 ? run(b, yes, no) : run(b, no, no);
+}
+
+hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st) {
+  if (a.M == 0) return hipSuccess;
+  auto with_group = [&](auto d, auto b) {
+    constexpr int DT = decltype(d)::value, BITS = decltype(b)::value;
+    return group == 32 ? start_dense<DT, BITS, true>(a, group, st) : start_dense<DT, BITS, false>(a, group, st);
+  };
+  auto with_bits = [&](auto d) {
+    return bits == 4 ? with_group(d, std::integral_constant<int, 4>{}) : with_group(d, std::integral_constant<int, 8>{});
+  };
+  if (dt == 0) return with_bits(std::integral_constant<int, 0>{});
+  if (dt == 1) return with_bits(std::integral_constant<int, 1>{});
+  return hipErrorInvalidValue;
+}
+
+}  // namespace mi_moe

@@ -44,7 +44,7 @@ __global__ __launch_bounds__(kDispThreads) void router_fused_kernel(
     const uint16_t *__restrict__ norm_w, float eps, uint16_t *__restrict__ xnorm,
     int T, int H, int E, int k, int mode, uint16_t *logits, uint32_t *topk_idx, uint16_t *topk_w,
     uint32_t *counters, int nbits, uint32_t *counts, uint32_t *offsets, uint32_t *perm,
-    uint32_t *inv_perm, uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, uint32_t big_thr) {
+    uint32_t *inv_perm, uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, uint32_t big_thr, ShortTiles shorts) {
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t last;
   const int tid = threadIdx.x;
@@ -93,11 +93,11 @@ __global__ __launch_bounds__(kDispThreads) void router_fused_kernel(
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   // at most 64 tokens, distinct experts per token: the mask form of the dispatch, where the host wants no tile lists (few
   // experts and more than 16 tokens in groups of 32 or 128 do)
-  if (mtiles == nullptr && T <= kMaskTokens)
+  if (mtiles == nullptr && shorts.list == nullptr && T <= kMaskTokens)
     dispatch_tokens_block(topk_idx, T, k, E, lds, counts, offsets, perm, inv_perm, src_of, work);
   else
     dispatch_block(topk_idx, (int64_t)T * k, E, nbits, k, lds, counts, offsets, perm, inv_perm, src_of,
-                   work, mtiles, cap256, big_thr);
+                   work, mtiles, cap256, big_thr, shorts);
 }
 
 // The same three stages with ONE exchange, for the smallest batches: every workgroup publishes its
@@ -173,14 +173,14 @@ hipError_t launch_router_fused(const uint16_t *x, const uint16_t *wg, const floa
                                uint16_t *topk_w, uint32_t *counters, uint32_t *counts,
                                uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
                                uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256,
-                               int big_thr, hipStream_t st) {
+                               int big_thr, ShortTiles shorts, hipStream_t st) {
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
   dim3 grid((unsigned)T, (unsigned)((E + kDispWaves - 1) / kDispWaves));
   const size_t lds = (size_t)(3 + kDispWaves) * E * sizeof(uint32_t);
   static_assert(kOneExchangeMaxTokens <= kOneExchangeRows * kDispWaves && kOneExchangeMaxTokens <= kMaskTokens,
                 "a wave selects for kOneExchangeRows tokens; the dispatch from LDS is the one of at most 64 tokens");
-  if (T <= kOneExchangeMaxTokens && mtiles == nullptr) {
+  if (T <= kOneExchangeMaxTokens && mtiles == nullptr && shorts.list == nullptr) {
     const size_t lds1 = ((size_t)4 * E + (size_t)T * k) * sizeof(uint32_t);
 #define MI_FUSED1(NV)                                                                             \
   router_fused1_kernel<NV><<<grid, kDispThreads, lds1, st>>>(                                      \
@@ -196,7 +196,7 @@ hipError_t launch_router_fused(const uint16_t *x, const uint16_t *wg, const floa
 #define MI_FUSED(NV)                                                                              \
   router_fused_kernel<NV><<<grid, kDispThreads, lds, st>>>(                                        \
       x, wg, bias, norm_w, eps, xnorm, (int)T, H, E, k, mode, logits, topk_idx, topk_w, counters, nbits, counts,      \
-      offsets, perm, inv_perm, src_of, work, mtiles, cap256, (uint32_t)big_thr)
+      offsets, perm, inv_perm, src_of, work, mtiles, cap256, (uint32_t)big_thr, shorts)
   if (E <= 64) MI_FUSED(1);
   else if (E <= 128) MI_FUSED(2);
   else if (E <= 256) MI_FUSED(4);

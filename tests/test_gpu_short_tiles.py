@@ -1,0 +1,82 @@
+"""Blocks whose segments all go through short tiles on raw codes (groups of 64, 4-bit, 65 tokens and more up to 96 rows per expert), and
+the tiles the dense products on raw codes choose from, against float64."""
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+from test_gpu_codes import BOUND, block_truth, product  # noqa: E402
+
+# hidden, intermediate, experts, k: K of 1, 3, 5 and 9 stages of 128 (windows of eight, whole and started), columns that fill no block of
+# 128 or 256, more experts than a wave has lanes
+BLOCKS = [(128, 384, 8, 2), (1152, 128, 9, 3), (640, 1152, 16, 8), (256, 256, 70, 8)]
+
+
+@pytest.mark.parametrize("hidden,inter,experts,k", BLOCKS)
+@pytest.mark.parametrize("rows", [8, 33, 64, 90])
+@pytest.mark.parametrize("zipf", [None, 1.4])
+def test_blocks_in_short_tiles(zipf, rows, hidden, inter, experts, k):
+    """On average `rows` rows an expert, at most 96: segments on both sides of 32 and 64 rows, and of several tiles.  Three roundings to
+    bfloat16 (h, y and the result), each at most 2^-8 of its values and typically 0.42 of that: 0.73 * 2^-8 together.  The built-in
+    scratch takes the same route; the order of the tokens changes no bit."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    tokens = max(rows * experts // k, 65, -(-512 // k))
+    if tokens * k > 96 * experts:
+        pytest.skip("more rows than this route takes")
+    cfg = m.MoeConfig(hidden, experts, k, inter, 4, 64, 0)
+    blk = synth.make_block(cfg, seed=rows, device="cuda", zipf_s=zipf, gen_device="cuda")
+    x = synth.make_tokens(cfg, tokens, seed=k, device="cuda")
+    out, routing = blk.forward(x, debug=True)
+    ref = block_truth(blk, x, routing)
+    err = (out.double() - ref).norm() / ref.norm()
+    assert float(err) <= 2.0 ** -8, float(err)
+    p = torch.randperm(tokens, generator=torch.Generator().manual_seed(3)).cuda()
+    assert torch.equal(blk.forward(x[p].contiguous()), out[p])
+    if blk.workspace_bytes(tokens) < 8 << 20:
+        assert torch.equal(blk.forward_static(x), out)
+
+
+def test_a_layer_around_short_tiles():
+    """The normalised rows' memory takes the group sums of h once they have been read: the residual form against its parts."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(256, 8, 2, 512, 4, 64, 0)
+    blk = synth.make_block(cfg, seed=4, device="cuda", zipf_s=1.1, gen_device="cuda")
+    x = synth.make_tokens(cfg, 300, seed=4, device="cuda")
+    w = (1.0 + 0.1 * torch.randn(256, generator=torch.Generator().manual_seed(1))).to(torch.bfloat16).cuda()
+    xn = m.ops.rms_norm(x, w, 1e-6)
+    out, routing = blk.forward_residual(x, w, 1e-6, debug=True)
+    ref = x.double() + block_truth(blk, xn, routing)
+    assert float((out.double() - ref).norm() / ref.norm()) <= 2.0 ** -8
+
+
+def test_short_tiles_with_a_gate_that_is_not_finite():
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(256, 8, 2, 384, 4, 64, 0)
+    blk = synth.make_block(cfg, seed=2, device="cuda", zipf_s=1.0, gen_device="cuda")
+    x = synth.make_tokens(cfg, 270, seed=1, device="cuda")
+    blk.gate_proj.biases[1, 5, 2] = float("inf")
+    blk.up_proj.biases[2, 7, 0] = float("-inf")
+    blk.down_proj.scales[3, 9, 1] = float("inf")
+    out, routing = blk.forward(x, debug=True)
+    ref = block_truth(blk, x, routing)
+    assert not ref.isfinite().all() and torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
+
+
+@pytest.mark.parametrize("dtype,group", [("float16", 32), ("float16", 64), ("float16", 128), ("bfloat16", 32), ("bfloat16", 64), ("bfloat16", 128)])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows,n,k", [(200, 4096, 1152), (260, 4090, 640), (1000, 4096, 1408), (1000, 4090, 2176)])
+def test_dense_tiles(rows, n, k, bits, dtype, group):
+    """Each tile of the rule that the smaller shapes of the other tests do not reach, with shares of K of an odd number of stages and
+    columns that end inside a tile."""
+    import mlx_rs_amd as m
+    dt = getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(rows + n + k)
+    q, s, b = m.ops.quantize(torch.randn((n, k), generator=gen, device="cuda") * 0.02, group, bits, dt)
+    x = torch.randn((rows, k), generator=gen, device="cuda").to(dt)
+    ref = product(x, q, s, b, group, bits)
+    y = m.ops.quantized_linear(x, q, s, b, group_size=group, bits=bits)
+    err = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= BOUND[dtype], float(err.max())
