@@ -471,28 +471,31 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     }
 }
 
-template <int DT, int BITS, bool G32>
+template <int DT, int BITS, bool G32, int KW>
 static hipError_t start_codes(const CodesArgs &a, int scale_shift, hipStream_t st) {
-  constexpr int MS = 2, WN = 4, KW = 2, NI = 32 * WN, BM = 32 * MS;
-  constexpr size_t bufs = (size_t)2 * KW * BM * kRow * 16 + WN * KW * 32 * 48, sums = (size_t)BM * 32 * WN * 4;
+  constexpr int MS = 2, WN = 4, NI = 32 * WN, BM = 32 * MS;
+  constexpr size_t bufs = (size_t)2 * KW * BM * kRow * 16 + WN * KW * 32 * 48, sums = KW > 1 ? (size_t)BM * 32 * WN * 4 : 0;
   constexpr size_t most = bufs > sums ? bufs : sums, lds = most > kLdsAtLeast ? most : kLdsAtLeast;
   static_assert(lds <= 160 * 1024, "more LDS than a CU has");
   const int n_ntiles = (a.N + NI - 1) / NI, mtiles = (int)((a.M + BM - 1) / BM);
   const int64_t grid = (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
   if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
   const auto kernel = &qmm_codes_kernel<DT, BITS, G32, MS, WN, KW>;
-  if (lds > 64 * 1024)
-    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        e != hipSuccess)
-      return e;
+  if (lds > 64 * 1024) {
+    static std::atomic<uint64_t> allowed{0};
+    if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), (int)lds, allowed); e != hipSuccess) return e;
+  }
   kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, mtiles, n_ntiles, scale_shift);
   return hipGetLastError();
 }
 
+// K is shared by two groups of waves while a CU gets one block at most.
 hipError_t launch_qmm_codes_middle(const CodesArgs &a, int group, int bits, int dt, hipStream_t st) {
+  const bool share = (a.M + 63) / 64 * ((a.N + 127) / 128) <= 256;
   auto with_group = [&](auto d, auto b) {
     constexpr int DT = decltype(d)::value, BITS = decltype(b)::value;
-    return group == 32 ? start_codes<DT, BITS, true>(a, 0, st) : start_codes<DT, BITS, false>(a, group == 128, st);
+    if (group == 32) return share ? start_codes<DT, BITS, true, 2>(a, 0, st) : start_codes<DT, BITS, true, 1>(a, 0, st);
+    return share ? start_codes<DT, BITS, false, 2>(a, group == 128, st) : start_codes<DT, BITS, false, 1>(a, group == 128, st);
   };
   auto with_bits = [&](auto d) {
     return bits == 4 ? with_group(d, std::integral_constant<int, 4>{}) : with_group(d, std::integral_constant<int, 8>{});

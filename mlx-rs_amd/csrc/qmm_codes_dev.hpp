@@ -1,5 +1,7 @@
 // What the two tiled products on raw codes (qmm_tiles.hip, qmm_codes.hip) share: the layout of the prepared rows.
 #pragma once
+#include <atomic>
+
 #include "qmm_dev.hpp"
 
 namespace mi_moe {
@@ -20,6 +22,17 @@ __device__ __forceinline__ Pieces split3(float v) {
 
 constexpr bool paired_order(int bits) { return bits == 4; }  // 8-blocks as (0,4)(1,5)(2,6)(3,7)
 constexpr int padded_groups(int G) { return (G + 15) / 16 * 16; }  // whole windows of the bias product; the groups past the row's end are zeros
+
+// A kernel's leave to use more than 64 KB of LDS, asked for once a GPU (half a microsecond a launch otherwise).  done: a bit per GPU.
+inline hipError_t allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &done) {
+  int dev = 0;
+  if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+  const uint64_t bit = dev < 64 ? uint64_t{1} << dev : 0;
+  if (bit && (done.load(std::memory_order_relaxed) & bit)) return hipSuccess;
+  const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e == hipSuccess) done.fetch_or(bit, std::memory_order_relaxed);
+  return e;
+}
 
 // The middle of the range of dense products, which qmm_codes.hip still takes (see start_dense in qmm_tiles.hip).
 hipError_t launch_qmm_codes_middle(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);

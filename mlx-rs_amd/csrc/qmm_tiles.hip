@@ -678,10 +678,10 @@ static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_
   const int64_t grid = list ? ((int64_t)cap + 7) / 8 * 8 * n_ntiles : (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
   if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
   const auto kernel = &qmm_tiles_kernel<DT, BITS, G32, GLU, MID, MS, NT, WN, KW, S>;
-  if (lds > 64 * 1024)
-    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        e != hipSuccess)
-      return e;
+  if (lds > 64 * 1024) {
+    static std::atomic<uint64_t> allowed{0};
+    if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), (int)lds, allowed); e != hipSuccess) return e;
+  }
   kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, list, mtiles, n_ntiles, scale_shift);
   return hipGetLastError();
 }
@@ -696,7 +696,8 @@ static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_
 //   64 x 256, one group, 2 tiles a wave    51 / 59          - / 60.9          - / 62.0           - / 61.7          - / 39.9          - / 69.5          - / 114
 //   64 x 128, two groups, codes loaded into registers (qmm_codes.hip)
 //                                          - / -            32.4 / 32.9       37.9 / 36.0        37.1 / 34.9       26.9 / 25.4       63.4 / 60.4       - / 124
-// (32 x 64 was 18.6 / 19.2 in that kernel at 96 rows.)  bf16 takes the larger tiles (2048 rows) in qmm_large.hip.
+// (32 x 64 was 18.6 / 19.2 in that kernel at 96 rows.  Up to 400 of its tiles, one group from 257 on, against the larger ones here: (660, 3216, 1280)
+// 27.5 / 24.6 and 28.0 / 24.0, (1000, 3072, 4096) 56.8 / 53.0 and 55.5 / 53.5, f16 4-bit 52.4 and 53.2; (900, 4096, 2048), 480 tiles, 35.6 / 31.8 and 34.4 / 31.8.)  bf16 takes the larger tiles (2048 rows) in qmm_large.hip.
 template <int DT, int BITS, bool G32>
 static hipError_t start_dense(const CodesArgs &a, int group, hipStream_t st) {
   const int scale_shift = group == 128;
@@ -704,7 +705,7 @@ static hipError_t start_dense(const CodesArgs &a, int group, hipStream_t st) {
   if (tiles(32, 64) <= (BITS == 4 ? 256 : 512)) return start_tiles<DT, BITS, G32, false, false, 1, 1, 2, 4, 2>(a, scale_shift, nullptr, 0, st);
   if constexpr (BITS == 4)
     if (tiles(32, 128) <= 256) return start_tiles<DT, BITS, G32, false, false, 1, 1, 4, 4, 2>(a, scale_shift, nullptr, 0, st);
-  if (tiles(64, 128) <= 256) return launch_qmm_codes_middle(a, group, BITS, DT, st);
+  if (tiles(64, 128) <= 400) return launch_qmm_codes_middle(a, group, BITS, DT, st);
   if constexpr (BITS == 4) return start_tiles<DT, BITS, G32, false, false, 2, 2, 4, 2, 2>(a, scale_shift, nullptr, 0, st);
   if (tiles(64, 256) <= 256) return start_tiles<DT, BITS, G32, false, false, 2, 1, 4, 2, 2>(a, scale_shift, nullptr, 0, st);
   return start_tiles<DT, BITS, G32, false, false, 2, 2, 4, 1, 2>(a, scale_shift, nullptr, 0, st);
