@@ -8,6 +8,8 @@ patterns (torch has no arithmetic on uint32).
 """
 import ctypes as C
 import functools
+import importlib.util
+import os
 
 import torch
 
@@ -185,6 +187,21 @@ def _matmul_workspace_bytes(M, K, bits):
     return need.value
 
 
+@functools.lru_cache(maxsize=1)
+def _linear_call():
+    """csrc/linear_call.cpp bound to the library: the call around a linear layer without the interpreter."""
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_linear_call.so")
+    if not os.path.exists(path):
+        raise capi.MoeError(f"{path} is missing: build it with `make -C {os.path.dirname(path)}/csrc` (or __graft_entry__.build())")
+    spec = importlib.util.spec_from_file_location("_linear_call", path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    lib = load_library()
+    mod.bind(*(C.cast(getattr(lib, n), C.c_void_p).value for n in
+               ("mi_moe_quantized_linear_typed", "mi_moe_quantized_matmul_typed", "mi_moe_quantized_matmul_workspace_size")))
+    return mod.quantized_linear
+
+
 def quantized_matmul(x, w, scales, biases, transpose=False, group_size=64, bits=4):
     """ops::quantized_matmul (mlx-rs/src/ops/quantization.rs:91-122), same argument order and defaults
     (``transpose`` defaults to False as there; QuantizedLinear passes True, mlx-rs/src/nn/quantized.rs:363-386).
@@ -199,6 +216,11 @@ def quantized_linear(x, w, scales, biases, linear_bias=None, transpose=True, gro
     """QuantizedLinear::forward (mlx-rs/src/nn/quantized.rs:363-386): quantized_matmul with
     transpose = True, then ``+ linear_bias`` ([N], x's type) when the layer has one; each of the two
     ops rounds to x's type, as the reference's."""
+    y = _linear_call()(x, w, scales, biases, linear_bias, transpose, group_size, bits)
+    if y is not None:  # (else: operands that are not plain ones, or are refused)
+        if type(y) is int:
+            check(y)
+        return y
     lib = load_library()
     dt = _float_dtype(x, "x")
     _need(w, torch.int32, "w")
