@@ -189,9 +189,9 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws) {
   f.perm = cv.take<uint32_t>((size_t)P);
   f.inv_perm = cv.take<uint32_t>((size_t)P);
   f.src_of = cv.take<uint32_t>((size_t)P);
-  f.disp_scratch = cv.take<char>(dispatch_workspace_bytes(c.n_experts, P));
   f.hh = cv.take<uint16_t>((size_t)P * c.intermediate);
   f.y = cv.take<uint16_t>((size_t)P * c.hidden);
+  f.disp_scratch = f.y;  // (per-block histograms, read before the first product: at most 4 E bytes for 1024 pairs, and one block's)
   f.xperm = cv.take<uint16_t>(f.tiled && c.bits == 4 ? (size_t)T * c.hidden : 0);
   f.xnorm = cv.take<uint16_t>((size_t)T * c.hidden);  // rms_norm(x) of the residual variant
   RowsArgs up{}, down{};  // (the extents only)

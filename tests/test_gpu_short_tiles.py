@@ -80,3 +80,14 @@ def test_dense_tiles(rows, n, k, bits, dtype, group):
     y = m.ops.quantized_linear(x, q, s, b, group_size=group, bits=bits)
     err = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
     assert float(err.max()) <= BOUND[dtype], float(err.max())
+
+
+@pytest.mark.parametrize("pairs,experts", [(2047, 8), (2048, 128), (2049, 8), (2049, 512), (4095, 70)])
+def test_dispatch_around_one_block(pairs, experts):
+    """The last pair count of the one-block kernel and the first of the two-launch form."""
+    import mlx_rs_amd as m
+    e = torch.randint(0, experts, (pairs,), generator=torch.Generator().manual_seed(pairs), dtype=torch.int32)
+    counts, offsets, perm, inv = (t.cpu().long() for t in m.ops.dispatch(e.cuda(), experts))
+    want = torch.argsort(e.long(), stable=True)
+    assert torch.equal(counts, torch.bincount(e.long(), minlength=experts)) and torch.equal(offsets[1:], counts.cumsum(0))
+    assert torch.equal(perm, want) and torch.equal(inv[perm], torch.arange(pairs))
