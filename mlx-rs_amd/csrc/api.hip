@@ -541,6 +541,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   ca.w1 = h->w.up.w; ca.s1 = h->w.up.scales; ca.b1 = h->w.up.biases;
   ca.y = f.hh;
   ca.y_paired = copied;
+  ca.y_sums = f.raw_hsums;
   ca.N = c.intermediate; ca.K = c.hidden;
   cd.x = f.hh;
   cd.x_rows = P;
@@ -556,10 +557,6 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     return launch_qmm_codes_tiles(ca, f.raw_tiles, f.raw_cap, c.group_size, c.bits, true, s);
   };
   auto tiles_down = [&](hipStream_t s) -> hipError_t {
-    // (the sums of all rows of h: those of other segments, which another stream may still be writing, are not read)
-    if (hipError_t e = launch_prepare_rows(f.hh, P, c.intermediate, c.group_size, MI_MOE_DTYPE_BF16, nullptr, f.raw_hsums, s);
-        e != hipSuccess)
-      return e;
     return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.group_size, c.bits, false, s);
   };
   if (mid) {

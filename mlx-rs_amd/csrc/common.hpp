@@ -358,6 +358,7 @@ struct CodesArgs {
   const void *bias;  // [N] added after the rounding of the product, with a rounding of its own; or nullptr
   void *y;
   bool y_paired;
+  uint16_t *y_sums;  // gate/up tiles: where the group sums of the output rows go as well, in the form of launch_prepare_rows; or nullptr
   int N, K;
   int64_t M;  // rows (dense launches)
 };

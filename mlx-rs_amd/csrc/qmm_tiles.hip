@@ -542,6 +542,10 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
   unsigned char *const mine = lds_raw + wave * (32 * ROWB);
   const int my_piece = lane % CPR, my_row = lane / CPR;
   const bool vec = N % PV == 0;
+  // The gate/up tiles also sum their rows over the quantisation groups, which the down product's bias term wants (columns in whole blocks of 128:
+  // 32 of them here, the rest of a group in the waves beside).  A kernel over the finished rows took 5 us.
+  const bool sums_too = GLU && a.y_sums != nullptr;
+  float *const parts_of_sums = reinterpret_cast<float *>(lds_raw + WN * (32 * ROWB));  // [wave][row]
 #pragma unroll
   for (int u = 0; u < MS * (GLU ? 1 : NT); ++u) {
     const int m = u / (GLU ? 1 : NT), t = u % (GLU ? 1 : NT), col = col0 + 32 * t;
@@ -603,10 +607,38 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
           for (int c = 0; c < PV && my_col + c < N; ++c) to[c] = from[c];
         }
       }
+      if constexpr (GLU) {
+        if (sums_too) {
+          const u32x4_t w = *reinterpret_cast<const u32x4_t *>(reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece);
+          float sum = ((bf16lo_to_f32(w[0]) + bf16hi_to_f32(w[0])) + (bf16lo_to_f32(w[1]) + bf16hi_to_f32(w[1]))) +
+                      ((bf16lo_to_f32(w[2]) + bf16hi_to_f32(w[2])) + (bf16lo_to_f32(w[3]) + bf16hi_to_f32(w[3])));
+          sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
+          sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
+          if (my_piece == 0) parts_of_sums[wave * (32 * MS) + tr] = sum;
+        }
+      }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  if constexpr (GLU) {
+    static_assert(KW == 1 && DT == 0 && WN == 4, "every wave comes here; four waves cover a group of 128");
+    if (!sums_too) return;
+    __syncthreads();
+    const int first = n0 >> glog, groups = N >> glog, here = 128 >> glog, waves = 1 << (glog - 5);  // (the output's groups are as long as the input's)
+    const int end = first + here >= groups ? padded_groups(groups) : first + here;  // the last block writes the zeros behind
+    for (int i = threadIdx.x; i < rows * (end - first); i += 64 * WN) {
+      const int row = i % rows, g = i / rows;
+      uint4 v = make_uint4(0, 0, 0, 0);
+      if (first + g < groups) {
+        float sum = 0.f;
+        for (int w = 0; w < waves; ++w) sum += parts_of_sums[(g * waves + w) * (32 * MS) + row];
+        const Pieces p = split3(sum);
+        v = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, 0u);
+      }
+      reinterpret_cast<uint4 *>(a.y_sums)[(row0 + row) * padded_groups(groups) + first + g] = v;
+    }
   }
 }
 
@@ -670,7 +702,7 @@ hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, in
 template <int DT, int BITS, bool G32, bool GLU, bool MID, int MS, int NT, int WN, int KW, int S>
 static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_t *list, int cap, hipStream_t st) {
   constexpr int NI = 32 * WN * (GLU ? 1 : NT), BM = 32 * MS;
-  constexpr int bufs = lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES), sums = KW > 1 ? BM * 32 * WN * NT * 4 : WN * 32 * 80;
+  constexpr int bufs = lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES), sums = KW > 1 ? BM * 32 * WN * NT * 4 : WN * (32 * 80 + BM * 4);
   constexpr int lds = bufs > sums ? bufs : sums;
   static_assert(lds <= 160 * 1024, "more LDS than a CU has");
   const int n_ntiles = (a.N + NI - 1) / NI;
