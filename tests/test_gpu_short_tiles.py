@@ -82,6 +82,23 @@ def test_dense_tiles(rows, n, k, bits, dtype, group):
     assert float(err.max()) <= BOUND[dtype], float(err.max())
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows,n,k", [(40, 2000, 2432), (70, 1532, 1152), (40, 1040, 7680), (40, 1040, 7808), (40, 1040, 8064), (150, 3840, 3200), (33, 1030, 384)])
+def test_scales_of_shares_that_begin_between_two_words(rows, n, k, bits, dtype):
+    """Groups of 128 and K shared by four groups of waves in shares of 5, 3, 15 (a window and its first place), 16, 16, 7 and 1 groups; rows of an
+    odd number of scales (19, 9, 61, 63, 25, 3).  One group with another's scale or bias is far outside each row's bound."""
+    import mlx_rs_amd as m
+    dt = getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(rows + n + k)
+    q, s, b = m.ops.quantize(torch.randn((n, k), generator=gen, device="cuda") * 0.02, 128, bits, dt)
+    x = torch.randn((rows, k), generator=gen, device="cuda").to(dt)
+    ref = product(x, q, s, b, 128, bits)
+    y = m.ops.quantized_linear(x, q, s, b, group_size=128, bits=bits)
+    err = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= BOUND[dtype], float(err.max())
+
+
 @pytest.mark.parametrize("pairs,experts", [(2047, 8), (2048, 128), (2049, 8), (2049, 512), (4095, 70)])
 def test_dispatch_around_one_block(pairs, experts):
     """The last pair count of the one-block kernel and the first of the two-launch form."""
