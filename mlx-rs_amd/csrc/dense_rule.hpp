@@ -1,4 +1,4 @@
-// How a product on raw codes shares K among the waves of a block: arithmetic alone, for host and device code.
+// Which tile a dense product on raw codes takes, and how it shares K among the waves of a block: arithmetic alone, for host and device code.
 #pragma once
 #include <cstdint>
 
@@ -8,6 +8,51 @@ namespace mi_moe {
 constexpr int share_of_k(int K, int n, bool pairs) {
   const int even = (K / 128 + n - 1) / n;
   return (pairs ? (even + 1) & ~1 : even) * 128;
+}
+
+// Tiles (rows x cols) of the fullest XCD: it takes every eighth column of tiles, with all its rows, for 32 CUs.  A launch is as long as that one's:
+// 12 x 18 tiles are fewer than 256, but two XCDs get 36 of them and run two rounds where a CU holds one block.
+constexpr int64_t tiles_of_an_xcd(int64_t M, int N, int rows, int cols) {
+  return (int64_t)(((N + cols - 1) / cols + 7) / 8) * ((M + rows - 1) / rows);
+}
+
+// The tiles (token rows x weight rows) and the groups of waves that share K.
+enum class DenseTile {
+  k32x64,            // four groups (qmm_tiles.hip): one block a CU with 4-bit codes, two with 8-bit ones
+  k32x128,           // four groups, 4-bit: one block
+  k64x256,           // two groups, one block (4-bit); one group, two blocks (8-bit)
+  kRegisters64x128,  // codes loaded into registers (qmm_codes.hip), one group: several blocks
+  kRegisters64x128Shared,  // two groups: one block
+};
+
+// Measured, us of the kernels from graph replays, with the tiles of the fullest XCD (x of 64 x 128 unless another is named):
+//   4-bit, K shared by four in 32 x 128 against registers: f16, 567 x 1280 x 3840, 36 of 32 x 128, 42.9 / 32.8; bf16 367 x 2304 x 2944, 36,
+//     38.9 / 28.7; bf16 414 x 1760 x 2944, 26, 24.1 / 28.5; f16 483 x 1664 x 3456 in groups of 32, 32, 31.0 / 36.6.  32 x 64 / 32 x 128: bf16
+//     221 x 2080 x 1408, 35 of 32 x 64, 20.1 / 16.2.
+//   4-bit, 64 x 256 against registers, one round of 64 x 256 (x = 52 to 64): K = 1024 25.0 / 21.9 (f16), 1408 29.4 / 27.9, 2560 42.1 / 40.0, 3072
+//     43.7 / 45.6 and 46.0 / 46.2, 4096 55.1 / 58.9 and 51.0 / 54.5; in groups of 32 2560 48.8 / 46.5, 3584 58.5 / 59.5, 4096 66.0 / 68.0;
+//     two rounds: 1535 x 3504 x 2688 (x = 96) 75.6 / 60.8, 1874 x 2576 x 4096 (90) 104 / 80.8, 1580 x 3968 x 3584 in groups of 128 (100) 83.7 / 87.1,
+//     1692 x 3504 x 4096 in groups of 32 (108) 119 / 126; more, in which registers' blocks, several on a CU, fill the gaps: 2345 x 3952 x 3584
+//     (148, three) 138 / 125, 3423 x 3264 x 3968 in groups of 128 (216, four) 189 / 160, 3784 x 3520 x 4096 (240, four) 195 / 206.
+//   8-bit, 32 x 64 against registers by its own tiles of an XCD: 50 20.5 / 23.4, 55 22.7 / 25.4, 64 27.4 / 33.1; 66 20.4 / 17.8, 70 23.4 / 19.6, 80
+//     21.9 / 18.0.
+//   8-bit, 64 x 256 against registers, with the most blocks of it on a CU, two at a time: 3872 x 1888 x 2688 (x = 122, two) 77.9 / 86.2, 3336 x 1424 x 1024
+//     (106, two) 32.7 / 36.3, 2706 x 3552 x 2560 in groups of 128 (172, three) 94.5 / 107, 3126 x 3456 x 2176 (196, four) 107 / 112, 2738 x 1488 x 3712
+//     (86, two) 84.2 / 77.0, 2544 x 2272 x 4096 (120, three) 142 / 111; in groups of 32 3146 x 1712 x 3840 (100, two) 114 / 127, 3683 x 4000 x 3328
+//     (232, four) 208 / 225, 1993 x 2928 x 2944 (96, two) 98.3 / 84.3, 3498 x 4080 x 1024 (220, four) 82.0 / 74.4.
+//   Registers, K shared by two / by one: f16 8-bit 743 x 2672 x 3072 (x = 36) 52.2 / 38.8; bf16 4-bit 998 x 1168 x 3840 (32) 36.2 / 38.7.
+constexpr DenseTile dense_tile(int64_t M, int N, int K, int bits, int group) {
+  const int64_t x = tiles_of_an_xcd(M, N, 64, 128), wide = tiles_of_an_xcd(M, N, 64, 256);
+  if (tiles_of_an_xcd(M, N, 32, 64) <= (bits == 4 ? 32 : 64)) return DenseTile::k32x64;
+  if (bits == 4) {
+    if (tiles_of_an_xcd(M, N, 32, 128) <= 32) return DenseTile::k32x128;
+    const int64_t rounds = (wide + 31) / 32;
+    if (K >= (group == 32 || rounds > 2 ? 3584 : rounds == 2 ? 3328 : 3072) && x >= (rounds <= 2 ? 50 : 60) * rounds) return DenseTile::k64x256;
+  } else {
+    const int64_t blocks = (wide + 31) / 32;
+    if (blocks >= 2 && x >= 49 * blocks && (group != 32 || K >= 1536)) return DenseTile::k64x256;
+  }
+  return x <= 32 ? DenseTile::kRegisters64x128Shared : DenseTile::kRegisters64x128;
 }
 
 }  // namespace mi_moe

@@ -1,5 +1,5 @@
-// The middle of the range of dense products on raw codes (which: start_dense in qmm_tiles.hip, whose contract, arithmetic and prepared
-// rows these are, with c = 8 or 128): tiles of 64 x 128 whose waves load their codes straight into the registers that unpack them.
+// The middle of the range of dense products on raw codes (which: dense_rule.hpp; contract, arithmetic and prepared rows: qmm_tiles.hip, with
+// c = 8 or 128): tiles of 64 x 128 whose waves load their codes straight into the registers that unpack them.
 #include <type_traits>
 
 #include "qmm_codes_dev.hpp"
@@ -489,9 +489,7 @@ static hipError_t start_codes(const CodesArgs &a, int scale_shift, hipStream_t s
   return hipGetLastError();
 }
 
-// K is shared by two groups of waves while a CU gets one block at most.
-hipError_t launch_qmm_codes_middle(const CodesArgs &a, int group, int bits, int dt, hipStream_t st) {
-  const bool share = (a.M + 63) / 64 * ((a.N + 127) / 128) <= 256;
+hipError_t launch_qmm_codes_middle(const CodesArgs &a, bool share, int group, int bits, int dt, hipStream_t st) {
   auto with_group = [&](auto d, auto b) {
     constexpr int DT = decltype(d)::value, BITS = decltype(b)::value;
     if (group == 32) return share ? start_codes<DT, BITS, true, 2>(a, 0, st) : start_codes<DT, BITS, true, 1>(a, 0, st);

@@ -34,7 +34,7 @@ inline hipError_t allow_lds(const void *kernel, int bytes, std::atomic<uint64_t>
   return e;
 }
 
-// The middle of the range of dense products, which qmm_codes.hip still takes (see start_dense in qmm_tiles.hip).
-hipError_t launch_qmm_codes_middle(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
+// The dense products that qmm_codes.hip takes (see dense_rule.hpp); share: K is shared by two groups of waves.
+hipError_t launch_qmm_codes_middle(const CodesArgs &a, bool share, int group, int bits, int dt, hipStream_t st);
 
 }  // namespace mi_moe

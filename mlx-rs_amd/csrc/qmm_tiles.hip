@@ -734,8 +734,8 @@ static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_
   return hipGetLastError();
 }
 
-// Which tile, from the number of tiles a launch of each has (256 CUs).  Measured, us of the whole call, bf16 4-bit / f16 8-bit, groups of 64
-// (M, N, K):                            (96, 4096, 4096) (200, 4096, 4096) (1000, 1024, 4096) (400, 4096, 4096) (640, 2304, 2304) (777, 4096, 4096) (2048, 4096, 4096)
+// Which tile: dense_tile (dense_rule.hpp).  Before that rule, us of the whole call, bf16 4-bit / f16 8-bit, groups of 64 (M, N, K):
+//                                       (96, 4096, 4096) (200, 4096, 4096) (1000, 1024, 4096) (400, 4096, 4096) (640, 2304, 2304) (777, 4096, 4096) (2048, 4096, 4096)
 //   32 x 64, K shared by four groups       16.9 / 17.5      29.0 / 24.6       40.1 / 28.8        55.7 / 45.1       43.5 / 33.6       102 / 90          - / 211
 //   32 x 128, four groups                  21.5 / 22.3      25.8 / 27.2       31.2 / 31.9        49.7 / 52.8       35.8 / 37.0       94 / 106          - / 214
 //   32 x 128, two groups                   22.9 / 25.0      27.7 / 31.0       34.3 / 35.3        42.7 / 40.1       29.6 / 26.5       79 / 81           - / 178
@@ -744,19 +744,21 @@ static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_
 //   64 x 256, one group, 2 tiles a wave    51 / 59          - / 60.9          - / 62.0           - / 61.7          - / 39.9          - / 69.5          - / 114
 //   64 x 128, two groups, codes loaded into registers (qmm_codes.hip)
 //                                          - / -            32.4 / 32.9       37.9 / 36.0        37.1 / 34.9       26.9 / 25.4       63.4 / 60.4       - / 124
-// (32 x 64 was 18.6 / 19.2 in that kernel at 96 rows.  Up to 400 of its tiles, one group from 257 on, against the larger ones here: (660, 3216, 1280)
-// 27.5 / 24.6 and 28.0 / 24.0, (1000, 3072, 4096) 56.8 / 53.0 and 55.5 / 53.5, f16 4-bit 52.4 and 53.2; (900, 4096, 2048), 480 tiles, 35.6 / 31.8 and 34.4 / 31.8.)  bf16 takes the larger tiles (2048 rows) in qmm_large.hip.
+// (8-bit, 64 x 128 and two groups here against registers, 777 x 4096 x 4096 and 900 x 4096 x 2048, either type, any group: 0.3 to 5 us slower.)
+// bf16 takes the larger tiles (2048 rows) in qmm_large.hip.
 template <int DT, int BITS, bool G32>
 static hipError_t start_dense(const CodesArgs &a, int group, hipStream_t st) {
   const int scale_shift = group == 128;
-  auto tiles = [&](int rows, int cols) { return (a.M + rows - 1) / rows * ((a.N + cols - 1) / cols); };
-  if (tiles(32, 64) <= (BITS == 4 ? 256 : 512)) return start_tiles<DT, BITS, G32, false, false, 1, 1, 2, 4, 2>(a, scale_shift, nullptr, 0, st);
-  if constexpr (BITS == 4)
-    if (tiles(32, 128) <= 256) return start_tiles<DT, BITS, G32, false, false, 1, 1, 4, 4, 2>(a, scale_shift, nullptr, 0, st);
-  if (tiles(64, 128) <= 400) return launch_qmm_codes_middle(a, group, BITS, DT, st);
-  if constexpr (BITS == 4) return start_tiles<DT, BITS, G32, false, false, 2, 2, 4, 2, 2>(a, scale_shift, nullptr, 0, st);
-  if (tiles(64, 256) <= 256) return start_tiles<DT, BITS, G32, false, false, 2, 1, 4, 2, 2>(a, scale_shift, nullptr, 0, st);
-  return start_tiles<DT, BITS, G32, false, false, 2, 2, 4, 1, 2>(a, scale_shift, nullptr, 0, st);
+  switch (dense_tile(a.M, a.N, a.K, BITS, group)) {
+    case DenseTile::k32x64: return start_tiles<DT, BITS, G32, false, false, 1, 1, 2, 4, 2>(a, scale_shift, nullptr, 0, st);
+    case DenseTile::k32x128:
+      if constexpr (BITS == 4) return start_tiles<DT, BITS, G32, false, false, 1, 1, 4, 4, 2>(a, scale_shift, nullptr, 0, st);
+      break;
+    case DenseTile::k64x256: return start_tiles<DT, BITS, G32, false, false, 2, 2, 4, BITS == 4 ? 2 : 1, 2>(a, scale_shift, nullptr, 0, st);
+    case DenseTile::kRegisters64x128: return launch_qmm_codes_middle(a, false, group, BITS, DT, st);
+    case DenseTile::kRegisters64x128Shared: return launch_qmm_codes_middle(a, true, group, BITS, DT, st);
+  }
+  return hipErrorInvalidValue;
 }
 
 // The tiles of a list in one launch: 64 rows x 256 weight rows (128 gate and the matching 128 up ones), two blocks a CU.

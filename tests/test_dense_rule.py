@@ -12,11 +12,14 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 def rule(tmp_path_factory):
     d = tmp_path_factory.mktemp("rule")
     (d / "rule.cpp").write_text('#include "dense_rule.hpp"\n'
-                                'extern "C" int share(int K, int n, int pairs) { return mi_moe::share_of_k(K, n, pairs != 0); }\n')
+                                'extern "C" int share(int K, int n, int pairs) { return mi_moe::share_of_k(K, n, pairs != 0); }\n'
+                                'extern "C" int tile(long M, int N, int K, int bits, int group) { return (int)mi_moe::dense_tile(M, N, K, bits, group); }\n')
     so = d / "rule.so"
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", os.path.join(ROOT, "mlx-rs_amd", "csrc"),
                     str(d / "rule.cpp"), "-o", str(so)], check=True)
-    return C.CDLL(str(so))
+    lib = C.CDLL(str(so))
+    lib.tile.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int, C.c_int]
+    return lib
 
 
 @pytest.mark.parametrize("n", [1, 2, 4])
@@ -27,3 +30,21 @@ def test_shares_of_k_are_as_even_as_whole_128s_can_be(rule, n):
         assert share == 128 * -(-units // n)
         assert pairs % 256 == 0 and share <= pairs <= share + 128
     assert rule.share(2432, 4, 0) == 640
+
+
+SMALL, COLUMNS, WIDE, REGISTERS, REGISTERS_SHARED = range(5)  # DenseTile
+
+
+@pytest.mark.parametrize("shape,bits,group,want", [
+    # rows, columns, K: launches of at most 256 tiles whose fullest XCD gets more than its 32 CUs hold at once
+    ((567, 1280, 3840), 4, 64, REGISTERS_SHARED), ((367, 2304, 2944), 4, 64, REGISTERS_SHARED), ((221, 2080, 1408), 4, 32, COLUMNS),
+    ((546, 1808, 4096), 8, 32, REGISTERS_SHARED), ((293, 3184, 1408), 8, 32, REGISTERS_SHARED), ((743, 2672, 3072), 8, 64, REGISTERS),
+    # and those that fit
+    ((77, 1680, 2432), 4, 32, SMALL), ((414, 1760, 2944), 4, 64, COLUMNS), ((661, 1488, 2432), 8, 64, SMALL), ((998, 1168, 3840), 4, 64, REGISTERS_SHARED),
+    # 64 x 256: rows of few values, rounds that are not full
+    ((991, 3392, 1024), 4, 64, REGISTERS), ((961, 3664, 4096), 4, 64, WIDE), ((1874, 2576, 4096), 4, 64, REGISTERS), ((3784, 3520, 4096), 4, 64, WIDE),
+    ((2544, 2272, 4096), 8, 64, REGISTERS), ((3872, 1888, 2688), 8, 64, WIDE), ((3281, 2896, 2432), 8, 32, REGISTERS), ((777, 4096, 4096), 8, 64, REGISTERS),
+])
+def test_the_tile_follows_the_fullest_xcd(rule, shape, bits, group, want):
+    """Each of these was measured with the other tiles too (dense_rule.hpp)."""
+    assert rule.tile(*shape, bits, group) == want
