@@ -19,9 +19,10 @@ constexpr int64_t tiles_of_an_xcd(int64_t M, int N, int rows, int cols) {
 // The tiles (token rows x weight rows) and the groups of waves that share K.
 enum class DenseTile {
   k32x64,            // four groups (qmm_tiles.hip): one block a CU with 4-bit codes, two with 8-bit ones
+  kRegisters32x64,   // four groups, codes loaded into registers (qmm_codes.hip), bf16 and 8-bit codes in groups of 32: one block
   k32x128,           // four groups, 4-bit: one block
   k64x256,           // two groups, one block (4-bit); one group, two blocks (8-bit)
-  kRegisters64x128,  // codes loaded into registers (qmm_codes.hip), one group: several blocks
+  kRegisters64x128,  // codes in registers, one group: several blocks
   kRegisters64x128Shared,  // two groups: one block
 };
 
@@ -40,10 +41,15 @@ enum class DenseTile {
 //     (106, two) 32.7 / 36.3, 2706 x 3552 x 2560 in groups of 128 (172, three) 94.5 / 107, 3126 x 3456 x 2176 (196, four) 107 / 112, 2738 x 1488 x 3712
 //     (86, two) 84.2 / 77.0, 2544 x 2272 x 4096 (120, three) 142 / 111; in groups of 32 3146 x 1712 x 3840 (100, two) 114 / 127, 3683 x 4000 x 3328
 //     (232, four) 208 / 225, 1993 x 2928 x 2944 (96, two) 98.3 / 84.3, 3498 x 4080 x 1024 (220, four) 82.0 / 74.4.
+//   8-bit, groups of 32, bf16, 32 x 64 against registers: K = 1024 10.8 / 11.7, 1152 12.2 / 12.3, 1408 12.8 / 12.7, 2560 16.7 / 16.0, 3328 20.3 / 19.0, 4096 22.8 / 21.3
+//     (stages of 64 K values hold two groups, each with a scaling of its sums and a conversion to float of every code; registers take 128 K
+//     values between two barriers); f16, whose codes need no conversion, 12.0 / 12.4 at K = 1408, 19.7 / 19.6 at 3712.
 //   Registers, K shared by two / by one: f16 8-bit 743 x 2672 x 3072 (x = 36) 52.2 / 38.8; bf16 4-bit 998 x 1168 x 3840 (32) 36.2 / 38.7.
-constexpr DenseTile dense_tile(int64_t M, int N, int K, int bits, int group) {
+constexpr DenseTile dense_tile(int64_t M, int N, int K, int bits, int group, bool bf16) {
   const int64_t x = tiles_of_an_xcd(M, N, 64, 128), wide = tiles_of_an_xcd(M, N, 64, 256);
-  if (tiles_of_an_xcd(M, N, 32, 64) <= (bits == 4 ? 32 : 64)) return DenseTile::k32x64;
+  const int64_t least = tiles_of_an_xcd(M, N, 32, 64);
+  if (bf16 && bits == 8 && group == 32 && K >= 1280 && least <= 32) return DenseTile::kRegisters32x64;
+  if (least <= (bits == 4 ? 32 : 64)) return DenseTile::k32x64;
   if (bits == 4) {
     if (tiles_of_an_xcd(M, N, 32, 128) <= 32) return DenseTile::k32x128;
     const int64_t rounds = (wide + 31) / 32;

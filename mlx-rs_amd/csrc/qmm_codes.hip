@@ -1,5 +1,5 @@
 // The middle of the range of dense products on raw codes (which: dense_rule.hpp; contract, arithmetic and prepared rows: qmm_tiles.hip, with
-// c = 8 or 128): tiles of 64 x 128 whose waves load their codes straight into the registers that unpack them.
+// c = 8 or 128): tiles of 64 x 128, and of 32 x 64 for bf16 and 8-bit codes in groups of 32, whose waves load their codes straight into the registers that unpack them.
 #include <type_traits>
 
 #include "qmm_codes_dev.hpp"
@@ -471,9 +471,9 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     }
 }
 
-template <int DT, int BITS, bool G32, int KW>
+template <int DT, int BITS, bool G32, int MS, int WN, int KW>
 static hipError_t start_codes(const CodesArgs &a, int scale_shift, hipStream_t st) {
-  constexpr int MS = 2, WN = 4, NI = 32 * WN, BM = 32 * MS;
+  constexpr int NI = 32 * WN, BM = 32 * MS;
   constexpr size_t bufs = (size_t)2 * KW * BM * kRow * 16 + WN * KW * 32 * 48, sums = KW > 1 ? (size_t)BM * 32 * WN * 4 : 0;
   constexpr size_t most = bufs > sums ? bufs : sums, lds = most > kLdsAtLeast ? most : kLdsAtLeast;
   static_assert(lds <= 160 * 1024, "more LDS than a CU has");
@@ -489,11 +489,13 @@ static hipError_t start_codes(const CodesArgs &a, int scale_shift, hipStream_t s
   return hipGetLastError();
 }
 
+hipError_t launch_qmm_codes_small(const CodesArgs &a, hipStream_t st) { return start_codes<0, 8, true, 1, 2, 4>(a, 0, st); }
+
 hipError_t launch_qmm_codes_middle(const CodesArgs &a, bool share, int group, int bits, int dt, hipStream_t st) {
   auto with_group = [&](auto d, auto b) {
     constexpr int DT = decltype(d)::value, BITS = decltype(b)::value;
-    if (group == 32) return share ? start_codes<DT, BITS, true, 2>(a, 0, st) : start_codes<DT, BITS, true, 1>(a, 0, st);
-    return share ? start_codes<DT, BITS, false, 2>(a, group == 128, st) : start_codes<DT, BITS, false, 1>(a, group == 128, st);
+    if (group == 32) return share ? start_codes<DT, BITS, true, 2, 4, 2>(a, 0, st) : start_codes<DT, BITS, true, 2, 4, 1>(a, 0, st);
+    return share ? start_codes<DT, BITS, false, 2, 4, 2>(a, group == 128, st) : start_codes<DT, BITS, false, 2, 4, 1>(a, group == 128, st);
   };
   auto with_bits = [&](auto d) {
     return bits == 4 ? with_group(d, std::integral_constant<int, 4>{}) : with_group(d, std::integral_constant<int, 8>{});

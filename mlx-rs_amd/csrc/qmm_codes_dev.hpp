@@ -34,7 +34,9 @@ inline hipError_t allow_lds(const void *kernel, int bytes, std::atomic<uint64_t>
   return e;
 }
 
-// The dense products that qmm_codes.hip takes (see dense_rule.hpp); share: K is shared by two groups of waves.
+// The dense products that qmm_codes.hip takes (see dense_rule.hpp); share: K is shared by two groups of waves.  small: bf16, 8-bit
+// codes in groups of 32.
 hipError_t launch_qmm_codes_middle(const CodesArgs &a, bool share, int group, int bits, int dt, hipStream_t st);
+hipError_t launch_qmm_codes_small(const CodesArgs &a, hipStream_t st);
 
 }  // namespace mi_moe

@@ -749,8 +749,9 @@ static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_
 template <int DT, int BITS, bool G32>
 static hipError_t start_dense(const CodesArgs &a, int group, hipStream_t st) {
   const int scale_shift = group == 128;
-  switch (dense_tile(a.M, a.N, a.K, BITS, group)) {
+  switch (dense_tile(a.M, a.N, a.K, BITS, group, DT == 0)) {
     case DenseTile::k32x64: return start_tiles<DT, BITS, G32, false, false, 1, 1, 2, 4, 2>(a, scale_shift, nullptr, 0, st);
+    case DenseTile::kRegisters32x64: return launch_qmm_codes_small(a, st);
     case DenseTile::k32x128:
       if constexpr (BITS == 4) return start_tiles<DT, BITS, G32, false, false, 1, 1, 4, 4, 2>(a, scale_shift, nullptr, 0, st);
       break;

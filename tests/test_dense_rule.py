@@ -13,12 +13,12 @@ def rule(tmp_path_factory):
     d = tmp_path_factory.mktemp("rule")
     (d / "rule.cpp").write_text('#include "dense_rule.hpp"\n'
                                 'extern "C" int share(int K, int n, int pairs) { return mi_moe::share_of_k(K, n, pairs != 0); }\n'
-                                'extern "C" int tile(long M, int N, int K, int bits, int group) { return (int)mi_moe::dense_tile(M, N, K, bits, group); }\n')
+                                'extern "C" int tile(long M, int N, int K, int bits, int group, int bf16) { return (int)mi_moe::dense_tile(M, N, K, bits, group, bf16 != 0); }\n')
     so = d / "rule.so"
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", os.path.join(ROOT, "mlx-rs_amd", "csrc"),
                     str(d / "rule.cpp"), "-o", str(so)], check=True)
     lib = C.CDLL(str(so))
-    lib.tile.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int, C.c_int]
+    lib.tile.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int]
     return lib
 
 
@@ -32,7 +32,7 @@ def test_shares_of_k_are_as_even_as_whole_128s_can_be(rule, n):
     assert rule.share(2432, 4, 0) == 640
 
 
-SMALL, COLUMNS, WIDE, REGISTERS, REGISTERS_SHARED = range(5)  # DenseTile
+SMALL, REGISTERS_SMALL, COLUMNS, WIDE, REGISTERS, REGISTERS_SHARED = range(6)  # DenseTile
 
 
 @pytest.mark.parametrize("shape,bits,group,want", [
@@ -47,4 +47,10 @@ SMALL, COLUMNS, WIDE, REGISTERS, REGISTERS_SHARED = range(5)  # DenseTile
 ])
 def test_the_tile_follows_the_fullest_xcd(rule, shape, bits, group, want):
     """Each of these was measured with the other tiles too (dense_rule.hpp)."""
-    assert rule.tile(*shape, bits, group) == want
+    assert rule.tile(*shape, bits, group, 0) == rule.tile(*shape, bits, group, 1) == want
+
+
+@pytest.mark.parametrize("shape,bits,group,bf16,want", [((102, 1808, 3584), 8, 32, 1, REGISTERS_SMALL), ((29, 2176, 1920), 8, 32, 1, REGISTERS_SMALL), ((49, 1200, 1024), 8, 32, 1, SMALL),
+                                                        ((258, 1744, 1408), 8, 32, 1, SMALL), ((102, 1808, 3584), 8, 32, 0, SMALL), ((102, 1808, 3584), 8, 64, 1, SMALL), ((102, 1808, 3584), 4, 32, 1, SMALL)])
+def test_small_tiles_with_every_code_converted_stay_in_registers(rule, shape, bits, group, bf16, want):
+    assert rule.tile(*shape, bits, group, bf16) == want
