@@ -152,6 +152,18 @@ bool codes_tiles_fit(const mi_moe_config &c, int64_t T) {
 bool raw_tiled_batch(const mi_moe_config &c, int64_t T) {
   return T > kRowsMost && T * c.top_k >= (int64_t)4 * c.n_experts && codes_tiles_fit(c, T);
 }
+// Groups of 32, 4-bit codes: below sixteen rows an expert on average those tiles have their codes in registers (qmm_codes.hip).  A block of the others
+// takes half of a CU's LDS and waits for it behind the short segments' blocks, which fill what falls free.  Measured, us of a forward, registers / LDS,
+// at an average of 5, 8, 12, 14, 16, 19.5 rows (experts, k, hidden, intermediate):
+//   128, 8, 2048, 768   Zipf-1.1 119, 124, 128, 135, 143, 158 / 141, 143, 148, 155, 157, 157; 1.3 116, 122, 126, 134, 134, 151 / 119, 121, 148, 153, 155, 158;
+//                       even 157, 166, 178, 194, 191, 234 / 148, 157, 186, 183, 181, 205
+//   64, 6, 2048, 1408   Zipf-1.1 110, 128, 131, 154, 159, 161 / 142, 152, 152, 158, 158, 161; 1.3 111, 119, 119, 145, 146, 149 / 141, 149, 150, 154, 155, 159;
+//                       even 143, 160, 183, 182, 185, 215 / 142, 159, 180, 186, 178, 201
+//   128, 8, 4096, 1536  Zipf-1.1 388, 460, 517, 571, 571, 632 / 421, 487, 550, 608, 614, 664; 1.3 344, 388, 432, 460, 459, 528 / 367, 420, 466, 497, 511, 558;
+//                       even 682, 748, 803, 782, 722, 672 / 682, 749, 818, 792, 722, 603
+//   8, 2, 4096, 7168    Zipf-1.1 at 5, 8, 12, 14 rows 234, 354, 335, 336 / 232, 311, 314, 380; even 228, 252, 359, 372 / 230, 252, 380, 341
+// 8-bit codes, and groups of 128, are faster in LDS at nearly all of these (0.94 to 1.35 times).
+bool raw_tiles_in_registers(const mi_moe_config &c, int64_t P) { return c.group_size == 32 && c.bits == 4 && P < (int64_t)16 * c.n_experts; }
 // Groups of 64, 4-bit codes: batches whose segments all go through short tiles on raw codes, in one launch a product on the caller's
 // stream (the others: streamed segments, and tiles of 256 weight rows on side streams).  From the batches on for which the tile lists
 // are built and the router has kernels of its own, up to 96 rows per expert on average.  Measured, us of a forward, other route / this one:
@@ -541,7 +553,8 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   ca.w1 = h->w.up.w; ca.s1 = h->w.up.scales; ca.b1 = h->w.up.biases;
   ca.y = f.hh;
   ca.y_paired = copied;
-  ca.y_sums = f.raw_hsums;
+  const bool in_registers = f.raw && raw_tiles_in_registers(c, P);
+  ca.y_sums = in_registers ? nullptr : f.raw_hsums;
   ca.N = c.intermediate; ca.K = c.hidden;
   cd.x = f.hh;
   cd.x_rows = P;
@@ -554,9 +567,15 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     return launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, s);
   };
   auto tiles_up = [&](hipStream_t s) -> hipError_t {
+    if (in_registers) return launch_qmm_codes_list(ca, f.raw_tiles, f.raw_cap, true, s);
     return launch_qmm_codes_tiles(ca, f.raw_tiles, f.raw_cap, c.group_size, c.bits, true, s);
   };
   auto tiles_down = [&](hipStream_t s) -> hipError_t {
+    if (in_registers) {
+      // (the sums of all rows of h: those of the short segments, which another stream may still be writing, are not read)
+      const hipError_t e = launch_prepare_rows(f.hh, P, c.intermediate, c.group_size, MI_MOE_DTYPE_BF16, nullptr, f.raw_hsums, s);
+      return e != hipSuccess ? e : launch_qmm_codes_list(cd, f.raw_tiles, f.raw_cap, false, s);
+    }
     return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.group_size, c.bits, false, s);
   };
   if (mid) {

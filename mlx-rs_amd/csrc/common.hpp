@@ -397,6 +397,8 @@ hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, in
                                uint16_t *sums, hipStream_t st);
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
 hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st);
+// the same tiles with the codes in registers (bf16, 4-bit, groups of 32); a.y_sums is not written
+hipError_t launch_qmm_codes_list(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
 hipError_t launch_quantize(const float *w, int64_t rows, int64_t cols, int group, int bits,
                            uint32_t *q, void *s, void *b, int dt, hipStream_t st);
 hipError_t launch_dequantize(const uint32_t *q, const void *s, const void *b,

@@ -184,6 +184,40 @@ products round gate and up as well (0.94 * 2^-8, over as few as 256 values): 1.5
         assert float((again.double() - ref).norm() / ref.norm()) <= bound
 
 
+@pytest.mark.parametrize("hidden,inter,experts,k", [(256, 384, 8, 2), (1152, 128, 9, 3), (128, 1152, 40, 8)])
+@pytest.mark.parametrize("rows", [5, 15.9, 16, 30])
+@pytest.mark.parametrize("bits,group", [(4, 32), (4, 128), (8, 32)])
+def test_long_segments_on_both_sides_of_sixteen_rows_an_expert(bits, group, rows, hidden, inter, experts, k):
+    """With 4-bit codes in groups of 32 the long segments' tiles hold their codes in registers below that average and in LDS from it on.
+    Uneven routing: segments of one to all the tokens, in tiles of 1 to 64 rows; columns and K of 1, 3 and 9 times 128.  The bound is
+    test_blocks_with_groups_of_32_and_128's.  The order of the tokens changes no bit of a row whose segment keeps its kernel."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    tokens = max(int(rows * experts / k), 17)
+    cfg = m.MoeConfig(hidden, experts, k, inter, bits, group, 0)
+    blk = synth.make_block(cfg, seed=int(rows), device="cuda", zipf_s=1.2, gen_device="cuda")
+    x = synth.make_tokens(cfg, tokens, seed=bits, device="cuda")
+    out, routing = blk.forward(x, debug=True)
+    ref = block_truth(blk, x, routing)
+    assert float((out.double() - ref).norm() / ref.norm()) <= 2.0 ** -8
+    p = torch.randperm(tokens, generator=torch.Generator().manual_seed(3)).cuda()
+    assert torch.equal(blk.forward(x[p].contiguous()), out[p])
+
+
+def test_a_gate_that_is_not_finite_in_tiles_with_codes_in_registers():
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(256, 8, 2, 384, 4, 32, 0)
+    blk = synth.make_block(cfg, seed=2, device="cuda", zipf_s=1.0, gen_device="cuda")
+    x = synth.make_tokens(cfg, 45, seed=1, device="cuda")
+    blk.gate_proj.biases[:, 5, 2] = float("inf")
+    blk.up_proj.biases[:, 7, 0] = float("-inf")
+    blk.down_proj.scales[:, 9, 1] = float("inf")
+    out, routing = blk.forward(x, debug=True)
+    ref = block_truth(blk, x, routing)
+    assert not ref.isfinite().all() and torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
+
+
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("group", [32, 64, 128])
