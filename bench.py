@@ -85,7 +85,8 @@ def time_steps(fn, steps, warmup, torch):
 
 def tile_class_rows(counts, cfg, T, capi):
     """Rows of the batch that each grouped-product kernel processes: [256-row tiles, 128-row tiles,
-    64-row tiles, streamed], by the library's own rule (capi.tile_rule, capi.segment_rows_by_kernel)."""
+    64-row tiles (on raw codes where the rule says so), streamed], by the library's own rule (capi.tile_rule,
+    capi.segment_rows_by_kernel)."""
     tiled, tmr = capi.tile_rule(cfg.c_struct(), T)
     rows = [0, 0, 0, 0]
     for c in counts:

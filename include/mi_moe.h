@@ -161,8 +161,10 @@ int mi_moe_rms_norm(const uint16_t *x, const uint16_t *weight, float eps, int64_
  * array of MI_MOE_N_KERNEL_TIMES, or NULL): the durations of the grouped-product kernels themselves,
  * each from the start and end time stamps of its own dispatch (what a profiler reports for the
  * kernel): gate/up + SwiGLU over the 256-row, 128-row and 64-row tile lists and over the streamed
- * segments, then the down product over the same four; 0 where no kernel was launched.  The kernels
- * run one after the other on `stream`.  For measurement; mlx-rs has no counterpart (it times with
+ * segments, then the down product over the same four; 0 where no kernel was launched.  Batches whose
+ * segments all go through 64-row tiles on raw codes (mi_moe_debug_tile_rule: 2) report those two launches
+ * as the 64-row ones; blocks with 2-bit codes or groups of 32 / 128 report no kernel.  The kernels
+ * run one after the other on `stream`, and the result has the bits of mi_moe_forward.  For measurement; mlx-rs has no counterpart (it times with
  * Instant::now() around eval, mlx-rs/examples/linear_regression.rs:40-59). */
 #define MI_MOE_N_STAGES 6
 #define MI_MOE_N_KERNEL_TIMES 8
@@ -312,7 +314,8 @@ int mi_moe_dequantize_native(const uint32_t *q, const void *scales, const void *
  * until the library is unloaded): the test suite uses them to show that no variant is left
  * without a parity-checked launch.  mi_moe_debug_plan_forward / _grouped write, into the host buffer
  * `out` (cap bytes, NUL-terminated, entries separated by ';'), the variants with grid and LDS bytes that
- * a forward of T tokens / one grouped product of the given extents WOULD launch, and launch nothing:
+ * a forward of T tokens (with a workspace of mi_moe_workspace_size) / one grouped product of the given extents
+ * WOULD launch, and launch nothing (an empty plan: a forward on other kernels, those on raw codes or the plain ones):
  * they need no GPU and touch no device memory (the host-side launch rules, checked on any machine).
  * _grouped: total_rows rows in max_active segments of at most max_rows_per_expert rows;
  * max_streamed_rows (0 = unknown) bounds the segments that are not tiled; tile_lists non-zero = M-tile
@@ -327,9 +330,10 @@ int mi_moe_debug_plan_grouped(int32_t N, int32_t K, int32_t bits, int32_t glu, i
                               int32_t max_active, int64_t max_rows_per_expert,
                               int64_t max_streamed_rows, int32_t tile_lists, int32_t paired_out,
                               char *out, size_t cap);
-/* which rows of a forward of T tokens go where: *tiled = M-tile lists are built; *tile_min_rows = a segment of
+/* which rows of a forward of T tokens go where: *tiled = 1: M-tile lists are built; *tile_min_rows = a segment of
  * at least that many rows is cut into 256-row tiles, with its remainder in the 256-, 128- or 64-row list that
- * holds it; shorter segments stream */
+ * holds it; shorter segments stream.  *tiled = 2: every segment is cut into 64-row tiles on raw codes (4-bit codes in
+ * groups of 64, batches between the streamed and the large tiles; given a workspace of mi_moe_workspace_size) */
 int mi_moe_debug_tile_rule(const mi_moe_config *cfg, int64_t T, int32_t *tiled, int32_t *tile_min_rows);
 int32_t mi_moe_debug_side_streams_created(void);
 

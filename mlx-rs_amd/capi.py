@@ -160,16 +160,18 @@ def _plan_entries(buf):
 
 def tile_rule(cfg, tokens):
     """(tile lists are built, rows from which a segment is tiled) for a forward of `tokens` tokens: the
-    library's own rule (needs no GPU)."""
+    library's own rule (needs no GPU).  The first is 2 where every segment goes in 64-row tiles on raw codes."""
     tiled, tmr = C.c_int32(), C.c_int32()
     check(load_library().mi_moe_debug_tile_rule(C.byref(cfg), tokens, C.byref(tiled), C.byref(tmr)))
-    return bool(tiled.value), tmr.value
+    return tiled.value, tmr.value
 
 
 def segment_rows_by_kernel(count, tiled, tmr):
     """Rows of a segment of `count` rows that each grouped-product kernel takes:
     [256-row tiles, 128-row tiles, 64-row tiles, streamed] (see tile_rule)."""
     count = int(count)
+    if tiled == 2:
+        return [0, 0, count, 0]
     if not tiled or count < tmr:
         return [0, 0, 0, count]
     full, r = divmod(count, 256)
@@ -184,7 +186,7 @@ def segment_rows_by_kernel(count, tiled, tmr):
 
 
 def plan_forward(cfg, tokens):
-    """The grouped-product kernel variants a forward of `tokens` tokens would launch, as
+    """The listed kernel variants (see kernel_launches) a forward of `tokens` tokens would launch, as
     [(name, {"grid": "AxB", "block": "256", "lds": bytes})]; launches nothing and needs no GPU."""
     lib = load_library()
     buf = C.create_string_buffer(4096)

@@ -478,7 +478,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   } while (0)
   if (ev) MI_HIP(hipEventRecord(ev[0], st));
   const bool fused_router = router_fused_applies(T, c.n_experts, c.top_k);
-  const bool mid = f.mid && !kt;  // (kt times the kernels of the other route)
+  const bool mid = f.mid;
   uint32_t *const tile_lists = f.tiled && !mid ? f.mtiles : nullptr;
   const int tile_cap = f.max_mtiles, tile_from = f.tmr;
   const ShortTiles shorts = {mid || f.raw ? f.raw_tiles : nullptr, (uint32_t)f.raw_from};
@@ -578,11 +578,21 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     }
     return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.group_size, c.bits, false, s);
   };
+  struct TimerScope {  // a timer never outlives the launch it is meant for
+    explicit TimerScope(KernelTimer *t) { g_kernel_timer = t; }
+    ~TimerScope() { g_kernel_timer = nullptr; }
+  };
   if (mid) {
     MI_HIP(prepare_x(st));
-    MI_HIP(tiles_up(st));
+    {
+      TimerScope scope(kt ? &kt[2] : nullptr);
+      MI_HIP(tiles_up(st));
+    }
     MI_STAGE_DONE();
-    MI_HIP(tiles_down(st));
+    {
+      TimerScope scope(kt ? &kt[4 + 2] : nullptr);
+      MI_HIP(tiles_down(st));
+    }
     MI_STAGE_DONE();
   } else if (f.raw) {
     // group sizes 32 / 128: short segments on the kernel of a few rows, longer ones (where lists are built) in tiles
@@ -743,10 +753,6 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   } else if (kt) {
     // one kernel after the other, each dispatch with a timer of its own: tile classes 0, 1, 2 (the
     // 256-, 128- and 64-row lists), then the streamed segments; gate/up first, then down
-    struct TimerScope {  // the timer never outlives the launch it is meant for
-      explicit TimerScope(KernelTimer *t) { g_kernel_timer = t; }
-      ~TimerScope() { g_kernel_timer = nullptr; }
-    };
     for (int half = 0; half < 2; ++half) {
       const GroupedArgs &g = half == 0 ? a : d;
       for (int cls = 0; cls < 3; ++cls) {
@@ -1415,9 +1421,13 @@ int mi_moe_debug_plan_forward(const mi_moe_config *cfg, int64_t T, char *out, si
   if (T < 1 || T * cfg->top_k > (int64_t)1 << 30) return fail("debug_plan_forward: token count out of range");
   if (plain_config(*cfg)) {
     if (out && cap) out[0] = 0;
-    return 0;  // the plain products: none of the listed kernels
+    return 0;  // products on raw codes or plain ones: none of the listed kernels
   }
   const ForwardWs f = carve_forward(*cfg, T, reinterpret_cast<void *>(uintptr_t{256}));
+  if (f.mid) {
+    if (out && cap) out[0] = 0;
+    return 0;  // (neither are the short tiles)
+  }
   mi_moe_weights w{};
   GroupedArgs a{}, d{};
   grouped_args(*cfg, w, f, reinterpret_cast<const uint16_t *>(uintptr_t{256}), T, a, d);
@@ -1431,8 +1441,8 @@ int mi_moe_debug_tile_rule(const mi_moe_config *cfg, int64_t T, int32_t *tiled, 
   if (check_config(cfg)) return 1;
   if (T < 0 || T * cfg->top_k > (int64_t)1 << 30) return fail("debug_tile_rule: token count out of range");
   const ForwardWs f = carve_forward(*cfg, T, nullptr);
-  if (tiled) *tiled = f.tiled ? 1 : 0;
-  if (tile_min_rows) *tile_min_rows = f.tmr;
+  if (tiled) *tiled = f.mid ? 2 : f.tiled ? 1 : 0;
+  if (tile_min_rows) *tile_min_rows = f.mid ? 1 : f.tmr;
   return 0;
 } MI_CATCH("debug_tile_rule")
 

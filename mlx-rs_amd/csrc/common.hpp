@@ -218,6 +218,15 @@ struct KernelTimer {
   bool used = false;  // a kernel was launched with these events
 };
 extern thread_local KernelTimer *g_kernel_timer;
+template <class Kernel, class... Args>
+inline void launch_or_time(Kernel kernel, dim3 grid, dim3 block, size_t lds, hipStream_t st, Args... args) {
+  if (KernelTimer *t = g_kernel_timer) {
+    hipExtLaunchKernelGGL(kernel, grid, block, (unsigned)lds, st, t->start, t->stop, 0, args...);
+    t->used = true;
+  } else {
+    kernel<<<grid, block, lds, st>>>(args...);
+  }
+}
 
 // ---------------------------------------------------------------- which kernels the library holds, and which ran
 // Every instantiation of the streaming and the 256-column grouped product (qmm.hip, qmm_large.hip) that a launcher can reach
@@ -248,12 +257,7 @@ inline void launch_kernel(KernelSlot &slot, Kernel kernel, dim3 grid, dim3 block
     return;
   }
   __atomic_fetch_add(&slot.launches, 1ull, __ATOMIC_RELAXED);
-  if (KernelTimer *t = g_kernel_timer) {
-    hipExtLaunchKernelGGL(kernel, grid, block, (unsigned)lds, st, t->start, t->stop, 0, args...);
-    t->used = true;
-  } else {
-    kernel<<<grid, block, lds, st>>>(args...);
-  }
+  launch_or_time(kernel, grid, block, lds, st, args...);
 }
 
 // ---------------------------------------------------------------- launchers (host)

@@ -730,7 +730,7 @@ static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_
     static std::atomic<uint64_t> allowed{0};
     if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), (int)lds, allowed); e != hipSuccess) return e;
   }
-  kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, list, mtiles, n_ntiles, scale_shift);
+  launch_or_time(kernel, dim3((unsigned)grid), dim3(64 * WN * KW), lds, st, a, list, mtiles, n_ntiles, scale_shift);
   return hipGetLastError();
 }
 

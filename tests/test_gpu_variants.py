@@ -77,6 +77,32 @@ def test_variant_reached_by_the_operator_only(orc):
     CHECKED.add(c["variant"])
 
 
+@pytest.mark.parametrize("H,I,E,k,T,bits,group", [(256, 256, 16, 4, 150, 4, 64), (256, 384, 8, 2, 300, 4, 64), (256, 256, 16, 4, 90, 4, 64), (256, 256, 16, 4, 500, 4, 64),
+                                                   (256, 256, 16, 4, 150, 8, 64), (256, 256, 16, 4, 150, 4, 32), (256, 256, 16, 4, 40, 8, 128)])
+def test_what_is_planned_and_timed_is_what_runs(H, I, E, k, T, bits, group):
+    """In the middle range (the first two; heavy, light and 8-bit batches, groups of 32 and 128 beside it) too: the plan against the launch counters, and the
+    timed forward against the forward, bit for bit, with the kernels' times where the tile rule puts the rows."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(H, E, k, I, bits, group)
+    blk = synth.make_block(cfg, seed=3, device="cuda", zipf_s=1.0, gen_device="cuda")
+    x = synth.make_tokens(cfg, T, seed=3, device="cuda")
+    blk.reserve(T)
+    before = m.capi.kernel_launches()
+    out = blk.forward(x)
+    torch.cuda.synchronize()
+    after = m.capi.kernel_launches()
+    assert {n for n in after if after[n] > before[n]} == {n for n, _ in m.capi.plan_forward(cfg.c_struct(), T)}
+    timed, stages, kernels = blk.forward_timed(x, kernels=True)
+    assert torch.equal(timed, out) and all(v > 0 for v in stages[3:])
+    if m.capi.tile_rule(cfg.c_struct(), T)[0] == 2:
+        assert [i for i, v in enumerate(kernels) if v > 0] == [2, 6]
+    elif group == 64:
+        assert sum(v > 0 for v in kernels) >= 2
+    else:
+        assert not any(kernels)
+
+
 def test_zz_every_variant_ran_on_checked_rows():
     import mlx_rs_amd as m
     now = m.capi.kernel_launches()

@@ -66,3 +66,15 @@ def test_rows_too_long_for_a_cu_are_refused_with_a_message(capi):
     # tiles need more LDS than a CU has
     with pytest.raises(capi.MoeError):
         capi.plan_grouped(384, 16256, 4, True, 48, 12, 16)
+
+
+def test_the_middle_range_is_planned_as_it_runs(capi):
+    """4-bit codes in groups of 64, 65 tokens and more up to 96 rows an expert: every segment goes in 64-row tiles on raw codes, none of
+    the listed kernels."""
+    shape = (2048, 128, 8, 768)
+    for tokens, mid in ((95, False), (96, True), (203, True), (1536, True), (1537, False)):
+        cfg = capi.Config(*shape, 4, 64, 0)
+        assert (capi.tile_rule(cfg, tokens) == (2, 1)) is mid, tokens
+        assert (capi.plan_forward(cfg, tokens) == []) is mid, tokens
+    assert capi.segment_rows_by_kernel(200, 2, 1) == [0, 0, 200, 0]
+    assert capi.tile_rule(capi.Config(*shape, 8, 64, 0), 400)[0] == 1 and capi.plan_forward(capi.Config(*shape, 8, 64, 0), 400)
