@@ -4,10 +4,12 @@
 //
 // quantized_linear(x, w, scales, biases, linear_bias, transpose, group_size, bits) returns the result, None for whatever is not a
 // plain device tensor of the expected type, shape, layout and alignment (the caller then goes the general way, which takes it or words
-// the refusal), or the library's status where that is not zero.  Nothing is kept between calls.
+// the refusal), or the library's status where that is not zero.  Nothing is kept between calls.  The interpreter is let go around the
+// allocations and the launch, any of which may wait (for memory, for room in a queue, for a kernel to load).
 #include <ATen/ATen.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <pybind11/pybind11.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/mi_moe.h"
@@ -65,14 +67,22 @@ PyObject *quantized_linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (g_workspace(M, (int32_t)K, (int32_t)bits, &need)) Py_RETURN_NONE;
     at::DimVector shape(x->sizes().begin(), x->sizes().end());
     shape.back() = N;
-    const at::TensorOptions on = at::TensorOptions().device(x->device());
-    at::Tensor y = at::empty(shape, on.dtype(type)), ws = at::empty({(int64_t)need + 256}, on.dtype(at::kByte));
-    void *const st = c10::hip::getCurrentHIPStream(c10::hip::current_device()).stream();
-    const int status =
-        lb ? g_linear(x->const_data_ptr(), static_cast<const uint32_t *>(w->const_data_ptr()), s->const_data_ptr(), b->const_data_ptr(), lb->const_data_ptr(), M,
-                      (int32_t)N, (int32_t)K, (int32_t)group, (int32_t)bits, dt, y.data_ptr(), ws.data_ptr(), need + 256, st)
-           : g_matmul(x->const_data_ptr(), static_cast<const uint32_t *>(w->const_data_ptr()), s->const_data_ptr(), b->const_data_ptr(), M, (int32_t)N,
-                      (int32_t)K, transpose, (int32_t)group, (int32_t)bits, dt, y.data_ptr(), ws.data_ptr(), need + 256, st);
+    // (the operands' own references: another thread may drop the caller's while the interpreter is let go)
+    const at::Tensor xk = *x, wk = *w, sk = *s, bk = *b, lk = lb ? *lb : at::Tensor();
+    at::Tensor y;
+    int status = 0;
+    {
+      pybind11::gil_scoped_release let_go;
+      const at::TensorOptions on = at::TensorOptions().device(xk.device());
+      y = at::empty(shape, on.dtype(type));
+      at::Tensor ws = at::empty({(int64_t)need + 256}, on.dtype(at::kByte));
+      void *const st = c10::hip::getCurrentHIPStream(c10::hip::current_device()).stream();
+      status = lk.defined()
+                   ? g_linear(xk.const_data_ptr(), static_cast<const uint32_t *>(wk.const_data_ptr()), sk.const_data_ptr(), bk.const_data_ptr(), lk.const_data_ptr(),
+                              M, (int32_t)N, (int32_t)K, (int32_t)group, (int32_t)bits, dt, y.data_ptr(), ws.data_ptr(), need + 256, st)
+                   : g_matmul(xk.const_data_ptr(), static_cast<const uint32_t *>(wk.const_data_ptr()), sk.const_data_ptr(), bk.const_data_ptr(), M, (int32_t)N,
+                              (int32_t)K, transpose, (int32_t)group, (int32_t)bits, dt, y.data_ptr(), ws.data_ptr(), need + 256, st);
+    }
     if (status) return PyLong_FromLong(status);
     return THPVariable_Wrap(std::move(y));
   } catch (const std::exception &) {  // (out of memory, a mode that refuses the allocation: the general path meets it again and words it)

@@ -84,3 +84,21 @@ def test_native_call_under_capture():
         torch.cuda.synchronize()
         assert torch.equal(y, want)
         assert torch.equal(m.ops.quantized_linear(x, q, s, b), want)
+
+
+def test_the_interpreter_is_let_go_around_the_launch():
+    """The library's functions replaced by CPython's own question whether this thread holds the interpreter: 0, as a status, is a result."""
+    import ctypes as C
+    import mlx_rs_amd as m
+    call = m.ops._linear_call()
+    q, s, b = layer(128, 256, torch.bfloat16)
+    x, lb = torch.randn((4, 256), device="cuda").to(torch.bfloat16), torch.ones(128, device="cuda", dtype=torch.bfloat16)
+    held = C.cast(C.pythonapi.PyGILState_Check, C.c_void_p).value
+    need = C.cast(m.load_library().mi_moe_quantized_matmul_workspace_size, C.c_void_p).value
+    try:
+        call.__self__.bind(held, held, need)
+        assert isinstance(call(x, q, s, b, None, True, 64, 4), torch.Tensor) and isinstance(call(x, q, s, b, lb, True, 64, 4), torch.Tensor)
+    finally:
+        m.ops._linear_call.cache_clear()
+        m.ops._linear_call()
+    assert torch.equal(m.ops.quantized_linear(x, q, s, b, lb), (m.ops.quantized_linear(x, q, s, b).float() + 1).bfloat16())
