@@ -11,6 +11,7 @@
 #include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/api/include/torch/version.h>
 
 #include "../../include/mi_moe.h"
 
@@ -108,4 +109,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_linear_call", nullptr, -1, method
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__linear_call() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__linear_call() {
+  PyObject *const m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_with", TORCH_VERSION)) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -10,6 +10,7 @@ import ctypes as C
 import functools
 import importlib.util
 import os
+import warnings
 
 import torch
 
@@ -189,14 +190,20 @@ def _matmul_workspace_bytes(M, K, bits):
 
 @functools.lru_cache(maxsize=1)
 def _linear_call():
-    """csrc/linear_call.cpp bound to the library: the call around a linear layer without the interpreter."""
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_linear_call.so")
-    if not os.path.exists(path):
-        raise capi.MoeError(f"{path} is missing: build it with `make -C {os.path.dirname(path)}/csrc` (or __graft_entry__.build())")
-    spec = importlib.util.spec_from_file_location("_linear_call", path)
-    mod = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(mod)
+    """csrc/linear_call.cpp bound to the library: the call around a linear layer without the interpreter.  It is built against one
+    torch; where it is missing or does not load, every call goes the general way, which takes any (with one warning: a call of a few
+    rows is then 4 us longer)."""
     lib = load_library()
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_linear_call.so")
+    try:
+        spec = importlib.util.spec_from_file_location("_linear_call", path)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        if mod.built_with != torch.__version__.split("+")[0]:
+            raise ImportError(f"{path} was built against torch {mod.built_with}")
+    except ImportError as err:  # (missing, or another torch's)
+        warnings.warn(f"quantized_linear without its native call ({err}); build it with `make -C {os.path.dirname(path)}/csrc`", RuntimeWarning)
+        return lambda *args: None
     mod.bind(*(C.cast(getattr(lib, n), C.c_void_p).value for n in
                ("mi_moe_quantized_linear_typed", "mi_moe_quantized_matmul_typed", "mi_moe_quantized_matmul_workspace_size")))
     return mod.quantized_linear
