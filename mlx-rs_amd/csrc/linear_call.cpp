@@ -10,6 +10,7 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/api/include/torch/version.h>
 
@@ -86,9 +87,14 @@ PyObject *quantized_linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
     }
     if (status) return PyLong_FromLong(status);
     return THPVariable_Wrap(std::move(y));
-  } catch (const std::exception &) {  // (out of memory, a mode that refuses the allocation: the general path meets it again and words it)
-    Py_RETURN_NONE;
+  } catch (python_error &e) {  // what a mode written in Python raised from an allocation: the caller's
+    e.restore();
+  } catch (pybind11::error_already_set &e) {
+    e.restore();
+  } catch (const std::exception &) {  // (out of memory: the general path meets it again and words it)
   }
+  if (PyErr_Occurred()) return nullptr;
+  Py_RETURN_NONE;
 }
 
 // bind(addresses of the library's quantized_linear_typed, quantized_matmul_typed and quantized_matmul_workspace_size)

@@ -102,3 +102,29 @@ def test_the_interpreter_is_let_go_around_the_launch():
         m.ops._linear_call.cache_clear()
         m.ops._linear_call()
     assert torch.equal(m.ops.quantized_linear(x, q, s, b, lb), (m.ops.quantized_linear(x, q, s, b).float() + 1).bfloat16())
+
+
+@pytest.mark.parametrize("after", [0, 1])
+def test_what_a_mode_raises_from_an_allocation_is_what_the_caller_sees(after, general):
+    """From the result's allocation or the workspace's; the call after it is none the worse."""
+    import mlx_rs_amd as m
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Refuses(TorchDispatchMode):
+        left = after
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if "empty" in str(func):
+                self.left -= 1
+                if self.left < 0:
+                    raise LookupError("no allocations here")
+            return func(*args, **(kwargs or {}))
+
+    q, s, b = layer(128, 256, torch.bfloat16)
+    x = torch.randn((4, 256), device="cuda").to(torch.bfloat16)
+    want = m.ops.quantized_linear(x, q, s, b)
+    with pytest.raises(LookupError, match="no allocations here"), Refuses():
+        m.ops.quantized_linear(x, q, s, b)
+    with pytest.raises(LookupError, match="no allocations here"), Refuses():
+        general(lambda: m.ops.quantized_linear(x, q, s, b))
+    assert torch.equal(m.ops.quantized_linear(x, q, s, b), want)
