@@ -957,9 +957,11 @@ int mi_moe_dispatch(const uint32_t *expert_of_pair, int64_t P, int32_t n_experts
   if (P > 0 && !expert_of_pair) return fail("dispatch: expert_of_pair is NULL");
   size_t need = 0;
   mi_moe_dispatch_workspace_size(n_experts, P, &need);
-  if (!workspace || workspace_bytes < need) return fail("dispatch: workspace too small (need %zu bytes)", need);
+  // (512 bytes were all that up to 4096 pairs needed before the two-launch form took those from 2049 on: one block does without)
+  const size_t least = align_up(dispatch_workspace_least(n_experts, P)) + 256;
+  if (!workspace || workspace_bytes < least) return fail("dispatch: workspace too small (need %zu bytes)", need);
   Carver cv(workspace);
-  void *scratch = cv.take<char>(dispatch_workspace_bytes(n_experts, P));
+  void *scratch = workspace_bytes < need ? nullptr : cv.take<char>(dispatch_workspace_bytes(n_experts, P));
   hipStream_t st = static_cast<hipStream_t>(stream);
   MI_HIP(launch_dispatch(expert_of_pair, P, n_experts, 1, counts, offsets, perm, inv_perm, nullptr, nullptr,
                          nullptr, 0, 0, ShortTiles{}, scratch, st));
@@ -1027,9 +1029,12 @@ static int gather_qmm_impl(const void *x, const uint32_t *w, const void *scales,
   const int64_t rows = n_idx * M;
   size_t need = 0;
   mi_moe_gather_qmm_workspace_size(n_experts, n_idx, M, &need);
-  if (!workspace || workspace_bytes < need) return fail("gather_qmm: workspace too small (need %zu bytes)", need);
+  const size_t full = dispatch_workspace_bytes(n_experts, rows), little = dispatch_workspace_least(n_experts, rows);
+  const size_t least = need - align_up(full) + align_up(little);  // (as in mi_moe_dispatch)
+  if (!workspace || workspace_bytes < least) return fail("gather_qmm: workspace too small (need %zu bytes)", need);
   Carver cv(workspace);
-  void *scratch = cv.take<char>(dispatch_workspace_bytes(n_experts, rows));
+  void *scratch = cv.take<char>(workspace_bytes < need ? little : full);
+  if (workspace_bytes < need) scratch = nullptr;
   uint32_t *counts = cv.take<uint32_t>(n_experts + 1);
   uint32_t *offsets = cv.take<uint32_t>(n_experts + 1);
   uint32_t *work = cv.take<uint32_t>((size_t)n_experts * 16);

@@ -305,6 +305,8 @@ hipError_t launch_router_tile(const uint16_t *x, const uint16_t *wg, const float
 hipError_t launch_router_select(const uint16_t *logits, int64_t T, int E, int k, int mode,
                                 uint32_t *topk_idx, uint16_t *topk_w, hipStream_t st);
 size_t dispatch_workspace_bytes(int E, int64_t P);
+// what the dispatch of P pairs can do with: up to 4096 one block of its own takes them where there is no scratch (nullptr)
+size_t dispatch_workspace_least(int E, int64_t P);
 hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, uint32_t *counts,
                            uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
                            uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, int big_thr,

@@ -106,6 +106,8 @@ size_t dispatch_workspace_bytes(int E, int64_t P) {
   return (size_t)nb * E * sizeof(uint32_t) + 256;
 }
 
+size_t dispatch_workspace_least(int E, int64_t P) { return P <= kSingleAtMostP ? 256 : dispatch_workspace_bytes(E, P); }
+
 hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, uint32_t *counts,
                            uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
                            uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, int big_thr,
@@ -113,7 +115,8 @@ hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, ui
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
   if (k_div < 1) k_div = 1;
-  if (P <= kSingleMaxP) {
+  if (P <= kSingleMaxP || !scratch) {
+    if (P > kSingleAtMostP) return hipErrorInvalidValue;
     size_t lds = (size_t)(3 + kDispWaves) * E * sizeof(uint32_t);
     dispatch_single_kernel<<<1, kDispThreads, lds, st>>>(flat, P, E, nbits, k_div, counts, offsets,
                                                         perm, inv_perm, src_of, work, mtiles, cap256, (uint32_t)big_thr, shorts);

@@ -248,6 +248,7 @@ __device__ __forceinline__ void dispatch_block(const uint32_t *flat, int64_t P, 
 // Pairs up to which one block dispatches: its passes of 1024 follow each other.  128 experts, us of the kernels, one block / histograms and scatter
 // of blocks side by side: 4096 pairs 13.4 .. 15.3 / 8.4 .. 12; 1624 pairs 9 / no less.
 constexpr int64_t kSingleMaxP = 2048;
+constexpr int64_t kSingleAtMostP = 4096;  // without memory for the histograms
 
 // The dispatch of at most 64 tokens whose k experts are distinct per token (what the selection
 // produces), by one block.  The stable order by pair index is then the order by token, and a

@@ -1,5 +1,7 @@
 """Blocks whose segments all go through short tiles on raw codes (groups of 64, 4-bit, 65 tokens and more up to 96 rows per expert), and
 the tiles the dense products on raw codes choose from, against float64."""
+import ctypes as C
+
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -108,3 +110,34 @@ def test_dispatch_around_one_block(pairs, experts):
     want = torch.argsort(e.long(), stable=True)
     assert torch.equal(counts, torch.bincount(e.long(), minlength=experts)) and torch.equal(offsets[1:], counts.cumsum(0))
     assert torch.equal(perm, want) and torch.equal(inv[perm], torch.arange(pairs))
+
+
+@pytest.mark.parametrize("pairs,experts", [(2049, 8), (4096, 512), (3000, 70)])
+def test_dispatch_with_the_workspace_of_one_block(pairs, experts):
+    """512 bytes are enough up to 4096 pairs, as before the two-launch form, for the products by index too; the results are those of a full workspace."""
+    import mlx_rs_amd as m
+    lib = m.load_library()
+    e = torch.randint(0, experts, (pairs,), generator=torch.Generator().manual_seed(pairs), dtype=torch.int32).cuda()
+    perm, ws = torch.empty_like(e), torch.empty(512, dtype=torch.uint8, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+
+    def dispatch(size, n=pairs):
+        return lib.mi_moe_dispatch(e.data_ptr(), n, experts, None, None, perm.data_ptr(), None, ws.data_ptr(), size, st)
+    assert dispatch(512) == 0 and torch.equal(perm.cpu().long(), torch.argsort(e.cpu().long(), stable=True))
+    assert dispatch(511) != 0 and b"workspace too small" in lib.mi_moe_last_error()
+    assert lib.mi_moe_dispatch(e.data_ptr(), 4097, experts, None, None, perm.data_ptr(), None, ws.data_ptr(), 512, st) != 0  # (refused before anything is read)
+    need = C.c_size_t()
+    m.capi.check(lib.mi_moe_gather_qmm_workspace_size(experts, pairs, 1, C.byref(need)))
+    full = C.c_size_t()
+    m.capi.check(lib.mi_moe_dispatch_workspace_size(experts, pairs, C.byref(full)))
+    q, s, b = m.ops.quantize(torch.randn((experts * 16, 128), device="cuda") * 0.02, 64, 4)
+    x = torch.randn((pairs, 1, 128), device="cuda").bfloat16()
+    want = m.ops.gather_qmm(x, q.reshape(experts, 16, -1), s.reshape(experts, 16, -1), b.reshape(experts, 16, -1), rhs_indices=e)
+    least = need.value - (full.value - 512)
+    y, ws = torch.empty_like(want), torch.empty(least, dtype=torch.uint8, device="cuda")
+
+    def gather(size):
+        return lib.mi_moe_gather_qmm(x.data_ptr(), q.data_ptr(), s.data_ptr(), b.data_ptr(), None, e.data_ptr(), pairs, pairs, 1, 16, 128, experts, 1, 64, 4, 0,
+                                     y.data_ptr(), ws.data_ptr(), size, st)
+    assert gather(least) == 0 and torch.equal(y, want)
+    assert gather(least - 1) != 0 and b"workspace too small" in lib.mi_moe_last_error()
