@@ -65,7 +65,7 @@ def test_long_segments_and_imbalance(orc):
 
 
 def test_prefill_sized_dispatch(orc):
-    # P = 6000 pairs > 4096: the multi-block dispatch path
+    # P = 6000 pairs > 2048: the multi-block dispatch path
     _run_case(orc, 128, 64, 6, 128, 4, 1000, 0, seed=7, zipf_s=1.1)
 
 
@@ -110,10 +110,11 @@ def _fused_vs_separate(orc, m, H, E, k, I, batches):
 
 
 @pytest.mark.parametrize("T,E,k,bits,zipf", [(192, 8, 2, 4, None), (200, 8, 2, 4, 0.8), (700, 8, 2, 8, None),
-                                             (333, 16, 4, 4, 1.2), (1100, 4, 1, 4, None)])
+                                             (333, 16, 4, 4, 1.2), (500, 16, 4, 4, 1.2), (1100, 4, 1, 4, None)])
 def test_tile_classes(orc, T, E, k, bits, zipf):
     # segments of 9 rows and more are cut into 256-, 128- and 64-row tiles, shorter ones stream:
-    # these shapes put segments into every class, with remainders on both sides of each boundary
+    # these shapes put segments into every class, with remainders on both sides of each boundary (333 tokens: 83 rows
+    # an expert with 4-bit codes, which go in 64-row tiles on raw codes instead)
     _run_case(orc, 256, E, k, 384, bits, T, 0, seed=31 + T, zipf_s=zipf)
 
 
@@ -133,19 +134,19 @@ def test_two_token_groups_per_pass(orc, T, H, I):
 
 
 @pytest.mark.parametrize("T,H,E,k,I", [(64, 512, 64, 8, 1536), (100, 512, 64, 8, 2048), (65, 2048, 33, 6, 1536),
-                                       (160, 1024, 128, 8, 1536)])
+                                       (160, 1024, 128, 8, 1536), (80, 512, 40, 6, 2048), (64, 1024, 48, 8, 1536)])
 def test_two_token_groups_with_rows_in_slabs(orc, T, H, E, k, I):
     # the down product of a layer with many experts (more blocks than CUs) and rows of 1536 or 2048 values at 8
     # to 16 rows per expert: two token groups per pass, rows staged in slabs of 1024 (the last one of 512 values
-    # for 1536), one row tile per wave
+    # for 1536), one row tile per wave (100 and 160 tokens of these layers, 800 and 1280 pairs, go in 64-row tiles on raw codes)
     _run_case(orc, H, E, k, I, 4, T, 0, seed=300 + T)
 
 
-@pytest.mark.parametrize("T,E,k,zipf", [(100, 16, 2, 1.5), (40, 16, 4, 1.2), (150, 32, 4, 1.0), (150, 32, 4, None)])
+@pytest.mark.parametrize("T,E,k,zipf", [(100, 16, 2, 1.5), (40, 16, 4, 1.2), (150, 32, 4, 1.0), (150, 32, 4, None), (120, 32, 4, 1.0), (120, 32, 4, None)])
 def test_light_batches_tile_only_long_segments(orc, T, E, k, zipf):
     # 6 to 20 rows per expert on average (4-bit): the streamed segments lead on the caller's stream,
     # segments of 17 rows and more (uneven routing) are tiled on the side streams; 40 tokens: the
-    # one-launch router builds the tile lists
+    # one-launch router builds the tile lists (150 tokens: 600 pairs, which go in 64-row tiles on raw codes)
     _run_case(orc, 256, E, k, 384, 4, T, 0, seed=57 + T, zipf_s=zipf)
 
 
@@ -182,11 +183,11 @@ def test_norm_and_residual_around_the_block(orc, T, H, E, k, I, bits, mode, zipf
         blk.forward_residual(xd, nwd, 1e-6, out=xd)
 
 
-@pytest.mark.parametrize("T", [4, 70, 300])
+@pytest.mark.parametrize("T", [4, 70, 300, 500])
 def test_graph_replays_equal_eager(orc, T):
     """A forward captured into a HIP graph (decode: the one-launch router with its self-resetting
-    arrival counters; 70 tokens: streamed segments first, tiles beside them; prefill: the tiled
-    kernels) gives the eager result on every replay, with eager forwards of other sizes and
+    arrival counters; 70 tokens: streamed segments first, tiles beside them; 300: 64-row tiles on raw codes;
+    500: the tile classes beside each other) gives the eager result on every replay, with eager forwards of other sizes and
     synchronisations in between."""
     import mlx_rs_amd as m
     H, E, k, I = 256, 16, 4, 256

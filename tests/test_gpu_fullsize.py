@@ -24,8 +24,8 @@ CASES = [
     ("qwen3_30b_a3b", 24, None),    # 1.5 rows per expert: short segments, five rows per pass and four blocks per CU
     ("qwen3_30b_a3b", 32, None),
     ("qwen3_30b_a3b", 48, None),    # 3 rows per expert: eight rows per pass
-    ("qwen3_30b_a3b", 160, None),   # 10 rows per expert: two token groups per pass, rows staged in slabs of 1024
-    ("qwen3_30b_a3b", 200, 1.1),    # light batch, uneven routing: long segments tiled beside the streamed ones
+    ("qwen3_30b_a3b", 160, None),   # 10 rows per expert: 64-row tiles on raw codes, all of them short
+    ("qwen3_30b_a3b", 200, 1.1),    # uneven routing: segments of one to all the tokens in the same tiles
     ("qwen3_30b_a3b", 4096, 1.1),
     ("mixtral_8x7b", 1, None),
     ("mixtral_8x7b", 4, None),    # streamed; the down product's rows (K = 14336) and their scales go through LDS in slabs
@@ -36,8 +36,8 @@ CASES = [
     ("mixtral_8x7b", 2048, None),
     ("qwen3_235b_a22b", 2, None),   # K split over the waves, rows of 4096 4-bit values
     ("qwen3_235b_a22b", 32, None),  # streamed, 4-bit rows of 4096 values (two blocks per CU)
-    ("qwen3_235b_a22b", 160, None), # 10 rows per expert: two token groups per pass; the down product's rows of 1536 values in slabs of 1024 + 512
-    ("qwen3_235b_a22b", 384, 1.3),  # light batch, uneven routing
+    ("qwen3_235b_a22b", 160, None), # 10 rows per expert: 64-row tiles on raw codes; the down product's K of 1536 in a window and a half
+    ("qwen3_235b_a22b", 384, 1.3),  # the same, uneven routing
     ("qwen3_235b_a22b", 8192, 1.3),
 ]
 
