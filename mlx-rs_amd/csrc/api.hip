@@ -172,7 +172,12 @@ bool raw_tiles_in_registers(const mi_moe_config &c, int64_t P) { return c.group_
 //   hidden 4096, intermediate 1536, even at 128 / 256 / 512 / 1024 / 2048 tokens 536, 587, 665, 785, 1144 / 372, 375, 449, 649, 1101; Zipf-1.3
 //   315, 442, 510, 698, 1079 / 271, 354, 477, 693, 1123.
 // Longer segments in 256-row tiles beside this (a fork, six launches more): 203 for 169 at 512 tokens, 516 for 490 at 4096.
-// 8-bit codes (8 experts, 4096 x 14336, 256 / 512 tokens): 741, 737 / 835, 1107.  Few pairs or experts leave most of the chip idle.
+//   fewer experts, even and Zipf-1.1, (experts, k, hidden, intermediate): 64, 6, 2048, 1408 at 128, 300, 700, 1000 tokens 166, 200, 260, 265 and 139, 193, 249,
+//   269 / 110, 135, 198, 238 and 113, 147, 202, 245; 32, 4, 2048, 1024 at 128, 300, 700 120, 109, 134 and 132, 159, 166 / 60, 75, 102 and 73, 87, 113;
+//   16, 4, 4096, 6400 at 128, 256, 384 414, 531, 526 and 479, 521, 609 / 273, 374, 474 and 330, 366, 461; 16, 2, 2048, 2048 at 256, 512, 760 110, 161, 139 and
+//   169, 173, 185 / 81, 98, 105 and 89, 99, 115; 8, 2, 4096, 14336 at 256, 300, 384 642, 723, 644 and 677, 719, 771 / 492, 499, 525 and 485, 481, 516.
+// 8-bit codes (8 experts, 4096 x 14336, 256 / 512 tokens): 741, 737 / 835, 1107.  Fewer than 512 pairs, or than eight experts, keep the other route, though
+// these tiles are faster there as well (144 to 504 pairs, 4 to 16 experts: 1.08 to 2.1 times).
 bool mid_batch(const mi_moe_config &c, int64_t T, bool tiled) {
   const int64_t P = T * c.top_k;
   return tiled && c.bits == 4 && T > kFusedRouterMaxTokens && P <= (int64_t)96 * c.n_experts && P >= 512 && c.n_experts >= 8 && codes_tiles_fit(c, T);
