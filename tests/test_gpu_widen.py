@@ -72,9 +72,11 @@ def test_reference_gather_qmm_in_float32(m):
         assert torch.allclose(c1, c2, rtol=1e-4, atol=1e-4), f"x batch {xb}: max difference {(c1 - c2).abs().max().item():.2e}"
 
 
-@pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-5), (torch.float16, 2e-3)])
-@pytest.mark.parametrize("bits,group,transpose", [(4, 64, True), (8, 32, True), (2, 128, True), (4, 32, False), (8, 128, False)])
-def test_typed_products_against_float64(m, dtype, tol, bits, group, transpose):
+@pytest.mark.parametrize("bits,group,transpose,dtype,tol", [
+    (*form, *of) for form in [(4, 64, True), (8, 32, True), (2, 128, True), (4, 32, False), (8, 128, False), (2, 64, False)]
+    for of in [(torch.float32, 2e-5), (torch.float16, 2e-3)]
+] + [(2, 64, False, torch.bfloat16, 4e-3)])  # (sums in float32 and one rounding of the result: at most 2^-8 of it)
+def test_typed_products_against_float64(m, bits, group, transpose, dtype, tol):
     """Random codes, scales and biases (so nothing depends on a quantizer): every element type, group
     size, bit width and weight layout of the plain kernels against the same sum in float64."""
     g = torch.Generator().manual_seed(bits * 1000 + group)
