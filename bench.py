@@ -251,6 +251,8 @@ def run_workload(name, args, torch, m, synth, dev):
         cls = max(range(3), key=lambda i: head["class_rows"][i])
         k_ms, k_rows = head["kern"][cls], head["class_rows"][cls]
         k_name = "qmm_large_kernel (gate/up + SwiGLU, %d-row tiles)" % (256, 128, 64)[cls]
+        if m.capi.tile_rule(cfg.c_struct(), headline)[0] >= 2:
+            k_name = "qmm_pieces_kernel (gate/up + SwiGLU, all tiled segments)"
         k_flops = k_rows * head["per_row_gu_flops"]
         achieved = k_flops / (k_ms * 1e-3) / 1e12
         roofline = {"kernel": k_name, "bound": "mfma",

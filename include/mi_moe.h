@@ -162,7 +162,7 @@ int mi_moe_rms_norm(const uint16_t *x, const uint16_t *weight, float eps, int64_
  * each from the start and end time stamps of its own dispatch (what a profiler reports for the
  * kernel): gate/up + SwiGLU over the 256-row, 128-row and 64-row tile lists and over the streamed
  * segments, then the down product over the same four; 0 where no kernel was launched.  Batches whose
- * segments all go through 64-row tiles on raw codes (mi_moe_debug_tile_rule: 2) report those two launches
+ * segments go through tiles on raw codes (mi_moe_debug_tile_rule: 2, 3) report those two launches
  * as the 64-row ones; blocks with 2-bit codes or groups of 32 / 128 report no kernel.  The kernels
  * run one after the other on `stream`, and the result has the bits of mi_moe_forward.  For measurement; mlx-rs has no counterpart (it times with
  * Instant::now() around eval, mlx-rs/examples/linear_regression.rs:40-59). */
@@ -332,8 +332,9 @@ int mi_moe_debug_plan_grouped(int32_t N, int32_t K, int32_t bits, int32_t glu, i
                               char *out, size_t cap);
 /* which rows of a forward of T tokens go where: *tiled = 1: M-tile lists are built; *tile_min_rows = a segment of
  * at least that many rows is cut into 256-row tiles, with its remainder in the 256-, 128- or 64-row list that
- * holds it; shorter segments stream.  *tiled = 2: every segment is cut into 64-row tiles on raw codes (4-bit codes in
- * groups of 64, batches between the streamed and the large tiles; given a workspace of mi_moe_workspace_size) */
+ * holds it; shorter segments stream.  *tiled = 2: every segment is cut into tiles of up to 128 rows on raw codes (4-bit
+ * codes in groups of 64, batches beyond the streamed ones; given a workspace of mi_moe_workspace_size); 3: so is every segment of
+ * *tile_min_rows rows and more (larger batches), shorter segments stream */
 int mi_moe_debug_tile_rule(const mi_moe_config *cfg, int64_t T, int32_t *tiled, int32_t *tile_min_rows);
 int32_t mi_moe_debug_side_streams_created(void);
 

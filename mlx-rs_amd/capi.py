@@ -160,7 +160,8 @@ def _plan_entries(buf):
 
 def tile_rule(cfg, tokens):
     """(tile lists are built, rows from which a segment is tiled) for a forward of `tokens` tokens: the
-    library's own rule (needs no GPU).  The first is 2 where every segment goes in 64-row tiles on raw codes."""
+    library's own rule (needs no GPU).  The first is 2 where every segment goes in tiles on raw codes, 3 where those from the
+    second's rows on do and the others stream."""
     tiled, tmr = C.c_int32(), C.c_int32()
     check(load_library().mi_moe_debug_tile_rule(C.byref(cfg), tokens, C.byref(tiled), C.byref(tmr)))
     return tiled.value, tmr.value
@@ -168,12 +169,14 @@ def tile_rule(cfg, tokens):
 
 def segment_rows_by_kernel(count, tiled, tmr):
     """Rows of a segment of `count` rows that each grouped-product kernel takes:
-    [256-row tiles, 128-row tiles, 64-row tiles, streamed] (see tile_rule)."""
+    [256-row tiles, 128-row tiles, 64-row tiles and tiles on raw codes, streamed] (see tile_rule)."""
     count = int(count)
     if tiled == 2:
         return [0, 0, count, 0]
     if not tiled or count < tmr:
         return [0, 0, 0, count]
+    if tiled == 3:
+        return [0, 0, count, 0]
     full, r = divmod(count, 256)
     rows = [full * 256, 0, 0, 0]
     if r > 128:

@@ -127,11 +127,13 @@ struct ForwardWs {
   void *disp_scratch;
   uint16_t *hh, *y, *xperm, *xnorm;
   uint16_t *gu;  // plain products only: the gate and the up product, [P, I] each
-  bool mid;             // groups of 64: all segments in short tiles (see mid_batch)
+  bool mid;             // groups of 64: all segments in pieces on raw codes (see mid_batch)
+  bool pieces;          // the same tiles for the segments of a heavy batch that are tiled, the others streamed
   bool raw;             // group sizes 32 / 128: the products on raw codes (qmm_rows, qmm_codes)
   uint32_t *raw_tiles;  // the short tiles of qmm_codes, the paired copy of x (4-bit) and the group sums of x and h, or nullptr:
   int raw_cap;          // (groups of 32 / 128) all segments go through the kernel of a few rows, in as many passes as they need
   int raw_from;         // segments of this many rows and more are cut into short tiles
+  int raw_piece;        // of this many rows
   uint16_t *raw_copy, *raw_xsums, *raw_hsums;
   size_t bytes_raw;     // up to the end of those
   void *router_scratch;  // byte planes of x and of the router matrix (logits on the int8 matrix cores), or nullptr
@@ -183,7 +185,19 @@ bool mid_batch(const mi_moe_config &c, int64_t T, bool tiled) {
   return tiled && c.bits == 4 && T > kFusedRouterMaxTokens && P <= (int64_t)96 * c.n_experts && P >= 512 && c.n_experts >= 8 && codes_tiles_fit(c, T);
 }
 
-ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws) {
+// Rows of a piece.  Longer ones read a weight row for more token rows; but a block's time grows with its rows, and until the pieces are several times what
+// the chip holds at once, the longest segments' blocks are what a launch waits for.  Gate/up and down kernels, us, pieces of 64 / 96 / 128 rows (128 experts,
+// hidden 2048) at an average of 13, 32, 64, 94 rows: Zipf-1.1 70, 109, 161, 217 / 85, 117, 164, 219 / 93, 124, 181, 224; even 91, 116, 163, 223 / 90, 116, 147,
+// 212 / 89, 113, 151, 183; at 256 rows, Zipf-1.1, 446 / 421 / 422.
+int piece_rows(int64_t pairs, int n_experts) { return pairs < (int64_t)48 * n_experts ? 64 : pairs < (int64_t)80 * n_experts ? 96 : kPieceM; }
+
+bool piece_batch(const mi_moe_config &c, int64_t T, bool heavy) {
+  const int64_t P = T * c.top_k;
+  return heavy && c.bits == 4 && T > kFusedRouterMaxTokens && P >= 512 && c.n_experts >= 8 && codes_tiles_fit(c, T);
+}
+
+// norm: the normalised rows of the residual variant are kept as long as their segments stream.
+ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) {
   const int64_t P = T * c.top_k;
   Carver cv(ws);
   ForwardWs f;
@@ -224,22 +238,37 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws) {
   f.raw_tiles = nullptr;
   f.raw_cap = 0;
   f.raw_from = kRowsMost + 1;
+  f.raw_piece = kShortTileM;
   f.bytes_min = cv.off;
   f.mid = mid_batch(c, T, f.tiled);
+  f.pieces = !f.mid && piece_batch(c, T, f.heavy);
   if (f.mid) {
     // All of it lies in memory that is free at the time where it fits, so that batches which have to fit a scratch of a given size take
     // this route as well: the list in place of the work records (nothing is streamed), the group sums of x where the down product writes
     // its rows later, those of h in the normalised rows, which only the router and the copy of x read.
     f.raw_from = 1;
-    f.raw_cap = short_list_cap(P, c.n_experts, 1);
-    const size_t list = short_list_words(f.raw_cap), xsums = codes_sums_bytes(T, c.hidden, c.group_size), hsums = codes_sums_bytes(P, c.intermediate, c.group_size);
+    f.raw_piece = piece_rows(P, c.n_experts);
+    f.raw_cap = short_list_cap(P, c.n_experts, 1, f.raw_piece);
+    const size_t list = short_list_words(f.raw_cap), xsums = codes_sums_bytes(T, c.hidden, c.group_size, true), hsums = codes_sums_bytes(P, c.intermediate, c.group_size, true);
     f.raw_tiles = list <= (size_t)c.n_experts * 16 ? f.work : cv.take<uint32_t>(list);
     f.raw_copy = f.xperm;
     f.raw_xsums = xsums <= (size_t)P * c.hidden * 2 ? f.y : cv.take<uint16_t>(xsums / 2);
     f.raw_hsums = hsums <= (size_t)T * c.hidden * 2 ? f.xnorm : cv.take<uint16_t>(hsums / 2);
   }
+  if (f.pieces) {
+    f.raw_from = f.tmr;
+    f.raw_piece = piece_rows(P, c.n_experts);
+    f.raw_cap = short_list_cap(P, c.n_experts, f.raw_from, f.raw_piece);
+    // (as above; nothing reads the 256-column tiles' lists, and where there is no norm the place of its rows is free)
+    const size_t list = short_list_words(f.raw_cap), xsums = codes_sums_bytes(T, c.hidden, c.group_size, true), hsums = codes_sums_bytes(P, c.intermediate, c.group_size, true);
+    const bool in_norm = !norm && xsums + hsums <= (size_t)T * c.hidden * 2;
+    f.raw_tiles = list <= tile_list_words(f.max_mtiles, c.n_experts) ? f.mtiles : cv.take<uint32_t>(list);
+    f.raw_copy = f.xperm;
+    f.raw_xsums = in_norm ? f.xnorm : cv.take<uint16_t>(xsums / 2);
+    f.raw_hsums = in_norm ? f.xnorm + xsums / 2 : cv.take<uint16_t>(hsums / 2);
+  }
   if (f.raw && raw_tiled_batch(c, T)) {
-    f.raw_cap = short_list_cap(P, c.n_experts, f.raw_from);
+    f.raw_cap = short_list_cap(P, c.n_experts, f.raw_from, f.raw_piece);
     f.raw_tiles = cv.take<uint32_t>(short_list_words(f.raw_cap));
     f.raw_copy = cv.take<uint16_t>(codes_copy_bytes(c.bits, T, c.hidden) / 2);
     f.raw_xsums = cv.take<uint16_t>(codes_sums_bytes(T, c.hidden, c.group_size) / 2);
@@ -399,7 +428,7 @@ int mi_moe_workspace_size(const mi_moe_config *cfg, int64_t max_tokens, size_t *
   if (check_config(cfg)) return 1;
   if (max_tokens < 0) return fail("workspace_size: negative token count");
   if (max_tokens * cfg->top_k > (int64_t)1 << 30) return fail("workspace_size: too many (token, expert) pairs");
-  *bytes = carve_forward(*cfg, max_tokens, nullptr).bytes + 256;
+  *bytes = carve_forward(*cfg, max_tokens, nullptr, true).bytes + 256;
   return 0;
 } MI_CATCH("workspace_size")
 
@@ -412,9 +441,10 @@ static void grouped_args(const mi_moe_config &c, const mi_moe_weights &w, const 
   a = GroupedArgs{};
   a.work = f.work;
   a.max_active = (int)(P < c.n_experts ? P : c.n_experts);
-  a.mtiles = f.tiled ? f.mtiles : nullptr;
+  const bool lists = f.tiled && !f.pieces;
+  a.mtiles = lists ? f.mtiles : nullptr;
   a.max_mtiles = f.max_mtiles;
-  a.tile_cap_e = f.tiled ? c.n_experts : 0;
+  a.tile_cap_e = lists ? c.n_experts : 0;
   a.bits = c.bits;
   a.total_rows = P;
   a.max_rows_per_expert = T;  // a token picks an expert at most once
@@ -468,12 +498,12 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   if (P > (int64_t)1 << 30) return fail("forward: too many (token, expert) pairs");
   if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u))
     return fail("forward: workspace must be non-NULL and 256-byte aligned");
-  ForwardWs f = carve_forward(c, T, workspace);
+  ForwardWs f = carve_forward(c, T, workspace, norm_weight != nullptr);
   if (workspace_bytes < f.bytes_min)
     return fail("forward: workspace too small (%zu bytes, need %zu)", workspace_bytes, f.bytes);
   if (workspace_bytes < f.bytes_raw) {
     f.raw_tiles = nullptr;
-    f.mid = false;
+    f.mid = f.pieces = false;
   }
   if (workspace_bytes < f.bytes) f.router_scratch = nullptr;  // room for everything but the byte planes: fp64 logits, same bits
   int stage = 0;
@@ -483,10 +513,10 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   } while (0)
   if (ev) MI_HIP(hipEventRecord(ev[0], st));
   const bool fused_router = router_fused_applies(T, c.n_experts, c.top_k);
-  const bool mid = f.mid;
-  uint32_t *const tile_lists = f.tiled && !mid ? f.mtiles : nullptr;
+  const bool mid = f.mid, raw_codes = mid || f.pieces;
+  uint32_t *const tile_lists = f.tiled && !raw_codes ? f.mtiles : nullptr;
   const int tile_cap = f.max_mtiles, tile_from = f.tmr;
-  const ShortTiles shorts = {mid || f.raw ? f.raw_tiles : nullptr, (uint32_t)f.raw_from};
+  const ShortTiles shorts = {raw_codes || f.raw ? f.raw_tiles : nullptr, (uint32_t)f.raw_from, (uint32_t)f.raw_piece};
   uint32_t *const records = mid ? nullptr : f.work;
   if (norm_weight) {  // the block's input is rms_norm(x); x itself is added back in the combine
     if (!fused_router) MI_HIP(launch_rms_norm(x_in, norm_weight, eps, T, c.hidden, f.xnorm, st));
@@ -498,7 +528,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   // registers anyway, or by a kernel of its own (light batches pair the rows beside their streamed segments)
   const bool paired = c.bits == 4;
   const bool streamed_first = f.tiled && !f.heavy && !ev && !mid;  // light batches start their streamed segments first
-  const bool pair_in_router = f.tiled && paired && !mid && !streamed_first && !fused_router && !plain_config(c) &&
+  const bool pair_in_router = f.tiled && paired && !raw_codes && !streamed_first && !fused_router && !plain_config(c) &&
                               router_logits_pairs_rows(T, c.hidden);
   if (fused_router) {
     // decode: one launch for the three stages (the stage times then all land in the first)
@@ -540,10 +570,10 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   GroupedArgs a{}, d{};
   grouped_args(c, h->w, f, x, T, a, d);
   const int max_active = a.max_active;
-  if (f.tiled && paired && !streamed_first && !pair_in_router && !mid) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));
+  if (f.tiled && paired && !streamed_first && !pair_in_router && !raw_codes) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));
   // independent chains run beside each other where side streams are to be had, whose lock is held until they have been joined back
   std::unique_lock<std::mutex> streams_guard;
-  const bool chains = !ev && !mid && (f.raw ? f.raw_tiles != nullptr : !plain_config(c) && large_qmm_applies(a));
+  const bool chains = !ev && !mid && (f.raw ? f.raw_tiles != nullptr : !plain_config(c) && (f.pieces || large_qmm_applies(a)));
   if (chains) streams_guard = std::unique_lock<std::mutex>(h->streams->lock);
   const bool fork = chains && may_fork(st, *h->streams);
   if (!fork && streamed_first && paired && large_qmm_applies(a)) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));  // (a side stream's work)
@@ -569,16 +599,18 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   cd.y = f.y;
   cd.N = c.hidden; cd.K = c.intermediate;
   auto prepare_x = [&](hipStream_t s) -> hipError_t {
-    return launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, s);
+    return launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, raw_codes, s);
   };
   auto tiles_up = [&](hipStream_t s) -> hipError_t {
+    if (raw_codes) return launch_qmm_pieces(ca, f.raw_tiles, f.raw_cap, true, s);
     if (in_registers) return launch_qmm_codes_list(ca, f.raw_tiles, f.raw_cap, true, s);
     return launch_qmm_codes_tiles(ca, f.raw_tiles, f.raw_cap, c.group_size, c.bits, true, s);
   };
   auto tiles_down = [&](hipStream_t s) -> hipError_t {
+    if (raw_codes) return launch_qmm_pieces(cd, f.raw_tiles, f.raw_cap, false, s);
     if (in_registers) {
       // (the sums of all rows of h: those of the short segments, which another stream may still be writing, are not read)
-      const hipError_t e = launch_prepare_rows(f.hh, P, c.intermediate, c.group_size, MI_MOE_DTYPE_BF16, nullptr, f.raw_hsums, s);
+      const hipError_t e = launch_prepare_rows(f.hh, P, c.intermediate, c.group_size, MI_MOE_DTYPE_BF16, nullptr, f.raw_hsums, false, s);
       return e != hipSuccess ? e : launch_qmm_codes_list(cd, f.raw_tiles, f.raw_cap, false, s);
     }
     return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.group_size, c.bits, false, s);
@@ -599,6 +631,35 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
       MI_HIP(tiles_down(st));
     }
     MI_STAGE_DONE();
+  } else if (f.pieces && fork) {
+    // The tiles here, the streamed segments beside them: they share no rows, and what streams waits for memory while the tiles multiply.
+    DeviceStreams &ds = *h->streams;
+    hipStream_t s = ds.side[0];
+    MI_HIP(hipEventRecord(ds.fork, st));
+    MI_HIP(hipStreamWaitEvent(s, ds.fork, 0));
+    hipError_t e = prepare_x(st);
+    if (e == hipSuccess) e = tiles_up(st);
+    if (e == hipSuccess) e = tiles_down(st);
+    if (e == hipSuccess) e = launch_small_qmm(a, true, s);
+    if (e == hipSuccess) e = launch_small_qmm(d, false, s);
+    // whatever happened: the caller's stream waits for what the side stream was given
+    hipError_t je = hipEventRecord(ds.join[0], s);
+    if (je == hipSuccess) je = hipStreamWaitEvent(st, ds.join[0], 0);
+    MI_HIP(e);
+    MI_HIP(je);
+  } else if (f.pieces) {
+    MI_HIP(prepare_x(st));
+    for (int half = 0; half < 2; ++half) {
+      {
+        TimerScope scope(kt ? &kt[4 * half + 2] : nullptr);
+        MI_HIP(half == 0 ? tiles_up(st) : tiles_down(st));
+      }
+      {
+        TimerScope scope(kt ? &kt[4 * half + 3] : nullptr);
+        MI_HIP(launch_small_qmm(half == 0 ? a : d, half == 0, st));
+      }
+      MI_STAGE_DONE();
+    }
   } else if (f.raw) {
     // group sizes 32 / 128: short segments on the kernel of a few rows, longer ones (where lists are built) in tiles
     RowsArgs ra{}, rd{};
@@ -802,7 +863,7 @@ int mi_moe_forward_static(mi_moe_handle h, const uint16_t *x, int64_t T, uint16_
   if (!h) return fail("forward_static: handle is NULL");
   if (T < 0) return fail("forward_static: negative token count");
   if (T * (int64_t)h->cfg.top_k > (int64_t)1 << 30) return fail("forward_static: too many (token, expert) pairs");
-  const size_t need = carve_forward(h->cfg, T, nullptr).bytes_min;
+  const size_t need = carve_forward(h->cfg, T, nullptr, false).bytes_min;
   if (need > (size_t)MI_MOE_STATIC_SCRATCH_BYTES)
     return fail("forward_static: %lld tokens of this layer need %zu bytes of workspace, the built-in scratch holds %zu "
                 "(use mi_moe_forward with a workspace of the caller's)",
@@ -1189,7 +1250,7 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
     const size_t copy_bytes = codes_copy_bytes(bits, M, K);
     uint16_t *copy = copy_bytes ? reinterpret_cast<uint16_t *>(cv.take<char>(copy_bytes)) : nullptr;
     uint16_t *sums = reinterpret_cast<uint16_t *>(cv.take<char>(codes_sums_bytes(M, K, group_size)));
-    MI_HIP(launch_prepare_rows(x, M, K, group_size, dtype, copy, sums, st));
+    MI_HIP(launch_prepare_rows(x, M, K, group_size, dtype, copy, sums, false, st));
     CodesArgs a{};
     a.x = copy ? copy : x;
     a.x_rows = M;
@@ -1433,7 +1494,7 @@ int mi_moe_debug_plan_forward(const mi_moe_config *cfg, int64_t T, char *out, si
     if (out && cap) out[0] = 0;
     return 0;  // products on raw codes or plain ones: none of the listed kernels
   }
-  const ForwardWs f = carve_forward(*cfg, T, reinterpret_cast<void *>(uintptr_t{256}));
+  const ForwardWs f = carve_forward(*cfg, T, reinterpret_cast<void *>(uintptr_t{256}), true);
   if (f.mid) {
     if (out && cap) out[0] = 0;
     return 0;  // (neither are the short tiles)
@@ -1450,8 +1511,8 @@ int mi_moe_debug_plan_forward(const mi_moe_config *cfg, int64_t T, char *out, si
 int mi_moe_debug_tile_rule(const mi_moe_config *cfg, int64_t T, int32_t *tiled, int32_t *tile_min_rows) try {
   if (check_config(cfg)) return 1;
   if (T < 0 || T * cfg->top_k > (int64_t)1 << 30) return fail("debug_tile_rule: token count out of range");
-  const ForwardWs f = carve_forward(*cfg, T, nullptr);
-  if (tiled) *tiled = f.mid ? 2 : f.tiled ? 1 : 0;
+  const ForwardWs f = carve_forward(*cfg, T, nullptr, true);
+  if (tiled) *tiled = f.mid ? 2 : f.pieces ? 3 : f.tiled ? 1 : 0;
   if (tile_min_rows) *tile_min_rows = f.mid ? 1 : f.tmr;
   return 0;
 } MI_CATCH("debug_tile_rule")

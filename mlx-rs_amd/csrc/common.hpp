@@ -177,15 +177,16 @@ __host__ __device__ inline P *tile_list(P *base, int cls, int cap256, int n_expe
 }
 
 // A list of the same form for the tiles of the products on raw codes: segments of `from` rows and more that the three lists do
-// not take, in pieces of kShortTileM rows; experts in ascending order.
-constexpr int kShortTileM = 64;
+// not take, in pieces of `piece` rows; experts in ascending order.
+constexpr int kShortTileM = 64, kPieceM = 128;
 struct ShortTiles {
   uint32_t *list = nullptr;
   uint32_t from = 1;
+  uint32_t piece = kShortTileM;
 };
 __host__ __device__ inline size_t short_list_words(int cap) { return 4 + 4 * (size_t)cap; }
-inline int short_list_cap(int64_t pairs, int n_experts, int from) {  // full pieces, and a segment's last one
-  return (int)(pairs / kShortTileM + (pairs / from < n_experts ? pairs / from : n_experts));
+inline int short_list_cap(int64_t pairs, int n_experts, int from, int piece) {  // full pieces, and a segment's last one
+  return (int)(pairs / piece + (pairs / from < n_experts ? pairs / from : n_experts));
 }
 
 // ---------------------------------------------------------------- element types
@@ -398,11 +399,14 @@ struct ColsArgs {
 bool qmm_cols_applies(const ColsArgs &a, int bits, int dt);
 hipError_t launch_qmm_cols(const ColsArgs &a, int group, int bits, int dt, hipStream_t st);
 size_t codes_copy_bytes(int bits, int64_t rows, int K);
-size_t codes_sums_bytes(int64_t rows, int K, int group);
+// plain: for the products on codes without a centre (launch_qmm_pieces)
+size_t codes_sums_bytes(int64_t rows, int K, int group, bool plain = false);
 hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
-                               uint16_t *sums, hipStream_t st);
+                               uint16_t *sums, bool plain, hipStream_t st);
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
 hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st);
+// 4-bit codes in groups of 64, a list of pieces of kPieceM rows
+hipError_t launch_qmm_pieces(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
 // the same tiles with the codes in registers (bf16, 4-bit, groups of 32); a.y_sums is not written
 hipError_t launch_qmm_codes_list(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
 hipError_t launch_quantize(const float *w, int64_t rows, int64_t cols, int group, int bits,

@@ -166,17 +166,17 @@ __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint
         rec[3] = 0u;
       }
       t256 += __shfl(incl, kWave - 1, kWave);
-      if (shorts.list) {  // pieces of kShortTileM rows
-        const uint32_t n = brief ? (c + kShortTileM - 1) / kShortTileM : 0u;
+      if (shorts.list) {  // pieces of shorts.piece rows
+        const uint32_t n = brief ? (c + shorts.piece - 1) / shorts.piece : 0u;
         uint32_t before = n;
         for (int d = 1; d < kWave; d <<= 1) {
           const uint32_t v = __shfl_up(before, d, kWave);
           if (tid >= d) before += v;
         }
         for (uint32_t i = 0; i < n; ++i) {
-          const uint32_t left = c - i * kShortTileM;
+          const uint32_t left = c - i * shorts.piece;
           reinterpret_cast<uint4 *>(shorts.list)[1 + t_short + before - n + i] =
-              make_uint4((uint32_t)e, cnt[e] + i * kShortTileM, left < (uint32_t)kShortTileM ? left : (uint32_t)kShortTileM, 0u);
+              make_uint4((uint32_t)e, cnt[e] + i * shorts.piece, left < shorts.piece ? left : shorts.piece, 0u);
         }
         t_short += __shfl(before, kWave - 1, kWave);
       }

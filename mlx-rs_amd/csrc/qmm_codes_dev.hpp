@@ -7,6 +7,8 @@
 namespace mi_moe {
 
 constexpr int kSlots = 8;  // K slots of a group in the bias product
+// Codes multiplied without a centre leave the bias as it is, one bf16: three slots hold the products with it, and the fourth nothing.
+constexpr int sum_slots(bool plain_codes) { return plain_codes ? 4 : kSlots; }
 
 // v = h + m + l exactly, each a bf16 (8 significant bits; by truncation, so nothing overflows).  A value that is not
 // finite gives a NaN.
@@ -18,6 +20,13 @@ __device__ __forceinline__ Pieces split3(float v) {
   const uint32_t mu = __float_as_uint(r) & 0xffff0000u;
   const float q = r - __uint_as_float(mu);
   return Pieces{hu >> 16, mu >> 16, __float_as_uint(q) >> 16};
+}
+
+// A group sum of a row as the bias product's operand: the pieces against those of the biases (six products), or against one.
+__device__ __forceinline__ void put_sums(uint16_t *to, int slots, float sum) {
+  const Pieces p = split3(sum);
+  if (slots == kSlots) *reinterpret_cast<uint4 *>(to) = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, 0u);
+  else *reinterpret_cast<uint2 *>(to) = make_uint2(p.h | p.m << 16, p.l);
 }
 
 constexpr bool paired_order(int bits) { return bits == 4; }  // 8-blocks as (0,4)(1,5)(2,6)(3,7)

@@ -29,10 +29,11 @@
 namespace mi_moe {
 
 // One thread per eight values of x.
+// slots: K slots of a group in the bias product (sum_slots).
 template <int DT>
 __global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf<DT>::type *__restrict__ x, int64_t n_octets,
                                                            int octets_per_row, int lanes_log2,
-                                                           uint16_t *__restrict__ copy, uint16_t *__restrict__ sums, int sums_row) {
+                                                           uint16_t *__restrict__ copy, uint16_t *__restrict__ sums, int sums_row, int slots) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n_octets) return;  // whole groups leave together
   float v[8];
@@ -67,11 +68,10 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf
   if ((i & ((1 << lanes_log2) - 1)) == 0) {
     const int64_t row = i / octets_per_row;
     const int g = (int)(i % octets_per_row) >> lanes_log2, G = octets_per_row >> lanes_log2;
-    const Pieces p = split3(sum);
-    uint4 *const to = reinterpret_cast<uint4 *>(sums + row * sums_row) + g;
-    *to = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, 0u);
+    uint16_t *const to = sums + row * sums_row + g * slots;
+    put_sums(to, slots, sum);
     if (g == G - 1)
-      for (int k = 1; g + k < sums_row / kSlots; ++k) to[k] = make_uint4(0, 0, 0, 0);
+      for (int k = slots; g * slots + k < sums_row; k += 4) *reinterpret_cast<uint2 *>(to + k) = make_uint2(0, 0);
   }
 }
 
@@ -188,6 +188,273 @@ struct Tile {
 };
 
 
+// The bias product of a window of sixteen groups where the codes have no centre: the group sums' three pieces against the bias, a bf16 as it is.  A lane
+// has two groups of a token row in 16 bytes (`place` of its row in LDS), and their two biases in a word.  Groups from `real` on are not this product's.
+template <int MS, int NT, class Place>
+__device__ __forceinline__ void add_plain_biases(float (&tot)[MS][NT][16], const unsigned char *rows_at, int row_bytes, Place place, const unsigned char *biases, int real, int ln, int kb) {
+  u32x4_t o[NT][4];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int g = 4 * i + 2 * kb;
+      const uint32_t b = g < real ? *reinterpret_cast<const uint32_t *>(biases + t * 1024 + g * 2) : 0u;  // (an even number of groups)
+      o[t][i] = u32x4_t{__builtin_amdgcn_perm(b, b, 0x01000100u), b & 0xffffu, __builtin_amdgcn_perm(b, b, 0x03020302u), b >> 16};
+    }
+#pragma unroll
+  for (int m = 0; m < MS; ++m) {
+    u32x4_t F[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) F[i] = *reinterpret_cast<const u32x4_t *>(rows_at + (32 * m + ln) * row_bytes + place(2 * i + kb));
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      f32x16_t sum = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum = mfma<0>(F[i], o[t][i], sum);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) tot[m][t][v] += sum[v];
+    }
+  }
+}
+
+// The results of a tile (see multiply_tile) go out, GLU: as silu(gate) up.  Every wave comes here with GLU.
+template <int DT, int BITS, bool GLU, int MS, int NT, int WN, class WeightRow>
+__device__ __forceinline__ void write_tile(const CodesArgs &a, const float (&tot)[MS][NT][16], int wave, int lane, int n0, int col0, int64_t row0, int rows,
+                                           int64_t ebase, int glog, WeightRow weight_row, unsigned char *lds_raw) {
+  // ---- epilogue: a wave turns its 32 x 32 sub-tiles round in a private piece of LDS and stores 16 bytes a lane
+  typedef typename ElemOf<DT>::type T;
+  const int N = a.N, K = a.K, G = K >> glog, row_bytes = K * BITS / 8;
+  const int ln = lane & 31, kb = lane >> 5;
+  constexpr int ROWB = 32 * (int)sizeof(T) + 16;
+  constexpr int PV = 16 / (int)sizeof(T);             // values per 16-byte piece
+  constexpr int CPR = 32 / PV;                        // pieces per row
+  constexpr int RPI = 64 / CPR;                       // rows one store instruction covers
+  unsigned char *const mine = lds_raw + wave * (32 * ROWB);
+  const int my_piece = lane % CPR, my_row = lane / CPR;
+  const bool vec = N % PV == 0;
+  // The gate/up tiles also sum their rows over the quantisation groups, which the down product's bias term wants (columns in whole blocks of 128:
+  // 32 of them here, the rest of a group in the waves beside).  A kernel over the finished rows took 5 us.
+  const bool sums_too = GLU && a.y_sums != nullptr;
+  float *const parts_of_sums = reinterpret_cast<float *>(lds_raw + WN * (32 * ROWB));  // [wave][row]
+#pragma unroll
+  for (int u = 0; u < MS * (GLU ? 1 : NT); ++u) {
+    const int m = u / (GLU ? 1 : NT), t = u % (GLU ? 1 : NT), col = col0 + 32 * t;
+    const float lb = a.bias ? as_f32(static_cast<const T *>(a.bias)[col + ln < N ? col + ln : N - 1]) : 0.f;
+    auto put = [&](int r, float v, float up) __attribute__((always_inline)) {
+      if constexpr (GLU) v = v / (1.0f + __expf(-v)) * up;
+      T o = rounded<T>(v);
+      if (a.bias) o = rounded<T>(as_f32(o) + lb);
+      reinterpret_cast<T *>(mine + (8 * (r >> 2) + 4 * kb + (r & 3)) * ROWB)[ln] = o;
+    };
+    uint32_t again = 0;  // (bits: which of the sixteen sums are not finite)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float v = tot[m][t][r], up = GLU ? tot[m][NT - 1][r] : 0.f;
+      put(r, v, up);
+      again |= (not_finite(v) || (GLU && not_finite(up)) ? 1u : 0u) << r;
+    }
+#pragma unroll 1
+    for (int quad = 0; __builtin_expect(again != 0, 0); ++quad, again >>= 4) {  // rows 8 quad + 4 kb + 0 .. 3
+      uint32_t open = again & 15u;
+      const T *xs[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        int tr = 32 * m + 8 * quad + 4 * kb + i;
+        if (tr >= rows) {  // (never stored)
+          open &= ~(1u << i);
+          tr = rows - 1;
+        }
+        xs[i] = static_cast<const T *>(a.x) + (int64_t)(a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr)) * K;
+      }
+      if (!open) continue;
+      float v[GLU ? 2 : 1][4];
+#pragma unroll
+      for (int i = 0; i < (GLU ? 2 : 1); ++i) {
+        const int64_t wrow = ebase + weight_row(GLU ? i : t, ln);
+        plain_rows<BITS, 4, T>(xs, paired_order(BITS), (GLU && i ? a.w1 : a.w0) + wrow * (row_bytes / 4),
+                               static_cast<const T *>(GLU && i ? a.s1 : a.s0) + wrow * G,
+                               static_cast<const T *>(GLU && i ? a.b1 : a.b0) + wrow * G, K, K / G, open, v[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (open >> i & 1u) put(4 * quad + i, v[0][i], v[GLU ? 1 : 0][i]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int my_col = col + PV * my_piece;
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) {
+      const int row = RPI * i + my_row;
+      const int tr = 32 * m + row;
+      if (tr < rows && my_col < N) {
+        const int64_t dst = a.dst_rows ? (int64_t)a.dst_rows[row0 + tr] : row0 + tr;
+        T *const to = static_cast<T *>(a.y) + dst * N + my_col;
+        const T *const from = reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece;
+        if (vec) {
+          *reinterpret_cast<u32x4_t *>(to) = *reinterpret_cast<const u32x4_t *>(from);
+        } else {
+          for (int c = 0; c < PV && my_col + c < N; ++c) to[c] = from[c];
+        }
+      }
+      if constexpr (GLU) {
+        if (sums_too) {
+          const u32x4_t w = *reinterpret_cast<const u32x4_t *>(reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece);
+          float sum = ((bf16lo_to_f32(w[0]) + bf16hi_to_f32(w[0])) + (bf16lo_to_f32(w[1]) + bf16hi_to_f32(w[1]))) +
+                      ((bf16lo_to_f32(w[2]) + bf16hi_to_f32(w[2])) + (bf16lo_to_f32(w[3]) + bf16hi_to_f32(w[3])));
+          sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
+          sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
+          if (my_piece == 0) parts_of_sums[wave * (32 * MS) + tr] = sum;
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  if constexpr (GLU) {
+    static_assert(DT == 0 && WN == 4, "four waves cover a group of 128");
+    if (!sums_too) return;
+    __syncthreads();
+    const int first = n0 >> glog, groups = N >> glog, here = 128 >> glog, waves = 1 << (glog - 5);  // (the output's groups are as long as the input's)
+    const int end = first + here >= groups ? padded_groups(groups) : first + here;  // the last block writes the zeros behind
+    for (int i = threadIdx.x; i < rows * (end - first); i += 64 * WN) {
+      const int row = i % rows, g = i / rows;
+      float sum = 0.f;
+      if (first + g < groups)
+        for (int w = 0; w < waves; ++w) sum += parts_of_sums[(g * waves + w) * (32 * MS) + row];
+      put_sums(a.y_sums + ((row0 + row) * padded_groups(groups) + first + g) * kSlots, kSlots, sum);
+    }
+  }
+}
+
+// Where rows l and 64 + l of a piece go, in lane l.
+__device__ __forceinline__ void output_rows(const CodesArgs &a, int64_t row0, int rows, int lane, uint32_t (&dst)[2]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int64_t r = row0 + (64 * h + lane < rows ? 64 * h + lane : rows - 1);
+    dst[h] = a.dst_rows ? a.dst_rows[r] : (uint32_t)r;
+  }
+}
+// silu(g) u, fp32.  The quotient is as the division gives it: 1 + exp(-g) is a normal number from 1 on, so a reciprocal and one correction do (an
+// infinite g comes out as no number, and is looked at again with all that are not finite).
+__device__ __forceinline__ float gated(float g, float u) {
+  const float d = 1.0f + __expf(fminf(-g, 88.0f)), r = __builtin_amdgcn_rcpf(d), q = g * r;
+  return __builtin_fmaf(__builtin_fmaf(-d, q, g), r, q) * u;
+}
+// The results of a piece of up to 32 MS rows x 256 weight rows (4-bit codes in groups of 64; four waves, 64 weight rows each) go out: N is a multiple of
+// 128, there is no bias of the layer's.  Two rows of a column become one register, neighbouring lanes swap halves, and the rows are turned round in LDS:
+// GLU: by the whole block, whose 256 bytes a row are two quantisation groups of h, of which the lanes that store them also write the group sums;
+// else by each wave, 128 bytes a row.  (Rows found and stored 16 at a time behind a load of their places each: 12 us of the 37 of a block of 128 rows, K = 768.)
+template <bool GLU, int MS, class WeightRow>
+__device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&tot)[MS][2][16], int wave, int lane, int n0, int64_t row0, int rows, int64_t ebase,
+                                            WeightRow weight_row, const uint32_t (&dst)[2], unsigned char *lds_raw) {
+  constexpr int ROWB = GLU ? 272 : 144;  // (16 bytes keep rows off each other's banks)
+  const int N = a.N, K = a.K, G = K >> 6, row_bytes = K / 2, ln = lane & 31, kb = lane >> 5;
+  unsigned char *const mine = GLU ? lds_raw + wave * 64 : lds_raw + wave * (32 * ROWB);
+  auto value = [&](int m, int t, int r) __attribute__((always_inline)) { return GLU ? gated(tot[m][0][r], tot[m][1][r]) : tot[m][t][r]; };
+  float odd = 0.f;  // no number once a result was not finite
+  uint64_t again[GLU ? 1 : 2] = {};
+  auto turn = [&](int m, int at) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < (GLU ? 1 : 2); ++t)
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        const float v0 = value(m, t, r), v1 = value(m, t, r + 1);
+        odd = __builtin_fmaf(v1, 0.f, __builtin_fmaf(v0, 0.f, odd));
+        const uint32_t own = cvt_pk_bf16(v0, v1), theirs = dpp_u32<kDppXor1>(own);
+        // even lane: row r of columns c, c + 1; odd lane: row r + 1
+        const uint32_t both = __builtin_amdgcn_perm(theirs, own, (ln & 1) ? 0x03020706u : 0x05040100u);
+        *reinterpret_cast<uint32_t *>(mine + (at + 8 * (r >> 2) + 4 * kb + (r & 3) + (ln & 1)) * ROWB + (32 * t + (ln & ~1)) * 2) = both;
+      }
+  };
+  // sums that are not finite, again on the dequantised weights (see plain_rows)
+  auto repair = [&](int m_first, int m_end, int at) __attribute__((always_inline)) {
+#pragma unroll
+    for (int m = 0; m < MS; ++m)
+#pragma unroll
+      for (int t = 0; t < (GLU ? 1 : 2); ++t) {
+        uint32_t bits = 0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bits |= (not_finite(tot[m][t][r]) || (GLU && not_finite(tot[m][1][r])) ? 1u : 0u) << r;
+        again[GLU ? 0 : t] |= (uint64_t)bits << (16 * m);
+      }
+#pragma unroll 1
+    for (int i = m_first * 4 * (GLU ? 1 : 2); i < m_end * 4 * (GLU ? 1 : 2); ++i) {  // four rows of a column at a time
+      const int t = GLU ? 0 : i & 1, quad = GLU ? i : i >> 1;  // rows 8 quad + 4 kb + 0 .. 3
+      uint32_t open = (uint32_t)((t ? again[GLU ? 0 : 1] : again[0]) >> (4 * quad)) & 15u;
+      const uint16_t *xs[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        int tr = 8 * quad + 4 * kb + j;
+        if (tr >= rows) {  // (never stored)
+          open &= ~(1u << j);
+          tr = rows - 1;
+        }
+        xs[j] = static_cast<const uint16_t *>(a.x) + (int64_t)(a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr)) * K;
+      }
+      if (!open) continue;
+      float v[GLU ? 2 : 1][4];
+#pragma unroll
+      for (int j = 0; j < (GLU ? 2 : 1); ++j) {
+        const int64_t wrow = ebase + weight_row(GLU ? j : t, ln);
+        plain_rows<4, 4, uint16_t>(xs, true, (j ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const uint16_t *>(j ? a.s1 : a.s0) + wrow * G,
+                                   static_cast<const uint16_t *>(j ? a.b1 : a.b0) + wrow * G, K, 64, open, v[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (open >> j & 1u) {
+          const float o = GLU ? v[0][j] / (1.0f + __expf(-v[0][j])) * v[GLU ? 1 : 0][j] : v[0][j];
+          reinterpret_cast<uint16_t *>(mine + (8 * quad + 4 * kb + j - at) * ROWB)[32 * t + ln] = rounded<uint16_t>(o);
+        }
+    }
+  };
+  if constexpr (GLU) {
+#pragma unroll
+    for (int m = 0; m < MS; ++m) turn(m, 32 * m);
+    if (__builtin_expect(odd != odd, 0)) repair(0, MS, 0);
+    __syncthreads();
+    const int groups = N >> 6, padded = padded_groups(groups);
+#pragma unroll
+    for (int i = 0; i < 2 * MS; ++i) {
+      const int row = 16 * i + (int)(threadIdx.x >> 4), piece = threadIdx.x & 15;
+      const u32x4_t w = *reinterpret_cast<const u32x4_t *>(lds_raw + row * ROWB + piece * 16);
+      float sum = ((bf16lo_to_f32(w[0]) + bf16hi_to_f32(w[0])) + (bf16lo_to_f32(w[1]) + bf16hi_to_f32(w[1]))) +
+                  ((bf16lo_to_f32(w[2]) + bf16hi_to_f32(w[2])) + (bf16lo_to_f32(w[3]) + bf16hi_to_f32(w[3])));
+      sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
+      sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
+      sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
+      if (row < rows) {
+        *reinterpret_cast<u32x4_t *>(static_cast<uint16_t *>(a.y) + (row0 + row) * N + n0 + 8 * piece) = w;
+        if ((piece & 7) == 0) put_sums(a.y_sums + ((row0 + row) * padded + (n0 >> 6) + (piece >> 3)) * sum_slots(true), sum_slots(true), sum);
+      }
+    }
+    if (n0 + 128 >= N && groups < padded)  // the last block of a row writes the zeros behind its sums
+      for (int i = threadIdx.x; i < rows * (padded - groups); i += 256)
+        put_sums(a.y_sums + ((row0 + i / (padded - groups)) * padded + groups + i % (padded - groups)) * sum_slots(true), sum_slots(true), 0.f);
+  } else {
+    const bool inside = n0 + 64 * wave < N;  // (else the wave's columns repeat the last one)
+#pragma unroll
+    for (int m = 0; m < MS; ++m) {
+      turn(m, 0);
+      if (__builtin_expect(odd != odd, 0)) repair(m, m + 1, 32 * m);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 8 * i + (lane >> 3), tr = 32 * m + row;
+        const u32x4_t w = *reinterpret_cast<const u32x4_t *>(mine + row * ROWB + (lane & 7) * 16);
+        const uint32_t to = (uint32_t)__shfl((int)dst[m / 2], tr & 63, 64);
+        if (tr < rows && inside) *reinterpret_cast<u32x4_t *>(static_cast<uint16_t *>(a.y) + (int64_t)to * N + n0 + 64 * wave + 8 * (lane & 7)) = w;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  }
+}
+
 // One tile: 32 MS token rows from sorted row `row0` (`rows` of them real) x 32 WN NT weight rows from n0 of matrix e (GLU: of two matrices).
 // A wave owns 32 NT weight rows for all the tile's token rows.  K runs in stages of 64 bytes of codes a weight row; token rows and codes are
 // copied straight into a ring of S stages in LDS, the rows for all waves (one barrier a stage), the codes for the wave that
@@ -223,7 +490,7 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
 
   // ---- operands.  Offsets are 32 bits: the host takes this kernel for operands below 4 GiB only.
   const int64_t ebase = (int64_t)e * N;
-  const int ext = padded_groups(G) * kSlots;
+  const int ext = padded_groups(G) * sum_slots(P::kPlainCodes);
   const i32x4_t xr = words_of(a.x, (uint32_t)(a.x_rows * K * sizeof(T))), xsr = words_of(a.sums, (uint32_t)(a.x_rows * ext * 2));
   const T *s_of[NM], *b_of[NM];
   i32x4_t wr[NM], sr[NM], br[NM];
@@ -303,7 +570,7 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
     i32x4_t from;
 #pragma unroll
     for (int w = 0; w < 4; ++w) from[w] = bias ? xsr[w] : xr[w];
-    copy_to_lds(from, x_row[c] * (uint32_t)(bias ? ext * 2 : K * (int)sizeof(T)) + x_piece[c], bias ? (k >> glog) * 16 : k * (int)sizeof(T),
+    copy_to_lds(from, x_row[c] * (uint32_t)(bias ? ext * 2 : K * (int)sizeof(T)) + x_piece[c], bias ? (k >> glog) * (2 * sum_slots(P::kPlainCodes)) : k * (int)sizeof(T),
                 ring_at + slot * R::STAGE + (wave * R::XI + c) % XALL * 1024);
   };
   auto copy_weights = [&](int slot) __attribute__((always_inline)) {
@@ -333,7 +600,7 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
 #pragma unroll
       for (int t = 0; t < NT; ++t) sum[m][t] = zero;
 #pragma unroll 1
-    for (int i = 0; i < GB / 2; ++i) {
+    for (int i = 0; i < GB / 2 && !P::kPlainCodes; ++i) {
       const int g = 2 * i + kb;
       u32x4_t F[MS];
 #pragma unroll
@@ -357,7 +624,13 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
   };
   auto bias_stage = [&](int k, const unsigned char *at) __attribute__((always_inline)) {
     const int g0 = k >> glog, real = (k_end >> glog) - g0;  // (groups past the share's end are another share's)
-    if (in_place) {
+    if constexpr (P::kPlainCodes) {
+      const unsigned char *const mine = at + R::X + wave * R::W;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) *reinterpret_cast<u32x4_t *>(scales + t * 1024 + lane * 16) = *reinterpret_cast<const u32x4_t *>(mine + t * 1024 + lane * 16);
+      add_plain_biases<MS, NT>(tot, at, R::XROW, [&](int piece) __attribute__((always_inline)) { return (piece ^ turned(ln)) << 4; },
+                               mine + NT * 1024 + ln * 32, real, ln, kb);
+    } else if (in_place) {
       bias_product(at, real, [&](int t, int g, float &sv, float &bv) __attribute__((always_inline)) {
         const uint32_t from = first_scale[t] + g0 + (g < real ? g : 0);
         const T s1 = s_of[GLU ? t : 0][from];
@@ -516,6 +789,8 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
     wait_copies<0>();
     block_barrier();
   }
+  uint32_t dst[2] = {};
+  if constexpr (P::kPlainCodes && !GLU) output_rows(a, row0, rows, lane, dst);
   wait_copies<0>();
   block_barrier();
 
@@ -553,112 +828,236 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
     if (kg != 0) return;
   }
 
-  // ---- epilogue: a wave turns its 32 x 32 sub-tiles round in a private piece of LDS and stores 16 bytes a lane
-  constexpr int ROWB = 32 * (int)sizeof(T) + 16;
-  constexpr int PV = 16 / (int)sizeof(T);             // values per 16-byte piece
-  constexpr int CPR = 32 / PV;                        // pieces per row
-  constexpr int RPI = 64 / CPR;                       // rows one store instruction covers
-  unsigned char *const mine = lds_raw + wave * (32 * ROWB);
-  const int my_piece = lane % CPR, my_row = lane / CPR;
-  const bool vec = N % PV == 0;
-  // The gate/up tiles also sum their rows over the quantisation groups, which the down product's bias term wants (columns in whole blocks of 128:
-  // 32 of them here, the rest of a group in the waves beside).  A kernel over the finished rows took 5 us.
-  const bool sums_too = GLU && a.y_sums != nullptr;
-  float *const parts_of_sums = reinterpret_cast<float *>(lds_raw + WN * (32 * ROWB));  // [wave][row]
+  if constexpr (P::kPlainCodes) write_piece<GLU, MS>(a, tot, wave, lane, n0, row0, rows, ebase, weight_row, dst, lds_raw);
+  else write_tile<DT, BITS, GLU, MS, NT, WN>(a, tot, wave, lane, n0, col0, row0, rows, ebase, glog, weight_row, lds_raw);
+}
+
+
+// A tile of 65 to 128 token rows of a block with 4-bit codes in groups of 64: 32 MS rows x 256 weight rows by four waves, each of which owns 64 weight rows
+// (GLU: 32 gate and 32 up rows) for all the token rows.  What multiply_tile does, with the pipeline that so many sums a wave leave room for:
+//   token rows  two places of 64 K values, one barrier each; copied while the other place is multiplied;
+//   codes       two places of 128 K values, the wave's own; unpacked while the last token rows of the 64 values before are multiplied.
+// Two blocks share a CU and fill each other's waits.
+struct LongRing {
+  static constexpr int XROW = 128, W = 4096, WALL = 4 * W, WINDOWS = 4 * 2048;
+  static constexpr int bytes(int ms) { return 2 * (32 * ms * XROW) + 2 * WALL + WINDOWS + ms * 1024; }
+};
+template <bool GLU, int MS>
+__device__ __forceinline__ void multiply_long_tile(const CodesArgs &a, int e, int64_t row0, int rows, int n0, unsigned char *lds_raw) {
+  typedef Tile<0, 4, false, true, MS, 2, 4, 2> P;
+  typedef LongRing R;
+  constexpr int NM = GLU ? 2 : 1, X = 32 * MS * R::XROW, XI = MS;  // copies a wave makes of a place of token rows
+  const int lane = threadIdx.x & 63, ln = lane & 31, kb = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int N = a.N, K = a.K, G = K >> 6, row_bytes = K / 2, ext = padded_groups(G) * sum_slots(true);
+  const int64_t ebase = (int64_t)e * N;
+  const uint32_t ring_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds_raw;
+  unsigned char *const codes_at = lds_raw + 2 * X + wave * R::W, *const scales = lds_raw + 2 * X + 2 * R::WALL + wave * 2048;
+  const i32x4_t xr = words_of(a.x, (uint32_t)(a.x_rows * K * 2)), xsr = words_of(a.sums, (uint32_t)(a.x_rows * ext * 2));
+  i32x4_t wr[NM], sr[NM], br[NM];
 #pragma unroll
-  for (int u = 0; u < MS * (GLU ? 1 : NT); ++u) {
-    const int m = u / (GLU ? 1 : NT), t = u % (GLU ? 1 : NT), col = col0 + 32 * t;
-    const float lb = a.bias ? as_f32(static_cast<const T *>(a.bias)[col + ln < N ? col + ln : N - 1]) : 0.f;
-    auto put = [&](int r, float v, float up) __attribute__((always_inline)) {
-      if constexpr (GLU) v = v / (1.0f + __expf(-v)) * up;
-      T o = rounded<T>(v);
-      if (a.bias) o = rounded<T>(as_f32(o) + lb);
-      reinterpret_cast<T *>(mine + (8 * (r >> 2) + 4 * kb + (r & 3)) * ROWB)[ln] = o;
-    };
-    uint32_t again = 0;  // (bits: which of the sixteen sums are not finite)
+  for (int t = 0; t < NM; ++t) {
+    wr[t] = words_of((t ? a.w1 : a.w0) + ebase * (row_bytes / 4), (uint32_t)N * row_bytes);
+    sr[t] = words_of(static_cast<const uint16_t *>(t ? a.s1 : a.s0) + ebase * G, (uint32_t)N * G * 2);
+    br[t] = words_of(static_cast<const uint16_t *>(t ? a.b1 : a.b0) + ebase * G, (uint32_t)N * G * 2);
+  }
+  const int col0 = n0 + (GLU ? 32 : 64) * wave;
+  auto weight_row = [&](int t, int at) __attribute__((always_inline)) {
+    const int p = a.y_paired ? ((at & ~7) | (((at & 7) >> 1) + ((at & 1) ? 4 : 0))) : at, row = col0 + (GLU ? 0 : 32 * t) + p;
+    return row < N ? row : N - 1;
+  };
+  auto turned = [](int row) __attribute__((always_inline)) { return (row >> 1) & 7; };
+  uint32_t x_off[XI], w_off[4], window_row[2];
+  uint32_t *const sums_off = reinterpret_cast<uint32_t *>(lds_raw + 2 * X + 2 * R::WALL + R::WINDOWS) + wave * (64 * XI) + lane;  // (read once a window)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float v = tot[m][t][r], up = GLU ? tot[m][NT - 1][r] : 0.f;
-      put(r, v, up);
-      again |= (not_finite(v) || (GLU && not_finite(up)) ? 1u : 0u) << r;
+  for (int i = 0; i < XI; ++i) {
+    const int r = (wave * XI + i) * 8 + lane / 8, tr = r < rows ? r : rows - 1;  // rows past the end repeat the last one (never stored)
+    const uint32_t row = a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr), piece = (uint32_t)((lane % 8) ^ turned(r)) << 4;
+    x_off[i] = row * (uint32_t)(K * 2) + piece;
+    sums_off[64 * i] = row * (uint32_t)(ext * 2) + piece;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int at = 16 * (i & 1) + (lane >> 2);
+    w_off[i] = (uint32_t)weight_row(i / 2, at) * row_bytes + (((lane & 3) ^ ((at >> 2) & 3)) << 4);
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) window_row[t] = (uint32_t)weight_row(t, lane >> 1) * G * 2 + ((lane & 1) << 4);
+
+  // ---- copies.  K runs in windows of 16 groups; place 0 of a window is its bias product (group sums; scales and biases), then come its K values.
+  struct Next { int k, pos; } next_x = {0, 0}, next_w = {0, 0};
+  int xs = 0, ws = 0;  // the places being read
+  auto copy_rows = [&](int slot, auto sums_too) __attribute__((always_inline)) {  // sums_too: a window's group sums may be what comes next
+    const int k = next_x.k < K ? next_x.k : K - 64;  // (past the end the last ones again)
+    const bool sums = decltype(sums_too)::value && next_x.pos == 0;
+    i32x4_t from;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) from[w] = sums ? xsr[w] : xr[w];
+#pragma unroll
+    for (int c = 0; c < XI; ++c) {
+      uint32_t off = x_off[c];
+      if constexpr (decltype(sums_too)::value) {
+        const uint32_t other = sums_off[64 * c];
+        off = sums ? other : off;
+      }
+      copy_to_lds(from, off, sums ? (k >> 6) * 8 : k * 2, ring_at + slot * X + (wave * XI + c) * 1024);
     }
+    if (!sums) next_x.k += 64;
+    next_x.pos = next_x.pos == 16 ? 0 : next_x.pos + 1;
+  };
+  auto copy_weights = [&](int slot) __attribute__((always_inline)) {
+    const int k = next_w.k < K ? next_w.k : K - 128;
+    const bool bias = next_w.pos == 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // codes: two copies a tile; bias product: the tiles' scales, then their biases
+      i32x4_t from;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) from[w] = bias ? (i < 2 ? sr : br)[GLU ? i % 2 : 0][w] : wr[GLU ? i / 2 : 0][w];
+      copy_to_lds(from, bias ? window_row[i % 2] : w_off[i], bias ? (k >> 6) * 2 : k / 2, ring_at + 2 * X + slot * R::WALL + wave * R::W + i * 1024);
+    }
+    if (!bias) next_w.k += 128;
+    next_w.pos = next_w.pos == 8 ? 0 : next_w.pos + 1;
+  };
+
+  float tot[MS][2][16];
+#pragma unroll
+  for (int m = 0; m < MS; ++m)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) tot[m][t][v] = 0.f;
+  const f32x16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  f32x16_t acc[2] = {zero, zero};  // the group sums being multiplied, and those before them, which are still to be scaled
+  float pending_s = 0.f;
+  u32x4_t op[2][4], q[2][1];  // the codes of 64 K values as operands, and as they are
+  uint32_t xa[4], wa[2];
+#pragma unroll
+  for (int h = 0; h < 4; ++h) xa[h] = ln * R::XROW + (((4 * kb + h) ^ turned(ln)) << 4);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) wa[i] = ln * 64 + (((2 * i + kb) ^ ((ln >> 2) & 3)) << 4);
+  auto fetch_codes = [&](int slot, int half) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) q[t][0] = *reinterpret_cast<const u32x4_t *>(codes_at + slot * R::WALL + wa[half] + t * 2048);
+  };
+
+  // 64 K values: the token rows from place xs, the operands in registers; those of the 64 values behind are made on the way, from half next_half of
+  // place next_slot.  Program order is kept as it stands.
+  auto multiply = [&](int group, int next_slot, int next_half, auto await) __attribute__((always_inline)) {
+    const unsigned char *const at = lds_raw + xs * X;
+    u32x4_t F[4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) F[h] = *reinterpret_cast<const u32x4_t *>(at + xa[h]);
+    float s[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) s[t] = as_f32(*reinterpret_cast<const uint16_t *>(scales + t * 1024 + ln * 32 + group * 2));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < MS; ++m) {
+      if (m == MS - 1) {
+        await();
+        fetch_codes(next_slot, next_half);
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int cur = t, pm = t ? m : (m ? m - 1 : MS - 1), pt = t ^ 1;  // the pending sums' place
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          acc[cur] = mfma<0>(F[h], op[t][h], h ? acc[cur] : zero);
+#pragma unroll
+          for (int v = 4 * h; v < 4 * h + 4; ++v) tot[pm][pt][v] = __builtin_fmaf(pending_s, acc[cur ^ 1][v], tot[pm][pt][v]);
+          if (t == 1 && m + 1 < MS) F[h] = *reinterpret_cast<const u32x4_t *>(at + xa[h] + (m + 1) * (32 * R::XROW));
+          if (m == MS - 1) P::unpack(q[t], h, op[t][h]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        pending_s = s[t];
+      }
+    }
+  };
+  auto begin = [&](auto left) __attribute__((always_inline)) {  // what this step reads has arrived, in every wave, and the place copied to next is free
+    wait_copies<decltype(left)::value>();
+    block_barrier();
+  };
+  const std::integral_constant<int, 0> all{};
+  const std::integral_constant<int, 4> but_codes{};
+
+  const std::true_type yes{};
+  const std::false_type no{};
+  copy_rows(0, yes);
+  copy_weights(0);
+  for (int k = 0; k < K;) {
+    const int k_window = k, k_last = k + 1024 < K ? k + 1024 : K;
+    begin(all);
+    copy_rows(xs ^ 1, no);
+    copy_weights(ws ^ 1);
+    {
+      const unsigned char *const mine = codes_at + ws * R::WALL;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) *reinterpret_cast<u32x4_t *>(scales + t * 1024 + lane * 16) = *reinterpret_cast<const u32x4_t *>(mine + t * 1024 + lane * 16);
+      add_plain_biases<MS, 2>(tot, lds_raw + xs * X, R::XROW, [&](int piece) __attribute__((always_inline)) { return (piece ^ turned(ln)) << 4; },
+                              mine + 2048 + ln * 32, (K - k) >> 6, ln, kb);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    xs ^= 1;
+    ws ^= 1;
+    wait_copies<0>();  // (this wave's codes: unpacked ahead of the barrier)
+    fetch_codes(ws, 0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int h = 0; h < 4; ++h) P::unpack(q[t], h, op[t][h]);
 #pragma unroll 1
-    for (int quad = 0; __builtin_expect(again != 0, 0); ++quad, again >>= 4) {  // rows 8 quad + 4 kb + 0 .. 3
-      uint32_t open = again & 15u;
-      const T *xs[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        int tr = 32 * m + 8 * quad + 4 * kb + i;
-        if (tr >= rows) {  // (never stored)
-          open &= ~(1u << i);
-          tr = rows - 1;
-        }
-        xs[i] = static_cast<const T *>(a.x) + (int64_t)(a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr)) * K;
-      }
-      if (!open) continue;
-      float v[GLU ? 2 : 1][4];
-#pragma unroll
-      for (int i = 0; i < (GLU ? 2 : 1); ++i) {
-        const int64_t wrow = ebase + weight_row(GLU ? i : t, ln);
-        plain_rows<BITS, 4, T>(xs, paired_order(BITS), (GLU && i ? a.w1 : a.w0) + wrow * (row_bytes / 4),
-                               static_cast<const T *>(GLU && i ? a.s1 : a.s0) + wrow * G,
-                               static_cast<const T *>(GLU && i ? a.b1 : a.b0) + wrow * G, K, K / G, open, v[i]);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (open >> i & 1u) put(4 * quad + i, v[0][i], v[GLU ? 1 : 0][i]);
+    for (; k < k_last; k += 128) {
+      begin(all);
+      copy_rows(xs ^ 1, no);
+      copy_weights(ws ^ 1);
+      multiply((k - k_window) >> 6, ws, 1, [] {});
+      xs ^= 1;
+      begin(but_codes);
+      copy_rows(xs ^ 1, yes);
+      multiply(((k - k_window) >> 6) + 1, ws ^ 1, 0, [&]() __attribute__((always_inline)) {  // the next codes were asked for before the rows
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(XI) : "memory");
+      });
+      xs ^= 1;
+      ws ^= 1;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int my_col = col + PV * my_piece;
+    // (the window's last sums ahead of the next one's bias product: every sum in the order of multiply_tile, wherever its row stands)
 #pragma unroll
-    for (int i = 0; i < 32 / RPI; ++i) {
-      const int row = RPI * i + my_row;
-      const int tr = 32 * m + row;
-      if (tr < rows && my_col < N) {
-        const int64_t dst = a.dst_rows ? (int64_t)a.dst_rows[row0 + tr] : row0 + tr;
-        T *const to = static_cast<T *>(a.y) + dst * N + my_col;
-        const T *const from = reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece;
-        if (vec) {
-          *reinterpret_cast<u32x4_t *>(to) = *reinterpret_cast<const u32x4_t *>(from);
-        } else {
-          for (int c = 0; c < PV && my_col + c < N; ++c) to[c] = from[c];
-        }
-      }
-      if constexpr (GLU) {
-        if (sums_too) {
-          const u32x4_t w = *reinterpret_cast<const u32x4_t *>(reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece);
-          float sum = ((bf16lo_to_f32(w[0]) + bf16hi_to_f32(w[0])) + (bf16lo_to_f32(w[1]) + bf16hi_to_f32(w[1]))) +
-                      ((bf16lo_to_f32(w[2]) + bf16hi_to_f32(w[2])) + (bf16lo_to_f32(w[3]) + bf16hi_to_f32(w[3])));
-          sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
-          sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
-          if (my_piece == 0) parts_of_sums[wave * (32 * MS) + tr] = sum;
-        }
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int v = 0; v < 16; ++v) tot[MS - 1][1][v] = __builtin_fmaf(pending_s, acc[1][v], tot[MS - 1][1][v]);
+    pending_s = 0.f;
   }
-  if constexpr (GLU) {
-    static_assert(KW == 1 && DT == 0 && WN == 4, "every wave comes here; four waves cover a group of 128");
-    if (!sums_too) return;
-    __syncthreads();
-    const int first = n0 >> glog, groups = N >> glog, here = 128 >> glog, waves = 1 << (glog - 5);  // (the output's groups are as long as the input's)
-    const int end = first + here >= groups ? padded_groups(groups) : first + here;  // the last block writes the zeros behind
-    for (int i = threadIdx.x; i < rows * (end - first); i += 64 * WN) {
-      const int row = i % rows, g = i / rows;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (first + g < groups) {
-        float sum = 0.f;
-        for (int w = 0; w < waves; ++w) sum += parts_of_sums[(g * waves + w) * (32 * MS) + row];
-        const Pieces p = split3(sum);
-        v = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, 0u);
-      }
-      reinterpret_cast<uint4 *>(a.y_sums)[(row0 + row) * padded_groups(groups) + first + g] = v;
-    }
-  }
+  uint32_t dst[2] = {};
+  if constexpr (!GLU) output_rows(a, row0, rows, lane, dst);
+  wait_copies<0>();
+  block_barrier();
+  write_piece<GLU, MS>(a, tot, wave, lane, n0, row0, rows, ebase, weight_row, dst, lds_raw);
+}
+
+// The tiles of a list of pieces of up to 128 rows (ShortTiles::piece), 4-bit codes in groups of 64: by their rows, 32 at a time.
+// Ids are dealt round-robin over the 8 XCDs: `run` tiles that follow each other in the list, often one expert's, share an XCD, and
+// their blocks of one stretch of weight rows stand side by side, so that its L2 serves the weights to all but the first.
+constexpr int kPieceTiles = 1;
+template <bool GLU>
+__global__ __launch_bounds__(256, 2) void qmm_pieces_kernel(CodesArgs a, const uint32_t *__restrict__ list, int n_ntiles) {
+  constexpr int NI = GLU ? 128 : 256;
+  const uint32_t xcd = blockIdx.x & 7, j = blockIdx.x >> 3, per_run = (uint32_t)n_ntiles * kPieceTiles;
+  const uint32_t id = (j / per_run * 8u + xcd) * kPieceTiles + j % kPieceTiles;
+  const int nt = (int)(j % per_run / kPieceTiles);
+  if (id >= list[0]) return;
+  const uint4 rec = reinterpret_cast<const uint4 *>(list)[1 + id];
+  const int e = __builtin_amdgcn_readfirstlane((int)rec.x), rows = __builtin_amdgcn_readfirstlane((int)rec.z);
+  const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane((int)rec.y);
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  if (rows > 96) return multiply_long_tile<GLU, 4>(a, e, row0, rows, nt * NI, lds_raw);
+  if (rows > 64) return multiply_long_tile<GLU, 3>(a, e, row0, rows, nt * NI, lds_raw);
+  if (rows > 32) return multiply_tile<0, 4, false, GLU, true, 2, 2, 4, 1, 2>(a, e, row0, rows, nt * NI, 0, lds_raw);
+  typedef Ring<4, 1, 2, 4, 2> Short;
+  constexpr int S1 = (kHalfLds - 4 * Short::WINDOW) / Short::STAGE;  // as many stages as fit
+  multiply_tile<0, 4, false, GLU, true, 1, 2, 4, 1, S1>(a, e, row0, rows, nt * NI, 0, lds_raw);
 }
 
 // A block computes 32 MS token rows x 32 WN weight rows with WN KW waves (see codes_tile), tiles of up to 32 rows with half the
@@ -704,16 +1103,16 @@ __global__ __launch_bounds__(64 * WN * KW, waves_of(WN * KW, lds_of(KW, Ring<BIT
 size_t codes_copy_bytes(int bits, int64_t rows, int K) {
   return paired_order(bits) ? (size_t)rows * K * 2 : 0;
 }
-size_t codes_sums_bytes(int64_t rows, int K, int group) { return (size_t)rows * padded_groups(K / group) * kSlots * 2; }
+size_t codes_sums_bytes(int64_t rows, int K, int group, bool plain) { return (size_t)rows * padded_groups(K / group) * sum_slots(plain) * 2; }
 
 hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
-                               uint16_t *sums, hipStream_t st) {
+                               uint16_t *sums, bool plain, hipStream_t st) {
   const int64_t n = rows * (K / 8);
   if (n == 0) return hipSuccess;
   const unsigned grid = (unsigned)((n + 255) / 256);
-  const int ll = group == 32 ? 2 : (group == 64 ? 3 : 4), row = padded_groups(K / group) * kSlots;
-  if (dt == 0) prepare_rows_kernel<0><<<grid, 256, 0, st>>>(static_cast<const uint16_t *>(x), n, K / 8, ll, copy, sums, row);
-  else if (dt == 1) prepare_rows_kernel<1><<<grid, 256, 0, st>>>(static_cast<const _Float16 *>(x), n, K / 8, ll, copy, sums, row);
+  const int ll = group == 32 ? 2 : (group == 64 ? 3 : 4), slots = sum_slots(plain), row = padded_groups(K / group) * slots;
+  if (dt == 0) prepare_rows_kernel<0><<<grid, 256, 0, st>>>(static_cast<const uint16_t *>(x), n, K / 8, ll, copy, sums, row, slots);
+  else if (dt == 1) prepare_rows_kernel<1><<<grid, 256, 0, st>>>(static_cast<const _Float16 *>(x), n, K / 8, ll, copy, sums, row, slots);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
@@ -765,24 +1164,41 @@ static hipError_t start_dense(const CodesArgs &a, int group, hipStream_t st) {
   return hipErrorInvalidValue;
 }
 
+// The tiles of a list of pieces in one launch (see qmm_pieces_kernel).
+template <bool GLU>
+static hipError_t start_pieces(const CodesArgs &a, const uint32_t *list, int cap, hipStream_t st) {
+  constexpr int NI = GLU ? 128 : 256, lds = kHalfLds;
+  static_assert(LongRing::bytes(4) <= lds && Ring<4, 2, 2, 4, 2>::BYTES <= lds, "two blocks share a CU");
+  const int n_ntiles = (a.N + NI - 1) / NI;
+  const int64_t grid = ((int64_t)cap + 8 * kPieceTiles - 1) / (8 * kPieceTiles) * (8 * kPieceTiles) * n_ntiles;
+  if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
+  static std::atomic<uint64_t> allowed{0};
+  if (hipError_t e = allow_lds(reinterpret_cast<const void *>(&qmm_pieces_kernel<GLU>), lds, allowed); e != hipSuccess) return e;
+  launch_or_time(&qmm_pieces_kernel<GLU>, dim3((unsigned)grid), dim3(256), lds, st, a, list, n_ntiles);
+  return hipGetLastError();
+}
+hipError_t launch_qmm_pieces(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st) {
+  return glu ? start_pieces<true>(a, list, cap, st) : start_pieces<false>(a, list, cap, st);
+}
+
 // The tiles of a list in one launch: 64 rows x 256 weight rows (128 gate and the matching 128 up ones), two blocks a CU.
 // Groups of 32, 512 tokens and even routing (128 experts, hidden 2048), us of gate/up / down: 107 / 57; tiles of 64 x 128 with the codes loaded into
 // registers, gate and up in one wave, 121 / 77.  One tile a wave in eight waves: 20 % slower; blocks of two waves, or of one CU each with more stages: slower.
 hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st) {
-  auto run = [&](auto b, auto g32, auto mid) {
+  auto run = [&](auto b, auto g32) {
     constexpr int BITS = decltype(b)::value;
-    constexpr bool G32 = decltype(g32)::value, MID = decltype(mid)::value;
-    if (glu) return start_tiles<0, BITS, G32, true, MID, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
-    return start_tiles<0, BITS, G32, false, MID, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
+    constexpr bool G32 = decltype(g32)::value;
+    if (glu) return start_tiles<0, BITS, G32, true, false, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
+    return start_tiles<0, BITS, G32, false, false, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
   };
   const std::true_type yes{};
   const std::false_type no{};
   if (bits == 4) {
     const std::integral_constant<int, 4> b{};
-    return group == 32 ? run(b, yes, no) : group == 64 ? run(b, no, yes) : run(b, no, no);
+    return group == 32 ? run(b, yes) : run(b, no);
   }
   const std::integral_constant<int, 8> b{};
-  return group == 32 ? run(b, yes, no) : run(b, no, no);
+  return group == 32 ? run(b, yes) : run(b, no);
 }
 
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st) {

@@ -41,6 +41,37 @@ def test_blocks_in_short_tiles(zipf, rows, hidden, inter, experts, k):
         assert torch.equal(blk.forward_static(x), out)
 
 
+# an average of 97 rows and more: K of one window of sixteen groups and of two, h of more groups than a window, fewer columns than a block's
+@pytest.mark.parametrize("hidden,inter,experts,k", [(128, 384, 8, 2), (1152, 1280, 9, 3), (256, 128, 64, 2)])
+@pytest.mark.parametrize("rows", [70, 97, 128, 300])
+@pytest.mark.parametrize("zipf", [None, 1.4])
+def test_blocks_in_longer_pieces(zipf, rows, hidden, inter, experts, k):
+    """Pieces of 96 and 128 rows (70 rows an expert; beyond 96 with the segments of fewer than nine rows streamed beside them) and their last ones of every
+    length, with the bound of test_blocks_in_short_tiles: the same roundings.  The scratch that is built in, the residual form and a
+    workspace that ends before the sums' own places take the same tiles."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    tokens = rows * experts // k
+    cfg = m.MoeConfig(hidden, experts, k, inter, 4, 64, 0)
+    assert m.capi.tile_rule(cfg.c_struct(), tokens) == ((2, 1) if rows <= 96 else (3, 9))
+    blk = synth.make_block(cfg, seed=rows, device="cuda", zipf_s=zipf, gen_device="cuda")
+    x = synth.make_tokens(cfg, tokens, seed=k, device="cuda")
+    out, routing = blk.forward(x, debug=True)
+    ref = block_truth(blk, x, routing)
+    assert float((out.double() - ref).norm() / ref.norm()) <= 2.0 ** -8
+    rms = ref.square().mean(1).sqrt()  # (a row in another's place would be as far off as itself)
+    assert float(((out.double() - ref).norm(dim=1) / (rms * hidden ** 0.5)).max()) <= 2.0 ** -6
+    p = torch.randperm(tokens, generator=torch.Generator().manual_seed(3)).cuda()
+    assert torch.equal(blk.forward(x[p].contiguous()), out[p])
+    if blk.workspace_bytes(tokens) < 8 << 20:
+        assert torch.equal(blk.forward_static(x), out)
+    one = torch.ones(hidden, dtype=torch.bfloat16, device="cuda")
+    xn = m.ops.rms_norm(x, one, 1e-6)
+    own, routing = blk.forward_residual(x, one, 1e-6, debug=True)
+    ref = x.double() + block_truth(blk, xn, routing)
+    assert float((own.double() - ref).norm() / ref.norm()) <= 2.0 ** -8
+
+
 def test_a_layer_around_short_tiles():
     """The normalised rows' memory takes the group sums of h once they have been read: the residual form against its parts."""
     import mlx_rs_amd as m
