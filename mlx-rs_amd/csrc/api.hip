@@ -129,6 +129,7 @@ struct ForwardWs {
   uint16_t *gu;  // plain products only: the gate and the up product, [P, I] each
   bool mid;             // groups of 64: all segments in pieces on raw codes (see mid_batch)
   bool pieces;          // the same tiles for the segments of a heavy batch that are tiled, the others streamed
+  bool raw_all;         // groups of 32 / 128: all segments in tiles (see raw_all_tiles)
   bool raw;             // group sizes 32 / 128: the products on raw codes (qmm_rows, qmm_codes)
   uint32_t *raw_tiles;  // the short tiles of qmm_codes, the paired copy of x (4-bit) and the group sums of x and h, or nullptr:
   int raw_cap;          // (groups of 32 / 128) all segments go through the kernel of a few rows, in as many passes as they need
@@ -154,18 +155,24 @@ bool codes_tiles_fit(const mi_moe_config &c, int64_t T) {
 bool raw_tiled_batch(const mi_moe_config &c, int64_t T) {
   return T > kRowsMost && T * c.top_k >= (int64_t)4 * c.n_experts && codes_tiles_fit(c, T);
 }
-// Groups of 32, 4-bit codes: below sixteen rows an expert on average those tiles have their codes in registers (qmm_codes.hip).  A block of the others
-// takes half of a CU's LDS and waits for it behind the short segments' blocks, which fill what falls free.  Measured, us of a forward, registers / LDS,
-// at an average of 5, 8, 12, 14, 16, 19.5 rows (experts, k, hidden, intermediate):
-//   128, 8, 2048, 768   Zipf-1.1 119, 124, 128, 135, 143, 158 / 141, 143, 148, 155, 157, 157; 1.3 116, 122, 126, 134, 134, 151 / 119, 121, 148, 153, 155, 158;
-//                       even 157, 166, 178, 194, 191, 234 / 148, 157, 186, 183, 181, 205
-//   64, 6, 2048, 1408   Zipf-1.1 110, 128, 131, 154, 159, 161 / 142, 152, 152, 158, 158, 161; 1.3 111, 119, 119, 145, 146, 149 / 141, 149, 150, 154, 155, 159;
-//                       even 143, 160, 183, 182, 185, 215 / 142, 159, 180, 186, 178, 201
-//   128, 8, 4096, 1536  Zipf-1.1 388, 460, 517, 571, 571, 632 / 421, 487, 550, 608, 614, 664; 1.3 344, 388, 432, 460, 459, 528 / 367, 420, 466, 497, 511, 558;
-//                       even 682, 748, 803, 782, 722, 672 / 682, 749, 818, 792, 722, 603
-//   8, 2, 4096, 7168    Zipf-1.1 at 5, 8, 12, 14 rows 234, 354, 335, 336 / 232, 311, 314, 380; even 228, 252, 359, 372 / 230, 252, 380, 341
-// 8-bit codes, and groups of 128, are faster in LDS at nearly all of these (0.94 to 1.35 times).
-bool raw_tiles_in_registers(const mi_moe_config &c, int64_t P) { return c.group_size == 32 && c.bits == 4 && P < (int64_t)16 * c.n_experts; }
+// Batches of those sizes whose segments all go through the tiles, in one launch a product on the caller's stream.  The others (8-bit codes, twenty to forty
+// rows an expert) keep the short segments on the kernel of a few rows, beside the tiles on a side stream: with skewed routing that is 1 to 12 % faster
+// there, with even routing 7 to 15 % slower.  Measured, us of a forward, side by side / all in tiles, at an average of 5, 8, 12, 16, 24, 32, 48, 96 rows
+// (experts, k, hidden, intermediate, bits, group; below sixteen rows with 4-bit codes in groups of 32 the other tiles had their codes in registers):
+//   128, 8, 2048, 768, 4, 32   even 155, 169, 182, 183, 198, 211, 247, 357 / 151, 151, 153, 155, 166, 186, 226, 335; Zipf-1.1 126, 131, 135, 164, 166, 184, 238,
+//                              359 / 108, 113, 126, 144, 168, 185, 217, 336; 1.3 121, 129, 131, 160, 158, 177, 225, 346 / 91, 110, 116, 125, 156, 174, 210, 309
+//   128, 8, 2048, 768, 4, 128  even 139, 150, 157, 168, 158, 171, 199, 280 / 118, 119, 123, 124, 133, 144, 169, 256; Zipf-1.1 118, 122, 128, 138, 138, 153, 194,
+//                              282 / 84, 89, 101, 109, 129, 143, 173, 262
+//   64, 6, 2048, 1408, 4, 32   Zipf-1.1 120, 135, 135, 162, 177, 187, 225, 333 / 121, 129, 148, 157, 164, 189, 224, 315; even 143, 165, 181, 192, 182, 190, 224, 318 /
+//                              143, 142, 143, 144, 153, 173, 196, 298
+//   8, 2, 4096, 7168, 4, 32    even 229, 252, 304, 319, 259, 295, 297, 407 / 207, 207, 208, 208, 219, 270, 272, 385; Zipf-1.1 234, 352, 340, 382, 384, 356, 416,
+//                              403 / 207, 207, 208, 258, 270, 331, 367, 385
+//   128, 8, 2048, 768, 8, 32   Zipf-1.1 144, 167, 171, 181, 196, 224, 280, 406 / 123, 125, 146, 184, 207, 229, 271, 396; 1.3 133, 144, 160, 176, 178, 208, 272, 387 /
+//                              108, 121, 129, 147, 198, 213, 255, 360
+bool raw_all_tiles(const mi_moe_config &c, int64_t T) {
+  const int64_t P = T * c.top_k, E = c.n_experts;
+  return raw_tiled_batch(c, T) && (c.bits == 4 || P < 20 * E || P >= 40 * E);
+}
 // Groups of 64, 4-bit codes: batches whose segments all go through short tiles on raw codes, in one launch a product on the caller's
 // stream (the others: streamed segments, and tiles of 256 weight rows on side streams).  From the batches on for which the tile lists
 // are built and the router has kernels of its own, up to 96 rows per expert on average.  Measured, us of a forward, other route / this one:
@@ -252,7 +259,8 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
     const size_t list = short_list_words(f.raw_cap), xsums = codes_sums_bytes(T, c.hidden, c.group_size, true), hsums = codes_sums_bytes(P, c.intermediate, c.group_size, true);
     f.raw_tiles = list <= (size_t)c.n_experts * 16 ? f.work : cv.take<uint32_t>(list);
     f.raw_copy = f.xperm;
-    f.raw_xsums = xsums <= (size_t)P * c.hidden * 2 ? f.y : cv.take<uint16_t>(xsums / 2);
+    const size_t hist = align_up(dispatch_workspace_bytes(c.n_experts, P));  // (which are read while the sums are made)
+    f.raw_xsums = hist + xsums <= (size_t)P * c.hidden * 2 ? f.y + hist / 2 : cv.take<uint16_t>(xsums / 2);
     f.raw_hsums = hsums <= (size_t)T * c.hidden * 2 ? f.xnorm : cv.take<uint16_t>(hsums / 2);
   }
   if (f.pieces) {
@@ -267,7 +275,9 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
     f.raw_xsums = in_norm ? f.xnorm : cv.take<uint16_t>(xsums / 2);
     f.raw_hsums = in_norm ? f.xnorm + xsums / 2 : cv.take<uint16_t>(hsums / 2);
   }
+  f.raw_all = f.raw && raw_all_tiles(c, T);
   if (f.raw && raw_tiled_batch(c, T)) {
+    if (f.raw_all) f.raw_from = 1;
     f.raw_cap = short_list_cap(P, c.n_experts, f.raw_from, f.raw_piece);
     f.raw_tiles = cv.take<uint32_t>(short_list_words(f.raw_cap));
     f.raw_copy = cv.take<uint16_t>(codes_copy_bytes(c.bits, T, c.hidden) / 2);
@@ -503,7 +513,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     return fail("forward: workspace too small (%zu bytes, need %zu)", workspace_bytes, f.bytes);
   if (workspace_bytes < f.bytes_raw) {
     f.raw_tiles = nullptr;
-    f.mid = f.pieces = false;
+    f.mid = f.pieces = f.raw_all = false;
   }
   if (workspace_bytes < f.bytes) f.router_scratch = nullptr;  // room for everything but the byte planes: fp64 logits, same bits
   int stage = 0;
@@ -564,7 +574,9 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
       MI_STAGE_DONE();
     }
     MI_HIP(launch_dispatch(f.topk_idx, P, c.n_experts, c.top_k, f.counts, f.offsets, f.perm, f.inv_perm,
-                           f.src_of, records, tile_lists, tile_cap, tile_from, shorts, f.disp_scratch, st));
+                           f.src_of, records, tile_lists, tile_cap, tile_from, shorts,
+                           raw_codes || f.raw_all ? prepare_args(x, T, c.hidden, c.group_size, codes_copy_bytes(c.bits, T, c.hidden) ? f.raw_copy : nullptr, f.raw_xsums, raw_codes)
+                                                  : PrepareArgs{}, f.disp_scratch, st));
     MI_STAGE_DONE();
   }
   GroupedArgs a{}, d{};
@@ -573,7 +585,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   if (f.tiled && paired && !streamed_first && !pair_in_router && !raw_codes) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));
   // independent chains run beside each other where side streams are to be had, whose lock is held until they have been joined back
   std::unique_lock<std::mutex> streams_guard;
-  const bool chains = !ev && !mid && (f.raw ? f.raw_tiles != nullptr : !plain_config(c) && (f.pieces || large_qmm_applies(a)));
+  const bool chains = !ev && !mid && !f.raw_all && (f.raw ? f.raw_tiles != nullptr : !plain_config(c) && large_qmm_applies(a));
   if (chains) streams_guard = std::unique_lock<std::mutex>(h->streams->lock);
   const bool fork = chains && may_fork(st, *h->streams);
   if (!fork && streamed_first && paired && large_qmm_applies(a)) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));  // (a side stream's work)
@@ -587,9 +599,8 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   ca.w0 = h->w.gate.w; ca.s0 = h->w.gate.scales; ca.b0 = h->w.gate.biases;
   ca.w1 = h->w.up.w; ca.s1 = h->w.up.scales; ca.b1 = h->w.up.biases;
   ca.y = f.hh;
-  ca.y_paired = copied;
-  const bool in_registers = f.raw && raw_tiles_in_registers(c, P);
-  ca.y_sums = in_registers ? nullptr : f.raw_hsums;
+  ca.y_order = !copied ? RowOrder::kPlain : raw_codes ? RowOrder::kQuads : RowOrder::kPaired;
+  ca.y_sums = f.raw_hsums;
   ca.N = c.intermediate; ca.K = c.hidden;
   cd.x = f.hh;
   cd.x_rows = P;
@@ -599,20 +610,14 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   cd.y = f.y;
   cd.N = c.hidden; cd.K = c.intermediate;
   auto prepare_x = [&](hipStream_t s) -> hipError_t {
-    return launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, raw_codes, s);
+    return launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, false, s);
   };
   auto tiles_up = [&](hipStream_t s) -> hipError_t {
     if (raw_codes) return launch_qmm_pieces(ca, f.raw_tiles, f.raw_cap, true, s);
-    if (in_registers) return launch_qmm_codes_list(ca, f.raw_tiles, f.raw_cap, true, s);
     return launch_qmm_codes_tiles(ca, f.raw_tiles, f.raw_cap, c.group_size, c.bits, true, s);
   };
   auto tiles_down = [&](hipStream_t s) -> hipError_t {
     if (raw_codes) return launch_qmm_pieces(cd, f.raw_tiles, f.raw_cap, false, s);
-    if (in_registers) {
-      // (the sums of all rows of h: those of the short segments, which another stream may still be writing, are not read)
-      const hipError_t e = launch_prepare_rows(f.hh, P, c.intermediate, c.group_size, MI_MOE_DTYPE_BF16, nullptr, f.raw_hsums, false, s);
-      return e != hipSuccess ? e : launch_qmm_codes_list(cd, f.raw_tiles, f.raw_cap, false, s);
-    }
     return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.group_size, c.bits, false, s);
   };
   struct TimerScope {  // a timer never outlives the launch it is meant for
@@ -620,7 +625,6 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     ~TimerScope() { g_kernel_timer = nullptr; }
   };
   if (mid) {
-    MI_HIP(prepare_x(st));
     {
       TimerScope scope(kt ? &kt[2] : nullptr);
       MI_HIP(tiles_up(st));
@@ -631,35 +635,24 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
       MI_HIP(tiles_down(st));
     }
     MI_STAGE_DONE();
-  } else if (f.pieces && fork) {
-    // The tiles here, the streamed segments beside them: they share no rows, and what streams waits for memory while the tiles multiply.
-    DeviceStreams &ds = *h->streams;
-    hipStream_t s = ds.side[0];
-    MI_HIP(hipEventRecord(ds.fork, st));
-    MI_HIP(hipStreamWaitEvent(s, ds.fork, 0));
-    hipError_t e = prepare_x(st);
-    if (e == hipSuccess) e = tiles_up(st);
-    if (e == hipSuccess) e = tiles_down(st);
-    if (e == hipSuccess) e = launch_small_qmm(a, true, s);
-    if (e == hipSuccess) e = launch_small_qmm(d, false, s);
-    // whatever happened: the caller's stream waits for what the side stream was given
-    hipError_t je = hipEventRecord(ds.join[0], s);
-    if (je == hipSuccess) je = hipStreamWaitEvent(st, ds.join[0], 0);
-    MI_HIP(e);
-    MI_HIP(je);
   } else if (f.pieces) {
-    MI_HIP(prepare_x(st));
     for (int half = 0; half < 2; ++half) {
-      {
-        TimerScope scope(kt ? &kt[4 * half + 2] : nullptr);
-        MI_HIP(half == 0 ? tiles_up(st) : tiles_down(st));
-      }
       {
         TimerScope scope(kt ? &kt[4 * half + 3] : nullptr);
         MI_HIP(launch_small_qmm(half == 0 ? a : d, half == 0, st));
       }
+      {
+        TimerScope scope(kt ? &kt[4 * half + 2] : nullptr);
+        MI_HIP(half == 0 ? tiles_up(st) : tiles_down(st));
+      }
       MI_STAGE_DONE();
     }
+  } else if (f.raw_all) {
+    if (fused_router) MI_HIP(prepare_x(st));
+    MI_HIP(tiles_up(st));
+    MI_STAGE_DONE();
+    MI_HIP(tiles_down(st));
+    MI_STAGE_DONE();
   } else if (f.raw) {
     // group sizes 32 / 128: short segments on the kernel of a few rows, longer ones (where lists are built) in tiles
     RowsArgs ra{}, rd{};
@@ -680,24 +673,17 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     rd.y = f.y;
     rd.N = c.hidden; rd.K = c.intermediate;
     if (fork) {
-      // The two chains share no rows.  The tiles run on a side stream beside the short segments: which of the two is the
-      // longer depends on the routing, and with even routing one of them is all but empty.  Measured, 128-expert shape,
-      // groups of 32, us of a forward at 64 / 96 / 128 / 200 / 512 tokens:
-      //   all segments through the kernel of a few rows  even 125 / 137 / 146 / 181 / 328   Zipf-1.1 183 / 256 / 324 / 458 / 1017
-      //   one chain after the other                           145 / 153 / 178 / 224 / 252            171 / 221 / 236 / 246 / 310
-      //   side by side                                        148 / 158 / 174 / 198 / 263            152 / 177 / 198 / 224 / 274
-      // (the plain kernels, which these shapes ran on before: 5630 at 512 tokens; with centred codes side by side, even, 512 tokens: 251)
+      // The two chains share no rows (which batches come here: raw_all_tiles): the short segments beside the tiles, which are the longer chain as far as the
+      // host can tell.  All segments through the kernel of a few rows: 328 us for 512 tokens and even routing, Zipf-1.1 1017 (128 experts, groups of 32).
       DeviceStreams &ds = *h->streams;
       hipStream_t s = ds.side[0];
       MI_HIP(hipEventRecord(ds.fork, st));
       MI_HIP(hipStreamWaitEvent(s, ds.fork, 0));
-      const bool tiles_lead = P >= (int64_t)20 * c.n_experts;  // the longer chain, as far as the host can tell, stays here
-      const hipStream_t ts = tiles_lead ? st : s, rs = tiles_lead ? s : st;
-      hipError_t e = prepare_x(ts);
-      if (e == hipSuccess) e = tiles_up(ts);
-      if (e == hipSuccess) e = tiles_down(ts);
-      if (e == hipSuccess) e = launch_qmm_rows(ra, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true, rs);
-      if (e == hipSuccess) e = launch_qmm_rows(rd, c.group_size, c.bits, MI_MOE_DTYPE_BF16, false, rs);
+      hipError_t e = prepare_x(st);
+      if (e == hipSuccess) e = tiles_up(st);
+      if (e == hipSuccess) e = tiles_down(st);
+      if (e == hipSuccess) e = launch_qmm_rows(ra, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true, s);
+      if (e == hipSuccess) e = launch_qmm_rows(rd, c.group_size, c.bits, MI_MOE_DTYPE_BF16, false, s);
       // whatever happened: the caller's stream waits for what the side stream was given
       hipError_t je = hipEventRecord(ds.join[0], s);
       if (je == hipSuccess) je = hipStreamWaitEvent(st, ds.join[0], 0);
@@ -1030,7 +1016,7 @@ int mi_moe_dispatch(const uint32_t *expert_of_pair, int64_t P, int32_t n_experts
   void *scratch = workspace_bytes < need ? nullptr : cv.take<char>(dispatch_workspace_bytes(n_experts, P));
   hipStream_t st = static_cast<hipStream_t>(stream);
   MI_HIP(launch_dispatch(expert_of_pair, P, n_experts, 1, counts, offsets, perm, inv_perm, nullptr, nullptr,
-                         nullptr, 0, 0, ShortTiles{}, scratch, st));
+                         nullptr, 0, 0, ShortTiles{}, PrepareArgs{}, scratch, st));
   return 0;
 } MI_CATCH("dispatch")
 
@@ -1108,7 +1094,7 @@ static int gather_qmm_impl(const void *x, const uint32_t *w, const void *scales,
   uint32_t *src_rows = cv.take<uint32_t>((size_t)rows);
   uint32_t *dst_rows = cv.take<uint32_t>((size_t)rows);
   MI_HIP(launch_dispatch(rhs_indices, n_idx, n_experts, 1, counts, offsets, perm, nullptr, nullptr, work,
-                         nullptr, 0, 0, ShortTiles{}, scratch, st));
+                         nullptr, 0, 0, ShortTiles{}, PrepareArgs{}, scratch, st));
   MI_HIP(launch_row_maps(perm, lhs_indices, n_lhs, offsets, n_idx, M, n_experts, src_rows, dst_rows, work, st));
   GroupedArgs a{};
   a.x = static_cast<const uint16_t *>(x);

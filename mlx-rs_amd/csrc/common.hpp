@@ -308,13 +308,33 @@ hipError_t launch_router_select(const uint16_t *logits, int64_t T, int E, int k,
 size_t dispatch_workspace_bytes(int E, int64_t P);
 // what the dispatch of P pairs can do with: up to 4096 one block of its own takes them where there is no scratch (nullptr)
 size_t dispatch_workspace_least(int E, int64_t P);
+// prepare: bf16 rows that are made ready beside it, by blocks of their own
+struct PrepareArgs;
 hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, uint32_t *counts,
                            uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
                            uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, int big_thr,
-                           ShortTiles shorts, void *scratch, hipStream_t st);
+                           ShortTiles shorts, const PrepareArgs &prepare, void *scratch, hipStream_t st);
 // decode-sized batches: logits + selection + dispatch in one launch.  counters: 1 +
 // kFusedRouterMaxTokens zero-initialised words that the kernel leaves zeroed again.  norm_w != nullptr:
 // the rows are RMS-normalised first (weight norm_w, eps) and kept in xnorm.
+// The order of the values of every 8-block of a row of activations: as they are; (0,4)(1,5)(2,6)(3,7), which one and-or a register unpacks 4-bit codes to;
+// (0,2)(1,3)(4,6)(5,7), which is how a conversion of two bytes a register leaves them.
+enum class RowOrder { kPlain, kPaired, kQuads };
+__host__ __device__ constexpr int place_of_value(RowOrder order, int v) {  // of an 8-block
+  return order == RowOrder::kPaired ? (v & 3) << 1 | v >> 2 : order == RowOrder::kQuads ? (v & 4) | (v & 1) << 1 | (v >> 1 & 1) : v;
+}
+__host__ __device__ constexpr int value_at_place(RowOrder order, int p) {
+  return order == RowOrder::kPaired ? (p & 1) << 2 | p >> 1 : order == RowOrder::kQuads ? (p & 4) | (p & 1) << 1 | (p >> 1 & 1) : p;
+}
+// What preparing rows for the products on raw codes (launch_prepare_rows) reads and writes.
+struct PrepareArgs {
+  const void *x = nullptr;
+  int64_t octets = 0;  // 8-blocks of x in all, and of a row; 0: nothing to prepare
+  int octets_per_row = 0, lanes_log2 = 0;  // (of a group)
+  uint16_t *copy = nullptr, *sums = nullptr;
+  int sums_row = 0, slots = 0;
+  RowOrder order = RowOrder::kPlain;
+};
 bool router_fused_applies(int64_t T, int E, int k);
 hipError_t launch_router_fused(const uint16_t *x, const uint16_t *wg, const float *bias,
                                const uint16_t *norm_w, float eps, uint16_t *xnorm, int64_t T,
@@ -364,7 +384,7 @@ struct CodesArgs {
   const void *s0, *b0, *s1, *b1;
   const void *bias;  // [N] added after the rounding of the product, with a rounding of its own; or nullptr
   void *y;
-  bool y_paired;
+  RowOrder y_order;
   uint16_t *y_sums;  // gate/up tiles: where the group sums of the output rows go as well, in the form of launch_prepare_rows; or nullptr
   int N, K;
   int64_t M;  // rows (dense launches)
@@ -401,14 +421,13 @@ hipError_t launch_qmm_cols(const ColsArgs &a, int group, int bits, int dt, hipSt
 size_t codes_copy_bytes(int bits, int64_t rows, int K);
 // plain: for the products on codes without a centre (launch_qmm_pieces)
 size_t codes_sums_bytes(int64_t rows, int K, int group, bool plain = false);
+PrepareArgs prepare_args(const void *x, int64_t rows, int K, int group, uint16_t *copy, uint16_t *sums, bool plain);
 hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
                                uint16_t *sums, bool plain, hipStream_t st);
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
 hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st);
 // 4-bit codes in groups of 64, a list of pieces of kPieceM rows
 hipError_t launch_qmm_pieces(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
-// the same tiles with the codes in registers (bf16, 4-bit, groups of 32); a.y_sums is not written
-hipError_t launch_qmm_codes_list(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
 hipError_t launch_quantize(const float *w, int64_t rows, int64_t cols, int group, int bits,
                            uint32_t *q, void *s, void *b, int dt, hipStream_t st);
 hipError_t launch_dequantize(const uint32_t *q, const void *s, const void *b,

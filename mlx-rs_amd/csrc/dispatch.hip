@@ -8,16 +8,28 @@
 // argsort gives, whatever order blocks and waves run in.  Also emits the list of
 // experts that received at least one pair (what the grouped products iterate over).
 #include "dispatch_dev.hpp"
+#include "qmm_codes_dev.hpp"
 
 namespace mi_moe {
+
+// Blocks from `first` on prepare rows (PrepareArgs) beside the dispatch, which is a chain of latencies on few CUs: in launches of their own they took
+// 4 us at 203 tokens and 8 at 4096 (hidden 2048), and the gap before them.
+__device__ __forceinline__ bool prepares(const PrepareArgs &a, int first) {
+  if ((int)blockIdx.x < first) return false;
+  const int64_t i = (int64_t)((int)blockIdx.x - first) * kDispThreads + threadIdx.x;
+  if (i < a.octets) prepare_octet<0>(a, i);  // (whole groups leave together)
+  return true;
+}
+static unsigned prepare_blocks(const PrepareArgs &a) { return (unsigned)((a.octets + kDispThreads - 1) / kDispThreads); }
 
 // ---- one block does everything (decode-sized P)
 __global__ __launch_bounds__(kDispThreads) void dispatch_single_kernel(
     const uint32_t *flat, int64_t P, int E, int nbits, int k_div,
     uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets, uint32_t *__restrict__ perm,
     uint32_t *__restrict__ inv_perm, uint32_t *__restrict__ src_of,
-    uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr, ShortTiles shorts) {
+    uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr, ShortTiles shorts, PrepareArgs prepare) {
   extern __shared__ uint32_t lds[];
+  if (prepares(prepare, 1)) return;
   dispatch_block(flat, P, E, nbits, k_div, lds, counts, offsets, perm, inv_perm, src_of, work, mtiles, cap256, big_thr, shorts);
 }
 
@@ -49,9 +61,10 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     const uint32_t *flat, int64_t P, int E, int nbits, int k_div, int64_t span,
     const uint32_t *__restrict__ blockhist, int nb, uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets,
     uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr, ShortTiles shorts,
-    uint32_t *__restrict__ perm, uint32_t *__restrict__ inv_perm, uint32_t *__restrict__ src_of) {
+    uint32_t *__restrict__ perm, uint32_t *__restrict__ inv_perm, uint32_t *__restrict__ src_of, PrepareArgs prepare) {
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t n_active, total;
+  if (prepares(prepare, nb + 1)) return;
   uint32_t *cnt = lds, *tmp = lds + E, *cur = lds + 2 * E, *wcnt = lds + 3 * E;  // tmp: at least kDispWaves words
   const int tid = threadIdx.x;
   const int mine = (int)blockIdx.x;
@@ -111,15 +124,15 @@ size_t dispatch_workspace_least(int E, int64_t P) { return P <= kSingleAtMostP ?
 hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, uint32_t *counts,
                            uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
                            uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, int big_thr,
-                           ShortTiles shorts, void *scratch, hipStream_t st) {
+                           ShortTiles shorts, const PrepareArgs &prepare, void *scratch, hipStream_t st) {
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
   if (k_div < 1) k_div = 1;
   if (P <= kSingleMaxP || !scratch) {
     if (P > kSingleAtMostP) return hipErrorInvalidValue;
     size_t lds = (size_t)(3 + kDispWaves) * E * sizeof(uint32_t);
-    dispatch_single_kernel<<<1, kDispThreads, lds, st>>>(flat, P, E, nbits, k_div, counts, offsets,
-                                                        perm, inv_perm, src_of, work, mtiles, cap256, (uint32_t)big_thr, shorts);
+    dispatch_single_kernel<<<1 + prepare_blocks(prepare), kDispThreads, lds, st>>>(flat, P, E, nbits, k_div, counts, offsets,
+                                                        perm, inv_perm, src_of, work, mtiles, cap256, (uint32_t)big_thr, shorts, prepare);
     return hipGetLastError();
   }
   uint32_t *blockhist = reinterpret_cast<uint32_t *>(scratch);
@@ -129,9 +142,9 @@ hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, ui
   // partial-sum arrays [G][E] (G E <= 1024)
   const size_t e3 = (size_t)3 * (E > kDispWaves ? E : kDispWaves);
   const size_t tail = (size_t)kDispWaves * E > 2u * kDispThreads ? (size_t)kDispWaves * E : 2u * kDispThreads;
-  dispatch_scatter_kernel<<<nb + 1, kDispThreads, (e3 + tail) * 4, st>>>(flat, P, E, nbits, k_div, kSpan, blockhist, nb, counts,
+  dispatch_scatter_kernel<<<nb + 1 + prepare_blocks(prepare), kDispThreads, (e3 + tail) * 4, st>>>(flat, P, E, nbits, k_div, kSpan, blockhist, nb, counts,
                                                                         offsets, work, mtiles, cap256, (uint32_t)big_thr, shorts, perm,
-                                                                        inv_perm, src_of);
+                                                                        inv_perm, src_of, prepare);
   return hipGetLastError();
 }
 

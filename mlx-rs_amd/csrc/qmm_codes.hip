@@ -1,6 +1,5 @@
-// The middle of the range of dense products on raw codes (which: dense_rule.hpp) and the long segments of the smaller blocks with 4-bit codes in
-// groups of 32 (contract, arithmetic and prepared rows: qmm_tiles.hip, with c = 8 or 128): tiles of 64 x 128, and of 32 x 64 for bf16 and 8-bit
-// codes in groups of 32, whose waves load their codes straight into the registers that unpack them.
+// The middle of the range of dense products on raw codes (which: dense_rule.hpp; contract, arithmetic and prepared rows: qmm_tiles.hip, with
+// c = 8 or 128): tiles of 64 x 128, and of 32 x 64 for bf16 and 8-bit codes in groups of 32, whose waves load their codes straight into the registers that unpack them.
 #include <type_traits>
 
 #include "qmm_codes_dev.hpp"
@@ -28,8 +27,8 @@ __device__ __forceinline__ Split<SPLIT, F> with_split(F f) { return Split<SPLIT,
 
 }  // namespace
 
-// A block computes 32 MS token rows x 32 WN weight rows with WN KW waves (GLU: and the 32 WN matching ones of the up matrix).  A wave owns 32 weight
-// rows (and 32 of the up matrix) for all the block's token rows, so it loads its own codes straight
+// A block computes 32 MS token rows x 32 WN weight rows with WN KW waves.  A wave owns 32 weight
+// rows for all the block's token rows, so it loads its own codes straight
 // into the lanes that multiply them and unpacks them in registers: nothing of the weights passes through LDS, and no
 // wave unpacks what another one does.  A lane (weight row l % 32, half l / 32) loads 16 bytes; which K values its
 // eight codes of a multiply stand for is free as long as the token operand agrees:
@@ -46,14 +45,12 @@ __device__ __forceinline__ Split<SPLIT, F> with_split(F f) { return Split<SPLIT,
 // the loads 1350.  The loads cost their line visits: a wave's codes sit in 32 rows.
 // KW > 1: the block's waves form KW groups that share K among them, each with LDS buffers of its own; their sums meet in
 // LDS at the end, added in group order.  For launches that give a CU one block or less.
-// DT: 0 bf16, 1 f16.  G32: groups of 32; otherwise a group is one or two steps (scale_shift).  LIST: the tiles of a list (see ShortTiles).
-template <int DT, int BITS, bool G32, bool LIST, bool GLU, int MS, int WN, int KW>
+// DT: 0 bf16, 1 f16.  G32: groups of 32; otherwise a group is one or two steps (scale_shift).
+template <int DT, int BITS, bool G32, int MS, int WN, int KW>
 __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2, 4))) void qmm_codes_kernel(
-    CodesArgs a, const uint32_t *__restrict__ list, int n_mtiles, int n_ntiles, int scale_shift) {
-  static_assert(!GLU || (LIST && KW == 1), "gate/up products are a list's");
-  constexpr int NT = GLU ? 2 : 1;  // a gate tile and its up tile
+    CodesArgs a, int n_mtiles, int n_ntiles, int scale_shift) {
   typedef typename ElemOf<DT>::type T;
-  constexpr int BM = 32 * MS;
+  constexpr int BM = 32 * MS, NT = 1;        // (weight tiles of a wave)
   constexpr int NI = 32 * WN;                // output columns per block
   constexpr int NA = BM * 8 / (64 * WN);     // 16-byte activation loads per thread, piece and step
   constexpr int RS = 8 * WN;                 // rows one such load of a group covers
@@ -64,26 +61,13 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   constexpr int A_SZ = BM * kRow, BUF = A_SZ;                      // 16-byte units
   static_assert(BM % RS == 0, "whole loads");
 
-  // block -> (M tile, N tile).  Ids are dealt round-robin over the 8 XCDs.  Dense: an XCD takes every eighth N tile and all M tiles of it, so its
-  // L2 holds the weights of a few N tiles and x streams through.  A list: whole M tiles per XCD (the blocks of one share its gathered rows).
+  // block -> (M tile, N tile).  Ids are dealt round-robin over the 8 XCDs: an XCD takes every eighth N tile and all M tiles of it, so its
+  // L2 holds the weights of a few N tiles and x streams through.
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-  int e = 0, rows, nt;
-  int64_t row0;
-  if constexpr (LIST) {
-    const uint32_t id = (uint32_t)(j / n_ntiles) * 8u + xcd;
-    nt = j % n_ntiles;
-    if (id >= list[0]) return;
-    const uint4 rec = reinterpret_cast<const uint4 *>(list)[1 + id];
-    e = (int)rec.x;
-    row0 = (int64_t)rec.y;
-    rows = (int)rec.z;
-  } else {
-    nt = j / n_mtiles * 8 + xcd;
-    if (nt >= n_ntiles) return;
-    row0 = (int64_t)(j % n_mtiles) * BM;
-    rows = a.M - row0 < BM ? (int)(a.M - row0) : BM;
-  }
-  auto x_row = [&](int tr) __attribute__((always_inline)) { return LIST && a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr); };
+  const int nt = j / n_mtiles * 8 + xcd;
+  if (nt >= n_ntiles) return;
+  const int64_t row0 = (int64_t)(j % n_mtiles) * BM;
+  const int rows = a.M - row0 < BM ? (int)(a.M - row0) : BM;
 
   const int lane = threadIdx.x & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -106,28 +90,17 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   for (int i = 0; i < NA; ++i) {
     int tr = arg + RS * i;
     tr = tr < rows ? tr : rows - 1;  // rows past the end repeat the last one (never stored)
-    const uint32_t r = x_row(tr);
+    const uint32_t r = (uint32_t)(row0 + tr);
     x_voff[i] = (r * (uint32_t)K + acp * 8) * sizeof(T);
     xs_voff[i] = (r * (uint32_t)ext + acp * 8) * 2;
   }
   // ---- the weight rows of this lane
   const int ln = lane & 31, kb = lane >> 5;
-  const int64_t ebase = (int64_t)e * N;
-  __amdgpu_buffer_rsrc_t wr[NT], sr[NT], br[NT];
-  uint32_t w_voff[NT], s_voff[NT];
-  int w_row[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    // paired output (see GroupedArgs::y_paired): the lane at place p of an 8-block takes the row whose result belongs there
-    int row = n0 + 32 * wave + (LIST && a.y_paired ? ((ln & ~7) | (((ln & 7) >> 1) + ((ln & 1) ? 4 : 0))) : ln);
-    row = row < N ? row : N - 1;  // columns past the end repeat the last one (never stored)
-    wr[t] = rsrc_of((t ? a.w1 : a.w0) + ebase * (row_bytes / 4), (uint32_t)N * row_bytes);
-    sr[t] = rsrc_of(static_cast<const T *>(t ? a.s1 : a.s0) + ebase * G, (uint32_t)N * G * sizeof(T));  // (read in words: the host takes an even number of them)
-    br[t] = rsrc_of(static_cast<const T *>(t ? a.b1 : a.b0) + ebase * G, (uint32_t)N * G * sizeof(T));
-    w_row[t] = row;
-    w_voff[t] = (uint32_t)row * row_bytes + kb * 16;
-    s_voff[t] = (uint32_t)row * G * sizeof(T);
-  }
+  const int w_row[NT] = {n0 + 32 * wave + ln < N ? n0 + 32 * wave + ln : N - 1};  // columns past the end repeat the last one (never stored)
+  const __amdgpu_buffer_rsrc_t wr[NT] = {rsrc_of(a.w0, (uint32_t)N * row_bytes)};
+  const __amdgpu_buffer_rsrc_t sr[NT] = {rsrc_of(a.s0, (uint32_t)N * G * sizeof(T))};  // (read in words: the host takes an even number of them)
+  const __amdgpu_buffer_rsrc_t br[NT] = {rsrc_of(a.b0, (uint32_t)N * G * sizeof(T))};
+  const uint32_t w_voff[NT] = {(uint32_t)w_row[0] * row_bytes + kb * 16}, s_voff[NT] = {(uint32_t)(w_row[0] * G * (int)sizeof(T))};
 
   f32x16_t tot[MS][NT];
   const f32x16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -430,8 +403,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     const int col0 = n0 + 32 * wave;
     const int bc = col0 + ln < N ? col0 + ln : N - 1;
     const float lb = a.bias ? as_f32(static_cast<const T *>(a.bias)[bc]) : 0.f;
-    auto put = [&](int r, float v, float up) __attribute__((always_inline)) {
-      if constexpr (GLU) v = v / (1.0f + __expf(-v)) * up;
+    auto put = [&](int r, float v) __attribute__((always_inline)) {
       T o = rounded<T>(v);
       if (a.bias) o = rounded<T>(as_f32(o) + lb);
       reinterpret_cast<T *>(mine + (8 * (r >> 2) + 4 * kb + (r & 3)) * ROWB)[ln] = o;
@@ -439,9 +411,8 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
     uint32_t again = 0;  // (bits: which of the sixteen sums are not finite)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const float v = tot[m][0][r], up = tot[m][NT - 1][r];
-      put(r, v, up);
-      again |= (not_finite(v) || not_finite(up) ? 1u : 0u) << r;
+      put(r, tot[m][0][r]);
+      again |= (not_finite(tot[m][0][r]) ? 1u : 0u) << r;
     }
 #pragma unroll 1
     for (int quad = 0; __builtin_expect(again != 0, 0); ++quad, again >>= 4) {  // rows 8 quad + 4 kb + 0 .. 3
@@ -454,19 +425,15 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
           open &= ~(1u << i);
           tr = rows - 1;
         }
-        xs[i] = static_cast<const T *>(a.x) + (int64_t)x_row(tr) * K;
+        xs[i] = static_cast<const T *>(a.x) + (row0 + tr) * K;
       }
       if (!open) continue;
-      float v[NT][4];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int64_t wrow = ebase + w_row[t];
-        plain_rows<BITS, 4, T>(xs, paired_order(BITS), (t ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const T *>(t ? a.s1 : a.s0) + wrow * G,
-                               static_cast<const T *>(t ? a.b1 : a.b0) + wrow * G, K, K / G, open, v[t]);
-      }
+      float v[4];
+      plain_rows<BITS, 4, T>(xs, row_order(BITS), a.w0 + (int64_t)w_row[0] * (row_bytes / 4), static_cast<const T *>(a.s0) + (int64_t)w_row[0] * G,
+                             static_cast<const T *>(a.b0) + (int64_t)w_row[0] * G, K, K / G, open, v);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (open >> i & 1u) put(4 * quad + i, v[0][i], v[NT - 1][i]);
+        if (open >> i & 1u) put(4 * quad + i, v[i]);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -477,8 +444,7 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
       const int row = RPI * i + my_row;
       const int tr = 32 * m + row;
       if (tr < rows && my_col < N) {
-        const int64_t dst = LIST && a.dst_rows ? (int64_t)a.dst_rows[row0 + tr] : row0 + tr;
-        T *const to = static_cast<T *>(a.y) + dst * N + my_col;
+        T *const to = static_cast<T *>(a.y) + (row0 + tr) * N + my_col;
         const T *const from = reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece;
         if (vec) {
           *reinterpret_cast<u32x4_t *>(to) = *reinterpret_cast<const u32x4_t *>(from);
@@ -493,29 +459,25 @@ __global__ __launch_bounds__(64 * WN * KW) __attribute__((amdgpu_waves_per_eu(2,
   }
 }
 
-template <int DT, int BITS, bool G32, int MS, int WN, int KW, bool LIST = false, bool GLU = false>
-static hipError_t start_codes(const CodesArgs &a, int scale_shift, hipStream_t st, const uint32_t *list = nullptr, int cap = 0) {
-  constexpr int NI = 32 * WN, BM = 32 * MS, NT = GLU ? 2 : 1;
-  constexpr size_t bufs = (size_t)2 * KW * BM * kRow * 16 + WN * KW * NT * 32 * 48, sums = KW > 1 ? (size_t)BM * 32 * WN * 4 : 0;
+template <int DT, int BITS, bool G32, int MS, int WN, int KW>
+static hipError_t start_codes(const CodesArgs &a, int scale_shift, hipStream_t st) {
+  constexpr int NI = 32 * WN, BM = 32 * MS;
+  constexpr size_t bufs = (size_t)2 * KW * BM * kRow * 16 + WN * KW * 32 * 48, sums = KW > 1 ? (size_t)BM * 32 * WN * 4 : 0;
   constexpr size_t most = bufs > sums ? bufs : sums, lds = most > kLdsAtLeast ? most : kLdsAtLeast;
   static_assert(lds <= 160 * 1024, "more LDS than a CU has");
-  const int n_ntiles = (a.N + NI - 1) / NI, mtiles = LIST ? cap : (int)((a.M + BM - 1) / BM);
-  const int64_t grid = LIST ? ((int64_t)cap + 7) / 8 * 8 * n_ntiles : (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
+  const int n_ntiles = (a.N + NI - 1) / NI, mtiles = (int)((a.M + BM - 1) / BM);
+  const int64_t grid = (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
   if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
-  const auto kernel = &qmm_codes_kernel<DT, BITS, G32, LIST, GLU, MS, WN, KW>;
+  const auto kernel = &qmm_codes_kernel<DT, BITS, G32, MS, WN, KW>;
   if (lds > 64 * 1024) {
     static std::atomic<uint64_t> allowed{0};
     if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), (int)lds, allowed); e != hipSuccess) return e;
   }
-  kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, list, mtiles, n_ntiles, scale_shift);
+  kernel<<<(unsigned)grid, 64 * WN * KW, lds, st>>>(a, mtiles, n_ntiles, scale_shift);
   return hipGetLastError();
 }
 
 hipError_t launch_qmm_codes_small(const CodesArgs &a, hipStream_t st) { return start_codes<0, 8, true, 1, 2, 4>(a, 0, st); }
-
-hipError_t launch_qmm_codes_list(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st) {
-  return glu ? start_codes<0, 4, true, 2, 4, 1, true, true>(a, 0, st, list, cap) : start_codes<0, 4, true, 2, 4, 1, true, false>(a, 0, st, list, cap);
-}
 
 hipError_t launch_qmm_codes_middle(const CodesArgs &a, bool share, int group, int bits, int dt, hipStream_t st) {
   auto with_group = [&](auto d, auto b) {

@@ -29,8 +29,50 @@ __device__ __forceinline__ void put_sums(uint16_t *to, int slots, float sum) {
   else *reinterpret_cast<uint2 *>(to) = make_uint2(p.h | p.m << 16, p.l);
 }
 
-constexpr bool paired_order(int bits) { return bits == 4; }  // 8-blocks as (0,4)(1,5)(2,6)(3,7)
+constexpr RowOrder row_order(int bits) { return bits == 4 ? RowOrder::kPaired : RowOrder::kPlain; }
 constexpr int padded_groups(int G) { return (G + 15) / 16 * 16; }  // whole windows of the bias product; the groups past the row's end are zeros
+
+// One thread's part of preparing rows: eight values of x (octet i of all rows).  Whole groups go through lanes of one wave.
+template <int DT>
+__device__ __forceinline__ void prepare_octet(const PrepareArgs &a, int64_t i) {
+  float v[8];
+  const uint4 w = reinterpret_cast<const uint4 *>(a.x)[i];
+  const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if constexpr (DT == 0) {
+      v[2 * j] = bf16lo_to_f32(u[j]);
+      v[2 * j + 1] = bf16hi_to_f32(u[j]);
+    } else {
+      const half2_t hh = __builtin_bit_cast(half2_t, u[j]);
+      v[2 * j] = (float)hh.x;
+      v[2 * j + 1] = (float)hh.y;
+    }
+  }
+  if (a.copy) {
+    const bool quads = a.order == RowOrder::kQuads;
+    const uint32_t y = quads ? w.z : w.y, z = quads ? w.y : w.z;  // the words that meet: 0 and 2, 1 and 3, or neighbours
+    uint4 p;
+    p.x = (w.x & 0xffffu) | (z << 16);
+    p.y = (w.x >> 16) | (z & 0xffff0000u);
+    p.z = (y & 0xffffu) | (w.w << 16);
+    p.w = (y >> 16) | (w.w & 0xffff0000u);
+    *reinterpret_cast<uint4 *>(a.copy + 8 * i) = p;
+  }
+  float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
+  sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
+  if (a.lanes_log2 >= 3) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
+  if (a.lanes_log2 == 4) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
+  if ((i & ((1 << a.lanes_log2) - 1)) == 0) {
+    const int64_t row = i / a.octets_per_row;
+    const int g = (int)(i % a.octets_per_row) >> a.lanes_log2, G = a.octets_per_row >> a.lanes_log2;
+    uint16_t *const to = a.sums + row * a.sums_row + g * a.slots;
+    put_sums(to, a.slots, sum);
+    if (g == G - 1)
+      for (int k = a.slots; g * a.slots + k < a.sums_row; k += 4) *reinterpret_cast<uint2 *>(to + k) = make_uint2(0, 0);
+  }
+}
 
 // A kernel's leave to use more than 64 KB of LDS, asked for once a GPU (half a microsecond a launch otherwise).  done: a bit per GPU.
 inline hipError_t allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &done) {

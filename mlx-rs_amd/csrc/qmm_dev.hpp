@@ -65,14 +65,14 @@ __device__ __forceinline__ uint32_t f16_centred(uint32_t v) {  // two halves 102
 
 // ROWS rows of x against one row of weights packed along K, an fma per k on the dequantised weight, in the order of k.  The products
 // on raw codes take it where their own sum is not finite: an infinity against codes and biases apart cancels to no number where
-// the dequantised weight keeps its sign, and sums of unscaled codes overflow earlier.  paired: x has every 8-block as
-// (0,4)(1,5)(2,6)(3,7).  open: the rows that are wanted.  K and the group are multiples of 32, x and w are aligned for 16 bytes.
+// the dequantised weight keeps its sign, and sums of unscaled codes overflow earlier.  order: of the 8-blocks of
+// x.  open: the rows that are wanted.  K and the group are multiples of 32, x and w are aligned for 16 bytes.
 // It is one lane's chain over K and the latency of its loads, so 32 values of each row are fetched at a time.
 // us of a product 4096 x 4096 with finite rows / one infinity in one row / one in each: bf16 4-bit 1 row 12 / 79, 16 rows 17 / 89 / 284, 200 rows 36 /
 // 200 / 1460, 1000 rows 66 / 274 / 1840; f16 8-bit 777 rows 58 / 222 / 1830 (one row and word at a time 12 / 108, 17 / 118 / 480, 38 / 174 / 5530, 73 /
 // 268 / 11800, 61 / 290 / 24000; a wave per output element 3160 for the last).  Rows of NaNs cost next to nothing.
 template <int BITS, int ROWS, class T>
-__device__ __forceinline__ void plain_rows(const T *const (&x)[ROWS], bool paired, const uint32_t *w, const T *s, const T *b, int K, int group,
+__device__ __forceinline__ void plain_rows(const T *const (&x)[ROWS], RowOrder order, const uint32_t *w, const T *s, const T *b, int K, int group,
                                            uint32_t open, float (&sum)[ROWS]) {
   static_assert(sizeof(T) == 2, "eight values are 16 bytes");
   constexpr int PER = 32 / BITS;  // codes of a word
@@ -90,7 +90,7 @@ __device__ __forceinline__ void plain_rows(const T *const (&x)[ROWS], bool paire
     const float sc = as_f32(s[k / group]), bi = as_f32(b[k / group]);
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
-      const int at = i & 7, from = paired ? (at & 3) << 1 | at >> 2 : at;
+      const int at = i & 7, from = place_of_value(order, at);
       const float wf = __builtin_fmaf(sc, (float)((words[i / PER] >> (i % PER * BITS)) & ((1u << BITS) - 1u)), bi);
 #pragma unroll
       for (int r = 0; r < ROWS; ++r) {

@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
         float v[NM][1];
 #pragma unroll
         for (int m = 0; m < NM; ++m)
-          plain_rows<BITS, 1, T>(xr, false, (m ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const T *>(m ? a.s1 : a.s0) + wrow * G,
+          plain_rows<BITS, 1, T>(xr, RowOrder::kPlain, (m ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const T *>(m ? a.s1 : a.s0) + wrow * G,
                                  static_cast<const T *>(m ? a.b1 : a.b0) + wrow * G, K, GROUP, 1u, v[m]);
         put(r, v[0][0], v[NM - 1][0]);
       }

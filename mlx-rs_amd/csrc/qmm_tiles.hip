@@ -29,50 +29,10 @@
 namespace mi_moe {
 
 // One thread per eight values of x.
-// slots: K slots of a group in the bias product (sum_slots).
 template <int DT>
-__global__ __launch_bounds__(256) void prepare_rows_kernel(const typename ElemOf<DT>::type *__restrict__ x, int64_t n_octets,
-                                                           int octets_per_row, int lanes_log2,
-                                                           uint16_t *__restrict__ copy, uint16_t *__restrict__ sums, int sums_row, int slots) {
+__global__ __launch_bounds__(256) void prepare_rows_kernel(PrepareArgs a) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n_octets) return;  // whole groups leave together
-  float v[8];
-  {
-    const uint4 w = reinterpret_cast<const uint4 *>(x)[i];
-    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if constexpr (DT == 0) {
-        v[2 * j] = bf16lo_to_f32(u[j]);
-        v[2 * j + 1] = bf16hi_to_f32(u[j]);
-      } else {
-        const half2_t hh = __builtin_bit_cast(half2_t, u[j]);
-        v[2 * j] = (float)hh.x;
-        v[2 * j + 1] = (float)hh.y;
-      }
-    }
-    if (copy) {
-      uint4 p;
-      p.x = (w.x & 0xffffu) | (w.z << 16);
-      p.y = (w.x >> 16) | (w.z & 0xffff0000u);
-      p.z = (w.y & 0xffffu) | (w.w << 16);
-      p.w = (w.y >> 16) | (w.w & 0xffff0000u);
-      *reinterpret_cast<uint4 *>(copy + 8 * i) = p;
-    }
-  }
-  float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-  sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
-  sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
-  if (lanes_log2 >= 3) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
-  if (lanes_log2 == 4) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
-  if ((i & ((1 << lanes_log2) - 1)) == 0) {
-    const int64_t row = i / octets_per_row;
-    const int g = (int)(i % octets_per_row) >> lanes_log2, G = octets_per_row >> lanes_log2;
-    uint16_t *const to = sums + row * sums_row + g * slots;
-    put_sums(to, slots, sum);
-    if (g == G - 1)
-      for (int k = slots; g * slots + k < sums_row; k += 4) *reinterpret_cast<uint2 *>(to + k) = make_uint2(0, 0);
-  }
+  if (i < a.octets) prepare_octet<DT>(a, i);  // (whole groups leave together)
 }
 
 // ---- copies from memory straight into LDS
@@ -150,7 +110,7 @@ struct Tile {
   static __device__ __forceinline__ void unpack(const u32x4_t (&q)[NQ], int h, u32x4_t &o) {
       if constexpr (kPlainCodes) {
         // a byte of 0 to 15 is that many 2^-9 as an 8-bit float (four exponent bits, three of mantissa): the conversion takes two at a time
-        const uint32_t w = __builtin_amdgcn_perm(q[0][h], q[0][h], 0x03010200u), even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
+        const uint32_t w = q[0][h], even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
         o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false));
         o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false));
         o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true));
@@ -217,10 +177,10 @@ __device__ __forceinline__ void add_plain_biases(float (&tot)[MS][NT][16], const
   }
 }
 
-// The results of a tile (see multiply_tile) go out, GLU: as silu(gate) up.  Every wave comes here with GLU.
-template <int DT, int BITS, bool GLU, int MS, int NT, int WN, class WeightRow>
-__device__ __forceinline__ void write_tile(const CodesArgs &a, const float (&tot)[MS][NT][16], int wave, int lane, int n0, int col0, int64_t row0, int rows,
-                                           int64_t ebase, int glog, WeightRow weight_row, unsigned char *lds_raw) {
+// The results of a dense tile (see multiply_tile) go out.
+template <int DT, int BITS, int MS, int NT, int WN, class WeightRow>
+__device__ __forceinline__ void write_tile(const CodesArgs &a, const float (&tot)[MS][NT][16], int wave, int lane, int col0, int64_t row0, int rows,
+                                           int glog, WeightRow weight_row, unsigned char *lds_raw) {
   // ---- epilogue: a wave turns its 32 x 32 sub-tiles round in a private piece of LDS and stores 16 bytes a lane
   typedef typename ElemOf<DT>::type T;
   const int N = a.N, K = a.K, G = K >> glog, row_bytes = K * BITS / 8;
@@ -232,16 +192,11 @@ __device__ __forceinline__ void write_tile(const CodesArgs &a, const float (&tot
   unsigned char *const mine = lds_raw + wave * (32 * ROWB);
   const int my_piece = lane % CPR, my_row = lane / CPR;
   const bool vec = N % PV == 0;
-  // The gate/up tiles also sum their rows over the quantisation groups, which the down product's bias term wants (columns in whole blocks of 128:
-  // 32 of them here, the rest of a group in the waves beside).  A kernel over the finished rows took 5 us.
-  const bool sums_too = GLU && a.y_sums != nullptr;
-  float *const parts_of_sums = reinterpret_cast<float *>(lds_raw + WN * (32 * ROWB));  // [wave][row]
 #pragma unroll
-  for (int u = 0; u < MS * (GLU ? 1 : NT); ++u) {
-    const int m = u / (GLU ? 1 : NT), t = u % (GLU ? 1 : NT), col = col0 + 32 * t;
+  for (int u = 0; u < MS * NT; ++u) {
+    const int m = u / NT, t = u % NT, col = col0 + 32 * t;
     const float lb = a.bias ? as_f32(static_cast<const T *>(a.bias)[col + ln < N ? col + ln : N - 1]) : 0.f;
-    auto put = [&](int r, float v, float up) __attribute__((always_inline)) {
-      if constexpr (GLU) v = v / (1.0f + __expf(-v)) * up;
+    auto put = [&](int r, float v) __attribute__((always_inline)) {
       T o = rounded<T>(v);
       if (a.bias) o = rounded<T>(as_f32(o) + lb);
       reinterpret_cast<T *>(mine + (8 * (r >> 2) + 4 * kb + (r & 3)) * ROWB)[ln] = o;
@@ -249,9 +204,8 @@ __device__ __forceinline__ void write_tile(const CodesArgs &a, const float (&tot
     uint32_t again = 0;  // (bits: which of the sixteen sums are not finite)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const float v = tot[m][t][r], up = GLU ? tot[m][NT - 1][r] : 0.f;
-      put(r, v, up);
-      again |= (not_finite(v) || (GLU && not_finite(up)) ? 1u : 0u) << r;
+      put(r, tot[m][t][r]);
+      again |= (not_finite(tot[m][t][r]) ? 1u : 0u) << r;
     }
 #pragma unroll 1
     for (int quad = 0; __builtin_expect(again != 0, 0); ++quad, again >>= 4) {  // rows 8 quad + 4 kb + 0 .. 3
@@ -267,17 +221,13 @@ __device__ __forceinline__ void write_tile(const CodesArgs &a, const float (&tot
         xs[i] = static_cast<const T *>(a.x) + (int64_t)(a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr)) * K;
       }
       if (!open) continue;
-      float v[GLU ? 2 : 1][4];
-#pragma unroll
-      for (int i = 0; i < (GLU ? 2 : 1); ++i) {
-        const int64_t wrow = ebase + weight_row(GLU ? i : t, ln);
-        plain_rows<BITS, 4, T>(xs, paired_order(BITS), (GLU && i ? a.w1 : a.w0) + wrow * (row_bytes / 4),
-                               static_cast<const T *>(GLU && i ? a.s1 : a.s0) + wrow * G,
-                               static_cast<const T *>(GLU && i ? a.b1 : a.b0) + wrow * G, K, K / G, open, v[i]);
-      }
+      float v[4];
+      const int64_t wrow = weight_row(t, ln);
+      plain_rows<BITS, 4, T>(xs, row_order(BITS), a.w0 + wrow * (row_bytes / 4), static_cast<const T *>(a.s0) + wrow * G, static_cast<const T *>(a.b0) + wrow * G, K, K / G,
+                             open, v);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (open >> i & 1u) put(4 * quad + i, v[0][i], v[GLU ? 1 : 0][i]);
+        if (open >> i & 1u) put(4 * quad + i, v[i]);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -297,34 +247,10 @@ __device__ __forceinline__ void write_tile(const CodesArgs &a, const float (&tot
           for (int c = 0; c < PV && my_col + c < N; ++c) to[c] = from[c];
         }
       }
-      if constexpr (GLU) {
-        if (sums_too) {
-          const u32x4_t w = *reinterpret_cast<const u32x4_t *>(reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece);
-          float sum = ((bf16lo_to_f32(w[0]) + bf16hi_to_f32(w[0])) + (bf16lo_to_f32(w[1]) + bf16hi_to_f32(w[1]))) +
-                      ((bf16lo_to_f32(w[2]) + bf16hi_to_f32(w[2])) + (bf16lo_to_f32(w[3]) + bf16hi_to_f32(w[3])));
-          sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
-          sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
-          if (my_piece == 0) parts_of_sums[wave * (32 * MS) + tr] = sum;
-        }
-      }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
-  if constexpr (GLU) {
-    static_assert(DT == 0 && WN == 4, "four waves cover a group of 128");
-    if (!sums_too) return;
-    __syncthreads();
-    const int first = n0 >> glog, groups = N >> glog, here = 128 >> glog, waves = 1 << (glog - 5);  // (the output's groups are as long as the input's)
-    const int end = first + here >= groups ? padded_groups(groups) : first + here;  // the last block writes the zeros behind
-    for (int i = threadIdx.x; i < rows * (end - first); i += 64 * WN) {
-      const int row = i % rows, g = i / rows;
-      float sum = 0.f;
-      if (first + g < groups)
-        for (int w = 0; w < waves; ++w) sum += parts_of_sums[(g * waves + w) * (32 * MS) + row];
-      put_sums(a.y_sums + ((row0 + row) * padded_groups(groups) + first + g) * kSlots, kSlots, sum);
-    }
   }
 }
 
@@ -342,15 +268,16 @@ __device__ __forceinline__ float gated(float g, float u) {
   const float d = 1.0f + __expf(fminf(-g, 88.0f)), r = __builtin_amdgcn_rcpf(d), q = g * r;
   return __builtin_fmaf(__builtin_fmaf(-d, q, g), r, q) * u;
 }
-// The results of a piece of up to 32 MS rows x 256 weight rows (4-bit codes in groups of 64; four waves, 64 weight rows each) go out: N is a multiple of
+// The results of a piece of up to 32 MS rows x 256 weight rows (of a block; four waves, 64 weight rows each) go out: N is a multiple of
 // 128, there is no bias of the layer's.  Two rows of a column become one register, neighbouring lanes swap halves, and the rows are turned round in LDS:
-// GLU: by the whole block, whose 256 bytes a row are two quantisation groups of h, of which the lanes that store them also write the group sums;
+// GLU: by the whole block, whose 256 bytes a row are one to four quantisation groups of h, of which the lanes that store them also write the group sums;
 // else by each wave, 128 bytes a row.  (Rows found and stored 16 at a time behind a load of their places each: 12 us of the 37 of a block of 128 rows, K = 768.)
-template <bool GLU, int MS, class WeightRow>
-__device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&tot)[MS][2][16], int wave, int lane, int n0, int64_t row0, int rows, int64_t ebase,
+template <int BITS, bool PLAIN, bool GLU, int MS, class WeightRow>
+__device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&tot)[MS][2][16], int wave, int lane, int n0, int64_t row0, int rows, int64_t ebase, int glog,
                                             WeightRow weight_row, const uint32_t (&dst)[2], unsigned char *lds_raw) {
   constexpr int ROWB = GLU ? 272 : 144;  // (16 bytes keep rows off each other's banks)
-  const int N = a.N, K = a.K, G = K >> 6, row_bytes = K / 2, ln = lane & 31, kb = lane >> 5;
+  constexpr int SLOTS = sum_slots(PLAIN);
+  const int N = a.N, K = a.K, G = K >> glog, row_bytes = K * BITS / 8, ln = lane & 31, kb = lane >> 5;
   unsigned char *const mine = GLU ? lds_raw + wave * 64 : lds_raw + wave * (32 * ROWB);
   auto value = [&](int m, int t, int r) __attribute__((always_inline)) { return GLU ? gated(tot[m][0][r], tot[m][1][r]) : tot[m][t][r]; };
   float odd = 0.f;  // no number once a result was not finite
@@ -398,8 +325,8 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
 #pragma unroll
       for (int j = 0; j < (GLU ? 2 : 1); ++j) {
         const int64_t wrow = ebase + weight_row(GLU ? j : t, ln);
-        plain_rows<4, 4, uint16_t>(xs, true, (j ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const uint16_t *>(j ? a.s1 : a.s0) + wrow * G,
-                                   static_cast<const uint16_t *>(j ? a.b1 : a.b0) + wrow * G, K, 64, open, v[j]);
+        plain_rows<BITS, 4, uint16_t>(xs, PLAIN ? RowOrder::kQuads : row_order(BITS), (j ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const uint16_t *>(j ? a.s1 : a.s0) + wrow * G,
+                                   static_cast<const uint16_t *>(j ? a.b1 : a.b0) + wrow * G, K, 1 << glog, open, v[j]);
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -414,7 +341,7 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
     for (int m = 0; m < MS; ++m) turn(m, 32 * m);
     if (__builtin_expect(odd != odd, 0)) repair(0, MS, 0);
     __syncthreads();
-    const int groups = N >> 6, padded = padded_groups(groups);
+    const int groups = N >> glog, padded = padded_groups(groups), lanes = 1 << (glog - 3);  // (the output's groups are as long as the input's)
 #pragma unroll
     for (int i = 0; i < 2 * MS; ++i) {
       const int row = 16 * i + (int)(threadIdx.x >> 4), piece = threadIdx.x & 15;
@@ -423,15 +350,16 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
                   ((bf16lo_to_f32(w[2]) + bf16hi_to_f32(w[2])) + (bf16lo_to_f32(w[3]) + bf16hi_to_f32(w[3])));
       sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
       sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
-      sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
+      if (PLAIN || glog >= 6) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
+      if (!PLAIN && glog == 7) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
       if (row < rows) {
         *reinterpret_cast<u32x4_t *>(static_cast<uint16_t *>(a.y) + (row0 + row) * N + n0 + 8 * piece) = w;
-        if ((piece & 7) == 0) put_sums(a.y_sums + ((row0 + row) * padded + (n0 >> 6) + (piece >> 3)) * sum_slots(true), sum_slots(true), sum);
+        if ((piece & (lanes - 1)) == 0) put_sums(a.y_sums + ((row0 + row) * padded + (n0 >> glog) + (piece >> (glog - 3))) * SLOTS, SLOTS, sum);
       }
     }
     if (n0 + 128 >= N && groups < padded)  // the last block of a row writes the zeros behind its sums
       for (int i = threadIdx.x; i < rows * (padded - groups); i += 256)
-        put_sums(a.y_sums + ((row0 + i / (padded - groups)) * padded + groups + i % (padded - groups)) * sum_slots(true), sum_slots(true), 0.f);
+        put_sums(a.y_sums + ((row0 + i / (padded - groups)) * padded + groups + i % (padded - groups)) * SLOTS, SLOTS, 0.f);
   } else {
     const bool inside = n0 + 64 * wave < N;  // (else the wave's columns repeat the last one)
 #pragma unroll
@@ -471,7 +399,7 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
 // 58.7 us for the call = 444 TFLOP/s (tiles of 64 x 128 with the codes loaded into registers 63.4).
 // Blocks (128 experts, hidden 2048, 4-bit, groups of 64), us of a forward at 128 / 320 / 1024 tokens, even routing: 127 / 132 / 221; with streamed
 // segments, 256-column tiles and a copy of x on four streams, which they took before, 151 / 216 / 266.
-template <int DT, int BITS, bool G32, bool GLU, bool MID, int MS, int NT, int WN, int KW, int S>
+template <int DT, int BITS, bool G32, bool LIST, bool GLU, bool MID, int MS, int NT, int WN, int KW, int S>
 __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t row0, int rows, int n0, int scale_shift, unsigned char *lds_raw) {
   typedef Tile<DT, BITS, G32, MID, MS, NT, WN, S> P;
   typedef typename P::R R;
@@ -500,11 +428,11 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
     wr[t] = words_of((t ? a.w1 : a.w0) + ebase * (row_bytes / 4), (uint32_t)N * row_bytes);
     sr[t] = words_of(s_of[t], (uint32_t)N * G * sizeof(T)), br[t] = words_of(b_of[t], (uint32_t)N * G * sizeof(T));  // (read in words: the host takes an even number of them)
   }
-  // weight row of place `at` (0 .. 31) of the wave's tile t.  Columns past the end repeat the last one (never stored).  Paired output
-  // (see GroupedArgs::y_paired): the place p of an 8-block takes the row whose result belongs there.
+  // weight row of place `at` (0 .. 31) of the wave's tile t.  Columns past the end repeat the last one (never stored).  Order of the output
+  // (CodesArgs::y_order): the place p of an 8-block takes the row whose result belongs there.
   const int col0 = n0 + 32 * (GLU ? 1 : NT) * wave;
   auto weight_row = [&](int t, int at) __attribute__((always_inline)) {
-    const int p = a.y_paired ? ((at & ~7) | (((at & 7) >> 1) + ((at & 1) ? 4 : 0))) : at, row = col0 + (GLU ? 0 : 32 * t) + p;
+    const int p = (at & ~7) | value_at_place(a.y_order, at & 7), row = col0 + (GLU ? 0 : 32 * t) + p;
     return row < N ? row : N - 1;
   };
   // ---- what a lane copies, and where it lies in LDS.  LDS gives 256 bytes a cycle, sixteen lanes' pieces, if they lie in different
@@ -790,7 +718,7 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
     block_barrier();
   }
   uint32_t dst[2] = {};
-  if constexpr (P::kPlainCodes && !GLU) output_rows(a, row0, rows, lane, dst);
+  if constexpr (LIST && !GLU) output_rows(a, row0, rows, lane, dst);
   wait_copies<0>();
   block_barrier();
 
@@ -828,8 +756,8 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
     if (kg != 0) return;
   }
 
-  if constexpr (P::kPlainCodes) write_piece<GLU, MS>(a, tot, wave, lane, n0, row0, rows, ebase, weight_row, dst, lds_raw);
-  else write_tile<DT, BITS, GLU, MS, NT, WN>(a, tot, wave, lane, n0, col0, row0, rows, ebase, glog, weight_row, lds_raw);
+  if constexpr (LIST) write_piece<BITS, P::kPlainCodes, GLU, MS>(a, tot, wave, lane, n0, row0, rows, ebase, glog, weight_row, dst, lds_raw);
+  else write_tile<DT, BITS, MS, NT, WN>(a, tot, wave, lane, col0, row0, rows, glog, weight_row, lds_raw);
 }
 
 
@@ -863,7 +791,7 @@ __device__ __forceinline__ void multiply_long_tile(const CodesArgs &a, int e, in
   }
   const int col0 = n0 + (GLU ? 32 : 64) * wave;
   auto weight_row = [&](int t, int at) __attribute__((always_inline)) {
-    const int p = a.y_paired ? ((at & ~7) | (((at & 7) >> 1) + ((at & 1) ? 4 : 0))) : at, row = col0 + (GLU ? 0 : 32 * t) + p;
+    const int p = (at & ~7) | value_at_place(a.y_order, at & 7), row = col0 + (GLU ? 0 : 32 * t) + p;
     return row < N ? row : N - 1;
   };
   auto turned = [](int row) __attribute__((always_inline)) { return (row >> 1) & 7; };
@@ -1034,7 +962,7 @@ __device__ __forceinline__ void multiply_long_tile(const CodesArgs &a, int e, in
   if constexpr (!GLU) output_rows(a, row0, rows, lane, dst);
   wait_copies<0>();
   block_barrier();
-  write_piece<GLU, MS>(a, tot, wave, lane, n0, row0, rows, ebase, weight_row, dst, lds_raw);
+  write_piece<4, true, GLU, MS>(a, tot, wave, lane, n0, row0, rows, ebase, 6, weight_row, dst, lds_raw);
 }
 
 // The tiles of a list of pieces of up to 128 rows (ShortTiles::piece), 4-bit codes in groups of 64: by their rows, 32 at a time.
@@ -1054,18 +982,18 @@ __global__ __launch_bounds__(256, 2) void qmm_pieces_kernel(CodesArgs a, const u
   extern __shared__ __align__(16) unsigned char lds_raw[];
   if (rows > 96) return multiply_long_tile<GLU, 4>(a, e, row0, rows, nt * NI, lds_raw);
   if (rows > 64) return multiply_long_tile<GLU, 3>(a, e, row0, rows, nt * NI, lds_raw);
-  if (rows > 32) return multiply_tile<0, 4, false, GLU, true, 2, 2, 4, 1, 2>(a, e, row0, rows, nt * NI, 0, lds_raw);
+  if (rows > 32) return multiply_tile<0, 4, false, true, GLU, true, 2, 2, 4, 1, 2>(a, e, row0, rows, nt * NI, 0, lds_raw);
   typedef Ring<4, 1, 2, 4, 2> Short;
   constexpr int S1 = (kHalfLds - 4 * Short::WINDOW) / Short::STAGE;  // as many stages as fit
-  multiply_tile<0, 4, false, GLU, true, 1, 2, 4, 1, S1>(a, e, row0, rows, nt * NI, 0, lds_raw);
+  multiply_tile<0, 4, false, true, GLU, true, 1, 2, 4, 1, S1>(a, e, row0, rows, nt * NI, 0, lds_raw);
 }
 
 // A block computes 32 MS token rows x 32 WN weight rows with WN KW waves (see codes_tile), tiles of up to 32 rows with half the
 // token operand.
-template <int DT, int BITS, bool G32, bool GLU, bool MID, int MS, int NT, int WN, int KW, int S>
+template <int DT, int BITS, bool G32, bool LIST, bool GLU, int MS, int NT, int WN, int KW, int S>
 __global__ __launch_bounds__(64 * WN * KW, waves_of(WN * KW, lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES))) void qmm_tiles_kernel(
     CodesArgs a, const uint32_t *__restrict__ list, int n_mtiles, int n_ntiles, int scale_shift) {
-  static_assert(!GLU || NT == 2, "a gate tile and its up tile");
+  static_assert(LIST ? DT == 0 && NT == 2 && WN == 4 && KW == 1 : !GLU, "write_piece: a gate tile and its up tile, or two tiles a wave");
   constexpr int BM = 32 * MS;
   constexpr int NI = 32 * WN * (GLU ? 1 : NT);  // distinct output columns per block
   // block -> (M tile, N tile).  Ids are dealt round-robin over the 8 XCDs.  Dense: an XCD takes every eighth N tile
@@ -1074,7 +1002,7 @@ __global__ __launch_bounds__(64 * WN * KW, waves_of(WN * KW, lds_of(KW, Ring<BIT
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
   int e = 0, rows, nt;
   int64_t row0;
-  if (list) {
+  if constexpr (LIST) {
     const uint32_t id = (uint32_t)(j / n_ntiles) * 8u + xcd;
     nt = j % n_ntiles;
     if (id >= list[0]) return;
@@ -1093,41 +1021,53 @@ __global__ __launch_bounds__(64 * WN * KW, waves_of(WN * KW, lds_of(KW, Ring<BIT
     if (rows <= 32) {
       typedef Ring<BITS, 1, NT, WN, 2> Short;
       constexpr int S1 = (lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES) / KW - WN * Short::WINDOW) / Short::STAGE;  // as many stages as fit
-      multiply_tile<DT, BITS, G32, GLU, MID, 1, NT, WN, KW, S1>(a, e, row0, rows, nt * NI, scale_shift, lds_raw);
+      multiply_tile<DT, BITS, G32, LIST, GLU, false, 1, NT, WN, KW, S1>(a, e, row0, rows, nt * NI, scale_shift, lds_raw);
       return;
     }
   }
-  multiply_tile<DT, BITS, G32, GLU, MID, MS, NT, WN, KW, S>(a, e, row0, rows, nt * NI, scale_shift, lds_raw);
+  multiply_tile<DT, BITS, G32, LIST, GLU, false, MS, NT, WN, KW, S>(a, e, row0, rows, nt * NI, scale_shift, lds_raw);
 }
 
 size_t codes_copy_bytes(int bits, int64_t rows, int K) {
-  return paired_order(bits) ? (size_t)rows * K * 2 : 0;
+  return row_order(bits) != RowOrder::kPlain ? (size_t)rows * K * 2 : 0;
 }
 size_t codes_sums_bytes(int64_t rows, int K, int group, bool plain) { return (size_t)rows * padded_groups(K / group) * sum_slots(plain) * 2; }
 
+PrepareArgs prepare_args(const void *x, int64_t rows, int K, int group, uint16_t *copy, uint16_t *sums, bool plain) {
+  PrepareArgs a;
+  a.x = x;
+  a.octets = rows * (K / 8);
+  a.octets_per_row = K / 8;
+  a.lanes_log2 = group == 32 ? 2 : (group == 64 ? 3 : 4);
+  a.copy = copy;
+  a.sums = sums;
+  a.slots = sum_slots(plain);
+  a.sums_row = padded_groups(K / group) * a.slots;
+  a.order = plain ? RowOrder::kQuads : RowOrder::kPaired;
+  return a;
+}
 hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
                                uint16_t *sums, bool plain, hipStream_t st) {
-  const int64_t n = rows * (K / 8);
-  if (n == 0) return hipSuccess;
-  const unsigned grid = (unsigned)((n + 255) / 256);
-  const int ll = group == 32 ? 2 : (group == 64 ? 3 : 4), slots = sum_slots(plain), row = padded_groups(K / group) * slots;
-  if (dt == 0) prepare_rows_kernel<0><<<grid, 256, 0, st>>>(static_cast<const uint16_t *>(x), n, K / 8, ll, copy, sums, row, slots);
-  else if (dt == 1) prepare_rows_kernel<1><<<grid, 256, 0, st>>>(static_cast<const _Float16 *>(x), n, K / 8, ll, copy, sums, row, slots);
+  const PrepareArgs a = prepare_args(x, rows, K, group, copy, sums, plain);
+  if (a.octets == 0) return hipSuccess;
+  const unsigned grid = (unsigned)((a.octets + 255) / 256);
+  if (dt == 0) prepare_rows_kernel<0><<<grid, 256, 0, st>>>(a);
+  else if (dt == 1) prepare_rows_kernel<1><<<grid, 256, 0, st>>>(a);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
-template <int DT, int BITS, bool G32, bool GLU, bool MID, int MS, int NT, int WN, int KW, int S>
+template <int DT, int BITS, bool G32, bool LIST, bool GLU, int MS, int NT, int WN, int KW, int S>
 static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_t *list, int cap, hipStream_t st) {
   constexpr int NI = 32 * WN * (GLU ? 1 : NT), BM = 32 * MS;
-  constexpr int bufs = lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES), sums = KW > 1 ? BM * 32 * WN * NT * 4 : WN * (32 * 80 + BM * 4);
+  constexpr int bufs = lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES), sums = KW > 1 ? BM * 32 * WN * NT * 4 : 0;
   constexpr int lds = bufs > sums ? bufs : sums;
   static_assert(lds <= 160 * 1024, "more LDS than a CU has");
   const int n_ntiles = (a.N + NI - 1) / NI;
-  const int mtiles = list ? cap : (int)((a.M + BM - 1) / BM);
-  const int64_t grid = list ? ((int64_t)cap + 7) / 8 * 8 * n_ntiles : (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
+  const int mtiles = LIST ? cap : (int)((a.M + BM - 1) / BM);
+  const int64_t grid = LIST ? ((int64_t)cap + 7) / 8 * 8 * n_ntiles : (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
   if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
-  const auto kernel = &qmm_tiles_kernel<DT, BITS, G32, GLU, MID, MS, NT, WN, KW, S>;
+  const auto kernel = &qmm_tiles_kernel<DT, BITS, G32, LIST, GLU, MS, NT, WN, KW, S>;
   if (lds > 64 * 1024) {
     static std::atomic<uint64_t> allowed{0};
     if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), (int)lds, allowed); e != hipSuccess) return e;
@@ -1188,8 +1128,8 @@ hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int 
   auto run = [&](auto b, auto g32) {
     constexpr int BITS = decltype(b)::value;
     constexpr bool G32 = decltype(g32)::value;
-    if (glu) return start_tiles<0, BITS, G32, true, false, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
-    return start_tiles<0, BITS, G32, false, false, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
+    if (glu) return start_tiles<0, BITS, G32, true, true, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
+    return start_tiles<0, BITS, G32, true, false, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
   };
   const std::true_type yes{};
   const std::false_type no{};

@@ -72,6 +72,30 @@ def test_blocks_in_longer_pieces(zipf, rows, hidden, inter, experts, k):
     assert float((own.double() - ref).norm() / ref.norm()) <= 2.0 ** -8
 
 
+@pytest.mark.parametrize("group", [32, 128])
+@pytest.mark.parametrize("bits", [4, 8])
+# a decode batch (the router's one launch) and larger ones; rows of an odd number of groups of 128, of more than a window, columns that fill no block;
+# the last two around the rows an expert between which 8-bit codes keep short segments apart
+@pytest.mark.parametrize("hidden,inter,experts,k,tokens", [(128, 384, 8, 2, 17), (384, 128, 4, 2, 64), (2176, 640, 9, 3, 70), (384, 1152, 16, 8, 300),
+                                                           (256, 256, 8, 2, 79), (256, 256, 8, 2, 80)])
+def test_blocks_all_in_tiles(hidden, inter, experts, k, tokens, bits, group):
+    """Groups of 32 and 128, segments of every length in tiles; the bound is test_blocks_in_short_tiles'."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(hidden, experts, k, inter, bits, group, 0)
+    blk = synth.make_block(cfg, seed=group, device="cuda", zipf_s=0.7, gen_device="cuda")
+    x = synth.make_tokens(cfg, tokens, seed=bits, device="cuda")
+    out, routing = blk.forward(x, debug=True)
+    ref = block_truth(blk, x, routing)
+    assert float((out.double() - ref).norm() / ref.norm()) <= 2.0 ** -8
+    p = torch.randperm(tokens, generator=torch.Generator().manual_seed(3)).cuda()
+    assert torch.equal(blk.forward(x[p].contiguous()), out[p])
+    one = torch.ones(hidden, dtype=torch.bfloat16, device="cuda")
+    own, routing = blk.forward_residual(x, one, 1e-6, debug=True)
+    ref = x.double() + block_truth(blk, m.ops.rms_norm(x, one, 1e-6), routing)
+    assert float((own.double() - ref).norm() / ref.norm()) <= 2.0 ** -8
+
+
 def test_a_layer_around_short_tiles():
     """The normalised rows' memory takes the group sums of h once they have been read: the residual form against its parts."""
     import mlx_rs_amd as m
