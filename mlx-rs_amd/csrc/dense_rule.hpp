@@ -61,4 +61,18 @@ constexpr DenseTile dense_tile(int64_t M, int N, int K, int bits, int group, boo
   return x <= 32 ? DenseTile::kRegisters64x128Shared : DenseTile::kRegisters64x128;
 }
 
+// Tiles of 96 or 128 token rows x 128 weight rows, K shared by two groups of waves, one block a CU (qmm_tiles.hip): where they fill the chip in one round and
+// tiles of 64 x 128 would give some CUs two blocks and others one.  0: dense_tile's.  Measured, us of the call, dense_tile's / these (84 shapes of 96 rows with
+// 4-bit codes, 64 with 8-bit ones, 1.00 to 1.33 times as fast, longer K more):
+//   96 rows   bf16 4-bit 640 x 4096 x 4096 53.2 / 41.1, 650 x 2864 x 1152 22.1 / 20.8, 902 x 2288 x 3584 49.1 / 39.2, in groups of 32 926 x 2928 x 3584 58.6 / 48.0,
+//             542 x 3248 x 1152 24.9 / 24.1, of 128 549 x 3888 x 3840 48.6 / 36.6; f16 8-bit 868 x 2944 x 2688 35.7 / 30.9, in groups of 32 718 x 4016 x 1152
+//             23.3 / 23.5, of 128 562 x 3760 x 3456 40.7 / 32.8
+//   128 rows  8-bit: K = 3072 43.8 / 42.5, 40.0 / 36.8, 44.3 / 42.0 (128), 55.1 / 51.9 (32), 3328 44.2 / 41.5, 4096 51.1 / 46.3, 62.0 / 59.3 (32); below
+//             that 1664 26.8 / 27.3, 2688 38.7 / 38.3, 43.3 / 45.3 (32), 1152 21.2 / 22.1, 1280 24.2 / 27.2 (32).  4-bit: two groups' stages are more LDS than a CU has
+constexpr int long_tile_rows(int64_t M, int N, int K, int bits) {
+  if (K < 1024 || tiles_of_an_xcd(M, N, 64, 128) <= 32) return 0;
+  if (tiles_of_an_xcd(M, N, 96, 128) <= 32) return 96;
+  return bits == 8 && K >= 3072 && tiles_of_an_xcd(M, N, 128, 128) <= 32 ? 128 : 0;
+}
+
 }  // namespace mi_moe

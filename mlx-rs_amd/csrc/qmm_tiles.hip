@@ -1076,7 +1076,7 @@ static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_
   return hipGetLastError();
 }
 
-// Which tile: dense_tile (dense_rule.hpp).  Before that rule, us of the whole call, bf16 4-bit / f16 8-bit, groups of 64 (M, N, K):
+// Which tile: long_tile_rows, else dense_tile (dense_rule.hpp).  Before those rules, us of the whole call, bf16 4-bit / f16 8-bit, groups of 64 (M, N, K):
 //                                       (96, 4096, 4096) (200, 4096, 4096) (1000, 1024, 4096) (400, 4096, 4096) (640, 2304, 2304) (777, 4096, 4096) (2048, 4096, 4096)
 //   32 x 64, K shared by four groups       16.9 / 17.5      29.0 / 24.6       40.1 / 28.8        55.7 / 45.1       43.5 / 33.6       102 / 90          - / 211
 //   32 x 128, four groups                  21.5 / 22.3      25.8 / 27.2       31.2 / 31.9        49.7 / 52.8       35.8 / 37.0       94 / 106          - / 214
@@ -1090,7 +1090,10 @@ static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_
 // bf16 takes the larger tiles (2048 rows) in qmm_large.hip.
 template <int DT, int BITS, bool G32>
 static hipError_t start_dense(const CodesArgs &a, int group, hipStream_t st) {
-  const int scale_shift = group == 128;
+  const int scale_shift = group == 128, longer = long_tile_rows(a.M, a.N, a.K, BITS);
+  if (longer == 96) return start_tiles<DT, BITS, G32, false, false, 3, 1, 4, 2, BITS == 4 ? 2 : 3>(a, scale_shift, nullptr, 0, st);
+  if constexpr (BITS == 8)
+    if (longer == 128) return start_tiles<DT, BITS, G32, false, false, 4, 1, 4, 2, 3>(a, scale_shift, nullptr, 0, st);
   switch (dense_tile(a.M, a.N, a.K, BITS, group, DT == 0)) {
     case DenseTile::k32x64: return start_tiles<DT, BITS, G32, false, false, 1, 1, 2, 4, 2>(a, scale_shift, nullptr, 0, st);
     case DenseTile::kRegisters32x64: return launch_qmm_codes_small(a, st);

@@ -13,12 +13,14 @@ def rule(tmp_path_factory):
     d = tmp_path_factory.mktemp("rule")
     (d / "rule.cpp").write_text('#include "dense_rule.hpp"\n'
                                 'extern "C" int share(int K, int n, int pairs) { return mi_moe::share_of_k(K, n, pairs != 0); }\n'
-                                'extern "C" int tile(long M, int N, int K, int bits, int group, int bf16) { return (int)mi_moe::dense_tile(M, N, K, bits, group, bf16 != 0); }\n')
+                                'extern "C" int tile(long M, int N, int K, int bits, int group, int bf16) { return (int)mi_moe::dense_tile(M, N, K, bits, group, bf16 != 0); }\n'
+                                'extern "C" int longer(long M, int N, int K, int bits) { return mi_moe::long_tile_rows(M, N, K, bits); }\n')
     so = d / "rule.so"
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", os.path.join(ROOT, "mlx-rs_amd", "csrc"),
                     str(d / "rule.cpp"), "-o", str(so)], check=True)
     lib = C.CDLL(str(so))
     lib.tile.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int]
+    lib.longer.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int]
     return lib
 
 
@@ -54,3 +56,11 @@ def test_the_tile_follows_the_fullest_xcd(rule, shape, bits, group, want):
                                                         ((258, 1744, 1408), 8, 32, 1, SMALL), ((102, 1808, 3584), 8, 32, 0, SMALL), ((102, 1808, 3584), 8, 64, 1, SMALL), ((102, 1808, 3584), 4, 32, 1, SMALL)])
 def test_small_tiles_with_every_code_converted_stay_in_registers(rule, shape, bits, group, bf16, want):
     assert rule.tile(*shape, bits, group, bf16) == want
+
+
+@pytest.mark.parametrize("shape,bits,want", [
+    ((512, 4096, 4096), 8, 0), ((513, 4096, 4096), 8, 96), ((768, 4096, 4096), 4, 96), ((769, 4096, 4096), 8, 128), ((1024, 4096, 4096), 8, 128), ((1025, 4096, 4096), 8, 0),
+    ((769, 4096, 4096), 4, 0), ((769, 4096, 2944), 8, 0), ((769, 4096, 3072), 8, 128), ((640, 4096, 896), 4, 0), ((640, 4096, 1024), 4, 96),
+    ((640, 2304, 2304), 4, 0), ((641, 2304, 2304), 4, 96), ((960, 2304, 2304), 8, 96), ((961, 2304, 4096), 8, 128)])
+def test_longer_tiles_where_they_are_one_round(rule, shape, bits, want):
+    assert rule.longer(*shape, bits) == want

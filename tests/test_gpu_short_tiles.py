@@ -178,6 +178,48 @@ def test_every_dense_tile_loses_no_more_than_plain_sums(rows, tiles, bits, dtype
     assert share <= allowed, (share, allowed)
 
 
+@pytest.mark.parametrize("dtype,group", [("float16", 32), ("float16", 64), ("float16", 128), ("bfloat16", 32), ("bfloat16", 64), ("bfloat16", 128)])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows,n,k", [(585, 4090, 1024), (550, 4096, 1152), (640, 3200, 2176), (770, 4090, 3072), (1000, 4096, 3200)])
+def test_longer_tiles_lose_no_more_than_plain_sums(rows, n, k, bits, dtype, group, rule):
+    """96 and 128 rows: a last tile of 9, 2 and 104 rows, columns that end inside one, shares of 4 and 4, 5 and 4, 9 and 8, 13 and 12 stages of 128 values.  The
+    bounds are test_every_dense_tile_loses_no_more_than_plain_sums'."""
+    import mlx_rs_amd as m
+    want = 96 if rows < 700 else 128 if bits == 8 else 0
+    assert rule.longer(rows, n, k, bits) == want
+    if not want:
+        pytest.skip("another tile with 4-bit codes")
+    dt = getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(rows + group + bits)
+    q, s, b = m.ops.quantize(torch.randn((n, k), generator=gen, device="cuda") * 0.02, group, bits, dt)
+    x = torch.randn((rows, k), generator=gen, device="cuda").to(dt)
+    x[rows - 1, 5] = float("inf")  # (one result in a row of its own that is computed again)
+    ref = product(x, q, s, b, group, bits)
+    y = m.ops.quantized_linear(x, q, s, b, group_size=group, bits=bits)
+    assert torch.equal(y[-1].double().nan_to_num(), ref[-1].nan_to_num())
+    y, ref = y[:-1], ref[:-1]
+    err = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= BOUND[dtype], float(err.max())
+    share, allowed = share_off_nearest(y, ref, 2.0 ** -22 * ref.square().mean().sqrt())
+    assert share <= allowed, (share, allowed)
+
+
+# (the tiles of 64 x 128 in registers where a tile of 96 or 128 rows does not fill a round: 8-bit codes, K below 3072)
+@pytest.mark.parametrize("dtype,group", [("float16", 32), ("float16", 64), ("bfloat16", 64), ("bfloat16", 128)])
+def test_tiles_in_registers_beside_longer_ones(dtype, group, rule):
+    import mlx_rs_amd as m
+    rows, n, k = 777, 4096, 2048
+    assert rule.longer(rows, n, k, 8) == 0 and rule.tile(rows, n, k, 8, group, dtype == "bfloat16") == REGISTERS
+    dt = getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(group)
+    q, s, b = m.ops.quantize(torch.randn((n, k), generator=gen, device="cuda") * 0.02, group, 8, dt)
+    x = torch.randn((rows, k), generator=gen, device="cuda").to(dt)
+    ref = product(x, q, s, b, group, 8)
+    y = m.ops.quantized_linear(x, q, s, b, group_size=group, bits=8)
+    share, allowed = share_off_nearest(y, ref, 2.0 ** -22 * ref.square().mean().sqrt())
+    assert share <= allowed, (share, allowed)
+
+
 def one_hot(n, value):
     """A bank's matrix, 4-bit in groups of 64: `value` on the diagonal, or in column 0 (n < 0), exactly."""
     codes = torch.zeros((abs(n), abs(n)), dtype=torch.int64)
