@@ -15,10 +15,12 @@
 // third pieces (another step inside the loop would spill): the weights are those of the plain product in every case.
 // A result that is not finite is computed again the plain way, one fma per k: pieces of an infinity are no numbers, and
 // where nothing but a piece has overflowed that gives the number.  That is a lane's own chain over K, for eight results at a time.
-// us of the call with finite rows / one infinity in one row / one in each: 1000 x 2048 x 4096 bf16 48 / 425 / 960 (a thread per packed word 1360;
+// us of the call with finite rows / one infinity in one row / one in each (before the weights left LDS): 1000 x 2048 x 4096 bf16 48 / 425 / 960 (a thread per packed word 1360;
 // one result at a time 50 / 1620 / 11700); 20 rows f16 20 / 256 / 270, weights beyond 64 270 (4120).
 #include <type_traits>
 
+#include "dense_rule.hpp"
+#include "lds_copies.hpp"
 #include "qmm_dev.hpp"
 
 namespace mi_moe {
@@ -50,14 +52,14 @@ __device__ __forceinline__ void split_pair(float v0, float v1, uint32_t (&to)[P]
   }
 }
 
-// LDS of a wave: x [pieces][32 MS rows][32 K values], w [pieces][32 NT columns][32 K values], (s, b) of 32 K values of
-// two groups.  A row is four 16-byte chunks; chunk c of row r sits at c ^ (r / 4 % 4), so that the 16 lanes of one LDS
+// LDS of a wave: x [pieces, or two steps in turn][32 MS rows][32 K values], (s, b) of 32 K values of two groups.  A row is four 16-byte chunks; chunk c of row r sits at c ^ (r / 4 % 4), so that the 16 lanes of one LDS
 // cycle, which read one chunk of 16 rows or write four chunks of four, meet 16 different places.
 constexpr int kRowPieces = 4;
 __device__ __forceinline__ int at(int row, int chunk) { return row * kRowPieces + (chunk ^ ((row >> 2) & 3)); }
 constexpr int kScaleRow = 32 * 8 + 16;  // bytes of one group's (s, b) pairs
+constexpr bool rows_copied(int dt, int nt) { return dt != 2 && nt == 2; }
 constexpr int wave_lds(int dt, int ms, int nt) {
-  return (pieces_of_x(dt) * ms + pieces_of_w(dt) * nt) * 32 * kRowPieces * 16 + 2 * kScaleRow;
+  return (rows_copied(dt, nt) ? 2 : pieces_of_x(dt)) * ms * 32 * kRowPieces * 16 + 2 * kScaleRow;
 }
 
 }  // namespace
@@ -65,27 +67,29 @@ constexpr int wave_lds(int dt, int ms, int nt) {
 // A block computes 32 MS rows x 32 NT columns; its KW waves share K among them, each on LDS of its own, and meet only to
 // add their sums: no wave waits for another in the loop, so the unpacking of one runs beside the multiplies of the other
 // on its SIMD.  A lane unpacks eight K values of 2 NT consecutive columns (a byte to a word of eight rows): the eight
-// values of a column are then one 16-byte chunk of a weight operand, and no exchange between lanes is needed although
-// memory holds the codes the other way round.  The columns are dealt to the sub-tiles so that a lane ends up with NT
+// values of a column are then one 16-byte chunk of a weight operand.  Sixteen lanes hold an octet of K values, a multiply takes octets 2 h and 2 h + 1, and
+// an exchange of sixteen lanes between two columns' registers (v_permlane16_swap) brings each where it is multiplied: the weights never
+// pass through LDS.  The columns are dealt to the sub-tiles so that a lane ends up with NT
 // consecutive ones: column n = 2 NT u + j goes to place 16 (j % NT * 2 + j / NT) + u, that is
 // sub-tile j % NT, lane 16 (j / NT) + u.
 // What bounds it (128 x 64 tiles, bf16): a step of a wave is 1024 cycles of matrix work (two products) beside about 800 of
-// unpacking and 32 KB through LDS, each near the CU's rate.  1000 x 2048 x 4096, 4-bit, groups of 64: 47 us for the call,
-// 360 TFLOP/s of the product (a thread per packed word of an output row, one k after the other: 1360 us); 8 rows 19 us
-// (1450); f32 141 us (1350).
+// unpacking and 16 KB of rows through LDS.  1000 x 2048 x 4096, 4-bit, groups of 64: 41.5 us for the call, 400 TFLOP/s of the product
+// (weights through LDS as well, rows by way of registers 46.5, of which unpacking was 6, the second product 7, the rows' LDS traffic 9).  Unpacking the next step between the multiplies of this one: 41.5 too.
+// 1 row 17.8 us (19.1), f32 118 (124).
 // Error: share of results that are not the float64 product's nearest value, here / a thread per packed word: 300 x 2048 x 2048 bf16 1.1e-4
 // to 2.2e-4 / 1.8e-4 to 5.4e-4, f16 1.2e-3 / 3.6e-3; groups at 1 + q / 2^13 and rows that sum to zero, bf16, 3e-3 to 1.1e-2 / 1.4e-3 to
-// 3.2e-3 (two pieces alone: 0.11 to 0.14); f32 against 64 bits 4.9e-7 / 1.07e-6.  What looking at the scales costs: 1 us of 47.
+// 3.2e-3 (two pieces alone: 0.11 to 0.14); f32 against 64 bits 4.9e-7 / 1.07e-6.  What looking at the scales cost: 1 us of 47.
 template <int DT, int BITS, int MS, int NT, int KW>
 __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mtiles, int n_ntiles, int group_log2) {
   typedef typename ElemOf<DT>::type T;
   typedef typename std::conditional<BITS * NT == 4, uint8_t, typename std::conditional<BITS * NT == 16, uint32_t, uint16_t>::type>::type Codes;
   constexpr int PX = pieces_of_x(DT), PW = pieces_of_w(DT);
   constexpr float kFactor = factor_of_w(DT);
+  constexpr bool kCopied = rows_copied(DT, NT);
   constexpr int CN = 2 * NT;          // columns a lane unpacks
   constexpr int NX = 2 * MS;          // 16-row pieces of the token rows
   constexpr int XP = DT == 2 ? 2 : 1; // 16-byte pieces of eight values of x
-  constexpr int X_SZ = 32 * MS * kRowPieces, W_SZ = 32 * NT * kRowPieces;
+  constexpr int X_SZ = 32 * MS * kRowPieces;
   static_assert(sizeof(Codes) * 8 == BITS * CN, "a lane's columns of one row are one load");
 
   // block -> tile.  Ids are dealt round-robin over the 8 XCDs: an XCD takes every eighth column tile and all row tiles
@@ -101,13 +105,12 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
   u32x4_t *const Xs = reinterpret_cast<u32x4_t *>(lds_raw + wave * wave_lds(DT, MS, NT));
-  u32x4_t *const Ws = Xs + PX * X_SZ;
-  unsigned char *const Ss = reinterpret_cast<unsigned char *>(Ws + PW * W_SZ);
+  unsigned char *const Ss = reinterpret_cast<unsigned char *>(Xs + (kCopied ? 2 : PX) * X_SZ);
 
   // ---- this lane's share of a step: rows xrow + 16 i and chunk oct of x; columns CN u .. and rows 8 oct .. of the codes;
   // row lane % 32 of the scales and biases, of the tile's first (lane / 32 = 0) or second 32 columns
   const int xrow = lane >> 2, xoct = lane & 3;
-  const int u = lane & 15, oct = lane >> 4;
+  const int u = lane & 15, oct = (lane >> 4 & 1) * 2 + (lane >> 5);
   int wcol = n0 + CN * u;
   wcol = wcol < N ? wcol : N - CN;  // columns past the end repeat the last ones (never stored)
   const int skl = lane & 31;
@@ -115,22 +118,36 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
   sgroup = sgroup < G ? sgroup : G - 1;
   const T *const sp = static_cast<const T *>(a.s), *const bp = static_cast<const T *>(a.b);
 
+  const uint32_t x_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds_raw + (uint32_t)(wave * wave_lds(DT, MS, NT));
+  // Rows of the tiles of 64 columns are copied straight into LDS, a step ahead of the one that is multiplied, whose multiplies cover the copies; narrower
+  // tiles' do not (32 x 32 tiles, one row x 2048 x 4096 17.8 us, copied 27.0), and f32 rows are split on the way.
+  auto copy_rows = [&](int ks, int place) __attribute__((always_inline)) {
+    const int k = ks * kStep;
+    const i32x4_t from = words_of(static_cast<const T *>(a.x) + row0 * K + k, ((uint32_t)rows * K - k) * (uint32_t)sizeof(T));
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int row = xrow + 16 * i, chunk = xoct ^ (row >> 2 & 3);
+      copy_to_lds(from, k + 8 * chunk < K ? (row * (uint32_t)K + 8 * chunk) * (uint32_t)sizeof(T) : kOutside, 0, x_at + place * (X_SZ * 16) + i * 1024);
+    }
+  };
   struct Stage {
-    u32x4_t x[NX][XP];
+    u32x4_t x[kCopied ? 1 : NX][XP];
     uint32_t q[8];
     T s, b;
   };
   auto load = [&](int ks, Stage &R) __attribute__((always_inline)) {
     const int k = ks * kStep;
     // rows past the end are past the descriptor, K values past the end are sent there: both read zeros
-    const __amdgpu_buffer_rsrc_t xr = rsrc_of(static_cast<const T *>(a.x) + row0 * K + k, ((uint32_t)rows * K - k) * (uint32_t)sizeof(T));
+    if constexpr (!kCopied) {
+      const __amdgpu_buffer_rsrc_t xr = rsrc_of(static_cast<const T *>(a.x) + row0 * K + k, ((uint32_t)rows * K - k) * (uint32_t)sizeof(T));
 #pragma unroll
-    for (int i = 0; i < NX; ++i)
+      for (int i = 0; i < NX; ++i)
 #pragma unroll
-      for (int p = 0; p < XP; ++p) {
-        const uint32_t off = ((xrow + 16 * i) * (uint32_t)K + 8 * xoct) * (uint32_t)sizeof(T) + 16 * p;
-        R.x[i][p] = __builtin_amdgcn_raw_buffer_load_b128(xr, k + 8 * xoct < K ? off : kOutside, 0, 0);
-      }
+        for (int p = 0; p < XP; ++p) {
+          const uint32_t off = ((xrow + 16 * i) * (uint32_t)K + 8 * xoct) * (uint32_t)sizeof(T) + 16 * p;
+          R.x[i][p] = __builtin_amdgcn_raw_buffer_load_b128(xr, k + 8 * xoct < K ? off : kOutside, 0, 0);
+        }
+    }
     const int left = K - k < kStep ? K - k : kStep;  // rows past the end read zeros, with a scale and a bias of zero
     const __amdgpu_buffer_rsrc_t wr = rsrc_of(reinterpret_cast<const unsigned char *>(a.w) + (int64_t)k * row_bytes, (uint32_t)left * row_bytes);
 #pragma unroll
@@ -162,26 +179,29 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
     most = ahead > most ? ahead : most;
     least = b << 1 != 0u && ahead < least ? ahead : least;
   };
+  u32x4_t op[2][NT][PW];  // the weights of a step as operands of its two multiplies
   // rows, and pieces FIRST .. FIRST + COUNT - 1 of the weights
   auto put = [&](const Stage &R, auto first, auto count) __attribute__((always_inline)) {
     constexpr int FIRST = decltype(first)::value, COUNT = decltype(count)::value;
     *reinterpret_cast<float2 *>(Ss + (lane >> 5) * kScaleRow + skl * 8) = make_float2(kFactor * as_f32(R.s), kFactor * as_f32(R.b));
+    if constexpr (!kCopied) {
 #pragma unroll
-    for (int i = 0; i < NX; ++i) {
-      u32x4_t *const to = Xs + at(xrow + 16 * i, xoct);
-      if constexpr (DT != 2) {
-        *to = R.x[i][0];
-      } else {
-        u32x4_t o[PX];
+      for (int i = 0; i < NX; ++i) {
+        u32x4_t *const to = Xs + at(xrow + 16 * i, xoct);
+        if constexpr (DT != 2) {
+          *to = R.x[i][0];
+        } else {
+          u32x4_t o[PX];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          uint32_t pc[PX];
-          split_pair<DT, PX>(__uint_as_float(R.x[i][c >> 1][2 * (c & 1)]), __uint_as_float(R.x[i][c >> 1][2 * (c & 1) + 1]), pc);
+          for (int c = 0; c < 4; ++c) {
+            uint32_t pc[PX];
+            split_pair<DT, PX>(__uint_as_float(R.x[i][c >> 1][2 * (c & 1)]), __uint_as_float(R.x[i][c >> 1][2 * (c & 1) + 1]), pc);
 #pragma unroll
-          for (int p = 0; p < PX; ++p) o[p][c] = pc[p];
+            for (int p = 0; p < PX; ++p) o[p][c] = pc[p];
+          }
+#pragma unroll
+          for (int p = 0; p < PX; ++p) to[p * X_SZ] = o[p];
         }
-#pragma unroll
-        for (int p = 0; p < PX; ++p) to[p * X_SZ] = o[p];
       }
     }
     wave_fence();
@@ -201,11 +221,17 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
         for (int p = 0; p < COUNT; ++p) o[c][p][r] = pc[FIRST + p];
       }
     }
+    // columns t and NT + t of the lanes of octets 0 and 2 (1 and 3): an exchange of sixteen lanes leaves each octet in the half that multiplies it
 #pragma unroll
-    for (int c = 0; c < CN; ++c)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int p = 0; p < COUNT; ++p) Ws[p * W_SZ + at(16 * (c % NT * 2 + c / NT) + u, oct)] = o[c][p];
-    wave_fence();
+      for (int p = 0; p < COUNT; ++p)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const auto v = __builtin_amdgcn_permlane16_swap(o[t][p][r], o[NT + t][p][r], false, false);
+          op[0][t][p][r] = v[0];
+          op[1][t][p][r] = v[1];
+        }
   };
 
   f32x16_t tot[MS][NT];
@@ -216,27 +242,22 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
 #pragma unroll
       for (int r = 0; r < 16; ++r) tot[m][t][r] = 0.f;
   const int ln = lane & 31, kb = lane >> 5;
-  auto multiply = [&](auto pieces) __attribute__((always_inline)) {
+  auto multiply = [&](auto pieces, int place) __attribute__((always_inline)) {
     constexpr int COUNT = decltype(pieces)::value;  // of the weights
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      u32x4_t wv[NT][COUNT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int p = 0; p < COUNT; ++p) wv[t][p] = Ws[p * W_SZ + at(32 * t + ln, 2 * h + kb)];
 #pragma unroll
       for (int m = 0; m < MS; ++m) {
         u32x4_t xv[PX];
 #pragma unroll
-        for (int p = 0; p < PX; ++p) xv[p] = Xs[p * X_SZ + at(32 * m + ln, 2 * h + kb)];
+        for (int p = 0; p < PX; ++p) xv[p] = Xs[(p + place) * X_SZ + at(32 * m + ln, 2 * h + kb)];
 #pragma unroll
         for (int px = PX - 1; px >= 0; --px)
 #pragma unroll
           for (int pw = COUNT - 1; pw >= 0; --pw)
             if (px + pw < PW)
 #pragma unroll
-              for (int t = 0; t < NT; ++t) tot[m][t] = mfma<DT>(xv[px], wv[t][pw], tot[m][t]);
+              for (int t = 0; t < NT; ++t) tot[m][t] = mfma<DT>(xv[px], op[h][t][pw], tot[m][t]);
       }
     }
     wave_fence();
@@ -247,12 +268,18 @@ __global__ __launch_bounds__(64 * KW) void qmm_cols_kernel(ColsArgs a, int n_mti
   auto pass = [&](auto first, auto count) __attribute__((always_inline)) {
     Stage R;
     load(k0, R);
+    if constexpr (kCopied) copy_rows(k0, 0);
+    int place = 0;
     for (int ks = k0; ks < k1; ++ks) {
+      if constexpr (kCopied) wait_copies<0>();  // this step's, asked for ahead of the multiplies before it
       if constexpr (DT != 2) see_scale(R);
       put(R, first, count);
       load(ks + 1 < k1 ? ks + 1 : ks, R);
-      multiply(count);
+      if constexpr (kCopied) copy_rows(ks + 1 < k1 ? ks + 1 : ks, place ^ 1);
+      multiply(count, place);
+      if constexpr (kCopied) place ^= 1;
     }
+    if constexpr (kCopied) wait_copies<0>();
   };
   if (k0 < k1) {
     pass(std::integral_constant<int, 0>{}, std::integral_constant<int, PW>{});
@@ -391,21 +418,24 @@ bool qmm_cols_applies(const ColsArgs &a, int bits, int dt) {
   return bits != 2 && a.K % 8 == 0 && 128 * (int64_t)a.K * elem < most && 32 * (int64_t)a.N * bits / 8 < most && a.N % 32 == 0;
 }
 
-// Which tile: the smallest one of which the launch has at most one a CU; a CU's time is that of its unpacking and
-// multiplies, so a second tile on some CUs costs a whole further round.  Measured, 4-bit, groups of 64, bf16, N = 2048,
-// K = 4096, us of the call with 32 x 32 / 64 x 32 / 64 x 64 / 128 x 64 tiles at 64 / 130 / 300 / 1000 rows:
+// Which tile: the smallest one of which the fullest XCD gets at most one a CU; a CU's time is that of its unpacking and
+// multiplies, so a second tile on some CUs costs a whole further round (700 x 1408 x 2944: 242 tiles of 64 x 64, but 33 on some XCDs, 39.2 us, of 128 x 64
+// 24.3; 48 shapes at that line 1.14 to 1.45 times as fast as with 256 tiles counted).  Measured, 4-bit, groups of 64, bf16, N = 2048,
+// K = 4096, us of the call with 32 x 32 / 64 x 32 / 64 x 64 / 128 x 64 tiles at 64 / 130 / 300 / 1000 rows, before the weights went through no LDS:
 // 21.0, 26.2, 28.4, 37.0 / 32.2, 21.6, 29.4, 38.0 / 47.9, 40.8, 31.3, 39.8 / 136, 86.7, 65.9, 46.3 (f16 the same to 5 %).
 // f32 holds three times the rows in LDS and multiplies three times as much: at 64 / 130 / 300 / 1000 rows 27.8, 38.5,
-// 80.2, 118 / 54.2, 40.7, 88.0, 121 / 85.2, 78.0, 91.0, 121 / 249, 174, 196, 141, so 64 x 32 for two rounds, and 128 x 64
-// beyond (K shared by four waves there: what LDS holds).
+// 80.2, 118 / 54.2, 40.7, 88.0, 121 / 85.2, 78.0, 91.0, 121 / 249, 174, 196, 141, so 64 x 32 for two rounds of the chip (counted by XCD: 259 x 3200 x 4096
+// 113.6 for 104.8), and 128 x 64 beyond (K shared by four waves there: what LDS holds).
 template <int DT, int BITS>
 static hipError_t pick_cols(const ColsArgs &a, int group_log2, hipStream_t st) {
-  auto tiles = [&](int ms, int nt) { return (a.M + 32 * ms - 1) / (32 * ms) * ((a.N + 32 * nt - 1) / (32 * nt)); };
-  constexpr int kCus = 256;
-  if (tiles(1, 1) <= kCus) return start_cols<DT, BITS, 1, 1, 8>(a, group_log2, st);
-  if (tiles(2, 1) <= (DT == 2 ? 2 : 1) * kCus) return start_cols<DT, BITS, 2, 1, 8>(a, group_log2, st);
-  if constexpr (DT != 2)
-    if (tiles(2, 2) <= kCus) return start_cols<DT, BITS, 2, 2, 8>(a, group_log2, st);
+  auto fits = [&](int ms, int nt) { return tiles_of_an_xcd(a.M, a.N, 32 * ms, 32 * nt) <= 32; };
+  if (fits(1, 1)) return start_cols<DT, BITS, 1, 1, 8>(a, group_log2, st);
+  if constexpr (DT == 2) {
+    if ((a.M + 63) / 64 * ((a.N + 31) / 32) <= 512) return start_cols<DT, BITS, 2, 1, 8>(a, group_log2, st);
+  } else {
+    if (fits(2, 1)) return start_cols<DT, BITS, 2, 1, 8>(a, group_log2, st);
+    if (fits(2, 2)) return start_cols<DT, BITS, 2, 2, 8>(a, group_log2, st);
+  }
   return start_cols<DT, BITS, 4, 2, DT == 2 ? 4 : 8>(a, group_log2, st);
 }
 

@@ -50,6 +50,14 @@ def test_input_gradient(rows, n, k, bits, group, dtype):
     assert err <= 1.01 * perr + 2.0 ** -24, (err, perr)  # (both have the same rounding of the result; sums in another order)
 
 
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("bits", [4, 8])
+# the last rows of a tile whose launch gives an XCD 32 of them and the first of the next larger one's; K of no whole number of steps, and of one
+@pytest.mark.parametrize("rows,n,k", [(64, 2688, 72), (65, 2688, 72), (128, 2688, 296), (129, 2688, 296), (256, 2688, 520), (320, 2688, 32), (321, 2688, 520)])
+def test_tiles_around_a_round_of_an_xcd(rows, n, k, bits, dtype):
+    test_input_gradient(rows, n, k, bits, 64, dtype)
+
+
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
 @pytest.mark.parametrize("bits", [4, 8])
 def test_values_that_are_not_finite_or_leave_the_pieces(bits, dtype):
