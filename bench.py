@@ -34,7 +34,6 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16
 # inside this script: the figure is carried from the named file under profiles/, it is not measured by this run.
 CARRIED_TRAFFIC = {
     "decode": (1.975e8, "profiles/qmm_small_kernel_decode_batch32_hbm_traffic.txt"),
-    "prefill": (4.054e8, "profiles/qmm_large_kernel_prefill_tokens4096_counters.txt"),
     "mixtral_decode": (2.528e8, "profiles/qmm_small_kernel_decode_mixtral_batch1.txt"),
 }
 
@@ -263,7 +262,7 @@ def run_workload(name, args, torch, m, synth, dev):
                     "kernel_us": k_ms * 1e3,
                     "kernel_us_source": "start/end time stamps of the dispatch (hipExtLaunchKernelGGL events), mean over the timed steps, "
                                         "kernels launched one after the other on one stream (mi_moe_forward_timed); the timed step itself "
-                                        "(ms_per_step) runs mi_moe_forward's own schedule, tile classes side by side on two to four streams",
+                                        "(ms_per_step) runs mi_moe_forward's own schedule (8-bit codes: tile classes side by side on two to four streams)",
                     "serial_kernels_us_sum_vs_step_us": [round((sum(head["kern"]) + sum(head["stage_ms"][i] for i in (0, 1, 2, 5))) * 1e3, 1),
                                                          round(head["ms"] * 1e3, 1)],
                     "dense_gemm_yardstick": dense_gemm_yardstick(torch, int(round(k_rows)), 2 * cfg.intermediate, cfg.hidden, dev),

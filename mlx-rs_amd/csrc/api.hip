@@ -173,9 +173,9 @@ bool raw_all_tiles(const mi_moe_config &c, int64_t T) {
   const int64_t P = T * c.top_k, E = c.n_experts;
   return raw_tiled_batch(c, T) && (c.bits == 4 || P < 20 * E || P >= 40 * E);
 }
-// Groups of 64, 4-bit codes: batches whose segments all go through short tiles on raw codes, in one launch a product on the caller's
+// Groups of 64, 4-bit codes: batches whose segments all go through pieces on raw codes, in one launch a product on the caller's
 // stream (the others: streamed segments, and tiles of 256 weight rows on side streams).  From the batches on for which the tile lists
-// are built and the router has kernels of its own, up to 96 rows per expert on average.  Measured, us of a forward, other route / this one:
+// are built and the router has kernels of its own, up to 96 rows per expert on average.  Measured when pieces had 64 rows, us of a forward, other route / this one:
 //   128 experts, hidden 2048, even routing at 96 / 128 / 203 / 320 / 512 / 1024 / 2048 / 4096 tokens 145, 151, 176, 216, 218, 266, 360, 484 /
 //   128, 124, 128, 134, 168, 221, 350, 566; Zipf-1.1 136, 139, 160, 173, 193, 237, 344, 490 / 92, 95, 114, 134, 157, 219, 341, 560;
 //   hidden 4096, intermediate 1536, even at 128 / 256 / 512 / 1024 / 2048 tokens 536, 587, 665, 785, 1144 / 372, 375, 449, 649, 1101; Zipf-1.3
@@ -198,6 +198,10 @@ bool mid_batch(const mi_moe_config &c, int64_t T, bool tiled) {
 // 212 / 89, 113, 151, 183; at 256 rows, Zipf-1.1, 446 / 421 / 422.
 int piece_rows(int64_t pairs, int n_experts) { return pairs < (int64_t)48 * n_experts ? 64 : pairs < (int64_t)80 * n_experts ? 96 : kPieceM; }
 
+// Larger batches: the same pieces for the segments of nine rows and more, the others streamed ahead of them.  Us of a forward, tiles of 256 weight rows in three
+// classes on two streams / this: 128 experts, hidden 2048, 4096 tokens, Zipf-1.1 501 / 492; hidden 4096, 8192 tokens, Zipf-1.3 3052 / 2972; gate/up and down
+// kernels of 8192 tokens, even routing, 840 / 800.  Nearer to float64 as well (3.87e-3 / 2.87e-3), since the weights are not rounded.  Streaming them
+// beside the tiles on a side stream, or from two or four rows on through the tiles: the same times.
 bool piece_batch(const mi_moe_config &c, int64_t T, bool heavy) {
   const int64_t P = T * c.top_k;
   return heavy && c.bits == 4 && T > kFusedRouterMaxTokens && P >= 512 && c.n_experts >= 8 && codes_tiles_fit(c, T);
