@@ -34,6 +34,7 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16
 # inside this script: the figure is carried from the named file under profiles/, it is not measured by this run.
 CARRIED_TRAFFIC = {
     "decode": (1.975e8, "profiles/qmm_small_kernel_decode_batch32_hbm_traffic.txt"),
+    "prefill": (7.77e8, "profiles/qmm_pieces_kernel_prefill_tokens4096_hbm_traffic.txt"),
     "mixtral_decode": (2.528e8, "profiles/qmm_small_kernel_decode_mixtral_batch1.txt"),
 }
 
