@@ -302,7 +302,12 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
 // library's code object.  Every GPU that loads the library holds its own copy at its own address until
 // the process ends.  In host code the name is only a handle for hipGetSymbolAddress: the address a
 // kernel may use is looked up once per handle (mi_moe_create, on the handle's device) and kept there.
-static __device__ __align__(256) unsigned char scratch[MI_MOE_STATIC_SCRATCH_BYTES];
+// A batch is taken whose least workspace (ForwardWs::bytes_min) is MI_MOE_STATIC_SCRATCH_BYTES or less.  The same again lies behind it for what the tiles on raw
+// codes want beyond that (bytes_raw), so that such a batch takes the kernels that mi_moe_forward gives it.  That is never more: the copy of x has the size of the
+// normalised rows, its group sums at most that of the down product's rows, those of h at most h's (K is a multiple of 128 there, and 16 groups of sums, to whole
+// numbers of which they are padded, are no larger than 128 values), and a list of at least four rows a segment is smaller than two of the arrays of pairs.
+constexpr size_t kStaticScratch = (size_t)2 * MI_MOE_STATIC_SCRATCH_BYTES;
+static __device__ __align__(256) unsigned char scratch[kStaticScratch];
 
 // Prefill-sized batches: the tile classes and the streamed segments are independent chains (gate/up then
 // down over the same rows); three of the four run on side streams, forked from and joined back into the
@@ -853,14 +858,14 @@ int mi_moe_forward_static(mi_moe_handle h, const uint16_t *x, int64_t T, uint16_
   if (!h) return fail("forward_static: handle is NULL");
   if (T < 0) return fail("forward_static: negative token count");
   if (T * (int64_t)h->cfg.top_k > (int64_t)1 << 30) return fail("forward_static: too many (token, expert) pairs");
-  const size_t need = carve_forward(h->cfg, T, nullptr, false).bytes_min;
+  const ForwardWs f = carve_forward(h->cfg, T, nullptr, false);
+  const size_t need = f.bytes_min;
   if (need > (size_t)MI_MOE_STATIC_SCRATCH_BYTES)
     return fail("forward_static: %lld tokens of this layer need %zu bytes of workspace, the built-in scratch holds %zu "
                 "(use mi_moe_forward with a workspace of the caller's)",
                 (long long)T, need, (size_t)MI_MOE_STATIC_SCRATCH_BYTES);
   // no allocation from here on: the kernels get the address looked up by mi_moe_create
-  return forward_impl(h, x, T, out, h->scratch_dev, (size_t)MI_MOE_STATIC_SCRATCH_BYTES, dbg,
-                      static_cast<hipStream_t>(stream), nullptr);
+  return forward_impl(h, x, T, out, h->scratch_dev, f.bytes_raw < kStaticScratch ? f.bytes_raw : kStaticScratch, dbg, static_cast<hipStream_t>(stream), nullptr);
 } MI_CATCH("forward_static")
 
 int mi_moe_forward_residual(mi_moe_handle h, const uint16_t *x, const uint16_t *norm_weight, float eps,

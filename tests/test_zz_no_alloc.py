@@ -67,3 +67,19 @@ def test_static_scratch_refuses_what_does_not_fit(orc):
     assert torch.equal(got.view(torch.int16), blk.forward(x[:156].contiguous()).view(torch.int16))
     with pytest.raises(m.MoeError, match="negative"):
         m.capi.check(lib.mi_moe_forward_static(blk._handle, x.data_ptr(), -1, out.data_ptr(), None, st))
+
+
+# Layers whose tiles on raw codes want more than the least workspace: pieces (group sums beyond the normalised rows' place), groups of 32 and 128, and
+# a middle batch with more group sums of h than the normalised rows' place holds
+@pytest.mark.parametrize("H,E,k,I,bits,group,T", [(256, 8, 4, 512, 4, 64, 1100), (128, 8, 4, 1024, 4, 64, 840), (256, 64, 4, 1152, 4, 64, 640),
+                                                   (256, 8, 2, 512, 4, 32, 2000), (256, 8, 2, 512, 8, 128, 2000)])
+def test_static_scratch_takes_the_forward_s_own_kernels(H, E, k, I, bits, group, T):
+    """Batches whose least workspace fits 8 MiB and whose full one does not: the results are mi_moe_forward's bit for bit there as well."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    lib = m.load_library()
+    cfg = m.MoeConfig(H, E, k, I, bits, group, 0)
+    blk = synth.make_block(cfg, seed=7, device="cuda", zipf_s=0.5, gen_device="cuda")
+    assert blk.workspace_bytes(T) - 256 > m.capi.STATIC_SCRATCH_BYTES
+    x = synth.make_tokens(cfg, T, seed=7, device="cuda")
+    assert torch.equal(_static(lib, m, blk, x).view(torch.int16), blk.forward(x).view(torch.int16))
