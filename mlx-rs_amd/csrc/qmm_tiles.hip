@@ -240,11 +240,12 @@ __device__ __forceinline__ void output_rows(const CodesArgs &a, int64_t row0, in
     dst[h] = a.dst_rows ? a.dst_rows[r] : (uint32_t)r;
   }
 }
-// silu(g) u, fp32.  The quotient is as the division gives it: 1 + exp(-g) is a normal number from 1 on, so a reciprocal and one correction do (an
-// infinite g comes out as no number, and is looked at again with all that are not finite).
+// silu(g) u, fp32.  The quotient is as the division gives it.  1 + exp(-g) reaches 2^128, so the reciprocal is taken of a quarter of it (beyond 2^126 that of a
+// normal number is none, and v_rcp_f32 gives zero) and one correction follows; where the sum is infinite the quotient is zero, and no correction (an infinite g
+// comes out as no number, and is looked at again with all that are not finite).
 __device__ __forceinline__ float gated(float g, float u) {
-  const float d = 1.0f + __expf(fminf(-g, 88.0f)), r = __builtin_amdgcn_rcpf(d), q = g * r;
-  return __builtin_fmaf(__builtin_fmaf(-d, q, g), r, q) * u;
+  const float d = 1.0f + __expf(-g), r = __builtin_amdgcn_rcpf(0.25f * d) * 0.25f, q = g * r;
+  return (d < INFINITY ? __builtin_fmaf(__builtin_fmaf(-d, q, g), r, q) : q) * u;
 }
 // The results of a piece of up to 32 MS rows x 256 weight rows (of a block; four waves, 64 weight rows each) go out: N is a multiple of
 // 128, there is no bias of the layer's.  Two rows of a column become one register, neighbouring lanes swap halves, and the rows are turned round in LDS:

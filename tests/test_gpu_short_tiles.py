@@ -124,6 +124,34 @@ def test_short_tiles_with_a_gate_that_is_not_finite():
     assert not ref.isfinite().all() and torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
 
 
+# 540, 1000 and 400 pairs on 8 experts: pieces of up to 96 rows, of 128 beside streamed segments, and the list of groups of 32 and 128
+@pytest.mark.parametrize("group,tokens", [(64, 270), (64, 500), (32, 200), (128, 200)])
+def test_tiles_with_gates_far_below_zero(group, tokens):
+    """silu of gates around -88, where 1 + exp(-g) leaves the numbers whose reciprocal is normal, and far beyond, where it is infinite and the quotient zero.
+    Column 0 of x is the gate and column 64 (one) times 2^100 the up product, exactly (scales of zero, biases in those columns' groups), so h is large enough to
+    see; the down product is half the sum of a group of h, 128 equal values.  Three roundings to bfloat16 (h, y and the result), and the two routing weights
+    sum to one up to 2^-8."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(256, 8, 2, 256, 4, group, 0)
+    blk = synth.make_block(cfg, seed=6, device="cuda", zipf_s=0.7, gen_device="cuda")
+    gates = torch.tensor([-1e38, -1e30, -1000.0, -100.0, -89.0, -88.5, -88.0, -87.5, -87.0, -60.0, -3.0, -0.0, 0.25, 5.0, 88.0, 100.0]).bfloat16()
+    x = torch.zeros((tokens, 256), dtype=torch.bfloat16, device="cuda")
+    x[:, 0] = gates.repeat(tokens // 16 + 1)[:tokens].cuda()
+    x[:, 128] = 1.0
+    x[:, 129:] = torch.randn((tokens, 127), generator=torch.Generator().manual_seed(2)).bfloat16().cuda() * (torch.arange(129, 256, device="cuda") >= 128 + group)
+    blk.gate_weight[:, 0] = 0.0  # (the routing is that of the rest)
+    for bank, column, value in ((blk.gate_proj, 0, 1.0), (blk.up_proj, 128, 2.0 ** 100), (blk.down_proj, 0, 0.5 / group)):
+        bank.scales.zero_()
+        bank.biases.zero_()
+        bank.biases[:, :, column // group] = value
+    out, routing = blk.forward(x, debug=True)
+    g = x[:, 0].float()
+    ref = (g / (1.0 + torch.exp(-g))).double() * 2.0 ** 99 * routing["topk_w"].double().sum(1)
+    assert bool(out.isfinite().all())
+    assert bool(((out.double() - ref[:, None]).abs() <= 2.0 ** -7 * ref.abs()[:, None]).all())
+
+
 @pytest.mark.parametrize("dtype,group", [("float16", 32), ("float16", 64), ("float16", 128), ("bfloat16", 32), ("bfloat16", 64), ("bfloat16", 128)])
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("rows,n,k", [(200, 4096, 1152), (260, 4090, 640), (1000, 4096, 1408), (1000, 4090, 2176)])
