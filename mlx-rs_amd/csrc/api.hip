@@ -619,7 +619,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   cd.y = f.y;
   cd.N = c.hidden; cd.K = c.intermediate;
   auto prepare_x = [&](hipStream_t s) -> hipError_t {
-    return launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, false, s);
+    return launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, s);
   };
   auto tiles_up = [&](hipStream_t s) -> hipError_t {
     if (raw_codes) return launch_qmm_pieces(ca, f.raw_tiles, f.raw_cap, true, s);
@@ -1245,7 +1245,7 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
     const size_t copy_bytes = codes_copy_bytes(bits, M, K);
     uint16_t *copy = copy_bytes ? reinterpret_cast<uint16_t *>(cv.take<char>(copy_bytes)) : nullptr;
     uint16_t *sums = reinterpret_cast<uint16_t *>(cv.take<char>(codes_sums_bytes(M, K, group_size)));
-    MI_HIP(launch_prepare_rows(x, M, K, group_size, dtype, copy, sums, false, st));
+    MI_HIP(launch_prepare_rows(x, M, K, group_size, dtype, copy, sums, st));
     CodesArgs a{};
     a.x = copy ? copy : x;
     a.x_rows = M;

@@ -332,8 +332,8 @@ struct PrepareArgs {
   int64_t octets = 0;  // 8-blocks of x in all, and of a row; 0: nothing to prepare
   int octets_per_row = 0, lanes_log2 = 0;  // (of a group)
   uint16_t *copy = nullptr, *sums = nullptr;
-  int sums_row = 0, slots = 0;
-  RowOrder order = RowOrder::kPlain;
+  int sums_row = 0;
+  bool plain = false;  // for the products on codes without a centre (launch_qmm_pieces)
 };
 bool router_fused_applies(int64_t T, int E, int k);
 hipError_t launch_router_fused(const uint16_t *x, const uint16_t *wg, const float *bias,
@@ -423,7 +423,7 @@ size_t codes_copy_bytes(int bits, int64_t rows, int K);
 size_t codes_sums_bytes(int64_t rows, int K, int group, bool plain = false);
 PrepareArgs prepare_args(const void *x, int64_t rows, int K, int group, uint16_t *copy, uint16_t *sums, bool plain);
 hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
-                               uint16_t *sums, bool plain, hipStream_t st);
+                               uint16_t *sums, hipStream_t st);
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
 hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st);
 // 4-bit codes in groups of 64, a list of pieces of kPieceM rows

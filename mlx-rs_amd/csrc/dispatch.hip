@@ -17,7 +17,9 @@ namespace mi_moe {
 __device__ __forceinline__ bool prepares(const PrepareArgs &a, int first) {
   if ((int)blockIdx.x < first) return false;
   const int64_t i = (int64_t)((int)blockIdx.x - first) * kDispThreads + threadIdx.x;
-  if (i < a.octets) prepare_octet<0>(a, i);  // (whole groups leave together)
+  if (i >= a.octets) return true;  // (whole groups leave together)
+  if (a.plain) prepare_octet<0, true>(a, i);
+  else prepare_octet<0, false>(a, i);
   return true;
 }
 static unsigned prepare_blocks(const PrepareArgs &a) { return (unsigned)((a.octets + kDispThreads - 1) / kDispThreads); }

@@ -32,9 +32,13 @@ __device__ __forceinline__ void put_sums(uint16_t *to, int slots, float sum) {
 constexpr RowOrder row_order(int bits) { return bits == 4 ? RowOrder::kPaired : RowOrder::kPlain; }
 constexpr int padded_groups(int G) { return (G + 15) / 16 * 16; }  // whole windows of the bias product; the groups past the row's end are zeros
 
-// One thread's part of preparing rows: eight values of x (octet i of all rows).  Whole groups go through lanes of one wave.
-template <int DT>
+// One thread's part of preparing rows: eight values of x (octet i of all rows).  Whole groups go through lanes of one wave.  PLAIN: PrepareArgs::plain.
+// What bounds it is latency: as a launch of its own 4.6 us for 61 rows of 2176 and 5.2 for 611 of 1152 (bf16, with a profiler's overhead).  One lane writes all the
+// zeros behind a row's sums, so it writes 16 bytes at a time: with 8, and the two forms told apart at run time, products whose groups fill no multiple of sixteen
+// took 0.2 to 0.7 us more (61 x 2320 x 2176 4-bit 14.6 us for 14.0, 611 x 2864 x 1152 18.6 for 17.9, 494 x 960 x 2432 8-bit 17.3 for 16.6).
+template <int DT, bool PLAIN>
 __device__ __forceinline__ void prepare_octet(const PrepareArgs &a, int64_t i) {
+  constexpr int SLOTS = sum_slots(PLAIN);
   float v[8];
   const uint4 w = reinterpret_cast<const uint4 *>(a.x)[i];
   const uint32_t u[4] = {w.x, w.y, w.z, w.w};
@@ -50,8 +54,7 @@ __device__ __forceinline__ void prepare_octet(const PrepareArgs &a, int64_t i) {
     }
   }
   if (a.copy) {
-    const bool quads = a.order == RowOrder::kQuads;
-    const uint32_t y = quads ? w.z : w.y, z = quads ? w.y : w.z;  // the words that meet: 0 and 2, 1 and 3, or neighbours
+    const uint32_t y = PLAIN ? w.z : w.y, z = PLAIN ? w.y : w.z;  // the words that meet: neighbours (kQuads), or 0 and 2, 1 and 3 (kPaired)
     uint4 p;
     p.x = (w.x & 0xffffu) | (z << 16);
     p.y = (w.x >> 16) | (z & 0xffff0000u);
@@ -67,10 +70,10 @@ __device__ __forceinline__ void prepare_octet(const PrepareArgs &a, int64_t i) {
   if ((i & ((1 << a.lanes_log2) - 1)) == 0) {
     const int64_t row = i / a.octets_per_row;
     const int g = (int)(i % a.octets_per_row) >> a.lanes_log2, G = a.octets_per_row >> a.lanes_log2;
-    uint16_t *const to = a.sums + row * a.sums_row + g * a.slots;
-    put_sums(to, a.slots, sum);
-    if (g == G - 1)
-      for (int k = a.slots; g * a.slots + k < a.sums_row; k += 4) *reinterpret_cast<uint2 *>(to + k) = make_uint2(0, 0);
+    uint16_t *const to = a.sums + row * a.sums_row;
+    put_sums(to + g * SLOTS, SLOTS, sum);
+    if (g == G - 1)  // (an even number of groups where a group has four slots)
+      for (int k = G * SLOTS; k < a.sums_row; k += 8) *reinterpret_cast<uint4 *>(to + k) = make_uint4(0, 0, 0, 0);
   }
 }
 

@@ -33,7 +33,7 @@ namespace mi_moe {
 template <int DT>
 __global__ __launch_bounds__(256) void prepare_rows_kernel(PrepareArgs a) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < a.octets) prepare_octet<DT>(a, i);  // (whole groups leave together)
+  if (i < a.octets) prepare_octet<DT, false>(a, i);  // (whole groups leave together)
 }
 
 // What a launch of the kernel below is made of, for its two sides.
@@ -407,11 +407,11 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
     wr[t] = words_of((t ? a.w1 : a.w0) + ebase * (row_bytes / 4), (uint32_t)N * row_bytes);
     sr[t] = words_of(s_of[t], (uint32_t)N * G * sizeof(T)), br[t] = words_of(b_of[t], (uint32_t)N * G * sizeof(T));  // (read in words: the host takes an even number of them)
   }
-  // weight row of place `at` (0 .. 31) of the wave's tile t.  Columns past the end repeat the last one (never stored).  Order of the output
+  // weight row of place `at` (0 .. 31) of the wave's tile t.  Columns past the end repeat the last one (never stored).  Order of h
   // (CodesArgs::y_order): the place p of an 8-block takes the row whose result belongs there.
   const int col0 = n0 + 32 * (GLU ? 1 : NT) * wave;
   auto weight_row = [&](int t, int at) __attribute__((always_inline)) {
-    const int p = (at & ~7) | value_at_place(a.y_order, at & 7), row = col0 + (GLU ? 0 : 32 * t) + p;
+    const int p = GLU ? (at & ~7) | value_at_place(a.y_order, at & 7) : at, row = col0 + (GLU ? 0 : 32 * t) + p;
     return row < N ? row : N - 1;
   };
   // ---- what a lane copies, and where it lies in LDS.  LDS gives 256 bytes a cycle, sixteen lanes' pieces, if they lie in different
@@ -774,7 +774,7 @@ __device__ __forceinline__ void multiply_long_tile(const CodesArgs &a, int e, in
   }
   const int col0 = n0 + (GLU ? 32 : 64) * wave;
   auto weight_row = [&](int t, int at) __attribute__((always_inline)) {
-    const int p = (at & ~7) | value_at_place(a.y_order, at & 7), row = col0 + (GLU ? 0 : 32 * t) + p;
+    const int p = GLU ? (at & ~7) | value_at_place(a.y_order, at & 7) : at, row = col0 + (GLU ? 0 : 32 * t) + p;
     return row < N ? row : N - 1;
   };
   auto turned = [](int row) __attribute__((always_inline)) { return (row >> 1) & 7; };
@@ -1024,14 +1024,13 @@ PrepareArgs prepare_args(const void *x, int64_t rows, int K, int group, uint16_t
   a.lanes_log2 = group == 32 ? 2 : (group == 64 ? 3 : 4);
   a.copy = copy;
   a.sums = sums;
-  a.slots = sum_slots(plain);
-  a.sums_row = padded_groups(K / group) * a.slots;
-  a.order = plain ? RowOrder::kQuads : RowOrder::kPaired;
+  a.sums_row = padded_groups(K / group) * sum_slots(plain);
+  a.plain = plain;
   return a;
 }
 hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
-                               uint16_t *sums, bool plain, hipStream_t st) {
-  const PrepareArgs a = prepare_args(x, rows, K, group, copy, sums, plain);
+                               uint16_t *sums, hipStream_t st) {
+  const PrepareArgs a = prepare_args(x, rows, K, group, copy, sums, false);
   if (a.octets == 0) return hipSuccess;
   const unsigned grid = (unsigned)((a.octets + 255) / 256);
   if (dt == 0) prepare_rows_kernel<0><<<grid, 256, 0, st>>>(a);
