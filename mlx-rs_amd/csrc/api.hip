@@ -158,7 +158,8 @@ bool raw_tiled_batch(const mi_moe_config &c, int64_t T) {
 // Batches of those sizes whose segments all go through the tiles, in one launch a product on the caller's stream.  The others (8-bit codes, twenty to forty
 // rows an expert) keep the short segments on the kernel of a few rows, beside the tiles on a side stream: with skewed routing that is 1 to 12 % faster
 // there, with even routing 7 to 15 % slower.  Measured, us of a forward, side by side / all in tiles, at an average of 5, 8, 12, 16, 24, 32, 48, 96 rows
-// (experts, k, hidden, intermediate, bits, group; below sixteen rows with 4-bit codes in groups of 32 the other tiles had their codes in registers):
+// (experts, k, hidden, intermediate, bits, group; below sixteen rows with 4-bit codes in groups of 32 the other tiles had their codes in registers; all in tiles
+// before their list had the longest pieces first):
 //   128, 8, 2048, 768, 4, 32   even 155, 169, 182, 183, 198, 211, 247, 357 / 151, 151, 153, 155, 166, 186, 226, 335; Zipf-1.1 126, 131, 135, 164, 166, 184, 238,
 //                              359 / 108, 113, 126, 144, 168, 185, 217, 336; 1.3 121, 129, 131, 160, 158, 177, 225, 346 / 91, 110, 116, 125, 156, 174, 210, 309
 //   128, 8, 2048, 768, 4, 128  even 139, 150, 157, 168, 158, 171, 199, 280 / 118, 119, 123, 124, 133, 144, 169, 256; Zipf-1.1 118, 122, 128, 138, 138, 153, 194,
@@ -169,6 +170,9 @@ bool raw_tiled_batch(const mi_moe_config &c, int64_t T) {
 //                              403 / 207, 207, 208, 258, 270, 331, 367, 385
 //   128, 8, 2048, 768, 8, 32   Zipf-1.1 144, 167, 171, 181, 196, 224, 280, 406 / 123, 125, 146, 184, 207, 229, 271, 396; 1.3 133, 144, 160, 176, 178, 208, 272, 387 /
 //                              108, 121, 129, 147, 198, 213, 255, 360
+// With it the skewed batches of 4-bit codes in groups of 32 that had become slower are not: 128 experts, Zipf-1.1 at 160 / 256 / 400 tokens 178, 191, 201 / 175, 185,
+// 199; left are 64 experts at 128 tokens (12 rows), 169 / 171, and 128 at 512 (32 rows), 215 / 221, where even routing has 182 / 141 and 212 / 173: the host does
+// not see which it is.
 bool raw_all_tiles(const mi_moe_config &c, int64_t T) {
   const int64_t P = T * c.top_k, E = c.n_experts;
   return raw_tiled_batch(c, T) && (c.bits == 4 || P < 20 * E || P >= 40 * E);

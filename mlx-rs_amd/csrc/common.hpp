@@ -177,7 +177,7 @@ __host__ __device__ inline P *tile_list(P *base, int cls, int cap256, int n_expe
 }
 
 // A list of the same form for the tiles of the products on raw codes: segments of `from` rows and more that the three lists do
-// not take, in pieces of `piece` rows; experts in ascending order.
+// not take, in pieces of `piece` rows (64, 96 or 128), the longest first (list_pieces).
 constexpr int kShortTileM = 64, kPieceM = 128;
 struct ShortTiles {
   uint32_t *list = nullptr;

@@ -112,6 +112,66 @@ __device__ __forceinline__ TileSplit split_segment(uint32_t c) {
   return t;
 }
 
+// The list of ShortTiles, by one wave: first[E] are the segments' first sorted rows.  Full pieces come first, in the order of the experts, then the remainders, those
+// of more 32s of rows before those of fewer (a block's time goes by these): launches of these tiles are one to three rounds of the chip, and a long block that starts
+// last is what they wait for.  Us of a forward, everything in the experts' order / this (128 experts, hidden 2048): groups of 64, even routing at 203 / 700 / 1100 / 1500 /
+// 3000 / 4096 tokens 118, 159, 189, 221, 386, 474 / 117, 153, 182, 209, 363, 464, Zipf-1.1 137, 183, 225, 265, 411, 491 / 133, 178, 210, 239, 394, 472; groups of 32,
+// Zipf-1.1 at 96 / 160 / 256 / 400 / 512 tokens 154, 181, 189, 204, 219 / 147, 175, 185, 200, 221, even at 512 185 / 174; with 8-bit codes, 256 tokens, 245 / 236.
+__device__ __forceinline__ void list_pieces(const uint32_t *first, uint32_t total, int E, uint32_t big_thr, const ShortTiles &shorts) {
+  constexpr int kClasses = kPieceM / 32;
+  const int lane = lane_id();
+  struct Segment {
+    uint32_t row, full, rest;  // first row, full pieces, rows behind them
+    uint64_t of[kClasses];     // lanes whose remainder is of each number of 32s
+  };
+  auto segment = [&](int e0) __attribute__((always_inline)) {
+    Segment s{};
+    const int e = e0 + lane;
+    uint32_t rows = 0;
+    if (e < E) {
+      s.row = first[e];
+      rows = (e + 1 < E ? first[e + 1] : total) - s.row;
+    }
+    if (rows < shorts.from || (big_thr != 0u && rows >= big_thr)) rows = 0;
+    s.full = rows / shorts.piece;
+    s.rest = rows - s.full * shorts.piece;
+    for (int c = 0; c < kClasses; ++c) s.of[c] = __ballot(s.rest != 0u && (s.rest - 1u) / 32u == (uint32_t)c);
+    return s;
+  };
+  auto sum_up_to = [&](uint32_t v) __attribute__((always_inline)) {
+    for (int d = 1; d < kWave; d <<= 1) {
+      const uint32_t up = __shfl_up(v, d, kWave);
+      if (lane >= d) v += up;
+    }
+    return v;
+  };
+  uint32_t full = 0, next[kClasses] = {};  // where the next full piece and the next remainder of each class go
+  for (int e0 = 0; e0 < E; e0 += kWave) {
+    const Segment s = segment(e0);
+    full += s.full;
+    for (int c = 0; c < kClasses; ++c) next[c] += __popcll(s.of[c]);
+  }
+  uint32_t end = __shfl(sum_up_to(full), kWave - 1, kWave);
+  for (int c = kClasses - 1; c >= 0; --c) {
+    const uint32_t n = next[c];
+    next[c] = end;
+    end += n;
+  }
+  if (lane == 0) shorts.list[0] = end;
+  uint4 *const list = reinterpret_cast<uint4 *>(shorts.list) + 1;
+  full = 0;
+  for (int e0 = 0; e0 < E; e0 += kWave) {
+    const Segment s = segment(e0);
+    const uint32_t e = (uint32_t)(e0 + lane), upto = sum_up_to(s.full);
+    for (uint32_t i = 0; i < s.full; ++i) list[full + upto - s.full + i] = make_uint4(e, s.row + i * shorts.piece, shorts.piece, 0u);
+    full += __shfl(upto, kWave - 1, kWave);
+    for (int c = 0; c < kClasses; ++c) {
+      if (s.of[c] >> lane & 1u) list[next[c] + __popcll(s.of[c] & lanemask_lt())] = make_uint4(e, s.row + s.full * shorts.piece, s.rest, 0u);
+      next[c] += __popcll(s.of[c]);
+    }
+  }
+}
+
 // counts -> offsets, work records, M tiles and short tiles; runs in one block.  LDS cnt[E] in, cur[E] out.
 __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint32_t *cur, int E,
                               uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets,
@@ -128,11 +188,12 @@ __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint
   }
   if (tid == 0 && offsets) offsets[E] = total;
   __syncthreads();
-  // experts with rows, in ascending order, by wave 0
+  // experts with rows, in ascending order, by wave 0, and the tiles on raw codes by wave 1
+  if (tid >= kWave && tid < 2 * kWave && shorts.list) list_pieces(cnt, total, E, mtiles ? big_thr : 0u, shorts);
   if (tid < kWave) {
     uint32_t *const l256 = mtiles, *const l128 = mtiles ? tile_list(mtiles, 1, cap256, E) : nullptr,
                    *const l64 = mtiles ? tile_list(mtiles, 2, cap256, E) : nullptr;
-    uint32_t base = 0, t256 = 0, t128 = 0, t64 = 0, t_short = 0;
+    uint32_t base = 0, t256 = 0, t128 = 0, t64 = 0;
     for (int e0 = 0; e0 < E; e0 += kWave) {
       const int e = e0 + tid;
       uint32_t c = 0;
@@ -166,20 +227,6 @@ __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint
         rec[3] = 0u;
       }
       t256 += __shfl(incl, kWave - 1, kWave);
-      if (shorts.list) {  // pieces of shorts.piece rows
-        const uint32_t n = brief ? (c + shorts.piece - 1) / shorts.piece : 0u;
-        uint32_t before = n;
-        for (int d = 1; d < kWave; d <<= 1) {
-          const uint32_t v = __shfl_up(before, d, kWave);
-          if (tid >= d) before += v;
-        }
-        for (uint32_t i = 0; i < n; ++i) {
-          const uint32_t left = c - i * shorts.piece;
-          reinterpret_cast<uint4 *>(shorts.list)[1 + t_short + before - n + i] =
-              make_uint4((uint32_t)e, cnt[e] + i * shorts.piece, left < shorts.piece ? left : shorts.piece, 0u);
-        }
-        t_short += __shfl(before, kWave - 1, kWave);
-      }
       const bool r128 = big && ts.r != 0u && ts.rcls == 1, r64 = big && ts.r != 0u && ts.rcls == 2;
       const uint64_t b128 = __ballot(r128), b64 = __ballot(r64);
       if (r128 || r64) {
@@ -205,7 +252,6 @@ __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint
         l128[0] = t128;
         l64[0] = t64;
       }
-      if (shorts.list) shorts.list[0] = t_short;
     }
   }
   __syncthreads();

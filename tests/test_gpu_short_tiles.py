@@ -124,6 +124,31 @@ def test_short_tiles_with_a_gate_that_is_not_finite():
     assert not ref.isfinite().all() and torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
 
 
+# (pieces of 64, 96 and 128 rows, the last beside streamed segments; the list of groups of 32; more experts than waves have lanes, and not a multiple of those)
+@pytest.mark.parametrize("experts,group,lengths,piece", [(70, 64, [0, 1, 31, 32, 33, 63, 64, 65], 64), (130, 64, [64, 96, 97, 32, 95, 0, 128, 33], 96),
+                                                         (9, 64, [127, 128, 129, 9, 8, 255, 96, 97, 32], 128), (200, 32, [0, 64, 1, 63, 65, 32, 129, 33], 64)])
+def test_segments_of_chosen_lengths(experts, group, lengths, piece):
+    """Lengths on both sides of every one at which the list of pieces starts another, in the order of the experts: a piece that is left out, listed twice or
+    listed for another expert leaves rows that are far off.  Every token has its expert's column large, and the router is the unit matrix.  The bound of a row
+    is one and a half times test_blocks_in_short_tiles' of the whole."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(256, experts, 1, 128, 4, group, 0)
+    blk = synth.make_block(cfg, seed=4, device="cuda", gen_device="cuda")
+    blk.gate_weight.copy_(torch.eye(256)[:experts])
+    of = torch.cat([torch.full((lengths[e % len(lengths)],), e) for e in range(experts)]).cuda()
+    tokens = of.numel()
+    assert piece == (64 if group != 64 or tokens < 48 * experts else 96 if tokens < 80 * experts else 128)
+    of = of[torch.randperm(tokens, generator=torch.Generator().manual_seed(1)).cuda()]
+    x = synth.make_tokens(cfg, tokens, seed=4, device="cuda")
+    x[torch.arange(tokens, device="cuda"), of] = 16.0
+    out, routing = blk.forward(x, debug=True)
+    assert torch.equal(routing["topk_idx"][:, 0].long(), of)
+    ref = block_truth(blk, x, routing)
+    err = (out.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= 1.5 * 2.0 ** -8, float(err.max())
+
+
 # 540, 1000 and 400 pairs on 8 experts: pieces of up to 96 rows, of 128 beside streamed segments, and the list of groups of 32 and 128
 @pytest.mark.parametrize("group,tokens", [(64, 270), (64, 500), (32, 200), (128, 200)])
 def test_tiles_with_gates_far_below_zero(group, tokens):
