@@ -260,7 +260,6 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
   unsigned char *const mine = GLU ? lds_raw + wave * 64 : lds_raw + wave * (32 * ROWB);
   auto value = [&](int m, int t, int r) __attribute__((always_inline)) { return GLU ? gated(tot[m][0][r], tot[m][1][r]) : tot[m][t][r]; };
   float odd = 0.f;  // no number once a result was not finite
-  uint64_t again[GLU ? 1 : 2] = {};
   auto turn = [&](int m, int at) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < (GLU ? 1 : 2); ++t)
@@ -276,6 +275,7 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
   };
   // sums that are not finite, again on the dequantised weights (see plain_rows)
   auto repair = [&](int m_first, int m_end, int at) __attribute__((always_inline)) {
+    uint64_t again = 0, again_1 = 0;  // (which of a column's rows, of the wave's first and second 32 columns: not an array, which would lie in scratch memory)
 #pragma unroll
     for (int m = 0; m < MS; ++m)
 #pragma unroll
@@ -283,12 +283,12 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
         uint32_t bits = 0;
 #pragma unroll
         for (int r = 0; r < 16; ++r) bits |= (not_finite(tot[m][t][r]) || (GLU && not_finite(tot[m][1][r])) ? 1u : 0u) << r;
-        again[GLU ? 0 : t] |= (uint64_t)bits << (16 * m);
+        (t ? again_1 : again) |= (uint64_t)bits << (16 * m);
       }
 #pragma unroll 1
     for (int i = m_first * 4 * (GLU ? 1 : 2); i < m_end * 4 * (GLU ? 1 : 2); ++i) {  // four rows of a column at a time
       const int t = GLU ? 0 : i & 1, quad = GLU ? i : i >> 1;  // rows 8 quad + 4 kb + 0 .. 3
-      uint32_t open = (uint32_t)((t ? again[GLU ? 0 : 1] : again[0]) >> (4 * quad)) & 15u;
+      uint32_t open = (uint32_t)((t ? again_1 : again) >> (4 * quad)) & 15u;
       const uint16_t *xs[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
