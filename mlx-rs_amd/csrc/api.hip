@@ -273,7 +273,7 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
   }
   if (f.pieces) {
     f.raw_from = f.tmr;
-    f.raw_piece = piece_rows(P, c.n_experts);
+    f.raw_piece = kPieceM;  // (more rows an expert than the middle range has: piece_rows' last)
     f.raw_cap = short_list_cap(P, c.n_experts, f.raw_from, f.raw_piece);
     // (as above; nothing reads the 256-column tiles' lists, and where there is no norm the place of its rows is free)
     const size_t list = short_list_words(f.raw_cap), xsums = codes_sums_bytes(T, c.hidden, c.group_size, true), hsums = codes_sums_bytes(P, c.intermediate, c.group_size, true);

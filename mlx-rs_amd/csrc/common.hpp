@@ -314,9 +314,6 @@ hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, ui
                            uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
                            uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, int big_thr,
                            ShortTiles shorts, const PrepareArgs &prepare, void *scratch, hipStream_t st);
-// decode-sized batches: logits + selection + dispatch in one launch.  counters: 1 +
-// kFusedRouterMaxTokens zero-initialised words that the kernel leaves zeroed again.  norm_w != nullptr:
-// the rows are RMS-normalised first (weight norm_w, eps) and kept in xnorm.
 // The order of the values of every 8-block of a row of activations: as they are; (0,4)(1,5)(2,6)(3,7), which one and-or a register unpacks 4-bit codes to;
 // (0,2)(1,3)(4,6)(5,7), which is how a conversion of two bytes a register leaves them.
 enum class RowOrder { kPlain, kPaired, kQuads };
@@ -335,6 +332,9 @@ struct PrepareArgs {
   int sums_row = 0;
   bool plain = false;  // for the products on codes without a centre (launch_qmm_pieces)
 };
+// decode-sized batches: logits + selection + dispatch in one launch.  counters: 1 +
+// kFusedRouterMaxTokens zero-initialised words that the kernel leaves zeroed again.  norm_w != nullptr:
+// the rows are RMS-normalised first (weight norm_w, eps) and kept in xnorm.
 bool router_fused_applies(int64_t T, int E, int k);
 hipError_t launch_router_fused(const uint16_t *x, const uint16_t *wg, const float *bias,
                                const uint16_t *norm_w, float eps, uint16_t *xnorm, int64_t T,
@@ -426,7 +426,7 @@ hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, in
                                uint16_t *sums, hipStream_t st);
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
 hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st);
-// 4-bit codes in groups of 64, a list of pieces of kPieceM rows
+// 4-bit codes in groups of 64, a list of pieces of 64, 96 or 128 rows (ShortTiles::piece)
 hipError_t launch_qmm_pieces(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
 hipError_t launch_quantize(const float *w, int64_t rows, int64_t cols, int group, int bits,
                            uint32_t *q, void *s, void *b, int dt, hipStream_t st);

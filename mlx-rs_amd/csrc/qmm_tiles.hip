@@ -196,7 +196,7 @@ __device__ __forceinline__ void write_tile(const CodesArgs &a, const float (&tot
           open &= ~(1u << i);
           tr = rows - 1;
         }
-        xs[i] = static_cast<const T *>(a.x) + (int64_t)(a.src_rows ? a.src_rows[row0 + tr] : (uint32_t)(row0 + tr)) * K;
+        xs[i] = static_cast<const T *>(a.x) + (row0 + tr) * K;
       }
       if (!open) continue;
       float v[4];
@@ -216,8 +216,7 @@ __device__ __forceinline__ void write_tile(const CodesArgs &a, const float (&tot
       const int row = RPI * i + my_row;
       const int tr = 32 * m + row;
       if (tr < rows && my_col < N) {
-        const int64_t dst = a.dst_rows ? (int64_t)a.dst_rows[row0 + tr] : row0 + tr;
-        T *const to = static_cast<T *>(a.y) + dst * N + my_col;
+        T *const to = static_cast<T *>(a.y) + (row0 + tr) * N + my_col;
         const T *const from = reinterpret_cast<const T *>(mine + row * ROWB) + PV * my_piece;
         if (vec) {
           *reinterpret_cast<u32x4_t *>(to) = *reinterpret_cast<const u32x4_t *>(from);
@@ -949,15 +948,13 @@ __device__ __forceinline__ void multiply_long_tile(const CodesArgs &a, int e, in
 }
 
 // The tiles of a list of pieces of up to 128 rows (ShortTiles::piece), 4-bit codes in groups of 64: by their rows, 32 at a time.
-// Ids are dealt round-robin over the 8 XCDs: `run` tiles that follow each other in the list, often one expert's, share an XCD, and
-// their blocks of one stretch of weight rows stand side by side, so that its L2 serves the weights to all but the first.
-constexpr int kPieceTiles = 1;
+// Ids are dealt round-robin over the 8 XCDs, whole pieces to each (the blocks of one share its gathered rows).  Two or four pieces that follow each other in the
+// list on one XCD: fewer bytes (an expert's weights are read once by every XCD that has a piece of it), 0 to 2 % slower.
 template <bool GLU>
 __global__ __launch_bounds__(256, 2) void qmm_pieces_kernel(CodesArgs a, const uint32_t *__restrict__ list, int n_ntiles) {
   constexpr int NI = GLU ? 128 : 256;
-  const uint32_t xcd = blockIdx.x & 7, j = blockIdx.x >> 3, per_run = (uint32_t)n_ntiles * kPieceTiles;
-  const uint32_t id = (j / per_run * 8u + xcd) * kPieceTiles + j % kPieceTiles;
-  const int nt = (int)(j % per_run / kPieceTiles);
+  const uint32_t xcd = blockIdx.x & 7, j = blockIdx.x >> 3, id = j / (uint32_t)n_ntiles * 8u + xcd;
+  const int nt = (int)(j % (uint32_t)n_ntiles);
   if (id >= list[0]) return;
   const uint4 rec = reinterpret_cast<const uint4 *>(list)[1 + id];
   const int e = __builtin_amdgcn_readfirstlane((int)rec.x), rows = __builtin_amdgcn_readfirstlane((int)rec.z);
@@ -971,7 +968,7 @@ __global__ __launch_bounds__(256, 2) void qmm_pieces_kernel(CodesArgs a, const u
   multiply_tile<0, 4, false, true, GLU, true, 1, 2, 4, 1, S1>(a, e, row0, rows, nt * NI, 0, lds_raw);
 }
 
-// A block computes 32 MS token rows x 32 WN weight rows with WN KW waves (see codes_tile), tiles of up to 32 rows with half the
+// A block computes 32 MS token rows x 32 WN weight rows with WN KW waves (see multiply_tile), tiles of up to 32 rows with half the
 // token operand.
 template <int DT, int BITS, bool G32, bool LIST, bool GLU, int MS, int NT, int WN, int KW, int S>
 __global__ __launch_bounds__(64 * WN * KW, waves_of(WN * KW, lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES))) void qmm_tiles_kernel(
@@ -1095,7 +1092,7 @@ static hipError_t start_pieces(const CodesArgs &a, const uint32_t *list, int cap
   constexpr int NI = GLU ? 128 : 256, lds = kHalfLds;
   static_assert(LongRing::bytes(4) <= lds && Ring<4, 2, 2, 4, 2>::BYTES <= lds, "two blocks share a CU");
   const int n_ntiles = (a.N + NI - 1) / NI;
-  const int64_t grid = ((int64_t)cap + 8 * kPieceTiles - 1) / (8 * kPieceTiles) * (8 * kPieceTiles) * n_ntiles;
+  const int64_t grid = ((int64_t)cap + 7) / 8 * 8 * n_ntiles;
   if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
   static std::atomic<uint64_t> allowed{0};
   if (hipError_t e = allow_lds(reinterpret_cast<const void *>(&qmm_pieces_kernel<GLU>), lds, allowed); e != hipSuccess) return e;
