@@ -34,7 +34,7 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16
 # inside this script: the figure is carried from the named file under profiles/, it is not measured by this run.
 CARRIED_TRAFFIC = {
     "decode": (1.975e8, "profiles/qmm_small_kernel_decode_batch32_hbm_traffic.txt"),
-    "prefill": (7.77e8, "profiles/qmm_pieces_kernel_prefill_tokens4096_hbm_traffic.txt"),
+    "prefill": (7.38e8, "profiles/qmm_pieces_kernel_prefill_tokens4096_hbm_traffic.txt"),
     "mixtral_decode": (2.528e8, "profiles/qmm_small_kernel_decode_mixtral_batch1.txt"),
 }
 
@@ -63,7 +63,7 @@ def parse():
     ap.add_argument("--no-graph", action="store_true", help="launch eagerly instead of replaying a HIP graph")
     ap.add_argument("--serial-kernels", action="store_true",
                     help="every step through mi_moe_forward_timed: kernels run one after the other on one stream "
-                         "(for per-kernel profiles; a prefill-sized mi_moe_forward runs four chains side by side)")
+                         "(for per-kernel profiles; a prefill-sized mi_moe_forward of 8-bit codes runs chains side by side)")
     ap.add_argument("--seed", type=int, default=0)
     ap.add_argument("--only-headline", action="store_true", help="run only the headline batch of the workload")
     ap.add_argument("--batches", default="", help="comma-separated batch sizes to run besides the headline batch")

@@ -130,8 +130,8 @@ struct ForwardWs {
   bool mid;             // groups of 64: all segments in pieces on raw codes (see mid_batch)
   bool pieces;          // the same tiles for the segments of a heavy batch that are tiled, the others streamed
   bool raw_all;         // groups of 32 / 128: all segments in tiles (see raw_all_tiles)
-  bool raw;             // group sizes 32 / 128: the products on raw codes (qmm_rows, qmm_codes)
-  uint32_t *raw_tiles;  // the short tiles of qmm_codes, the paired copy of x (4-bit) and the group sums of x and h, or nullptr:
+  bool raw;             // group sizes 32 / 128: the products on raw codes (qmm_rows, qmm_tiles)
+  uint32_t *raw_tiles;  // the list of tiles on raw codes, the paired copy of x (4-bit) and the group sums of x and h, or nullptr:
   int raw_cap;          // (groups of 32 / 128) all segments go through the kernel of a few rows, in as many passes as they need
   int raw_from;         // segments of this many rows and more are cut into short tiles
   int raw_piece;        // of this many rows
@@ -179,7 +179,8 @@ bool raw_all_tiles(const mi_moe_config &c, int64_t T) {
 }
 // Groups of 64, 4-bit codes: batches whose segments all go through pieces on raw codes, in one launch a product on the caller's
 // stream (the others: streamed segments, and tiles of 256 weight rows on side streams).  From the batches on for which the tile lists
-// are built and the router has kernels of its own, up to 96 rows per expert on average.  Measured when pieces had 64 rows, us of a forward, other route / this one:
+// are built and the router has kernels of its own, up to 96 rows per expert on average (beyond: piece_batch).  Measured when pieces had 64 rows, in the experts' order, us
+// of a forward, other route / this one (now, same card as the first table of list_pieces: 117 at 203 tokens, 153 at 700, 182 at 1100, even routing):
 //   128 experts, hidden 2048, even routing at 96 / 128 / 203 / 320 / 512 / 1024 / 2048 / 4096 tokens 145, 151, 176, 216, 218, 266, 360, 484 /
 //   128, 124, 128, 134, 168, 221, 350, 566; Zipf-1.1 136, 139, 160, 173, 193, 237, 344, 490 / 92, 95, 114, 134, 157, 219, 341, 560;
 //   hidden 4096, intermediate 1536, even at 128 / 256 / 512 / 1024 / 2048 tokens 536, 587, 665, 785, 1144 / 372, 375, 449, 649, 1101; Zipf-1.3
@@ -205,7 +206,10 @@ int piece_rows(int64_t pairs, int n_experts) { return pairs < (int64_t)48 * n_ex
 // Larger batches: the same pieces for the segments of nine rows and more, the others streamed ahead of them.  Us of a forward, tiles of 256 weight rows in three
 // classes on two streams / this: 128 experts, hidden 2048, 4096 tokens, Zipf-1.1 501 / 492; hidden 4096, 8192 tokens, Zipf-1.3 3052 / 2972; gate/up and down
 // kernels of 8192 tokens, even routing, 840 / 800.  Nearer to float64 as well (3.87e-3 / 2.87e-3), since the weights are not rounded.  Streaming them
-// beside the tiles on a side stream, or from two or four rows on through the tiles: the same times.
+// beside the tiles on a side stream, or only those of one row, or of one to three: the same times, since each way keeps both launches.  Without them, every segment
+// in pieces as in the middle range, streamed / not, even and Zipf-1.1 at 1600 / 2048 / 3000 / 4096 / 8192 tokens (hidden 2048): 232, 282, 371, 473, 860 and 281, 303,
+// 400, 479, 851 / 227, 278, 367, 469, 855 and 261, 289, 377, 475, 842; hidden 4096, Zipf-1.3, 4096 and 8192 tokens 1635, 2923 / 1619, 2900.  So the line at 96 rows
+// an expert is where the 256-column tiles used to begin, and no longer where either side is the faster one.
 bool piece_batch(const mi_moe_config &c, int64_t T, bool heavy) {
   const int64_t P = T * c.top_k;
   return heavy && c.bits == 4 && T > kFusedRouterMaxTokens && P >= 512 && c.n_experts >= 8 && codes_tiles_fit(c, T);

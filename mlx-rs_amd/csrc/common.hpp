@@ -372,7 +372,7 @@ hipError_t launch_qmm_plain(const void *x, const uint32_t *w, const void *scales
                             const uint32_t *lhs, const uint32_t *rhs, const uint32_t *rhs_map,
                             const uint32_t *dst_map, uint32_t n_lhs, uint32_t n_rhs, int64_t rows, int M, int N,
                             int K, int group, int bits, bool transpose, int dt, void *y, hipStream_t st);
-// The tiled product on raw codes (qmm_codes.hip): bfloat16 and float16, groups of 32 / 64 / 128, 4- and 8-bit codes,
+// The tiled products on raw codes (qmm_tiles.hip, qmm_codes.hip): bfloat16 and float16, groups of 32 / 64 / 128, 4- and 8-bit codes,
 // transposed weights.  x: what launch_prepare_rows made of the rows (`copy` where codes_copy_bytes is not zero, else
 // the rows themselves), sums: the group sums it wrote.
 struct CodesArgs {

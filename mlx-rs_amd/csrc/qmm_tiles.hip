@@ -375,8 +375,8 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
 // sub-tile) issue beside the matrix instructions at 4 cycles each, about 1250 cycles a stage of 64 x 64 x 128 in c = 0 where its multiplies are
 // 1024; two waves a SIMD reach 0.55 of that, as reads, copies and the barrier of a stage add their latencies.  4096 x 4096, 777 rows, bf16 4-bit:
 // 58.7 us for the call = 444 TFLOP/s (tiles of 64 x 128 with the codes loaded into registers 63.4).
-// Blocks (128 experts, hidden 2048, 4-bit, groups of 64), us of a forward at 128 / 320 / 1024 tokens, even routing: 127 / 132 / 221; with streamed
-// segments, 256-column tiles and a copy of x on four streams, which they took before, 151 / 216 / 266.
+// Blocks (128 experts, hidden 2048, 4-bit, groups of 64), us of a forward at 128 / 320 / 1024 tokens, even routing: 110 / 121 / 174; with streamed
+// segments, 256-column tiles and a copy of x on four streams, which they took at first, 151 / 216 / 266.
 template <int DT, int BITS, bool G32, bool LIST, bool GLU, bool MID, int MS, int NT, int WN, int KW, int S>
 __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t row0, int rows, int n0, int scale_shift, unsigned char *lds_raw) {
   typedef Tile<DT, BITS, G32, MID, MS, NT, WN, S> P;
@@ -745,9 +745,10 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
 //   codes       two places of 128 K values, the wave's own; unpacked while the last token rows of the 64 values before are multiplied.
 // Two blocks share a CU and fill each other's waits.
 // What bounds it: 2048 cycles of matrix work a wave and 128 K values beside 1640 of vector instructions (256 scaled additions, 112 of unpacking), the reads of
-// LDS, and the clock, 1.8 to 1.9 GHz under all of them: the loop alone, fed from LDS, 1390 TFLOP/s.  65536 rows of 128 experts, K = 2048, 1536
-// columns 504 us = 818 TFLOP/s; K = 4096, 3072 columns 948 (tiles of 256 x 256 with their weights dequantised once a block 764 and 900, all classes).  A block
-// takes 77 us a slot at K = 2048, some 12 of them its ends.
+// LDS, and the clock, 1.8 to 1.9 GHz under all of them on a warm card: a copy of the loop alone, fed from LDS, reached 1390 TFLOP/s.  65536 rows of 128 experts, K = 2048,
+// 1536 columns 504 us = 818 TFLOP/s; K = 4096, 3072 columns 948 (tiles of 256 x 256 with their weights dequantised once a block 764 and 900, all classes).  A block
+// takes 77 us a slot at K = 2048, some 12 of them its ends.  Counters, 32 620 rows, gate/up: matrix units 0.47 busy, 9.1 vector instructions a multiply with all that is
+// outside the loop.  GLU keeps 18 registers a lane in scratch memory around the loop over windows (else 12): 27 of the 81 MB that gate/up writes, 23 of down's 157.
 struct LongRing {
   static constexpr int XROW = 128, W = 4096, WALL = 4 * W, WINDOWS = 4 * 2048;
   static constexpr int bytes(int ms) { return 2 * (32 * ms * XROW) + 2 * WALL + WINDOWS + ms * 1024; }
