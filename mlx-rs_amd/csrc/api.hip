@@ -197,11 +197,20 @@ bool mid_batch(const mi_moe_config &c, int64_t T, bool tiled) {
   return tiled && c.bits == 4 && T > kFusedRouterMaxTokens && P <= (int64_t)96 * c.n_experts && P >= 512 && c.n_experts >= 8 && codes_tiles_fit(c, T);
 }
 
-// Rows of a piece.  Longer ones read a weight row for more token rows; but a block's time grows with its rows, and until the pieces are several times what
-// the chip holds at once, the longest segments' blocks are what a launch waits for.  Gate/up and down kernels, us, pieces of 64 / 96 / 128 rows (128 experts,
-// hidden 2048) at an average of 13, 32, 64, 94 rows: Zipf-1.1 70, 109, 161, 217 / 85, 117, 164, 219 / 93, 124, 181, 224; even 91, 116, 163, 223 / 90, 116, 147,
-// 212 / 89, 113, 151, 183; at 256 rows, Zipf-1.1, 446 / 421 / 422.
-int piece_rows(int64_t pairs, int n_experts) { return pairs < (int64_t)48 * n_experts ? 64 : pairs < (int64_t)80 * n_experts ? 96 : kPieceM; }
+// Batches whose pieces go to qmm_short_kernel, 64 rows and less.  Us of a forward, qmm_pieces_kernel (64 rows up to 48 an expert on average, 96 from there) / this, one card:
+//   128 experts, hidden 2048, even routing at 96 / 160 / 240 / 330 / 512 / 700 / 900 / 1024 / 1280 tokens 107, 111, 113, 121, 135, 151, 168, 170, 194 / 95, 99, 104, 113, 122,
+//   137, 156, 179, 220; Zipf-1.1 at 512 / 700 / 1024 / 1500 tokens 159, 179, 197, 244 / 149, 169, 196, 242; 1.3 at 96 / 250 / 700 / 1500 tokens 99, 84, 181, 251 / 88, 81, 170, 248;
+//   hidden 4096, intermediate 1536, even at 96 / 250 / 400 / 700 / 900 / 1024 tokens 343, 357, 370, 476, 507, 525 / 319, 340, 357, 443, 492, 604; Zipf-1.3 at 96 / 250 / 700
+//   tokens 312, 299, 552 / 288, 284, 526;
+//   64 experts, 6, hidden 2048, intermediate 1408, even at 100 / 165 / 600 / 900 tokens (56 and 84 rows) 99, 102, 148, 174 / 90, 95, 144, 192; 64, 4, 4096 x 2048, 200 tokens 244 / 230;
+//   256 experts, 8, 2048 x 512, 200 / 500 tokens 145, 151 / 132, 145.
+// With even routing most segments leave a second piece from about 60 rows on average on, and the line lies there; with skewed routing it makes no difference.
+bool short_pieces(int64_t pairs, int n_experts) { return pairs < (int64_t)60 * n_experts; }
+
+// Rows of a piece beyond those.  Longer ones read a weight row for more token rows; but a block's time grows with its rows, and until the pieces are several times what
+// the chip holds at once, the longest segments' blocks are what a launch waits for.  Gate/up and down kernels, us, pieces of 96 / 128 rows (128 experts,
+// hidden 2048) at an average of 64, 94 rows: Zipf-1.1 164, 219 / 181, 224; even 147, 212 / 151, 183; at 256 rows, Zipf-1.1, 421 / 422.
+int piece_rows(int64_t pairs, int n_experts) { return short_pieces(pairs, n_experts) ? kShortTileM : pairs < (int64_t)80 * n_experts ? 96 : kPieceM; }
 
 // Larger batches: the same pieces for the segments of nine rows and more, the others streamed ahead of them.  Us of a forward, tiles of 256 weight rows in three
 // classes on two streams / this: 128 experts, hidden 2048, 4096 tokens, Zipf-1.1 501 / 492; hidden 4096, 8192 tokens, Zipf-1.3 3052 / 2972; gate/up and down
@@ -630,10 +639,12 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     return launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, s);
   };
   auto tiles_up = [&](hipStream_t s) -> hipError_t {
+    if (mid && short_pieces(P, c.n_experts)) return launch_qmm_short(ca, f.raw_tiles, f.raw_cap, true, s);
     if (raw_codes) return launch_qmm_pieces(ca, f.raw_tiles, f.raw_cap, true, s);
     return launch_qmm_codes_tiles(ca, f.raw_tiles, f.raw_cap, c.group_size, c.bits, true, s);
   };
   auto tiles_down = [&](hipStream_t s) -> hipError_t {
+    if (mid && short_pieces(P, c.n_experts)) return launch_qmm_short(cd, f.raw_tiles, f.raw_cap, false, s);
     if (raw_codes) return launch_qmm_pieces(cd, f.raw_tiles, f.raw_cap, false, s);
     return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.group_size, c.bits, false, s);
   };

@@ -426,8 +426,9 @@ hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, in
                                uint16_t *sums, hipStream_t st);
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
 hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st);
-// 4-bit codes in groups of 64, a list of pieces of 64, 96 or 128 rows (ShortTiles::piece)
+// 4-bit codes in groups of 64, a list of pieces of 96 or 128 rows (ShortTiles::piece), or of 64 (qmm_short.hip)
 hipError_t launch_qmm_pieces(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
+hipError_t launch_qmm_short(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
 hipError_t launch_quantize(const float *w, int64_t rows, int64_t cols, int group, int bits,
                            uint32_t *q, void *s, void *b, int dt, hipStream_t st);
 hipError_t launch_dequantize(const uint32_t *q, const void *s, const void *b,

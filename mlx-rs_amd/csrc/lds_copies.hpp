@@ -24,6 +24,7 @@ template <int N>
 __device__ __forceinline__ void wait_copies() {  // all but the last N have arrived; LDS reads are done
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
+__device__ __forceinline__ void wait_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }  // of LDS, and writes to it
 __device__ __forceinline__ void block_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
 }  // namespace mi_moe

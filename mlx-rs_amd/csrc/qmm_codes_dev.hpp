@@ -77,6 +77,24 @@ __device__ __forceinline__ void prepare_octet(const PrepareArgs &a, int64_t i) {
   }
 }
 
+// The eight codes of a word as bf16, in the order kQuads.  A byte of 0 to 15 is that many 2^-9 as an 8-bit float (four exponent bits, three of mantissa): the
+// conversion takes two at a time.
+__device__ __forceinline__ void plain_codes(uint32_t w, u32x4_t &o) {
+  const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
+  o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false));
+  o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false));
+  o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true));
+  o[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, true));
+}
+
+// silu(g) u, fp32.  The quotient is as the division gives it.  1 + exp(-g) reaches 2^128, so the reciprocal is taken of a quarter of it (beyond 2^126 that of a
+// normal number is none, and v_rcp_f32 gives zero) and one correction follows; where the sum is infinite the quotient is zero, and no correction (an infinite g
+// comes out as no number, and is looked at again with all that are not finite).
+__device__ __forceinline__ float gated(float g, float u) {
+  const float d = 1.0f + __expf(-g), r = __builtin_amdgcn_rcpf(0.25f * d) * 0.25f, q = g * r;
+  return (d < INFINITY ? __builtin_fmaf(__builtin_fmaf(-d, q, g), r, q) : q) * u;
+}
+
 // A kernel's leave to use more than 64 KB of LDS, asked for once a GPU (half a microsecond a launch otherwise).  done: a bit per GPU.
 inline hipError_t allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &done) {
   int dev = 0;

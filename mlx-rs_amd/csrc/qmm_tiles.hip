@@ -87,12 +87,7 @@ struct Tile {
   // the eight codes of multiply h
   static __device__ __forceinline__ void unpack(const u32x4_t (&q)[NQ], int h, u32x4_t &o) {
       if constexpr (kPlainCodes) {
-        // a byte of 0 to 15 is that many 2^-9 as an 8-bit float (four exponent bits, three of mantissa): the conversion takes two at a time
-        const uint32_t w = q[0][h], even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
-        o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false));
-        o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false));
-        o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true));
-        o[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, true));
+        plain_codes(q[0][h], o);
       } else if constexpr (BITS == 4 && DT == 0) {
         float v[8];
         centred_codes(q[0][h], v);
@@ -238,13 +233,6 @@ __device__ __forceinline__ void output_rows(const CodesArgs &a, int64_t row0, in
     const int64_t r = row0 + (64 * h + lane < rows ? 64 * h + lane : rows - 1);
     dst[h] = a.dst_rows ? a.dst_rows[r] : (uint32_t)r;
   }
-}
-// silu(g) u, fp32.  The quotient is as the division gives it.  1 + exp(-g) reaches 2^128, so the reciprocal is taken of a quarter of it (beyond 2^126 that of a
-// normal number is none, and v_rcp_f32 gives zero) and one correction follows; where the sum is infinite the quotient is zero, and no correction (an infinite g
-// comes out as no number, and is looked at again with all that are not finite).
-__device__ __forceinline__ float gated(float g, float u) {
-  const float d = 1.0f + __expf(-g), r = __builtin_amdgcn_rcpf(0.25f * d) * 0.25f, q = g * r;
-  return (d < INFINITY ? __builtin_fmaf(__builtin_fmaf(-d, q, g), r, q) : q) * u;
 }
 // The results of a piece of up to 32 MS rows x 256 weight rows (of a block; four waves, 64 weight rows each) go out: N is a multiple of
 // 128, there is no bias of the layer's.  Two rows of a column become one register, neighbouring lanes swap halves, and the rows are turned round in LDS:
