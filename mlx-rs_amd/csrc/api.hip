@@ -129,11 +129,11 @@ struct ForwardWs {
   uint16_t *gu;  // plain products only: the gate and the up product, [P, I] each
   bool mid;             // groups of 64: all segments in pieces on raw codes (see mid_batch)
   bool pieces;          // the same tiles for the segments of a heavy batch that are tiled, the others streamed
-  bool raw_all;         // groups of 32 / 128: all segments in tiles (see raw_all_tiles)
-  bool raw;             // group sizes 32 / 128: the products on raw codes (qmm_rows, qmm_tiles)
-  uint32_t *raw_tiles;  // the list of tiles on raw codes, the paired copy of x (4-bit) and the group sums of x and h, or nullptr:
+  bool raw_all;         // groups of 32 / 128: all segments in pieces (see raw_list_batch)
+  bool raw;             // group sizes 32 / 128: the products on raw codes (qmm_rows, qmm_short)
+  uint32_t *raw_tiles;  // the list of pieces, the copy of x in their order (4-bit) and the group sums of x and h, or nullptr:
   int raw_cap;          // (groups of 32 / 128) all segments go through the kernel of a few rows, in as many passes as they need
-  int raw_from;         // segments of this many rows and more are cut into short tiles
+  int raw_from;         // segments of this many rows and more are cut into pieces
   int raw_piece;        // of this many rows
   uint16_t *raw_copy, *raw_xsums, *raw_hsums;
   size_t bytes_raw;     // up to the end of those
@@ -142,9 +142,7 @@ struct ForwardWs {
   size_t bytes;
 };
 
-// Group sizes 32 and 128: tile lists are built (for segments of more rows than one pass of the kernel of a few rows, which
-// a segment of at most T rows has to be able to have) from an average of four rows per expert on; see forward_impl for what that
-// costs and gives.  The tiled kernel takes operands below 2 GiB, in multiples of 128 values.
+// The kernels that take a list of pieces: operands below 2 GiB, in multiples of 128 values.
 bool codes_tiles_fit(const mi_moe_config &c, int64_t T) {
   const int64_t P = T * c.top_k, most = (int64_t)1 << 31;
   return c.hidden % 128 == 0 && c.intermediate % 128 == 0 && T * c.hidden * 2 < most &&
@@ -152,30 +150,17 @@ bool codes_tiles_fit(const mi_moe_config &c, int64_t T) {
          (int64_t)codes_sums_bytes(T, c.hidden, c.group_size) < most &&
          (int64_t)c.hidden * c.intermediate * c.bits / 8 < most;
 }
-bool raw_tiled_batch(const mi_moe_config &c, int64_t T) {
+// Group sizes 32 and 128: batches whose segments all go in pieces (qmm_short_kernel), one launch a product; the others go through the kernel of a few rows, which a
+// segment of at most T rows has to be more than one pass of.  Us of a forward, tiles of 32 x 32 results (qmm_tiles.hip; with 8-bit codes between twenty and forty rows
+// an expert short segments on the kernel of a few rows beside them, on another stream) / pieces, (experts, k, hidden, intermediate, bits, group):
+//   128, 8, 2048, 768, 4, 32   even at 100 / 160 / 256 / 400 / 512 tokens 150, 150, 153, 169, 175 / 120, 123, 130, 147, 151; Zipf-1.1 at 100 / 256 / 512 145, 118, 164 / 116, 102, 145
+//   128, 8, 2048, 768, 4, 128  even at 100 / 256 / 512 114, 121, 137 / 92, 108, 119; Zipf-1.1 at 512 171 / 149
+//   128, 8, 2048, 768, 8, 32   even at 100 / 330 / 512 199, 236, 248 / 187, 200, 208; Zipf-1.1 at 330 / 512 260, 213 / 234, 193; 1.3 at 500 189 / 180
+//   128, 8, 2048, 768, 8, 128  even at 330 / 512 194, 198 / 160, 169; Zipf-1.1 at 330 / 512 229, 180 / 184, 151
+//   64, 6, 2048, 1408, 4, 32   128 tokens, even and Zipf-1.1 140, 170 / 115, 137; 8, 2, 4096, 7168, 4, 32 at 256 tokens 348 / 297; 8, 2, 4096, 14336, 8, 32 at 100 645 / 515
+// All segments on the kernel of a few rows (4-bit, 32): 512 tokens and even routing 328, Zipf-1.1 1017.
+bool raw_list_batch(const mi_moe_config &c, int64_t T) {
   return T > kRowsMost && T * c.top_k >= (int64_t)4 * c.n_experts && codes_tiles_fit(c, T);
-}
-// Batches of those sizes whose segments all go through the tiles, in one launch a product on the caller's stream.  The others (8-bit codes, twenty to forty
-// rows an expert) keep the short segments on the kernel of a few rows, beside the tiles on a side stream: with skewed routing that is 1 to 12 % faster
-// there, with even routing 7 to 15 % slower.  Measured, us of a forward, side by side / all in tiles, at an average of 5, 8, 12, 16, 24, 32, 48, 96 rows
-// (experts, k, hidden, intermediate, bits, group; below sixteen rows with 4-bit codes in groups of 32 the other tiles had their codes in registers; all in tiles
-// before their list had the longest pieces first):
-//   128, 8, 2048, 768, 4, 32   even 155, 169, 182, 183, 198, 211, 247, 357 / 151, 151, 153, 155, 166, 186, 226, 335; Zipf-1.1 126, 131, 135, 164, 166, 184, 238,
-//                              359 / 108, 113, 126, 144, 168, 185, 217, 336; 1.3 121, 129, 131, 160, 158, 177, 225, 346 / 91, 110, 116, 125, 156, 174, 210, 309
-//   128, 8, 2048, 768, 4, 128  even 139, 150, 157, 168, 158, 171, 199, 280 / 118, 119, 123, 124, 133, 144, 169, 256; Zipf-1.1 118, 122, 128, 138, 138, 153, 194,
-//                              282 / 84, 89, 101, 109, 129, 143, 173, 262
-//   64, 6, 2048, 1408, 4, 32   Zipf-1.1 120, 135, 135, 162, 177, 187, 225, 333 / 121, 129, 148, 157, 164, 189, 224, 315; even 143, 165, 181, 192, 182, 190, 224, 318 /
-//                              143, 142, 143, 144, 153, 173, 196, 298
-//   8, 2, 4096, 7168, 4, 32    even 229, 252, 304, 319, 259, 295, 297, 407 / 207, 207, 208, 208, 219, 270, 272, 385; Zipf-1.1 234, 352, 340, 382, 384, 356, 416,
-//                              403 / 207, 207, 208, 258, 270, 331, 367, 385
-//   128, 8, 2048, 768, 8, 32   Zipf-1.1 144, 167, 171, 181, 196, 224, 280, 406 / 123, 125, 146, 184, 207, 229, 271, 396; 1.3 133, 144, 160, 176, 178, 208, 272, 387 /
-//                              108, 121, 129, 147, 198, 213, 255, 360
-// With it the skewed batches of 4-bit codes in groups of 32 that had become slower are not: 128 experts, Zipf-1.1 at 160 / 256 / 400 tokens 178, 191, 201 / 175, 185,
-// 199; left are 64 experts at 128 tokens (12 rows), 169 / 171, and 128 at 512 (32 rows), 215 / 221, where even routing has 182 / 141 and 212 / 173: the host does
-// not see which it is.
-bool raw_all_tiles(const mi_moe_config &c, int64_t T) {
-  const int64_t P = T * c.top_k, E = c.n_experts;
-  return raw_tiled_batch(c, T) && (c.bits == 4 || P < 20 * E || P >= 40 * E);
 }
 // Groups of 64, 4-bit codes: batches whose segments all go through pieces on raw codes, in one launch a product on the caller's
 // stream (the others: streamed segments, and tiles of 256 weight rows on side streams).  From the batches on for which the tile lists
@@ -265,7 +250,7 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
   f.gu = cv.take<uint16_t>(plain_config(c) && !f.raw ? 2 * (size_t)P * c.intermediate : 0);
   f.raw_tiles = nullptr;
   f.raw_cap = 0;
-  f.raw_from = kRowsMost + 1;
+  f.raw_from = 1;
   f.raw_piece = kShortTileM;
   f.bytes_min = cv.off;
   f.mid = mid_batch(c, T, f.tiled);
@@ -274,7 +259,6 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
     // All of it lies in memory that is free at the time where it fits, so that batches which have to fit a scratch of a given size take
     // this route as well: the list in place of the work records (nothing is streamed), the group sums of x where the down product writes
     // its rows later, those of h in the normalised rows, which only the router and the copy of x read.
-    f.raw_from = 1;
     f.raw_piece = piece_rows(P, c.n_experts);
     f.raw_cap = short_list_cap(P, c.n_experts, 1, f.raw_piece);
     const size_t list = short_list_words(f.raw_cap), xsums = codes_sums_bytes(T, c.hidden, c.group_size, true), hsums = codes_sums_bytes(P, c.intermediate, c.group_size, true);
@@ -296,9 +280,8 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
     f.raw_xsums = in_norm ? f.xnorm : cv.take<uint16_t>(xsums / 2);
     f.raw_hsums = in_norm ? f.xnorm + xsums / 2 : cv.take<uint16_t>(hsums / 2);
   }
-  f.raw_all = f.raw && raw_all_tiles(c, T);
-  if (f.raw && raw_tiled_batch(c, T)) {
-    if (f.raw_all) f.raw_from = 1;
+  f.raw_all = f.raw && raw_list_batch(c, T);
+  if (f.raw_all) {
     f.raw_cap = short_list_cap(P, c.n_experts, f.raw_from, f.raw_piece);
     f.raw_tiles = cv.take<uint32_t>(short_list_words(f.raw_cap));
     f.raw_copy = cv.take<uint16_t>(codes_copy_bytes(c.bits, T, c.hidden) / 2);
@@ -611,11 +594,11 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   if (f.tiled && paired && !streamed_first && !pair_in_router && !raw_codes) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));
   // independent chains run beside each other where side streams are to be had, whose lock is held until they have been joined back
   std::unique_lock<std::mutex> streams_guard;
-  const bool chains = !ev && !mid && !f.raw_all && (f.raw ? f.raw_tiles != nullptr : !plain_config(c) && large_qmm_applies(a));
+  const bool chains = !ev && !mid && !f.raw_all && !plain_config(c) && large_qmm_applies(a);
   if (chains) streams_guard = std::unique_lock<std::mutex>(h->streams->lock);
   const bool fork = chains && may_fork(st, *h->streams);
   if (!fork && streamed_first && paired && large_qmm_applies(a)) MI_HIP(launch_pair_rows(x, T, c.hidden, f.xperm, st));  // (a side stream's work)
-  // the short tiles on raw codes
+  // the pieces
   CodesArgs ca{}, cd{};
   const bool copied = codes_copy_bytes(c.bits, T, c.hidden) > 0;
   ca.x = copied ? f.raw_copy : x;
@@ -625,7 +608,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   ca.w0 = h->w.gate.w; ca.s0 = h->w.gate.scales; ca.b0 = h->w.gate.biases;
   ca.w1 = h->w.up.w; ca.s1 = h->w.up.scales; ca.b1 = h->w.up.biases;
   ca.y = f.hh;
-  ca.y_order = !copied ? RowOrder::kPlain : raw_codes ? RowOrder::kQuads : RowOrder::kPaired;
+  ca.y_order = copied ? RowOrder::kQuads : RowOrder::kPlain;
   ca.y_sums = f.raw_hsums;
   ca.N = c.intermediate; ca.K = c.hidden;
   cd.x = f.hh;
@@ -635,18 +618,13 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   cd.w0 = h->w.down.w; cd.s0 = h->w.down.scales; cd.b0 = h->w.down.biases;
   cd.y = f.y;
   cd.N = c.hidden; cd.K = c.intermediate;
-  auto prepare_x = [&](hipStream_t s) -> hipError_t {
-    return launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, copied ? f.raw_copy : nullptr, f.raw_xsums, s);
-  };
   auto tiles_up = [&](hipStream_t s) -> hipError_t {
-    if (mid && short_pieces(P, c.n_experts)) return launch_qmm_short(ca, f.raw_tiles, f.raw_cap, true, s);
-    if (raw_codes) return launch_qmm_pieces(ca, f.raw_tiles, f.raw_cap, true, s);
-    return launch_qmm_codes_tiles(ca, f.raw_tiles, f.raw_cap, c.group_size, c.bits, true, s);
+    if (f.raw_piece > kShortTileM) return launch_qmm_pieces(ca, f.raw_tiles, f.raw_cap, true, s);
+    return launch_qmm_short(ca, f.raw_tiles, f.raw_cap, c.group_size, c.bits, true, s);
   };
   auto tiles_down = [&](hipStream_t s) -> hipError_t {
-    if (mid && short_pieces(P, c.n_experts)) return launch_qmm_short(cd, f.raw_tiles, f.raw_cap, false, s);
-    if (raw_codes) return launch_qmm_pieces(cd, f.raw_tiles, f.raw_cap, false, s);
-    return launch_qmm_codes_tiles(cd, f.raw_tiles, f.raw_cap, c.group_size, c.bits, false, s);
+    if (f.raw_piece > kShortTileM) return launch_qmm_pieces(cd, f.raw_tiles, f.raw_cap, false, s);
+    return launch_qmm_short(cd, f.raw_tiles, f.raw_cap, c.group_size, c.bits, false, s);
   };
   struct TimerScope {  // a timer never outlives the launch it is meant for
     explicit TimerScope(KernelTimer *t) { g_kernel_timer = t; }
@@ -676,17 +654,18 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
       MI_STAGE_DONE();
     }
   } else if (f.raw_all) {
-    if (fused_router) MI_HIP(prepare_x(st));
+    if (fused_router)
+      MI_HIP(launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, true, copied ? f.raw_copy : nullptr, f.raw_xsums, st));
     MI_HIP(tiles_up(st));
     MI_STAGE_DONE();
     MI_HIP(tiles_down(st));
     MI_STAGE_DONE();
   } else if (f.raw) {
-    // group sizes 32 / 128: short segments on the kernel of a few rows, longer ones (where lists are built) in tiles
+    // group sizes 32 / 128 without lists: the kernel of a few rows
     RowsArgs ra{}, rd{};
     ra.work = f.work;
     ra.max_active = max_active;
-    ra.max_rows = f.raw_tiles ? kRowsMost : T;
+    ra.max_rows = T;
     rd = ra;
     ra.x = x;
     ra.src_rows = f.src_of;
@@ -700,34 +679,10 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     rd.w0 = h->w.down.w; rd.s0 = h->w.down.scales; rd.b0 = h->w.down.biases;
     rd.y = f.y;
     rd.N = c.hidden; rd.K = c.intermediate;
-    if (fork) {
-      // The two chains share no rows (which batches come here: raw_all_tiles): the short segments beside the tiles, which are the longer chain as far as the
-      // host can tell.  All segments through the kernel of a few rows: 328 us for 512 tokens and even routing, Zipf-1.1 1017 (128 experts, groups of 32).
-      DeviceStreams &ds = *h->streams;
-      hipStream_t s = ds.side[0];
-      MI_HIP(hipEventRecord(ds.fork, st));
-      MI_HIP(hipStreamWaitEvent(s, ds.fork, 0));
-      hipError_t e = prepare_x(st);
-      if (e == hipSuccess) e = tiles_up(st);
-      if (e == hipSuccess) e = tiles_down(st);
-      if (e == hipSuccess) e = launch_qmm_rows(ra, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true, s);
-      if (e == hipSuccess) e = launch_qmm_rows(rd, c.group_size, c.bits, MI_MOE_DTYPE_BF16, false, s);
-      // whatever happened: the caller's stream waits for what the side stream was given
-      hipError_t je = hipEventRecord(ds.join[0], s);
-      if (je == hipSuccess) je = hipStreamWaitEvent(st, ds.join[0], 0);
-      MI_HIP(e);
-      MI_HIP(je);
-    } else {
-      if (f.raw_tiles) {
-        MI_HIP(prepare_x(st));
-        MI_HIP(tiles_up(st));
-      }
-      MI_HIP(launch_qmm_rows(ra, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true, st));
-      MI_STAGE_DONE();
-      if (f.raw_tiles) MI_HIP(tiles_down(st));
-      MI_HIP(launch_qmm_rows(rd, c.group_size, c.bits, MI_MOE_DTYPE_BF16, false, st));
-      MI_STAGE_DONE();
-    }
+    MI_HIP(launch_qmm_rows(ra, c.group_size, c.bits, MI_MOE_DTYPE_BF16, true, st));
+    MI_STAGE_DONE();
+    MI_HIP(launch_qmm_rows(rd, c.group_size, c.bits, MI_MOE_DTYPE_BF16, false, st));
+    MI_STAGE_DONE();
   } else if (plain_config(c)) {
     // 2-bit codes, or rows the kernels on raw codes do not take: the plain products, one output row per sorted pair.  Row r of
     // the sorted order belongs to pair perm[r], token src_of[r], expert topk_idx[perm[r]].
@@ -1264,7 +1219,7 @@ static int quantized_matmul_impl(const void *x, const uint32_t *w, const void *s
     const size_t copy_bytes = codes_copy_bytes(bits, M, K);
     uint16_t *copy = copy_bytes ? reinterpret_cast<uint16_t *>(cv.take<char>(copy_bytes)) : nullptr;
     uint16_t *sums = reinterpret_cast<uint16_t *>(cv.take<char>(codes_sums_bytes(M, K, group_size)));
-    MI_HIP(launch_prepare_rows(x, M, K, group_size, dtype, copy, sums, st));
+    MI_HIP(launch_prepare_rows(x, M, K, group_size, dtype, false, copy, sums, st));
     CodesArgs a{};
     a.x = copy ? copy : x;
     a.x_rows = M;

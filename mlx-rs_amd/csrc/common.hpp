@@ -329,8 +329,7 @@ struct PrepareArgs {
   int64_t octets = 0;  // 8-blocks of x in all, and of a row; 0: nothing to prepare
   int octets_per_row = 0, lanes_log2 = 0;  // (of a group)
   uint16_t *copy = nullptr, *sums = nullptr;
-  int sums_row = 0;
-  bool plain = false;  // for the products on codes without a centre (launch_qmm_pieces)
+  int sums_row = 0, slots = 0;  // of a row of sums; of a group's: 4 for the products on codes without a centre (4-bit blocks in groups of 64), else 8
 };
 // decode-sized batches: logits + selection + dispatch in one launch.  counters: 1 +
 // kFusedRouterMaxTokens zero-initialised words that the kernel leaves zeroed again.  norm_w != nullptr:
@@ -419,16 +418,16 @@ struct ColsArgs {
 bool qmm_cols_applies(const ColsArgs &a, int bits, int dt);
 hipError_t launch_qmm_cols(const ColsArgs &a, int group, int bits, int dt, hipStream_t st);
 size_t codes_copy_bytes(int bits, int64_t rows, int K);
-// plain: for the products on codes without a centre (launch_qmm_pieces)
+// plain: for the products on codes without a centre
 size_t codes_sums_bytes(int64_t rows, int K, int group, bool plain = false);
 PrepareArgs prepare_args(const void *x, int64_t rows, int K, int group, uint16_t *copy, uint16_t *sums, bool plain);
-hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
+// list: for the pieces of a list (4-bit codes: the copy in the order kQuads), else for a dense product (kPaired)
+hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, bool list, uint16_t *copy,
                                uint16_t *sums, hipStream_t st);
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st);
-hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st);
-// 4-bit codes in groups of 64, a list of pieces of 96 or 128 rows (ShortTiles::piece), or of 64 (qmm_short.hip)
+// A list of pieces of up to 64 rows (ShortTiles::piece), bf16; 4-bit codes in groups of 64 also of 96 or 128
+hipError_t launch_qmm_short(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st);
 hipError_t launch_qmm_pieces(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
-hipError_t launch_qmm_short(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
 hipError_t launch_quantize(const float *w, int64_t rows, int64_t cols, int group, int bits,
                            uint32_t *q, void *s, void *b, int dt, hipStream_t st);
 hipError_t launch_dequantize(const uint32_t *q, const void *s, const void *b,

@@ -18,8 +18,8 @@ __device__ __forceinline__ bool prepares(const PrepareArgs &a, int first) {
   if ((int)blockIdx.x < first) return false;
   const int64_t i = (int64_t)((int)blockIdx.x - first) * kDispThreads + threadIdx.x;
   if (i >= a.octets) return true;  // (whole groups leave together)
-  if (a.plain) prepare_octet<0, true>(a, i);
-  else prepare_octet<0, false>(a, i);
+  if (a.slots == sum_slots(true)) prepare_octet<0, RowOrder::kQuads, sum_slots(true)>(a, i);
+  else prepare_octet<0, RowOrder::kQuads, sum_slots(false)>(a, i);
   return true;
 }
 static unsigned prepare_blocks(const PrepareArgs &a) { return (unsigned)((a.octets + kDispThreads - 1) / kDispThreads); }

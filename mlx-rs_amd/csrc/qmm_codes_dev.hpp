@@ -22,23 +22,24 @@ __device__ __forceinline__ Pieces split3(float v) {
   return Pieces{hu >> 16, mu >> 16, __float_as_uint(q) >> 16};
 }
 
-// A group sum of a row as the bias product's operand: the pieces against those of the biases (six products), or against one.
-__device__ __forceinline__ void put_sums(uint16_t *to, int slots, float sum) {
+// A group sum of a row as the bias product's operand: the pieces against those of the biases (six products), or against one.  half: in a slot that is
+// multiplied with nothing, the sum of the group's first half, about (what of it a piece's sums start from in qmm_short.hip; the other half's start from the rest).
+__device__ __forceinline__ void put_sums(uint16_t *to, int slots, float sum, float half = 0.f) {
   const Pieces p = split3(sum);
-  if (slots == kSlots) *reinterpret_cast<uint4 *>(to) = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, 0u);
+  if (slots == kSlots) *reinterpret_cast<uint4 *>(to) = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, __float_as_uint(half) >> 16);
   else *reinterpret_cast<uint2 *>(to) = make_uint2(p.h | p.m << 16, p.l);
 }
 
 constexpr RowOrder row_order(int bits) { return bits == 4 ? RowOrder::kPaired : RowOrder::kPlain; }
 constexpr int padded_groups(int G) { return (G + 15) / 16 * 16; }  // whole windows of the bias product; the groups past the row's end are zeros
 
-// One thread's part of preparing rows: eight values of x (octet i of all rows).  Whole groups go through lanes of one wave.  PLAIN: PrepareArgs::plain.
+// One thread's part of preparing rows: eight values of x (octet i of all rows).  Whole groups go through lanes of one wave.  ORDER of the copy (kPaired or kQuads),
+// SLOTS of a group sum.
 // What bounds it is latency: as a launch of its own 4.6 us for 61 rows of 2176 and 5.2 for 611 of 1152 (bf16, with a profiler's overhead).  One lane writes all the
 // zeros behind a row's sums, so it writes 16 bytes at a time: with 8, and the two forms told apart at run time, products whose groups fill no multiple of sixteen
 // took 0.2 to 0.7 us more (61 x 2320 x 2176 4-bit 14.6 us for 14.0, 611 x 2864 x 1152 18.6 for 17.9, 494 x 960 x 2432 8-bit 17.3 for 16.6).
-template <int DT, bool PLAIN>
+template <int DT, RowOrder ORDER, int SLOTS>
 __device__ __forceinline__ void prepare_octet(const PrepareArgs &a, int64_t i) {
-  constexpr int SLOTS = sum_slots(PLAIN);
   float v[8];
   const uint4 w = reinterpret_cast<const uint4 *>(a.x)[i];
   const uint32_t u[4] = {w.x, w.y, w.z, w.w};
@@ -54,7 +55,8 @@ __device__ __forceinline__ void prepare_octet(const PrepareArgs &a, int64_t i) {
     }
   }
   if (a.copy) {
-    const uint32_t y = PLAIN ? w.z : w.y, z = PLAIN ? w.y : w.z;  // the words that meet: neighbours (kQuads), or 0 and 2, 1 and 3 (kPaired)
+    constexpr bool QUADS = ORDER == RowOrder::kQuads;
+    const uint32_t y = QUADS ? w.z : w.y, z = QUADS ? w.y : w.z;  // the words that meet: neighbours (kQuads), or 0 and 2, 1 and 3 (kPaired)
     uint4 p;
     p.x = (w.x & 0xffffu) | (z << 16);
     p.y = (w.x >> 16) | (z & 0xffff0000u);
@@ -66,12 +68,16 @@ __device__ __forceinline__ void prepare_octet(const PrepareArgs &a, int64_t i) {
   sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
   sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
   if (a.lanes_log2 >= 3) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
-  if (a.lanes_log2 == 4) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
+  float half = 0.f;
+  if (a.lanes_log2 == 4) {
+    if (ORDER == RowOrder::kQuads) half = sum;
+    sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
+  }
   if ((i & ((1 << a.lanes_log2) - 1)) == 0) {
     const int64_t row = i / a.octets_per_row;
     const int g = (int)(i % a.octets_per_row) >> a.lanes_log2, G = a.octets_per_row >> a.lanes_log2;
     uint16_t *const to = a.sums + row * a.sums_row;
-    put_sums(to + g * SLOTS, SLOTS, sum);
+    put_sums(to + g * SLOTS, SLOTS, sum, half);
     if (g == G - 1)  // (an even number of groups where a group has four slots)
       for (int k = G * SLOTS; k < a.sums_row; k += 8) *reinterpret_cast<uint4 *>(to + k) = make_uint4(0, 0, 0, 0);
   }

@@ -30,10 +30,10 @@
 namespace mi_moe {
 
 // One thread per eight values of x.
-template <int DT>
+template <int DT, RowOrder ORDER>
 __global__ __launch_bounds__(256) void prepare_rows_kernel(PrepareArgs a) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < a.octets) prepare_octet<DT, false>(a, i);  // (whole groups leave together)
+  if (i < a.octets) prepare_octet<DT, ORDER, kSlots>(a, i);  // (whole groups leave together)
 }
 
 // What a launch of the kernel below is made of, for its two sides.
@@ -959,42 +959,26 @@ __global__ __launch_bounds__(256, 2) void qmm_pieces_kernel(CodesArgs a, const u
 
 // A block computes 32 MS token rows x 32 WN weight rows with WN KW waves (see multiply_tile), tiles of up to 32 rows with half the
 // token operand.
-template <int DT, int BITS, bool G32, bool LIST, bool GLU, int MS, int NT, int WN, int KW, int S>
+template <int DT, int BITS, bool G32, int MS, int NT, int WN, int KW, int S>
 __global__ __launch_bounds__(64 * WN * KW, waves_of(WN * KW, lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES))) void qmm_tiles_kernel(
-    CodesArgs a, const uint32_t *__restrict__ list, int n_mtiles, int n_ntiles, int scale_shift) {
-  static_assert(LIST ? DT == 0 && NT == 2 && WN == 4 && KW == 1 : !GLU, "write_piece: a gate tile and its up tile, or two tiles a wave");
-  constexpr int BM = 32 * MS;
-  constexpr int NI = 32 * WN * (GLU ? 1 : NT);  // distinct output columns per block
-  // block -> (M tile, N tile).  Ids are dealt round-robin over the 8 XCDs.  Dense: an XCD takes every eighth N tile
-  // and all M tiles of it, so its L2 holds the weights of a few N tiles and x streams through.  A tile list: whole M
-  // tiles per XCD (the blocks of one share its gathered rows).
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-  int e = 0, rows, nt;
-  int64_t row0;
-  if constexpr (LIST) {
-    const uint32_t id = (uint32_t)(j / n_ntiles) * 8u + xcd;
-    nt = j % n_ntiles;
-    if (id >= list[0]) return;
-    const uint4 rec = reinterpret_cast<const uint4 *>(list)[1 + id];
-    e = __builtin_amdgcn_readfirstlane((int)rec.x);
-    row0 = (int64_t)__builtin_amdgcn_readfirstlane((int)rec.y);
-    rows = __builtin_amdgcn_readfirstlane((int)rec.z);
-  } else {
-    nt = j / n_mtiles * 8 + xcd;
-    if (nt >= n_ntiles) return;
-    row0 = (int64_t)(j % n_mtiles) * BM;
-    rows = a.M - row0 < BM ? (int)(a.M - row0) : BM;
-  }
+    CodesArgs a, int n_mtiles, int n_ntiles, int scale_shift) {
+  constexpr int BM = 32 * MS, NI = 32 * WN * NT;
+  // block -> (M tile, N tile).  Ids are dealt round-robin over the 8 XCDs: an XCD takes every eighth N tile
+  // and all M tiles of it, so its L2 holds the weights of a few N tiles and x streams through.
+  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3, nt = j / n_mtiles * 8 + xcd;
+  if (nt >= n_ntiles) return;
+  const int64_t row0 = (int64_t)(j % n_mtiles) * BM;
+  const int rows = a.M - row0 < BM ? (int)(a.M - row0) : BM;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   if constexpr (MS > 1) {
     if (rows <= 32) {
       typedef Ring<BITS, 1, NT, WN, 2> Short;
       constexpr int S1 = (lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES) / KW - WN * Short::WINDOW) / Short::STAGE;  // as many stages as fit
-      multiply_tile<DT, BITS, G32, LIST, GLU, false, 1, NT, WN, KW, S1>(a, e, row0, rows, nt * NI, scale_shift, lds_raw);
+      multiply_tile<DT, BITS, G32, false, false, false, 1, NT, WN, KW, S1>(a, 0, row0, rows, nt * NI, scale_shift, lds_raw);
       return;
     }
   }
-  multiply_tile<DT, BITS, G32, LIST, GLU, false, MS, NT, WN, KW, S>(a, e, row0, rows, nt * NI, scale_shift, lds_raw);
+  multiply_tile<DT, BITS, G32, false, false, false, MS, NT, WN, KW, S>(a, 0, row0, rows, nt * NI, scale_shift, lds_raw);
 }
 
 size_t codes_copy_bytes(int bits, int64_t rows, int K) {
@@ -1011,36 +995,36 @@ PrepareArgs prepare_args(const void *x, int64_t rows, int K, int group, uint16_t
   a.copy = copy;
   a.sums = sums;
   a.sums_row = padded_groups(K / group) * sum_slots(plain);
-  a.plain = plain;
+  a.slots = sum_slots(plain);
   return a;
 }
-hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, uint16_t *copy,
+hipError_t launch_prepare_rows(const void *x, int64_t rows, int K, int group, int dt, bool list, uint16_t *copy,
                                uint16_t *sums, hipStream_t st) {
   const PrepareArgs a = prepare_args(x, rows, K, group, copy, sums, false);
   if (a.octets == 0) return hipSuccess;
   const unsigned grid = (unsigned)((a.octets + 255) / 256);
-  if (dt == 0) prepare_rows_kernel<0><<<grid, 256, 0, st>>>(a);
-  else if (dt == 1) prepare_rows_kernel<1><<<grid, 256, 0, st>>>(a);
+  if (dt == 0 && list) prepare_rows_kernel<0, RowOrder::kQuads><<<grid, 256, 0, st>>>(a);
+  else if (dt == 0) prepare_rows_kernel<0, RowOrder::kPaired><<<grid, 256, 0, st>>>(a);
+  else if (dt == 1 && !list) prepare_rows_kernel<1, RowOrder::kPaired><<<grid, 256, 0, st>>>(a);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
-template <int DT, int BITS, bool G32, bool LIST, bool GLU, int MS, int NT, int WN, int KW, int S>
-static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_t *list, int cap, hipStream_t st) {
-  constexpr int NI = 32 * WN * (GLU ? 1 : NT), BM = 32 * MS;
+template <int DT, int BITS, bool G32, int MS, int NT, int WN, int KW, int S>
+static hipError_t start_tiles(const CodesArgs &a, int scale_shift, hipStream_t st) {
+  constexpr int NI = 32 * WN * NT, BM = 32 * MS;
   constexpr int bufs = lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES), sums = KW > 1 ? BM * 32 * WN * NT * 4 : 0;
   constexpr int lds = bufs > sums ? bufs : sums;
   static_assert(lds <= 160 * 1024, "more LDS than a CU has");
-  const int n_ntiles = (a.N + NI - 1) / NI;
-  const int mtiles = LIST ? cap : (int)((a.M + BM - 1) / BM);
-  const int64_t grid = LIST ? ((int64_t)cap + 7) / 8 * 8 * n_ntiles : (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
+  const int n_ntiles = (a.N + NI - 1) / NI, mtiles = (int)((a.M + BM - 1) / BM);
+  const int64_t grid = (int64_t)((n_ntiles + 7) / 8) * 8 * mtiles;
   if (grid <= 0 || grid > INT32_MAX) return hipErrorInvalidValue;
-  const auto kernel = &qmm_tiles_kernel<DT, BITS, G32, LIST, GLU, MS, NT, WN, KW, S>;
+  const auto kernel = &qmm_tiles_kernel<DT, BITS, G32, MS, NT, WN, KW, S>;
   if (lds > 64 * 1024) {
     static std::atomic<uint64_t> allowed{0};
     if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), (int)lds, allowed); e != hipSuccess) return e;
   }
-  launch_or_time(kernel, dim3((unsigned)grid), dim3(64 * WN * KW), lds, st, a, list, mtiles, n_ntiles, scale_shift);
+  launch_or_time(kernel, dim3((unsigned)grid), dim3(64 * WN * KW), lds, st, a, mtiles, n_ntiles, scale_shift);
   return hipGetLastError();
 }
 
@@ -1059,16 +1043,16 @@ static hipError_t start_tiles(const CodesArgs &a, int scale_shift, const uint32_
 template <int DT, int BITS, bool G32>
 static hipError_t start_dense(const CodesArgs &a, int group, hipStream_t st) {
   const int scale_shift = group == 128, longer = long_tile_rows(a.M, a.N, a.K, BITS);
-  if (longer == 96) return start_tiles<DT, BITS, G32, false, false, 3, 1, 4, 2, BITS == 4 ? 2 : 3>(a, scale_shift, nullptr, 0, st);
+  if (longer == 96) return start_tiles<DT, BITS, G32, 3, 1, 4, 2, BITS == 4 ? 2 : 3>(a, scale_shift, st);
   if constexpr (BITS == 8)
-    if (longer == 128) return start_tiles<DT, BITS, G32, false, false, 4, 1, 4, 2, 3>(a, scale_shift, nullptr, 0, st);
+    if (longer == 128) return start_tiles<DT, BITS, G32, 4, 1, 4, 2, 3>(a, scale_shift, st);
   switch (dense_tile(a.M, a.N, a.K, BITS, group, DT == 0)) {
-    case DenseTile::k32x64: return start_tiles<DT, BITS, G32, false, false, 1, 1, 2, 4, 2>(a, scale_shift, nullptr, 0, st);
+    case DenseTile::k32x64: return start_tiles<DT, BITS, G32, 1, 1, 2, 4, 2>(a, scale_shift, st);
     case DenseTile::kRegisters32x64: return launch_qmm_codes_small(a, st);
     case DenseTile::k32x128:
-      if constexpr (BITS == 4) return start_tiles<DT, BITS, G32, false, false, 1, 1, 4, 4, 2>(a, scale_shift, nullptr, 0, st);
+      if constexpr (BITS == 4) return start_tiles<DT, BITS, G32, 1, 1, 4, 4, 2>(a, scale_shift, st);
       break;
-    case DenseTile::k64x256: return start_tiles<DT, BITS, G32, false, false, 2, 2, 4, BITS == 4 ? 2 : 1, 2>(a, scale_shift, nullptr, 0, st);
+    case DenseTile::k64x256: return start_tiles<DT, BITS, G32, 2, 2, 4, BITS == 4 ? 2 : 1, 2>(a, scale_shift, st);
     case DenseTile::kRegisters64x128: return launch_qmm_codes_middle(a, false, group, BITS, DT, st);
     case DenseTile::kRegisters64x128Shared: return launch_qmm_codes_middle(a, true, group, BITS, DT, st);
   }
@@ -1090,26 +1074,6 @@ static hipError_t start_pieces(const CodesArgs &a, const uint32_t *list, int cap
 }
 hipError_t launch_qmm_pieces(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st) {
   return glu ? start_pieces<true>(a, list, cap, st) : start_pieces<false>(a, list, cap, st);
-}
-
-// The tiles of a list in one launch: 64 rows x 256 weight rows (128 gate and the matching 128 up ones), two blocks a CU.
-// Groups of 32, 512 tokens and even routing (128 experts, hidden 2048), us of gate/up / down: 107 / 57; tiles of 64 x 128 with the codes loaded into
-// registers, gate and up in one wave, 121 / 77.  One tile a wave in eight waves: 20 % slower; blocks of two waves, or of one CU each with more stages: slower.
-hipError_t launch_qmm_codes_tiles(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st) {
-  auto run = [&](auto b, auto g32) {
-    constexpr int BITS = decltype(b)::value;
-    constexpr bool G32 = decltype(g32)::value;
-    if (glu) return start_tiles<0, BITS, G32, true, true, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
-    return start_tiles<0, BITS, G32, true, false, 2, 2, 4, 1, 2>(a, group == 128, list, cap, st);
-  };
-  const std::true_type yes{};
-  const std::false_type no{};
-  if (bits == 4) {
-    const std::integral_constant<int, 4> b{};
-    return group == 32 ? run(b, yes) : run(b, no);
-  }
-  const std::integral_constant<int, 8> b{};
-  return group == 32 ? run(b, yes) : run(b, no);
 }
 
 hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int dt, hipStream_t st) {
