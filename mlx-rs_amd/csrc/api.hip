@@ -204,9 +204,20 @@ int piece_rows(int64_t pairs, int n_experts) { return short_pieces(pairs, n_expe
 // in pieces as in the middle range, streamed / not, even and Zipf-1.1 at 1600 / 2048 / 3000 / 4096 / 8192 tokens (hidden 2048): 232, 282, 371, 473, 860 and 281, 303,
 // 400, 479, 851 / 227, 278, 367, 469, 855 and 261, 289, 377, 475, 842; hidden 4096, Zipf-1.3, 4096 and 8192 tokens 1635, 2923 / 1619, 2900.  So the line at 96 rows
 // an expert is where the 256-column tiles used to begin, and no longer where either side is the faster one.
+// 8-bit codes: pieces of up to 128 rows on dequantised weights (qmm_bytes.hip) for the segments of seventeen rows and more, the others streamed.  Us of a forward, the other
+// route (tiles of 256 weight rows in three classes on two to four streams) / this, (experts, k, hidden, intermediate):
+//   8, 2, 4096, 14336  even at 70 / 100 / 160 / 256 / 400 / 700 / 1400 / 2048 tokens 578, 573, 591, 734, 696, 940, 1430, 1788 / 532, 418, 456, 519, 587, 810, 1285, 1741;
+//                      Zipf-1.1 at 100 / 300 / 1000 572, 810, 1161 / 544, 595, 988
+//   128, 8, 2048, 768  even at 300 / 512 / 1024 / 2048 / 2500 / 3200 / 4096 tokens 259, 251, 299, 398, 457, 447, 534 / 207, 189, 226, 349, 419, 455, 541; Zipf-1.1 at 400 / 1024 /
+//                      4096 209, 276, 549 / 163, 238, 529
+//   64, 6, 2048, 1408  even at 400 / 1400 / 2000 232, 372, 381 / 181, 320, 398; Zipf-1.1 at 1400 / 2400 400, 486 / 326, 438
+//   16, 4, 4096, 6400  even at 100 / 400 459, 565 / 374, 469
+// Rows of 2048 values are short enough for a block's ends to weigh, and with even routing and 180 rows an expert and more the other route's blocks have fewer of them:
+// there it stays, up to rows of 4096.
 bool piece_batch(const mi_moe_config &c, int64_t T, bool heavy) {
   const int64_t P = T * c.top_k;
-  return heavy && c.bits == 4 && T > kFusedRouterMaxTokens && P >= 512 && c.n_experts >= 8 && codes_tiles_fit(c, T);
+  if (!heavy || T <= kFusedRouterMaxTokens || c.n_experts < 8 || !codes_tiles_fit(c, T)) return false;
+  return c.bits == 4 ? P >= 512 : c.hidden >= 4096 || P < (int64_t)176 * c.n_experts;
 }
 
 // norm: the normalised rows of the residual variant are kept as long as their segments stream.
@@ -273,7 +284,8 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
     f.raw_piece = kPieceM;  // (more rows an expert than the middle range has: piece_rows' last)
     f.raw_cap = short_list_cap(P, c.n_experts, f.raw_from, f.raw_piece);
     // (as above; nothing reads the 256-column tiles' lists, and where there is no norm the place of its rows is free)
-    const size_t list = short_list_words(f.raw_cap), xsums = codes_sums_bytes(T, c.hidden, c.group_size, true), hsums = codes_sums_bytes(P, c.intermediate, c.group_size, true);
+    const size_t list = short_list_words(f.raw_cap);
+    const size_t xsums = c.bits == 4 ? codes_sums_bytes(T, c.hidden, c.group_size, true) : 0, hsums = c.bits == 4 ? codes_sums_bytes(P, c.intermediate, c.group_size, true) : 0;
     const bool in_norm = !norm && xsums + hsums <= (size_t)T * c.hidden * 2;
     f.raw_tiles = list <= tile_list_words(f.max_mtiles, c.n_experts) ? f.mtiles : cv.take<uint32_t>(list);
     f.raw_copy = f.xperm;
@@ -584,7 +596,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     }
     MI_HIP(launch_dispatch(f.topk_idx, P, c.n_experts, c.top_k, f.counts, f.offsets, f.perm, f.inv_perm,
                            f.src_of, records, tile_lists, tile_cap, tile_from, shorts,
-                           raw_codes || f.raw_all ? prepare_args(x, T, c.hidden, c.group_size, codes_copy_bytes(c.bits, T, c.hidden) ? f.raw_copy : nullptr, f.raw_xsums, raw_codes)
+                           (raw_codes && c.bits == 4) || f.raw_all ? prepare_args(x, T, c.hidden, c.group_size, codes_copy_bytes(c.bits, T, c.hidden) ? f.raw_copy : nullptr, f.raw_xsums, raw_codes)
                                                   : PrepareArgs{}, f.disp_scratch, st));
     MI_STAGE_DONE();
   }
@@ -619,10 +631,12 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   cd.y = f.y;
   cd.N = c.hidden; cd.K = c.intermediate;
   auto tiles_up = [&](hipStream_t s) -> hipError_t {
+    if (f.pieces && c.bits == 8) return launch_qmm_bytes(ca, f.raw_tiles, f.raw_cap, true, s);
     if (f.raw_piece > kShortTileM) return launch_qmm_pieces(ca, f.raw_tiles, f.raw_cap, true, s);
     return launch_qmm_short(ca, f.raw_tiles, f.raw_cap, c.group_size, c.bits, true, s);
   };
   auto tiles_down = [&](hipStream_t s) -> hipError_t {
+    if (f.pieces && c.bits == 8) return launch_qmm_bytes(cd, f.raw_tiles, f.raw_cap, false, s);
     if (f.raw_piece > kShortTileM) return launch_qmm_pieces(cd, f.raw_tiles, f.raw_cap, false, s);
     return launch_qmm_short(cd, f.raw_tiles, f.raw_cap, c.group_size, c.bits, false, s);
   };
@@ -1481,7 +1495,7 @@ int mi_moe_debug_tile_rule(const mi_moe_config *cfg, int64_t T, int32_t *tiled, 
   if (check_config(cfg)) return 1;
   if (T < 0 || T * cfg->top_k > (int64_t)1 << 30) return fail("debug_tile_rule: token count out of range");
   const ForwardWs f = carve_forward(*cfg, T, nullptr, true);
-  if (tiled) *tiled = f.mid ? 2 : f.pieces ? 3 : f.tiled ? 1 : 0;
+  if (tiled) *tiled = f.mid ? 2 : f.pieces && cfg->bits == 4 ? 3 : f.tiled ? 1 : 0;
   if (tile_min_rows) *tile_min_rows = f.mid ? 1 : f.tmr;
   return 0;
 } MI_CATCH("debug_tile_rule")

@@ -428,6 +428,8 @@ hipError_t launch_qmm_codes_dense(const CodesArgs &a, int group, int bits, int d
 // A list of pieces of up to 64 rows (ShortTiles::piece), bf16; 4-bit codes in groups of 64 also of 96 or 128
 hipError_t launch_qmm_short(const CodesArgs &a, const uint32_t *list, int cap, int group, int bits, bool glu, hipStream_t st);
 hipError_t launch_qmm_pieces(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
+// 8-bit codes in groups of 64, up to 128 rows: weights dequantised (no group sums)
+hipError_t launch_qmm_bytes(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st);
 hipError_t launch_quantize(const float *w, int64_t rows, int64_t cols, int group, int bits,
                            uint32_t *q, void *s, void *b, int dt, hipStream_t st);
 hipError_t launch_dequantize(const uint32_t *q, const void *s, const void *b,

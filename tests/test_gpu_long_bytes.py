@@ -1,0 +1,48 @@
+"""Pieces of up to 128 rows with 8-bit codes in groups of 64, against float64."""
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+from test_gpu_codes import block_truth  # noqa: E402
+from test_gpu_short_pieces import chosen_block  # noqa: E402
+
+EDGES = [0, 1, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 145, 257]  # both sides of every length at which another kernel, body or piece begins
+
+
+# K of 1, 2, 3, 8, 9 and 17 times 128 values: windows of 512 whole and started; 18 experts and few columns: K shared by two groups of waves where it is whole 256s,
+# many columns: one group; output columns that fill no block of 256
+@pytest.mark.parametrize("hidden,inter,experts", [(128, 384, 18), (384, 128, 18), (256, 512, 18), (1024, 1152, 18), (1152, 1024, 18), (2176, 256, 36), (256, 2176, 36), (768, 768, 90)])
+def test_lengths_around_every_body_b(hidden, inter, experts):
+    """Roundings to bfloat16 of the weights of three products, h, y and the result, each typically 0.42 * 2^-8 of its values: 1.03 * 2^-8 together; a row's bound is twice
+    that.  Rows do not depend on their order in the batch."""
+    blk, x, of = chosen_block(hidden, inter, EDGES, experts, 8, 64)
+    out, routing = blk.forward(x, debug=True)
+    assert torch.equal(routing["topk_idx"][:, 0].long(), of)
+    ref = block_truth(blk, x, routing)
+    err = (out.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= 2.06 * 2.0 ** -8, float(err.max())
+    order = torch.randperm(len(of), generator=torch.Generator().manual_seed(3)).cuda()
+    assert torch.equal(blk.forward(x[order].contiguous()), out[order])
+
+
+@pytest.mark.parametrize("tokens,zipf", [(150, 1.0), (400, None)])
+def test_infinities_of_long_pieces(tokens, zipf):
+    """Infinite biases of each matrix and rows that are not finite."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(256, 16, 6, 384, 8, 64, 0)
+    blk = synth.make_block(cfg, seed=2, device="cuda", zipf_s=zipf, gen_device="cuda")
+    x = synth.make_tokens(cfg, tokens, seed=1, device="cuda")
+    blk.gate_proj.biases[1, 5, 1] = float("inf")
+    blk.up_proj.biases[2, 7, 0] = float("-inf")
+    blk.down_proj.biases[3, 9, 1] = float("inf")
+    x[7, 3] = float("inf")
+    x[11, 200] = float("nan")
+    blk.gate_weight[:, 3] = blk.gate_weight[:, 200] = 0.0
+    finite = torch.ones(tokens, dtype=torch.bool, device="cuda")
+    finite[[7, 11]] = False  # (the routing of these is no number's)
+    out, routing = blk.forward(x, debug=True)
+    ref = block_truth(blk, x, routing)
+    assert not ref[finite].isfinite().all()
+    assert torch.equal(out[finite].isnan(), ref[finite].isnan()) and torch.equal(out[finite].isinf(), ref[finite].isinf())

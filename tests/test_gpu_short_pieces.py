@@ -10,7 +10,7 @@ from test_gpu_short_tiles import share_off_nearest  # noqa: E402
 EDGES = [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65]  # lengths on both sides of every one at which another body or another piece begins
 
 
-def chosen(hidden, inter, lengths, experts, bits=4, group=64):
+def chosen_block(hidden, inter, lengths, experts, bits, group):
     """A block whose expert e gets lengths[e % len(lengths)] tokens: the expert's column of a token is large, and the router is the unit matrix."""
     import mlx_rs_amd as m
     from mlx_rs_amd import synth
@@ -19,10 +19,17 @@ def chosen(hidden, inter, lengths, experts, bits=4, group=64):
     blk.gate_weight.copy_(torch.eye(hidden)[:experts])
     of = torch.cat([torch.full((lengths[e % len(lengths)],), e) for e in range(experts)]).cuda()
     tokens = of.numel()
-    assert max(512, 6 * experts) <= tokens < 60 * experts and (group != 64 or m.capi.tile_rule(cfg.c_struct(), tokens) == (2, 1))
     of = of[torch.randperm(tokens, generator=torch.Generator().manual_seed(1)).cuda()]
     x = synth.make_tokens(cfg, tokens, seed=4, device="cuda")
     x[torch.arange(tokens, device="cuda"), of] = 16.0
+    return blk, x, of
+
+
+def chosen(hidden, inter, lengths, experts, bits=4, group=64):
+    import mlx_rs_amd as m
+    blk, x, of = chosen_block(hidden, inter, lengths, experts, bits, group)
+    tokens = of.numel()
+    assert max(512, 6 * experts) <= tokens < 60 * experts and (group != 64 or m.capi.tile_rule(blk.config.c_struct(), tokens) == (2, 1))
     return blk, x, of
 
 
