@@ -22,7 +22,7 @@ __device__ __forceinline__ void copy_to_lds(i32x4_t rsrc, uint32_t voff, uint32_
 }
 // The same by lanes 0 to 31, where all lanes are active: no branch, in which the compiler may hold a scalar operand in a vector register.
 __device__ __forceinline__ void copy_half_to_lds(i32x4_t rsrc, uint32_t voff, uint32_t soff, uint32_t to) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_hi, 0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\ts_mov_b32 exec_hi, -1" ::"s"(to), "v"(voff), "s"(rsrc), "s"(soff) : "m0", "memory");
+  asm volatile("s_mov_b32 exec_hi, 0\n\ts_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\ts_mov_b32 exec_hi, -1" ::"s"(to), "v"(voff), "s"(rsrc), "s"(soff) : "m0", "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_copies() {  // all but the last N have arrived; LDS reads are done
