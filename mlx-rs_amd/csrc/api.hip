@@ -162,6 +162,19 @@ bool codes_tiles_fit(const mi_moe_config &c, int64_t T) {
 bool raw_list_batch(const mi_moe_config &c, int64_t T) {
   return T > kRowsMost && T * c.top_k >= (int64_t)4 * c.n_experts && codes_tiles_fit(c, T);
 }
+// Groups of 64, 8-bit codes: the same for batches of a few rows an expert, where a popular expert's segment is many passes of the streaming kernel and a tile of 256
+// weight rows mostly padding.  Us of a forward, other route (streamed; pieces on dequantised weights from 17 rows an expert on) / this, (experts, k, hidden, intermediate):
+//   128, 8, 2048, 768  even at 64 / 80 / 150 / 200 / 300 tokens 153, 164, 179, 213, 196 / 156, 157, 161, 165, 164; Zipf-1.1 at 64 / 100 / 200 160, 232, 443 / 90, 101, 113
+//   64, 6, 2048, 1408  even at 60 / 100 / 200 148, 170, 191 / 139, 143, 151; 16, 4, 4096, 6400 at 30 / 50 / 100 415, 499, 375 / 345, 352, 367, Zipf-1.1 at 50 524 / 347
+//   8, 2, 4096, 14336  even at 32 / 40 / 48 / 56 / 64 / 80 / 100 / 130 tokens 350, 378, 362 to 399, 474, 500, 538, 463, 436 / 400, 405, 404, 406, 409, 426, 427, 434; Zipf-1.1 at 40 / 64 / 100
+//                      475, 615, 520 / 412, 420, 571
+// With fewer blocks in the down product than CUs its blocks are what a forward waits for, whatever their rows, and streaming stays ahead up to some thirteen rows.  At 25 and 32 rows
+// an expert 128 experts would still gain (400 / 512 tokens 206, 189 / 167, 174, skewed 163 / 153) and eight skewed ones lose (above); from 24 on the launch plan of 8-bit
+// batches holds streamed segments beside tiles, as its callers know it.
+bool mid_bytes_batch(const mi_moe_config &c, int64_t T) {
+  const int64_t P = T * c.top_k, E = c.n_experts, least = E * (c.hidden / 256) >= 256 ? 6 : 14;
+  return c.bits == 8 && c.group_size == 64 && E >= 8 && P >= least * E && P < 24 * E && codes_tiles_fit(c, T);
+}
 // Groups of 64, 4-bit codes: batches whose segments all go through pieces on raw codes, in one launch a product on the caller's
 // stream (the others: streamed segments, and tiles of 256 weight rows on side streams).  From the batches on for which the tile lists
 // are built and the router has kernels of its own, up to 96 rows per expert on average (beyond: piece_batch).  Measured when pieces had 64 rows, in the experts' order, us
@@ -179,6 +192,7 @@ bool raw_list_batch(const mi_moe_config &c, int64_t T) {
 // these tiles are faster there as well (144 to 504 pairs, 4 to 16 experts: 1.08 to 2.1 times).
 bool mid_batch(const mi_moe_config &c, int64_t T, bool tiled) {
   const int64_t P = T * c.top_k;
+  if (c.bits == 8) return mid_bytes_batch(c, T);
   return tiled && c.bits == 4 && T > kFusedRouterMaxTokens && P <= (int64_t)96 * c.n_experts && P >= 512 && c.n_experts >= 8 && codes_tiles_fit(c, T);
 }
 
@@ -266,7 +280,12 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
   f.bytes_min = cv.off;
   f.mid = mid_batch(c, T, f.tiled);
   f.pieces = !f.mid && piece_batch(c, T, f.heavy);
-  if (f.mid) {
+  if (f.mid && c.bits == 8) {
+    f.raw_cap = short_list_cap(P, c.n_experts, 1, f.raw_piece);
+    f.raw_tiles = cv.take<uint32_t>(short_list_words(f.raw_cap));
+    f.raw_xsums = cv.take<uint16_t>(codes_sums_bytes(T, c.hidden, c.group_size) / 2);
+    f.raw_hsums = cv.take<uint16_t>(codes_sums_bytes(P, c.intermediate, c.group_size) / 2);
+  } else if (f.mid) {
     // All of it lies in memory that is free at the time where it fits, so that batches which have to fit a scratch of a given size take
     // this route as well: the list in place of the work records (nothing is streamed), the group sums of x where the down product writes
     // its rows later, those of h in the normalised rows, which only the router and the copy of x read.
@@ -548,7 +567,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   uint32_t *const tile_lists = f.tiled && !raw_codes ? f.mtiles : nullptr;
   const int tile_cap = f.max_mtiles, tile_from = f.tmr;
   const ShortTiles shorts = {raw_codes || f.raw ? f.raw_tiles : nullptr, (uint32_t)f.raw_from, (uint32_t)f.raw_piece};
-  uint32_t *const records = mid ? nullptr : f.work;
+  uint32_t *const records = mid && !fused_router ? nullptr : f.work;
   if (norm_weight) {  // the block's input is rms_norm(x); x itself is added back in the combine
     if (!fused_router) MI_HIP(launch_rms_norm(x_in, norm_weight, eps, T, c.hidden, f.xnorm, st));
     x = f.xnorm;      // decode: written by the router kernel below
@@ -596,8 +615,9 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     }
     MI_HIP(launch_dispatch(f.topk_idx, P, c.n_experts, c.top_k, f.counts, f.offsets, f.perm, f.inv_perm,
                            f.src_of, records, tile_lists, tile_cap, tile_from, shorts,
-                           (raw_codes && c.bits == 4) || f.raw_all ? prepare_args(x, T, c.hidden, c.group_size, codes_copy_bytes(c.bits, T, c.hidden) ? f.raw_copy : nullptr, f.raw_xsums, raw_codes)
-                                                  : PrepareArgs{}, f.disp_scratch, st));
+                           mid || f.raw_all || (f.pieces && c.bits == 4)
+                               ? prepare_args(x, T, c.hidden, c.group_size, codes_copy_bytes(c.bits, T, c.hidden) ? f.raw_copy : nullptr, f.raw_xsums, raw_codes && c.bits == 4)
+                               : PrepareArgs{}, f.disp_scratch, st));
     MI_STAGE_DONE();
   }
   GroupedArgs a{}, d{};
@@ -645,6 +665,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
     ~TimerScope() { g_kernel_timer = nullptr; }
   };
   if (mid) {
+    if (fused_router) MI_HIP(launch_prepare_rows(x, T, c.hidden, c.group_size, MI_MOE_DTYPE_BF16, true, nullptr, f.raw_xsums, st));  // (8-bit codes: no copy)
     {
       TimerScope scope(kt ? &kt[2] : nullptr);
       MI_HIP(tiles_up(st));

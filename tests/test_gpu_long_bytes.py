@@ -46,3 +46,49 @@ def test_infinities_of_long_pieces(tokens, zipf):
     ref = block_truth(blk, x, routing)
     assert not ref[finite].isfinite().all()
     assert torch.equal(out[finite].isnan(), ref[finite].isnan()) and torch.equal(out[finite].isinf(), ref[finite].isinf())
+
+
+FEW = [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65] + 10 * [0]  # twenty rows an expert on average
+
+
+@pytest.mark.parametrize("hidden,inter", [(128, 384), (384, 128), (1024, 1152), (1152, 1024), (2176, 256), (256, 2176)])
+def test_all_segments_of_a_few_rows_in_pieces(hidden, inter):
+    """From fourteen to 24 rows an expert (six where the down product has a block for every CU): raw codes, so three roundings to bfloat16 (h, y and the result), each typically 0.42 * 2^-8 of its values: 0.73 * 2^-8 together; a
+    row's bound is twice that."""
+    import mlx_rs_amd as m
+    blk, x, of = chosen_block(hidden, inter, FEW, 24, 8, 64)
+    assert m.capi.tile_rule(blk.config.c_struct(), len(of)) == (2, 1)
+    out, routing = blk.forward(x, debug=True)
+    assert torch.equal(routing["topk_idx"][:, 0].long(), of)
+    ref = block_truth(blk, x, routing)
+    err = (out.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= 1.5 * 2.0 ** -8, float(err.max())
+    order = torch.randperm(len(of), generator=torch.Generator().manual_seed(3)).cuda()
+    assert torch.equal(blk.forward(x[order].contiguous()), out[order])
+
+
+@pytest.mark.parametrize("tokens", [57, 64, 65])
+@pytest.mark.parametrize("residual", [False, True])
+def test_few_rows_behind_either_router(tokens, residual):
+    """Up to 64 tokens the router is one launch and the rows are prepared behind it; the same bits with a workspace that a larger batch has left."""
+    import mlx_rs_amd as m
+    from mlx_rs_amd import synth
+    cfg = m.MoeConfig(512, 8, 2, 384, 8, 64, 0)
+    assert m.capi.tile_rule(cfg.c_struct(), tokens) == (2, 1)
+    blk = synth.make_block(cfg, seed=6, device="cuda", zipf_s=1.1, gen_device="cuda")
+    x = synth.make_tokens(cfg, tokens, seed=6, device="cuda")
+    if residual:
+        w = torch.ones(512, dtype=torch.bfloat16, device="cuda")
+        out = blk.forward_residual(x, w, 1e-6)
+        blk.forward_residual(synth.make_tokens(cfg, 700, seed=7, device="cuda"), w, 1e-6)
+        assert torch.equal(blk.forward_residual(x, w, 1e-6), out)
+        n = m.ops.rms_norm(x, w, 1e-6)
+        got, ref = out.double(), x.double() + blk.forward(n).double()
+        assert float((got - ref).norm() / ref.norm()) <= 2.0 ** -8  # (one rounding for two)
+    else:
+        out, routing = blk.forward(x, debug=True)
+        blk.forward(synth.make_tokens(cfg, 700, seed=7, device="cuda"))
+        assert torch.equal(blk.forward(x), out)
+        ref = block_truth(blk, x, routing)
+        err = (out.double() - ref).norm(dim=1) / ref.norm(dim=1)
+        assert float(err.max()) <= 1.5 * 2.0 ** -8, float(err.max())
