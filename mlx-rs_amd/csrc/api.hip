@@ -120,6 +120,7 @@ struct ForwardWs {
   uint32_t *topk_idx;
   uint16_t *topk_w;
   uint32_t *counts, *offsets, *work, *mtiles, *perm, *inv_perm, *src_of;
+  Records records;  // the streamed segments', in `work` or (split) in a place of their own
   int max_mtiles;
   bool tiled;  // tile lists are built
   bool heavy;  // most rows are tiled: see heavy_batch()
@@ -312,6 +313,18 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
     f.raw_hsums = in_norm ? f.xnorm + xsums / 2 : cv.take<uint16_t>(hsums / 2);
   }
   f.raw_all = f.raw && raw_list_batch(c, T);
+  // Where everything streams, or goes through the kernel of a few rows, a segment of several passes is as many records, whose blocks run beside each other: with skewed
+  // routing one block would go over a popular expert's weights pass after pass, long after the others are done.  Us of a forward, a record a segment / a pass (same bits):
+  //   128, 8, 2048, 768, 4 bits  Zipf-1.1 at 16 / 24 / 32 / 48 / 64 / 80 / 95 tokens 63, 81, 82, 116, 141, 176, 201 / 50, 57, 52, 68, 73, 88, 94; 1.3 at 32 / 95 82, 203 / 48, 89; even
+  //                              at 16 / 32 / 64 / 95 65, 83, 97, 120 / 64, 83, 95, 114
+  //   128, 8, 4096, 1536, 4 bits Zipf-1.3 at 24 / 64 / 95 221, 374, 527 / 155, 234, 303; 64, 6, 2048, 1408, 4 bits, Zipf-1.1 at 40 102 / 67
+  //   128, 8, 2048, 768, 8 bits  Zipf-1.1 at 64 159 / 93; 8, 2, 4096, 14336, 8 bits at 32 / 48 416, 533 / 348, 457
+  f.records = Records(f.work);
+  const bool rows_kernel = f.raw && !f.raw_all, streams = !plain_config(c) && !f.tiled && !f.mid;
+  if (const int log2 = c.bits == 4 && streams ? 3 : 4; (streams || rows_kernel) && T > 1 << log2) {  // (rows of a pass)
+    const int64_t most = P < c.n_experts ? P : c.n_experts, slots = most + ((P - most) >> log2);
+    f.records = Records(cv.take<uint32_t>((size_t)slots * 16), log2, (int)slots);
+  }
   if (f.raw_all) {
     f.raw_cap = short_list_cap(P, c.n_experts, f.raw_from, f.raw_piece);
     f.raw_tiles = cv.take<uint32_t>(short_list_words(f.raw_cap));
@@ -489,8 +502,9 @@ static void grouped_args(const mi_moe_config &c, const mi_moe_weights &w, const 
   const int64_t P = T * c.top_k;
   const bool paired = c.bits == 4;
   a = GroupedArgs{};
-  a.work = f.work;
+  a.work = f.records.at;
   a.max_active = (int)(P < c.n_experts ? P : c.n_experts);
+  a.max_records = f.records.slots;
   const bool lists = f.tiled && !f.pieces;
   a.mtiles = lists ? f.mtiles : nullptr;
   a.max_mtiles = f.max_mtiles;
@@ -554,6 +568,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   if (workspace_bytes < f.bytes_raw) {
     f.raw_tiles = nullptr;
     f.mid = f.pieces = f.raw_all = false;
+    f.records = Records(f.work);
   }
   if (workspace_bytes < f.bytes) f.router_scratch = nullptr;  // room for everything but the byte planes: fp64 logits, same bits
   int stage = 0;
@@ -567,7 +582,7 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   uint32_t *const tile_lists = f.tiled && !raw_codes ? f.mtiles : nullptr;
   const int tile_cap = f.max_mtiles, tile_from = f.tmr;
   const ShortTiles shorts = {raw_codes || f.raw ? f.raw_tiles : nullptr, (uint32_t)f.raw_from, (uint32_t)f.raw_piece};
-  uint32_t *const records = mid && !fused_router ? nullptr : f.work;
+  const Records records = mid && !fused_router ? Records() : f.records;
   if (norm_weight) {  // the block's input is rms_norm(x); x itself is added back in the combine
     if (!fused_router) MI_HIP(launch_rms_norm(x_in, norm_weight, eps, T, c.hidden, f.xnorm, st));
     x = f.xnorm;      // decode: written by the router kernel below
@@ -698,8 +713,9 @@ static int forward_impl(mi_moe_handle h, const uint16_t *x_in, int64_t T, uint16
   } else if (f.raw) {
     // group sizes 32 / 128 without lists: the kernel of a few rows
     RowsArgs ra{}, rd{};
-    ra.work = f.work;
+    ra.work = f.records.at;
     ra.max_active = max_active;
+    ra.max_records = f.records.slots;
     ra.max_rows = T;
     rd = ra;
     ra.x = x;

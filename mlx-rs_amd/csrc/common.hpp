@@ -184,6 +184,12 @@ struct ShortTiles {
   uint32_t from = 1;
   uint32_t piece = kShortTileM;
 };
+// Where the work records of the streamed segments go (dispatch_dev.hpp): a segment in records of at most 2^log2 rows, `slots` of them (0: as many as experts).
+struct Records {
+  uint32_t *at;
+  int log2, slots;
+  __host__ __device__ Records(uint32_t *p = nullptr, int l = 31, int n = 0) : at(p), log2(l), slots(n) {}
+};
 __host__ __device__ inline size_t short_list_words(int cap) { return 4 + 4 * (size_t)cap; }
 inline int short_list_cap(int64_t pairs, int n_experts, int from, int piece) {  // full pieces, and a segment's last one
   return (int)(pairs / piece + (pairs / from < n_experts ? pairs / from : n_experts));
@@ -273,7 +279,8 @@ struct GroupedArgs {
   bool src_in_work;         // the records' inline source rows equal src_rows (saves a dependent load)
   const uint32_t *dst_rows; // output row of sorted row r, or nullptr = r
   const uint32_t *work;        // 16-word records {expert, first row, rows, has_src, src[12]}, count 0 = end
-  int max_active;              // upper bound of the number of records known on the host
+  int max_active;              // upper bound of the number of segments known on the host
+  int max_records;             // and of records, where segments are split over several (0: max_active)
   const uint32_t *mtiles;      // M-tile lists (tiled MFMA kernel), or nullptr
   int max_mtiles;              // capacity of the 256-row list
   int tile_cap_e;              // capacity of the 128- and 64-row lists (the number of experts)
@@ -312,7 +319,7 @@ size_t dispatch_workspace_least(int E, int64_t P);
 struct PrepareArgs;
 hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, uint32_t *counts,
                            uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
-                           uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, int big_thr,
+                           uint32_t *src_of, Records work, uint32_t *mtiles, int cap256, int big_thr,
                            ShortTiles shorts, const PrepareArgs &prepare, void *scratch, hipStream_t st);
 // The order of the values of every 8-block of a row of activations: as they are; (0,4)(1,5)(2,6)(3,7), which one and-or a register unpacks 4-bit codes to;
 // (0,2)(1,3)(4,6)(5,7), which is how a conversion of two bytes a register leaves them.
@@ -340,7 +347,7 @@ hipError_t launch_router_fused(const uint16_t *x, const uint16_t *wg, const floa
                                int H, int E, int k, int mode, uint16_t *logits, uint32_t *topk_idx,
                                uint16_t *topk_w, uint32_t *counters, uint32_t *counts,
                                uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
-                               uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256,
+                               uint32_t *src_of, Records work, uint32_t *mtiles, int cap256,
                                int big_thr, ShortTiles shorts, hipStream_t st);
 hipError_t launch_grouped_qmm(const GroupedArgs &a, bool glu, hipStream_t st);
 hipError_t launch_large_qmm(const GroupedArgs &a, bool glu, hipStream_t st);
@@ -394,8 +401,8 @@ struct RowsArgs {
   const void *x;
   const uint32_t *src_rows, *dst_rows, *work;  // as in GroupedArgs
   bool src_in_work;
-  int max_active;
-  int64_t max_rows;  // of a record, at most
+  int max_active, max_records;  // as in GroupedArgs
+  int64_t max_rows;  // of a segment, at most
   const uint32_t *w0, *w1;
   const void *s0, *b0, *s1, *b1;
   const void *bias;  // as in CodesArgs

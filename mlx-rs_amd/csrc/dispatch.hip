@@ -29,7 +29,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_single_kernel(
     const uint32_t *flat, int64_t P, int E, int nbits, int k_div,
     uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets, uint32_t *__restrict__ perm,
     uint32_t *__restrict__ inv_perm, uint32_t *__restrict__ src_of,
-    uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr, ShortTiles shorts, PrepareArgs prepare) {
+    Records work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr, ShortTiles shorts, PrepareArgs prepare) {
   extern __shared__ uint32_t lds[];
   if (prepares(prepare, 1)) return;
   dispatch_block(flat, P, E, nbits, k_div, lds, counts, offsets, perm, inv_perm, src_of, work, mtiles, cap256, big_thr, shorts);
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_hist_kernel(
 __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     const uint32_t *flat, int64_t P, int E, int nbits, int k_div, int64_t span,
     const uint32_t *__restrict__ blockhist, int nb, uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets,
-    uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr, ShortTiles shorts,
+    Records work, uint32_t *__restrict__ mtiles, int cap256, uint32_t big_thr, ShortTiles shorts,
     uint32_t *__restrict__ perm, uint32_t *__restrict__ inv_perm, uint32_t *__restrict__ src_of, PrepareArgs prepare) {
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t n_active, total;
@@ -125,7 +125,7 @@ size_t dispatch_workspace_least(int E, int64_t P) { return P <= kSingleAtMostP ?
 
 hipError_t launch_dispatch(const uint32_t *flat, int64_t P, int E, int k_div, uint32_t *counts,
                            uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
-                           uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, int big_thr,
+                           uint32_t *src_of, Records work, uint32_t *mtiles, int cap256, int big_thr,
                            ShortTiles shorts, const PrepareArgs &prepare, void *scratch, hipStream_t st) {
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;

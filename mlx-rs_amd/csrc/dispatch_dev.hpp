@@ -87,9 +87,9 @@ __device__ __forceinline__ void scatter_range(const uint32_t *flat, int64_t j0, 
 }
 
 // Work records consumed by the grouped products: one 64-byte record per expert that received
-// rows, in ascending expert order, then records with count 0 up to n_experts.
+// rows (or several, see Records), in ascending expert order, then records with count 0 up to the number of slots.
 //   [0] expert id  [1] first sorted row  [2] row count  [3] 1 if [4..15] are filled
-//   [4..15] source row (pair index / k_div) of the first 12 rows of the segment
+//   [4..15] source row (pair index / k_div) of its first 12 rows
 constexpr int kWorkWords = 16;
 constexpr int kWorkSrc = 12;
 
@@ -175,8 +175,9 @@ __device__ __forceinline__ void list_pieces(const uint32_t *first, uint32_t tota
 // counts -> offsets, work records, M tiles and short tiles; runs in one block.  LDS cnt[E] in, cur[E] out.
 __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint32_t *cur, int E,
                               uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets,
-                              uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256,
+                              Records records, uint32_t *__restrict__ mtiles, int cap256,
                               uint32_t big_thr, ShortTiles shorts, uint32_t *n_active_lds) {
+  uint32_t *const __restrict__ work = records.at;
   __shared__ uint32_t total;
   const int tid = threadIdx.x;
   if (tid < E && counts) counts[tid] = cnt[tid];
@@ -201,15 +202,22 @@ __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint
       const bool big = mtiles && big_thr != 0u && c >= big_thr;
       const bool brief = shorts.list && !big && c >= shorts.from;
       const bool small = c != 0u && !big && !brief;
-      const uint64_t bm = __ballot(small);
-      if (small && work) {
-        uint32_t *rec = work + (size_t)(base + __popcll(bm & lanemask_lt())) * kWorkWords;
-        rec[0] = (uint32_t)e;
-        rec[1] = cnt[e];
-        rec[2] = c;
-        rec[3] = 0u;
+      uint32_t upto = small ? ((c - 1u) >> records.log2) + 1u : 0u;  // records of this lane's segment, then up to it
+      const uint32_t own = upto;
+      for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t v = __shfl_up(upto, d, kWave);
+        if (tid >= d) upto += v;
       }
-      base += __popcll(bm);
+      if (work)
+        for (uint32_t i = 0; i < own; ++i) {
+          uint32_t *rec = work + (size_t)(base + upto - own + i) * kWorkWords;
+          const uint32_t first = i << records.log2, left = c - first, most = 1u << records.log2;
+          rec[0] = (uint32_t)e;
+          rec[1] = cnt[e] + first;
+          rec[2] = left < most ? left : most;
+          rec[3] = 0u;
+        }
+      base += __shfl(upto, kWave - 1, kWave);
       // M tiles: exclusive scan of the 256-row tile counts over the wave, ballots for the others
       TileSplit ts = split_segment(big ? c : 0u);
       uint32_t incl = ts.n256;
@@ -241,7 +249,7 @@ __device__ __forceinline__ void finish_counts(uint32_t *cnt, uint32_t *tmp, uint
       t64 += __popcll(b64);
     }
     if (work)
-      for (int sl = base + tid; sl < E; sl += kWave) {
+      for (int sl = base + tid; sl < (records.slots ? records.slots : E); sl += kWave) {
         work[(size_t)sl * kWorkWords + 2] = 0u;
         work[(size_t)sl * kWorkWords + 3] = 0u;
       }
@@ -264,8 +272,9 @@ __device__ __forceinline__ void dispatch_block(const uint32_t *flat, int64_t P, 
                                uint32_t *lds, uint32_t *__restrict__ counts,
                                uint32_t *__restrict__ offsets, uint32_t *__restrict__ perm,
                                uint32_t *__restrict__ inv_perm, uint32_t *__restrict__ src_of,
-                               uint32_t *__restrict__ work, uint32_t *__restrict__ mtiles, int cap256,
+                               Records records, uint32_t *__restrict__ mtiles, int cap256,
                                uint32_t big_thr, ShortTiles shorts) {
+  uint32_t *const __restrict__ work = records.at;
   __shared__ uint32_t n_active;
   uint32_t *cnt = lds, *tmp = lds + E, *cur = lds + 2 * E, *wcnt = lds + 3 * E;
   const int tid = threadIdx.x;
@@ -276,7 +285,7 @@ __device__ __forceinline__ void dispatch_block(const uint32_t *flat, int64_t P, 
     atomicAdd(&cnt[e < (uint32_t)E ? e : (uint32_t)E - 1u], 1u);
   }
   __syncthreads();
-  finish_counts(cnt, tmp, cur, E, counts, offsets, work, mtiles, cap256, big_thr, shorts, &n_active);
+  finish_counts(cnt, tmp, cur, E, counts, offsets, records, mtiles, cap256, big_thr, shorts, &n_active);
   scatter_range(flat, 0, P, E, nbits, k_div, cur, wcnt, perm, inv_perm, src_of);
   // source rows of the first rows of every segment, so that a consumer needs one load
   if (work) {
@@ -308,7 +317,8 @@ template <bool FLAT_LOCAL = false>
 __device__ __forceinline__ void dispatch_tokens_block(const uint32_t *flat, int T, int k, int E, uint32_t *lds,
                                       uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets,
                                       uint32_t *__restrict__ perm, uint32_t *__restrict__ inv_perm,
-                                      uint32_t *__restrict__ src_of, uint32_t *__restrict__ work) {
+                                      uint32_t *__restrict__ src_of, Records records) {
+  uint32_t *const __restrict__ work = records.at;
   uint32_t *const mlo = lds, *const mhi = lds + E, *const off = lds + 2 * E, *const ridx = lds + 3 * E;
   const int tid = threadIdx.x;
   const int P = T * k;
@@ -329,41 +339,44 @@ __device__ __forceinline__ void dispatch_tokens_block(const uint32_t *flat, int 
     }
   }
   __syncthreads();
-  // wave 0: counts, their exclusive scan, one work record per expert with rows (ascending ids)
+  // wave 0: counts and records of the experts (ascending ids), and the exclusive scan of both at once (less than 2^16 each)
   if (tid < kWave) {
     uint32_t base = 0, n_active = 0;
     for (int e0 = 0; e0 < E; e0 += kWave) {
       const int e = e0 + tid;
       const uint32_t c = e < E ? (uint32_t)(__popc(mlo[e]) + __popc(mhi[e])) : 0u;
-      uint32_t incl = c;
+      const uint32_t own = c != 0u ? ((c - 1u) >> records.log2) + 1u : 0u, both = c | own << 16;
+      uint32_t incl = both;
       for (int d = 1; d < kWave; d <<= 1) {
         const uint32_t v = __shfl_up(incl, d, kWave);
         if (tid >= d) incl += v;
       }
-      const uint32_t excl = base + incl - c;
-      const uint64_t bm = __ballot(c != 0u);
+      const uint32_t excl = base + ((incl - both) & 0xffffu);
       if (e < E) {
         off[e] = excl;
         if (counts) counts[e] = c;
         if (offsets) offsets[e] = excl;
         if (c != 0u) {
-          const uint32_t r = n_active + __popcll(bm & lanemask_lt());
+          const uint32_t r = n_active + ((incl - both) >> 16);
           ridx[e] = r;
-          if (work) {
-            uint32_t *rec = work + (size_t)r * kWorkWords;
-            rec[0] = (uint32_t)e;
-            rec[1] = excl;
-            rec[2] = c;
-            rec[3] = 1u;  // the source rows follow below
-          }
+          if (work)
+            for (uint32_t i = 0; i < own; ++i) {
+              uint32_t *rec = work + (size_t)(r + i) * kWorkWords;
+              const uint32_t first = i << records.log2, left = c - first, most = 1u << records.log2;
+              rec[0] = (uint32_t)e;
+              rec[1] = excl + first;
+              rec[2] = left < most ? left : most;
+              rec[3] = 1u;  // the source rows follow below
+            }
         }
       }
-      base += __shfl(incl, kWave - 1, kWave);
-      n_active += __popcll(bm);
+      const uint32_t last = __shfl(incl, kWave - 1, kWave);
+      base += last & 0xffffu;
+      n_active += last >> 16;
     }
     if (tid == 0 && offsets) offsets[E] = base;
     if (work)
-      for (int sl = (int)n_active + tid; sl < E; sl += kWave) {
+      for (int sl = (int)n_active + tid; sl < (records.slots ? records.slots : E); sl += kWave) {
         work[(size_t)sl * kWorkWords + 2] = 0u;
         work[(size_t)sl * kWorkWords + 3] = 0u;
       }
@@ -382,8 +395,9 @@ __device__ __forceinline__ void dispatch_tokens_block(const uint32_t *flat, int 
       perm[pos] = (uint32_t)j;
       if (inv_perm) inv_perm[j] = pos;
       if (src_of) src_of[pos] = t;
-      // source rows of the first rows of every segment, so that a consumer needs one load
-      if (work && below < (uint32_t)kWorkSrc) work[(size_t)ridx[e] * kWorkWords + 4 + below] = t;
+      // source rows of the first rows of every record, so that a consumer needs one load
+      const uint32_t of = below >> records.log2, in = below & ((1u << records.log2) - 1u);
+      if (work && in < (uint32_t)kWorkSrc) work[(size_t)(ridx[e] + of) * kWorkWords + 4 + in] = t;
     }
   }
 }

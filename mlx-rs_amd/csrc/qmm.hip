@@ -843,7 +843,7 @@ static hipError_t launch_small(const GroupedArgs &a, hipStream_t st) {
   }
   const int nw = 4 / kw;
   const int wave_rows = pair ? 32 : 16;  // weight rows per wave
-  dim3 grid((unsigned)((a.N + wave_rows * nw - 1) / (wave_rows * nw)), (unsigned)a.max_active);
+  dim3 grid((unsigned)((a.N + wave_rows * nw - 1) / (wave_rows * nw)), (unsigned)(a.max_records ? a.max_records : a.max_active));
   // blocks a CU holds: by LDS (160 KB) and by registers (4 with the gate/up kernel, 6 otherwise)
   const int by_lds = (int)((size_t)160 * 1024 / (lds > 0 ? lds : 1));
   const bool precise = (by_lds < regs_blocks ? by_lds : regs_blocks) <= MI_MOE_PRECISE_BELOW;

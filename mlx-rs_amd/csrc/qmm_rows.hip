@@ -361,7 +361,7 @@ static hipError_t start_rows(const RowsArgs &a, int sk, int tt, hipStream_t st) 
     if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, L.bytes);
         e != hipSuccess)
       return e;
-  const dim3 grid((unsigned)((a.N + 16 * (4 / KW) - 1) / (16 * (4 / KW))), (unsigned)(a.work ? a.max_active : 1));
+  const dim3 grid((unsigned)((a.N + 16 * (4 / KW) - 1) / (16 * (4 / KW))), (unsigned)(a.work ? a.max_records ? a.max_records : a.max_active : 1));
   kernel<<<grid, 256, (size_t)L.bytes, st>>>(a, tt, sk);
   return hipGetLastError();
 }

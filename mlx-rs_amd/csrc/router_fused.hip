@@ -44,7 +44,7 @@ __global__ __launch_bounds__(kDispThreads) void router_fused_kernel(
     const uint16_t *__restrict__ norm_w, float eps, uint16_t *__restrict__ xnorm,
     int T, int H, int E, int k, int mode, uint16_t *logits, uint32_t *topk_idx, uint16_t *topk_w,
     uint32_t *counters, int nbits, uint32_t *counts, uint32_t *offsets, uint32_t *perm,
-    uint32_t *inv_perm, uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256, uint32_t big_thr, ShortTiles shorts) {
+    uint32_t *inv_perm, uint32_t *src_of, Records work, uint32_t *mtiles, int cap256, uint32_t big_thr, ShortTiles shorts) {
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t last;
   const int tid = threadIdx.x;
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kDispThreads) void router_fused1_kernel(
     const uint16_t *__restrict__ norm_w, float eps, uint16_t *__restrict__ xnorm,
     int T, int H, int E, int k, int mode, uint16_t *logits, uint32_t *topk_idx, uint16_t *topk_w,
     uint32_t *counters, uint32_t *counts, uint32_t *offsets, uint32_t *perm,
-    uint32_t *inv_perm, uint32_t *src_of, uint32_t *work) {
+    uint32_t *inv_perm, uint32_t *src_of, Records work) {
   extern __shared__ uint32_t lds[];  // dispatch: 4 E words; selected experts: T k words behind them
   __shared__ uint32_t last;
   const int tid = threadIdx.x;
@@ -172,7 +172,7 @@ hipError_t launch_router_fused(const uint16_t *x, const uint16_t *wg, const floa
                                int H, int E, int k, int mode, uint16_t *logits, uint32_t *topk_idx,
                                uint16_t *topk_w, uint32_t *counters, uint32_t *counts,
                                uint32_t *offsets, uint32_t *perm, uint32_t *inv_perm,
-                               uint32_t *src_of, uint32_t *work, uint32_t *mtiles, int cap256,
+                               uint32_t *src_of, Records work, uint32_t *mtiles, int cap256,
                                int big_thr, ShortTiles shorts, hipStream_t st) {
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
