@@ -312,7 +312,7 @@ constexpr int64_t kSingleAtMostP = 4096;  // without memory for the histograms
 // of the general path; the same outputs bit for bit.
 // LDS (dynamic, passed in): 4 * E words.  P = T * k <= kSingleMaxP.
 constexpr int kMaskTokens = 64;
-// FLAT_LOCAL: `flat` was written by this workgroup (LDS, or memory behind a barrier): plain loads.
+// FLAT_LOCAL: `flat` was written by this workgroup (LDS, or memory behind a barrier): plain loads; and there are no more tokens than a record takes rows.
 template <bool FLAT_LOCAL = false>
 __device__ __forceinline__ void dispatch_tokens_block(const uint32_t *flat, int T, int k, int E, uint32_t *lds,
                                       uint32_t *__restrict__ counts, uint32_t *__restrict__ offsets,
@@ -345,7 +345,7 @@ __device__ __forceinline__ void dispatch_tokens_block(const uint32_t *flat, int 
     for (int e0 = 0; e0 < E; e0 += kWave) {
       const int e = e0 + tid;
       const uint32_t c = e < E ? (uint32_t)(__popc(mlo[e]) + __popc(mhi[e])) : 0u;
-      const uint32_t own = c != 0u ? ((c - 1u) >> records.log2) + 1u : 0u, both = c | own << 16;
+      const uint32_t own = c == 0u ? 0u : FLAT_LOCAL ? 1u : ((c - 1u) >> records.log2) + 1u, both = c | own << 16;
       uint32_t incl = both;
       for (int d = 1; d < kWave; d <<= 1) {
         const uint32_t v = __shfl_up(incl, d, kWave);
@@ -365,7 +365,7 @@ __device__ __forceinline__ void dispatch_tokens_block(const uint32_t *flat, int 
               const uint32_t first = i << records.log2, left = c - first, most = 1u << records.log2;
               rec[0] = (uint32_t)e;
               rec[1] = excl + first;
-              rec[2] = left < most ? left : most;
+              rec[2] = FLAT_LOCAL || left < most ? left : most;
               rec[3] = 1u;  // the source rows follow below
             }
         }
@@ -396,7 +396,7 @@ __device__ __forceinline__ void dispatch_tokens_block(const uint32_t *flat, int 
       if (inv_perm) inv_perm[j] = pos;
       if (src_of) src_of[pos] = t;
       // source rows of the first rows of every record, so that a consumer needs one load
-      const uint32_t of = below >> records.log2, in = below & ((1u << records.log2) - 1u);
+      const uint32_t of = FLAT_LOCAL ? 0u : below >> records.log2, in = FLAT_LOCAL ? below : below & ((1u << records.log2) - 1u);
       if (work && in < (uint32_t)kWorkSrc) work[(size_t)(ridx[e] + of) * kWorkWords + 4 + in] = t;
     }
   }
