@@ -333,8 +333,9 @@ int mi_moe_debug_plan_grouped(int32_t N, int32_t K, int32_t bits, int32_t glu, i
                               char *out, size_t cap);
 /* which rows of a forward of T tokens go where: *tiled = 1: M-tile lists are built; *tile_min_rows = a segment of
  * at least that many rows is cut into 256-row tiles, with its remainder in the 256-, 128- or 64-row list that
- * holds it; shorter segments stream.  *tiled = 2: every segment is cut into tiles of up to 128 rows on raw codes (4-bit
- * codes in groups of 64, batches beyond the streamed ones; given a workspace of mi_moe_workspace_size); 3: so is every segment of
+ * holds it; shorter segments stream.  (8-bit codes in groups of 64 from 24 rows an expert on: into
+ * pieces of up to 128 rows instead, given a workspace of mi_moe_workspace_size.)  *tiled = 2: every segment is cut into tiles of up to 128 rows on raw codes (groups
+ * of 64, batches beyond the streamed ones; given such a workspace); 3: so is every segment of
  * *tile_min_rows rows and more (larger batches), shorter segments stream */
 int mi_moe_debug_tile_rule(const mi_moe_config *cfg, int64_t T, int32_t *tiled, int32_t *tile_min_rows);
 int32_t mi_moe_debug_side_streams_created(void);
