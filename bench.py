@@ -253,6 +253,9 @@ def run_workload(name, args, torch, m, synth, dev):
         k_name = "qmm_large_kernel (gate/up + SwiGLU, %d-row tiles)" % (256, 128, 64)[cls]
         if m.capi.tile_rule(cfg.c_struct(), headline)[0] >= 2:
             k_name = "qmm_pieces_kernel (gate/up + SwiGLU, all tiled segments)"
+        elif k_ms == 0.0:  # 8-bit pieces: one list, one launch, reported as the 64-row tiles
+            k_ms, k_rows = head["kern"][2], sum(head["class_rows"][:3])
+            k_name = "qmm_bytes_kernel (gate/up + SwiGLU, all tiled segments)"
         k_flops = k_rows * head["per_row_gu_flops"]
         achieved = k_flops / (k_ms * 1e-3) / 1e12
         roofline = {"kernel": k_name, "bound": "mfma",
@@ -263,7 +266,7 @@ def run_workload(name, args, torch, m, synth, dev):
                     "kernel_us": k_ms * 1e3,
                     "kernel_us_source": "start/end time stamps of the dispatch (hipExtLaunchKernelGGL events), mean over the timed steps, "
                                         "kernels launched one after the other on one stream (mi_moe_forward_timed); the timed step itself "
-                                        "(ms_per_step) runs mi_moe_forward's own schedule (8-bit codes: tile classes side by side on two to four streams)",
+                                        "(ms_per_step) runs mi_moe_forward's own schedule (classes of 256-column tiles: side by side on two to four streams)",
                     "serial_kernels_us_sum_vs_step_us": [round((sum(head["kern"]) + sum(head["stage_ms"][i] for i in (0, 1, 2, 5))) * 1e3, 1),
                                                          round(head["ms"] * 1e3, 1)],
                     "dense_gemm_yardstick": dense_gemm_yardstick(torch, int(round(k_rows)), 2 * cfg.intermediate, cfg.hidden, dev),

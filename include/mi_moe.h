@@ -163,7 +163,7 @@ int mi_moe_rms_norm(const uint16_t *x, const uint16_t *weight, float eps, int64_
  * each from the start and end time stamps of its own dispatch (what a profiler reports for the
  * kernel): gate/up + SwiGLU over the 256-row, 128-row and 64-row tile lists and over the streamed
  * segments, then the down product over the same four; 0 where no kernel was launched.  Batches whose
- * segments go through tiles on raw codes (mi_moe_debug_tile_rule: 2, 3) report those two launches
+ * segments go through tiles on raw codes (mi_moe_debug_tile_rule: 2, 3), or through pieces with 8-bit codes, report those two launches
  * as the 64-row ones; blocks with 2-bit codes or groups of 32 / 128 report no kernel.  The kernels
  * run one after the other on `stream`, and the result has the bits of mi_moe_forward.  For measurement; mlx-rs has no counterpart (it times with
  * Instant::now() around eval, mlx-rs/examples/linear_regression.rs:40-59). */
