@@ -221,7 +221,7 @@ int piece_rows(int64_t pairs, int n_experts) { return short_pieces(pairs, n_expe
 // an expert is where the 256-column tiles used to begin, and no longer where either side is the faster one.
 // 8-bit codes: pieces of up to 128 rows on dequantised weights (qmm_bytes.hip) for the segments of seventeen rows and more, the others streamed.  Us of a forward, the other
 // route (tiles of 256 weight rows in three classes on two to four streams) / this, (experts, k, hidden, intermediate):
-//   8, 2, 4096, 14336  even at 70 / 100 / 160 / 256 / 400 / 700 / 1400 / 2048 tokens 578, 573, 591, 734, 696, 940, 1430, 1788 / 532, 418, 456, 519, 587, 810, 1285, 1741;
+//   8, 2, 4096, 14336  even at 100 / 160 / 256 / 400 / 700 / 1400 / 2048 tokens 573, 591, 734, 696, 940, 1430, 1788 / 382 to 425, 400, 437, 497, 810, 1285, 1741;
 //                      Zipf-1.1 at 100 / 300 / 1000 572, 810, 1161 / 544, 595, 988
 //   128, 8, 2048, 768  even at 300 / 512 / 1024 / 2048 / 2500 / 3200 / 4096 tokens 259, 251, 299, 398, 457, 447, 534 / 207, 189, 226, 349, 419, 455, 541; Zipf-1.1 at 400 / 1024 /
 //                      4096 209, 276, 549 / 163, 238, 529

@@ -10,16 +10,16 @@
 namespace mi_moe {
 
 constexpr int kBytesLds = 80 * 1024;
-// What a block of 32 MS token rows and four waves holds in LDS: two places of 64 K values of token rows, the codes of 128 K values (64 weight rows a wave), and two
+// What a block of 32 MS token rows and four waves holds in LDS: two places of 64 K values of token rows, the codes of 128 K values (32 NT weight rows a wave), and two
 // windows of a wave's scales and biases (8 groups, 16 bytes a weight row each).
-template <int MS>
+template <int MS, int NT>
 struct Bytes {
-  static constexpr int XROW = 128, X = 32 * MS * XROW, W = 8192, WINDOW = 2048, LDS = 2 * X + 4 * W + 8 * WINDOW;
+  static constexpr int XROW = 128, X = 32 * MS * XROW, W = NT * 4096, WINDOW = 2048, LDS = 2 * X + 4 * W + 8 * WINDOW;
   static_assert(LDS <= kBytesLds, "two blocks share a CU");
 };
 
-// 32 MS token rows from sorted row `row0` (`rows` of them real) x 256 weight rows of expert e by four waves: GLU, 128 columns of h from n0, a wave 32 gate and the
-// matching 32 up rows; else 256 columns from n0, 64 a wave.  A wave multiplies all the tile's token rows with its own weights, which it dequantises straight into
+// 32 MS token rows from sorted row `row0` (`rows` of them real) x 128 NT weight rows of expert e by four waves: GLU, 128 columns of h from n0, a wave 32 gate and the
+// matching 32 up rows; else 128 NT columns from n0, 32 NT a wave.  A wave multiplies all the tile's token rows with its own weights, which it dequantises straight into
 // the matrix instruction's operands: its codes go to no other wave, and a stage (64 K values) has one barrier, for the token rows.
 //   operands  eight a stage (two sub-tiles of 32 weight rows, four multiplies of 16 K values).  K runs outside, token rows inside, so that two operands are free again
 //             after every quarter of a stage; the next stage's are made there, four vector instructions behind each multiply (128 rows).
@@ -29,9 +29,10 @@ struct Bytes {
 // cycles an XCD at 1.7 GHz, matrix units busy 0.53 of them; without the dequantisation (8 vector instructions a word of codes, 4.5 a multiply) the same cycles at 2.0 GHz, with all
 // copies out of L2 9 % fewer, with half the codes 14 %.  Codes copied in pieces of 64 bytes, a stage at a time: 1029 us for 975, down 606 for 556.
 //   KW = 2    two groups of four waves share K, each with an LDS place of its own; the second one's sums go to the first through LDS at the end.
-template <bool GLU, int MS, int KW>
+template <bool GLU, int MS, int KW, int NT>
 __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_t row0, int rows, int n0, unsigned char *block_lds) {
-  typedef Bytes<MS> R;
+  typedef Bytes<MS, NT> R;
+  static_assert(!GLU || NT == 2, "a gate and an up row's sub-tile");
   constexpr int NM = GLU ? 2 : 1;
   const int lane = threadIdx.x & 63, ln = lane & 31, kb = lane >> 5;
   const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wave_all % 4, kg = wave_all / 4;
@@ -48,7 +49,7 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
     sr[t] = words_of(static_cast<const uint16_t *>(t ? a.s1 : a.s0) + ebase * G, (uint32_t)N * G * 2);
     br[t] = words_of(static_cast<const uint16_t *>(t ? a.b1 : a.b0) + ebase * G, (uint32_t)N * G * 2);
   }
-  const int col0 = n0 + (GLU ? 32 : 64) * wave, own0 = col0 < N ? col0 : N - 64;  // (columns past the end are others again, and never stored)
+  const int col0 = n0 + (GLU ? 32 : 32 * NT) * wave, own0 = col0 < N ? col0 : N - 32 * NT;  // (columns past the end are others again, and never stored)
   // ---- what a lane copies.  Sixteen-byte pieces of a row are turned by a number of the row's, so that sixteen rows' pieces of one number lie in different banks.
   auto turned = [](int row) __attribute__((always_inline)) { return (row >> 1) & 7; };
   uint32_t x_off[MS], w_off[2];
@@ -60,14 +61,14 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
 #pragma unroll
   for (int i = 0; i < 2; ++i)  // rows 8 i + lane / 8; 16 rows on the pieces are turned alike
     w_off[i] = (uint32_t)(own0 + 8 * i + lane / 8) * (uint32_t)K + ((uint32_t)((lane % 8) ^ turned(8 * i + lane / 8)) << 4);
-  const uint32_t window_off = (uint32_t)(own0 + (GLU ? ln : lane)) * (uint32_t)(G * 2);
+  const uint32_t window_off = (uint32_t)(own0 + (GLU || NT == 1 ? ln : lane)) * (uint32_t)(G * 2);
   auto copy_rows = [&](int k, uint32_t place) __attribute__((always_inline)) {  // (past the end the last values again)
 #pragma unroll
     for (int c = 0; c < MS; ++c) copy_to_lds(xr, x_off[c], (k < K ? k : K - 64) * 2, ring_at + place * R::X + (wave * MS + c) * 1024);
   };
   auto copy_codes = [&](int k) __attribute__((always_inline)) {  // of 128 K values
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 4 * NT; ++i)
       copy_to_lds(wr[GLU ? i / 4 : 0], w_off[i & 1], (k < K ? k : K - 128) + ((i & 2) + (GLU ? 0 : i & 4)) * 8 * K, ring_at + kCodes + wave * R::W + i * 1024);
   };
   auto copy_window = [&](int k) __attribute__((always_inline)) {  // the 8 groups from K value k on: 16 bytes a weight row of scales, 1024 bytes behind them of biases
@@ -79,23 +80,26 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
         copy_half_to_lds(sr[t], window_off, from, to + t * 512);
         copy_half_to_lds(br[t], window_off, from, to + 1024 + t * 512);
       }
+    } else if constexpr (NT == 1) {
+      copy_half_to_lds(sr[0], window_off, from, to);
+      copy_half_to_lds(br[0], window_off, from, to + 1024);
     } else {
       copy_to_lds(sr[0], window_off, from, to);
       copy_to_lds(br[0], window_off, from, to + 1024);
     }
   };
 
-  f32x16_t tot[MS][2];
+  f32x16_t tot[MS][NT];
 #pragma unroll
   for (int m = 0; m < MS; ++m)
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int v = 0; v < 16; ++v) tot[m][t][v] = 0.f;
-  u32x4_t op[2][4], q[2][2][2];  // operands; sixteen codes of a weight row: of each of two stages, K values 0 .. 31 of it and those behind
-  u32x2_t rest[2];               // the codes of a pair's last multiply
-  float scale[2], offset[2];
-  uint32_t s_now[2], b_now[2];
+  u32x4_t op[NT][4], q[2][2][NT];  // operands; sixteen codes of a weight row: of each of two stages, K values 0 .. 31 of it and those behind
+  u32x2_t rest[NT];               // the codes of a pair's last multiply
+  float scale[NT], offset[NT];
+  uint32_t s_now[NT], b_now[NT];
   // Piece 2 kb + (h & 1) + 4 (h / 2) of a token row is multiply h's, piece 2 i + kb of a row of codes quarter i of a pair: made out of the first ones where they are wanted.
   uint32_t xa = ln * R::XROW + ((2 * kb ^ turned(ln)) << 4), wa = kCodes + wave * R::W + ln * 128 + ((kb ^ turned(ln)) << 4);
   // Two weights of a word of codes, behind the exponent of 1024 as f16 (exact) and back out of it in the fma that scales them.
@@ -108,24 +112,24 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) q[i >> 1][i & 1][t] = *reinterpret_cast<const u32x4_t *>(lds_raw + (wa ^ i << 5) + t * 4096);
+      for (int t = 0; t < NT; ++t) q[i >> 1][i & 1][t] = *reinterpret_cast<const u32x4_t *>(lds_raw + (wa ^ i << 5) + t * 4096);
   };
   auto fetch_scales = [&](int k) __attribute__((always_inline)) {
     const unsigned char *const at = lds_raw + kScales + (wave * 2 + (k >> 9 & 1)) * R::WINDOW + (k >> 6 & 7) * 2 + ln * 16;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < NT; ++t) {
       s_now[t] = *reinterpret_cast<const uint16_t *>(at + t * 512);
       b_now[t] = *reinterpret_cast<const uint16_t *>(at + t * 512 + 1024);
     }
   };
   auto take_scales = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < NT; ++t) {
       scale[t] = __uint_as_float(s_now[t] << 16);
       offset[t] = __builtin_fmaf(-1024.0f, scale[t], __uint_as_float(b_now[t] << 16));
     }
   };
-  // word i (0 .. 7) of the two operands that quarter `made` of a pair's stage consumes
+  // word i (0 .. 4 NT - 1) of the operands that quarter `made` of a pair's stage consumes
   auto make = [&](int stage, int made, int i) __attribute__((always_inline)) {
     const int t = i >> 2, w = i & 3;
     const uint32_t codes = stage == 1 && made == 3 ? rest[t][w >> 1] : q[stage][made >> 1][t][2 * (made & 1) + (w >> 1)];
@@ -157,12 +161,12 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+      for (int t = 0; t < NT; ++t) {
         tot[m][t] = mfma<0>(F[j % AHEAD], op[t][h], tot[m][t]);
-        if (t == 1 && j + AHEAD < STEPS) fetch(j + AHEAD);
-        const int u = 2 * m + t;
+        if (t == NT - 1 && j + AHEAD < STEPS) fetch(j + AHEAD);
+        const int u = NT * m + t;
 #pragma unroll
-        for (int i = u * 8 / (2 * MS); i < (u + 1) * 8 / (2 * MS); ++i) make(h == 0 ? STAGE : STAGE ^ 1, (h + 3) & 3, i);
+        for (int i = u * 4 / MS; i < (u + 1) * 4 / MS; ++i) make(h == 0 ? STAGE : STAGE ^ 1, (h + 3) & 3, i);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -178,18 +182,18 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
   fetch_codes();
   take_scales();
 #pragma unroll
-  for (int i = 0; i < 24; ++i) make(0, i >> 3, i & 7);
+  for (int i = 0; i < 12 * NT; ++i) make(0, i / (4 * NT), i % (4 * NT));
   wait_reads();
   if ((k_first + 128 & 511) == 0) copy_window(k_first + 128);
   copy_codes(k_first + 128);
 #pragma unroll 1
   for (int k = k_first; k < k_end; k += 128) {
-    wait_copies<8>();  // this stage's token rows have arrived, in every wave, and the place copied to next has been read; the next pair's codes may still be coming
+    wait_copies<4 * NT>();  // this stage's token rows have arrived, in every wave, and the place copied to next has been read; the next pair's codes may still be coming
     block_barrier();
     copy_rows(k + 64, 1);
     multiply(k, first);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) rest[t] = u32x2_t{q[1][1][t][2], q[1][1][t][3]};
+    for (int t = 0; t < NT; ++t) rest[t] = u32x2_t{q[1][1][t][2], q[1][1][t][3]};
     wait_copies<0>();
     block_barrier();
     copy_rows(k + 128, 0);
@@ -199,23 +203,23 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
   wait_copies<0>();
   block_barrier();
   if constexpr (KW == 2) {
-    float4 *const parts = reinterpret_cast<float4 *>(block_lds) + wave * (MS * 8 * 64) + lane;
+    float4 *const parts = reinterpret_cast<float4 *>(block_lds) + wave * (MS * NT * 4 * 64) + lane;
 #pragma unroll
     for (int m = 0; m < MS; ++m)
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (kg == 1) parts[((m * 2 + t) * 4 + r) * 64] = make_float4(tot[m][t][4 * r], tot[m][t][4 * r + 1], tot[m][t][4 * r + 2], tot[m][t][4 * r + 3]);
+          if (kg == 1) parts[((m * NT + t) * 4 + r) * 64] = make_float4(tot[m][t][4 * r], tot[m][t][4 * r + 1], tot[m][t][4 * r + 2], tot[m][t][4 * r + 3]);
     __syncthreads();
     if (kg == 1) return;
 #pragma unroll
     for (int m = 0; m < MS; ++m)
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float4 v = parts[((m * 2 + t) * 4 + r) * 64];
+          const float4 v = parts[((m * NT + t) * 4 + r) * 64];
           tot[m][t][4 * r] += v.x;
           tot[m][t][4 * r + 1] += v.y;
           tot[m][t][4 * r + 2] += v.z;
@@ -234,8 +238,8 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
       dst[h] = a.dst_rows ? a.dst_rows[r] : (uint32_t)r;
     }
   }
-  constexpr int ROWB = GLU ? 272 : 144;  // (16 bytes keep rows off each other's banks)
-  static_assert((GLU ? 32 * MS * 272 : 4 * 32 * 144) <= R::LDS, "the results' place");
+  constexpr int ROWB = GLU ? 272 : 64 * NT + 16, PIECES = 4 * NT;  // (16 bytes keep rows off each other's banks)
+  static_assert((GLU ? 32 * MS * 272 : 4 * 32 * ROWB) <= R::LDS, "the results' place");
   unsigned char *const mine = GLU ? lds_raw + wave * 64 : lds_raw + wave * (32 * ROWB);
   float odd = 0.f;  // no number once a result was not finite
   auto turn = [&](int m, int at, auto plain) __attribute__((always_inline)) {
@@ -245,7 +249,7 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
       return decltype(plain)::value ? g / (1.0f + __expf(-g)) * u : gated(g, u);
     };
 #pragma unroll
-    for (int t = 0; t < (GLU ? 1 : 2); ++t)
+    for (int t = 0; t < (GLU ? 1 : NT); ++t)
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
         const float v0 = value(t, r), v1 = value(t, r + 1);
@@ -278,11 +282,11 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = 8 * i + (lane >> 3), tr = 32 * m + row;
-        const u32x4_t w = *reinterpret_cast<const u32x4_t *>(mine + row * ROWB + (lane & 7) * 16);
+      for (int i = 0; i < PIECES / 2; ++i) {
+        const int row = 64 / PIECES * i + lane / PIECES, tr = 32 * m + row;
+        const u32x4_t w = *reinterpret_cast<const u32x4_t *>(mine + row * ROWB + lane % PIECES * 16);
         const uint32_t to = (uint32_t)__shfl((int)dst[m / 2], tr & 63, 64);
-        if (tr < rows && col0 < N) *reinterpret_cast<u32x4_t *>(static_cast<uint16_t *>(a.y) + (int64_t)to * N + col0 + 8 * (lane & 7)) = w;
+        if (tr < rows && col0 < N) *reinterpret_cast<u32x4_t *>(static_cast<uint16_t *>(a.y) + (int64_t)to * N + col0 + 8 * (lane % PIECES)) = w;
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -295,39 +299,45 @@ __device__ __forceinline__ void multiply_bytes(const CodesArgs &a, int e, int64_
 // in the list, mostly of one expert, so that its L2 holds their codes once: 8 experts, 4096 x 14336 at 512 / 2048 tokens 704 / 1721 us a forward, pieces each on their
 // own 739 / 1745, two 720 / 1723, eight 737 / 1732.
 constexpr uint32_t kRun = 4;
-template <bool GLU, int KW>
+template <bool GLU, int KW, int NT>
 __global__ __launch_bounds__(256 * KW, 2) void qmm_bytes_kernel(CodesArgs a, const uint32_t *__restrict__ list, int n_ntiles) {
   const uint32_t xcd = blockIdx.x & 7, j = blockIdx.x >> 3, unit = j / kRun * 8u + xcd;
   const uint32_t id = unit / (uint32_t)n_ntiles * kRun + j % kRun;
   if (id >= list[0]) return;
-  const int n0 = (int)(unit % (uint32_t)n_ntiles) * (GLU ? 128 : 256);
+  const int n0 = (int)(unit % (uint32_t)n_ntiles) * (GLU ? 128 : 128 * NT);
   const uint4 rec = reinterpret_cast<const uint4 *>(list)[1 + id];
   const int e = __builtin_amdgcn_readfirstlane((int)rec.x), rows = __builtin_amdgcn_readfirstlane((int)rec.z);
   const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane((int)rec.y);
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  if (rows > 96) multiply_bytes<GLU, 4, KW>(a, e, row0, rows, n0, lds_raw);
-  else if (rows > 64) multiply_bytes<GLU, 3, KW>(a, e, row0, rows, n0, lds_raw);
-  else if (rows > 32) multiply_bytes<GLU, 2, KW>(a, e, row0, rows, n0, lds_raw);
-  else multiply_bytes<GLU, 1, KW>(a, e, row0, rows, n0, lds_raw);
+  if (rows > 96) multiply_bytes<GLU, 4, KW, NT>(a, e, row0, rows, n0, lds_raw);
+  else if (rows > 64) multiply_bytes<GLU, 3, KW, NT>(a, e, row0, rows, n0, lds_raw);
+  else if (rows > 32) multiply_bytes<GLU, 2, KW, NT>(a, e, row0, rows, n0, lds_raw);
+  else multiply_bytes<GLU, 1, KW, NT>(a, e, row0, rows, n0, lds_raw);
 }
 
-template <bool GLU, int KW>
-static hipError_t start_bytes(const CodesArgs &a, const uint32_t *list, int cap, int n_ntiles, hipStream_t st) {
+template <bool GLU, int KW, int NT>
+static hipError_t start_bytes(const CodesArgs &a, const uint32_t *list, int cap, hipStream_t st) {
+  constexpr int NI = GLU ? 128 : 128 * NT;
+  const int n_ntiles = (a.N + NI - 1) / NI;
   const int64_t units = ((int64_t)cap + kRun - 1) / kRun * n_ntiles, grid = (units + 7) / 8 * 8 * kRun;
   if (grid <= 0 || grid > INT32_MAX || a.N % 128 || a.K % (128 * KW)) return hipErrorInvalidValue;
-  const auto kernel = &qmm_bytes_kernel<GLU, KW>;
+  const auto kernel = &qmm_bytes_kernel<GLU, KW, NT>;
   static std::atomic<uint64_t> allowed{0};
   if (hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), KW * kBytesLds, allowed); e != hipSuccess) return e;
   launch_or_time(kernel, dim3((unsigned)grid), dim3(256 * KW), KW * kBytesLds, st, a, list, n_ntiles);
   return hipGetLastError();
 }
+// Where no CU gets two blocks (a down product of few experts: 8 pieces are 128 blocks of 256 of 4096 columns), the length of a block's K is what counts, and two groups of waves
+// share it; and where there are fewer blocks still, they are of 128 columns, so that more CUs have one.  8 experts, 4096 x 14336, us of a forward, K not shared / 256 columns / 128:
+// 100 tokens 441 / 425 / 382 to 425, 160 481 / 448 / 400, 200 488 / 455 / 410, 256 534 / 485 / 437, 400 tokens - / 563 / 497; 512 tokens (two pieces an expert) - / 674 / 706.
 template <bool GLU>
 static hipError_t start_bytes(const CodesArgs &a, const uint32_t *list, int cap, hipStream_t st) {
   constexpr int NI = GLU ? 128 : 256;
-  const int n_ntiles = (a.N + NI - 1) / NI;
-  // Where no CU gets two blocks (a down product of few experts: 8 pieces are 128 blocks of 4096 columns), the length of a block's K is what counts, and two groups of waves
-  // share it: 8 experts, 4096 x 14336 at 100 / 160 / 200 / 256 tokens 441, 481, 488, 534 us a forward without / 418, 456, 459, 519 with.
-  return (int64_t)cap * n_ntiles <= 256 && a.K % 256 == 0 ? start_bytes<GLU, 2>(a, list, cap, n_ntiles, st) : start_bytes<GLU, 1>(a, list, cap, n_ntiles, st);
+  const int64_t blocks = (int64_t)cap * ((a.N + NI - 1) / NI);
+  if (blocks > 256 || a.K % 256) return start_bytes<GLU, 1, 2>(a, list, cap, st);
+  if constexpr (!GLU)
+    if (blocks < 256) return start_bytes<GLU, 2, 1>(a, list, cap, st);
+  return start_bytes<GLU, 2, 2>(a, list, cap, st);
 }
 hipError_t launch_qmm_bytes(const CodesArgs &a, const uint32_t *list, int cap, bool glu, hipStream_t st) {
   return glu ? start_bytes<true>(a, list, cap, st) : start_bytes<false>(a, list, cap, st);

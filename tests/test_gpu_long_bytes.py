@@ -10,13 +10,22 @@ from test_gpu_short_pieces import chosen_block  # noqa: E402
 EDGES = [0, 1, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 145, 257]  # both sides of every length at which another kernel, body or piece begins
 
 
-# K of 1, 2, 3, 8, 9 and 17 times 128 values: windows of 512 whole and started; 18 experts and few columns: K shared by two groups of waves where it is whole 256s,
+# K of 1, 2, 3, 8, 9 and 17 times 128 values: windows of 512 whole and started; 18 experts and few columns: K shared by two groups of waves where it is whole 256s, blocks of 128 columns;
 # many columns: one group; output columns that fill no block of 256
 @pytest.mark.parametrize("hidden,inter,experts", [(128, 384, 18), (384, 128, 18), (256, 512, 18), (1024, 1152, 18), (1152, 1024, 18), (2176, 256, 36), (256, 2176, 36), (768, 768, 90)])
 def test_lengths_around_every_body_b(hidden, inter, experts):
     """Roundings to bfloat16 of the weights of three products, h, y and the result, each typically 0.42 * 2^-8 of its values: 1.03 * 2^-8 together; a row's bound is twice
     that.  Rows do not depend on their order in the batch."""
-    blk, x, of = chosen_block(hidden, inter, EDGES, experts, 8, 64)
+    check(hidden, inter, EDGES, experts)
+
+
+def test_as_many_blocks_as_cus():
+    """32 pieces at most by eight blocks of 256 columns: K shared by two groups of waves of 64 columns each."""
+    check(2048, 256, [45, 30, 60], 24)
+
+
+def check(hidden, inter, lengths, experts):
+    blk, x, of = chosen_block(hidden, inter, lengths, experts, 8, 64)
     out, routing = blk.forward(x, debug=True)
     assert torch.equal(routing["topk_idx"][:, 0].long(), of)
     ref = block_truth(blk, x, routing)
