@@ -172,9 +172,10 @@ bool raw_list_batch(const mi_moe_config &c, int64_t T) {
 // With fewer blocks in the down product than CUs its blocks are what a forward waits for, whatever their rows, and streaming stays ahead up to some thirteen rows.  At 25 and 32 rows
 // an expert 128 experts would still gain (400 / 512 tokens 206, 189 / 167, 174, skewed 163 / 153) and eight skewed ones lose (above); from 24 on the launch plan of 8-bit
 // batches holds streamed segments beside tiles, as its callers know it.
+bool few_rows_batch(const mi_moe_config &c, int64_t T) { return T * c.top_k < (int64_t)24 * c.n_experts; }
 bool mid_bytes_batch(const mi_moe_config &c, int64_t T) {
   const int64_t P = T * c.top_k, E = c.n_experts, least = E * (c.hidden / 256) >= 256 ? 6 : 14;
-  return c.bits == 8 && c.group_size == 64 && E >= 8 && P >= least * E && P < 24 * E && codes_tiles_fit(c, T);
+  return c.bits == 8 && c.group_size == 64 && E >= 8 && P >= least * E && few_rows_batch(c, T) && codes_tiles_fit(c, T);
 }
 // Groups of 64, 4-bit codes: batches whose segments all go through pieces on raw codes, in one launch a product on the caller's
 // stream (the others: streamed segments, and tiles of 256 weight rows on side streams).  From the batches on for which the tile lists
@@ -491,7 +492,26 @@ int mi_moe_workspace_size(const mi_moe_config *cfg, int64_t max_tokens, size_t *
   if (check_config(cfg)) return 1;
   if (max_tokens < 0) return fail("workspace_size: negative token count");
   if (max_tokens * cfg->top_k > (int64_t)1 << 30) return fail("workspace_size: too many (token, expert) pairs");
-  *bytes = carve_forward(*cfg, max_tokens, nullptr, true).bytes + 256;
+  // A caller keeps one workspace for its largest batch: it has to hold what every smaller one takes.  That grows with the tokens except where a route ends whose regions
+  // the next one does without: 8-bit batches of a few rows an expert, and operands that reach 2 GiB.
+  const mi_moe_config &c = *cfg;
+  auto last_of = [](int64_t most, auto takes) {  // up to `most` tokens, the largest batch of a route that takes all smaller ones
+    int64_t lo = 0, hi = most;
+    while (lo < hi) {
+      const int64_t mid = lo + (hi - lo + 1) / 2;
+      if (takes(mid)) lo = mid;
+      else hi = mid - 1;
+    }
+    return lo;
+  };
+  const int64_t fits = last_of(max_tokens, [&](int64_t T) { return codes_tiles_fit(c, T); });
+  const int64_t few = last_of(fits, [&](int64_t T) { return few_rows_batch(c, T); });
+  size_t most = 0;
+  for (const int64_t T : {max_tokens, fits, few}) {
+    const size_t need = carve_forward(c, T, nullptr, true).bytes;
+    most = need > most ? need : most;
+  }
+  *bytes = most + 256;
   return 0;
 } MI_CATCH("workspace_size")
 
