@@ -322,9 +322,12 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
   //   128, 8, 2048, 768, 8 bits  Zipf-1.1 at 64 159 / 93; 8, 2, 4096, 14336, 8 bits at 32 / 48 416, 533 / 348, 457
   f.records = Records(f.work);
   const bool rows_kernel = f.raw && !f.raw_all, streams = !plain_config(c) && !f.tiled && !f.mid;
-  if (const int log2 = c.bits == 4 && streams ? 3 : 4; (streams || rows_kernel) && T > 1 << log2) {  // (rows of a pass)
-    const int64_t most = P < c.n_experts ? P : c.n_experts, slots = most + ((P - most) >> log2);
-    f.records = Records(cv.take<uint32_t>((size_t)slots * 16), log2, (int)slots);
+  if (int log2 = c.bits == 4 && streams ? 3 : 4; (streams || rows_kernel) && T > 1 << log2) {  // (rows of a pass)
+    const int64_t most = P < c.n_experts ? P : c.n_experts;
+    auto slots = [&]() { return most + ((P - most) >> log2); };
+    uint32_t *const at = cv.take<uint32_t>((size_t)(slots() < kMostRecords ? slots() : kMostRecords) * 16);
+    while (slots() > kMostRecords) ++log2;  // (from half a million pairs on: several passes)
+    f.records = Records(at, log2, (int)slots());
   }
   if (f.raw_all) {
     f.raw_cap = short_list_cap(P, c.n_experts, f.raw_from, f.raw_piece);

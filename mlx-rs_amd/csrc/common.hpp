@@ -190,6 +190,7 @@ struct Records {
   int log2, slots;
   __host__ __device__ Records(uint32_t *p = nullptr, int l = 31, int n = 0) : at(p), log2(l), slots(n) {}
 };
+constexpr int kMostRecords = 65535;  // they are a launch's y extent, which goes no further
 __host__ __device__ inline size_t short_list_words(int cap) { return 4 + 4 * (size_t)cap; }
 inline int short_list_cap(int64_t pairs, int n_experts, int from, int piece) {  // full pieces, and a segment's last one
   return (int)(pairs / piece + (pairs / from < n_experts ? pairs / from : n_experts));
