@@ -75,4 +75,22 @@ constexpr int long_tile_rows(int64_t M, int N, int K, int bits) {
   return bits == 8 && K >= 3072 && tiles_of_an_xcd(M, N, 128, 128) <= 32 ? 128 : 0;
 }
 
+// Dense float32 rows: tiles on the float32 matrix instructions (qmm_f32.hip), or the plain kernel (quantize.hip).  A launch of tiles takes as long as the fullest XCD's rounds, whatever share of
+// a round there is: at K = 4096 28 us for one of 32 x 32, 47 of 64 x 32, 86 a round of 64 x 64.  The plain kernel's time is that of its blocks, of 8 rows (4 with 8-bit codes) x 16
+// columns here: up to 1024 of them run at once in 20 to 30 us, 2048 take 49 to 60, then 0.024 us each and, where rows are no multiple of 1024 values (K = 4096 apart), a third more; with
+// 8-bit codes 0.017.  The lines lie where the two meet: of 2000 shapes and group sizes (64 to 9000 rows, 16 to 4096 columns, K = 1024 to 16384) the tiles take 900, and are slower than the plain
+// kernel in three, by 2 %.  Us, plain / tiles, 4-bit unless named:
+//   tiles  64 / 250 / 1000 x 3072 x 3072 38.9, 112, 561 / 22.1, 67.5, 197; 96 x 1536 x 2048 20 / 16; 192 x 1024 x 4096 42 / 28; 700 x 256 x 8192 81 / 55; 116 x 1176 x 3712 40 / 25; 700 x 1024 x 4096
+//          132 / 86; 8-bit 64 / 1000 x 4096 x 4096 74, 1082 / 28, 335; 96 x 1024 x 4096 32 / 28; 1000 x 128 x 2048 20 / 16
+//   plain  64 x 256 x 16384 20 / 105; 72 x 256 x 8192 17 / 53; 64 x 1024 x 4096 18 / 28; 2228 x 104 x 5632 90 / 226; 2510 x 136 x 1280 39 / 60; 400 x 64 x 8192 21 / 54; 8-bit 72 x 512 x 8192 32 / 53
+//   fewer rows, which keep a row's sums whatever their number: 24 / 32 / 48 x 3072 x 3072 22, 22, 37 / 25, 26, 27
+// Shorter K keeps the plain sums for their error: at K = 384 and 8-bit codes the plain kernel's 64 sums of six values lose 3 % less.
+constexpr bool float32_tiles(int64_t rows, int N, int K, int bits) {
+  if (rows < 64 || K < 1024) return false;
+  const int64_t plain = (bits == 4 ? (rows + 7) / 8 : (rows + 3) / 4) * ((N + 15) / 16), rounds = (tiles_of_an_xcd(rows, N, 64, 64) + 31) / 32;
+  const int size = tiles_of_an_xcd(rows, N, 32, 32) <= 32 ? 0 : tiles_of_an_xcd(rows, N, 64, 32) <= 32 ? 1 : 2;
+  if (bits == 8) return plain > (size == 0 ? 1350 : size == 1 ? 2500 : 5300 * rounds);
+  return K % 1024 == 0 ? plain > (size == 0 ? 1024 : size == 1 ? 1700 : 3600 * rounds) : plain > (size == 0 ? 900 : size == 1 ? 1550 : 2750 * rounds);
+}
+
 }  // namespace mi_moe

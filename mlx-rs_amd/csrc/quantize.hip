@@ -8,6 +8,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "dense_rule.hpp"
 
 namespace mi_moe {
 
@@ -268,7 +269,7 @@ __global__ __launch_bounds__(256) void qmm_plain_t_kernel(const T *__restrict__ 
 
 // The same product of dense float32 rows, 4- and 8-bit codes, R rows by C columns a wave: a word of codes is read and
 // dequantised once for R rows, a value of x once for C columns.  Every sum runs over the same lanes in the same order as
-// in qmm_plain_t_kernel, so the bits are the same.  (The matrix cores on raw codes lose two bits: see qmm_codes.hip; from 64 rows on qmm_f32.hip.)
+// in qmm_plain_t_kernel, so the bits are the same.  (The matrix cores on raw codes lose two bits: see qmm_codes.hip; many rows and columns: qmm_f32.hip.)
 // Sums meet by halving: at lane distance d each lane hands the half of its sums that its partner keeps; an addition
 // commutes, so the tree of a sum does not depend on the lane that holds it.
 // What bounds it: the vector unit, an fma per value and sum (430 us of it at 1000 x 4096 x 4096) beside the loads of x.
@@ -421,13 +422,6 @@ static hipError_t launch_plain_f32(const float *x, const uint32_t *w, const floa
   return run(two, std::integral_constant<int, 1>{});
 }
 
-// From here on tiles on the float32 matrix instructions (qmm_f32.hip) are faster than the kernel above.
-// Us of the call, the kernel above / those (rows x N x K): 4-bit 64 / 250 / 1000 x 3072 x 3072 38.9, 112, 561 / 22.1, 67.5, 197; in groups of 128 100 / 200 x 2064 x 4096 55, 105 / 47, 87; in
-// groups of 32 150 / 200 / 1000 x 1024 x 1024 14.0, 16.4, 68 / 9.1, 9.1, 27; 8-bit 64 / 1000 x 4096 x 4096 74, 1082 / 28, 335; 64 / 200 x 1152 x 2048 19, 37 / 17, 28.
-// Below: 4-bit 24 / 32 / 48 x 3072 x 3072 22, 22, 37 / 25, 26, 27; 64 x 1024 x 1024 7.0 / 9.9.  Fewer than 64 rows keep the sums of a row by itself, bit for bit.
-// Shorter rows keep them for their error: at K = 384 and 8-bit codes the plain kernel's 64 sums of six values lose 3 % less.
-static bool float32_tiles(int64_t rows, int N, int K) { return rows >= 64 && K >= 1024 && rows * N >= (int64_t)150000000 / K; }
-
 // dt: 0 bf16, 1 fp16, 2 fp32.  rows = n_idx * M output rows (at most 2^31 - 1: they are the grid's x extent).
 hipError_t launch_qmm_plain(const void *x, const uint32_t *w, const void *scales, const void *biases,
                             const uint32_t *lhs, const uint32_t *rhs, const uint32_t *rhs_map,
@@ -438,7 +432,7 @@ hipError_t launch_qmm_plain(const void *x, const uint32_t *w, const void *scales
   const PlainMaps mp{lhs, rhs, rhs_map, dst_map, n_lhs, n_rhs};
   if (dt == 2 && transpose && bits != 2 && rows > 1 && !lhs && !rhs && !dst_map && (reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
     const float *xs = static_cast<const float *>(x), *ss = static_cast<const float *>(scales), *bs = static_cast<const float *>(biases);
-    if (float32_tiles(rows, N, K)) return launch_qmm_f32(xs, w, ss, bs, rows, N, K, group, bits, static_cast<float *>(y), st);
+    if (float32_tiles(rows, N, K, bits)) return launch_qmm_f32(xs, w, ss, bs, rows, N, K, group, bits, static_cast<float *>(y), st);
     if (bits == 4) return launch_plain_f32<4>(xs, w, ss, bs, rows, N, K, group, static_cast<float *>(y), st);
     return launch_plain_f32<8>(xs, w, ss, bs, rows, N, K, group, static_cast<float *>(y), st);
   }
