@@ -154,11 +154,11 @@ bool codes_tiles_fit(const mi_moe_config &c, int64_t T) {
 // Group sizes 32 and 128: batches whose segments all go in pieces (qmm_short_kernel), one launch a product; the others go through the kernel of a few rows, which a
 // segment of at most T rows has to be more than one pass of.  Us of a forward, tiles of 32 x 32 results (qmm_tiles.hip; with 8-bit codes between twenty and forty rows
 // an expert short segments on the kernel of a few rows beside them, on another stream) / pieces, (experts, k, hidden, intermediate, bits, group):
-//   128, 8, 2048, 768, 4, 32   even at 100 / 160 / 256 / 400 / 512 tokens 150, 150, 153, 169, 175 / 120, 123, 130, 147, 151; Zipf-1.1 at 100 / 256 / 512 145, 118, 164 / 116, 102, 145
-//   128, 8, 2048, 768, 4, 128  even at 100 / 256 / 512 114, 121, 137 / 92, 108, 119; Zipf-1.1 at 512 171 / 149
+//   128, 8, 2048, 768, 4, 32   even at 100 / 160 / 256 / 400 / 512 tokens 147, 150, 152, 168, 175 / 122, 127, 134, 140, 149; Zipf-1.1 at 100 / 256 / 512 98, 116, 163 / 86, 100, 143
+//   128, 8, 2048, 768, 4, 128  even at 100 / 256 / 512 113, 120, 138 / 93, 107, 118; Zipf-1.1 78, 91, 124 / 71, 83, 115
 //   128, 8, 2048, 768, 8, 32   even at 100 / 330 / 512 199, 236, 248 / 187, 200, 208; Zipf-1.1 at 330 / 512 260, 213 / 234, 193; 1.3 at 500 189 / 180
 //   128, 8, 2048, 768, 8, 128  even at 330 / 512 194, 198 / 160, 169; Zipf-1.1 at 330 / 512 229, 180 / 184, 151
-//   64, 6, 2048, 1408, 4, 32   128 tokens, even and Zipf-1.1 140, 170 / 115, 137; 8, 2, 4096, 7168, 4, 32 at 256 tokens 348 / 297; 8, 2, 4096, 14336, 8, 32 at 100 645 / 515
+//   64, 6, 2048, 1408, 4, 32   128 tokens, even and Zipf-1.1 139, 131 / 119, 105; 8, 2, 4096, 7168, 4, 32 at 256 tokens 346 / 280; 8, 2, 4096, 14336, 8, 32 at 100 645 / 515
 // All segments on the kernel of a few rows (4-bit, 32): 512 tokens and even routing 328, Zipf-1.1 1017.
 bool raw_list_batch(const mi_moe_config &c, int64_t T) {
   return T > kRowsMost && T * c.top_k >= (int64_t)4 * c.n_experts && codes_tiles_fit(c, T);

@@ -22,11 +22,10 @@ __device__ __forceinline__ Pieces split3(float v) {
   return Pieces{hu >> 16, mu >> 16, __float_as_uint(q) >> 16};
 }
 
-// A group sum of a row as the bias product's operand: the pieces against those of the biases (six products), or against one.  half: in a slot that is
-// multiplied with nothing, the sum of the group's first half, about (what of it a piece's sums start from in qmm_short.hip; the other half's start from the rest).
-__device__ __forceinline__ void put_sums(uint16_t *to, int slots, float sum, float half = 0.f) {
+// A group sum of a row as the bias product's operand: the pieces against those of the biases (six products), or against one.
+__device__ __forceinline__ void put_sums(uint16_t *to, int slots, float sum) {
   const Pieces p = split3(sum);
-  if (slots == kSlots) *reinterpret_cast<uint4 *>(to) = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, __float_as_uint(half) >> 16);
+  if (slots == kSlots) *reinterpret_cast<uint4 *>(to) = make_uint4(p.h | p.m << 16, p.l | p.h << 16, p.m | p.h << 16, 0u);
   else *reinterpret_cast<uint2 *>(to) = make_uint2(p.h | p.m << 16, p.l);
 }
 
@@ -68,16 +67,12 @@ __device__ __forceinline__ void prepare_octet(const PrepareArgs &a, int64_t i) {
   sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
   sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
   if (a.lanes_log2 >= 3) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
-  float half = 0.f;
-  if (a.lanes_log2 == 4) {
-    if (ORDER == RowOrder::kQuads) half = sum;
-    sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
-  }
+  if (a.lanes_log2 == 4) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
   if ((i & ((1 << a.lanes_log2) - 1)) == 0) {
     const int64_t row = i / a.octets_per_row;
     const int g = (int)(i % a.octets_per_row) >> a.lanes_log2, G = a.octets_per_row >> a.lanes_log2;
     uint16_t *const to = a.sums + row * a.sums_row;
-    put_sums(to + g * SLOTS, SLOTS, sum, half);
+    put_sums(to + g * SLOTS, SLOTS, sum);
     if (g == G - 1)  // (an even number of groups where a group has four slots)
       for (int k = G * SLOTS; k < a.sums_row; k += 8) *reinterpret_cast<uint4 *>(to + k) = make_uint4(0, 0, 0, 0);
   }
@@ -85,12 +80,20 @@ __device__ __forceinline__ void prepare_octet(const PrepareArgs &a, int64_t i) {
 
 // The eight codes of a word as bf16, in the order kQuads.  A byte of 0 to 15 is that many 2^-9 as an 8-bit float (four exponent bits, three of mantissa): the
 // conversion takes two at a time.
-__device__ __forceinline__ void plain_codes(uint32_t w, u32x4_t &o) {
-  const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
+__device__ __forceinline__ void quads_of(uint32_t even, uint32_t odd, u32x4_t &o) {
   o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false));
   o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false));
   o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true));
   o[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, true));
+}
+__device__ __forceinline__ void plain_codes(uint32_t w, u32x4_t &o) { quads_of(w & 0x0f0f0f0fu, (w >> 4) & 0x0f0f0f0fu, o); }
+// The same less 8: sizes of 0 to 8 in all eight nibbles at once (a code under the centre is its complement and one more), the sign in front of them in a byte.  Five instructions
+// more than without a centre, for a word.
+__device__ __forceinline__ void signed_codes(uint32_t w, u32x4_t &o) {
+  uint32_t under = ~w & 0x88888888u;
+  asm("" : "+v"(under));  // (bits that are known to be zero would be taken out of the selections below, an instruction each)
+  const uint32_t one = under >> 3, size = (w ^ (0x88888888u - one)) + one;
+  quads_of((size & 0x0f0f0f0fu) | (under << 4 & 0xf0f0f0f0u), (size >> 4 & 0x0f0f0f0fu) | (under & 0xf0f0f0f0u), o);
 }
 
 // silu(g) u, fp32.  The quotient is as the division gives it.  1 + exp(-g) reaches 2^128, so the reciprocal is taken of a quarter of it (beyond 2^126 that of a

@@ -1,10 +1,12 @@
 // Grouped quantized product of short pieces: the segments of a mixture-of-experts block in pieces of up to 64 token rows, 4- and 8-bit codes.
 //
 // Contract: mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:160-230).  The arithmetic is qmm_tiles.hip's: raw codes, the scale applied to the sums
-// of a group, the bias term a product of its own over the group sums.  4-bit codes in groups of 64 have no centre.  Other 4-bit codes are multiplied as they are as
-// well, but a group's sums (of 128: a half's) start from -8 times the sum of x, so that they end as the centred codes'; 8-bit codes are centred on the way in.  Share of
-// results that are not the float64 product's nearest value, before (codes centred on the way in) / now, K = 2048: groups of 32
-// 1.1e-4 to 1.3e-4 / 1.2e-4 to 1.3e-4, of 128 0.8e-4 to 0.9e-4 / 1.2e-4 to 1.4e-4 (plain float32 sums 0.9e-4 to 1.5e-4); one start for all of 128 2.1e-4.
+// of a group, the bias term a product of its own over the group sums.  4-bit codes in groups of 64 have no centre, others are centred on the way in (signed_codes,
+// centred_codes).  Share of results that are not the float64 product's nearest value, tiles of 32 x 32 results, which had these pieces before / here, K = 1024, 2048,
+// 4096 (1e-4): 4-bit groups of 32 0.93, 1.21, 1.63 / the same, of 128 0.71, 0.89, 1.18 / 0.51, 0.66, 0.92 (scaled once for 128 values); 8-bit, of 32 0.87, 1.24, 1.71 / the same, of 128 0.75,
+// 1.00, 1.24 / 0.76, 1.00, 1.24.  4-bit codes as they are, in sums that start from -8 times the sum of x, lose more (0.99, 1.28, 1.71; 0.98, 1.21, 1.74) and are no faster: us of a
+// forward, those / centred, 128 experts, hidden 2048, groups of 32 at 100 / 256 / 512 tokens, even 121, 130, 149 / 122, 134, 149, Zipf-1.1 83, 101, 143 / 86, 100, 143; of 128 92, 108, 119 /
+// 93, 107, 118 and 69, 84, 113 / 71, 83, 115.
 #include <type_traits>
 
 #include "lds_copies.hpp"
@@ -17,16 +19,16 @@ constexpr int kWaves = 8, kHalf = kWaves / 2, kShortLds = 80 * 1024;  // two blo
 // What a block of 16 MT token rows is made of.  A stage is 64 bytes of codes a weight row, 32 weight rows a wave.
 template <int BITS, int GROUP, int MT>
 struct Short {
-  static constexpr bool kPlain = BITS == 4 && GROUP == 64, kStart = BITS == 4 && !kPlain;  // no centre; sums that start from the centre's share
+  static constexpr bool kPlain = BITS == 4 && GROUP == 64;  // no centre
   static constexpr int KS = BITS == 4 ? 128 : 64, XROW = KS * 2;                            // K values of a stage, bytes of a token row
-  static constexpr int SUB = GROUP == 32 ? 32 : 64, NG = KS / SUB, H = SUB / 32;            // what is scaled at once, of a stage; multiplies of that
+  static constexpr int SUB = GROUP < KS ? GROUP : KS, NG = KS / SUB, H = SUB / 32;         // what is scaled at once, of a stage; multiplies of that
   // A window's groups: its scales are fetched 16 at a time, or from a word on where a row has an odd number of them (groups of 128), and its group sums
   // have to fit a token row's place.
   static constexpr int GW = BITS == 8 ? (GROUP == 128 ? 4 : 8) : (GROUP == 128 ? 8 : 16), NW = GW * GROUP / KS;
   static constexpr int SLOTS = sum_slots(kPlain);
-  static constexpr int X = 16 * MT * XROW, W = 2048, STAGE = X + kWaves * W, WINDOW = 1024, STARTS = kStart ? NW * NG * 16 * MT * 4 : 0;
-  static constexpr int S = 3 * STAGE + kWaves * WINDOW + STARTS <= kShortLds ? 3 : 2;
-  static constexpr int BYTES = S * STAGE + kWaves * WINDOW + STARTS;
+  static constexpr int X = 16 * MT * XROW, W = 2048, STAGE = X + kWaves * W, WINDOW = 1024;
+  static constexpr int S = 3 * STAGE + kWaves * WINDOW <= kShortLds ? 3 : 2;
+  static constexpr int BYTES = S * STAGE + kWaves * WINDOW;
   static constexpr int XALL = X / 1024, XI = (XALL + kWaves - 1) / kWaves;  // copies of a stage's token rows, and of a wave (where they do not go round, waves make the same ones)
   static constexpr int COPIES = XI + 2;
   static_assert(BYTES <= kShortLds && 16 * MT * (272 + 132 * 4) <= kShortLds && (NW == 4 || NW == 8), "two blocks share a CU");
@@ -34,8 +36,7 @@ struct Short {
 
 // 16 MT token rows from sorted row `row0` (`rows` of them real) x 256 weight rows of expert e by eight waves of 32 weight rows each: GLU, 128 columns of h from n0:
 // waves 0 to 3 the gate rows, 4 to 7 the up rows; else 256 columns from n0.
-// A lane (weight row or token l % 16, quarter l / 16) multiplies 16 consecutive K values of a group in two steps of v_mfma_f32_16x16x32_bf16; the sums of a group
-// are scaled once.
+// A lane (weight row or token l % 16, quarter l / 16) multiplies a quarter of the K values that are scaled at once in steps of eight, v_mfma_f32_16x16x32_bf16.
 // What bounds it: at few rows an expert memory (128 experts, K = 2048, 1536 columns, 100 tokens: 226 MB in 47 us), then the latency of a stage, a chain of reads of LDS,
 // unpacking and multiplies that four waves of a SIMD fill up for each other.  That is why it is four: tiles of 32 x 32 results (qmm_pieces_kernel, which
 // took these pieces) want 250 registers and leave two, whose stages took 2700 cycles where their vector instructions are 1630.  And why the stages are written
@@ -113,9 +114,8 @@ __device__ __forceinline__ void multiply_short(const CodesArgs &a, int e, int64_
     weights_of(0, p + 1);
   }
   unsigned char *const mine_at = lds_raw + R::X + wave * R::W, *const scales = lds_raw + S * R::STAGE + wave * R::WINDOW;  // [weight row][16]
-  float *const starts = reinterpret_cast<float *>(lds_raw + S * R::STAGE + kWaves * R::WINDOW);                           // [SUB values][token row]
   // Where a lane's pieces lie, each in a register whose parts the compiler does not see: constants beyond 64 KB of LDS would each take one of their own.
-  uint32_t f_at[NG * H], q_at[NG], s_at[2], start_at = S * R::STAGE + kWaves * R::WINDOW + 16 * kq;
+  uint32_t f_at[NG * H], q_at[NG], s_at[2];
 #pragma unroll
   for (int i = 0; i < NG * H; ++i) f_at[i] = ln * XROW + (((i / H * (R::SUB / 8) + kq * H + i % H) ^ turned(ln)) << 4);
 #pragma unroll
@@ -134,23 +134,19 @@ __device__ __forceinline__ void multiply_short(const CodesArgs &a, int e, int64_
   for (int i = 0; i < NG * H; ++i) asm volatile("" : "+v"(f_at[i]));
 #pragma unroll
   for (int g = 0; g < NG; ++g) asm volatile("" : "+v"(q_at[g]));
-  asm volatile("" : "+v"(start_at));
   auto code_stage = [&](int k, int n) __attribute__((always_inline)) {
     uint32_t from = place(n);
     if constexpr ((NW + 1) % S != 0) asm volatile("" : "+s"(from));  // (added where it is wanted: every stage's addresses at once do not fit the registers)
     begin();
     rows_of(k, n + S - 1);
-    constexpr int STEPS = NG * MT, AHEAD = MT < 2 && H == 2 ? 1 : 2;  // sixteen rows of SUB values each; fetched ahead
+    constexpr int STEPS = NG * MT, AHEAD = (MT < 2 && H == 2) || H == 4 ? 1 : 2;  // sixteen rows of SUB values each; fetched ahead
     uint32_t q[2][4], s2[2][2];
     u32x4_t F[AHEAD][H];
-    f32x4_t start[R::kStart ? AHEAD : 1];
     auto fetch = [&](int i) __attribute__((always_inline)) {
       if (i >= STEPS) return;
       const int g = i / MT, m = i % MT;
 #pragma unroll
       for (int h = 0; h < H; ++h) F[i % AHEAD][h] = *reinterpret_cast<const u32x4_t *>(lds_raw + f_at[g * H + h] + from + m * (16 * XROW));
-      if constexpr (R::kStart)
-        start[i % AHEAD] = *reinterpret_cast<const f32x4_t *>(lds_raw + start_at + ((n - 1) * NG + g) * (64 * MT) + 64 * m);
     };
 #pragma unroll
     for (int g = 0; g < NG; ++g)
@@ -173,7 +169,8 @@ __device__ __forceinline__ void multiply_short(const CodesArgs &a, int e, int64_
         for (int h = 0; h < H; ++h) {
           const int i = g * H + h;
           if constexpr (BITS == 4) {
-            plain_codes(q[j][i], op[j][h]);
+            if constexpr (R::kPlain) plain_codes(q[j][i], op[j][h]);
+            else signed_codes(q[j][i], op[j][h]);
           } else {
 #pragma unroll
             for (int w = 0; w < 2; ++w) {
@@ -198,7 +195,7 @@ __device__ __forceinline__ void multiply_short(const CodesArgs &a, int e, int64_
 #pragma unroll
         for (int h = 0; h < H; ++h)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) acc[j] = mfma<0>(F[i % AHEAD][h], op[j][h], h ? acc[j] : R::kStart ? start[R::kStart ? i % AHEAD : 0] : zero);
+          for (int j = 0; j < 2; ++j) acc[j] = mfma<0>(F[i % AHEAD][h], op[j][h], h ? acc[j] : zero);
         fetch(i + AHEAD);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -220,11 +217,18 @@ __device__ __forceinline__ void multiply_short(const CodesArgs &a, int e, int64_
       begin();
       rows_of(k, S - 1);
       const int real = G - (k >> GLOG);
-      constexpr int PER = 32 / R::SLOTS, NB = (R::GW + PER - 1) / PER;  // groups of a multiply, multiplies
+      // groups of a multiply, multiplies; the four groups of 128 of a window are added with the next one's, by every other window (one rounding for two)
+      constexpr int PER = 32 / R::SLOTS, NB = (R::GW + PER - 1) / PER, MOST = R::GW == 4 ? 2 * NB : NB;
+      const int here = MOST == NB ? NB : k & NW * KS ? 0 : MOST;
       const unsigned char *const rows_at = lds_raw + place(0), *const mine = mine_at + place(0);
       f32x4_t sum[2][MT];
 #pragma unroll
-      for (int i = 0; i < NB; ++i) {
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) sum[j][m] = zero;
+#pragma unroll
+      for (int i = 0; i < MOST; ++i) {
+        if (i >= here) break;
         u32x4_t F[MT], o[2];
 #pragma unroll
         for (int m = 0; m < MT; ++m) F[m] = *reinterpret_cast<const u32x4_t *>(rows_at + m * (16 * XROW) + ln * XROW + (((4 * i + kq) ^ turned(ln)) << 4));
@@ -245,20 +249,9 @@ __device__ __forceinline__ void multiply_short(const CodesArgs &a, int e, int64_
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) sum[j][m] = mfma<0>(F[m], o[j], i ? sum[j][m] : zero);
+          for (int j = 0; j < 2; ++j) sum[j][m] = mfma<0>(F[m], o[j], sum[j][m]);
       }
       *reinterpret_cast<u32x4_t *>(scales + lane * 16) = *reinterpret_cast<const u32x4_t *>(mine + lane * 16);
-      if constexpr (R::kStart) {  // (the barrier of the next stage is between this and what reads it)
-#pragma unroll
-        for (int i0 = 0; i0 < R::STARTS / 4; i0 += 64 * kWaves) {
-          const int i = i0 + (int)threadIdx.x, part = i / (16 * MT), row = i % (16 * MT), g = GROUP == 128 ? part / 2 : part;
-          if (i < R::STARTS / 4) {
-            const uint4 p = *reinterpret_cast<const uint4 *>(rows_at + row * XROW + ((g ^ turned(row)) << 4));
-            const float sum = (bf16lo_to_f32(p.x) + bf16hi_to_f32(p.x)) + bf16lo_to_f32(p.y), half = bf16lo_to_f32(p.w);
-            starts[i] = (GROUP != 128 ? sum : part & 1 ? sum - half : half) * -centre_of(BITS);
-          }
-        }
-      }
       wait_reads();
       weights_of(k, S);
 #pragma unroll
@@ -368,12 +361,11 @@ __device__ __forceinline__ void multiply_short(const CodesArgs &a, int e, int64_
       sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
       sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
       if (GROUP >= 64) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
-      const float half = GROUP == 128 ? sum : 0.f;
       if (GROUP == 128) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
       if (row < rows) {
         *reinterpret_cast<u32x4_t *>(static_cast<uint16_t *>(a.y) + (row0 + row) * N + n0 + 8 * piece) = w;
         uint16_t *const sums = a.y_sums + (row0 + row) * padded * R::SLOTS;
-        if (piece % LANES == 0) put_sums(sums + g0 * R::SLOTS, R::SLOTS, sum, half);
+        if (piece % LANES == 0) put_sums(sums + g0 * R::SLOTS, R::SLOTS, sum);
         if (n0 + 128 >= N)  // the last block of a row writes the zeros behind its sums
           for (int g = groups + piece; g < padded; g += 16) put_sums(sums + g * R::SLOTS, R::SLOTS, 0.f);
       }
