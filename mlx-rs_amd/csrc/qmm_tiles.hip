@@ -1,5 +1,5 @@
 // Tiled quantized product on raw codes: activations in bfloat16 or float16, groups of 32, 64 or 128, any number of
-// output columns; dense, or the tiles of a list (the segments of a mixture-of-experts block).
+// output columns; dense, or (4-bit codes in groups of 64) the pieces of a mixture-of-experts block's segments.
 //
 // Contract: mlx_quantized_matmul / mlx_gather_qmm with transpose = true (mlx-rs/src/ops/quantization.rs:91-122,160-230).
 //
@@ -60,12 +60,14 @@ constexpr int waves_of(int waves, int lds) {
   return blocks * waves > 8 ? blocks * waves / 4 : 2;
 }
 
-template <int DT, int BITS, bool G32, bool MID, int MS, int NT, int WN, int S>
+// LIST: pieces of a block with 4-bit codes in groups of 64 (bf16); else dense.
+template <int DT, int BITS, bool G32, bool LIST, int MS, int NT, int WN, int S>
 struct Tile {
+  static_assert(!LIST || (DT == 0 && BITS == 4 && !G32), "other blocks' pieces: qmm_short.hip, qmm_bytes.hip");
   typedef typename ElemOf<DT>::type T;
   typedef Ring<BITS, MS, NT, WN, S> R;
   static constexpr bool SPLIT = BITS == 8 || G32;  // which K values a multiply takes: see unpack
-  static constexpr bool kPlainCodes = MID && BITS == 4 && DT == 0;
+  static constexpr bool kPlainCodes = LIST;
   static constexpr float kCentre = kPlainCodes ? 0.0f : centre_of(BITS);                       // the codes are multiplied as
   static constexpr float kUnit = BITS == 4 && DT == 0 && !kPlainCodes ? 0.0625f : 1.0f;  // (q - kCentre) / kUnit
   static constexpr int JS = R::KS / 64;  // steps of a stage
@@ -236,14 +238,14 @@ __device__ __forceinline__ void output_rows(const CodesArgs &a, int64_t row0, in
 }
 // The results of a piece of up to 32 MS rows x 256 weight rows (of a block; four waves, 64 weight rows each) go out: N is a multiple of
 // 128, there is no bias of the layer's.  Two rows of a column become one register, neighbouring lanes swap halves, and the rows are turned round in LDS:
-// GLU: by the whole block, whose 256 bytes a row are one to four quantisation groups of h, of which the lanes that store them also write the group sums;
+// GLU: by the whole block, whose 256 bytes a row are two quantisation groups of h, of which the lanes that store them also write the group sums;
 // else by each wave, 128 bytes a row.  (Rows found and stored 16 at a time behind a load of their places each: 12 us of the 37 of a block of 128 rows, K = 768.)
-template <int BITS, bool PLAIN, bool GLU, int MS, class WeightRow>
-__device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&tot)[MS][2][16], int wave, int lane, int n0, int64_t row0, int rows, int64_t ebase, int glog,
+template <bool GLU, int MS, class WeightRow>
+__device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&tot)[MS][2][16], int wave, int lane, int n0, int64_t row0, int rows, int64_t ebase,
                                             WeightRow weight_row, const uint32_t (&dst)[2], unsigned char *lds_raw) {
   constexpr int ROWB = GLU ? 272 : 144;  // (16 bytes keep rows off each other's banks)
-  constexpr int SLOTS = sum_slots(PLAIN);
-  const int N = a.N, K = a.K, G = K >> glog, row_bytes = K * BITS / 8, ln = lane & 31, kb = lane >> 5;
+  constexpr int SLOTS = sum_slots(true);
+  const int N = a.N, K = a.K, G = K >> 6, row_bytes = K / 2, ln = lane & 31, kb = lane >> 5;
   unsigned char *const mine = GLU ? lds_raw + wave * 64 : lds_raw + wave * (32 * ROWB);
   auto value = [&](int m, int t, int r) __attribute__((always_inline)) { return GLU ? gated(tot[m][0][r], tot[m][1][r]) : tot[m][t][r]; };
   float odd = 0.f;  // no number once a result was not finite
@@ -291,8 +293,8 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
 #pragma unroll
       for (int j = 0; j < (GLU ? 2 : 1); ++j) {
         const int64_t wrow = ebase + weight_row(GLU ? j : t, ln);
-        plain_rows<BITS, 4, uint16_t>(xs, PLAIN ? RowOrder::kQuads : row_order(BITS), (j ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const uint16_t *>(j ? a.s1 : a.s0) + wrow * G,
-                                   static_cast<const uint16_t *>(j ? a.b1 : a.b0) + wrow * G, K, 1 << glog, open, v[j]);
+        plain_rows<4, 4, uint16_t>(xs, RowOrder::kQuads, (j ? a.w1 : a.w0) + wrow * (row_bytes / 4), static_cast<const uint16_t *>(j ? a.s1 : a.s0) + wrow * G,
+                                   static_cast<const uint16_t *>(j ? a.b1 : a.b0) + wrow * G, K, 64, open, v[j]);
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -307,7 +309,7 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
     for (int m = 0; m < MS; ++m) turn(m, 32 * m);
     if (__builtin_expect(odd != odd, 0)) repair(0, MS, 0);
     __syncthreads();
-    const int groups = N >> glog, padded = padded_groups(groups), lanes = 1 << (glog - 3);  // (the output's groups are as long as the input's)
+    const int groups = N >> 6, padded = padded_groups(groups);
 #pragma unroll
     for (int i = 0; i < 2 * MS; ++i) {
       const int row = 16 * i + (int)(threadIdx.x >> 4), piece = threadIdx.x & 15;
@@ -316,11 +318,10 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
                   ((bf16lo_to_f32(w[2]) + bf16hi_to_f32(w[2])) + (bf16lo_to_f32(w[3]) + bf16hi_to_f32(w[3])));
       sum += __uint_as_float(dpp_u32<kDppXor1>(__float_as_uint(sum)));
       sum += __uint_as_float(dpp_u32<kDppXor2>(__float_as_uint(sum)));
-      if (PLAIN || glog >= 6) sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
-      if (!PLAIN && glog == 7) sum += __uint_as_float(dpp_u32<kDppMirror>(__float_as_uint(sum)));
+      sum += __uint_as_float(dpp_u32<kDppHalfMirror>(__float_as_uint(sum)));
       if (row < rows) {
         *reinterpret_cast<u32x4_t *>(static_cast<uint16_t *>(a.y) + (row0 + row) * N + n0 + 8 * piece) = w;
-        if ((piece & (lanes - 1)) == 0) put_sums(a.y_sums + ((row0 + row) * padded + (n0 >> glog) + (piece >> (glog - 3))) * SLOTS, SLOTS, sum);
+        if ((piece & 7) == 0) put_sums(a.y_sums + ((row0 + row) * padded + (n0 >> 6) + (piece >> 3)) * SLOTS, SLOTS, sum);
       }
     }
     if (n0 + 128 >= N && groups < padded)  // the last block of a row writes the zeros behind its sums
@@ -365,9 +366,9 @@ __device__ __forceinline__ void write_piece(const CodesArgs &a, const float (&to
 // 58.7 us for the call = 444 TFLOP/s (tiles of 64 x 128 with the codes loaded into registers 63.4).
 // Blocks (128 experts, hidden 2048, 4-bit, groups of 64), us of a forward at 128 / 320 / 1024 tokens, even routing: 110 / 121 / 174; with streamed
 // segments, 256-column tiles and a copy of x on four streams, which they took at first, 151 / 216 / 266.
-template <int DT, int BITS, bool G32, bool LIST, bool GLU, bool MID, int MS, int NT, int WN, int KW, int S>
+template <int DT, int BITS, bool G32, bool LIST, bool GLU, int MS, int NT, int WN, int KW, int S>
 __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t row0, int rows, int n0, int scale_shift, unsigned char *lds_raw) {
-  typedef Tile<DT, BITS, G32, MID, MS, NT, WN, S> P;
+  typedef Tile<DT, BITS, G32, LIST, MS, NT, WN, S> P;
   typedef typename P::R R;
   typedef typename P::T T;
   constexpr int GB = P::GB;
@@ -722,7 +723,7 @@ __device__ __forceinline__ void multiply_tile(const CodesArgs &a, int e, int64_t
     if (kg != 0) return;
   }
 
-  if constexpr (LIST) write_piece<BITS, P::kPlainCodes, GLU, MS>(a, tot, wave, lane, n0, row0, rows, ebase, glog, weight_row, dst, lds_raw);
+  if constexpr (LIST) write_piece<GLU, MS>(a, tot, wave, lane, n0, row0, rows, ebase, weight_row, dst, lds_raw);
   else write_tile<DT, BITS, MS, NT, WN>(a, tot, wave, lane, col0, row0, rows, glog, weight_row, lds_raw);
 }
 
@@ -933,7 +934,7 @@ __device__ __forceinline__ void multiply_long_tile(const CodesArgs &a, int e, in
   if constexpr (!GLU) output_rows(a, row0, rows, lane, dst);
   wait_copies<0>();
   block_barrier();
-  write_piece<4, true, GLU, MS>(a, tot, wave, lane, n0, row0, rows, ebase, 6, weight_row, dst, lds_raw);
+  write_piece<GLU, MS>(a, tot, wave, lane, n0, row0, rows, ebase, weight_row, dst, lds_raw);
 }
 
 // The tiles of a list of pieces of up to 128 rows (ShortTiles::piece), 4-bit codes in groups of 64: by their rows, 32 at a time.
@@ -951,10 +952,10 @@ __global__ __launch_bounds__(256, 2) void qmm_pieces_kernel(CodesArgs a, const u
   extern __shared__ __align__(16) unsigned char lds_raw[];
   if (rows > 96) return multiply_long_tile<GLU, 4>(a, e, row0, rows, nt * NI, lds_raw);
   if (rows > 64) return multiply_long_tile<GLU, 3>(a, e, row0, rows, nt * NI, lds_raw);
-  if (rows > 32) return multiply_tile<0, 4, false, true, GLU, true, 2, 2, 4, 1, 2>(a, e, row0, rows, nt * NI, 0, lds_raw);
+  if (rows > 32) return multiply_tile<0, 4, false, true, GLU, 2, 2, 4, 1, 2>(a, e, row0, rows, nt * NI, 0, lds_raw);
   typedef Ring<4, 1, 2, 4, 2> Short;
   constexpr int S1 = (kHalfLds - 4 * Short::WINDOW) / Short::STAGE;  // as many stages as fit
-  multiply_tile<0, 4, false, true, GLU, true, 1, 2, 4, 1, S1>(a, e, row0, rows, nt * NI, 0, lds_raw);
+  multiply_tile<0, 4, false, true, GLU, 1, 2, 4, 1, S1>(a, e, row0, rows, nt * NI, 0, lds_raw);
 }
 
 // A block computes 32 MS token rows x 32 WN weight rows with WN KW waves (see multiply_tile), tiles of up to 32 rows with half the
@@ -974,11 +975,11 @@ __global__ __launch_bounds__(64 * WN * KW, waves_of(WN * KW, lds_of(KW, Ring<BIT
     if (rows <= 32) {
       typedef Ring<BITS, 1, NT, WN, 2> Short;
       constexpr int S1 = (lds_of(KW, Ring<BITS, MS, NT, WN, S>::BYTES) / KW - WN * Short::WINDOW) / Short::STAGE;  // as many stages as fit
-      multiply_tile<DT, BITS, G32, false, false, false, 1, NT, WN, KW, S1>(a, 0, row0, rows, nt * NI, scale_shift, lds_raw);
+      multiply_tile<DT, BITS, G32, false, false, 1, NT, WN, KW, S1>(a, 0, row0, rows, nt * NI, scale_shift, lds_raw);
       return;
     }
   }
-  multiply_tile<DT, BITS, G32, false, false, false, MS, NT, WN, KW, S>(a, 0, row0, rows, nt * NI, scale_shift, lds_raw);
+  multiply_tile<DT, BITS, G32, false, false, MS, NT, WN, KW, S>(a, 0, row0, rows, nt * NI, scale_shift, lds_raw);
 }
 
 size_t codes_copy_bytes(int bits, int64_t rows, int K) {
