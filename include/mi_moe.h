@@ -116,6 +116,7 @@ void mi_moe_set_error_handler(void (*handler)(const char *msg, void *data), void
  * mlx-lm/src/models/qwen3.rs:204-255, call site :321-324) ---- */
 int mi_moe_create(const mi_moe_config *cfg, const mi_moe_weights *weights, mi_moe_handle *out);
 int mi_moe_destroy(mi_moe_handle h);
+/* the workspace with which a batch of max_tokens, and every smaller one, takes the kernels it is given in one of its own */
 int mi_moe_workspace_size(const mi_moe_config *cfg, int64_t max_tokens, size_t *bytes);
 /* x: bf16 [T, H] -> out: bf16 [T, H].  workspace: device memory of at least
  * mi_moe_workspace_size(cfg, T) bytes, 256-byte aligned, contents irrelevant. */
@@ -331,12 +332,12 @@ int mi_moe_debug_plan_grouped(int32_t N, int32_t K, int32_t bits, int32_t glu, i
                               int32_t max_active, int64_t max_rows_per_expert,
                               int64_t max_streamed_rows, int32_t tile_lists, int32_t paired_out,
                               char *out, size_t cap);
-/* which rows of a forward of T tokens go where: *tiled = 1: M-tile lists are built; *tile_min_rows = a segment of
- * at least that many rows is cut into 256-row tiles, with its remainder in the 256-, 128- or 64-row list that
- * holds it; shorter segments stream.  (8-bit codes in groups of 64 from 24 rows an expert on: into
- * pieces of up to 128 rows instead, given a workspace of mi_moe_workspace_size.)  *tiled = 2: every segment is cut into tiles of up to 128 rows on raw codes (groups
- * of 64, batches beyond the streamed ones; given such a workspace); 3: so is every segment of
- * *tile_min_rows rows and more (larger batches), shorter segments stream */
+/* which rows of a forward of T tokens go where: *tiled = 1: a segment of at least *tile_min_rows rows is cut into 256-row
+ * tiles, with its remainder in the 256-, 128- or 64-row list that holds it; shorter segments stream.  (Most 8-bit batches from
+ * 24 rows an expert on are answered so, too, but have pieces of up to 128 rows in place of the tiles, given a workspace of
+ * mi_moe_workspace_size: mi_moe_forward_timed then reports one launch beside the streamed one.)  *tiled = 2: every segment is
+ * cut into pieces of up to 128 rows on raw codes (batches beyond the streamed ones; given such a workspace); 3: so is every
+ * segment of *tile_min_rows rows and more (larger batches with 4-bit codes), shorter segments stream */
 int mi_moe_debug_tile_rule(const mi_moe_config *cfg, int64_t T, int32_t *tiled, int32_t *tile_min_rows);
 int32_t mi_moe_debug_side_streams_created(void);
 

@@ -160,8 +160,9 @@ def _plan_entries(buf):
 
 def tile_rule(cfg, tokens):
     """(tile lists are built, rows from which a segment is tiled) for a forward of `tokens` tokens: the
-    library's own rule (needs no GPU).  The first is 2 where every segment goes in tiles on raw codes, 3 where those from the
-    second's rows on do and the others stream."""
+    library's own rule (needs no GPU).  The first is 2 where every segment goes in pieces on raw codes, 3 where those from the
+    second's rows on do and the others stream; 1 also for 8-bit batches whose segments of that many rows go in pieces on
+    dequantised weights."""
     tiled, tmr = C.c_int32(), C.c_int32()
     check(load_library().mi_moe_debug_tile_rule(C.byref(cfg), tokens, C.byref(tiled), C.byref(tmr)))
     return tiled.value, tmr.value

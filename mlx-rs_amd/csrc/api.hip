@@ -228,8 +228,11 @@ int piece_rows(int64_t pairs, int n_experts) { return short_pieces(pairs, n_expe
 //                      4096 209, 276, 549 / 163, 238, 529
 //   64, 6, 2048, 1408  even at 400 / 1400 / 2000 232, 372, 381 / 181, 320, 398; Zipf-1.1 at 1400 / 2400 400, 486 / 326, 438
 //   16, 4, 4096, 6400  even at 100 / 400 459, 565 / 374, 469
-// Rows of 2048 values are short enough for a block's ends to weigh, and with even routing and 180 rows an expert and more the other route's blocks have fewer of them:
-// there it stays, up to rows of 4096.
+// Even routing from 170 to 255 rows an expert on average is where the other route is at its best, one tile of 256 rows for nearly every expert and two pieces here: 64, 6, 4096, 1408 at 1800 /
+// 2200 / 2600 / 3000 tokens 679, 689, 793, 1000 / 688, 735, 818, 940; 128, 8, 4096, 1536 at 2500 / 3200 / 3600 / 4096 1429, 1456, 1525, 1852 / 1408, 1551, 1635, 1800; 32, 4, 4096, 2048 at 1300 /
+// 1900 / 2100 490, 552, 667 / 507, 582, 625; 64, 8, 6144, 2048 at 1700 1373 / 1488.  Any skew turns it round, and the host does not see which it is: Zipf-0.5 and 1.1, 64, 6, 4096, 1408 at 2200 794,
+// 813 / 712, 745, 128, 8, 4096, 1536 at 3200 1547, 1627 / 1425, 1517; Zipf-1.1, 32, 4, 4096, 2048 at 1900 661 / 542, 64, 8, 6144, 2048 at 1700 1567 / 1424.  Rows of 2048 values are short enough
+// for a block's ends to weigh, and there the other route stays from 176 rows an expert on.
 bool piece_batch(const mi_moe_config &c, int64_t T, bool heavy) {
   const int64_t P = T * c.top_k;
   if (!heavy || T <= kFusedRouterMaxTokens || c.n_experts < 8 || !codes_tiles_fit(c, T)) return false;
@@ -353,7 +356,8 @@ ForwardWs carve_forward(const mi_moe_config &c, int64_t T, void *ws, bool norm) 
 // A batch is taken whose least workspace (ForwardWs::bytes_min) is MI_MOE_STATIC_SCRATCH_BYTES or less.  The same again lies behind it for what the tiles on raw
 // codes want beyond that (bytes_raw), so that such a batch takes the kernels that mi_moe_forward gives it.  That is never more: the copy of x has the size of the
 // normalised rows, its group sums at most that of the down product's rows, those of h at most h's (K is a multiple of 128 there, and 16 groups of sums, to whole
-// numbers of which they are padded, are no larger than 128 values), and a list of at least four rows a segment is smaller than two of the arrays of pairs.
+// numbers of which they are padded, are no larger than 128 values), and a list of at least four rows a segment is smaller than two of the arrays of pairs.  Records of
+// several a segment, where there are no tiles, are the experts' and 8 bytes a pair, less than the pairs' rows.
 constexpr size_t kStaticScratch = (size_t)2 * MI_MOE_STATIC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char scratch[kStaticScratch];
 

@@ -414,9 +414,9 @@ struct RowsArgs {
 constexpr int kRowsMost = 16;  // rows of one pass of that kernel
 bool qmm_rows_applies(const RowsArgs &a, int group, int bits, int dt, bool glu);
 hipError_t launch_qmm_rows(const RowsArgs &a, int group, int bits, int dt, bool glu, hipStream_t st);
-// The tiled product over weights packed along N (qmm_cols.hip): x [M, K], w [K, N].
 // The product of dense float32 rows on the float32 matrix instructions (qmm_f32.hip).
 hipError_t launch_qmm_f32(const float *x, const uint32_t *w, const float *s, const float *b, int64_t rows, int N, int K, int group, int bits, float *y, hipStream_t st);
+// The tiled product over weights packed along N (qmm_cols.hip): x [M, K], w [K, N].
 struct ColsArgs {
   const void *x;
   const uint32_t *w;

@@ -329,7 +329,10 @@ static hipError_t start_bytes(const CodesArgs &a, const uint32_t *list, int cap,
 }
 // Where no CU gets two blocks (a down product of few experts: 8 pieces are 128 blocks of 256 of 4096 columns), the length of a block's K is what counts, and two groups of waves
 // share it; and where there are fewer blocks still, they are of 128 columns, so that more CUs have one.  8 experts, 4096 x 14336, us of a forward, K not shared / 256 columns / 128:
-// 100 tokens 441 / 425 / 382 to 425, 160 481 / 448 / 400, 200 488 / 455 / 410, 256 534 / 485 / 437, 400 tokens - / 563 / 497; 512 tokens (two pieces an expert) - / 674 / 706.
+// 100 tokens 446 / 418 / 373, 200 476 / 446 / 400, 256 503 / 466 / 420, 400 574 / 546 / 474.  As many blocks as CUs (the list's capacity, which holds a second piece for every expert): a second
+// piece of an expert then finds no CU left among blocks of 128, and K not shared leaves CUs with one block: 512 tokens 656 / 624 / 654, 540 735 / 694 / 737, Zipf-1.1 632 / 606 / 624 and
+// 651 / 634 / 658; 16 experts, 4 a token, 2048 x 6400 at 512 / 543 tokens 322, 344 / 313, 335 / 319, 348, Zipf-1.1 376, 392 / 366, 383 / 375, 392.  More blocks: 576 and 700 tokens 761, 789 / 749,
+// 780 / 803, 843, 1000 962 / 1002 / 1045; 16 experts, 4096 x 6400 at 512 / 600 tokens 548, 684 / 592, 726 / 595, 753.
 template <bool GLU>
 static hipError_t start_bytes(const CodesArgs &a, const uint32_t *list, int cap, hipStream_t st) {
   constexpr int NI = GLU ? 128 : 256;
