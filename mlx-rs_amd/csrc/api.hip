@@ -205,7 +205,11 @@ bool mid_batch(const mi_moe_config &c, int64_t T, bool tiled) {
 //   tokens 312, 299, 552 / 288, 284, 526;
 //   64 experts, 6, hidden 2048, intermediate 1408, even at 100 / 165 / 600 / 900 tokens (56 and 84 rows) 99, 102, 148, 174 / 90, 95, 144, 192; 64, 4, 4096 x 2048, 200 tokens 244 / 230;
 //   256 experts, 8, 2048 x 512, 200 / 500 tokens 145, 151 / 132, 145.
-// With even routing most segments leave a second piece from about 60 rows on average on, and the line lies there; with skewed routing it makes no difference.
+// With even routing most segments leave a second piece from about 60 rows on average on, and the line lies there.  From 48 rows on, where the others are pieces of 96, the two are near each
+// other, and which is ahead goes by the routing, which the host does not see: 128 experts at 800 / 850 / 900 / 955 tokens, hidden 2048, even 163, 163, 166, 171 / 151, 157, 161, 167, Zipf-0.5 166, 168,
+// 173, 176 / 171, 175, 176, 182, 1.1 147, 152, 162, 169 / 151, 156, 160, 169, 1.3 138, 141, 145, 150 / 145, 148, 150, 153; hidden 4096, even 482, 494, 514, 529 / 460, 481, 525, 553, Zipf-1.1 563, 587, 601,
+// 627 / 559, 581, 588, 623; 256 experts, 2048 x 512, 1800 tokens, even and Zipf-1.1 226, 208 / 230, 210; 64 experts at 560 / 639 tokens 146, 152 / 140, 147 and 158, 167 / 154, 165; 16 experts,
+// 2048 x 4096, 220 tokens 127, 144 / 108, 121.
 bool short_pieces(int64_t pairs, int n_experts) { return pairs < (int64_t)60 * n_experts; }
 
 // Rows of a piece beyond those.  Longer ones read a weight row for more token rows; but a block's time grows with its rows, and until the pieces are several times what
